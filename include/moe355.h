@@ -455,6 +455,10 @@ int moe355_token_unpermute(const void *permuted, int dtype, const int32_t *sorte
  *   the arithmetic of moe355_token_unpermute; expert_tokens [num_experts] int64 receives the number of pairs of
  *   every expert (what moe355_init_routing returns as counts), counted by one more workgroup of the same launch.
  *   num_experts <= 2048. */
+/* moe355_pair_order: whether a layer runs a batch in this order when its ids come straight from the gate
+ * (num_logits experts scored, num_experts physical ones). */
+int moe355_pair_order(int64_t num_tokens, int top_k, int num_logits, int num_experts, int64_t hidden,
+                      int64_t intermediate);
 int moe355_gmm_pairs_supported(int64_t num_tokens, int top_k, int64_t n, int64_t k);
 size_t moe355_gmm1_swiglu_quant_pairs_workspace(int64_t num_tokens, int top_k, int64_t n);
 int moe355_gmm1_swiglu_quant_pairs(const int8_t *x, const float *x_scale, const int32_t *topk_ids, int64_t num_tokens,
@@ -500,6 +504,42 @@ int moe355_profile_next_gemm(void *start_event, void *stop_event);
  * epilogue: 0 raw int32 (moe355_gmm_i32), 1 SwiGLU (moe355_gmm1_swiglu_quant), 2 dequant (moe355_gmm2_dequant).
  * A pure function of its arguments, for benchmarks and profiles (no counterpart in the reference). */
 const char *moe355_gmm_kernel_name(int epilogue, int64_t rows, int64_t k, int64_t n, int num_experts);
+
+/* ---------------------------------------------------------------------------
+ * The whole layer in one call: (router gate,) gating, dispatch, expert MLPs, shared expert and combine, enqueued
+ * without a return to the caller in between.  Stands in for AscendRoutedExperts.forward_impl
+ * (vllm_ascend/ops/fused_moe/routed_experts.py:496-609) with the W8A8-dynamic and W4A8-dynamic methods
+ * (quantization/methods/w8a8_dynamic.py:224-301, w4a8.py:155-240), SiLU, no expert map; the operators it enqueues are
+ * the ones above, chosen by the same rules, so the result is the operator sequence's, bit for bit.
+ */
+typedef struct moe355_layer {
+    int64_t hidden, intermediate;
+    int32_t num_experts, top_k;
+    int32_t k_group, group_count, renorm, norm_type; /* group_select_mode is 1, as the router passes it */
+    float routed_scaling_factor, eps, swiglu_limit;
+    int32_t x_dtype;          /* of hidden states, result and routing weights */
+    const void *bias;         /* [E] in the dtype of the logits, or NULL */
+    int32_t weights;          /* 0: int8 tensors; 1: device tables of per-expert int8 tensors; 2: int4 tensors */
+    int32_t pair_order;       /* 0: never; 1: where moe355_pair_order() says so (weights 0 and 1) */
+    const void *w13, *s13, *w2, *s2;
+    int64_t group13, group2;  /* int4: weights along K that share a scale */
+    int32_t *sync_counter;    /* of moe355_route_quant_small; NULL: that launch is not used */
+    /* router gate inside the layer, or NULL */
+    const float *gate_weight, *gate_bias;
+    /* shared expert: 0 none, 1 in line, 2 on shared_stream next to the routed experts */
+    int32_t shared;
+    float shared_limit, shared_alpha, shared_beta;
+    int64_t shared_intermediate;
+    const int8_t *shared_w13, *shared_w2;
+    const float *shared_s13, *shared_s2;
+    void *shared_stream;
+    int64_t *load;            /* [E] int64: the rows of every expert are added to it; or NULL */
+} moe355_layer;
+
+size_t moe355_layer_workspace(const moe355_layer *layer /* host */, int64_t num_tokens);
+/* logits [T, E] of logits_dtype; ignored with a gate inside the layer.  out [T, H]. */
+int moe355_layer_forward(const moe355_layer *layer /* host */, const void *x, const void *logits, int logits_dtype,
+                         int64_t num_tokens, void *out, void *workspace, size_t workspace_bytes, void *stream);
 
 #ifdef __cplusplus
 }

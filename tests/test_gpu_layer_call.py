@@ -1,0 +1,68 @@
+"""The layer as one native call (``layer(x, logits)``) against the operator-by-operator form
+(``layer.forward_impl``): the same bits, over the forms the call chooses between."""
+import copy
+import dataclasses
+
+import pytest
+import torch
+
+from _inputs import CONFIGS, make_layer
+from _layer_utils import build_layer
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _pair(name, tokens, **kw):
+    cfg = dataclasses.replace(CONFIGS[name], T=tokens)
+    d = make_layer(cfg, seed=tokens)
+    return cfg, build_layer(cfg, d, DEV, **kw), d["x"].to(DEV), d["logits"].to(DEV)
+
+
+# one token; the borders of the pair-order forms (three pairs per expert, 1024 pairs) and of the one-launch index maps
+# (4096 pairs); a batch with a ragged end on the sorted path
+@pytest.mark.parametrize("tokens", [1, 24, 25, 127, 128, 129, 512, 513, 1031])
+@pytest.mark.parametrize("name", ["c2_small", "c4_small", "c5_small"])
+def test_one_call_equals_the_operators(name, tokens):
+    cfg, layer, x, logits = _pair(name, tokens, shared=CONFIGS[name].shared)
+    got = layer(x, logits)
+    assert layer._layer_plan.desc is not None
+    assert torch.equal(got, layer.forward_impl(x, logits).routed_out)
+
+
+@pytest.mark.parametrize("tokens", [3, 40, 300])
+@pytest.mark.parametrize("overlap", [False, True])
+def test_shared_expert_in_the_call(tokens, overlap):
+    cfg, layer, x, logits = _pair("c4_small", tokens, shared=True, overlap=overlap)
+    want = layer.forward_impl(x, logits).routed_out
+    for _ in range(3):
+        assert torch.equal(layer(x, logits), want)
+
+
+@pytest.mark.parametrize("tokens", [2, 60, 300])
+def test_weight_lists_and_expert_loads(tokens):
+    cfg, layer, x, logits = _pair("c7_small", tokens, dynamic_eplb=True, collect_expert_load=True)
+    res = layer.forward_impl(x, logits)
+    layer.clear_moe_load()
+    assert torch.equal(layer(x, logits), res.routed_out)
+    assert torch.equal(layer(x, logits), res.routed_out)
+    assert torch.equal(layer.moe_load, 2 * res.expert_tokens)
+    layer.w13_weight_list[1] = layer.w13_weight_list[0].clone()  # one expert swapped: the next call sees it
+    assert torch.equal(layer(x, logits), layer.forward_impl(x, logits).routed_out)
+
+
+def test_the_call_follows_the_layer():
+    """Options that change between calls, and a copied layer."""
+    cfg, layer, x, logits = _pair("c2_small", 40)
+    layer(x, logits)
+    for change in (dict(use_pair_order=False), dict(use_fused_small_batch=False), dict(use_fused_small_batch=True)):
+        for k, v in change.items():
+            setattr(layer, k, v)
+        assert torch.equal(layer(x, logits), layer.forward_impl(x, logits).routed_out)
+    layer.router.renormalize = not layer.router.renormalize
+    assert torch.equal(layer(x, logits), layer.forward_impl(x, logits).routed_out)
+    half = logits.to(torch.bfloat16)
+    assert torch.equal(layer(x, half), layer.forward_impl(x, half).routed_out)
+    assert torch.equal(layer(x[::2], logits[::2]), layer.forward_impl(x[::2], logits[::2]).routed_out)
+    twin = copy.deepcopy(layer)
+    assert torch.equal(twin(x, logits), layer.forward_impl(x, logits).routed_out)

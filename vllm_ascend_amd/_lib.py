@@ -18,6 +18,23 @@ GL_CUMSUM, GL_COUNT = 0, 1
 
 ABI_VERSION = 1
 
+
+
+class Layer(ctypes.Structure):
+    """``moe355_layer``: one layer's weights, options and streams, as the whole-layer call takes them."""
+
+    _fields_ = [
+        ("hidden", c_int64), ("intermediate", c_int64), ("num_experts", c_int), ("top_k", c_int), ("k_group", c_int),
+        ("group_count", c_int), ("renorm", c_int), ("norm_type", c_int), ("routed_scaling_factor", c_float),
+        ("eps", c_float), ("swiglu_limit", c_float), ("x_dtype", c_int), ("bias", c_void_p), ("weights", c_int),
+        ("pair_order", c_int), ("w13", c_void_p), ("s13", c_void_p), ("w2", c_void_p), ("s2", c_void_p),
+        ("group13", c_int64), ("group2", c_int64), ("sync_counter", c_void_p), ("gate_weight", c_void_p),
+        ("gate_bias", c_void_p), ("shared", c_int), ("shared_limit", c_float), ("shared_alpha", c_float),
+        ("shared_beta", c_float), ("shared_intermediate", c_int64), ("shared_w13", c_void_p), ("shared_w2", c_void_p), ("shared_s13", c_void_p),
+        ("shared_s2", c_void_p), ("shared_stream", c_void_p), ("load", c_void_p),
+    ]
+
+
 # name -> (restype, argtypes); mirrors include/moe355.h one to one
 PROTOTYPES = {
     "moe355_abi_version": (c_int, []),
@@ -100,6 +117,10 @@ PROTOTYPES = {
                                                   c_int64, c_int, c_void_p, c_int, c_void_p]),
     "moe355_token_unpermute_pairs": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_int64, c_int, c_int64, c_int,
                                              c_void_p, c_void_p, c_void_p, c_void_p]),
+    "moe355_pair_order": (c_int, [c_int64, c_int, c_int, c_int, c_int64, c_int64]),
+    "moe355_layer_workspace": (c_size_t, [c_void_p, c_int64]),
+    "moe355_layer_forward": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int64, c_void_p, c_void_p, c_size_t,
+                                     c_void_p]),
     "moe355_profile_next_gemm": (c_int, [c_void_p, c_void_p]),
     "moe355_gmm_kernel_name": (c_char_p, [c_int, c_int64, c_int64, c_int64, c_int]),
     "moe355_token_unpermute": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_int64, c_int, c_int64, c_int64, c_void_p,

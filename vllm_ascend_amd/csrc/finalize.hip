@@ -1,7 +1,7 @@
 // Weighted un-permute (finalize routing): one workgroup per token, each lane
 // owns runs of 8 hidden elements (16-byte loads), accumulating the k expert
 // rows in fp32 in slot order.
-#include "moe355_common.h"
+#include "layer_parts.h"
 
 namespace moe355 {
 
@@ -21,14 +21,20 @@ __global__ __launch_bounds__(256) void token_unpermute_kernel(const uint16_t* __
                                                               const uint16_t* __restrict__ residual,
                                                               uint16_t* __restrict__ out,
                                                               const int32_t* __restrict__ hist_ids, int hist_experts,
-                                                              int64_t* __restrict__ hist_out)
+                                                              int64_t* __restrict__ hist_out,
+                                                              const int64_t* __restrict__ load_counts,
+                                                              int64_t* __restrict__ load)
 {
     __shared__ int32_t srow[64];
     __shared__ float sw[64];
     const int top_k = TOPK > 0 ? TOPK : top_k_rt;
-    if (hist_ids && blockIdx.x == gridDim.x - 1) {
+    if ((hist_ids || load) && blockIdx.x == gridDim.x - 1) {
         __shared__ int32_t hcnt[kHistMaxExperts];
         if (blockIdx.y != 0) return;
+        if (!hist_ids) {
+            for (int e = threadIdx.x; e < hist_experts; e += 256) load[e] += load_counts[e];
+            return;
+        }
         for (int e = threadIdx.x; e < hist_experts; e += 256) hcnt[e] = 0;
         __syncthreads();
         for (int64_t f = threadIdx.x; f < permuted_rows; f += 256) {
@@ -36,7 +42,10 @@ __global__ __launch_bounds__(256) void token_unpermute_kernel(const uint16_t* __
             if (e >= 0 && e < hist_experts) atomicAdd(&hcnt[e], 1);
         }
         __syncthreads();
-        for (int e = threadIdx.x; e < hist_experts; e += 256) hist_out[e] = (int64_t)hcnt[e];
+        for (int e = threadIdx.x; e < hist_experts; e += 256) {
+            hist_out[e] = (int64_t)hcnt[e];
+            if (load) load[e] += (int64_t)hcnt[e];
+        }
         return;
     }
     const int64_t t = blockIdx.x;
@@ -103,9 +112,10 @@ __global__ __launch_bounds__(256) void token_unpermute_kernel(const uint16_t* __
 
 using namespace moe355;
 
-static int unpermute_impl(const void* permuted, int dtype, const int32_t* sorted_indices, const void* probs,
-                          int64_t num_tokens, int top_k, int64_t hidden, int64_t permuted_rows, const void* residual,
-                          void* out, const int32_t* hist_ids, int hist_experts, int64_t* hist_out, void* stream)
+int moe355::unpermute_impl(const void* permuted, int dtype, const int32_t* sorted_indices, const void* probs,
+                           int64_t num_tokens, int top_k, int64_t hidden, int64_t permuted_rows, const void* residual,
+                           void* out, const int32_t* hist_ids, int hist_experts, int64_t* hist_out,
+                           const int64_t* load_counts, int64_t* load, void* stream)
 {
     if (num_tokens < 0 || top_k <= 0 || hidden <= 0 || permuted_rows < 0) return MOE355_E_ARG;
     if (dtype != MOE355_DT_BF16 && dtype != MOE355_DT_F16) return MOE355_E_UNSUPPORTED;
@@ -123,9 +133,10 @@ static int unpermute_impl(const void* permuted, int dtype, const int32_t* sorted
         if (pieces < 1) pieces = 1;
     }
 #define MOE355_UNPERMUTE(K, D)                                                                                    \
-    hipLaunchKernelGGL((token_unpermute_kernel<K, D>), dim3((unsigned)num_tokens + (hist_ids ? 1u : 0u), pieces), dim3(256), 0, (hipStream_t)stream, \
+    hipLaunchKernelGGL((token_unpermute_kernel<K, D>), dim3((unsigned)num_tokens + (hist_ids || load ? 1u : 0u), pieces), dim3(256), 0, (hipStream_t)stream, \
                        (const uint16_t*)permuted, sorted_indices, (const uint16_t*)probs, top_k, hidden,             \
-                       permuted_rows, (const uint16_t*)residual, (uint16_t*)out, hist_ids, hist_experts, hist_out)
+                       permuted_rows, (const uint16_t*)residual, (uint16_t*)out, hist_ids, hist_experts, hist_out,  \
+                       load_counts, load)
     if (dtype == MOE355_DT_F16) {
         // fp16 models: the common fan-outs unrolled, the rest through the generic loop
         if (top_k == 8) MOE355_UNPERMUTE(8, MOE355_DT_F16);
@@ -151,7 +162,7 @@ extern "C" int moe355_token_unpermute(const void* permuted, int dtype, const int
 {
     if (num_tokens > 0 && !sorted_indices) return MOE355_E_ARG;
     return unpermute_impl(permuted, dtype, sorted_indices, probs, num_tokens, top_k, hidden, permuted_rows, residual, out,
-                          nullptr, 0, nullptr, stream);
+                          nullptr, 0, nullptr, nullptr, nullptr, stream);
 }
 
 extern "C" int moe355_token_unpermute_pairs(const void* rows, int dtype, const void* probs, const int32_t* topk_ids,
@@ -162,7 +173,7 @@ extern "C" int moe355_token_unpermute_pairs(const void* rows, int dtype, const v
     if (num_experts > kHistMaxExperts) return MOE355_E_SHAPE;
     if (num_tokens > 0 && (!topk_ids || !expert_tokens)) return MOE355_E_ARG;
     return unpermute_impl(rows, dtype, nullptr, probs, num_tokens, top_k, hidden, num_tokens * top_k, residual, out,
-                          topk_ids, num_experts, expert_tokens, stream);
+                          topk_ids, num_experts, expert_tokens, nullptr, nullptr, stream);
 }
 
 extern "C" int moe355_abi_version(void) { return MOE355_ABI_VERSION; }

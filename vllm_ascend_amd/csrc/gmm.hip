@@ -16,6 +16,7 @@
 
 #include "gmm_common.h"
 #include "gmm_tiled.h"
+#include "layer_parts.h"
 
 namespace moe355 {
 
@@ -813,11 +814,11 @@ extern "C" size_t moe355_gmm1_swiglu_quant_workspace(int64_t rows, int64_t n, in
     return (((size_t)rows * (size_t)(n / 2) * 4 + 255) & ~(size_t)255) + tiled_ws_max(rows, num_experts);
 }
 
-static int gmm1_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list,
-                     const float* weight_scale, const float* const* scale_list, const float* x_scale,
-                     const int64_t* group_list, int group_list_type, int64_t rows, int64_t k, int64_t n,
-                     int num_experts, float swiglu_limit, int8_t* out, float* out_scale, void* workspace,
-                     size_t workspace_bytes, void* stream, const int32_t* row_src = nullptr)
+int moe355::gmm1_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list,
+                      const float* weight_scale, const float* const* scale_list, const float* x_scale,
+                      const int64_t* group_list, int group_list_type, int64_t rows, int64_t k, int64_t n,
+                      int num_experts, float swiglu_limit, int8_t* out, float* out_scale, void* workspace,
+                      size_t workspace_bytes, void* stream, const int32_t* row_src)
 {
     const void* wany = weight_list ? (const void*)weight_list : (const void*)weight_nz;
     int rc = check_gmm(x, wany, group_list, group_list_type, rows, k, n, num_experts);
@@ -894,10 +895,10 @@ extern "C" size_t moe355_gmm2_dequant_workspace(int64_t rows, int64_t n, int64_t
     return tiled_ws_max(rows, num_experts);
 }
 
-static int gmm2_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list, const float* scale,
-                     const float* const* scale_list, const float* per_token_scale, const int64_t* group_list,
-                     int group_list_type, int64_t rows, int64_t k, int64_t n, int num_experts, void* out,
-                     int out_dtype, void* workspace, size_t workspace_bytes, void* stream)
+int moe355::gmm2_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list, const float* scale,
+                      const float* const* scale_list, const float* per_token_scale, const int64_t* group_list,
+                      int group_list_type, int64_t rows, int64_t k, int64_t n, int num_experts, void* out,
+                      int out_dtype, void* workspace, size_t workspace_bytes, void* stream)
 {
     const void* wany = weight_list ? (const void*)weight_list : (const void*)weight_nz;
     int rc = check_gmm(x, wany, group_list, group_list_type, rows, k, n, num_experts);
@@ -953,6 +954,23 @@ extern "C" int moe355_gmm_pairs_supported(int64_t num_tokens, int top_k, int64_t
     return num_tokens > 0 && top_k > 0 && num_tokens * top_k <= kPairMax && n > 0 && k > 0 && n % 64 == 0 && k % 32 == 0;
 }
 
+// Whether a batch whose ids come straight from the gate runs in pair order: at most 1024 (token, slot) pairs that the
+// grouped GEMMs would stream the weights for anyway, and experts that the bit map of the lookup can hold.  A product
+// of a GiB and more has a second kernel family for hot experts on the sorted path (gemm_plan), pair order streams
+// every expert: DeepSeek-V3 shape under Zipf(1.1) routing, 112 / 128 tokens 668 / 742 us in pair order, 625 / 641 us
+// sorted; on uniform routing pair order leads by 1 % there.
+extern "C" int moe355_pair_order(int64_t num_tokens, int top_k, int num_logits, int num_experts, int64_t hidden,
+                                 int64_t intermediate)
+{
+    if (!moe355_gmm_pairs_supported(num_tokens, top_k, 2 * intermediate, hidden) ||
+        !moe355_gmm_pairs_supported(num_tokens, top_k, hidden, intermediate) ||
+        !moe355_gate_quant_supported(num_tokens, top_k, num_logits) || num_experts <= 0 || num_experts > 2048)
+        return 0;
+    const int64_t pairs = num_tokens * top_k;
+    if ((int64_t)num_experts * 2 * intermediate * hidden >= (1ll << 30) && pairs > 768) return 0;
+    return pairs < 1024 || pairs / num_experts < 12;  // where the sorted form streams as well (tiled_bm)
+}
+
 // pair order: how many places the grid gets.  A place per expert lets a workgroup request its first weight tiles
 // before it has seen a single id, which is the fastest form when nearly every expert has pairs -- and makes every
 // idle expert cost the dispatch of its workgroups plus 32 KiB of weights requested for nothing.  A slot per pair
@@ -980,110 +998,31 @@ extern "C" size_t moe355_gmm1_swiglu_quant_pairs_workspace(int64_t num_tokens, i
     return (((size_t)num_tokens * top_k * (size_t)(n / 2) * 4 + 255) & ~(size_t)255);
 }
 
-extern "C" int moe355_gmm1_swiglu_quant_pairs(const int8_t* x, const float* x_scale, const int32_t* topk_ids,
-                                              int64_t num_tokens, int top_k, const int8_t* weight_nz,
-                                              const float* weight_scale, int64_t k, int64_t n, int num_experts,
-                                              float swiglu_limit, int8_t* out, float* out_scale, void* workspace,
-                                              size_t workspace_bytes, void* stream)
+// gate_up GEMM + SwiGLU in pair order: fp32 values to y, and with `out` the re-quantised rows.  The weights are one
+// tensor (w.one) or per-expert tensors (w.list and w.scale_list).
+int moe355::gmm1_pairs_impl(const int8_t* x, const float* x_scale, const int32_t* topk_ids, int64_t num_tokens,
+                            int top_k, const PairWeights& w, int64_t k, int64_t n, int num_experts, float swiglu_limit,
+                            float* y, int8_t* out, float* out_scale, void* stream)
 {
     if (num_tokens < 0 || top_k <= 0 || k <= 0 || n <= 0 || num_experts <= 0) return MOE355_E_ARG;
     if (num_tokens == 0) return MOE355_OK;
     if (!moe355_gmm_pairs_supported(num_tokens, top_k, n, k)) return MOE355_E_SHAPE;
     if ((int64_t)num_experts * (n / 64) >= 0x7fffffffLL) return MOE355_E_SHAPE;
-    if (!x || !x_scale || !topk_ids || !weight_nz || !weight_scale || !out || !out_scale) return MOE355_E_ARG;
-    if (((uintptr_t)x & 15) || ((uintptr_t)weight_nz & 15) || ((uintptr_t)weight_scale & 15) || ((uintptr_t)out & 3))
-        return MOE355_E_SHAPE;
-    if (!workspace || ((uintptr_t)workspace & 255) ||
-        workspace_bytes < moe355_gmm1_swiglu_quant_pairs_workspace(num_tokens, top_k, n))
-        return MOE355_E_WORKSPACE;
+    if (!x || !x_scale || !topk_ids || !w.complete() || !y) return MOE355_E_ARG;
+    if (((uintptr_t)x & 15) || !w.aligned() || ((uintptr_t)y & 15) || ((uintptr_t)out & 3)) return MOE355_E_SHAPE;
     hipStream_t st = (hipStream_t)stream;
     const int64_t rows = num_tokens * top_k;
-    const int I = (int)(n / 2);
     GmmArgs a = {};
     a.x = x;
-    a.w = weight_nz;
+    a.w = w.one;
+    a.ch_scale = w.scale;
+    a.w_list = w.list;
+    a.s_list = w.scale_list;
     a.R = rows;
     a.K = (int)k;
     a.N = (int)n;
     a.E = num_experts;
     a.row_scale = x_scale;
-    a.ch_scale = weight_scale;
-    a.limit = swiglu_limit;
-    a.y = (float*)workspace;
-    a.pair_ids = topk_ids;
-    a.pair_k = top_k;
-    a.pair_gather = 1;
-    hipEvent_t ev0, ev1;
-    take_profile_events(ev0, ev1);
-    const int64_t units = (int64_t)pair_places(a) * (n / 64);
-    launch_gemm(gmm_stream_kernel<EPI_SWIGLU, 4, 4, 3, false, true, true>, dim3((unsigned)units), st, a, ev0, ev1);
-    launch_swiglu_requant(a.y, nullptr, 0, num_experts, rows, I, out, out_scale, st);
-    return launch_status();
-}
-
-extern "C" int moe355_gmm2_dequant_pairs(const int8_t* x, const int8_t* weight_nz, const float* scale,
-                                         const float* per_token_scale, const int32_t* topk_ids, int64_t num_tokens,
-                                         int top_k, int64_t k, int64_t n, int num_experts, void* out, int out_dtype,
-                                         void* stream)
-{
-    if (num_tokens < 0 || top_k <= 0 || k <= 0 || n <= 0 || num_experts <= 0) return MOE355_E_ARG;
-    if (out_dtype != MOE355_DT_BF16 && out_dtype != MOE355_DT_F16) return MOE355_E_UNSUPPORTED;
-    if (num_tokens == 0) return MOE355_OK;
-    if (!moe355_gmm_pairs_supported(num_tokens, top_k, n, k)) return MOE355_E_SHAPE;
-    if ((int64_t)num_experts * (n / 64) >= 0x7fffffffLL) return MOE355_E_SHAPE;
-    if (!x || !weight_nz || !scale || !per_token_scale || !topk_ids || !out) return MOE355_E_ARG;
-    if (((uintptr_t)x & 15) || ((uintptr_t)weight_nz & 15) || ((uintptr_t)scale & 15) || ((uintptr_t)out & 15))
-        return MOE355_E_SHAPE;
-    hipStream_t st = (hipStream_t)stream;
-    GmmArgs a = {};
-    a.x = x;
-    a.w = weight_nz;
-    a.R = num_tokens * top_k;
-    a.K = (int)k;
-    a.N = (int)n;
-    a.E = num_experts;
-    a.row_scale = per_token_scale;
-    a.ch_scale = scale;
-    a.out = (uint16_t*)out;
-    a.out_f16 = out_dtype == MOE355_DT_F16;
-    a.pair_ids = topk_ids;
-    a.pair_k = top_k;
-    a.pair_gather = 0;
-    hipEvent_t ev0, ev1;
-    take_profile_events(ev0, ev1);
-    const int64_t units = (int64_t)pair_places(a) * (n / 64);
-    // as the sorted form chooses: a wavefront per unit when there are enough units and K is short, and the units
-    // of an expert come in fours (a workgroup collects the pairs of one expert)
-    if (units >= 2048 && k < 2048 && (n / 64) % 4 == 0)
-        launch_gemm(gmm_stream_kernel<EPI_DEQUANT, 1, 4, 2, false, true, true>, dim3((unsigned)((units + 3) / 4)), st, a,
-                    ev0, ev1);
-    else
-        launch_gemm(gmm_stream_kernel<EPI_DEQUANT, 4, 4, 3, false, true, true>, dim3((unsigned)units), st, a, ev0, ev1);
-    return launch_status();
-}
-
-// gate_up GEMM + SwiGLU in pair order, the fp32 values left as they are (the down GEMM below re-quantises them)
-extern "C" int moe355_gmm1_swiglu_pairs(const int8_t* x, const float* x_scale, const int32_t* topk_ids,
-                                        int64_t num_tokens, int top_k, const int8_t* weight_nz,
-                                        const float* weight_scale, int64_t k, int64_t n, int num_experts,
-                                        float swiglu_limit, float* y, void* stream)
-{
-    if (num_tokens < 0 || top_k <= 0 || k <= 0 || n <= 0 || num_experts <= 0) return MOE355_E_ARG;
-    if (num_tokens == 0) return MOE355_OK;
-    if (!moe355_gmm_pairs_supported(num_tokens, top_k, n, k)) return MOE355_E_SHAPE;
-    if ((int64_t)num_experts * (n / 64) >= 0x7fffffffLL) return MOE355_E_SHAPE;
-    if (!x || !x_scale || !topk_ids || !weight_nz || !weight_scale || !y) return MOE355_E_ARG;
-    if (((uintptr_t)x & 15) || ((uintptr_t)weight_nz & 15) || ((uintptr_t)weight_scale & 15) || ((uintptr_t)y & 15))
-        return MOE355_E_SHAPE;
-    GmmArgs a = {};
-    a.x = x;
-    a.w = weight_nz;
-    a.R = num_tokens * top_k;
-    a.K = (int)k;
-    a.N = (int)n;
-    a.E = num_experts;
-    a.row_scale = x_scale;
-    a.ch_scale = weight_scale;
     a.limit = swiglu_limit;
     a.y = y;
     a.pair_ids = topk_ids;
@@ -1092,9 +1031,93 @@ extern "C" int moe355_gmm1_swiglu_pairs(const int8_t* x, const float* x_scale, c
     hipEvent_t ev0, ev1;
     take_profile_events(ev0, ev1);
     const int64_t units = (int64_t)pair_places(a) * (n / 64);
-    launch_gemm(gmm_stream_kernel<EPI_SWIGLU, 4, 4, 3, false, true, true>, dim3((unsigned)units), (hipStream_t)stream, a,
-                ev0, ev1);
+    launch_gemm(gmm_stream_kernel<EPI_SWIGLU, 4, 4, 3, false, true, true>, dim3((unsigned)units), st, a, ev0, ev1);
+    if (out) launch_swiglu_requant(y, nullptr, 0, num_experts, rows, (int)(n / 2), out, out_scale, st);
     return launch_status();
+}
+
+// down GEMM + dequant in pair order on re-quantised rows (x and per_token_scale), or on the fp32 SwiGLU values of the
+// gate_up GEMM (y), which the workgroups then re-quantise themselves
+int moe355::gmm2_pairs_impl(const int8_t* x, const float* per_token_scale, const float* y, const PairWeights& w,
+                            const int32_t* topk_ids, int64_t num_tokens, int top_k, int64_t k, int64_t n,
+                            int num_experts, void* out, int out_dtype, void* stream)
+{
+    if (num_tokens < 0 || top_k <= 0 || k <= 0 || n <= 0 || num_experts <= 0) return MOE355_E_ARG;
+    if (out_dtype != MOE355_DT_BF16 && out_dtype != MOE355_DT_F16) return MOE355_E_UNSUPPORTED;
+    if (num_tokens == 0) return MOE355_OK;
+    if (!moe355_gmm_pairs_supported(num_tokens, top_k, n, k)) return MOE355_E_SHAPE;
+    if (y && !moe355_gmm2_requant_pairs_supported(num_tokens, top_k, n, k, num_experts)) return MOE355_E_SHAPE;
+    if ((int64_t)num_experts * (n / 64) >= 0x7fffffffLL) return MOE355_E_SHAPE;
+    if (!w.complete() || !topk_ids || !out || (!y && (!x || !per_token_scale))) return MOE355_E_ARG;
+    if (((uintptr_t)x & 15) || ((uintptr_t)y & 15) || !w.aligned() || ((uintptr_t)out & 15)) return MOE355_E_SHAPE;
+    hipStream_t st = (hipStream_t)stream;
+    GmmArgs a = {};
+    a.x = x;
+    a.y_in = y;
+    a.w = w.one;
+    a.ch_scale = w.scale;
+    a.w_list = w.list;
+    a.s_list = w.scale_list;
+    a.R = num_tokens * top_k;
+    a.K = (int)k;
+    a.N = (int)n;
+    a.E = num_experts;
+    a.row_scale = per_token_scale;
+    a.out = (uint16_t*)out;
+    a.out_f16 = out_dtype == MOE355_DT_F16;
+    a.pair_ids = topk_ids;
+    a.pair_k = top_k;
+    a.pair_gather = 0;
+    hipEvent_t ev0, ev1;
+    take_profile_events(ev0, ev1);
+    const int64_t units = (int64_t)pair_places(a) * (n / 64);
+    const dim3 by_four((unsigned)((units + 3) / 4));
+    if (y) {
+        const unsigned lds = (unsigned)(32 * (k + 16));
+        auto kernel = gmm_stream_kernel<EPI_DEQUANT, 1, 4, 2, false, true, true, true>;
+        if (ev0 || ev1) hipExtLaunchKernelGGL(kernel, by_four, dim3(256), lds, st, ev0, ev1, 0, a);
+        else hipLaunchKernelGGL(kernel, by_four, dim3(256), lds, st, a);
+    } else if (units >= 2048 && k < 2048 && (n / 64) % 4 == 0) {
+        // as the sorted form chooses: a wavefront per unit when there are enough units and K is short, and the units
+        // of an expert come in fours (a workgroup collects the pairs of one expert)
+        launch_gemm(gmm_stream_kernel<EPI_DEQUANT, 1, 4, 2, false, true, true>, by_four, st, a, ev0, ev1);
+    } else {
+        launch_gemm(gmm_stream_kernel<EPI_DEQUANT, 4, 4, 3, false, true, true>, dim3((unsigned)units), st, a, ev0, ev1);
+    }
+    return launch_status();
+}
+
+extern "C" int moe355_gmm1_swiglu_quant_pairs(const int8_t* x, const float* x_scale, const int32_t* topk_ids,
+                                              int64_t num_tokens, int top_k, const int8_t* weight_nz,
+                                              const float* weight_scale, int64_t k, int64_t n, int num_experts,
+                                              float swiglu_limit, int8_t* out, float* out_scale, void* workspace,
+                                              size_t workspace_bytes, void* stream)
+{
+    if (num_tokens > 0 && (!out || !out_scale)) return MOE355_E_ARG;
+    if (num_tokens > 0 && (!workspace || ((uintptr_t)workspace & 255) ||
+                           workspace_bytes < moe355_gmm1_swiglu_quant_pairs_workspace(num_tokens, top_k, n)))
+        return MOE355_E_WORKSPACE;
+    return gmm1_pairs_impl(x, x_scale, topk_ids, num_tokens, top_k, PairWeights{weight_nz, weight_scale}, k, n,
+                           num_experts, swiglu_limit, (float*)workspace, out, out_scale, stream);
+}
+
+extern "C" int moe355_gmm2_dequant_pairs(const int8_t* x, const int8_t* weight_nz, const float* scale,
+                                         const float* per_token_scale, const int32_t* topk_ids, int64_t num_tokens,
+                                         int top_k, int64_t k, int64_t n, int num_experts, void* out, int out_dtype,
+                                         void* stream)
+{
+    return gmm2_pairs_impl(x, per_token_scale, nullptr, PairWeights{weight_nz, scale}, topk_ids, num_tokens, top_k, k,
+                           n, num_experts, out, out_dtype, stream);
+}
+
+// gate_up GEMM + SwiGLU in pair order, the fp32 values left as they are (the down GEMM below re-quantises them)
+extern "C" int moe355_gmm1_swiglu_pairs(const int8_t* x, const float* x_scale, const int32_t* topk_ids,
+                                        int64_t num_tokens, int top_k, const int8_t* weight_nz,
+                                        const float* weight_scale, int64_t k, int64_t n, int num_experts,
+                                        float swiglu_limit, float* y, void* stream)
+{
+    return gmm1_pairs_impl(x, x_scale, topk_ids, num_tokens, top_k, PairWeights{weight_nz, weight_scale}, k, n,
+                           num_experts, swiglu_limit, y, nullptr, nullptr, stream);
 }
 
 // the form of the down GEMM that re-quantises: a wavefront per unit (many units, a short K) and 32 rows of K + 16
@@ -1114,33 +1137,7 @@ extern "C" int moe355_gmm2_requant_dequant_pairs(const float* y, const int8_t* w
                                                  const int32_t* topk_ids, int64_t num_tokens, int top_k, int64_t k,
                                                  int64_t n, int num_experts, void* out, int out_dtype, void* stream)
 {
-    if (num_tokens < 0 || top_k <= 0 || k <= 0 || n <= 0 || num_experts <= 0) return MOE355_E_ARG;
-    if (out_dtype != MOE355_DT_BF16 && out_dtype != MOE355_DT_F16) return MOE355_E_UNSUPPORTED;
-    if (num_tokens == 0) return MOE355_OK;
-    if (!moe355_gmm2_requant_pairs_supported(num_tokens, top_k, n, k, num_experts)) return MOE355_E_SHAPE;
-    if (!y || !weight_nz || !scale || !topk_ids || !out) return MOE355_E_ARG;
-    if (((uintptr_t)y & 15) || ((uintptr_t)weight_nz & 15) || ((uintptr_t)scale & 15) || ((uintptr_t)out & 15))
-        return MOE355_E_SHAPE;
-    GmmArgs a = {};
-    a.y_in = y;
-    a.w = weight_nz;
-    a.R = num_tokens * top_k;
-    a.K = (int)k;
-    a.N = (int)n;
-    a.E = num_experts;
-    a.ch_scale = scale;
-    a.out = (uint16_t*)out;
-    a.out_f16 = out_dtype == MOE355_DT_F16;
-    a.pair_ids = topk_ids;
-    a.pair_k = top_k;
-    a.pair_gather = 0;
-    hipEvent_t ev0, ev1;
-    take_profile_events(ev0, ev1);
-    const int64_t units = (int64_t)pair_places(a) * (n / 64);
-    const unsigned lds = (unsigned)(32 * (k + 16));
-    auto kernel = gmm_stream_kernel<EPI_DEQUANT, 1, 4, 2, false, true, true, true>;
-    const dim3 grid((unsigned)((units + 3) / 4));
-    if (ev0 || ev1) hipExtLaunchKernelGGL(kernel, grid, dim3(256), lds, (hipStream_t)stream, ev0, ev1, 0, a);
-    else hipLaunchKernelGGL(kernel, grid, dim3(256), lds, (hipStream_t)stream, a);
-    return launch_status();
+    if (num_tokens > 0 && !y) return MOE355_E_ARG;
+    return gmm2_pairs_impl(nullptr, nullptr, y, PairWeights{weight_nz, scale}, topk_ids, num_tokens, top_k, k, n,
+                           num_experts, out, out_dtype, stream);
 }

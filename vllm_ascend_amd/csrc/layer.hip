@@ -1,0 +1,299 @@
+// The whole layer in one call.  Host code only: it lays out one scratch buffer and enqueues the operators of the
+// layer, so that a decode step costs the launches themselves (2 to 3 us each) instead of an interpreter round trip,
+// a handful of allocations and three event records around every one of them: a recorded event alone is a 5.6 us gap
+// on the GPU, three of them per layer.
+#include <mutex>
+#include <vector>
+
+#include "layer_parts.h"
+
+using namespace moe355;
+
+namespace {
+
+struct Arena {
+    char* base;
+    size_t used = 0;
+    template <typename T>
+    T* take(size_t bytes)
+    {
+        T* p = (T*)(base + used);
+        used += (bytes + 255) & ~(size_t)255;
+        return p;
+    }
+};
+
+enum { W_INT8 = 0, W_INT8_LIST = 1, W_INT4 = 2 };
+
+// the buffers of one call, all in the caller's workspace
+struct Buffers {
+    void* topk_weights;
+    int32_t* topk_ids;
+    int8_t* xq;
+    float* x_scale;
+    int64_t* expert_tokens;
+    int64_t* one_group;
+    int32_t* dst;
+    int32_t* row_token;
+    void* map_ws;
+    float* logits;
+    void* gate_ws;
+    void* mlp_ws;  // fp32 SwiGLU values, behind them the scratch of the gate_up GEMM
+    int8_t* q1;
+    float* q1_scale;
+    void* o;
+    void* gmm2_ws;
+    int32_t* sh_acc;
+    void* sh_ws;
+    int8_t* sh_q;
+    float* sh_q_scale;
+    void* sh_ws2;
+    void* sh_out;
+    size_t map_bytes, gate_bytes, mlp_bytes, gmm2_bytes, sh_bytes, sh2_bytes, total;
+};
+
+struct Forms {
+    bool pairs;    // pair order
+    bool requant;  // ... with the re-quantisation inside the down GEMM
+    bool small;    // sorted, gating + sort + quantisation in one launch
+};
+
+Forms forms_of(const moe355_layer& l, int64_t T)
+{
+    Forms f = {};
+    f.pairs = l.weights != W_INT4 && l.pair_order &&
+              moe355_pair_order(T, l.top_k, l.num_experts, l.num_experts, l.hidden, l.intermediate);
+    f.requant = f.pairs && moe355_gmm2_requant_pairs_supported(T, l.top_k, l.hidden, l.intermediate, l.num_experts);
+    f.small = !f.pairs && l.sync_counter && moe355_route_quant_small_supported(T, l.top_k, l.num_experts);
+    return f;
+}
+
+Buffers lay_out(const moe355_layer& l, const Forms& f, int64_t T, void* base)
+{
+    Arena a = {(char*)base};
+    Buffers b = {};
+    const int64_t R = T * l.top_k, H = l.hidden, I = l.intermediate;
+    const int E = l.num_experts;
+    b.topk_weights = a.take<void>((size_t)R * 2);
+    b.topk_ids = a.take<int32_t>((size_t)R * 4);
+    b.xq = a.take<int8_t>((size_t)T * H);
+    b.x_scale = a.take<float>((size_t)T * 4);
+    b.expert_tokens = a.take<int64_t>((size_t)E * 8);
+    b.one_group = a.take<int64_t>(8);
+    if (l.gate_weight) {
+        b.logits = a.take<float>((size_t)T * E * 4);
+        b.gate_bytes = moe355_router_gate_workspace(T, (int)H, E);
+        b.gate_ws = b.gate_bytes ? a.take<void>(b.gate_bytes) : nullptr;
+    }
+    b.q1 = a.take<int8_t>((size_t)R * I);
+    b.q1_scale = a.take<float>((size_t)R * 4);
+    if (f.pairs) {
+        b.mlp_bytes = moe355_gmm1_swiglu_quant_pairs_workspace(T, l.top_k, 2 * I);
+        b.mlp_ws = a.take<void>(b.mlp_bytes);
+        b.o = a.take<void>((size_t)R * H * 2);
+    } else {
+        b.dst = a.take<int32_t>((size_t)R * 4);
+        b.row_token = a.take<int32_t>((size_t)R * 4);
+        b.map_bytes = moe355_init_routing_workspace(T, l.top_k, E);
+        b.map_ws = a.take<void>(b.map_bytes);
+        // the down GEMM writes its rows where the SwiGLU values were: those are dead once re-quantised
+        const size_t y = ((size_t)R * I * 4 + 255) & ~(size_t)255, o = (size_t)R * H * 2;
+        b.mlp_bytes = l.weights == W_INT4 ? y : moe355_gmm1_swiglu_quant_workspace(R, 2 * I, H, E);
+        b.mlp_ws = a.take<void>(b.mlp_bytes > o ? b.mlp_bytes : o);
+        b.o = b.mlp_ws;
+        b.gmm2_bytes = l.weights == W_INT4 ? 0 : moe355_gmm2_dequant_workspace(R, H, I, E);
+        b.gmm2_ws = a.take<void>(b.gmm2_bytes);
+    }
+    if (l.shared) {
+        const int64_t S = l.shared_intermediate;
+        b.sh_acc = a.take<int32_t>((size_t)T * 2 * S * 4);
+        b.sh_bytes = moe355_gmm_i32_workspace(T, 2 * S, H, 1);
+        b.sh_ws = a.take<void>(b.sh_bytes);
+        b.sh_q = a.take<int8_t>((size_t)T * S);
+        b.sh_q_scale = a.take<float>((size_t)T * 4);
+        b.sh2_bytes = moe355_gmm2_dequant_workspace(T, H, S, 1);
+        b.sh_ws2 = a.take<void>(b.sh2_bytes);
+        b.sh_out = a.take<void>((size_t)T * H * 2);
+    }
+    b.total = a.used;
+    return b;
+}
+
+int check_layer(const moe355_layer* l)
+{
+    if (!l || l->hidden <= 0 || l->intermediate <= 0 || l->num_experts <= 0 || l->top_k <= 0) return MOE355_E_ARG;
+    if (l->weights < W_INT8 || l->weights > W_INT4 || l->shared < 0 || l->shared > 2) return MOE355_E_ARG;
+    if (!l->w13 || !l->s13 || !l->w2 || !l->s2) return MOE355_E_ARG;
+    if (l->shared && l->shared_intermediate <= 0) return MOE355_E_ARG;
+    if (l->shared && (!l->shared_w13 || !l->shared_s13 || !l->shared_w2 || !l->shared_s2)) return MOE355_E_ARG;
+    if (l->x_dtype != MOE355_DT_BF16 && l->x_dtype != MOE355_DT_F16) return MOE355_E_UNSUPPORTED;
+    return MOE355_OK;
+}
+
+// Events that order the side stream's work against the caller's stream.  A wait takes the state of the event at the
+// time of the call, so a pair is free again once its waits are enqueued: it goes back to the list then, and the list
+// is as long as there were calls at the same time.  They live as long as the process (there is no safe moment to
+// destroy them after the runtime has gone).
+struct ForkJoin {
+    hipEvent_t fork = nullptr, join = nullptr;
+    int dev = -1;
+};
+constexpr int kDevices = 64;
+std::mutex g_events_mutex;
+std::vector<ForkJoin> g_events[kDevices];
+
+struct ForkJoinLease {
+    ForkJoin fj;
+    bool take()
+    {
+        int dev = -1;
+        if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kDevices) return false;
+        {
+            std::lock_guard<std::mutex> lock(g_events_mutex);
+            if (!g_events[dev].empty()) {
+                fj = g_events[dev].back();
+                g_events[dev].pop_back();
+                return true;
+            }
+        }
+        if (hipEventCreateWithFlags(&fj.fork, hipEventDisableTiming) != hipSuccess) return false;
+        if (hipEventCreateWithFlags(&fj.join, hipEventDisableTiming) != hipSuccess) {
+            (void)hipEventDestroy(fj.fork);
+            return false;
+        }
+        fj.dev = dev;
+        return true;
+    }
+    ~ForkJoinLease()
+    {
+        if (fj.dev < 0) return;
+        std::lock_guard<std::mutex> lock(g_events_mutex);
+        g_events[fj.dev].push_back(fj);
+    }
+};
+
+// dense W8A8 MLP over all tokens, on the rows the routed experts quantised
+int shared_expert(const moe355_layer& l, const Buffers& b, int64_t T, void* st)
+{
+    const int64_t H = l.hidden, I = l.shared_intermediate;
+    int rc = moe355_gmm_i32(b.xq, l.shared_w13, b.one_group, MOE355_GL_CUMSUM, T, H, 2 * I, 1, b.sh_acc, b.sh_ws,
+                            b.sh_bytes, st);
+    if (rc != MOE355_OK) return rc;
+    rc = moe355_dequant_swiglu_quant_grouped(b.sh_acc, l.shared_s13, b.x_scale, nullptr, 0, nullptr, 1, T, 2 * I, 1, 1,
+                                             l.shared_limit, l.shared_alpha, l.shared_beta, 1, nullptr, 0, nullptr,
+                                             b.sh_q, b.sh_q_scale, st);
+    if (rc != MOE355_OK) return rc;
+    return moe355_gmm2_dequant(b.sh_q, l.shared_w2, l.shared_s2, b.sh_q_scale, b.one_group, MOE355_GL_CUMSUM, T, I, H, 1,
+                               b.sh_out, l.x_dtype, b.sh_ws2, b.sh2_bytes, st);
+}
+
+int routed_pairs(const moe355_layer& l, const Forms& f, const Buffers& b, int64_t T, void* st)
+{
+    const int64_t H = l.hidden, I = l.intermediate;
+    PairWeights w13 = {}, w2 = {};
+    if (l.weights == W_INT8_LIST) {
+        w13.list = (const int8_t* const*)l.w13;
+        w13.scale_list = (const float* const*)l.s13;
+        w2.list = (const int8_t* const*)l.w2;
+        w2.scale_list = (const float* const*)l.s2;
+    } else {
+        w13.one = (const int8_t*)l.w13;
+        w13.scale = (const float*)l.s13;
+        w2.one = (const int8_t*)l.w2;
+        w2.scale = (const float*)l.s2;
+    }
+    float* y = (float*)b.mlp_ws;
+    int rc = gmm1_pairs_impl(b.xq, b.x_scale, b.topk_ids, T, l.top_k, w13, H, 2 * I, l.num_experts, l.swiglu_limit, y,
+                             f.requant ? nullptr : b.q1, b.q1_scale, st);
+    if (rc != MOE355_OK) return rc;
+    return gmm2_pairs_impl(b.q1, b.q1_scale, f.requant ? y : nullptr, w2, b.topk_ids, T, l.top_k, I, H, l.num_experts,
+                           b.o, l.x_dtype, st);
+}
+
+int routed_sorted(const moe355_layer& l, const Buffers& b, int64_t T, void* st)
+{
+    const int64_t H = l.hidden, I = l.intermediate, R = T * l.top_k;
+    const int E = l.num_experts;
+    int rc;
+    if (l.weights == W_INT4) {
+        rc = moe355_gmm1_swiglu_quant_w4_gather(b.xq, b.x_scale, b.row_token, (const uint8_t*)l.w13,
+                                                (const float*)l.s13, l.group13, nullptr, b.expert_tokens,
+                                                MOE355_GL_COUNT, R, H, 2 * I, E, l.swiglu_limit, b.q1, b.q1_scale,
+                                                b.mlp_ws, b.mlp_bytes, st);
+        if (rc != MOE355_OK) return rc;
+        return moe355_gmm2_dequant_w4(b.q1, (const uint8_t*)l.w2, (const float*)l.s2, l.group2, nullptr, b.q1_scale,
+                                      b.expert_tokens, MOE355_GL_COUNT, R, I, H, E, b.o, l.x_dtype, st);
+    }
+    const bool list = l.weights == W_INT8_LIST;
+    rc = gmm1_impl(b.xq, list ? nullptr : (const int8_t*)l.w13, list ? (const int8_t* const*)l.w13 : nullptr,
+                   list ? nullptr : (const float*)l.s13, list ? (const float* const*)l.s13 : nullptr, b.x_scale,
+                   b.expert_tokens, MOE355_GL_COUNT, R, H, 2 * I, E, l.swiglu_limit, b.q1, b.q1_scale, b.mlp_ws,
+                   b.mlp_bytes, st, b.row_token);
+    if (rc != MOE355_OK) return rc;
+    return gmm2_impl(b.q1, list ? nullptr : (const int8_t*)l.w2, list ? (const int8_t* const*)l.w2 : nullptr,
+                     list ? nullptr : (const float*)l.s2, list ? (const float* const*)l.s2 : nullptr, b.q1_scale,
+                     b.expert_tokens, MOE355_GL_COUNT, R, I, H, E, b.o, l.x_dtype, b.gmm2_ws, b.gmm2_bytes, st);
+}
+
+}  // namespace
+
+extern "C" size_t moe355_layer_workspace(const moe355_layer* layer, int64_t num_tokens)
+{
+    if (check_layer(layer) != MOE355_OK || num_tokens <= 0) return 256;
+    return lay_out(*layer, forms_of(*layer, num_tokens), num_tokens, nullptr).total;
+}
+
+extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, const void* logits, int logits_dtype,
+                                    int64_t num_tokens, void* out, void* workspace, size_t workspace_bytes,
+                                    void* stream)
+{
+    int rc = check_layer(layer);
+    if (rc != MOE355_OK) return rc;
+    if (num_tokens < 0) return MOE355_E_ARG;
+    if (num_tokens == 0) return MOE355_OK;
+    const moe355_layer& l = *layer;
+    const int64_t T = num_tokens, R = T * l.top_k;
+    if (!x || !out || (!logits && !l.gate_weight)) return MOE355_E_ARG;
+    if (R >= 0x7fffffffLL) return MOE355_E_SHAPE;
+    const Forms f = forms_of(l, T);
+    const Buffers b = lay_out(l, f, T, workspace);
+    if (!workspace || ((uintptr_t)workspace & 255) || workspace_bytes < b.total) return MOE355_E_WORKSPACE;
+
+    GateCall g = {x, logits, l.bias, l.x_dtype, logits_dtype, T, l.hidden, l.num_experts, l.top_k, l.k_group,
+                  l.group_count, 1, l.renorm, l.norm_type, l.routed_scaling_factor, l.eps};
+    if (l.gate_weight) {
+        rc = moe355_router_gate(x, l.x_dtype, l.gate_weight, l.gate_bias, T, (int)l.hidden, l.num_experts, b.logits,
+                                b.gate_ws, b.gate_bytes, stream);
+        if (rc != MOE355_OK) return rc;
+        g.logits = b.logits;
+        g.logits_dtype = MOE355_DT_F32;
+    }
+    rc = gate_quant_impl(f.small, g, 1, b.topk_weights, b.topk_ids, b.xq, b.x_scale, b.dst, b.row_token,
+                         b.expert_tokens, l.sync_counter, l.shared ? b.one_group : nullptr, stream);
+    if (rc != MOE355_OK) return rc;
+
+    ForkJoinLease lease;
+    bool joined = true;
+    if (l.shared == 2) {
+        hipStream_t side = (hipStream_t)l.shared_stream, main = (hipStream_t)stream;
+        if (!lease.take() || hipEventRecord(lease.fj.fork, main) != hipSuccess ||
+            hipStreamWaitEvent(side, lease.fj.fork, 0) != hipSuccess)
+            return MOE355_E_LAUNCH;
+        rc = shared_expert(l, b, T, side);
+        // joined below even if a launch was refused: the caller frees the scratch in the order of its own stream
+        if (hipEventRecord(lease.fj.join, side) != hipSuccess) return MOE355_E_LAUNCH;
+        joined = false;
+    } else if (l.shared == 1) {
+        rc = shared_expert(l, b, T, stream);
+    }
+    if (rc == MOE355_OK && !f.pairs && !f.small)
+        rc = moe355_route_map(b.topk_ids, T, l.top_k, l.num_experts, 1, b.dst, b.row_token, b.expert_tokens, b.map_ws,
+                              b.map_bytes, stream);
+    if (rc == MOE355_OK) rc = f.pairs ? routed_pairs(l, f, b, T, stream) : routed_sorted(l, b, T, stream);
+    if (!joined && hipStreamWaitEvent((hipStream_t)stream, lease.fj.join, 0) != hipSuccess) return MOE355_E_LAUNCH;
+    if (rc != MOE355_OK) return rc;
+    const void* residual = l.shared ? b.sh_out : nullptr;
+    return unpermute_impl(b.o, l.x_dtype, f.pairs ? nullptr : b.dst, b.topk_weights, T, l.top_k, l.hidden, R, residual,
+                          out, f.pairs ? b.topk_ids : nullptr, l.num_experts, b.expert_tokens, b.expert_tokens, l.load,
+                          stream);
+}

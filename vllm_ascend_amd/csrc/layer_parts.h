@@ -1,0 +1,59 @@
+// Host entries that the layer call (layer.hip) shares with the exported operators: the same launches, with the
+// options that only a whole layer has (per-expert weight tables in pair order, the group list of a dense product
+// written by the routing launch, expert loads added up by the combine).
+#pragma once
+
+#include "moe355_common.h"
+
+namespace moe355 {
+
+// hidden states and logits of a batch, and how the router scores and groups the experts
+struct GateCall {
+    const void* x;       // [T, H] bf16 / fp16
+    const void* logits;  // [T, E]
+    const void* bias;    // [E] in the dtype of the logits, or null
+    int x_dtype, logits_dtype;
+    int64_t num_tokens, hidden;
+    int num_experts, top_k, k_group, group_count, group_select_mode, renorm, norm_type;
+    float routed_scaling_factor, eps;
+};
+
+// sort: the whole of moe355_route_quant_small; otherwise gating and quantisation only (any number of tokens).
+// one_group: receives num_tokens on the device, or null.
+int gate_quant_impl(bool sort, const GateCall& g, int tokens_num_type, void* topk_weights, int32_t* topk_ids,
+                    int8_t* xq, float* x_scale, int32_t* expanded_row_idx, int32_t* row_token, int64_t* expert_tokens,
+                    int32_t* sync_counter, int64_t* one_group, void* stream);
+
+// sorted_indices null: pair order (hist_ids = the ids, counts to hist_out).  load [hist_experts]: the counts of this
+// batch are added to it (from hist_ids, or load_counts where the rows are sorted).
+int unpermute_impl(const void* permuted, int dtype, const int32_t* sorted_indices, const void* probs,
+                   int64_t num_tokens, int top_k, int64_t hidden, int64_t permuted_rows, const void* residual,
+                   void* out, const int32_t* hist_ids, int hist_experts, int64_t* hist_out, const int64_t* load_counts,
+                   int64_t* load, void* stream);
+
+// Weights of a pair-order GEMM: one tiled tensor with its scales, or device tables of per-expert tensors.
+struct PairWeights {
+    const int8_t* one;
+    const float* scale;
+    const int8_t* const* list = nullptr;
+    const float* const* scale_list = nullptr;
+    bool complete() const { return (one && scale) || (list && scale_list); }
+    bool aligned() const { return !((uintptr_t)one & 15) && !((uintptr_t)scale & 15); }
+};
+
+int gmm1_pairs_impl(const int8_t* x, const float* x_scale, const int32_t* topk_ids, int64_t num_tokens, int top_k,
+                    const PairWeights& w, int64_t k, int64_t n, int num_experts, float swiglu_limit, float* y,
+                    int8_t* out, float* out_scale, void* stream);
+int gmm2_pairs_impl(const int8_t* x, const float* per_token_scale, const float* y, const PairWeights& w,
+                    const int32_t* topk_ids, int64_t num_tokens, int top_k, int64_t k, int64_t n, int num_experts,
+                    void* out, int out_dtype, void* stream);
+int gmm1_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list, const float* weight_scale,
+              const float* const* scale_list, const float* x_scale, const int64_t* group_list, int group_list_type,
+              int64_t rows, int64_t k, int64_t n, int num_experts, float swiglu_limit, int8_t* out, float* out_scale,
+              void* workspace, size_t workspace_bytes, void* stream, const int32_t* row_src = nullptr);
+int gmm2_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list, const float* scale,
+              const float* const* scale_list, const float* per_token_scale, const int64_t* group_list,
+              int group_list_type, int64_t rows, int64_t k, int64_t n, int num_experts, void* out, int out_dtype,
+              void* workspace, size_t workspace_bytes, void* stream);
+
+}  // namespace moe355

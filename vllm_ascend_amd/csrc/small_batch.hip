@@ -16,6 +16,7 @@
 #include <type_traits>
 
 #include "gating_body.h"
+#include "layer_parts.h"
 
 namespace moe355 {
 
@@ -41,6 +42,7 @@ struct SmallRouteArgs {
     int32_t* row_token;   // [T * k] token of every expert-sorted row
     int64_t* expert_tokens;  // [E]
     int32_t* arrived;     // one int32, zero between calls
+    int64_t* one_group;   // or null: receives T (the group list of a dense product over all tokens)
 };
 
 // the quantiser of the layer on one row, by the whole workgroup
@@ -100,6 +102,7 @@ __global__ __launch_bounds__(kSmallThreads) void route_quant_small_kernel(SmallR
     }
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int E = a.E, k = a.k, R = a.T * a.k;
+    if (a.one_group && blockIdx.x == 0 && tid == 0) *a.one_group = a.T;
     // ---------------- gating: one row per wavefront
     {
         int row[1] = {(int)blockIdx.x * kSmallWaves + wave};
@@ -207,14 +210,15 @@ extern "C" int moe355_route_quant_small_supported(int64_t num_tokens, int top_k,
            num_experts <= kSmallMaxExperts && top_k <= num_experts;
 }
 
-// sort: the whole of moe355_route_quant_small; otherwise gating and quantisation only (any number of tokens)
-static int gate_quant_impl(bool sort, const void* x, int x_dtype, const void* logits, int logits_dtype,
-                           const void* bias, int64_t num_tokens, int64_t hidden, int num_experts, int k, int k_group,
-                           int group_count, int group_select_mode, int renorm, int norm_type,
-                           float routed_scaling_factor, float eps, int tokens_num_type, void* topk_weights,
-                           int32_t* topk_ids, int8_t* xq, float* x_scale, int32_t* expanded_row_idx,
-                           int32_t* row_token, int64_t* expert_tokens, int32_t* sync_counter, void* stream)
+int moe355::gate_quant_impl(bool sort, const GateCall& g, int tokens_num_type, void* topk_weights, int32_t* topk_ids,
+                            int8_t* xq, float* x_scale, int32_t* expanded_row_idx, int32_t* row_token,
+                            int64_t* expert_tokens, int32_t* sync_counter, int64_t* one_group, void* stream)
 {
+    const void *x = g.x, *logits = g.logits, *bias = g.bias;
+    const int x_dtype = g.x_dtype, logits_dtype = g.logits_dtype, num_experts = g.num_experts, k = g.top_k;
+    const int k_group = g.k_group, group_count = g.group_count, group_select_mode = g.group_select_mode;
+    const int renorm = g.renorm, norm_type = g.norm_type;
+    const int64_t num_tokens = g.num_tokens, hidden = g.hidden;
     if (num_tokens < 0 || hidden <= 0 || num_experts <= 0 || k <= 0) return MOE355_E_ARG;
     if (norm_type != 0 && norm_type != 1) return MOE355_E_ARG;
     if (group_select_mode != 0 && group_select_mode != 1) return MOE355_E_ARG;
@@ -242,8 +246,8 @@ static int gate_quant_impl(bool sort, const void* x, int x_dtype, const void* lo
     a.mode = group_select_mode;
     a.renorm = renorm;
     a.norm_type = norm_type;
-    a.rsf = routed_scaling_factor;
-    a.eps = eps;
+    a.rsf = g.routed_scaling_factor;
+    a.eps = g.eps;
     a.tokens_num_type = tokens_num_type;
     a.topk_weights = topk_weights;
     a.x_dtype = x_dtype;
@@ -254,6 +258,7 @@ static int gate_quant_impl(bool sort, const void* x, int x_dtype, const void* lo
     a.row_token = row_token;
     a.expert_tokens = expert_tokens;
     a.arrived = sort ? sync_counter : nullptr;
+    a.one_group = one_group;
     const int E = num_experts;
     int per = 1;
     while (64 * per < E) per *= 2;
@@ -290,10 +295,10 @@ extern "C" int moe355_route_quant_small(const void* x, int x_dtype, const void* 
                                         int32_t* expanded_row_idx, int32_t* row_token, int64_t* expert_tokens,
                                         int32_t* sync_counter, void* stream)
 {
-    return gate_quant_impl(true, x, x_dtype, logits, logits_dtype, bias, num_tokens, hidden, num_experts, k, k_group,
-                           group_count, group_select_mode, renorm, norm_type, routed_scaling_factor, eps,
-                           tokens_num_type, topk_weights, topk_ids, xq, x_scale, expanded_row_idx, row_token,
-                           expert_tokens, sync_counter, stream);
+    const GateCall g = {x, logits, bias, x_dtype, logits_dtype, num_tokens, hidden, num_experts, k, k_group, group_count,
+                        group_select_mode, renorm, norm_type, routed_scaling_factor, eps};
+    return gate_quant_impl(true, g, tokens_num_type, topk_weights, topk_ids, xq, x_scale, expanded_row_idx, row_token,
+                           expert_tokens, sync_counter, nullptr, stream);
 }
 
 extern "C" int moe355_gate_quant(const void* x, int x_dtype, const void* logits, int logits_dtype, const void* bias,
@@ -302,7 +307,8 @@ extern "C" int moe355_gate_quant(const void* x, int x_dtype, const void* logits,
                                  float routed_scaling_factor, float eps, void* topk_weights, int32_t* topk_ids,
                                  int8_t* xq, float* x_scale, void* stream)
 {
-    return gate_quant_impl(false, x, x_dtype, logits, logits_dtype, bias, num_tokens, hidden, num_experts, k, k_group,
-                           group_count, group_select_mode, renorm, norm_type, routed_scaling_factor, eps, 1,
-                           topk_weights, topk_ids, xq, x_scale, nullptr, nullptr, nullptr, nullptr, stream);
+    const GateCall g = {x, logits, bias, x_dtype, logits_dtype, num_tokens, hidden, num_experts, k, k_group, group_count,
+                        group_select_mode, renorm, norm_type, routed_scaling_factor, eps};
+    return gate_quant_impl(false, g, 1, topk_weights, topk_ids, xq, x_scale, nullptr, nullptr, nullptr, nullptr, nullptr,
+                           stream);
 }

@@ -10,6 +10,7 @@ import torch
 from ..quantization.base import AscendMoEScheme
 from ..quantization.checkpoint import moe_weight_loader
 from .contracts import FusedExpertsResult, FusedMoEConfig
+from .layer_call import layer_call
 from .moe_comm_method import setup_moe_comm_method
 from .router import AscendFusedTopKRouter
 
@@ -135,6 +136,11 @@ class AscendRoutedExperts(torch.nn.Module):
         return self.quant_method.apply(self, hidden_states, topk_weights, topk_ids, self.shared_experts, None)
 
     def forward(self, hidden_states: torch.Tensor, router_logits: torch.Tensor | None = None) -> torch.Tensor:
+        # the whole layer in one native call where it can take this one; nobody reads the events and intermediate
+        # tensors of a FusedExpertsResult here
+        out = layer_call(self, hidden_states, router_logits)
+        if out is not None:
+            return out
         if router_logits is None:
             if self.gate is None:
                 raise ValueError("router_logits is required: this layer was built without an internal gate")

@@ -532,6 +532,10 @@ def gmm_pairs_supported(num_tokens: int, top_k: int, n: int, k: int) -> bool:
     return bool(_lib.load().moe355_gmm_pairs_supported(num_tokens, top_k, n, k))
 
 
+def pair_order(num_tokens: int, top_k: int, num_logits: int, num_experts: int, hidden: int, intermediate: int) -> bool:
+    return bool(_lib.load().moe355_pair_order(num_tokens, top_k, num_logits, num_experts, hidden, intermediate))
+
+
 def _check_pair_operands(name, x, x_rows, k, scale_rows, row_scale, topk_ids, weight_nz, n, ch_scale):
     for t, what in ((x, "x"), (row_scale, "row scale"), (topk_ids, "topk_ids"), (weight_nz, "weight"),
                     (ch_scale, "scale")):

@@ -206,26 +206,14 @@ class AscendW8A8DynamicFusedMoEMethod(AscendMoEScheme):
     # ------------------------------------------------------------------ decode batches: no sort at all
     @staticmethod
     def _pair_order(layer, x: torch.Tensor, router_logits: torch.Tensor, router) -> bool:
-        """At most 1024 (token, slot) pairs that the grouped GEMMs would stream the weights for anyway, ids
-        straight from the gate (always in range)."""
+        """The library's rule for batches whose ids come straight from the gate (always in range)."""
         from .. import kernels
 
         if not getattr(layer, "use_pair_order", True):
             return False
-        T, k, E = x.shape[0], router.top_k, router_logits.shape[1]
-        w13, w2 = layer.w13_weight, layer.w2_weight
-        if not (kernels.gmm_pairs_supported(T, k, w13.shape[2], w13.shape[1])
-                and kernels.gmm_pairs_supported(T, k, w2.shape[2], w2.shape[1])):
-            return False
-        experts = layer.w13_weight.shape[0]  # physical experts (more than E with redundant copies behind log2phy)
-        if not kernels.gate_quant_supported(T, k, E) or experts > 2048:
-            return False
-        if experts * w13.shape[1] * w13.shape[2] >= 1 << 30 and T * k > 768:
-            # A product of a GiB and more has a second kernel family for hot experts on the sorted path (csrc/gmm.hip:
-            # gemm_plan), pair order streams every expert: DeepSeek-V3 shape under Zipf(1.1) routing, 112 / 128 tokens
-            # 668 / 742 us in pair order, 625 / 641 us sorted; on uniform routing pair order leads by 1 % there.
-            return False
-        return T * k < 1024 or (T * k) // experts < 12  # where the sorted form streams as well (csrc/gmm.hip: tiled_bm)
+        w13 = layer.w13_weight  # [physical experts, H, 2I]; more experts than logits with redundant copies (log2phy)
+        return kernels.pair_order(x.shape[0], router.top_k, router_logits.shape[1], w13.shape[0], w13.shape[1],
+                                  w13.shape[2] // 2)
 
     def _experts_in_pair_order(self, layer, x, router_logits, router, shared_experts, shared_experts_input,
                                before_dispatch_evt):
