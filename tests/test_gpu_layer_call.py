@@ -19,9 +19,9 @@ def _pair(name, tokens, **kw):
     return cfg, build_layer(cfg, d, DEV, **kw), d["x"].to(DEV), d["logits"].to(DEV)
 
 
-# one token; the borders of the pair-order forms (three pairs per expert, 1024 pairs) and of the one-launch index maps
-# (4096 pairs); a batch with a ragged end on the sorted path
-@pytest.mark.parametrize("tokens", [1, 24, 25, 127, 128, 129, 512, 513, 1031])
+# one token; the borders of the form for a few tokens (16 pairs, 64 with a shared expert), of pair order (three pairs per expert, 1024
+# pairs) and of the one-launch index maps (4096 pairs); a batch with a ragged end on the sorted path
+@pytest.mark.parametrize("tokens", [1, 4, 5, 8, 9, 24, 25, 127, 128, 129, 512, 513, 1031])
 @pytest.mark.parametrize("name", ["c2_small", "c4_small", "c5_small"])
 def test_one_call_equals_the_operators(name, tokens):
     cfg, layer, x, logits = _pair(name, tokens, shared=CONFIGS[name].shared)
@@ -30,7 +30,7 @@ def test_one_call_equals_the_operators(name, tokens):
     assert torch.equal(got, layer.forward_impl(x, logits).routed_out)
 
 
-@pytest.mark.parametrize("tokens", [3, 40, 300])
+@pytest.mark.parametrize("tokens", [1, 8, 40, 300])
 @pytest.mark.parametrize("overlap", [False, True])
 def test_shared_expert_in_the_call(tokens, overlap):
     cfg, layer, x, logits = _pair("c4_small", tokens, shared=True, overlap=overlap)
@@ -39,7 +39,7 @@ def test_shared_expert_in_the_call(tokens, overlap):
         assert torch.equal(layer(x, logits), want)
 
 
-@pytest.mark.parametrize("tokens", [2, 60, 300])
+@pytest.mark.parametrize("tokens", [2, 4, 60, 300])
 def test_weight_lists_and_expert_loads(tokens):
     cfg, layer, x, logits = _pair("c7_small", tokens, dynamic_eplb=True, collect_expert_load=True)
     res = layer.forward_impl(x, logits)
@@ -48,6 +48,25 @@ def test_weight_lists_and_expert_loads(tokens):
     assert torch.equal(layer(x, logits), res.routed_out)
     assert torch.equal(layer.moe_load, 2 * res.expert_tokens)
     layer.w13_weight_list[1] = layer.w13_weight_list[0].clone()  # one expert swapped: the next call sees it
+    assert torch.equal(layer(x, logits), layer.forward_impl(x, logits).routed_out)
+
+
+# the full decode shapes: long K, shared expert with its own arithmetic, rows quantised in place (1 token) or by a launch
+@pytest.mark.parametrize("name, tokens", [("c2_qwen3_decode", 1), ("c2_qwen3_decode", 2), ("c6_dsv3_decode", 1),
+                                          ("c6_dsv3_decode", 4)])
+def test_a_few_tokens_at_full_size(name, tokens):
+    cfg = dataclasses.replace(CONFIGS[name], T=tokens)
+    d = make_layer(cfg, seed=tokens, gen_device=DEV)
+    layer = build_layer(cfg, d, DEV, shared=cfg.shared)
+    x = d["x"]
+    for shared_args in ((0.0, 1.0, 0.0), (1.5, 1.3, 0.25)):
+        if layer.shared_experts is not None:
+            layer.shared_experts.swiglu_limit, layer.shared_experts.swiglu_alpha, layer.shared_experts.swiglu_beta = shared_args
+        assert torch.equal(layer(x, d["logits"]), layer.forward_impl(x, d["logits"]).routed_out)
+    # every token on the same experts, and a row of zeros
+    logits = d["logits"][:1].expand(tokens, -1).contiguous()
+    x = x.clone()
+    x[-1] = 0
     assert torch.equal(layer(x, logits), layer.forward_impl(x, logits).routed_out)
 
 

@@ -33,6 +33,7 @@ struct Buffers {
     float* x_scale;
     int64_t* expert_tokens;
     int64_t* one_group;
+    float* ymax;  // a few tokens: maxima of the SwiGLU values, 16 at a time
     int32_t* dst;
     int32_t* row_token;
     void* map_ws;
@@ -53,14 +54,62 @@ struct Buffers {
 };
 
 struct Forms {
+    bool few;      // a few tokens: two launches behind the gating (few.hip)
     bool pairs;    // pair order
     bool requant;  // ... with the re-quantisation inside the down GEMM
     bool small;    // sorted, gating + sort + quantisation in one launch
 };
 
+FewArgs few_args(const moe355_layer& l, const Buffers& b, int64_t T)
+{
+    FewArgs a = {};
+    a.xq = b.xq;
+    a.x_scale = b.x_scale;
+    a.ids = b.topk_ids;
+    a.tw = (const uint16_t*)b.topk_weights;
+    a.T = (int)T;
+    a.k = l.top_k;
+    a.R = (int)T * l.top_k;
+    a.E = l.num_experts;
+    a.H = (int)l.hidden;
+    a.I = (int)l.intermediate;
+    if (l.weights == W_INT8_LIST) {
+        a.w13_list = (const int8_t* const*)l.w13;
+        a.s13_list = (const float* const*)l.s13;
+        a.w2_list = (const int8_t* const*)l.w2;
+        a.s2_list = (const float* const*)l.s2;
+    } else {
+        a.w13 = (const int8_t*)l.w13;
+        a.s13 = (const float*)l.s13;
+        a.w2 = (const int8_t*)l.w2;
+        a.s2 = (const float*)l.s2;
+    }
+    a.limit = l.swiglu_limit;
+    if (l.shared) {
+        a.S = (int)l.shared_intermediate;
+        a.sw13 = l.shared_w13;
+        a.sw2 = l.shared_w2;
+        a.ss13 = l.shared_s13;
+        a.ss2 = l.shared_s2;
+        a.sh_limit = l.shared_limit;
+        a.sh_alpha = l.shared_alpha;
+        a.sh_beta = l.shared_beta;
+    }
+    a.y = (float*)b.mlp_ws;
+    a.ymax = b.ymax;
+    a.q1 = b.q1;
+    a.q1_scale = b.q1_scale;
+    a.f16 = l.x_dtype == MOE355_DT_F16;
+    a.load = l.load;
+    return a;
+}
+
 Forms forms_of(const moe355_layer& l, int64_t T)
 {
     Forms f = {};
+    f.few = l.weights != W_INT4 && l.pair_order && T <= 64 && l.top_k <= 64 &&
+            moe355_gate_quant_supported(T, l.top_k, l.num_experts) && few_supported(few_args(l, Buffers{}, T));
+    if (f.few) return f;
     f.pairs = l.weights != W_INT4 && l.pair_order &&
               moe355_pair_order(T, l.top_k, l.num_experts, l.num_experts, l.hidden, l.intermediate);
     f.requant = f.pairs && moe355_gmm2_requant_pairs_supported(T, l.top_k, l.hidden, l.intermediate, l.num_experts);
@@ -84,6 +133,15 @@ Buffers lay_out(const moe355_layer& l, const Forms& f, int64_t T, void* base)
         b.logits = a.take<float>((size_t)T * E * 4);
         b.gate_bytes = moe355_router_gate_workspace(T, (int)H, E);
         b.gate_ws = b.gate_bytes ? a.take<void>(b.gate_bytes) : nullptr;
+    }
+    if (f.few) {
+        const size_t values = (size_t)R * I + (l.shared ? (size_t)T * l.shared_intermediate : 0);
+        b.ymax = a.take<float>(values / 16 * 4);
+        b.mlp_ws = a.take<void>(values * 4);
+        b.q1 = a.take<int8_t>(values);
+        b.q1_scale = a.take<float>((size_t)(R + T) * 4);
+        b.total = a.used;
+        return b;
     }
     b.q1 = a.take<int8_t>((size_t)R * I);
     b.q1_scale = a.take<float>((size_t)R * 4);
@@ -271,6 +329,12 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
     rc = gate_quant_impl(f.small, g, 1, b.topk_weights, b.topk_ids, b.xq, b.x_scale, b.dst, b.row_token,
                          b.expert_tokens, l.sync_counter, l.shared ? b.one_group : nullptr, stream);
     if (rc != MOE355_OK) return rc;
+    if (f.few) {
+        // the shared expert rides in the same two launches, whatever stream it was meant for
+        FewArgs a = few_args(l, b, T);
+        a.out = (uint16_t*)out;
+        return few_forward(a, (hipStream_t)stream);
+    }
 
     ForkJoinLease lease;
     bool joined = true;

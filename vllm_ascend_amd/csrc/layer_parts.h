@@ -56,4 +56,33 @@ int gmm2_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* wei
               int group_list_type, int64_t rows, int64_t k, int64_t n, int num_experts, void* out, int out_dtype,
               void* workspace, size_t workspace_bytes, void* stream);
 
+// ------------------------------------------------------------------ a few tokens (few.hip)
+struct FewArgs {
+    const int8_t* xq;        // [T, H]
+    const float* x_scale;    // [T]
+    const int32_t* ids;      // [T, k]
+    const uint16_t* tw;      // [T, k] routing weights, 16 bits
+    int T, k, R, E, H, I, S; // R = T * k; S: width of the shared expert
+    const int8_t *w13, *w2;  // tiled tensors with their scales, or device tables of per-expert tensors
+    const float *s13, *s2;
+    const int8_t* const* w13_list;
+    const float* const* s13_list;
+    const int8_t* const* w2_list;
+    const float* const* s2_list;
+    float limit;
+    const int8_t *sw13, *sw2;  // shared expert, or null
+    const float *ss13, *ss2;
+    float sh_limit, sh_alpha, sh_beta;
+    float* y;                // [R, I] SwiGLU values, then [T, S]
+    float* ymax;             // [R, I / 16] maxima of 16 values each, then [T, S / 16]
+    int8_t* q1;              // [R, I] then [T, S]
+    float* q1_scale;         // [R + T]
+    uint16_t* out;           // [T, H]
+    int f16;
+    int64_t* load;           // [E] or null: the rows of every expert are added
+};
+
+bool few_supported(const FewArgs& a);
+int few_forward(const FewArgs& a, hipStream_t st);
+
 }  // namespace moe355
