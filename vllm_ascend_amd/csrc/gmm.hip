@@ -650,6 +650,29 @@ static int dense_slabs(int64_t R, int K, int N, int E)
     return slabs < 1 ? 1 : slabs;
 }
 
+// the second family's tile map lies behind the first one's
+static void* second_map(const GmmArgs& a, void* tile_ws)
+{
+    return (char*)tile_ws + ((tiled_workspace_bytes(a.R, a.E, 64) + 255) & ~(size_t)255);
+}
+
+// The tile maps that launch_gemm_auto of this product will look for in tile_ws (at most two).
+int gemm_tile_specs(int64_t rows, int64_t k, int64_t n, int num_experts, void* tile_ws, TileSpec* specs)
+{
+    GmmArgs a = {};
+    a.R = rows;
+    a.K = (int)k;
+    a.N = (int)n;
+    a.E = num_experts;
+    if (dense_tiles(a)) return 0;
+    const GemmPlan plan = gemm_plan(a, true);
+    int count = 0;
+    if (plan.bm) specs[count++] = tile_spec(rows, num_experts, plan.bm, 0, plan.split, tile_ws);
+    if (plan.split > 0)
+        specs[count++] = tile_spec(rows, num_experts, plan.split_bm, plan.split + 1, 0, second_map(a, tile_ws));
+    return count;
+}
+
 template <int EPI>
 static int launch_gemm_auto(const GmmArgs& a_in, void* tile_ws, hipStream_t st, void* part_ws = nullptr,
                             size_t part_bytes = 0)
@@ -663,8 +686,7 @@ static int launch_gemm_auto(const GmmArgs& a_in, void* tile_ws, hipStream_t st, 
         return launch_status();
     }
     const GemmPlan plan = gemm_plan(a, tile_ws != nullptr);
-    // the second family's tile map lies behind the first one's
-    void* tile_ws2 = tile_ws ? (char*)tile_ws + ((tiled_workspace_bytes(a.R, a.E, 64) + 255) & ~(size_t)255) : nullptr;
+    void* tile_ws2 = tile_ws ? second_map(a, tile_ws) : nullptr;
     if (plan.split > 0) a.rows_max = plan.split;
     hipEvent_t first_stop = plan.split > 0 ? nullptr : ev1;
     if (plan.bm) {
@@ -806,6 +828,12 @@ extern "C" size_t moe355_gmm_i32_workspace(int64_t rows, int64_t n, int64_t k, i
     return bytes;
 }
 
+// where the tile maps lie in the gate_up product's workspace: behind the fp32 SwiGLU values
+void* moe355::gmm1_tile_ws(void* workspace, int64_t rows, int64_t n)
+{
+    return (char*)workspace + (((size_t)rows * (size_t)(n / 2) * 4 + 255) & ~(size_t)255);
+}
+
 extern "C" size_t moe355_gmm1_swiglu_quant_workspace(int64_t rows, int64_t n, int64_t k, int num_experts)
 {
     (void)k;
@@ -818,7 +846,7 @@ int moe355::gmm1_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* co
                       const float* weight_scale, const float* const* scale_list, const float* x_scale,
                       const int64_t* group_list, int group_list_type, int64_t rows, int64_t k, int64_t n,
                       int num_experts, float swiglu_limit, int8_t* out, float* out_scale, void* workspace,
-                      size_t workspace_bytes, void* stream, const int32_t* row_src)
+                      size_t workspace_bytes, void* stream, const int32_t* row_src, bool tiles_ready)
 {
     const void* wany = weight_list ? (const void*)weight_list : (const void*)weight_nz;
     int rc = check_gmm(x, wany, group_list, group_list_type, rows, k, n, num_experts);
@@ -848,7 +876,8 @@ int moe355::gmm1_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* co
     a.limit = swiglu_limit;
     a.y = y;
     a.row_src = row_src;
-    void* tile_ws = (char*)workspace + (((size_t)rows * I * 4 + 255) & ~(size_t)255);
+    a.tiles_ready = tiles_ready;
+    void* tile_ws = gmm1_tile_ws(workspace, rows, n);
     rc = launch_gemm_auto<EPI_SWIGLU>(a, tile_ws, st);
     if (rc != MOE355_OK) return rc;
     launch_swiglu_requant(y, group_list, group_list_type, num_experts, rows, I, out, out_scale, st);
@@ -898,7 +927,7 @@ extern "C" size_t moe355_gmm2_dequant_workspace(int64_t rows, int64_t n, int64_t
 int moe355::gmm2_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list, const float* scale,
                       const float* const* scale_list, const float* per_token_scale, const int64_t* group_list,
                       int group_list_type, int64_t rows, int64_t k, int64_t n, int num_experts, void* out,
-                      int out_dtype, void* workspace, size_t workspace_bytes, void* stream)
+                      int out_dtype, void* workspace, size_t workspace_bytes, void* stream, bool tiles_ready)
 {
     const void* wany = weight_list ? (const void*)weight_list : (const void*)weight_nz;
     int rc = check_gmm(x, wany, group_list, group_list_type, rows, k, n, num_experts);
@@ -925,6 +954,7 @@ int moe355::gmm2_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* co
     a.s_list = scale_list;
     a.out = (uint16_t*)out;
     a.out_f16 = out_dtype == MOE355_DT_F16;
+    a.tiles_ready = tiles_ready;
     return launch_gemm_auto<EPI_DEQUANT>(a, workspace, (hipStream_t)stream);
 }
 

@@ -51,6 +51,7 @@ struct GmmArgs {
     // A launch may cover only the experts whose row count lies in [rows_min, rows_max] (rows_max 0: no upper
     // bound): a batch with a skewed histogram is split over kernel families by expert, on the device.
     int rows_min, rows_max;
+    int tiles_ready;        // the tile maps of this call are in its workspace already (built by the routing launch)
     // outputs
     int32_t* acc;           // EPI_I32   [R, N]
     int32_t* acc_part;      // EPI_I32 with K cut into slabs: [slabs][R, N] partial sums (or null: atomics into acc)

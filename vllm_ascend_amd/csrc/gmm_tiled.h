@@ -2,19 +2,15 @@
 #pragma once
 
 #include "gmm_common.h"
+#include "tile_map.h"
 
 namespace moe355 {
 
-// (expert, row block) tiles of one launch, built on the device from the group list.
-struct TileMap {
-    int32_t* count;      // [1]
-    int32_t* expert;     // [max_tiles]
-    int32_t* row_begin;  // [max_tiles]
-    int32_t* row_end;    // [max_tiles] end of the expert's rows
-};
-
 // bytes of scratch for the tile map (BM = rows per tile: 64, 128 or 256)
 size_t tiled_workspace_bytes(int64_t rows, int E, int BM);
+
+// the tile map of a product over `rows` rows, laid out in a workspace of tiled_workspace_bytes()
+TileSpec tile_spec(int64_t rows, int E, int BM, int rows_min, int rows_max, void* workspace);
 
 // epi: EPI_*; bm: 64 or 128 (LDS-tiled kernel) or 256 (weight-streaming tiles).  ev0/ev1: optional events recorded around the GEMM kernel itself.
 void launch_tiled_any(int epi, int bm, const GmmArgs& a, void* workspace, hipStream_t st, hipEvent_t ev0,

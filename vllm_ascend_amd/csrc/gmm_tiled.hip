@@ -15,110 +15,20 @@
 #include <type_traits>
 
 #include "gmm_tiled.h"
+#include "tile_map.h"
 
 namespace moe355 {
 
-// One workgroup.  Thread t owns experts [t*seg, (t+1)*seg).  Tiles are numbered expert by expert.
-// by_length (the 256-row weight-streaming tiles): the tiles are listed longest first -- 161..192 rows, 129..160,
-// up to 128, then the tall ones (more than 192 rows, which become two shorter column items) -- so that the
-// workgroups that start last are the short ones and the compute units finish closer together.
-// rows_min / rows_max: experts whose row count lies outside [rows_min, rows_max] (rows_max 0: no upper bound) get
-// no tiles (another kernel of the same operator call covers them); their rows still count for the offsets.
-__global__ __launch_bounds__(256) void tile_map_kernel(const int64_t* __restrict__ gl, int gl_type, int E, int BM,
-                                                       int max_tiles, TileMap tm, int by_length, int rows_min,
-                                                       int rows_max)
+__global__ __launch_bounds__(256) void tile_map_kernel(const int64_t* __restrict__ gl, int gl_type, int E, TileSpec spec)
 {
-    auto tiled_rows = [&](int64_t m) -> int64_t { return (m >= rows_min && (rows_max == 0 || m <= rows_max)) ? m : 0; };
     __shared__ int32_t part_rows[16];
     __shared__ int32_t part_tiles[16];
-    if (by_length) {
-        // class of a tile with m rows left in its expert; per-thread counts per class, two classes per scan
-        auto cls = [](int64_t m) -> int { return m > 192 ? 3 : (m > 160 ? 0 : (m > 128 ? 1 : 2)); };
-        const int tid = threadIdx.x;
-        const int seg = (E + 255) / 256;
-        const int e0 = tid * seg;
-        auto rows_of = [&](int e) -> int64_t {
-            int64_t m = (gl_type == MOE355_GL_COUNT) ? gl[e] : gl[e] - (e > 0 ? gl[e - 1] : 0);
+    build_tile_map(
+        [&](int e) -> int64_t {
+            const int64_t m = (gl_type == MOE355_GL_COUNT) ? gl[e] : gl[e] - (e > 0 ? gl[e - 1] : 0);
             return m < 0 ? 0 : m;
-        };
-        int32_t rows = 0, n01 = 0, n23 = 0;  // counts packed 16 + 16 bits (at most max_tiles < 32768 tiles)
-        for (int j = 0; j < seg; ++j) {
-            const int e = e0 + j;
-            if (e < E) {
-                const int64_t m = rows_of(e);
-                rows += (int32_t)m;
-                for (int64_t r0 = 0; r0 < tiled_rows(m); r0 += BM) {
-                    const int c = cls(m - r0);
-                    if (c < 2) n01 += 1 << (16 * c);
-                    else n23 += 1 << (16 * (c - 2));
-                }
-            }
-        }
-        int32_t all_rows, all01, all23;
-        const int32_t rows_before = block_scan_exclusive_i32(rows, part_rows, all_rows);
-        const int32_t b01 = block_scan_exclusive_i32(n01, part_tiles, all01);
-        const int32_t b23 = block_scan_exclusive_i32(n23, part_tiles, all23);
-        const int32_t total[4] = {all01 & 0xffff, all01 >> 16, all23 & 0xffff, all23 >> 16};
-        const int32_t all_tiles = total[0] + total[1] + total[2] + total[3];
-        if (tid == 0) tm.count[0] = all_tiles < max_tiles ? all_tiles : max_tiles;
-        int32_t next[4] = {b01 & 0xffff, total[0] + (b01 >> 16), total[0] + total[1] + (b23 & 0xffff),
-                           total[0] + total[1] + total[2] + (b23 >> 16)};
-        int64_t row = rows_before;
-        for (int j = 0; j < seg; ++j) {
-            const int e = e0 + j;
-            if (e < E) {
-                const int64_t m = rows_of(e);
-                for (int64_t r0 = 0; r0 < tiled_rows(m); r0 += BM) {
-                    const int32_t t = next[cls(m - r0)]++;
-                    if (t < max_tiles) {
-                        tm.expert[t] = e;
-                        tm.row_begin[t] = (int32_t)(row + r0);
-                        tm.row_end[t] = (int32_t)(row + m);
-                    }
-                }
-                row += m;
-            }
-        }
-        return;
-    }
-    const int tid = threadIdx.x;
-    const int seg = (E + 255) / 256;
-    const int e0 = tid * seg;
-    auto rows_of = [&](int e) -> int64_t {
-        int64_t m = (gl_type == MOE355_GL_COUNT) ? gl[e] : gl[e] - (e > 0 ? gl[e - 1] : 0);
-        return m < 0 ? 0 : m;
-    };
-    int32_t rows = 0, tiles = 0;
-    for (int j = 0; j < seg; ++j) {
-        const int e = e0 + j;
-        if (e < E) {
-            const int64_t m = rows_of(e);
-            rows += (int32_t)m;
-            tiles += (int32_t)((tiled_rows(m) + BM - 1) / BM);
-        }
-    }
-    // exclusive prefix of rows and tiles over the threads (experts in order)
-    int32_t all_rows, all_tiles;
-    const int32_t rows_before = block_scan_exclusive_i32(rows, part_rows, all_rows);
-    const int32_t tiles_before = block_scan_exclusive_i32(tiles, part_tiles, all_tiles);
-    if (tid == 0) tm.count[0] = all_tiles < max_tiles ? all_tiles : max_tiles;
-    int64_t row = rows_before;
-    int32_t t = tiles_before;
-    for (int j = 0; j < seg; ++j) {
-        const int e = e0 + j;
-        if (e < E) {
-            const int64_t m = rows_of(e);
-            for (int64_t r0 = row; r0 < row + tiled_rows(m); r0 += BM) {
-                if (t < max_tiles) {
-                    tm.expert[t] = e;
-                    tm.row_begin[t] = (int32_t)r0;
-                    tm.row_end[t] = (int32_t)(row + m);
-                }
-                ++t;
-            }
-            row += m;
-        }
-    }
+        },
+        E, spec, part_rows, part_tiles);
 }
 
 constexpr int kBN = 256;  // channels per workgroup (4 wavefronts x 2 storage tiles)
@@ -852,6 +762,22 @@ __global__ __launch_bounds__(512, 1) void gmm_dense_kernel(GmmArgs a, int xn, in
 }
 
 // ------------------------------------------------------------------ host side
+TileSpec tile_spec(int64_t rows, int E, int BM, int rows_min, int rows_max, void* workspace)
+{
+    TileSpec t;
+    t.BM = BM;
+    t.by_length = BM == 256;
+    t.rows_min = rows_min;
+    t.rows_max = rows_max;
+    t.max_tiles = (int)(rows / BM + E);
+    const size_t arr = (size_t)(((size_t)t.max_tiles * 4 + 255) / 256) * 256;
+    t.tm.count = (int32_t*)workspace;
+    t.tm.expert = (int32_t*)((char*)workspace + 256);
+    t.tm.row_begin = (int32_t*)((char*)workspace + 256 + arr);
+    t.tm.row_end = (int32_t*)((char*)workspace + 256 + 2 * arr);
+    return t;
+}
+
 size_t tiled_workspace_bytes(int64_t rows, int E, int BM)
 {
     const int64_t max_tiles = rows / BM + E;
@@ -862,15 +788,11 @@ template <int EPI, int BMT, int RING>
 static void launch_tiled(const GmmArgs& a, void* workspace, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1)
 {
     constexpr int BM = 32 * BMT;
-    const int max_tiles = (int)(a.R / BM + a.E);
-    const size_t arr = (size_t)(((size_t)max_tiles * 4 + 255) / 256) * 256;
-    TileMap tm;
-    tm.count = (int32_t*)workspace;
-    tm.expert = (int32_t*)((char*)workspace + 256);
-    tm.row_begin = (int32_t*)((char*)workspace + 256 + arr);
-    tm.row_end = (int32_t*)((char*)workspace + 256 + 2 * arr);
-    hipLaunchKernelGGL(tile_map_kernel, dim3(1), dim3(256), 0, st, a.gl, a.gl_type, a.E, BM, max_tiles, tm, 0, a.rows_min,
-                       a.rows_max);
+    const TileSpec spec = tile_spec(a.R, a.E, BM, a.rows_min, a.rows_max, workspace);
+    const TileMap tm = spec.tm;
+    const int max_tiles = spec.max_tiles;
+    if (!a.tiles_ready)
+        hipLaunchKernelGGL(tile_map_kernel, dim3(1), dim3(256), 0, st, a.gl, a.gl_type, a.E, spec);
     const int channels = (EPI == EPI_SWIGLU) ? a.N / 2 : a.N;
     const int per_block = (EPI == EPI_SWIGLU) ? kBN / 2 : kBN;
     const int n_col_blocks = (channels + per_block - 1) / per_block;
@@ -898,15 +820,11 @@ static void launch_wide(const GmmArgs& a, void* workspace, hipStream_t st, hipEv
     static const hipError_t attr = hipFuncSetAttribute((const void*)gmm_wide_kernel<EPI>,
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     (void)attr;
-    const int max_tiles = (int)(a.R / BM + a.E);
-    const size_t arr = (size_t)(((size_t)max_tiles * 4 + 255) / 256) * 256;
-    TileMap tm;
-    tm.count = (int32_t*)workspace;
-    tm.expert = (int32_t*)((char*)workspace + 256);
-    tm.row_begin = (int32_t*)((char*)workspace + 256 + arr);
-    tm.row_end = (int32_t*)((char*)workspace + 256 + 2 * arr);
-    hipLaunchKernelGGL(tile_map_kernel, dim3(1), dim3(256), 0, st, a.gl, a.gl_type, a.E, BM, max_tiles, tm, 1, a.rows_min,
-                       a.rows_max);
+    const TileSpec spec = tile_spec(a.R, a.E, BM, a.rows_min, a.rows_max, workspace);
+    const TileMap tm = spec.tm;
+    const int max_tiles = spec.max_tiles;
+    if (!a.tiles_ready)
+        hipLaunchKernelGGL(tile_map_kernel, dim3(1), dim3(256), 0, st, a.gl, a.gl_type, a.E, spec);
     const int channels = (EPI == EPI_SWIGLU) ? a.N / 2 : a.N;
     const int per_block = (EPI == EPI_SWIGLU) ? kBN / 2 : kBN;
     const int n_col_blocks = (channels + per_block - 1) / per_block;

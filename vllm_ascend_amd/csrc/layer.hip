@@ -268,7 +268,7 @@ int routed_pairs(const moe355_layer& l, const Forms& f, const Buffers& b, int64_
                            b.o, l.x_dtype, st);
 }
 
-int routed_sorted(const moe355_layer& l, const Buffers& b, int64_t T, void* st)
+int routed_sorted(const moe355_layer& l, const Buffers& b, int64_t T, bool tiles_ready, void* st)
 {
     const int64_t H = l.hidden, I = l.intermediate, R = T * l.top_k;
     const int E = l.num_experts;
@@ -286,11 +286,12 @@ int routed_sorted(const moe355_layer& l, const Buffers& b, int64_t T, void* st)
     rc = gmm1_impl(b.xq, list ? nullptr : (const int8_t*)l.w13, list ? (const int8_t* const*)l.w13 : nullptr,
                    list ? nullptr : (const float*)l.s13, list ? (const float* const*)l.s13 : nullptr, b.x_scale,
                    b.expert_tokens, MOE355_GL_COUNT, R, H, 2 * I, E, l.swiglu_limit, b.q1, b.q1_scale, b.mlp_ws,
-                   b.mlp_bytes, st, b.row_token);
+                   b.mlp_bytes, st, b.row_token, tiles_ready);
     if (rc != MOE355_OK) return rc;
     return gmm2_impl(b.q1, list ? nullptr : (const int8_t*)l.w2, list ? (const int8_t* const*)l.w2 : nullptr,
                      list ? nullptr : (const float*)l.s2, list ? (const float* const*)l.s2 : nullptr, b.q1_scale,
-                     b.expert_tokens, MOE355_GL_COUNT, R, I, H, E, b.o, l.x_dtype, b.gmm2_ws, b.gmm2_bytes, st);
+                     b.expert_tokens, MOE355_GL_COUNT, R, I, H, E, b.o, l.x_dtype, b.gmm2_ws, b.gmm2_bytes, st,
+                     tiles_ready);
 }
 
 }  // namespace
@@ -350,10 +351,19 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
     } else if (l.shared == 1) {
         rc = shared_expert(l, b, T, stream);
     }
-    if (rc == MOE355_OK && !f.pairs && !f.small)
-        rc = moe355_route_map(b.topk_ids, T, l.top_k, l.num_experts, 1, b.dst, b.row_token, b.expert_tokens, b.map_ws,
-                              b.map_bytes, stream);
-    if (rc == MOE355_OK) rc = f.pairs ? routed_pairs(l, f, b, T, stream) : routed_sorted(l, b, T, stream);
+    bool tiles_ready = false;
+    if (rc == MOE355_OK && !f.pairs && !f.small) {
+        TileSpec specs[4];
+        int n = 0;
+        if (l.weights != W_INT4) {
+            n = gemm_tile_specs(R, l.hidden, 2 * l.intermediate, l.num_experts,
+                                gmm1_tile_ws(b.mlp_ws, R, 2 * l.intermediate), specs);
+            n += gemm_tile_specs(R, l.intermediate, l.hidden, l.num_experts, b.gmm2_ws, specs + n);
+        }
+        rc = route_map_impl(b.topk_ids, T, l.top_k, l.num_experts, 1, b.dst, b.row_token, b.expert_tokens, b.map_ws,
+                            b.map_bytes, specs, n, &tiles_ready, stream);
+    }
+    if (rc == MOE355_OK) rc = f.pairs ? routed_pairs(l, f, b, T, stream) : routed_sorted(l, b, T, tiles_ready, stream);
     if (!joined && hipStreamWaitEvent((hipStream_t)stream, lease.fj.join, 0) != hipSuccess) return MOE355_E_LAUNCH;
     if (rc != MOE355_OK) return rc;
     const void* residual = l.shared ? b.sh_out : nullptr;

@@ -3,7 +3,7 @@
 // written by the routing launch, expert loads added up by the combine).
 #pragma once
 
-#include "moe355_common.h"
+#include "tile_map.h"
 
 namespace moe355 {
 
@@ -50,11 +50,21 @@ int gmm2_pairs_impl(const int8_t* x, const float* per_token_scale, const float* 
 int gmm1_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list, const float* weight_scale,
               const float* const* scale_list, const float* x_scale, const int64_t* group_list, int group_list_type,
               int64_t rows, int64_t k, int64_t n, int num_experts, float swiglu_limit, int8_t* out, float* out_scale,
-              void* workspace, size_t workspace_bytes, void* stream, const int32_t* row_src = nullptr);
+              void* workspace, size_t workspace_bytes, void* stream, const int32_t* row_src = nullptr,
+              bool tiles_ready = false);
 int gmm2_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list, const float* scale,
               const float* const* scale_list, const float* per_token_scale, const int64_t* group_list,
               int group_list_type, int64_t rows, int64_t k, int64_t n, int num_experts, void* out, int out_dtype,
-              void* workspace, size_t workspace_bytes, void* stream);
+              void* workspace, size_t workspace_bytes, void* stream, bool tiles_ready = false);
+void* gmm1_tile_ws(void* workspace, int64_t rows, int64_t n);
+// tile maps (at most two) that a grouped product will look for in its workspace
+int gemm_tile_specs(int64_t rows, int64_t k, int64_t n, int num_experts, void* tile_ws, TileSpec* specs);
+
+// moe355_route_map with the tile maps of the two products (nspecs of them, at most 4) built by the same launch where it
+// is one launch (returns 1 in *built then)
+int route_map_impl(const int32_t* expert_idx, int64_t num_tokens, int top_k, int num_experts, int tokens_num_type,
+                   int32_t* expanded_row_idx, int32_t* row_token, int64_t* expert_tokens, void* workspace,
+                   size_t workspace_bytes, const TileSpec* specs, int nspecs, bool* built, void* stream);
 
 // ------------------------------------------------------------------ a few tokens (few.hip)
 struct FewArgs {

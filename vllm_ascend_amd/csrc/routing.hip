@@ -18,7 +18,7 @@
 #include <mutex>
 #include <type_traits>
 
-#include "moe355_common.h"
+#include "layer_parts.h"
 
 namespace moe355 {
 
@@ -322,59 +322,97 @@ __global__ __launch_bounds__(256) void route_gather_small_kernel(const int32_t* 
     gather_token_row<QUANT, DT>(x + (int64_t)t * H, H, top_k, drow, lds4, xs, sx, held);
 }
 
-// The index maps alone for at most 4096 pairs, in ONE launch of num_tokens + 1 workgroups: workgroup t finds the
-// destinations of its token's k pairs by counting (as above) and writes them and the row -> token map; the last
-// workgroup the per-expert counts.  Nobody waits for anybody.
-constexpr int kMapSmallIters = 16;  // 16 * 256 = 4096 pairs
+// The index maps alone in ONE launch: a workgroup of 1024 owns 1024 consecutive pairs, and instead of being told how
+// many pairs the others hold, it counts them itself -- every workgroup reads all ids (L2 hits) and counts them in LDS,
+// split into "in front of my pairs" and "the rest".  That is R / 1024 times the work of a histogram and no hand-off:
+// three launches (histogram, scan, scatter) of 4.5 to 7 us each in a row become one.  The ranks inside the 1024 pairs
+// come from per-wavefront counts and ballots.  Further workgroups build the tile maps of the grouped GEMMs behind it
+// (launches of 4.5 us each otherwise): they do the same counting for their row counts.
+struct RouteMapArgs {
+    const int32_t* ids;
+    int R, E, top_k, tokens_num_type, nbits, chunks, nspecs;
+    int32_t* dst;
+    int32_t* row_token;
+    int64_t* expert_tokens;
+    TileSpec specs[4];
+};
+constexpr int kMapThreads = 1024;
+constexpr int kMapWaves = kMapThreads / 64;
+constexpr int kMapMaxExperts = 512;
+constexpr int kMapMaxPairs = 65536;
 
-__global__ __launch_bounds__(256) void route_map_small_kernel(const int32_t* __restrict__ ids, int R, int E,
-                                                              int tokens_num_type, int32_t* __restrict__ off,
-                                                              int64_t* __restrict__ expert_tokens,
-                                                              int32_t* __restrict__ dst, int32_t* __restrict__ row_token,
-                                                              int top_k)
+__global__ __launch_bounds__(kMapThreads) void route_map_kernel(RouteMapArgs a)
 {
-    extern __shared__ int32_t sm[];  // the counting workgroup: [E] counts, [256] scan scratch
-    __shared__ int32_t wsum[4][64];
-    const int num_tokens = (int)gridDim.x - 1;
-    if ((int)blockIdx.x == num_tokens) {
-        small_hist_scan(ids, R, E, tokens_num_type, off, expert_tokens, sm);
+    extern __shared__ int32_t map_lds[];
+    int32_t* count = map_lds;          // [E] pairs of every expert: in front of this chunk << 16 | the rest
+    int32_t* part = count + a.E;       // [32] scan scratch
+    int32_t* whist = part + 32;        // [16][E] pairs of every wavefront, then the first row of its pairs
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int E = a.E, R = a.R;
+    const bool maps = (int)blockIdx.x >= a.chunks;  // a tile map instead of a chunk
+    const int begin = maps ? 0 : (int)blockIdx.x * kMapThreads;
+    for (int i = tid; i < E; i += kMapThreads) count[i] = 0;
+    if (!maps)
+        for (int i = tid; i < kMapWaves * E; i += kMapThreads) whist[i] = 0;
+    __syncthreads();
+    int mine = -1;  // this thread's pair of the chunk
+    for (int base = 0; base < R; base += 8 * kMapThreads) {
+        int id[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int f = base + j * kMapThreads + tid;
+            id[j] = f < R ? a.ids[f] : -1;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int f0 = base + j * kMapThreads;  // a multiple of 1024: a whole chunk
+            const int e = id[j];
+            if (e >= 0 && e < E) atomicAdd(&count[e], f0 < begin ? 0x10000 : 1);
+            if (f0 == begin) mine = e;
+        }
+    }
+    if (mine < 0 || mine >= E) mine = -1;
+    if (!maps && mine >= 0) atomicAdd(&whist[wave * E + mine], 1);
+    __syncthreads();
+    // at most 65536 pairs: only in a chunk that has none in front of it may the rest need more than 16 bits
+    auto in_front = [&](int e) { return begin == 0 ? 0 : (int)((uint32_t)count[e] >> 16); };
+    auto total = [&](int e) { return begin == 0 ? count[e] : (count[e] & 0xffff) + in_front(e); };
+    if (maps) {
+        build_tile_map([&](int e) -> int64_t { return total(e); }, E, a.specs[(int)blockIdx.x - a.chunks], part,
+                       part + 16);
         return;
     }
-    const int t = blockIdx.x;
-    const int tid = threadIdx.x;
-    int my_e[kMapSmallIters];
+    int all;
+    const int rows = tid < E ? total(tid) : 0;  // E <= 512
+    const int first = block_scan_exclusive_i32(rows, part, all);
+    if (tid < E) {
+        int run = first + in_front(tid);
 #pragma unroll
-    for (int it = 0; it < kMapSmallIters; ++it) {
-        const int f = it * 256 + tid;
-        int e = kInvalidExpert;
-        if (f < R) {
-            e = ids[f];
-            if (e < 0 || e >= E) e = kInvalidExpert;
+        for (int w = 0; w < kMapWaves; ++w) {
+            const int n = whist[w * E + tid];
+            whist[w * E + tid] = run;
+            run += n;
         }
-        my_e[it] = e;
-    }
-    const int iters = (R + 255) >> 8;
-    for (int j = 0; j < top_k; ++j) {
-        const int fj = t * top_k + j;
-        const int ej = ids[fj];
-        int c = 0;
-#pragma unroll
-        for (int it = 0; it < kMapSmallIters; ++it) {
-            if (it < iters) {
-                const int f = it * 256 + tid;
-                c += (my_e[it] < ej || (my_e[it] == ej && f < fj)) ? 1 : 0;
-            }
-        }
-        c = wave_sum_i32(c);
-        if ((tid & 63) == 0) wsum[tid >> 6][j] = c;
+        if (blockIdx.x == 0) a.expert_tokens[tid] = a.tokens_num_type == 1 ? (int64_t)rows : (int64_t)(first + rows);
     }
     __syncthreads();
-    if (tid < top_k) {
-        const int ej = ids[t * top_k + tid];
-        const bool valid = ej >= 0 && ej < E;
-        const int d = wsum[0][tid] + wsum[1][tid] + wsum[2][tid] + wsum[3][tid];
-        dst[t * top_k + tid] = valid ? d : R;  // a dropped pair points one past the last row
-        if (valid) row_token[d] = t;
+    // rank inside the wavefront's 64 pairs: lanes with the same expert find each other with ballots
+    const bool valid = mine >= 0;
+    unsigned long long same = __ballot(valid);
+    for (int b = 0; b < a.nbits; ++b) {
+        const bool bit = (mine >> b) & 1;
+        const unsigned long long bal = __ballot(valid && bit);
+        same &= bit ? bal : ~bal;
+    }
+    const int f = begin + tid;
+    if (f < R) {
+        int32_t d = R;  // a dropped pair points one past the last row
+        if (valid) {
+            const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+            d = whist[wave * E + mine] + __popcll(same & below);
+            a.row_token[d] = f / a.top_k;
+        }
+        a.dst[f] = d;
     }
 }
 
@@ -519,10 +557,12 @@ extern "C" int moe355_init_routing(const void* x, int x_dtype, int64_t num_token
                              workspace_bytes, stream);
 }
 
-extern "C" int moe355_route_map(const int32_t* expert_idx, int64_t num_tokens, int top_k, int num_experts,
-                                int tokens_num_type, int32_t* expanded_row_idx, int32_t* row_token,
-                                int64_t* expert_tokens, void* workspace, size_t workspace_bytes, void* stream)
+int moe355::route_map_impl(const int32_t* expert_idx, int64_t num_tokens, int top_k, int num_experts,
+                           int tokens_num_type, int32_t* expanded_row_idx, int32_t* row_token, int64_t* expert_tokens,
+                           void* workspace, size_t workspace_bytes, const TileSpec* specs, int nspecs, bool* built,
+                           void* stream)
 {
+    if (built) *built = false;
     if (num_tokens < 0 || top_k <= 0 || num_experts <= 0) return MOE355_E_ARG;
     if (tokens_num_type != 0 && tokens_num_type != 1) return MOE355_E_UNSUPPORTED;
     if (top_k > 64 || num_experts > 2048) return MOE355_E_SHAPE;
@@ -535,17 +575,37 @@ extern "C" int moe355_route_map(const int32_t* expert_idx, int64_t num_tokens, i
     if (R > 0 && (!expert_idx || !expanded_row_idx || !row_token)) return MOE355_E_ARG;
     int nch, parts, cpp, nbits;
     const RouteWs ws = route_ws_of(workspace, R, num_experts, nch, parts, cpp, nbits);
-    if (R > 0 && R <= kMapSmallIters * 256 && num_tokens <= 1024) {
-        // one launch instead of three short ones that wait for each other (every workgroup reads all ids: not for
-        // thousands of tokens with one slot each)
-        hipLaunchKernelGGL(route_map_small_kernel, dim3((unsigned)num_tokens + 1), dim3(256),
-                           ((size_t)num_experts + 256) * 4, (hipStream_t)stream, expert_idx, (int)R, num_experts,
-                           tokens_num_type, ws.off, expert_tokens, expanded_row_idx, row_token, top_k);
+    if (R > 0 && R <= kMapMaxPairs && num_experts <= kMapMaxExperts) {
+        RouteMapArgs a = {};
+        a.ids = expert_idx;
+        a.R = (int)R;
+        a.E = num_experts;
+        a.top_k = top_k;
+        a.tokens_num_type = tokens_num_type;
+        a.nbits = nbits;
+        a.chunks = (int)((R + kMapThreads - 1) / kMapThreads);
+        a.nspecs = nspecs;
+        a.dst = expanded_row_idx;
+        a.row_token = row_token;
+        a.expert_tokens = expert_tokens;
+        for (int i = 0; i < nspecs; ++i) a.specs[i] = specs[i];
+        const size_t lds = ((size_t)(kMapWaves + 1) * num_experts + 32) * 4;  // at most 35 KB
+        hipLaunchKernelGGL(route_map_kernel, dim3((unsigned)(a.chunks + nspecs)), dim3(kMapThreads), lds,
+                           (hipStream_t)stream, a);
+        if (built) *built = true;
         return launch_status();
     }
     launch_maps(expert_idx, R, num_experts, top_k, tokens_num_type, ws, nch, parts, cpp, nbits, expanded_row_idx,
                 row_token, expert_tokens, (hipStream_t)stream);
     return launch_status();
+}
+
+extern "C" int moe355_route_map(const int32_t* expert_idx, int64_t num_tokens, int top_k, int num_experts,
+                                int tokens_num_type, int32_t* expanded_row_idx, int32_t* row_token,
+                                int64_t* expert_tokens, void* workspace, size_t workspace_bytes, void* stream)
+{
+    return route_map_impl(expert_idx, num_tokens, top_k, num_experts, tokens_num_type, expanded_row_idx, row_token,
+                          expert_tokens, workspace, workspace_bytes, nullptr, 0, nullptr, stream);
 }
 
 extern "C" int moe355_init_routing_prequant(const int8_t* x, const float* x_scale, int64_t num_tokens, int64_t hidden,
