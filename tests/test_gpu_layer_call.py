@@ -70,6 +70,22 @@ def test_a_few_tokens_at_full_size(name, tokens):
     assert torch.equal(layer(x, logits), layer.forward_impl(x, logits).routed_out)
 
 
+# pair order with experts of several 32-row blocks (workgroups of their own), the others idle or with a few rows
+@pytest.mark.parametrize("tokens", [32, 33, 64, 65, 200])
+@pytest.mark.parametrize("rest", [0, 7])
+def test_hot_experts_in_pair_order(tokens, rest):
+    cfg, layer, x, logits = _pair("c2_small", tokens)
+    hot = logits[:1].expand(tokens, -1).contiguous()
+    if rest:
+        hot[::rest] = logits[::rest]
+    assert torch.equal(layer(x, hot), layer.forward_impl(x, hot).routed_out)
+    layer.use_fused_small_batch = False
+    assert torch.equal(layer(x, hot), layer.forward_impl(x, hot).routed_out)
+    want = layer.forward_impl(x, hot).routed_out
+    layer.use_fused_small_batch = True
+    assert torch.equal(layer(x, hot), want)  # against the operators on the sorted order
+
+
 def test_the_call_follows_the_layer():
     """Options that change between calls, and a copied layer."""
     cfg, layer, x, logits = _pair("c2_small", 40)

@@ -13,6 +13,7 @@
 #include <hip/hip_ext.h>
 #include <stdlib.h>
 #include <string.h>
+#include <type_traits>
 
 #include "gmm_common.h"
 #include "gmm_tiled.h"
@@ -83,6 +84,7 @@ __device__ __forceinline__ int nth_expert_with_rows(const int64_t* gl, int gl_ty
 }
 
 constexpr int kPairMax = 1024;
+constexpr int kPairExperts = 2048;  // that the lookups of the slots can hold
 
 // REQ (pair order, down GEMM): the activation is still the fp32 SwiGLU output; the workgroup re-quantises the rows
 // of its expert itself, 32 at a time, into LDS (row maximum through LDS atomics on the bit patterns, which order
@@ -99,19 +101,20 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
     extern __shared__ __attribute__((aligned(16))) int8_t qtile[];  // REQ: 32 rows of K + 16 bytes
     __shared__ uint32_t qmax[REQ ? 32 : 1];
     __shared__ float qscale[REQ ? 32 : 1];
-    __shared__ int32_t red[(KSPLIT > 1) ? 32 * 64 : 1];
+    constexpr int kRed = (KSPLIT > 1) ? 32 * 64 : 1;
+    __shared__ int32_t red[PAIRS && kRed < kPairExperts ? kPairExperts : kRed];
     __shared__ uint16_t plist[PAIRS ? kPairMax : 1];
     __shared__ int32_t pcount[4];
     __shared__ uint32_t pmap[PAIRS ? 64 : 1];  // one bit per expert (at most 2048) that has pairs
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // tell the compiler: addresses go to SGPRs
     const int lane = threadIdx.x & 63;
     const int NB = a.N >> 5, KB = a.K >> 5;
     const int upe = NB >> 1;  // units per expert
     const int64_t unit = (KSPLIT == 1) ? (int64_t)blockIdx.x * 4 + wave : (int64_t)blockIdx.x;
-    // pair order with fewer pairs than experts: the grid has a slot per pair instead of a place per expert (most
-    // experts are idle, and a workgroup that only finds that out still costs its dispatch: 28,000 of them are
-    // 150 us), and slot s belongs to the s-th expert that has pairs at all
-    const int places = (PAIRS && a.pair_slots > 0) ? a.pair_slots : (!PAIRS && !EARLY && a.gl_slots > 0) ? a.gl_slots : a.E;
+    // pair order: the grid has slots instead of a place per expert (an idle expert's workgroup only finds that out, but
+    // it still costs its dispatch -- 28,000 of them are 150 us -- and the weights it has requested by then), and slot s
+    // belongs to the s-th expert that has pairs; the workgroups that start first have places (pair_places below)
+    const int places = PAIRS ? a.pair_first + a.pair_slots + a.pair_extra : (!EARLY && a.gl_slots > 0) ? a.gl_slots : a.E;
     if (unit >= (int64_t)places * upe) return;  // KSPLIT == 1: no barriers below; KSPLIT == 4: whole workgroup leaves
     int e = (int)(unit / upe);
     const int p = (int)(unit % upe);
@@ -142,8 +145,36 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
             pid[c] = (c * 64 < Q && f < (int)a.R) ? a.pair_ids[f] : -1;
         }
     }
+    int block = 0;  // pair order: which 32 rows of the expert
     if constexpr (PAIRS) {
-        if (a.pair_slots > 0) {
+        if (e >= a.pair_first + a.pair_slots) {
+            // further blocks of experts with more than 32 rows, in the order of the experts: the pairs of every expert
+            // are counted in LDS and every wavefront walks the counts, 64 experts at a time
+            for (int i = threadIdx.x; i < a.E; i += 256) red[i] = 0;
+            __syncthreads();
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (pid[c] >= 0 && pid[c] < a.E) atomicAdd(&red[pid[c]], 1);
+            __syncthreads();
+            int left = e - a.pair_first - a.pair_slots;
+            e = -1;
+            for (int base = 0; base < a.E && e < 0; base += 64) {
+                const int n = base + lane < a.E ? red[base + lane] : 0;
+                const int more = n > 32 ? (n - 1) >> 5 : 0;
+                const int incl = wave_scan_inclusive_i32(more);
+                const bool has = left >= incl - more && left < incl;
+                const unsigned long long holder = __ballot(has);
+                if (holder) {
+                    const int h = __builtin_ctzll(holder);
+                    e = base + h;
+                    block = 1 + __builtin_amdgcn_readlane(left - (incl - more), h);
+                } else {
+                    left -= __builtin_amdgcn_readlane(incl, 63);
+                }
+            }
+            if (e < 0) return;  // not so many blocks (the same answer in all four wavefronts)
+            __syncthreads();    // the counts are read before the sums take their place
+        } else if (e >= a.pair_first) {  // the same answer in all four wavefronts (KSPLIT == 1: units come in fours)
             // the experts that have pairs, as a bit map in LDS; every wavefront then finds the expert of the
             // workgroup's slot by itself: a count of the bits in front of each word, and the word's bit
             if (threadIdx.x < 64) pmap[threadIdx.x] = 0u;
@@ -152,7 +183,9 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
             for (int c = 0; c < 4; ++c)
                 if (pid[c] >= 0 && pid[c] < a.E) atomicOr(&pmap[pid[c] >> 5], 1u << (pid[c] & 31));
             __syncthreads();
-            const uint32_t bits = pmap[lane];
+            const int mine0 = lane * 32;
+            const uint32_t bits = a.pair_first <= mine0 ? pmap[lane]
+                                  : a.pair_first >= mine0 + 32 ? 0u : pmap[lane] & (~0u << (a.pair_first - mine0));
             const int cnt = __popc(bits);
             int incl = cnt;
 #pragma unroll
@@ -161,18 +194,19 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
                 if (lane >= off) incl += t;
             }
             const int excl = incl - cnt;
-            const bool has = e >= excl && e < incl;
+            const int slot = e - a.pair_first;
+            const bool has = slot >= excl && slot < incl;
             const unsigned long long holder = __ballot(has);
             if (holder == 0ull) return;  // fewer experts with pairs than slots (the same answer in all four wavefronts)
             uint32_t t = bits;
-            for (int i = has ? e - excl : 0; i > 0; --i) t &= t - 1;
-            const int mine = lane * 32 + (t ? __builtin_ctz(t) : 0);
-            e = __shfl(mine, __builtin_ctzll(holder), 64);
+            for (int i = has ? slot - excl : 0; i > 0; --i) t &= t - 1;
+            const int mine = mine0 + (t ? __builtin_ctz(t) : 0);
+            e = __builtin_amdgcn_readlane(mine, __builtin_ctzll(holder));
         }
     }
     if constexpr (!PAIRS && !EARLY) {
         if (a.gl_slots > 0) {  // few rows over many experts: the workgroup's place is a slot, not an expert
-            e = nth_expert_with_rows(a.gl, a.gl_type, a.E, e, lane);
+            e = __builtin_amdgcn_readfirstlane(nth_expert_with_rows(a.gl, a.gl_type, a.E, e, lane));
             if (e < 0) return;
         }
     }
@@ -224,6 +258,10 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
         }
         __syncthreads();
         if (row1 == 0) return;  // the whole workgroup: nobody chose this expert
+        if (a.pair_extra > 0) {
+            row0 = 32 * block;
+            if (row1 > row0 + 32) row1 = row0 + 32;
+        }
     } else {
         expert_rows(a.gl, a.gl_type, e, lane, row0, row1);
         if (!expert_in_launch(a, row1 - row0)) return;  // another kernel of this operator call covers the expert
@@ -259,7 +297,8 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
 
     for (int64_t r0 = row0; r0 < row1; r0 += 32) {
         const bool valid = r0 + tok < row1;
-        int64_t row, src;  // where the row's result goes, where its values lie
+        using Index = std::conditional_t<PAIRS, int32_t, int64_t>;  // at most 1024 rows in pair order
+        Index row, src;  // where the row's result goes, where its values lie
         if constexpr (PAIRS) {
             row = plist[valid ? r0 + tok : 0];
             src = a.pair_gather ? row / a.pair_k : row;
@@ -267,9 +306,10 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
             row = r0 + tok;
             src = a.row_src ? (int64_t)a.row_src[valid ? row : row0] : row;
         }
-        const int8_t* xr;
+        const int8_t* xb = REQ ? qtile : a.x;
+        std::conditional_t<PAIRS, uint32_t, int64_t> xo;  // this lane's operand bytes of the row, behind xb
         float rs = 0.0f;
-        if constexpr (!REQ) xr = a.x + src * a.K + kh * 16;
+        if constexpr (!REQ) xo = src * a.K + kh * 16;
         if constexpr (REQ) {
             // rows r0 .. r0 + 31 of the expert -> int8 in LDS, every (row, four values) item by some thread
             const int pitch = a.K + 16;  // rows 16 bytes apart in the banks
@@ -307,7 +347,7 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
                 qscale[threadIdx.x] = (amax == 0.0f) ? 0.0f : amax / 127.0f;
             }
             __syncthreads();
-            xr = qtile + (valid ? tok : 0) * pitch + kh * 16;
+            xo = (valid ? tok : 0) * pitch + kh * 16;
             rs = qscale[valid ? tok : 0];
         } else if constexpr (EPI != EPI_I32) {
             rs = a.row_scale[(PAIRS || a.row_src) ? src : (valid ? row : row0)];
@@ -318,7 +358,7 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
             v4i b[UN];
 #pragma unroll
             for (int u = 0; u < UN; ++u)
-                b[u] = (valid && kb + u < kb_end) ? *(const v4i*)(xr + (kb + u) * 32) : (v4i){0, 0, 0, 0};
+                b[u] = (valid && kb + u < kb_end) ? *(const v4i*)(xb + (xo + (kb + u) * 32)) : (v4i){0, 0, 0, 0};
 #pragma unroll
             for (int u = 0; u < UN; ++u) {
                 c0 = mfma_i8(a0[u], b[u], c0);
@@ -355,14 +395,14 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
             if constexpr (EPI == EPI_I32 && SLABS) {
                 if (valid && a.acc_part) {
                     // the slab's partial sums to its own plane of the scratch; slab_sum_kernel adds the planes
-                    int32_t* plane = a.acc_part + ((int64_t)blockIdx.y * a.R + row) * a.N;
+                    int32_t* plane = a.acc_part + ((int64_t)blockIdx.y * a.R + (int64_t)row) * a.N;
                     *(v4i*)(plane + nb0 * 32 + ch) = (v4i){g[0], g[1], g[2], g[3]};
                     *(v4i*)(plane + nb1 * 32 + ch) = (v4i){u[0], u[1], u[2], u[3]};
                 } else if (valid) {
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        atomicAdd(a.acc + row * a.N + nb0 * 32 + ch + j, g[j]);
-                        atomicAdd(a.acc + row * a.N + nb1 * 32 + ch + j, u[j]);
+                        atomicAdd(a.acc + (int64_t)row * a.N + nb0 * 32 + ch + j, g[j]);
+                        atomicAdd(a.acc + (int64_t)row * a.N + nb1 * 32 + ch + j, u[j]);
                     }
                 }
             } else {
@@ -1001,25 +1041,33 @@ extern "C" int moe355_pair_order(int64_t num_tokens, int top_k, int num_logits, 
     return pairs < 1024 || pairs / num_experts < 12;  // where the sorted form streams as well (tiled_bm)
 }
 
-// pair order: how many places the grid gets.  A place per expert lets a workgroup request its first weight tiles
-// before it has seen a single id, which is the fastest form when nearly every expert has pairs -- and makes every
-// idle expert cost the dispatch of its workgroups plus 32 KiB of weights requested for nothing.  A slot per pair
-// (at most one per expert; the kernel looks up which expert a slot belongs to, and requests nothing before) costs
-// every launch one exposed lookup, and nothing for idle experts.  Measured, whole layer under graph replay:
-//   DeepSeek-V3 shape, uniform routing, 1 / 8 / 32 / 64 / 128 tokens: 307 -> 104, 567 -> 403, 1174 -> 1114,
-//     1492 -> 1475, 1641 -> 1639 us; Zipf(1.1) routing, 96 / 128 tokens: 719 -> 599, 839 -> 731 us
-//   Qwen3 shape, uniform, 1 / 4 / 16 / 64 / 128 tokens: 48 -> 38, 62 -> 42, 91 -> 86, 111.7 -> 114.3, 116 -> 120 us;
-//     Zipf(1.1), 24 / 64 / 128 tokens: 80.5 -> 63.3, 108.9 -> 83.0, 169.6 -> 127.4 us
-// The host cannot know the skew.  Slots wherever uniform routing loses nothing by them: up to two pairs per expert,
-// and at any number of pairs when an expert has 48 units and more (the DeepSeek-V3 shape); with more pairs over
-// experts of few units (the Qwen3 shape from 40 tokens on) a place per expert, which is the faster form on uniform
-// routing and the slower one on skewed routing.  The bit map of the lookup holds 2048 experts.
-static int pair_places(GmmArgs& a)
+// pair order: the places of the grid.
+// A place per expert lets a workgroup request its first weight tiles before it has seen a single id, and makes every
+// idle expert cost the dispatch of its workgroups plus 32 KiB of weights requested for nothing.  A slot (the kernel
+// looks up which expert it belongs to, and requests nothing before) costs one exposed lookup, and nothing for idle
+// experts.  The exposed lookup only shows in the workgroups that the chip starts with; later ones run beside others
+// that stream.  So, with more than two pairs per expert, the experts whose units are resident first have places and the
+// rest have slots; with fewer pairs idle experts are the rule and every place is a slot.  Whole layer of the Qwen3
+// shape, places / slots / both: 64 tokens uniform 110.1 / 110.4 / 109.1 us, Zipf(1.1) 90 / 78 / 77 us; 127 tokens
+// uniform 113.3 / 116.7 / 113.6 us.
+// An expert with more than 32 rows takes several passes over its weights, one after the other.  Where an expert has few
+// units (the launch is over after two or three rounds of workgroups) its further blocks of 32 rows become workgroups of
+// their own at the end of the grid: Qwen3 shape, Zipf(1.1), 64 / 100 / 127 tokens 77 / 118 / 135 -> 75 / 86 / 93 us,
+// uniform routing unchanged.  With 48 units and more the passes hide among the other workgroups, and the repeated
+// fetches at the end do not (DeepSeek-V3 shape, 64 tokens under Zipf(1.1): 444 us in passes, 477 in workgroups).
+// The lookups hold 2048 experts.
+static int pair_places(GmmArgs& a, int resident_units)
 {
-    const int64_t places = a.R < (int64_t)a.E ? a.R : (int64_t)a.E;
-    const bool slots = a.R <= 2 * (int64_t)a.E || a.N / 64 >= 48;
-    a.pair_slots = (slots && a.E <= 2048) ? (int)places : 0;
-    return (int)(a.pair_slots > 0 ? places : a.E);
+    a.pair_first = a.E;
+    a.pair_slots = a.pair_extra = 0;
+    if (a.E <= kPairExperts) {
+        a.pair_first = a.R > 2 * (int64_t)a.E ? resident_units / (a.N / 64) : 0;
+        if (a.pair_first > a.E) a.pair_first = a.E;
+        const int rest = a.E - a.pair_first;
+        a.pair_slots = a.R < (int64_t)rest ? (int)a.R : rest;
+        if (a.N / 64 < 48) a.pair_extra = (int)(a.R / 33);
+    }
+    return a.pair_first + a.pair_slots + a.pair_extra;
 }
 
 extern "C" size_t moe355_gmm1_swiglu_quant_pairs_workspace(int64_t num_tokens, int top_k, int64_t n)
@@ -1060,7 +1108,7 @@ int moe355::gmm1_pairs_impl(const int8_t* x, const float* x_scale, const int32_t
     a.pair_gather = 1;
     hipEvent_t ev0, ev1;
     take_profile_events(ev0, ev1);
-    const int64_t units = (int64_t)pair_places(a) * (n / 64);
+    const int64_t units = (int64_t)pair_places(a, 768) * (n / 64);
     launch_gemm(gmm_stream_kernel<EPI_SWIGLU, 4, 4, 3, false, true, true>, dim3((unsigned)units), st, a, ev0, ev1);
     if (out) launch_swiglu_requant(y, nullptr, 0, num_experts, rows, (int)(n / 2), out, out_scale, st);
     return launch_status();
@@ -1100,16 +1148,17 @@ int moe355::gmm2_pairs_impl(const int8_t* x, const float* per_token_scale, const
     a.pair_gather = 0;
     hipEvent_t ev0, ev1;
     take_profile_events(ev0, ev1);
-    const int64_t units = (int64_t)pair_places(a) * (n / 64);
+    // a wavefront per unit when there are enough units and K is short, and the units of an expert come in fours (a
+    // workgroup collects the pairs of one expert)
+    const bool unsplit = (int64_t)num_experts * (n / 64) >= 2048 && k < 2048 && (n / 64) % 4 == 0;
+    const int64_t units = (int64_t)pair_places(a, unsplit ? 2048 : 768) * (n / 64);
     const dim3 by_four((unsigned)((units + 3) / 4));
     if (y) {
         const unsigned lds = (unsigned)(32 * (k + 16));
         auto kernel = gmm_stream_kernel<EPI_DEQUANT, 1, 4, 2, false, true, true, true>;
         if (ev0 || ev1) hipExtLaunchKernelGGL(kernel, by_four, dim3(256), lds, st, ev0, ev1, 0, a);
         else hipLaunchKernelGGL(kernel, by_four, dim3(256), lds, st, a);
-    } else if (units >= 2048 && k < 2048 && (n / 64) % 4 == 0) {
-        // as the sorted form chooses: a wavefront per unit when there are enough units and K is short, and the units
-        // of an expert come in fours (a workgroup collects the pairs of one expert)
+    } else if (unsplit && units >= 2048) {
         launch_gemm(gmm_stream_kernel<EPI_DEQUANT, 1, 4, 2, false, true, true>, by_four, st, a, ev0, ev1);
     } else {
         launch_gemm(gmm_stream_kernel<EPI_DEQUANT, 4, 4, 3, false, true, true>, dim3((unsigned)units), st, a, ev0, ev1);

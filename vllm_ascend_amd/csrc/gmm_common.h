@@ -38,9 +38,10 @@ struct GmmArgs {
     // order) or in row f, and its result goes to row f.
     const int32_t* pair_ids;
     int pair_k, pair_gather;
-    // > 0: the grid has pair_slots places instead of E, and place s works on the s-th expert that has pairs (fewer
-    // pairs than experts: most experts are idle)
-    int pair_slots;
+    // The grid has a place for each of the experts [0, pair_first), and pair_slots places behind them: slot s works on
+    // the s-th of the other experts that have pairs (the idle ones cost nothing).  pair_extra > 0: those work on the
+    // first 32 rows of their expert, and as many more places at the end of the grid on further blocks of 32 rows.
+    int pair_first, pair_slots, pair_extra;
     // the same for a sorted activation with fewer rows than experts: place s works on the s-th expert whose group
     // is not empty
     int gl_slots;
