@@ -1065,7 +1065,8 @@ static int pair_places(GmmArgs& a, int resident_units)
         if (a.pair_first > a.E) a.pair_first = a.E;
         const int rest = a.E - a.pair_first;
         a.pair_slots = a.R < (int64_t)rest ? (int)a.R : rest;
-        if (a.N / 64 < 48) a.pair_extra = (int)(a.R / 33);
+        // an expert of c rows has (c - 1) / 32 further blocks: over all experts at most (R - 1) / 32
+        if (a.N / 64 < 48) a.pair_extra = (int)((a.R - 1) / 32);
     }
     return a.pair_first + a.pair_slots + a.pair_extra;
 }
