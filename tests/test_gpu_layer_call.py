@@ -30,10 +30,13 @@ def test_one_call_equals_the_operators(name, tokens):
     assert torch.equal(got, layer.forward_impl(x, logits).routed_out)
 
 
-@pytest.mark.parametrize("tokens", [1, 8, 40, 300])
-@pytest.mark.parametrize("overlap", [False, True])
-def test_shared_expert_in_the_call(tokens, overlap):
+# the form for a few tokens, the shared expert in the pair-order launches (blocks of 32 tokens; a clamp of its own; an
+# alpha that only its own operator knows), and the sorted path
+@pytest.mark.parametrize("tokens", [1, 8, 32, 33, 64, 96, 127, 300])
+@pytest.mark.parametrize("overlap, limit, alpha", [(False, 0.0, 1.0), (True, 0.7, 1.0), (True, 0.7, 1.5)])
+def test_shared_expert_in_the_call(tokens, overlap, limit, alpha):
     cfg, layer, x, logits = _pair("c4_small", tokens, shared=True, overlap=overlap)
+    layer.shared_experts.swiglu_limit, layer.shared_experts.swiglu_alpha = limit, alpha
     want = layer.forward_impl(x, logits).routed_out
     for _ in range(3):
         assert torch.equal(layer(x, logits), want)

@@ -114,10 +114,17 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
     // pair order: the grid has slots instead of a place per expert (an idle expert's workgroup only finds that out, but
     // it still costs its dispatch -- 28,000 of them are 150 us -- and the weights it has requested by then), and slot s
     // belongs to the s-th expert that has pairs; the workgroups that start first have places (pair_places below)
-    const int places = PAIRS ? a.pair_first + a.pair_slots + a.pair_extra : (!EARLY && a.gl_slots > 0) ? a.gl_slots : a.E;
+    const int places = PAIRS ? a.sh_blocks + a.pair_first + a.pair_slots + a.pair_extra : (!EARLY && a.gl_slots > 0) ? a.gl_slots : a.E;
     if (unit >= (int64_t)places * upe) return;  // KSPLIT == 1: no barriers below; KSPLIT == 4: whole workgroup leaves
     int e = (int)(unit / upe);
     const int p = (int)(unit % upe);
+    int block = 0;        // pair order: which 32 rows of the expert
+    bool shared = false;  // ... and whether it is the shared one (the same answer in all four wavefronts)
+    if constexpr (PAIRS) {
+        shared = e < a.sh_blocks;
+        if (shared) block = e;
+        e = shared ? 0 : e - a.sh_blocks;
+    }
     const int nb0 = (EPI == EPI_SWIGLU) ? p : 2 * p;
     const int nb1 = (EPI == EPI_SWIGLU) ? p + upe : 2 * p + 1;
 
@@ -145,9 +152,10 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
             pid[c] = (c * 64 < Q && f < (int)a.R) ? a.pair_ids[f] : -1;
         }
     }
-    int block = 0;  // pair order: which 32 rows of the expert
     if constexpr (PAIRS) {
-        if (e >= a.pair_first + a.pair_slots) {
+        if (shared) {
+            // nothing to look up
+        } else if (e >= a.pair_first + a.pair_slots) {
             // further blocks of experts with more than 32 rows, in the order of the experts: the pairs of every expert
             // are counted in LDS and every wavefront walks the counts, 64 experts at a time
             for (int i = threadIdx.x; i < a.E; i += 256) red[i] = 0;
@@ -210,7 +218,7 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
             if (e < 0) return;
         }
     }
-    const int8_t* we = expert_weights(a, e);
+    const int8_t* we = (PAIRS && shared) ? a.sh_w : expert_weights(a, e);
     const int8_t* w0 = we + ((int64_t)nb0 * KB) * 1024 + lane * 16;
     const int8_t* w1 = we + ((int64_t)nb1 * KB) * 1024 + lane * 16;
 
@@ -233,7 +241,10 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
     if constexpr (EARLY) load_weights(kb_begin);
 
     int64_t row0 = 0, row1 = 0;
-    if constexpr (PAIRS) {
+    if (PAIRS && shared) {
+        row0 = 32 * block;
+        row1 = row0 + 32 < a.sh_rows ? row0 + 32 : a.sh_rows;
+    } else if constexpr (PAIRS) {
         const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
         bool mine[4];
         int cnt = 0;
@@ -286,7 +297,7 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
             cs0[i] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
             cs1[i] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
             if constexpr (EPI != EPI_I32) {
-                const float* cs = expert_scales(a, e);
+                const float* cs = (PAIRS && shared) ? a.sh_scale : expert_scales(a, e);
                 const int ch = quad_channel(KSPLIT == 1 ? q_first + i : wave, lane);
                 cs0[i] = gload4f(cs + nb0 * 32 + ch);
                 cs1[i] = gload4f(cs + nb1 * 32 + ch);
@@ -300,8 +311,14 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
         using Index = std::conditional_t<PAIRS, int32_t, int64_t>;  // at most 1024 rows in pair order
         Index row, src;  // where the row's result goes, where its values lie
         if constexpr (PAIRS) {
-            row = plist[valid ? r0 + tok : 0];
-            src = a.pair_gather ? row / a.pair_k : row;
+            if (shared) {
+                const int t = valid ? (int)r0 + tok : (int)row0;
+                row = (int)a.R + t;
+                src = a.pair_gather ? t : row;
+            } else {
+                row = plist[valid ? r0 + tok : 0];
+                src = a.pair_gather ? row / a.pair_k : row;
+            }
         } else {
             row = r0 + tok;
             src = a.row_src ? (int64_t)a.row_src[valid ? row : row0] : row;
@@ -406,7 +423,8 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
                     }
                 }
             } else {
-                epilogue_run<EPI>(a, row, valid, nb0 * 32 + ch, nb1 * 32 + ch, g, u, rs, cs0[0], cs1[0]);
+                epilogue_run<EPI>(a, row, valid, nb0 * 32 + ch, nb1 * 32 + ch, g, u, rs, cs0[0], cs1[0],
+                                  PAIRS && shared);
             }
             __syncthreads();
         } else {
@@ -416,7 +434,8 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
                 int g[4] = {c0[4 * q], c0[4 * q + 1], c0[4 * q + 2], c0[4 * q + 3]};
                 int u[4] = {c1[4 * q], c1[4 * q + 1], c1[4 * q + 2], c1[4 * q + 3]};
                 const int ch = quad_channel(q, lane);
-                epilogue_run<EPI>(a, row, valid, nb0 * 32 + ch, nb1 * 32 + ch, g, u, rs, cs0[q % NQ], cs1[q % NQ]);
+                epilogue_run<EPI>(a, row, valid, nb0 * 32 + ch, nb1 * 32 + ch, g, u, rs, cs0[q % NQ], cs1[q % NQ],
+                                  PAIRS && shared);
             }
         }
     }
@@ -431,7 +450,7 @@ template <int NV>
 __global__ __launch_bounds__(256) void swiglu_requant_kernel(const float* __restrict__ y,
                                                              const int64_t* __restrict__ gl, int gl_type, int E,
                                                              int64_t R, int I, int8_t* __restrict__ q,
-                                                             float* __restrict__ qs)
+                                                             float* __restrict__ qs, int64_t shared_from)
 {
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
@@ -469,7 +488,8 @@ __global__ __launch_bounds__(256) void swiglu_requant_kernel(const float* __rest
         }
     }
     amax = wave_max(amax);
-    const float s = amax / 127.0f;
+    const bool shared = row >= shared_from;
+    const float s = shared ? amax * (float)(1.0 / 127.0) : amax / 127.0f;
     const float inv = 1.0f / s;
     if (lane == 0) qs[row] = (amax == 0.0f) ? 0.0f : s;
     uint32_t* qr = (uint32_t*)(q + row * I);
@@ -477,7 +497,7 @@ __global__ __launch_bounds__(256) void swiglu_requant_kernel(const float* __rest
         uint32_t pk = 0u;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            int8_t b = (amax == 0.0f) ? (int8_t)0 : sat_rint_i8(v[j] * inv);
+            int8_t b = (amax == 0.0f) ? (int8_t)0 : sat_rint_i8(shared ? v[j] / s : v[j] * inv);
             pk |= (uint32_t)(uint8_t)b << (8 * j);
         }
         return pk;
@@ -494,11 +514,11 @@ __global__ __launch_bounds__(256) void swiglu_requant_kernel(const float* __rest
 }
 
 void launch_swiglu_requant(const float* y, const int64_t* gl, int gl_type, int E, int64_t R, int I, int8_t* q,
-                           float* qs, hipStream_t st)
+                           float* qs, hipStream_t st, int64_t shared_from)
 {
     const dim3 grid((unsigned)((R + 3) / 4));
 #define MOE355_REQUANT(NV_) \
-    hipLaunchKernelGGL(swiglu_requant_kernel<NV_>, grid, dim3(256), 0, st, y, gl, gl_type, E, R, I, q, qs)
+    hipLaunchKernelGGL(swiglu_requant_kernel<NV_>, grid, dim3(256), 0, st, y, gl, gl_type, E, R, I, q, qs, shared_from)
     if (I <= 4 * 256) MOE355_REQUANT(4);
     else if (I <= 8 * 256) MOE355_REQUANT(8);
     else if (I <= 16 * 256) MOE355_REQUANT(16);
@@ -1061,14 +1081,15 @@ static int pair_places(GmmArgs& a, int resident_units)
     a.pair_first = a.E;
     a.pair_slots = a.pair_extra = 0;
     if (a.E <= kPairExperts) {
-        a.pair_first = a.R > 2 * (int64_t)a.E ? resident_units / (a.N / 64) : 0;
+        a.pair_first = a.R > 2 * (int64_t)a.E ? resident_units / (a.N / 64) - a.sh_blocks : 0;
         if (a.pair_first > a.E) a.pair_first = a.E;
+        if (a.pair_first < 0) a.pair_first = 0;
         const int rest = a.E - a.pair_first;
         a.pair_slots = a.R < (int64_t)rest ? (int)a.R : rest;
         // an expert of c rows has (c - 1) / 32 further blocks: over all experts at most (R - 1) / 32
         if (a.N / 64 < 48) a.pair_extra = (int)((a.R - 1) / 32);
     }
-    return a.pair_first + a.pair_slots + a.pair_extra;
+    return a.sh_blocks + a.pair_first + a.pair_slots + a.pair_extra;
 }
 
 extern "C" size_t moe355_gmm1_swiglu_quant_pairs_workspace(int64_t num_tokens, int top_k, int64_t n)
@@ -1081,7 +1102,7 @@ extern "C" size_t moe355_gmm1_swiglu_quant_pairs_workspace(int64_t num_tokens, i
 // tensor (w.one) or per-expert tensors (w.list and w.scale_list).
 int moe355::gmm1_pairs_impl(const int8_t* x, const float* x_scale, const int32_t* topk_ids, int64_t num_tokens,
                             int top_k, const PairWeights& w, int64_t k, int64_t n, int num_experts, float swiglu_limit,
-                            float* y, int8_t* out, float* out_scale, void* stream)
+                            float* y, int8_t* out, float* out_scale, void* stream, const PairShared* shared)
 {
     if (num_tokens < 0 || top_k <= 0 || k <= 0 || n <= 0 || num_experts <= 0) return MOE355_E_ARG;
     if (num_tokens == 0) return MOE355_OK;
@@ -1107,11 +1128,13 @@ int moe355::gmm1_pairs_impl(const int8_t* x, const float* x_scale, const int32_t
     a.pair_ids = topk_ids;
     a.pair_k = top_k;
     a.pair_gather = 1;
+    if (shared) shared->into(a, (int)num_tokens);
     hipEvent_t ev0, ev1;
     take_profile_events(ev0, ev1);
     const int64_t units = (int64_t)pair_places(a, 768) * (n / 64);
     launch_gemm(gmm_stream_kernel<EPI_SWIGLU, 4, 4, 3, false, true, true>, dim3((unsigned)units), st, a, ev0, ev1);
-    if (out) launch_swiglu_requant(y, nullptr, 0, num_experts, rows, (int)(n / 2), out, out_scale, st);
+    if (out)
+        launch_swiglu_requant(y, nullptr, 0, num_experts, rows + a.sh_rows, (int)(n / 2), out, out_scale, st, rows);
     return launch_status();
 }
 
@@ -1119,7 +1142,7 @@ int moe355::gmm1_pairs_impl(const int8_t* x, const float* x_scale, const int32_t
 // gate_up GEMM (y), which the workgroups then re-quantise themselves
 int moe355::gmm2_pairs_impl(const int8_t* x, const float* per_token_scale, const float* y, const PairWeights& w,
                             const int32_t* topk_ids, int64_t num_tokens, int top_k, int64_t k, int64_t n,
-                            int num_experts, void* out, int out_dtype, void* stream)
+                            int num_experts, void* out, int out_dtype, void* stream, const PairShared* shared)
 {
     if (num_tokens < 0 || top_k <= 0 || k <= 0 || n <= 0 || num_experts <= 0) return MOE355_E_ARG;
     if (out_dtype != MOE355_DT_BF16 && out_dtype != MOE355_DT_F16) return MOE355_E_UNSUPPORTED;
@@ -1147,6 +1170,7 @@ int moe355::gmm2_pairs_impl(const int8_t* x, const float* per_token_scale, const
     a.pair_ids = topk_ids;
     a.pair_k = top_k;
     a.pair_gather = 0;
+    if (shared && !y) shared->into(a, (int)num_tokens);
     hipEvent_t ev0, ev1;
     take_profile_events(ev0, ev1);
     // a wavefront per unit when there are enough units and K is short, and the units of an expert come in fours (a

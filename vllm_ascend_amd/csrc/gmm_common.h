@@ -42,6 +42,13 @@ struct GmmArgs {
     // the s-th of the other experts that have pairs (the idle ones cost nothing).  pair_extra > 0: those work on the
     // first 32 rows of their expert, and as many more places at the end of the grid on further blocks of 32 rows.
     int pair_first, pair_slots, pair_extra;
+    // Pair order with the shared expert in the same launch: sh_blocks places in front of the others, place b on rows
+    // 32 b .. of the sh_rows tokens.  Token t's values lie in row t (pair_gather) or R + t of x, its result goes to row
+    // R + t.  Its weights have the shape of a routed expert's.
+    int sh_blocks, sh_rows;
+    const int8_t* sh_w;
+    const float* sh_scale;
+    float sh_limit;
     // the same for a sorted activation with fewer rows than experts: place s works on the s-th expert whose group
     // is not empty
     int gl_slots;
@@ -97,9 +104,10 @@ __device__ __forceinline__ v4i mfma_i8_16(v4i a, v4i b, v4i c)
 // rs: the row's token scale; s0 / s1: the channel scales of the two runs.  The caller loads them before its
 // K loop: a load issued here, behind the stores of an earlier run, would wait for those stores (the memory
 // counter retires in order), one store round trip per run.
+// shared (SwiGLU only): the shared expert's operator multiplies by the channel scale first, then by the token scale.
 template <int EPI>
 __device__ __forceinline__ void epilogue_run(const GmmArgs& a, int64_t row, bool valid, int c0, int c1, const int* g,
-                                             const int* u, float rs, v4f s0, v4f s1)
+                                             const int* u, float rs, v4f s0, v4f s1, bool shared = false)
 {
     if (!valid) return;
     if constexpr (EPI == EPI_I32) {
@@ -120,15 +128,16 @@ __device__ __forceinline__ void epilogue_run(const GmmArgs& a, int64_t row, bool
     } else {
         // tile 0 = gate, tile 1 = the matching up tile (c1 = c0 + N/2)
         const int I = a.N >> 1;
+        const float limit = shared ? a.sh_limit : a.limit;
         v4f yv;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            float gg = ((float)g[j] * rs) * s0[j];
-            float uu = ((float)u[j] * rs) * s1[j];
-            if (a.limit > 0.0f) {
-                gg = gg > a.limit ? a.limit : gg;
-                uu = uu > a.limit ? a.limit : uu;
-                uu = uu < -a.limit ? -a.limit : uu;
+            float gg = ((float)g[j] * (shared ? s0[j] : rs)) * (shared ? rs : s0[j]);
+            float uu = ((float)u[j] * (shared ? s1[j] : rs)) * (shared ? rs : s1[j]);
+            if (limit > 0.0f) {
+                gg = gg > limit ? limit : gg;
+                uu = uu > limit ? limit : uu;
+                uu = uu < -limit ? -limit : uu;
             }
             yv[j] = m_silu(gg) * uu;
         }
@@ -151,7 +160,9 @@ __device__ __forceinline__ bool expert_in_launch(const GmmArgs& a, int64_t m)
 void take_profile_events(hipEvent_t& start, hipEvent_t& stop);
 
 // SwiGLU values y fp32 [R, I] -> per-row absmax -> int8 + scale (defined in gmm.hip).
+// Rows from shared_from on are the shared expert's: its operator's quantiser (scale = max * float(1/127), q = rint(v /
+// scale)) instead of the routed experts'.
 void launch_swiglu_requant(const float* y, const int64_t* gl, int gl_type, int E, int64_t R, int I, int8_t* q,
-                           float* qs, hipStream_t st);
+                           float* qs, hipStream_t st, int64_t shared_from = INT64_MAX);
 
 }  // namespace moe355

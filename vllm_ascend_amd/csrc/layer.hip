@@ -57,6 +57,7 @@ struct Forms {
     bool few;      // a few tokens: two launches behind the gating (few.hip)
     bool pairs;    // pair order
     bool requant;  // ... with the re-quantisation inside the down GEMM
+    bool merged;   // ... and the shared expert in the two GEMM launches
     bool small;    // sorted, gating + sort + quantisation in one launch
 };
 
@@ -113,6 +114,8 @@ Forms forms_of(const moe355_layer& l, int64_t T)
     f.pairs = l.weights != W_INT4 && l.pair_order &&
               moe355_pair_order(T, l.top_k, l.num_experts, l.num_experts, l.hidden, l.intermediate);
     f.requant = f.pairs && moe355_gmm2_requant_pairs_supported(T, l.top_k, l.hidden, l.intermediate, l.num_experts);
+    f.merged = f.pairs && !f.requant && l.shared && l.shared_intermediate == l.intermediate && l.shared_alpha == 1.0f &&
+               l.shared_beta == 0.0f;
     f.small = !f.pairs && l.sync_counter && moe355_route_quant_small_supported(T, l.top_k, l.num_experts);
     return f;
 }
@@ -143,12 +146,12 @@ Buffers lay_out(const moe355_layer& l, const Forms& f, int64_t T, void* base)
         b.total = a.used;
         return b;
     }
-    b.q1 = a.take<int8_t>((size_t)R * I);
-    b.q1_scale = a.take<float>((size_t)R * 4);
+    const int64_t rows = R + (f.merged ? T : 0);
+    b.q1 = a.take<int8_t>((size_t)rows * I);
+    b.q1_scale = a.take<float>((size_t)rows * 4);
     if (f.pairs) {
-        b.mlp_bytes = moe355_gmm1_swiglu_quant_pairs_workspace(T, l.top_k, 2 * I);
-        b.mlp_ws = a.take<void>(b.mlp_bytes);
-        b.o = a.take<void>((size_t)R * H * 2);
+        b.mlp_ws = a.take<void>((size_t)rows * I * 4);
+        b.o = a.take<void>((size_t)rows * H * 2);
     } else {
         b.dst = a.take<int32_t>((size_t)R * 4);
         b.row_token = a.take<int32_t>((size_t)R * 4);
@@ -162,7 +165,9 @@ Buffers lay_out(const moe355_layer& l, const Forms& f, int64_t T, void* base)
         b.gmm2_bytes = l.weights == W_INT4 ? 0 : moe355_gmm2_dequant_workspace(R, H, I, E);
         b.gmm2_ws = a.take<void>(b.gmm2_bytes);
     }
-    if (l.shared) {
+    if (f.merged) {
+        b.sh_out = (char*)b.o + (size_t)R * H * 2;
+    } else if (l.shared) {
         const int64_t S = l.shared_intermediate;
         b.sh_acc = a.take<int32_t>((size_t)T * 2 * S * 4);
         b.sh_bytes = moe355_gmm_i32_workspace(T, 2 * S, H, 1);
@@ -261,11 +266,12 @@ int routed_pairs(const moe355_layer& l, const Forms& f, const Buffers& b, int64_
         w2.scale = (const float*)l.s2;
     }
     float* y = (float*)b.mlp_ws;
+    const PairShared sh13 = {l.shared_w13, l.shared_s13, l.shared_limit}, sh2 = {l.shared_w2, l.shared_s2};
     int rc = gmm1_pairs_impl(b.xq, b.x_scale, b.topk_ids, T, l.top_k, w13, H, 2 * I, l.num_experts, l.swiglu_limit, y,
-                             f.requant ? nullptr : b.q1, b.q1_scale, st);
+                             f.requant ? nullptr : b.q1, b.q1_scale, st, f.merged ? &sh13 : nullptr);
     if (rc != MOE355_OK) return rc;
     return gmm2_pairs_impl(b.q1, b.q1_scale, f.requant ? y : nullptr, w2, b.topk_ids, T, l.top_k, I, H, l.num_experts,
-                           b.o, l.x_dtype, st);
+                           b.o, l.x_dtype, st, f.merged ? &sh2 : nullptr);
 }
 
 int routed_sorted(const moe355_layer& l, const Buffers& b, int64_t T, bool tiles_ready, void* st)
@@ -339,7 +345,10 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
 
     ForkJoinLease lease;
     bool joined = true;
-    if (l.shared == 2) {
+    if (f.merged) {
+        // in the GEMM launches of the routed experts, whatever stream it was meant for: 45 us of launches of its own
+        // become the time of its weights
+    } else if (l.shared == 2) {
         hipStream_t side = (hipStream_t)l.shared_stream, main = (hipStream_t)stream;
         if (!lease.take() || hipEventRecord(lease.fj.fork, main) != hipSuccess ||
             hipStreamWaitEvent(side, lease.fj.fork, 0) != hipSuccess)

@@ -41,12 +41,30 @@ struct PairWeights {
     bool aligned() const { return !((uintptr_t)one & 15) && !((uintptr_t)scale & 15); }
 };
 
+// The shared expert in the two pair-order launches (one GEMM each): tensors of a routed expert's shape.
+struct PairShared {
+    const int8_t* w;
+    const float* scale;
+    float limit = 0.0f;
+    template <typename Args>
+    void into(Args& a, int num_tokens) const
+    {
+        a.sh_w = w;
+        a.sh_scale = scale;
+        a.sh_limit = limit;
+        a.sh_rows = num_tokens;
+        a.sh_blocks = (num_tokens + 31) / 32;
+    }
+};
+
+// with `shared`, y, out and out_scale hold num_tokens more rows (the shared expert's, in token order); the same for x,
+// per_token_scale and out of the second
 int gmm1_pairs_impl(const int8_t* x, const float* x_scale, const int32_t* topk_ids, int64_t num_tokens, int top_k,
                     const PairWeights& w, int64_t k, int64_t n, int num_experts, float swiglu_limit, float* y,
-                    int8_t* out, float* out_scale, void* stream);
+                    int8_t* out, float* out_scale, void* stream, const PairShared* shared = nullptr);
 int gmm2_pairs_impl(const int8_t* x, const float* per_token_scale, const float* y, const PairWeights& w,
                     const int32_t* topk_ids, int64_t num_tokens, int top_k, int64_t k, int64_t n, int num_experts,
-                    void* out, int out_dtype, void* stream);
+                    void* out, int out_dtype, void* stream, const PairShared* shared = nullptr);
 int gmm1_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list, const float* weight_scale,
               const float* const* scale_list, const float* x_scale, const int64_t* group_list, int group_list_type,
               int64_t rows, int64_t k, int64_t n, int num_experts, float swiglu_limit, int8_t* out, float* out_scale,
