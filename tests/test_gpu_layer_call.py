@@ -89,6 +89,17 @@ def test_hot_experts_in_pair_order(tokens, rest):
     assert torch.equal(layer(x, hot), want)  # against the operators on the sorted order
 
 
+# int4 weights in pair order (up to 48 tokens): blocks of 16 and 32 rows, one scale per channel or per group, hot and idle experts
+@pytest.mark.parametrize("tokens", [1, 16, 17, 32, 33, 48, 49])
+@pytest.mark.parametrize("name", ["c5_small", "c5_small_perchannel"])
+def test_int4_pair_order(name, tokens):
+    cfg, layer, x, logits = _pair(name, tokens)
+    hot = logits[:1].expand(tokens, -1).contiguous()
+    hot[::5] = logits[::5]
+    for lg in (logits, hot):
+        assert torch.equal(layer(x, lg), layer.forward_impl(x, lg).routed_out)
+
+
 def test_the_call_follows_the_layer():
     """Options that change between calls, and a copied layer."""
     cfg, layer, x, logits = _pair("c2_small", 40)

@@ -14,6 +14,7 @@
 #include <type_traits>
 
 #include "gmm_common.h"
+#include "layer_parts.h"
 
 namespace moe355 {
 
@@ -423,6 +424,220 @@ __global__ __launch_bounds__(256, 2) void gmm_w4_stream_kernel(W4Args p)
     }
 }
 
+// ------------------------------------------------------------------ decode batches, pair order
+// The same product for at most kW4PairMax (token, slot) pairs whose ids come straight from the gate: an expert has one to
+// a few rows, so nothing is sorted (a row belongs to its pair throughout, as in gmm_stream_kernel's pair order), nothing
+// is staged and no wavefront waits for another one inside the K loop.  One wavefront per pair of 32-channel tiles over
+// the whole K range (the fp32 sum over the scale groups has one fixed order); tokens are the 16 columns of
+// v_mfma_i32_16x16x64_i8 (one or two times, for experts of more than 16 rows), so accumulators and fp32 sums are 16
+// registers each instead of 64 and the fold is a quarter of the work.  HBM-bound: DeepSeek-V3 shape, us a layer call
+// against the sorted chunks, uniform routing, 1 / 4 / 16 / 32 tokens 59 / 136 / 382 / 557 against 86 / 157 / 412 / 593
+// (16 tokens: 2.3 GB at 6.4 TB/s), Zipf(1.1), 24 / 32 / 48 tokens 148 / 177 / 217 against 163 / 206 / 227.  A ring of
+// 8, 10 or 12 blocks 389 to 393 us at 16 tokens, three wavefronts per SIMD the same as two and 191 us at 32 under Zipf.
+// An int4 tile (lane = channel l % 32, K half l / 32; low nibbles K 0..31, high nibbles K 32..63) becomes the operands of
+// its two groups of 16 channels by one exchange: rows of 16 lanes 1 and 3 of the low-nibble register against rows 0 and 2
+// of the high-nibble register (v_permlane16_swap) leave channels 0..15 in one register and 16..31 in the other, row r of
+// either holding the K slice 0, 32, 16 or 48 + 0..15 for r = 0, 1, 2, 3.  The tokens are read in that order.
+constexpr int kW4PairMax = 1024;
+constexpr int kW4PairTokens = 48;  // see w4_pairs_supported
+constexpr int kW4PairExperts = 2048;
+constexpr int kW4PairRing = 6;     // K blocks of weights and tokens in flight per wavefront
+
+__device__ __forceinline__ void w4_operands(v4i v, v4i& first, v4i& second)
+{
+    const v4i lo = nib_lo(v), hi = nib_hi(v);
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const auto r = __builtin_amdgcn_permlane16_swap((unsigned)lo[d], (unsigned)hi[d], false, false);
+        first[d] = (int)r[0];
+        second[d] = (int)r[1];
+    }
+}
+
+template <int EPI>
+__global__ __launch_bounds__(256, 2) void gmm_w4_pairs_kernel(W4Args p)
+{
+    const GmmArgs& a = p.g;
+    __shared__ uint16_t plist[kW4PairMax];       // the expert's pairs, ascending
+    __shared__ int32_t pcount[4];
+    __shared__ uint32_t pmap[kW4PairExperts / 32];  // one bit per expert that has pairs
+    __shared__ float Ss[4][kW4LdsGroups * 64];      // group scales of every wavefront's 64 channels
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    const int NB = a.N >> 5, KB64 = a.K >> 6;
+    const int upe = NB >> 1, quads = (upe + 3) >> 2;
+    const int slot = (int)(blockIdx.x / quads);
+    const int pi_raw = (int)(blockIdx.x % quads) * 4 + wave;
+    const bool have = pi_raw < upe;
+    const int pi = have ? pi_raw : 0;
+
+    // the slot's expert: the slot-th one that has pairs (see gmm_stream_kernel)
+    const int Q = (((int)a.R + 255) >> 8) << 6;
+    int pid[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const int f = wave * Q + c * 64 + lane;
+        pid[c] = (c * 64 < Q && f < (int)a.R) ? a.pair_ids[f] : -1;
+    }
+    if (threadIdx.x < kW4PairExperts / 32) pmap[threadIdx.x] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        if (pid[c] >= 0 && pid[c] < a.E) atomicOr(&pmap[pid[c] >> 5], 1u << (pid[c] & 31));
+    __syncthreads();
+    const uint32_t bits = pmap[lane];
+    const int cnt = __popc(bits);
+    const int incl = wave_scan_inclusive_i32(cnt);
+    const bool has = slot >= incl - cnt && slot < incl;
+    const unsigned long long holder = __ballot(has);
+    if (holder == 0ull) return;  // fewer experts with pairs than slots (the same answer in all four wavefronts)
+    uint32_t t = bits;
+    for (int i = has ? slot - (incl - cnt) : 0; i > 0; --i) t &= t - 1;
+    const int e = __builtin_amdgcn_readlane(lane * 32 + (t ? __builtin_ctz(t) : 0), __builtin_ctzll(holder));
+
+    const int nb0 = (EPI == EPI_SWIGLU) ? pi : 2 * pi;
+    const int nb1 = (EPI == EPI_SWIGLU) ? pi + upe : 2 * pi + 1;
+    const uint8_t* we = p.w4 + (int64_t)e * NB * KB64 * 1024;
+    const uint8_t* w0 = we + (int64_t)nb0 * KB64 * 1024 + lane * 16;
+    const uint8_t* w1 = we + (int64_t)nb1 * KB64 * 1024 + lane * 16;
+    const int n_groups = a.K / p.group, steps_per_group = p.group >> 6;
+    {
+        const float* gs = p.gscale + (int64_t)e * n_groups * a.N;
+        const int ch = lane < 32 ? nb0 * 32 + lane : nb1 * 32 + (lane - 32);
+        for (int g0 = 0; g0 < n_groups; g0 += 8) {  // eight loads in flight at a time
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = gs[(int64_t)(g0 + j < n_groups ? g0 + j : n_groups - 1) * a.N + ch];
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (g0 + j < n_groups) Ss[wave][(g0 + j) * 64 + lane] = v[j];
+        }
+    }
+    // the expert's pairs
+    int rows = 0;
+    {
+        const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+        bool mine[4];
+        int n = 0;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            mine[c] = pid[c] == e;
+            n += __popcll(__ballot(mine[c]));
+        }
+        if (lane == 0) pcount[wave] = n;
+        __syncthreads();
+        int base = 0;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            if (w < wave) base += pcount[w];
+            rows += pcount[w];
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const unsigned long long m = __ballot(mine[c]);
+            if (mine[c]) plist[base + __popcll(m & below)] = (uint16_t)(wave * Q + c * 64 + lane);
+            base += __popcll(m);
+        }
+        __syncthreads();  // the last barrier
+    }
+    if (!have) return;
+
+    const int tok = lane & 15, r16 = lane >> 4;
+    const int slice = 16 * ((r16 >> 1) + 2 * (r16 & 1));  // K 0, 32, 16, 48 for rows 0..3
+    constexpr int D = kW4PairRing;
+    // one pass over the weights for NT blocks of 16 rows
+    auto pass = [&](auto blocks, int first) {
+        constexpr int NT = decltype(blocks)::value;
+        v4i a0[D], a1[D], tk[D][NT];
+        bool valid[NT];
+        int row[NT];  // where the row's result goes
+        uint32_t xo[NT];
+        float rs[NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            valid[n] = first + 16 * n + tok < rows;
+            row[n] = plist[valid[n] ? first + 16 * n + tok : 0];
+            const int src = a.pair_gather ? row[n] / a.pair_k : row[n];
+            xo[n] = (uint32_t)src * (uint32_t)a.K + slice;
+            rs[n] = a.row_scale[src];
+        }
+        auto request = [&](int s, int kb) {
+            const int k = kb < KB64 ? kb : KB64 - 1;  // past the end: a valid block that is never used
+            a0[s] = gload16_nt(w0 + (int64_t)k * 1024);
+            a1[s] = gload16_nt(w1 + (int64_t)k * 1024);
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+                tk[s][n] = valid[n] ? *(const v4i*)(a.x + (xo[n] + k * 64)) : (v4i){0, 0, 0, 0};
+        };
+        v4i c[NT][2][2];  // [token block][tile][16 channels]
+        float f[NT][2][2][4];
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    c[n][i][h] = (v4i){0, 0, 0, 0};
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) f[n][i][h][j] = 0.0f;
+                }
+        int in_group = 0, grp = 0;
+        auto step = [&](int s, int kb) {  // s = kb % D, compile time
+            v4i l0, h0, l1, h1;
+            w4_operands(a0[s], l0, h0);
+            w4_operands(a1[s], l1, h1);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                c[n][0][0] = mfma_i8_16(l0, tk[s][n], c[n][0][0]);
+                c[n][0][1] = mfma_i8_16(h0, tk[s][n], c[n][0][1]);
+                c[n][1][0] = mfma_i8_16(l1, tk[s][n], c[n][1][0]);
+                c[n][1][1] = mfma_i8_16(h1, tk[s][n], c[n][1][1]);
+            }
+            request(s, kb + D);
+            if (++in_group == steps_per_group) {  // f += float(acc / 16) * scale[e, grp, channel]
+                const float* sl = &Ss[wave][grp * 64 + 4 * r16];
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const v4f sc = *(const v4f*)(sl + 32 * i + 16 * h);
+#pragma unroll
+                        for (int n = 0; n < NT; ++n) {
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+                                f[n][i][h][j] = f[n][i][h][j] + (float)(c[n][i][h][j] >> 4) * sc[j];
+                            c[n][i][h] = (v4i){0, 0, 0, 0};
+                        }
+                    }
+                in_group = 0;
+                ++grp;
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < D; ++i) request(i, i);
+        const int kb_full = (KB64 / D) * D;
+        for (int kb = 0; kb < kb_full; kb += D) {
+#pragma unroll
+            for (int i = 0; i < D; ++i) step(i, kb + i);
+        }
+#pragma unroll
+        for (int i = 0; i < D - 1; ++i)
+            if (kb_full + i < KB64) step(i, kb_full + i);
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int ch = 16 * h + 4 * r16;
+                epilogue_run_w4<EPI>(a, row[n], valid[n], nb0 * 32 + ch, nb1 * 32 + ch, f[n][0][h], f[n][1][h], rs[n]);
+            }
+    };
+    if (rows <= 16) {
+        pass(std::integral_constant<int, 1>{}, 0);
+    } else {
+        for (int first = 0; first < rows; first += 32) pass(std::integral_constant<int, 2>{}, first);
+    }
+}
+
 // workgroups: an upper bound of the number of 64-row chunks (known on the host without reading the group
 // list) times the groups of four tile pairs
 static int64_t w4_blocks(int64_t rows, int num_experts, int64_t n)
@@ -552,6 +767,71 @@ extern "C" int moe355_gmm1_swiglu_quant_w4_gather(const int8_t* x, const float* 
     if (rows > 0 && !row_token) return MOE355_E_ARG;
     return gmm1_w4_impl(x, weight_nz4, weight_scale, group_size, bias, x_scale, group_list, group_list_type, rows, k,
                         n, num_experts, swiglu_limit, out, out_scale, workspace, workspace_bytes, stream, row_token);
+}
+
+// Up to 48 tokens: an expert has at most that many rows, two passes of 32.  With 64 tokens uniform routing would still
+// gain (844 -> 795 us), but skewed routing loses by the repeated passes of its hot experts (250 -> 270 us; 128 tokens
+// 327 -> 479 us), and the host cannot know.
+bool moe355::w4_pairs_supported(int64_t num_tokens, int top_k, int num_experts, int64_t hidden, int64_t intermediate,
+                                int64_t group13, int64_t group2)
+{
+    return num_tokens > 0 && num_tokens <= kW4PairTokens && num_tokens * top_k <= kW4PairMax && num_experts <= kW4PairExperts && group13 > 0 && group2 > 0 &&
+           hidden / group13 <= kW4LdsGroups && intermediate / group2 <= kW4LdsGroups;
+}
+
+// one GEMM in pair order: the gate_up one (y set: fp32 SwiGLU values, rows re-quantised into out) or the down one
+static W4Args w4_pair_args(const int8_t* x, const float* x_scale, const int32_t* topk_ids, int64_t num_tokens, int top_k,
+                           const uint8_t* w, const float* scale, int64_t group, int64_t k, int64_t n, int num_experts)
+{
+    W4Args p = {};
+    p.g.x = x;
+    p.g.R = num_tokens * top_k;
+    p.g.K = (int)k;
+    p.g.N = (int)n;
+    p.g.E = num_experts;
+    p.g.row_scale = x_scale;
+    p.g.pair_ids = topk_ids;
+    p.g.pair_k = top_k;
+    p.w4 = w;
+    p.gscale = scale;
+    p.group = (int)group;
+    return p;
+}
+
+static dim3 w4_pair_grid(const W4Args& p)
+{
+    const int64_t slots = p.g.R < (int64_t)p.g.E ? p.g.R : (int64_t)p.g.E;
+    return dim3((unsigned)(slots * ((p.g.N / 64 + 3) / 4)));
+}
+
+int moe355::gmm1_w4_pairs(const int8_t* x, const float* x_scale, const int32_t* topk_ids, int64_t num_tokens, int top_k,
+                          const uint8_t* w, const float* scale, int64_t group, int64_t k, int64_t n, int num_experts,
+                          float swiglu_limit, float* y, int8_t* out, float* out_scale, hipStream_t st)
+{
+    if (!x || !x_scale || !topk_ids || !w || !scale || !y || !out || !out_scale) return MOE355_E_ARG;
+    if (n % 64 != 0 || k % 64 != 0 || group % 64 != 0 || k % group != 0) return MOE355_E_SHAPE;
+    if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)y & 15)) return MOE355_E_SHAPE;
+    W4Args p = w4_pair_args(x, x_scale, topk_ids, num_tokens, top_k, w, scale, group, k, n, num_experts);
+    p.g.pair_gather = 1;
+    p.g.limit = swiglu_limit;
+    p.g.y = y;
+    hipLaunchKernelGGL((gmm_w4_pairs_kernel<EPI_SWIGLU>), w4_pair_grid(p), dim3(256), 0, st, p);
+    launch_swiglu_requant(y, nullptr, 0, num_experts, p.g.R, (int)(n / 2), out, out_scale, st);
+    return launch_status();
+}
+
+int moe355::gmm2_w4_pairs(const int8_t* x, const float* x_scale, const int32_t* topk_ids, int64_t num_tokens, int top_k,
+                          const uint8_t* w, const float* scale, int64_t group, int64_t k, int64_t n, int num_experts,
+                          void* out, int out_dtype, hipStream_t st)
+{
+    if (!x || !x_scale || !topk_ids || !w || !scale || !out) return MOE355_E_ARG;
+    if (n % 64 != 0 || k % 64 != 0 || group % 64 != 0 || k % group != 0) return MOE355_E_SHAPE;
+    if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)out & 7)) return MOE355_E_SHAPE;
+    W4Args p = w4_pair_args(x, x_scale, topk_ids, num_tokens, top_k, w, scale, group, k, n, num_experts);
+    p.g.out = (uint16_t*)out;
+    p.g.out_f16 = out_dtype == MOE355_DT_F16;
+    hipLaunchKernelGGL((gmm_w4_pairs_kernel<EPI_DEQUANT>), w4_pair_grid(p), dim3(256), 0, st, p);
+    return launch_status();
 }
 
 extern "C" int moe355_gmm2_dequant_w4(const int8_t* x, const uint8_t* weight_nz4, const float* scale,

@@ -111,10 +111,14 @@ Forms forms_of(const moe355_layer& l, int64_t T)
     f.few = l.weights != W_INT4 && l.pair_order && T <= 64 && l.top_k <= 64 &&
             moe355_gate_quant_supported(T, l.top_k, l.num_experts) && few_supported(few_args(l, Buffers{}, T));
     if (f.few) return f;
-    f.pairs = l.weights != W_INT4 && l.pair_order &&
-              moe355_pair_order(T, l.top_k, l.num_experts, l.num_experts, l.hidden, l.intermediate);
-    f.requant = f.pairs && moe355_gmm2_requant_pairs_supported(T, l.top_k, l.hidden, l.intermediate, l.num_experts);
-    f.merged = f.pairs && !f.requant && l.shared && l.shared_intermediate == l.intermediate && l.shared_alpha == 1.0f &&
+    if (l.weights == W_INT4)
+        f.pairs = l.pair_order && moe355_gate_quant_supported(T, l.top_k, l.num_experts) &&
+                  w4_pairs_supported(T, l.top_k, l.num_experts, l.hidden, l.intermediate, l.group13, l.group2);
+    else
+        f.pairs = l.pair_order && moe355_pair_order(T, l.top_k, l.num_experts, l.num_experts, l.hidden, l.intermediate);
+    const bool int8_pairs = f.pairs && l.weights != W_INT4;
+    f.requant = int8_pairs && moe355_gmm2_requant_pairs_supported(T, l.top_k, l.hidden, l.intermediate, l.num_experts);
+    f.merged = int8_pairs && !f.requant && l.shared && l.shared_intermediate == l.intermediate && l.shared_alpha == 1.0f &&
                l.shared_beta == 0.0f;
     f.small = !f.pairs && l.sync_counter && moe355_route_quant_small_supported(T, l.top_k, l.num_experts);
     return f;
@@ -253,6 +257,14 @@ int shared_expert(const moe355_layer& l, const Buffers& b, int64_t T, void* st)
 int routed_pairs(const moe355_layer& l, const Forms& f, const Buffers& b, int64_t T, void* st)
 {
     const int64_t H = l.hidden, I = l.intermediate;
+    if (l.weights == W_INT4) {
+        int rc = gmm1_w4_pairs(b.xq, b.x_scale, b.topk_ids, T, l.top_k, (const uint8_t*)l.w13, (const float*)l.s13,
+                               l.group13, H, 2 * I, l.num_experts, l.swiglu_limit, (float*)b.mlp_ws, b.q1, b.q1_scale,
+                               (hipStream_t)st);
+        if (rc != MOE355_OK) return rc;
+        return gmm2_w4_pairs(b.q1, b.q1_scale, b.topk_ids, T, l.top_k, (const uint8_t*)l.w2, (const float*)l.s2, l.group2,
+                             I, H, l.num_experts, b.o, l.x_dtype, (hipStream_t)st);
+    }
     PairWeights w13 = {}, w2 = {};
     if (l.weights == W_INT8_LIST) {
         w13.list = (const int8_t* const*)l.w13;

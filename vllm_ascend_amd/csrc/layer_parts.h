@@ -78,6 +78,16 @@ void* gmm1_tile_ws(void* workspace, int64_t rows, int64_t n);
 // tile maps (at most two) that a grouped product will look for in its workspace
 int gemm_tile_specs(int64_t rows, int64_t k, int64_t n, int num_experts, void* tile_ws, TileSpec* specs);
 
+// int4 weights, pair order (gmm_w4.hip)
+bool w4_pairs_supported(int64_t num_tokens, int top_k, int num_experts, int64_t hidden, int64_t intermediate,
+                        int64_t group13, int64_t group2);
+int gmm1_w4_pairs(const int8_t* x, const float* x_scale, const int32_t* topk_ids, int64_t num_tokens, int top_k,
+                  const uint8_t* w, const float* scale, int64_t group, int64_t k, int64_t n, int num_experts,
+                  float swiglu_limit, float* y, int8_t* out, float* out_scale, hipStream_t st);
+int gmm2_w4_pairs(const int8_t* x, const float* x_scale, const int32_t* topk_ids, int64_t num_tokens, int top_k,
+                  const uint8_t* w, const float* scale, int64_t group, int64_t k, int64_t n, int num_experts, void* out,
+                  int out_dtype, hipStream_t st);
+
 // moe355_route_map with the tile maps of the two products (nspecs of them, at most 4) built by the same launch where it
 // is one launch (returns 1 in *built then)
 int route_map_impl(const int32_t* expert_idx, int64_t num_tokens, int top_k, int num_experts, int tokens_num_type,
