@@ -42,6 +42,29 @@ def test_shared_expert_in_the_call(tokens, overlap, limit, alpha):
         assert torch.equal(layer(x, logits), want)
 
 
+# the shared expert on its own: up to 16 tokens on the kernels for a few tokens (its rows quantised in place, or by a
+# launch), beyond that on the dense products
+@pytest.mark.parametrize("tokens", [1, 8, 16, 17])
+@pytest.mark.parametrize("overlap", [False, True])
+@pytest.mark.parametrize("experts", ["sorted int8", "int4"])
+def test_shared_expert_beside_the_call(experts, overlap, tokens):
+    from vllm_ascend_amd.fused_moe.shared_experts import AscendSharedExperts
+
+    if experts == "int4":
+        cfg, layer, x, logits = _pair("c5_small", tokens)
+        g = torch.Generator().manual_seed(tokens)
+        w = [torch.randint(-127, 128, s, generator=g, dtype=torch.int8).to(DEV) for s in ((2048, cfg.H), (cfg.H, 1024))]
+        s = [(torch.rand(n, generator=g) * 0.009 + 0.001).to(DEV) for n in (2048, cfg.H)]
+        layer.shared_experts = AscendSharedExperts(w[0], s[0], w[1], s[1], swiglu_limit=0.7, multistream_overlap=overlap)
+    else:
+        cfg, layer, x, logits = _pair("c4_small", tokens, shared=True, overlap=overlap)
+        layer.use_pair_order = False
+    want = layer.forward_impl(x, logits).routed_out
+    for _ in range(3):
+        assert torch.equal(layer(x, logits), want)
+    assert layer._layer_plan.desc is not None
+
+
 @pytest.mark.parametrize("tokens", [2, 4, 60, 300])
 def test_weight_lists_and_expert_loads(tokens):
     cfg, layer, x, logits = _pair("c7_small", tokens, dynamic_eplb=True, collect_expert_load=True)

@@ -58,6 +58,7 @@ struct Forms {
     bool pairs;    // pair order
     bool requant;  // ... with the re-quantisation inside the down GEMM
     bool merged;   // ... and the shared expert in the two GEMM launches
+    bool shared_few;  // the shared expert alone on the kernels for a few tokens
     bool small;    // sorted, gating + sort + quantisation in one launch
 };
 
@@ -105,6 +106,20 @@ FewArgs few_args(const moe355_layer& l, const Buffers& b, int64_t T)
     return a;
 }
 
+// the shared expert on its own: no pairs
+FewArgs shared_args(const moe355_layer& l, const Buffers& b, int64_t T)
+{
+    FewArgs a = few_args(l, b, T);
+    a.R = 0;
+    a.k = 0;
+    a.load = nullptr;
+    a.y = (float*)b.sh_acc;
+    a.q1 = b.sh_q;
+    a.q1_scale = b.sh_q_scale;
+    a.out = (uint16_t*)b.sh_out;
+    return a;
+}
+
 Forms forms_of(const moe355_layer& l, int64_t T)
 {
     Forms f = {};
@@ -120,6 +135,7 @@ Forms forms_of(const moe355_layer& l, int64_t T)
     f.requant = int8_pairs && moe355_gmm2_requant_pairs_supported(T, l.top_k, l.hidden, l.intermediate, l.num_experts);
     f.merged = int8_pairs && !f.requant && l.shared && l.shared_intermediate == l.intermediate && l.shared_alpha == 1.0f &&
                l.shared_beta == 0.0f;
+    f.shared_few = l.shared && !f.merged && T <= 16 && few_supported(shared_args(l, Buffers{}, T));
     f.small = !f.pairs && l.sync_counter && moe355_route_quant_small_supported(T, l.top_k, l.num_experts);
     return f;
 }
@@ -173,6 +189,7 @@ Buffers lay_out(const moe355_layer& l, const Forms& f, int64_t T, void* base)
         b.sh_out = (char*)b.o + (size_t)R * H * 2;
     } else if (l.shared) {
         const int64_t S = l.shared_intermediate;
+        if (f.shared_few) b.ymax = a.take<float>((size_t)T * (S / 16) * 4);
         b.sh_acc = a.take<int32_t>((size_t)T * 2 * S * 4);
         b.sh_bytes = moe355_gmm_i32_workspace(T, 2 * S, H, 1);
         b.sh_ws = a.take<void>(b.sh_bytes);
@@ -240,8 +257,9 @@ struct ForkJoinLease {
 };
 
 // dense W8A8 MLP over all tokens, on the rows the routed experts quantised
-int shared_expert(const moe355_layer& l, const Buffers& b, int64_t T, void* st)
+int shared_expert(const moe355_layer& l, const Forms& f, const Buffers& b, int64_t T, void* st)
 {
+    if (f.shared_few) return few_forward(shared_args(l, b, T), (hipStream_t)st);
     const int64_t H = l.hidden, I = l.shared_intermediate;
     int rc = moe355_gmm_i32(b.xq, l.shared_w13, b.one_group, MOE355_GL_CUMSUM, T, H, 2 * I, 1, b.sh_acc, b.sh_ws,
                             b.sh_bytes, st);
@@ -365,12 +383,12 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
         if (!lease.take() || hipEventRecord(lease.fj.fork, main) != hipSuccess ||
             hipStreamWaitEvent(side, lease.fj.fork, 0) != hipSuccess)
             return MOE355_E_LAUNCH;
-        rc = shared_expert(l, b, T, side);
+        rc = shared_expert(l, f, b, T, side);
         // joined below even if a launch was refused: the caller frees the scratch in the order of its own stream
         if (hipEventRecord(lease.fj.join, side) != hipSuccess) return MOE355_E_LAUNCH;
         joined = false;
     } else if (l.shared == 1) {
-        rc = shared_expert(l, b, T, stream);
+        rc = shared_expert(l, f, b, T, stream);
     }
     bool tiles_ready = false;
     if (rc == MOE355_OK && !f.pairs && !f.small) {
