@@ -135,7 +135,11 @@ Forms forms_of(const moe355_layer& l, int64_t T)
     f.requant = int8_pairs && moe355_gmm2_requant_pairs_supported(T, l.top_k, l.hidden, l.intermediate, l.num_experts);
     f.merged = int8_pairs && !f.requant && l.shared && l.shared_intermediate == l.intermediate && l.shared_alpha == 1.0f &&
                l.shared_beta == 0.0f;
-    f.shared_few = l.shared && !f.merged && T <= 16 && few_supported(shared_args(l, Buffers{}, T));
+    // Up to 16 tokens the kernels for a few tokens run a shared expert in two or three launches instead of four.  On the
+    // side stream that pays from 8 tokens on: below, their many workgroups take more from the routed GEMM beside them
+    // than they save.  int4 layer of the DeepSeek-V3 shape, us a call, four launches against these: in line, 2 / 8 / 16
+    // tokens 110 / 257 / 405 against 99 / 248 / 397; side stream 97 / 251 / 398 against 100 / 250 / 391.
+    f.shared_few = l.shared && !f.merged && T <= 16 && (l.shared == 1 || T >= 8) && few_supported(shared_args(l, Buffers{}, T));
     f.small = !f.pairs && l.sync_counter && moe355_route_quant_small_supported(T, l.top_k, l.num_experts);
     return f;
 }
