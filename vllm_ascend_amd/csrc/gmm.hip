@@ -585,11 +585,17 @@ static void launch_gemm(KernelT kernel, dim3 grid, hipStream_t st, const GmmArgs
     else hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, a);
 }
 
-// Rows per expert decide the kernel: few rows -> weight streaming over single wavefronts; many -> LDS-tiled
-// MFMA kernel with 128-row tiles; in between, when K is long enough to amortise a tile's fill and epilogue, the
-// weight-streaming tiles (up to 256 rows) that fetch an expert's weights once.  The host only knows the mean; the
-// histogram may be skewed (real routers are), so next to the family chosen from the mean a second family covers
-// the experts that fall outside its range, picked expert by expert on the device (GemmPlan below).
+// Rows per expert decide the kernel: a handful -> weight streaming over single wavefronts; more -> LDS-tiled MFMA
+// kernel with 128-row tiles; many, when K is long enough to amortise a tile's fill and epilogue, the weight-streaming
+// tiles (up to 256 rows) that fetch an expert's weights once.  The host only knows the mean, and the histogram may be
+// skewed (real routers are): the 128-row tiles cost a cold expert little more than streaming does (a short tile that
+// is its expert's only one reads its weights once, past the caches) and a hot one a fraction of it, so they start early.
+// products small enough to stream below 1024 rows, large enough to split (see GemmPlan)
+static bool split_size(int64_t weights)
+{
+    return weights >= (1ll << 30) && weights < (9ll << 27);
+}
+
 static int tiled_bm(const GmmArgs& a)
 {
     if (a.K % 64 != 0) return 0;
@@ -601,28 +607,28 @@ static int tiled_bm(const GmmArgs& a)
     if (force && force[0] == 'u') return 64;
 #endif
     const int64_t avg = a.R / a.E;
-    if (avg < 48) {
-        // Streaming wants every expert inside one 32-row pass.  Measured with uniform routing (the friendliest
-        // case for it) at K = 7168 / 2048: 24 rows per expert on average 1407 / 84 us streaming against 1288 / 74 us
-        // on the tiles, 32 rows 1957 / 115 against 1311 / 75, 16 rows 1223 / 73 against 1266 / 73, 8 rows 1119
-        // against 1244; under Zipf(1.1) routing at 16 rows on average the tiles win as well (1260 against 1521).
-        // Decode batches (fewer than 1024 rows) always stream.
-        if (a.R < 1024 || avg < 12) return 0;
-        // the list of 256-row tiles is built from 16-bit counters (tile_map_kernel, by_length)
-        const bool wide_small = a.K >= 4096 && a.R / 256 + a.E < 32768;
-        // 24..47 rows per expert: tiles.  With a long K the weight-streaming tiles (their one- and two-block forms
-        // for the experts of up to 32 / 64 rows): uniform routing over 256 experts, K = 7168, 24 / 32 / 48 rows
-        // 1255 / 1270 / 1286 us against 1283 / 1305 / 1322 us on the 128-row tiles (streaming 1373 / 1938 / 2706);
-        // at K = 2048 the two kinds of tiles measure the same (664 / 677 / 697 against 664 / 680 / 703).
-        if (avg >= 24) return wide_small ? 256 : 128;
-        // 12..23 rows per expert: large products split the experts between both families (gemm_plan; streaming
-        // alone leads the tiles up to 20 rows at K = 7168 and up to 24 at K = 2048: 612 against 654 us at 20); for
-        // small ones the second launch costs more than it brings and the tiles alone are as fast as streaming
-        return (int64_t)a.E * a.N * a.K >= (1ll << 30) ? 0 : 128;
-    }
+    const int64_t weights = (int64_t)a.E * a.N * a.K;
+    // Streaming or 128-row tiles, the whole layer through the sorted path in us, uniform routing and Zipf(1.1):
+    //   256 experts, K = 7168 / 2048 (7 and 3.5 GiB): 16 tokens (half a row per expert) 685 against 703 and 253
+    //     against 281; 32 tokens 1097 against 1100 and 351 against 328; 64 tokens 1455 against 1449 and 442 against
+    //     406; 96 tokens 1584 against 1592 and 508 against 423.  So from one row per expert on: tiles.
+    //   256 experts, K = 4096 / 1024 (2 and 1 GiB), 64 / 128 / 256 / 448 / 640 tokens: 475 / 514 / 539 / 568 / 591 with
+    //     the small product split, 481 / 516 / 535 / 555 / 565 on tiles; Zipf 162 / 201 / 221 / 264 / 305 against 149 /
+    //     193 / 212 / 250 / 290.
+    //   128 experts, K = 2048 / 768 (0.4 and 0.2 GB): 48 / 100 tokens 107 / 112 against 117 / 131 and 81 / 86 against
+    //     73 / 81, so decode batches (fewer than 1024 rows) stream; 130 / 190 tokens 120 / 123 against 123 / 126 and
+    //     153 / 183 against 80 / 88: tiles.
+    if (a.R < a.E) return 0;
+    if (avg < 48 && a.R < 1024 && (a.R < 128 || weights < (1ll << 30))) return 0;
+    // at a GiB of weights the experts are split between both families up to 23 rows per expert (gemm_plan)
+    if (avg < 24 && split_size(weights)) return 0;
     // the list of 256-row tiles is built from 16-bit counters (tile_map_kernel, by_length)
     const bool wide_ok = a.R / 256 + a.E < 32768;
-    if (avg <= 256 && a.K >= 4096 && wide_ok) return 256;
+    // K = 7168 / 2048, uniform routing, 28 / 40 / 48 / 56 / 64 / 94 rows per expert: the layer takes 1968 / 2028 / 2055 /
+    // 2091 / 2126 / 2280 us with the weight-streaming tiles in the first product, 1867 / 1975 / 2031 / 2088 / 2162 / 2512
+    // us on 128-row tiles; Zipf(1.1) at 28 / 40 / 64 / 94 / 128 1115 / 1361 / 1703 / 2164 / 2616 against 1069 / 1339 /
+    // 1667 / 2155 / 2648.  128 experts at K = 4096, 56 / 69 / 81 rows: 526 / 547 / 567 against 511 / 552 / 576.
+    if (avg >= 64 && avg <= 256 && a.K >= 4096 && wide_ok) return 256;
     // around 128 rows per expert most experts fit one wide tile of 128 or 160 rows and fetch their weights once,
     // which pays from K = 1024 on (measured: 6 % at K = 2048 and 1024, a loss at K = 768 and at 64 rows)
     if (avg >= 96 && avg <= 192 && a.K >= 1024 && wide_ok) return 256;
@@ -630,15 +636,14 @@ static int tiled_bm(const GmmArgs& a)
 }
 
 // What one operator call launches: the family chosen from the mean rows per expert, restricted to the experts it
-// is good at, and (split > 0) the 128-row tiles for the experts above that range.
-//   mean < 24 (12..23 for products of a GiB of weights and more, see tiled_bm; such products from one row per
-//     expert on, smaller ones from 1024 rows on): streaming
-//     for experts of at most 32 rows (one pass over their weights, and no request before the group list says that
-//     the expert is theirs), tiles for the others -- a 500-row expert would otherwise stream its weights 16 times
-//     while the units of the cold experts have long finished.  Measured at the DeepSeek-V3 shape with Zipf(1.1)
-//     routing, 4096 rows: 1154 us against 1260 (tiles alone) and 1521 (streaming alone) over 244 touched experts;
-//     533 against 568 and 1190 over the 90 touched experts of the benchmark's batch.
-//   The weight-streaming tiles (mean 48..256) keep every expert: sending those above 256 rows to the 128-row
+// is good at, and (split > 0) a second family for the experts above that range.
+//   Products of one GiB of weights, mean below 24, decode batches too from one row per expert on: streaming for
+//     experts of at most 32 rows (one pass over their weights, and no request before the group list says that the
+//     expert is theirs), tiles for the others -- a 500-row expert would otherwise stream its weights 16 times while the
+//     units of the cold experts have long finished.  It is the border between the small products, whose decode batches
+//     stream, and the large ones, which run on tiles: 256 experts, K = 4096 / 512, 64 / 128 / 256 tokens, uniform
+//     routing 245 / 283 / 286 us split, 256 / 285 / 285 us on tiles.
+//   The weight-streaming tiles (mean 64..256) keep every expert: sending those above 256 rows to the 128-row
 //     tiles measured the same on a Zipf(1.1) batch of 32,768 rows (2149 against 2180 us for the gate_up product,
 //     1136 against 1119 us for the down product) and would cost the uniform batches an empty launch.
 struct GemmPlan {
@@ -663,17 +668,11 @@ static GemmPlan gemm_plan(const GmmArgs& a, bool have_tile_ws)
         return p;
     }
 #endif
-    // a large product (a GiB of weights and more) over many experts with few rows on average.  Decode batches
-    // too, from one row per expert on: on uniform routing the second launch finds nothing to do and costs 3 to 8 us,
-    // on skewed routing the hot experts leave the streaming kernel (which also requests nothing for an idle expert
-    // in this form).  DeepSeek-V3 shape through the sorted path, 32 / 64 / 112 tokens: uniform 1216 -> 1159,
-    // 1500 -> 1490, 1648 -> 1656 us; Zipf(1.1) 529 -> 391, 640 -> 533, 796 -> 625 us.
-    if (p.bm == 0 && a.R >= 128 && a.R >= (int64_t)a.E && (int64_t)a.E * a.N * a.K >= (1ll << 30)) {
+    if (p.bm == 0 && a.R >= 128 && a.R >= (int64_t)a.E && split_size((int64_t)a.E * a.N * a.K)) {
         p.split = 32;
         // the experts above the border: weight-streaming tiles when K is long (an expert of up to 256 rows fetches
-        // its weights once), 128-row tiles otherwise.  Measured on 512 tokens of Zipf(1.1) routing at the
-        // DeepSeek-V3 shape: K = 7168 518 against 532 us for the pair of launches, K = 2048 the other way round
-        // by as much; a border of 16 or 64 rows instead of 32 costs 70 / 40 us.
+        // its weights once), 128-row tiles otherwise.  A border of 16 or 64 rows instead of 32 cost 70 / 40 us of
+        // 518 us on 512 tokens of Zipf(1.1) routing at K = 7168.
         if (a.K >= 4096 && a.R / 256 + a.E < 32768) p.split_bm = 256;
     }
     return p;
@@ -1044,11 +1043,11 @@ extern "C" int moe355_gmm_pairs_supported(int64_t num_tokens, int top_k, int64_t
     return num_tokens > 0 && top_k > 0 && num_tokens * top_k <= kPairMax && n > 0 && k > 0 && n % 64 == 0 && k % 32 == 0;
 }
 
-// Whether a batch whose ids come straight from the gate runs in pair order: at most 1024 (token, slot) pairs that the
-// grouped GEMMs would stream the weights for anyway, and experts that the bit map of the lookup can hold.  A product
-// of a GiB and more has a second kernel family for hot experts on the sorted path (gemm_plan), pair order streams
-// every expert: DeepSeek-V3 shape under Zipf(1.1) routing, 112 / 128 tokens 668 / 742 us in pair order, 625 / 641 us
-// sorted; on uniform routing pair order leads by 1 % there.
+// Whether a batch whose ids come straight from the gate runs in pair order: at most 1024 (token, slot) pairs, up to 12
+// per expert, and experts that the bit map of the lookup can hold.  Pair order streams every expert; the sorted path of
+// a product of a GiB and more has tiles for the hot ones.  DeepSeek-V3 shape, 70 / 80 / 96 tokens with the shared expert
+// in line: uniform routing 1500 / 1541 / 1581 us in pair order, 1575 / 1601 / 1641 us sorted; Zipf(1.1) 506 / 538 / 597
+// against 481 / 514 / 549; 128 tokens without it 742 against 457 us.
 extern "C" int moe355_pair_order(int64_t num_tokens, int top_k, int num_logits, int num_experts, int64_t hidden,
                                  int64_t intermediate)
 {
@@ -1058,7 +1057,7 @@ extern "C" int moe355_pair_order(int64_t num_tokens, int top_k, int num_logits, 
         return 0;
     const int64_t pairs = num_tokens * top_k;
     if ((int64_t)num_experts * 2 * intermediate * hidden >= (1ll << 30) && pairs > 768) return 0;
-    return pairs < 1024 || pairs / num_experts < 12;  // where the sorted form streams as well (tiled_bm)
+    return pairs < 1024 || pairs / num_experts < 12;
 }
 
 // pair order: the places of the grid.
