@@ -201,7 +201,12 @@ __device__ __forceinline__ bool find_chunk(const int64_t* gl, int gl_type, int E
 // The four wavefronts of a workgroup work on the same chunk (four neighbouring tile pairs), so the chunk's
 // tokens go through LDS once per workgroup: every thread loads one 16-byte piece of the 64 x 64-byte K block
 // (rows are read in 64-byte runs instead of 16-byte crumbs per lane), writes it in MFMA-operand order, and
-// each wavefront reads its four B operands back with conflict-free 1 KiB sweeps.
+// each wavefront reads its four B operands back with conflict-free 1 KiB sweeps; one barrier per two K blocks.
+// Besides HBM the vector ALU bounds it (the fold of 64 sums and the unpacking take longer than the MFMAs), so the fold is
+// conversion, product and sum alone: no shift (the scales in LDS are a sixteenth) and no clearing (the first product of a
+// group starts from the instruction's own zero).  DeepSeek-V3 shape, groups of 256, us a layer call before / after both
+// and the halved barriers: uniform 512 / 1024 / 2048 tokens 1040 / 1236 / 1765 -> 1030 / 1206 / 1707, Zipf(1.1) 128 / 512 /
+// 1024 tokens 334 / 595 / 929 -> 324 / 587 / 883; groups of 128 (scales from memory) 1237 -> 1193 at 512, 771 -> 729 Zipf.
 constexpr int kW4Chunk = 64;
 constexpr int kW4LdsGroups = 32;  // K groups whose scales are kept in LDS (8 KiB per wavefront)
 // LDS_SCALES: the group scales of the wavefront's channels fit LDS (K / group <= kW4LdsGroups)
@@ -233,7 +238,7 @@ __global__ __launch_bounds__(256, 2) void gmm_w4_stream_kernel(W4Args p)
     // weights and tokens: rings of RW single K blocks, requested RW - 1 blocks ahead of their MFMAs.  Both
     // rings have the same depth on purpose: the memory counter retires loads in order, so waiting for a
     // token block that was requested late would also wait for every weight block requested before it.
-    constexpr int RW = LDS_SCALES ? 6 : 5;  // scales read from memory inside the fold need the registers of one ring slot
+    constexpr int RW = LDS_SCALES ? 6 : 4;  // even; scales read from memory inside the fold need the registers of a slot
     v4i a0[RW], a1[RW];
     // STREAM: the expert has a single chunk, nobody else reads these weights: non-temporal loads (the faster
     // pure stream).  Otherwise the sibling chunks of the expert run at the same time on the same XCD (their
@@ -255,7 +260,7 @@ __global__ __launch_bounds__(256, 2) void gmm_w4_stream_kernel(W4Args p)
     const int n_groups = a.K / p.group;
     const float* gs = p.gscale + (int64_t)e * n_groups * a.N;
 
-    __shared__ __attribute__((aligned(16))) int8_t Bs[2][kW4Chunk * 64];  // two stages of 64 rows x 64 K bytes
+    __shared__ __attribute__((aligned(16))) int8_t Bs[2][2][kW4Chunk * 64];  // two stages of two blocks of 64 rows x 64 K bytes
     int64_t row[2];
     bool valid[2];
 #pragma unroll
@@ -288,7 +293,10 @@ __global__ __launch_bounds__(256, 2) void gmm_w4_stream_kernel(W4Args p)
     // The scales of this wavefront's 64 channels for every K group sit in LDS (when they fit: up to 32
     // groups), loaded once up front: the K loop then has no load whose result is needed at once, and its
     // waits for weights and tokens stay partial.
+    // Kept there as scale / 16: the sixteen of the accumulators then cancels in the product, bit for bit as long as the
+    // quotient is exact; a wavefront with a scale so small that it is not shifts its accumulators instead.
     __shared__ float Ss[4][LDS_SCALES ? kW4LdsGroups * 64 : 1];
+    bool shift = !LDS_SCALES;
     if constexpr (LDS_SCALES) {
         const int ch = lane < 32 ? nb0 * 32 + lane : nb1 * 32 + (lane - 32);
         for (int g0 = 0; g0 < n_groups; g0 += 8) {  // eight loads in flight at a time
@@ -296,25 +304,32 @@ __global__ __launch_bounds__(256, 2) void gmm_w4_stream_kernel(W4Args p)
 #pragma unroll
             for (int j = 0; j < 8; ++j) t[j] = gs[(int64_t)(g0 + j < n_groups ? g0 + j : n_groups - 1) * a.N + ch];
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (g0 + j < n_groups) Ss[wave][(g0 + j) * 64 + lane] = t[j];
+            for (int j = 0; j < 8; ++j) {
+                if (g0 + j < n_groups) Ss[wave][(g0 + j) * 64 + lane] = t[j] * 0.0625f;
+                shift |= (t[j] * 0.0625f) * 16.0f != t[j];
+            }
         }
+        shift = __ballot(shift) != 0;
+        if (shift)
+            for (int i = lane; i < n_groups * 64; i += 64) Ss[wave][i] = gs[(int64_t)(i >> 6) * a.N + ch];
     }
     int in_group = 0, grp = 0;
     // f += float(acc / 16) * scale[e, grp, channel]
     auto fold_with = [&](const v4f* s0, const v4f* s1) {
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
-            if (b == 1 && !two) break;  // no rows in the second token block: its accumulators stay zero
+            if (b == 1 && !two) break;  // no rows in the second token block
+            if (shift) {
+                c0[b] = c0[b] >> 4;
+                c1[b] = c1[b] >> 4;
+            }
 #pragma unroll
             for (int q = 0; q < 4; ++q)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    f0[b][4 * q + j] = f0[b][4 * q + j] + (float)(c0[b][4 * q + j] >> 4) * s0[q][j];
-                    f1[b][4 * q + j] = f1[b][4 * q + j] + (float)(c1[b][4 * q + j] >> 4) * s1[q][j];
+                    f0[b][4 * q + j] = f0[b][4 * q + j] + (float)c0[b][4 * q + j] * s0[q][j];
+                    f1[b][4 * q + j] = f1[b][4 * q + j] + (float)c1[b][4 * q + j] * s1[q][j];
                 }
-            c0[b] = (v16i){0};
-            c1[b] = (v16i){0};
         }
         in_group = 0;
         ++grp;
@@ -339,40 +354,46 @@ __global__ __launch_bounds__(256, 2) void gmm_w4_stream_kernel(W4Args p)
             fold_with(s0, s1);
         }
     };
-    // tokens: K block kb lives in LDS stage kb & 1; treg[(kb) % RW] carries block kb from its load (RW - 1
-    // steps before its MFMAs) until it is written to LDS in the step before it is used
+    // tokens: K blocks kb and kb + 1 (kb even) live in LDS stage (kb / 2) & 1; treg[kb % RW] carries block kb from its load
+    // until it is written to LDS two steps before it is used
     auto load_tokens = [&](int kb) { return *(const v4i*)(xs + (int64_t)(kb < KB64 ? kb : KB64 - 1) * 64); };
     v4i treg[RW];
     treg[0] = load_tokens(0);
-    *(v4i*)(&Bs[0][lds_off]) = treg[0];
+    treg[1] = load_tokens(1);
+    *(v4i*)(&Bs[0][0][lds_off]) = treg[0];
+    *(v4i*)(&Bs[0][1][lds_off]) = treg[1];
 #pragma unroll
-    for (int i = 1; i < RW; ++i) treg[i] = load_tokens(i);
+    for (int i = 2; i < RW + 2; ++i) treg[i % RW] = load_tokens(i);
     __syncthreads();
     auto step = [&](auto stream, int slot, int kb) {  // one 64-wide K block; slot = kb % RW (compile time)
         v4i bl[2], bh[2];  // [token block]: K 0..31 / 32..63 of the block
-        const int8_t* st = Bs[kb & 1];
+        const int8_t* st = Bs[(kb >> 1) & 1][kb & 1];
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
             bl[b] = *(const v4i*)(st + ((0 * 2 + b) * 64 + lane) * 16);
             bh[b] = *(const v4i*)(st + ((1 * 2 + b) * 64 + lane) * 16);
         }
-        *(v4i*)(&Bs[(kb + 1) & 1][lds_off]) = treg[(slot + 1) % RW];  // block kb + 1 (stage last read in step kb - 1)
-        treg[slot] = load_tokens(kb + RW);   // block kb has left its register in the step before
+        *(v4i*)(&Bs[((kb >> 1) & 1) ^ 1][kb & 1][lds_off]) = treg[(slot + 2) % RW];  // block kb + 2; its stage was last read before the last barrier
+        treg[(slot + 2) % RW] = load_tokens(kb + 2 + RW);
         const v4i l0 = nib_lo(a0[slot]), h0 = nib_hi(a0[slot]);
         const v4i l1 = nib_lo(a1[slot]), h1 = nib_hi(a1[slot]);
         load_weights(stream, (slot + RW - 1) % RW, kb + RW - 1);  // the slot block kb - 1 has just left
-        c0[0] = mfma_i8(l0, bl[0], c0[0]);
-        c0[0] = mfma_i8(h0, bh[0], c0[0]);
-        c1[0] = mfma_i8(l1, bl[0], c1[0]);
-        c1[0] = mfma_i8(h1, bh[0], c1[0]);
-        if (two) {
-            c0[1] = mfma_i8(l0, bl[1], c0[1]);
-            c0[1] = mfma_i8(h0, bh[1], c0[1]);
-            c1[1] = mfma_i8(l1, bl[1], c1[1]);
-            c1[1] = mfma_i8(h1, bh[1], c1[1]);
+        const bool first = in_group == 0;  // of its scale group: the accumulators start from the instruction's own zero
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            if (b == 1 && !two) break;
+            if (first) {
+                c0[b] = mfma_i8(l0, bl[b], (v16i){0});
+                c1[b] = mfma_i8(l1, bl[b], (v16i){0});
+            } else {
+                c0[b] = mfma_i8(l0, bl[b], c0[b]);
+                c1[b] = mfma_i8(l1, bl[b], c1[b]);
+            }
+            c0[b] = mfma_i8(h0, bh[b], c0[b]);
+            c1[b] = mfma_i8(h1, bh[b], c1[b]);
         }
         if (++in_group == steps_per_group) fold();
-        __syncthreads();  // block kb + 1 is visible; nobody still reads block kb
+        if (slot & 1) __syncthreads();  // blocks kb + 1 and kb + 2 are visible; nobody still reads kb - 1 and kb
     };
     // whole passes through the ring without a condition on kb; the remainder is peeled
     const int kb_full = (KB64 / RW) * RW;
