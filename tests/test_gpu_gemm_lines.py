@@ -39,3 +39,32 @@ def test_families_on_both_sides_of_a_line(R, E, Kd, N, family, skewed):
     torch.cuda.synchronize()
     assert np.array_equal(q.cpu().numpy(), q_want)
     assert np.array_equal(s.cpu().numpy().view(np.uint32), s_want.view(np.uint32))
+
+
+# rows of the down GEMM that re-quantises: shorter than, equal to and longer than the 256 values of one load, with a
+# remainder; an expert with two passes of 32 rows
+@pytest.mark.parametrize("T,E,I", [(56, 128, 320), (56, 128, 256), (56, 128, 32), (40, 128, 1408), (1, 128, 1504)])
+def test_requantising_down_gemm_gives_the_separate_launches_bits(T, E, I):
+    from vllm_ascend_amd import kernels as K
+    from vllm_ascend_amd._lib import W_ENK
+
+    H, k = 1024, 8
+    print(f"requant T={T} E={E} I={I}", flush=True)
+    assert K.gmm2_requant_pairs_supported(T, k, H, I, E)
+    g = torch.Generator().manual_seed(T + I)
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16).to("cuda")
+    ids = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)]).to(torch.int32)
+    ids[:, 0] = 5
+    ids = ids.to("cuda")
+    w13 = torch.randint(-128, 128, (E, 2 * I, H), generator=g, dtype=torch.int8).to("cuda")
+    w2 = torch.randint(-128, 128, (E, H, I), generator=g, dtype=torch.int8).to("cuda")
+    s13 = (torch.rand(E, 2 * I, generator=g) * 0.009 + 0.001).to("cuda")
+    s2 = (torch.rand(E, H, generator=g) * 0.009 + 0.001).to("cuda")
+    w13, w2 = K.format_cast_nz(w13, W_ENK), K.format_cast_nz(w2, W_ENK)
+    xq, xs = K.dynamic_quant(x)
+    q1, s1 = K.gmm1_swiglu_quant_pairs(xq, xs, ids, w13, s13, 2 * I, H)
+    want = K.gmm2_dequant_pairs(q1, w2, s2, s1, ids, H, I)
+    y = K.gmm1_swiglu_pairs(xq, xs, ids, w13, s13, 2 * I, H)
+    got = K.gmm2_requant_dequant_pairs(y, w2, s2, ids, H, I)
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))

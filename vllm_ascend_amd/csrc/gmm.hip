@@ -99,7 +99,6 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
     static_assert(!PAIRS || (!SLABS && EARLY && EPI != EPI_I32), "pair order: the two GEMMs of a decode layer");
     static_assert(!REQ || (PAIRS && EPI == EPI_DEQUANT), "the re-quantisation sits in the pair-order down GEMM");
     extern __shared__ __attribute__((aligned(16))) int8_t qtile[];  // REQ: 32 rows of K + 16 bytes
-    __shared__ uint32_t qmax[REQ ? 32 : 1];
     __shared__ float qscale[REQ ? 32 : 1];
     constexpr int kRed = (KSPLIT > 1) ? 32 * 64 : 1;
     __shared__ int32_t red[PAIRS && kRed < kPairExperts ? kPairExperts : kRed];
@@ -328,40 +327,44 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
         float rs = 0.0f;
         if constexpr (!REQ) xo = src * a.K + kh * 16;
         if constexpr (REQ) {
-            // rows r0 .. r0 + 31 of the expert -> int8 in LDS, every (row, four values) item by some thread
+            // rows r0 .. r0 + 31 of the expert -> int8 in LDS: a wavefront takes every fourth row and holds it in registers
+            // between its maximum and its quantisation (K < 2048).  One row at a time: two would hide the load of the
+            // second one (1 us of 52 at 24 tokens of skewed routing) and cost the fifth wavefront of a SIMD (6 %).
             const int pitch = a.K + 16;  // rows 16 bytes apart in the banks
             const int rows_now = (int)(row1 - r0 < 32 ? row1 - r0 : 32);
-            const int per_row = a.K >> 2, items = rows_now * per_row;
-            if (threadIdx.x < 32) qmax[threadIdx.x] = 0u;
-            __syncthreads();
-            for (int it = threadIdx.x; it < items; it += 256) {
-                const int rr = it / per_row, c4 = it - rr * per_row;
-                const v4f v = *(const v4f*)(a.y_in + (int64_t)plist[r0 + rr] * a.K + c4 * 4);
-                float m = 0.0f;
+            if (r0 != row0) __syncthreads();  // nobody still reads the rows of the pass before
+            for (int rr = wave; rr < rows_now; rr += 4) {
+                const float* y = a.y_in + (int64_t)plist[r0 + rr] * a.K + lane * 4;
+                v4f v[8];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float ab = __builtin_fabsf(v[j]);
-                    m = ab > m ? ab : m;
+                for (int i = 0; i < 8; ++i)
+                    v[i] = i * 256 + lane * 4 < a.K ? *(const v4f*)(y + i * 256) : (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+                float amax = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const float ab = __builtin_fabsf(v[i][j]);
+                        amax = ab > amax ? ab : amax;
+                    }
+#pragma unroll
+                for (int off = 32; off > 0; off >>= 1) {
+                    const float o = __shfl_xor(amax, off, 64);
+                    amax = o > amax ? o : amax;
                 }
-                atomicMax(&qmax[rr], __float_as_uint(m));
-            }
-            __syncthreads();
-            for (int it = threadIdx.x; it < items; it += 256) {
-                const int rr = it / per_row, c4 = it - rr * per_row;
-                const v4f v = *(const v4f*)(a.y_in + (int64_t)plist[r0 + rr] * a.K + c4 * 4);
-                const float amax = __uint_as_float(qmax[rr]);
                 const float inv = 1.0f / (amax / 127.0f);
-                uint32_t pk = 0u;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int8_t q = (amax == 0.0f) ? (int8_t)0 : sat_rint_i8(v[j] * inv);
-                    pk |= (uint32_t)(uint8_t)q << (8 * j);
+                for (int i = 0; i < 8; ++i) {
+                    if (i * 256 + lane * 4 >= a.K) break;
+                    uint32_t pk = 0u;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int8_t q = (amax == 0.0f) ? (int8_t)0 : sat_rint_i8(v[i][j] * inv);
+                        pk |= (uint32_t)(uint8_t)q << (8 * j);
+                    }
+                    *(uint32_t*)(qtile + rr * pitch + i * 256 + lane * 4) = pk;
                 }
-                *(uint32_t*)(qtile + rr * pitch + c4 * 4) = pk;
-            }
-            if (threadIdx.x < rows_now) {
-                const float amax = __uint_as_float(qmax[threadIdx.x]);
-                qscale[threadIdx.x] = (amax == 0.0f) ? 0.0f : amax / 127.0f;
+                if (lane == 0) qscale[rr] = (amax == 0.0f) ? 0.0f : amax / 127.0f;
             }
             __syncthreads();
             xo = (valid ? tok : 0) * pitch + kh * 16;
@@ -1230,10 +1233,11 @@ extern "C" int moe355_gmm2_requant_pairs_supported(int64_t num_tokens, int top_k
     if (!moe355_gmm_pairs_supported(num_tokens, top_k, n, k) || num_experts <= 0) return 0;
     const int64_t units = (int64_t)num_experts * (n / 64);
     if (!(units >= 2048 && k < 2048 && (n / 64) % 4 == 0 && k % 4 == 0 && 32 * (k + 16) <= 48 * 1024)) return 0;
-    // it pays up to about three rows per expert (measured on 128 experts of 2048 x 768: 24 / 32 / 48 tokens of eight
-    // slots 98.4 / 102.8 / 109.7 us against 101.3 / 104.8 / 110.5 us with the launch of its own, 64 tokens 112.0
-    // against 111.3, 128 tokens 119.6 against 115.8): every workgroup of an expert quantises all its rows again
-    return num_tokens * top_k <= 3 * (int64_t)num_experts;
+    // it pays up to about three and a half rows per expert: every workgroup of an expert quantises all its rows again.
+    // 128 experts of 2048 x 768, the layer in us with the launch of its own / inside: uniform routing 8 / 24 / 48 / 56 / 64
+    // tokens of eight slots 62.5 / 90.9 / 105.4 / 107.0 / 108.4 against 58.9 / 88.4 / 103.6 / 105.8 / 107.4; Zipf(1.1)
+    // 42.8 / 52.0 / 71.4 / 73.0 / 75.0 against 40.2 / 52.3 / 70.4 / 71.9 / 76.6, 96 tokens 85.2 against 87.0
+    return 2 * num_tokens * top_k <= 7 * (int64_t)num_experts;
 }
 
 extern "C" int moe355_gmm2_requant_dequant_pairs(const float* y, const int8_t* weight_nz, const float* scale,
