@@ -68,3 +68,22 @@ def test_requantising_down_gemm_gives_the_separate_launches_bits(T, E, I):
     got = K.gmm2_requant_dequant_pairs(y, w2, s2, ids, H, I)
     torch.cuda.synchronize()
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+# token quantisation with a row per wavefront: from 512 tokens on, rows of up to 2048 values, a last workgroup that is
+# not full
+@pytest.mark.parametrize("T,H", [(511, 2048), (512, 2048), (515, 1032), (513, 8), (777, 2056)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_token_rows_quantised_beside_the_gating(T, H, dtype):
+    from vllm_ascend_amd import kernels as K
+
+    print(f"gate_quant T={T} H={H} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(T + H)
+    x = torch.randn(T, H, generator=g).to(dtype)
+    x[3] = 0
+    x[-1] *= 1e-6
+    x, logits = x.to("cuda"), torch.randn(T, 128, generator=g).to("cuda")
+    got = K.gate_quant(x, logits, 8, 1, 1, 0, 1, 0, 1.0, 1e-20, None)
+    xq, xs = K.dynamic_quant(x)
+    torch.cuda.synchronize()
+    assert torch.equal(got[2], xq) and torch.equal(got[3].view(torch.int32), xs.view(torch.int32))
