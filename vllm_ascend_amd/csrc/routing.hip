@@ -356,12 +356,19 @@ __global__ __launch_bounds__(kMapThreads) void route_map_kernel(RouteMapArgs a)
         for (int i = tid; i < kMapWaves * E; i += kMapThreads) whist[i] = 0;
     __syncthreads();
     int mine = -1;  // this thread's pair of the chunk
+    int next[8];  // the ids of the next 8192 pairs are requested in front of the counting of these (15.9 -> 14.7 us at 65536)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) next[j] = j * kMapThreads + tid < R ? a.ids[j * kMapThreads + tid] : -1;
     for (int base = 0; base < R; base += 8 * kMapThreads) {
         int id[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int f = base + j * kMapThreads + tid;
-            id[j] = f < R ? a.ids[f] : -1;
+        for (int j = 0; j < 8; ++j) id[j] = next[j];
+        if (base + 8 * kMapThreads < R) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int f = base + (8 + j) * kMapThreads + tid;
+                next[j] = f < R ? a.ids[f] : -1;
+            }
         }
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
