@@ -453,14 +453,14 @@ __global__ __launch_bounds__(256, 2) void gmm_w4_stream_kernel(W4Args p)
 // v_mfma_i32_16x16x64_i8 (one or two times, for experts of more than 16 rows), so accumulators and fp32 sums are 16
 // registers each instead of 64 and the fold is a quarter of the work.  HBM-bound: DeepSeek-V3 shape, us a layer call
 // against the sorted chunks, uniform routing, 1 / 4 / 16 / 32 tokens 59 / 136 / 382 / 557 against 86 / 157 / 412 / 593
-// (16 tokens: 2.3 GB at 6.4 TB/s), Zipf(1.1), 24 / 32 / 48 tokens 148 / 177 / 217 against 163 / 206 / 227.  A ring of
+// (16 tokens: 2.3 GB at 6.4 TB/s), Zipf(1.1), 24 / 32 tokens 148 / 178 against 163 / 203.  A ring of
 // 8, 10 or 12 blocks 389 to 393 us at 16 tokens, three wavefronts per SIMD the same as two and 191 us at 32 under Zipf.
 // An int4 tile (lane = channel l % 32, K half l / 32; low nibbles K 0..31, high nibbles K 32..63) becomes the operands of
 // its two groups of 16 channels by one exchange: rows of 16 lanes 1 and 3 of the low-nibble register against rows 0 and 2
 // of the high-nibble register (v_permlane16_swap) leave channels 0..15 in one register and 16..31 in the other, row r of
 // either holding the K slice 0, 32, 16 or 48 + 0..15 for r = 0, 1, 2, 3.  The tokens are read in that order.
 constexpr int kW4PairMax = 1024;
-constexpr int kW4PairTokens = 48;  // see w4_pairs_supported
+constexpr int kW4PairTokens = 40;  // see w4_pairs_supported
 constexpr int kW4PairExperts = 2048;
 constexpr int kW4PairRing = 6;     // K blocks of weights and tokens in flight per wavefront
 
@@ -487,7 +487,7 @@ __global__ __launch_bounds__(256, 2) void gmm_w4_pairs_kernel(W4Args p)
     const int lane = threadIdx.x & 63;
     const int NB = a.N >> 5, KB64 = a.K >> 6;
     const int upe = NB >> 1, quads = (upe + 3) >> 2;
-    const int slot = (int)(blockIdx.x / quads);
+    const int slot = (int)(blockIdx.x / quads) - a.pair_extra;
     const int pi_raw = (int)(blockIdx.x % quads) * 4 + wave;
     const bool have = pi_raw < upe;
     const int pi = have ? pi_raw : 0;
@@ -511,10 +511,40 @@ __global__ __launch_bounds__(256, 2) void gmm_w4_pairs_kernel(W4Args p)
     const int incl = wave_scan_inclusive_i32(cnt);
     const bool has = slot >= incl - cnt && slot < incl;
     const unsigned long long holder = __ballot(has);
-    if (holder == 0ull) return;  // fewer experts with pairs than slots (the same answer in all four wavefronts)
-    uint32_t t = bits;
-    for (int i = has ? slot - (incl - cnt) : 0; i > 0; --i) t &= t - 1;
-    const int e = __builtin_amdgcn_readlane(lane * 32 + (t ? __builtin_ctz(t) : 0), __builtin_ctzll(holder));
+    int e, first = 0;
+    if (holder != 0ull) {  // the same answer in all four wavefronts
+        uint32_t t = bits;
+        for (int i = has ? slot - (incl - cnt) : 0; i > 0; --i) t &= t - 1;
+        e = __builtin_amdgcn_readlane(lane * 32 + (t ? __builtin_ctz(t) : 0), __builtin_ctzll(holder));
+    } else {
+        // the slots in front (and those past the last expert with pairs, which leave): the experts of more than 32 rows, for
+        // the rows from 32 on.  In the same workgroup one after the other they held up the launch: 40 tokens 212 / 252 /
+        // 262 us -> 216 / 214 / 262, slots behind all others instead 222 / 217 / 271.  The pairs are counted where the scales
+        // will lie.
+        if (slot >= 0) return;
+        const int j = slot + a.pair_extra;
+        int* count = (int*)&Ss[0][0];
+        for (int i = threadIdx.x; i < kW4PairExperts; i += 256) count[i] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (pid[c] >= 0 && pid[c] < a.E) atomicAdd(&count[pid[c]], 1);
+        __syncthreads();
+        int hot = -1, seen = 0;  // the j-th of them, experts lane, lane + 64, ... in rounds of 64
+        for (int i = 0; i < (a.E + 63) >> 6 && hot < 0; ++i) {
+            unsigned long long m = __ballot(i * 64 + lane < a.E && count[i * 64 + lane] > 32);
+            const int n = __popcll(m);
+            if (j < seen + n) {
+                for (int q = j - seen; q > 0; --q) m &= m - 1;
+                hot = i * 64 + __builtin_ctzll(m);
+            }
+            seen += n;
+        }
+        if (hot < 0) return;
+        __syncthreads();
+        e = hot;
+        first = 32;
+    }
 
     const int nb0 = (EPI == EPI_SWIGLU) ? pi : 2 * pi;
     const int nb1 = (EPI == EPI_SWIGLU) ? pi + upe : 2 * pi + 1;
@@ -652,10 +682,11 @@ __global__ __launch_bounds__(256, 2) void gmm_w4_pairs_kernel(W4Args p)
                 epilogue_run_w4<EPI>(a, row[n], valid[n], nb0 * 32 + ch, nb1 * 32 + ch, f[n][0][h], f[n][1][h], rs[n]);
             }
     };
-    if (rows <= 16) {
-        pass(std::integral_constant<int, 1>{}, 0);
+    if (first == 0 && a.pair_extra > 0 && rows > 32) rows = 32;  // another workgroup has the others
+    if (rows - first <= 16) {
+        pass(std::integral_constant<int, 1>{}, first);
     } else {
-        for (int first = 0; first < rows; first += 32) pass(std::integral_constant<int, 2>{}, first);
+        for (; first < rows; first += 32) pass(std::integral_constant<int, 2>{}, first);
     }
 }
 
@@ -790,9 +821,9 @@ extern "C" int moe355_gmm1_swiglu_quant_w4_gather(const int8_t* x, const float* 
                         n, num_experts, swiglu_limit, out, out_scale, workspace, workspace_bytes, stream, row_token);
 }
 
-// Up to 48 tokens: an expert has at most that many rows, two passes of 32.  With 64 tokens uniform routing would still
-// gain (844 -> 795 us), but skewed routing loses by the repeated passes of its hot experts (250 -> 270 us; 128 tokens
-// 327 -> 479 us), and the host cannot know.
+// Up to 40 tokens.  Uniform routing would gain beyond (47 tokens 750 -> 710 us, 64 844 -> 795 us), but skewed routing loses by
+// the second reading of its hot experts' weights: Zipf(1.1), three draws, 40 tokens 216 / 214 / 262 us against 220 / 232 /
+// 271 sorted, 47 tokens 232 / 251 / 274 against 235 / 237 / 274, 128 tokens 479 against 327; the host cannot know.
 bool moe355::w4_pairs_supported(int64_t num_tokens, int top_k, int num_experts, int64_t hidden, int64_t intermediate,
                                 int64_t group13, int64_t group2)
 {
@@ -816,13 +847,14 @@ static W4Args w4_pair_args(const int8_t* x, const float* x_scale, const int32_t*
     p.w4 = w;
     p.gscale = scale;
     p.group = (int)group;
+    p.g.pair_extra = num_tokens > 32 ? (int)(p.g.R / 33) : 0;  // a row of an expert per token
     return p;
 }
 
 static dim3 w4_pair_grid(const W4Args& p)
 {
     const int64_t slots = p.g.R < (int64_t)p.g.E ? p.g.R : (int64_t)p.g.E;
-    return dim3((unsigned)(slots * ((p.g.N / 64 + 3) / 4)));
+    return dim3((unsigned)((slots + p.g.pair_extra) * ((p.g.N / 64 + 3) / 4)));
 }
 
 int moe355::gmm1_w4_pairs(const int8_t* x, const float* x_scale, const int32_t* topk_ids, int64_t num_tokens, int top_k,
