@@ -1,17 +1,21 @@
 """Which calls the whole-layer call takes, and when it looks at the layer again: host code, no GPU."""
-import torch
+import ctypes
+import types
 
 import pytest
+import torch
 
+from vllm_ascend_amd import _lib
 from vllm_ascend_amd.fused_moe.contracts import FusedMoEConfig
 from vllm_ascend_amd.fused_moe.gate_linear import AscendGateLinear
 from vllm_ascend_amd.fused_moe.layer import AscendRoutedExperts
+from vllm_ascend_amd.fused_moe import layer_call as layer_call_module
 from vllm_ascend_amd.fused_moe.layer_call import layer_call
 from vllm_ascend_amd.fused_moe.router import AscendFusedTopKRouter
 from vllm_ascend_amd.fused_moe.shared_experts import AscendSharedExperts
 from vllm_ascend_amd.quantization import get_scheme_class
 
-E, K, H, I = 8, 2, 64, 32
+E, K, H, I = 8, 2, 128, 32
 
 
 def _layer(scheme="W8A8_DYNAMIC", cls=AscendRoutedExperts, shared=False, gate=False):
@@ -91,4 +95,119 @@ def test_a_gate_that_is_any_callable():
     layer = _layer()
     layer.gate = lambda x: (LOGITS, None)
     assert layer_call(layer, X, None) is None
+    assert layer_call(layer, X, LOGITS) is None
+
+
+# ---------------------------------------------------------------- what the library is told
+@pytest.fixture
+def told(monkeypatch):
+    """The descriptions that reach the library, which is not called."""
+    calls = []
+
+    def forward(ref, *args):
+        calls.append(_lib.Layer.from_buffer_copy(ctypes.string_at(ref, ctypes.sizeof(_lib.Layer))))
+        return 0
+
+    lib = types.SimpleNamespace(moe355_layer_forward=forward, moe355_layer_workspace=lambda ref, T: 256)
+    monkeypatch.setattr(_lib, "load", lambda: lib)
+    monkeypatch.setattr(layer_call_module, "_stream", lambda t: 0)
+    return calls
+
+
+def _as_gpu(layer):
+    layer.router.e_score_correction_bias = layer.router.e_score_correction_bias.as_subclass(_Gpu)
+    if layer.gate is not None:
+        for name, p in layer.gate._parameters.items():
+            layer.gate._parameters[name] = p.as_subclass(_Gpu)
+    return layer
+
+
+@pytest.fixture(params=["W8A8_DYNAMIC", "W4A8_DYNAMIC"])
+def scheme(request):
+    return request.param
+
+
+def _laid_out(scheme="W8A8_DYNAMIC", **kw):
+    layer = _layer(scheme, **kw)
+    p = layer._parameters
+    if scheme == "W8A8_DYNAMIC":
+        p["w13_weight"].data, p["w2_weight"].data = (torch.zeros(E, H, 2 * I, dtype=torch.int8),
+                                                     torch.zeros(E, I, H, dtype=torch.int8))
+    else:
+        p["w13_weight"].data, p["w2_weight"].data = (torch.zeros(E, H * I, dtype=torch.uint8),
+                                                     torch.zeros(E, H * I // 2, dtype=torch.uint8))
+        p["w13_weight_scale"].data, p["w2_weight_scale"].data = torch.zeros(E, 1, 2 * I), torch.zeros(E, 1, H)
+    return _as_gpu(layer)
+
+
+def test_a_laid_out_layer_is_one_call(told, scheme):
+    layer = _laid_out(scheme)
+    for _ in range(2):
+        assert layer_call(layer, X, LOGITS) is not None
+    assert len(told) == 2 and told[0].w13 == layer.w13_weight.data_ptr()
+    assert told[1].bias == layer.router.e_score_correction_bias.data_ptr()
+
+
+def test_a_bias_of_another_type_at_the_same_address(told):
+    layer = _laid_out()
+    layer_call(layer, X, LOGITS)
+    fp32 = layer.router.e_score_correction_bias
+    half = layer.router.e_score_correction_bias = fp32.view(torch.bfloat16)[:E]
+    assert half.data_ptr() == fp32.data_ptr()
+    layer_call(layer, X, LOGITS)
+    bias = layer.router.e_score_correction_bias
+    assert bias.dtype == torch.float32 and told[-1].bias == bias.data_ptr() != half.data_ptr()
+
+
+def test_a_narrower_gate_weight_at_the_same_address(told):
+    layer = _laid_out(gate=True)
+    assert layer_call(layer, X, None) is not None
+    weight = layer.gate._parameters["weight"]
+    layer.gate._parameters["weight"] = weight.view(-1)[: E * H // 2].view(E, H // 2)
+    assert layer.gate._parameters["weight"].data_ptr() == weight.data_ptr()
+    assert layer_call(layer, X, None) is None  # the gate refuses it
+
+
+# tensors that the operators convert, copy or refuse: at another address, or at the one that a plan was made with
+CHANGED = {
+    "weight of another shape": ("w13_weight", lambda t: t.data.view(E, 2 * I, H)),
+    "weight that is not contiguous": ("w2_weight", lambda t: torch.zeros(E, H, I, dtype=torch.int8).transpose(1, 2)),
+    "scale of another type, same address": ("w13_weight_scale_fp32",
+                                            lambda t: t.view(torch.float16)[:, : 2 * I].reshape(-1)[: E * 2 * I]),
+    "scale of another type": ("w2_weight_scale_fp32", lambda t: t.double()),
+    "scale with too few values": ("w2_weight_scale_fp32", lambda t: t[: E // 2]),
+    "scale that is not contiguous": ("w2_weight_scale_fp32", lambda t: torch.zeros(H, E).t()),
+}
+
+
+@pytest.mark.parametrize("planned", [False, True])
+@pytest.mark.parametrize("what", list(CHANGED))
+def test_tensors_the_library_cannot_read(told, what, planned):
+    layer = _laid_out()
+    if planned:
+        assert layer_call(layer, X, LOGITS) is not None
+    name, change = CHANGED[what]
+    if name in layer._parameters:
+        layer._parameters[name].data = change(layer._parameters[name])
+    else:
+        setattr(layer, name, change(getattr(layer, name)))
+    assert layer_call(layer, X, LOGITS) is None
+
+
+SHARED_CHANGED = {
+    "weight that is not contiguous": ("gate_up_weight", lambda t: torch.zeros(2 * I, H, dtype=torch.int8).t()),
+    "weight of another type": ("down_weight", lambda t: t.to(torch.int32)),
+    "scale of another type": ("down_scale_fp32", lambda t: t.half()),
+    "scale with too few values": ("gate_up_scale_fp32", lambda t: t[:I]),
+}
+
+
+@pytest.mark.parametrize("planned", [False, True])
+@pytest.mark.parametrize("what", list(SHARED_CHANGED))
+def test_shared_expert_tensors_the_library_cannot_read(told, what, planned):
+    layer = _laid_out(shared=True)
+    if planned:
+        assert layer_call(layer, X, LOGITS) is not None
+    name, change = SHARED_CHANGED[what]
+    setattr(layer.shared_experts, name, change(getattr(layer.shared_experts, name)))
     assert layer_call(layer, X, LOGITS) is None

@@ -23,13 +23,12 @@ from .shared_experts import AscendSharedExperts, shared_experts_calculation_stre
 
 _MAX_SIZES = 256  # batch sizes whose scratch size is remembered
 _INT8, _INT8_LIST, _INT4 = 0, 1, 2  # moe355_layer.weights
-_WEIGHTS = 2  # ... and where a key holds it
 
 
 class _Plan:
     """What one layer looks like to the library; ``desc`` is None when the native call cannot take it."""
 
-    __slots__ = ("key", "desc", "ref", "hidden", "experts", "sizes", "forward", "workspace")
+    __slots__ = ("key", "desc", "ref", "hidden", "experts", "sizes", "bias", "forward", "workspace")
 
     def __init__(self, key):
         self.key = key
@@ -40,8 +39,19 @@ class _Plan:
         return type(None), ()
 
 
-def _ptr(t):
-    return None if t is None else t.data_ptr()
+def _view(t):
+    """What the library is told of a tensor (its address) and what that address stands for.  All of it is compared on
+    every call and nothing keeps a tensor alive: an address alone may belong to another tensor of another type or size
+    by the time of the next call."""
+    return t.data_ptr(), t.dtype, t.shape, t.is_contiguous(), t.get_device()
+
+
+def _is(view, dtype, shape, device):
+    return view[1:] == (dtype, shape, True, device)
+
+
+def _holds(view, dtype, numel, device):
+    return view[1] == dtype and view[2].numel() == numel and view[3:] == (True, device)
 
 
 # what of a layer, its router and its shared expert a plan is made from
@@ -55,11 +65,11 @@ _ROUTER = itemgetter("top_k", "renormalize", "num_expert_group", "topk_group", "
 _SHARED = itemgetter("multistream_overlap", "swiglu_limit", "swiglu_alpha", "swiglu_beta", "gate_up_weight",
                      "down_weight", "gate_up_scale_fp32", "down_scale_fp32", "_forward_hooks", "_forward_pre_hooks")
 _INT8_SCALES = itemgetter("w13_weight_scale_fp32", "w2_weight_scale_fp32")
-_INT4_TENSORS = itemgetter("w13_weight", "w2_weight", "w13_weight_scale", "w2_weight_scale")
+_INT4_TENSORS = itemgetter("w13_weight", "w13_weight_scale", "w2_weight", "w2_weight_scale")
 _LISTS = itemgetter("w13_weight_list", "w13_weight_scale_fp32_list", "w2_weight_list", "w2_weight_scale_list")
 
 
-def _key(layer, x_dtype, logits_dtype):
+def _key(layer, x_dtype, device, logits_dtype):
     """Everything that the plan of such a call is made from, or None where the call goes operator by operator: an
     option or a part that the library has no whole form for, or a layer that is not put together as
     ``AscendRoutedExperts.__init__`` and the two schemes do it (another scheme, router or shared expert, a gate that is
@@ -80,13 +90,13 @@ def _key(layer, x_dtype, logits_dtype):
         p = d["_parameters"]
         if type(q) is AscendW8A8DynamicFusedMoEMethod:
             if q.use_expert_weight_list:
-                weights, w = _INT8_LIST, tuple(t.table.data_ptr() for t in _LISTS(d))
+                weights, w = _INT8_LIST, tuple((len(t), t.table.data_ptr(), _view(t[0])) for t in _LISTS(d))
             else:
                 s13, s2 = _INT8_SCALES(d)
                 weights = _INT8
-                w = (p["w13_weight"].data_ptr(), p["w2_weight"].data_ptr(), s13.data_ptr(), s2.data_ptr())
+                w = (_view(p["w13_weight"]), _view(s13), _view(p["w2_weight"]), _view(s2))
         elif type(q) is AscendW4A8DynamicFusedMoEMethod and not q.use_expert_weight_list:
-            weights, w = _INT4, tuple(t.data_ptr() for t in _INT4_TENSORS(p))
+            weights, w = _INT4, tuple(_view(t) for t in _INT4_TENSORS(p))
         else:
             return None
         if q.in_dtype != x_dtype:
@@ -102,7 +112,7 @@ def _key(layer, x_dtype, logits_dtype):
             sh = _SHARED(shared.__dict__)
             if sh[8] or sh[9]:
                 return None  # hooks
-            sh = (*sh[:4], sh[4].data_ptr(), sh[5].data_ptr(), sh[6].data_ptr(), sh[7].data_ptr())
+            sh = (*sh[:4], _view(sh[4]), _view(sh[5]), _view(sh[6]), _view(sh[7]))
         if logits_dtype is None:
             gate = m["gate"] if "gate" in m else d["gate"]
             if type(gate) is not AscendGateLinear:
@@ -112,88 +122,100 @@ def _key(layer, x_dtype, logits_dtype):
                 return None
             gp = s["_parameters"]
             gate_bias = gp["bias"] if "bias" in gp else s["bias"]
-            g = (gp["weight"].data_ptr(), None if gate_bias is None else gate_bias.data_ptr())
+            g = (_view(gp["weight"]), None if gate_bias is None else _view(gate_bias))
         if eplb and collecting:
             if staged:
                 return None  # one row of loads per pass, indexed on the device
-            load = d["_buffers"]["moe_load"].data_ptr()
-        return (x_dtype, logits_dtype, weights, w, sh, g, routing[:6], None if bias is None else bias.data_ptr(), pair_order,
-                load, cfg.num_experts, cfg.hidden_dim, cfg.intermediate_size_per_partition, cfg.swiglu_limit)
+            load = _view(d["_buffers"]["moe_load"])
+        return (x_dtype, device, logits_dtype, weights, w, sh, g, routing[:6], None if bias is None else _view(bias),
+                pair_order, load, cfg.num_experts, cfg.hidden_dim, cfg.intermediate_size_per_partition,
+                cfg.swiglu_limit)
     except (AttributeError, KeyError):
         return None
 
 
 def _make_plan(layer, x, logits, key) -> _Plan:
+    """What the key says, as the library takes it; no description where a tensor is not what the library would read
+    (weights that have not been laid out, a scale of another type, a tensor elsewhere): the operators convert it or say
+    what is wrong with it."""
     logits_dtype = torch.float32 if logits is None else logits.dtype
-    r, gate, shared, cfg = layer.router, layer.gate, layer.shared_experts, layer.moe_config
+    r = layer.router
     plan = _Plan(key)
     if x.dtype not in (torch.bfloat16, torch.float16) or not r.is_fused_supported(x):
         return plan
     bias = r.e_score_correction_bias
-    if bias is not None:
-        if bias.dtype != logits_dtype:
-            bias = r.e_score_correction_bias = bias.to(logits_dtype)
-            plan.key = _key(layer, x.dtype, None if logits is None else logits_dtype)
-        if bias.dim() != 1 or bias.numel() != cfg.num_experts or not bias.is_contiguous() or not bias.is_cuda:
+    if bias is not None and bias.dtype != logits_dtype:
+        bias = r.e_score_correction_bias = bias.to(logits_dtype)
+        key = plan.key = _key(layer, x.dtype, x.get_device(), None if logits is None else logits_dtype)
+        if key is None:
             return plan
-    lib = _lib.load()
-    E, I = cfg.num_experts, cfg.intermediate_size_per_partition
-    a = _lib.Layer()
-    a.hidden, a.intermediate, a.num_experts, a.top_k = cfg.hidden_dim, I, E, r.top_k
-    a.k_group = r.topk_group if r.topk_group is not None else 1
-    a.group_count = r.num_expert_group if r.num_expert_group is not None else 1
-    a.renorm, a.norm_type = int(r.renormalize), 0 if r.scoring_func == "softmax" else 1
-    a.routed_scaling_factor, a.eps, a.swiglu_limit = r.routed_scaling_factor, 1e-20, cfg.swiglu_limit or 0.0
-    a.x_dtype, a.bias = _DT[x.dtype], _ptr(bias)
-    a.weights = key[_WEIGHTS]
-    if a.weights == _INT8_LIST:
-        lists = (layer.w13_weight_list, layer.w13_weight_scale_fp32_list, layer.w2_weight_list,
-                 layer.w2_weight_scale_list)
-        a.w13, a.s13, a.w2, a.s2 = (t.table.data_ptr() for t in lists)
-        sizes = [(t[0].numel() * len(t), t[0].dtype) for t in lists]
-    elif a.weights == _INT4:
-        s13, s2 = layer.w13_weight_scale, layer.w2_weight_scale
-        a.group13, a.group2 = cfg.hidden_dim // s13.shape[1], I // s2.shape[1]
-        tensors = (layer.w13_weight, s13, layer.w2_weight, s2)
-        a.w13, a.s13, a.w2, a.s2 = (t.data_ptr() for t in tensors)
-        sizes = [(t.numel() * (2 if t.dtype == torch.uint8 else 1), t.dtype) for t in tensors]
+    # another thread's call with logits of another type may replace the converted bias while this call uses it
+    plan.bias = bias
+    (_, dev, _, weights, w, sh, g, routing, bias_view, pair_order, load, E, H, I, limit) = key
+    if bias_view is not None and not _is(bias_view, logits_dtype, (E,), dev):
+        return plan
+    if weights == _INT8_LIST:
+        if any(n != E for n, _, _ in w):
+            return plan
+        addresses, (w13, s13, w2, s2) = [table for _, table, _ in w], [first for _, _, first in w]
+        if not (_is(w13, torch.int8, (H, 2 * I), dev) and _holds(s13, torch.float32, 2 * I, dev)
+                and _is(w2, torch.int8, (I, H), dev) and _holds(s2, torch.float32, H, dev)):
+            return plan
     else:
-        tensors = (layer.w13_weight, layer.w13_weight_scale_fp32, layer.w2_weight, layer.w2_weight_scale_fp32)
-        a.w13, a.s13, a.w2, a.s2 = (t.data_ptr() for t in tensors)
-        sizes = [(t.numel(), t.dtype) for t in tensors]
-    H = cfg.hidden_dim
-    per13, per2 = (H // a.group13, I // a.group2) if a.weights == _INT4 else (1, 1)
-    wtype = torch.uint8 if a.weights == _INT4 else torch.int8
-    if sizes != [(E * 2 * I * H, wtype), (E * 2 * I * per13, torch.float32), (E * H * I, wtype),
-                 (E * H * per2, torch.float32)]:
-        return plan  # not laid out (process_weights_after_loading has not run): the operators say what is wrong
-    a.pair_order = int(layer.use_pair_order)
-    if a.weights == _INT4 or not a.pair_order:
+        addresses, (w13, s13, w2, s2) = [view[0] for view in w], w
+        if weights == _INT8:
+            if not (_is(w13, torch.int8, (E, H, 2 * I), dev) and _holds(s13, torch.float32, E * 2 * I, dev)
+                    and _is(w2, torch.int8, (E, I, H), dev) and _holds(s2, torch.float32, E * H, dev)):
+                return plan
+        else:
+            if len(s13[2]) != 3 or len(s2[2]) != 3:
+                return plan
+            G13, G2 = s13[2][1], s2[2][1]
+            if not (_holds(w13, torch.uint8, E * I * H, dev) and _is(s13, torch.float32, (E, G13, 2 * I), dev)
+                    and _holds(w2, torch.uint8, E * H * I // 2, dev) and _is(s2, torch.float32, (E, G2, H), dev)):
+                return plan
+    lib = _lib.load()
+    a = _lib.Layer()
+    a.hidden, a.intermediate, a.num_experts = H, I, E
+    a.top_k, renormalize, group_count, k_group, scoring_func, a.routed_scaling_factor = routing
+    a.k_group = k_group if k_group is not None else 1
+    a.group_count = group_count if group_count is not None else 1
+    a.renorm, a.norm_type = int(renormalize), 0 if scoring_func == "softmax" else 1
+    a.eps, a.swiglu_limit = 1e-20, limit or 0.0
+    a.x_dtype, a.bias = _DT[x.dtype], None if bias_view is None else bias_view[0]
+    a.weights = weights
+    a.w13, a.s13, a.w2, a.s2 = addresses
+    if weights == _INT4:
+        a.group13, a.group2 = H // G13, I // G2
+    a.pair_order = int(pair_order)
+    if weights == _INT4 or not a.pair_order:
         # the sorting launch's arrival counter, shared with the operator-by-operator path
         counter = getattr(layer, "_small_batch_counter", None)
         if counter is None or counter.device != x.device:
             counter = layer._small_batch_counter = torch.zeros((1,), dtype=torch.int32, device=x.device)
         a.sync_counter = counter.data_ptr()
-    if logits is None:
-        w, gb = gate.weight, gate.bias
-        if tuple(w.shape) != (E, H) or w.dtype != torch.float32 or not w.is_contiguous() or not w.is_cuda:
+    if g is not None:
+        weight, gate_bias = g
+        if not _is(weight, torch.float32, (E, H), dev):
             return plan
-        if gb is not None and (gb.dtype != torch.float32 or gb.numel() != E or not gb.is_contiguous()):
+        if gate_bias is not None and not _holds(gate_bias, torch.float32, E, dev):
             return plan
-        a.gate_weight, a.gate_bias = w.data_ptr(), _ptr(gb)
-    if shared is not None:
-        h, n = shared.gate_up_weight.shape
-        if h != H or n % 2 or tuple(shared.down_weight.shape) != (n // 2, H):
+        a.gate_weight, a.gate_bias = weight[0], None if gate_bias is None else gate_bias[0]
+    if sh is not None:
+        overlap, a.shared_limit, a.shared_alpha, a.shared_beta, up, down, up_scale, down_scale = sh
+        n = up[2][1] if len(up[2]) == 2 else 1
+        if n % 2 or not (_is(up, torch.int8, (H, n), dev) and _is(down, torch.int8, (n // 2, H), dev)
+                         and _holds(up_scale, torch.float32, n, dev) and _holds(down_scale, torch.float32, H, dev)):
             return plan
         a.shared_intermediate = n // 2
-        a.shared = 2 if shared.multistream_overlap else 1
-        a.shared_limit, a.shared_alpha, a.shared_beta = (shared.swiglu_limit, shared.swiglu_alpha, shared.swiglu_beta)
-        a.shared_w13, a.shared_w2 = shared.gate_up_weight.data_ptr(), shared.down_weight.data_ptr()
-        a.shared_s13, a.shared_s2 = shared.gate_up_scale_fp32.data_ptr(), shared.down_scale_fp32.data_ptr()
-        if a.shared == 2:
+        a.shared = 2 if overlap else 1
+        a.shared_w13, a.shared_s13, a.shared_w2, a.shared_s2 = up[0], up_scale[0], down[0], down_scale[0]
+        if overlap:
             a.shared_stream = shared_experts_calculation_stream().cuda_stream
-    if layer.dynamic_eplb and layer.eplb_heat_collection_status:
-        a.load = layer.moe_load.data_ptr()
+    if load is not None:
+        if not _is(load, torch.int64, (E,), dev):
+            return plan
+        a.load = load[0]
     plan.desc, plan.ref = a, ctypes.addressof(a)
     plan.hidden, plan.experts = H, E
     plan.forward, plan.workspace = lib.moe355_layer_forward, lib.moe355_layer_workspace
@@ -203,7 +225,8 @@ def _make_plan(layer, x, logits, key) -> _Plan:
 def layer_call(layer, x: torch.Tensor, logits: torch.Tensor | None) -> torch.Tensor | None:
     """The layer's output, or None when the call has to go operator by operator (an option the library has no whole
     form for, or arguments that the operators refuse with a message of their own)."""
-    key = _key(layer, x.dtype, None if logits is None else logits.dtype)
+    device = x.get_device()
+    key = _key(layer, x.dtype, device, None if logits is None else logits.dtype)
     shape = x.shape
     if key is None or not x.is_cuda or len(shape) != 2:
         return None
@@ -221,7 +244,7 @@ def layer_call(layer, x: torch.Tensor, logits: torch.Tensor | None) -> torch.Ten
     if T == 0:
         return None
     if logits is not None:
-        if logits.shape != (T, plan.experts) or not logits.is_contiguous() or not logits.is_cuda:
+        if logits.shape != (T, plan.experts) or not logits.is_contiguous() or logits.get_device() != device:
             return None
         logits_ptr, logits_dtype = logits.data_ptr(), _DT[logits.dtype]
     else:
