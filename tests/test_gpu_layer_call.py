@@ -138,3 +138,22 @@ def test_the_call_follows_the_layer():
     assert torch.equal(layer(x[::2], logits[::2]), layer.forward_impl(x[::2], logits[::2]).routed_out)
     twin = copy.deepcopy(layer)
     assert torch.equal(twin(x, logits), layer.forward_impl(x, logits).routed_out)
+
+
+@pytest.mark.parametrize("name", ["c2_small", "c5_small"])
+def test_a_router_with_a_selection_of_its_own(name):
+    """Its ids are the ones the experts run on, through the call and through the operators."""
+    cfg, layer, x, logits = _pair(name, 40)
+    stock = layer(x, logits)
+    select, seen = layer.router.select_experts, []
+
+    def shifted(*a, **kw):
+        weights, ids = select(*a, **kw)
+        seen.append(1)
+        return weights, ((ids + 1) % cfg.E).to(torch.int32)
+
+    layer.router.select_experts = shifted
+    weights, ids = shifted(x, logits)
+    want = layer.quant_method.apply(layer, x, weights, ids, None, None).routed_out
+    assert torch.equal(layer(x, logits), want) and torch.equal(layer.forward_impl(x, logits).routed_out, want)
+    assert len(seen) == 3 and not torch.equal(want, stock)

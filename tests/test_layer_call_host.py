@@ -211,3 +211,81 @@ def test_shared_expert_tensors_the_library_cannot_read(told, what, planned):
     name, change = SHARED_CHANGED[what]
     setattr(layer.shared_experts, name, change(getattr(layer.shared_experts, name)))
     assert layer_call(layer, X, LOGITS) is None
+
+
+# ---------------------------------------------------------------- methods of the caller's in the layer
+def _wrapped(obj, name):
+    fn = getattr(obj, name)
+    setattr(obj, name, lambda *a, **kw: fn(*a, **kw))
+
+
+REPLACED = {
+    "router.select_experts": lambda l: _wrapped(l.router, "select_experts"),
+    "router.is_fused_supported": lambda l: _wrapped(l.router, "is_fused_supported"),
+    "quant_method.apply_small_batch": lambda l: _wrapped(l.quant_method, "apply_small_batch"),
+    "moe_comm_method.finalize": lambda l: _wrapped(l.moe_comm_method, "finalize"),
+    "prepare_finalize.prepare": lambda l: _wrapped(l.moe_comm_method.prepare_finalize, "prepare"),
+    "shared_experts.forward": lambda l: _wrapped(l.shared_experts, "forward"),
+    "a hook of the shared expert": lambda l: l.shared_experts.register_forward_hook(lambda *a: None),
+    "gate.forward": lambda l: _wrapped(l.gate, "forward"),
+    "a hook of the gate": lambda l: l.gate.register_forward_pre_hook(lambda *a: None),
+}
+
+
+@pytest.mark.parametrize("planned", [False, True])
+@pytest.mark.parametrize("what", list(REPLACED))
+def test_replaced_methods_are_not_passed_by(told, what, planned):
+    layer = _laid_out(shared=True, gate=True)
+    if planned:
+        assert layer_call(layer, X, None) is not None
+    REPLACED[what](layer)
+    assert layer_call(layer, X, None) is None
+
+
+@pytest.mark.parametrize("cls, name", [(AscendFusedTopKRouter, "select_experts"), (AscendSharedExperts, "forward"),
+                                       (AscendGateLinear, "forward"),
+                                       (get_scheme_class("W8A8_DYNAMIC", "moe"), "apply_small_batch")])
+def test_patched_classes_are_not_passed_by(told, monkeypatch, cls, name):
+    layer = _laid_out(shared=True, gate=True)
+    assert layer_call(layer, X, None) is not None
+    fn = getattr(cls, name)
+    monkeypatch.setattr(cls, name, lambda *a, **kw: fn(*a, **kw))
+    assert layer_call(layer, X, None) is None
+
+
+@pytest.mark.parametrize("name", ["forward_impl", "_run_experts", "_record_expert_load"])
+@pytest.mark.parametrize("where", ["subclass", "instance", "class"])
+def test_a_layer_with_a_form_of_its_own(told, monkeypatch, name, where):
+    class Own(AscendRoutedExperts):
+        pass
+
+    layer = _laid_out(cls=Own)
+    assert layer(X, LOGITS) is not None and len(told) == 1  # a subclass alone changes nothing
+    owner = {"subclass": Own, "instance": layer, "class": AscendRoutedExperts}[where]
+    seen = []
+    result = types.SimpleNamespace(routed_out=X)
+    monkeypatch.setattr(owner, name, lambda *a, **kw: seen.append(name) or result)
+    if name == "_record_expert_load":  # called behind the operators, which the library of this test does not have
+        with pytest.raises(AttributeError, match="moe355_"):
+            layer(X, LOGITS)
+    else:
+        assert layer(X, LOGITS) is X and seen == [name]
+    assert len(told) == 1
+
+
+def test_routers_that_select_by_themselves():
+    from vllm_ascend_amd.fused_moe.router import replaces_selection
+
+    class Sub(AscendFusedTopKRouter):
+        pass
+
+    class Own(AscendFusedTopKRouter):
+        def _compute_routing(self, *a, **kw):
+            return super()._compute_routing(*a, **kw)
+
+    assert not replaces_selection(AscendFusedTopKRouter(K, E)) and not replaces_selection(Sub(K, E))
+    assert not replaces_selection(types.SimpleNamespace(top_k=K))  # numbers alone
+    assert replaces_selection(Own(K, E)) and replaces_selection(types.SimpleNamespace(select_experts=None))
+    router = AscendFusedTopKRouter(K, E)
+    _wrapped(router, "select_experts")
+    assert replaces_selection(router)

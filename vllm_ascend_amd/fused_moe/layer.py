@@ -137,12 +137,22 @@ class AscendRoutedExperts(torch.nn.Module):
 
     def forward(self, hidden_states: torch.Tensor, router_logits: torch.Tensor | None = None) -> torch.Tensor:
         # the whole layer in one native call where it can take this one; nobody reads the events and intermediate
-        # tensors of a FusedExpertsResult here
-        out = layer_call(self, hidden_states, router_logits)
-        if out is not None:
-            return out
+        # tensors of a FusedExpertsResult here.  A subclass (or a patch) that runs the experts or records their load in
+        # its own way goes on through forward_impl.
+        cls, d = type(self), self.__dict__
+        if (cls.forward_impl is _FORWARD_IMPL and cls._run_experts is _RUN_EXPERTS
+                and cls._record_expert_load is _RECORD_EXPERT_LOAD and "forward_impl" not in d
+                and "_run_experts" not in d and "_record_expert_load" not in d):
+            out = layer_call(self, hidden_states, router_logits)
+            if out is not None:
+                return out
         if router_logits is None:
             if self.gate is None:
                 raise ValueError("router_logits is required: this layer was built without an internal gate")
             router_logits, _ = self.gate(hidden_states)
         return self.forward_impl(hidden_states, router_logits).routed_out
+
+
+_FORWARD_IMPL = AscendRoutedExperts.forward_impl
+_RUN_EXPERTS = AscendRoutedExperts._run_experts
+_RECORD_EXPERT_LOAD = AscendRoutedExperts._record_expert_load

@@ -11,6 +11,7 @@ import ctypes
 from operator import itemgetter
 
 import torch
+from torch.nn.modules.module import _global_forward_hooks, _global_forward_pre_hooks
 
 from .. import _lib
 from ..kernels import _DT, _stream
@@ -64,6 +65,11 @@ _ROUTER = itemgetter("top_k", "renormalize", "num_expert_group", "topk_group", "
                      "routed_scaling_factor", "e_score_correction_bias")
 _SHARED = itemgetter("multistream_overlap", "swiglu_limit", "swiglu_alpha", "swiglu_beta", "gate_up_weight",
                      "down_weight", "gate_up_scale_fp32", "down_scale_fp32", "_forward_hooks", "_forward_pre_hooks")
+# what a call runs when nothing has been put in its place, in a subclass, on an instance or in the class itself
+_SELECT_EXPERTS, _GUARD = AscendFusedTopKRouter.select_experts, AscendFusedTopKRouter.is_fused_supported
+_SHARED_FORWARD, _GATE_FORWARD = AscendSharedExperts.forward, AscendGateLinear.forward
+_INT8_APPLY = AscendW8A8DynamicFusedMoEMethod.apply_small_batch
+_INT4_APPLY = AscendW4A8DynamicFusedMoEMethod.apply_small_batch
 _INT8_SCALES = itemgetter("w13_weight_scale_fp32", "w2_weight_scale_fp32")
 _INT4_TENSORS = itemgetter("w13_weight", "w13_weight_scale", "w2_weight", "w2_weight_scale")
 _LISTS = itemgetter("w13_weight_list", "w13_weight_scale_fp32_list", "w2_weight_list", "w2_weight_scale_list")
@@ -73,7 +79,8 @@ def _key(layer, x_dtype, device, logits_dtype):
     """Everything that the plan of such a call is made from, or None where the call goes operator by operator: an
     option or a part that the library has no whole form for, or a layer that is not put together as
     ``AscendRoutedExperts.__init__`` and the two schemes do it (another scheme, router or shared expert, a gate that is
-    any callable, a tensor registered under the name of an attribute).  Compared on every call, so plain dictionary
+    any callable, a tensor registered under the name of an attribute), or one with a method or hook of the caller's in
+    it.  Compared on every call, so plain dictionary
     lookups: types first, then what such types have."""
     d = layer.__dict__
     try:
@@ -87,8 +94,17 @@ def _key(layer, x_dtype, device, logits_dtype):
         if type(r) is not AscendFusedTopKRouter or type(comm) is not AllGatherCommImpl \
                 or type(comm.prepare_finalize) is not _IdentityPrepareFinalize:
             return None
+        rd, qd, cd = r.__dict__, q.__dict__, comm.__dict__
+        if (AscendFusedTopKRouter.select_experts is not _SELECT_EXPERTS or "select_experts" in rd
+                or "_compute_routing" in rd or AscendFusedTopKRouter.is_fused_supported is not _GUARD
+                or "is_fused_supported" in rd or "apply_small_batch" in qd or "supports_small_batch" in qd
+                or "apply" in qd or "prepare" in cd or "finalize" in cd or "fused_experts" in cd
+                or comm.prepare_finalize.__dict__):
+            return None
         p = d["_parameters"]
         if type(q) is AscendW8A8DynamicFusedMoEMethod:
+            if AscendW8A8DynamicFusedMoEMethod.apply_small_batch is not _INT8_APPLY:
+                return None
             if q.use_expert_weight_list:
                 weights, w = _INT8_LIST, tuple((len(t), t.table.data_ptr(), _view(t[0])) for t in _LISTS(d))
             else:
@@ -96,12 +112,14 @@ def _key(layer, x_dtype, device, logits_dtype):
                 weights = _INT8
                 w = (_view(p["w13_weight"]), _view(s13), _view(p["w2_weight"]), _view(s2))
         elif type(q) is AscendW4A8DynamicFusedMoEMethod and not q.use_expert_weight_list:
+            if AscendW4A8DynamicFusedMoEMethod.apply_small_batch is not _INT4_APPLY:
+                return None
             weights, w = _INT4, tuple(_view(t) for t in _INT4_TENSORS(p))
         else:
             return None
         if q.in_dtype != x_dtype:
             return None
-        routing = _ROUTER(r.__dict__)
+        routing = _ROUTER(rd)
         bias = routing[6]
         m = d["_modules"]
         shared = m["shared_experts"] if "shared_experts" in m else d["shared_experts"]
@@ -109,16 +127,19 @@ def _key(layer, x_dtype, device, logits_dtype):
         if shared is not None:
             if type(shared) is not AscendSharedExperts:
                 return None
-            sh = _SHARED(shared.__dict__)
-            if sh[8] or sh[9]:
-                return None  # hooks
+            s = shared.__dict__
+            sh = _SHARED(s)
+            if (AscendSharedExperts.forward is not _SHARED_FORWARD or "forward" in s or "_mlp" in s or "wait" in s
+                    or sh[8] or sh[9] or _global_forward_hooks or _global_forward_pre_hooks):
+                return None
             sh = (*sh[:4], _view(sh[4]), _view(sh[5]), _view(sh[6]), _view(sh[7]))
         if logits_dtype is None:
             gate = m["gate"] if "gate" in m else d["gate"]
             if type(gate) is not AscendGateLinear:
                 return None
             s = gate.__dict__
-            if s["_forward_hooks"] or s["_forward_pre_hooks"]:
+            if (AscendGateLinear.forward is not _GATE_FORWARD or "forward" in s or s["_forward_hooks"]
+                    or s["_forward_pre_hooks"] or _global_forward_hooks or _global_forward_pre_hooks):
                 return None
             gp = s["_parameters"]
             gate_bias = gp["bias"] if "bias" in gp else s["bias"]

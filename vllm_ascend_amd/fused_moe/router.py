@@ -79,3 +79,13 @@ class AscendFusedTopKRouter:
         if indices_type is not None and topk_ids.dtype != indices_type:
             topk_ids = topk_ids.to(indices_type)
         return topk_weights, topk_ids
+
+
+_SELECTION = {name: getattr(AscendFusedTopKRouter, name) for name in ("select_experts", "_compute_routing")}
+
+
+def replaces_selection(router) -> bool:
+    """Whether a router chooses experts in a way of its own (a subclass, another class, a method set on the instance):
+    the forms that run the gating op themselves, from the router's numbers, must not take such a call."""
+    return any(name in getattr(router, "__dict__", ()) or getattr(type(router), name, fn) is not fn
+               for name, fn in _SELECTION.items())

@@ -54,12 +54,15 @@ class AscendMoEScheme(ABC):
 # ---------------------------------------------------------------------- router + token quantisation, fused
 def fused_front_supported(layer, x: torch.Tensor, router_logits: torch.Tensor, router) -> bool:
     """Whether :func:`route_and_quantize` can take the call: 2-D logits of a supported type, no forced load
-    balance, at most 256 experts."""
+    balance, at most 256 experts, and a router whose selection is the fused op's."""
     from .. import kernels
+    from ..fused_moe.router import replaces_selection
 
     if router_logits.dim() != 2 or router_logits.dtype not in (torch.float32, torch.bfloat16, torch.float16):
         return False
     if getattr(layer, "enable_force_load_balance", False):
+        return False
+    if replaces_selection(router):
         return False
     guard = getattr(router, "is_fused_supported", None)
     if guard is not None and not guard(x):
