@@ -523,7 +523,9 @@ typedef struct moe355_layer {
     int32_t pair_order;       /* 0: never; 1: where moe355_pair_order() says so (weights 0 and 1) */
     const void *w13, *s13, *w2, *s2;
     int64_t group13, group2;  /* int4: weights along K that share a scale */
-    int32_t *sync_counter;    /* of moe355_route_quant_small; NULL: that launch is not used */
+    /* of moe355_route_quant_small, for a caller that runs the layer on one stream or graph at a time; NULL: that launch
+     * is not used, and calls may overlap in time as long as they share neither workspace nor output */
+    int32_t *sync_counter;
     /* router gate inside the layer, or NULL */
     const float *gate_weight, *gate_bias;
     /* shared expert: 0 none, 1 in line, 2 on shared_stream next to the routed experts */

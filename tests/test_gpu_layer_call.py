@@ -2,6 +2,7 @@
 (``layer.forward_impl``): the same bits, over the forms the call chooses between."""
 import copy
 import dataclasses
+import threading
 
 import pytest
 import torch
@@ -157,3 +158,78 @@ def test_a_router_with_a_selection_of_its_own(name):
     want = layer.quant_method.apply(layer, x, weights, ids, None, None).routed_out
     assert torch.equal(layer(x, logits), want) and torch.equal(layer.forward_impl(x, logits).routed_out, want)
     assert len(seen) == 3 and not torch.equal(want, stock)
+
+
+# one layer, several calls at a time: sorted batches small enough for one routing workgroup, pair order, the kernels for
+# a few tokens, the shared expert on its side stream
+AT_A_TIME = [("c5_small", 60, {}, {}), ("c2_small", 48, {}, dict(use_pair_order=False)), ("c2_small", 48, {}, {}),
+             ("c4_small", 8, dict(shared=True, overlap=True), {}),
+             ("c4_small", 300, dict(shared=True, overlap=True), {}),
+             ("c4_small", 96, dict(shared=True, overlap=True), dict(use_pair_order=False))]
+
+
+def _two_batches(name, tokens, kw, options):
+    cfg, layer, x, logits = _pair(name, tokens, **kw)
+    for k, v in options.items():
+        setattr(layer, k, v)
+    batches = [(x, logits), (x.flip(0).contiguous(), logits.roll(1, 1).contiguous()[: tokens - 1])]
+    batches[1] = (batches[1][0][: tokens - 1], batches[1][1])
+    return layer, batches, [layer.forward_impl(*b).routed_out for b in batches]
+
+
+@pytest.mark.parametrize("name, tokens, kw, options", AT_A_TIME)
+def test_one_layer_on_two_streams(name, tokens, kw, options):
+    print(f"two streams: {name} {tokens} {kw} {options}", flush=True)
+    layer, batches, want = _two_batches(name, tokens, kw, options)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    got = [[], []]
+    for _ in range(20):
+        for s, b, out in zip(streams, batches, got):
+            with torch.cuda.stream(s):
+                out.append(layer(*b))
+    torch.cuda.synchronize()
+    for out, w in zip(got, want):
+        assert all(torch.equal(o, w) for o in out)
+
+
+@pytest.mark.parametrize("name, tokens, kw, options", AT_A_TIME)
+def test_one_layer_on_two_threads(name, tokens, kw, options):
+    print(f"two threads: {name} {tokens} {kw} {options}", flush=True)
+    layer, batches, want = _two_batches(name, tokens, kw, options)
+    torch.cuda.synchronize()
+    got, failed = [[], []], []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(20):
+                    got[i].append(layer(*batches[i]))
+                torch.cuda.current_stream().synchronize()
+        except Exception as exc:  # noqa: BLE001 -- reported by the test's own thread
+            failed.append(exc)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not failed
+    for out, w in zip(got, want):
+        assert len(out) == 20 and all(torch.equal(o, w) for o in out)
+
+
+@pytest.mark.parametrize("name", ["c5_small", "c2_small"])
+def test_gating_sort_and_quantisation_in_one_launch(name):
+    """The form of a caller of the library that runs the layer on one stream and brings the counter."""
+    cfg, layer, x, logits = _pair(name, 60)
+    layer.use_pair_order = False
+    want = layer(x, logits)
+    counter = torch.zeros(1, dtype=torch.int32, device=DEV)
+    plan = layer._layer_plan
+    plan.desc.sync_counter = counter.data_ptr()
+    plan.sizes.clear()
+    for _ in range(3):
+        assert torch.equal(layer(x, logits), want)
+    assert layer._layer_plan is plan and int(counter) == 0

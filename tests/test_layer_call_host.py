@@ -289,3 +289,14 @@ def test_routers_that_select_by_themselves():
     router = AscendFusedTopKRouter(K, E)
     _wrapped(router, "select_experts")
     assert replaces_selection(router)
+
+
+# ---------------------------------------------------------------- state that calls would share
+@pytest.mark.parametrize("pair_order", [True, False])
+def test_no_counter_is_shared_between_calls(told, scheme, pair_order):
+    """A launch that counts its workgroups on device memory must not share it with one that may run at the same time:
+    the layer has no such memory, whatever form it takes."""
+    layer = _laid_out(scheme)
+    layer.use_pair_order = pair_order
+    assert layer_call(layer, X, LOGITS) is not None
+    assert not told[-1].sync_counter

@@ -208,13 +208,8 @@ def _make_plan(layer, x, logits, key) -> _Plan:
     a.w13, a.s13, a.w2, a.s2 = addresses
     if weights == _INT4:
         a.group13, a.group2 = H // G13, I // G2
+    # no sync_counter: one counter would be shared by all the streams, threads and graphs that run the layer
     a.pair_order = int(pair_order)
-    if weights == _INT4 or not a.pair_order:
-        # the sorting launch's arrival counter, shared with the operator-by-operator path
-        counter = getattr(layer, "_small_batch_counter", None)
-        if counter is None or counter.device != x.device:
-            counter = layer._small_batch_counter = torch.zeros((1,), dtype=torch.int32, device=x.device)
-        a.sync_counter = counter.data_ptr()
     if g is not None:
         weight, gate_bias = g
         if not _is(weight, torch.float32, (E, H), dev):

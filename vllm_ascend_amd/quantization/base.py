@@ -67,20 +67,21 @@ def fused_front_supported(layer, x: torch.Tensor, router_logits: torch.Tensor, r
     guard = getattr(router, "is_fused_supported", None)
     if guard is not None and not guard(x):
         return False  # the router's own guard decides (and refuses) on the operator-by-operator path
-    if getattr(layer, "log2phy", None) is not None:  # the ids are remapped between gating and dispatch
-        return kernels.gate_quant_supported(x.shape[0], router.top_k, router_logits.shape[1])
-    return (kernels.route_quant_small_supported(x.shape[0], router.top_k, router_logits.shape[1])
-            or kernels.gate_quant_supported(x.shape[0], router.top_k, router_logits.shape[1]))
+    return kernels.gate_quant_supported(x.shape[0], router.top_k, router_logits.shape[1])
 
 
 def route_and_quantize(layer, x: torch.Tensor, router_logits: torch.Tensor, router):
     """The router (``select_experts``), the per-token quantisation of the hidden states and the index maps of the
-    dispatch, in one launch for at most 1024 (token, slot) pairs and in two for larger batches (gating and
-    quantisation side by side, then the maps).  Returns ``(topk_weights, topk_ids, xq, x_scale,
-    expanded_row_idx, row_token, expert_tokens)``; the token rows stay in token order and the gate_up GEMM reads
-    them through ``row_token``.  Same values, bit for bit, as ``router.select_experts`` + ``npu_dynamic_quant`` +
-    ``npu_moe_init_routing_v2`` (``vllm_ascend/ops/fused_moe/routed_experts.py:496-540``,
-    ``token_dispatcher.py:404-420``)."""
+    dispatch in two launches: gating and quantisation side by side, then the maps.  Returns ``(topk_weights,
+    topk_ids, xq, x_scale, expanded_row_idx, row_token, expert_tokens)``; the token rows stay in token order and the
+    gate_up GEMM reads them through ``row_token``.  Same values, bit for bit, as ``router.select_experts`` +
+    ``npu_dynamic_quant`` + ``npu_moe_init_routing_v2`` (``vllm_ascend/ops/fused_moe/routed_experts.py:496-540``,
+    ``token_dispatcher.py:404-420``).
+
+    Batches of at most 1024 pairs could have all three in one launch (``kernels.route_quant_small``), but that launch
+    needs a counter that no other launch uses while it runs, and a layer does not know how many streams, threads or
+    replayed graphs run it at a time: two launches on one counter leave the maps unwritten, and the GEMMs then read
+    row counts that nobody wrote."""
     from .. import kernels
 
     bias = router.e_score_correction_bias
@@ -91,13 +92,6 @@ def route_and_quantize(layer, x: torch.Tensor, router_logits: torch.Tensor, rout
                  int(router.renormalize), 0 if router.scoring_func == "softmax" else 1,
                  router.routed_scaling_factor, 1e-20, bias)
     log2phy = getattr(layer, "log2phy", None)
-    if log2phy is None and kernels.route_quant_small_supported(x.shape[0], router.top_k, router_logits.shape[1]):
-        # the routing kernel's arrival counter: one zeroed int32 per layer (and device), which every call leaves
-        # at zero; created on the first call (run the layer once before capturing it into a graph)
-        counter = getattr(layer, "_small_batch_counter", None)
-        if counter is None or counter.device != x.device:
-            counter = layer._small_batch_counter = torch.zeros((1,), dtype=torch.int32, device=x.device)
-        return kernels.route_quant_small(x, router_logits, *gate_args, sync_counter=counter)
     topk_weights, topk_ids, xq, x_scale = kernels.gate_quant(x, router_logits, *gate_args)
     num_experts = router_logits.shape[1]
     if log2phy is not None:

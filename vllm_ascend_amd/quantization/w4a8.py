@@ -141,8 +141,7 @@ class AscendW4A8DynamicFusedMoEMethod(AscendMoEScheme):
 
     def apply_small_batch(self, layer, x: torch.Tensor, router_logits: torch.Tensor, router,
                           shared_experts: Any | None = None, shared_experts_input: torch.Tensor | None = None):
-        """router + ``apply`` with gating, token quantisation and (for small batches) the dispatch maps in one
-        launch; same results, bit for bit, as ``router.select_experts`` followed by ``apply``."""
+        """router + ``apply`` with gating and token quantisation in one launch; same results, bit for bit, as ``router.select_experts`` followed by ``apply``."""
         before_dispatch_evt = torch.cuda.current_stream().record_event()
         topk_weights, topk_ids, xq, x_scale, expanded_row_idx, row_token, expert_tokens = \
             route_and_quantize(layer, x, router_logits, router)

@@ -176,16 +176,15 @@ class AscendW8A8DynamicFusedMoEMethod(AscendMoEScheme):
     # ------------------------------------------------------------------ small batches (decode)
     def supports_small_batch(self, layer, x: torch.Tensor, router_logits: torch.Tensor, router) -> bool:
         """Whether ``apply_small_batch`` can take this call, router included: a plain call (see ``_plain_call``),
-        no forced load balance, at most 256 experts.  (The name is from the time when only batches of at most 1024
-        (token, slot) pairs had such a form; those still get gating, dispatch and quantisation in ONE launch,
-        larger ones gating and quantisation.)"""
+        no forced load balance, at most 256 experts.  (The name is from the time when only small batches had such a
+        form.)"""
         return self._plain_call(layer, x) and fused_front_supported(layer, x, router_logits, router)
 
     def apply_small_batch(self, layer, x: torch.Tensor, router_logits: torch.Tensor, router,
                           shared_experts: Any | None = None, shared_experts_input: torch.Tensor | None = None):
-        """router + ``apply`` for a small batch in four launches instead of six: gating and dispatch are one
-        kernel (the token rows are quantised once, in token order, and the gate_up GEMM reads them through the
-        row -> token map), then the gate_up GEMM with SwiGLU and re-quantisation, the down GEMM and the combine.
+        """router + ``apply``: gating and token quantisation are one kernel (the rows are quantised once, in token
+        order, and the gate_up GEMM reads them through the row -> token map), then the dispatch maps, the gate_up GEMM
+        with SwiGLU and re-quantisation, the down GEMM and the combine; decode batches in pair order have no maps.
         Same results, bit for bit, as ``router.select_experts`` followed by ``apply``
         (``vllm_ascend/ops/fused_moe/routed_experts.py:496-609``, ``w8a8_dynamic.py:224-301``)."""
         before_dispatch_evt = torch.cuda.current_stream().record_event()
