@@ -1,5 +1,5 @@
 """The grouped GEMMs on both sides of the lines between streaming and the tiles: 1023 / 1024 rows for a small product,
-fewer rows than experts / one row per expert for one of more than a GiB, 63 / 64 rows per expert at a long K."""
+fewer rows than experts / one row per expert for one of a GiB and more, 63 / 64 rows per expert at a long K."""
 import numpy as np
 import pytest
 import torch
@@ -8,7 +8,8 @@ pytestmark = pytest.mark.gpu
 
 LINES = [(1023, 128, 256, 128, "stream"), (1024, 128, 256, 128, "tiled"), (1100, 1200, 64, 64, "stream"),
          (63 * 8 + 7, 8, 4096, 128, "tiled"), (64 * 8, 8, 4096, 128, "wide"),
-         (287, 288, 2048, 2048, "stream"), (288, 288, 2048, 2048, "tiled")]
+         (287, 288, 2048, 2048, "stream"), (288, 288, 2048, 2048, "tiled"),
+         (255, 256, 2048, 2048, "stream"), (256, 256, 2048, 2048, "tiled"), (256 * 23, 256, 4096, 1024, "tiled")]
 
 
 @pytest.mark.parametrize("skewed", [False, True])

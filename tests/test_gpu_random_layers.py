@@ -1,7 +1,7 @@
 """The whole layer against the checker on seeded random configurations: shapes, fan-outs, expert counts, group
 structures, scoring functions, biases, scaling factors, skewed routing, shared expert and the W4A8 scheme drawn at
-random, so that the borders between the kernel families (pair order / sorted decode batches, streaming / tiled /
-split grouped GEMMs, fused / separate re-quantisation) are crossed in combinations nobody wrote down by hand.
+random, so that the borders between the kernel families (pair order / sorted decode batches, streaming / tiled
+grouped GEMMs, fused / separate re-quantisation) are crossed in combinations nobody wrote down by hand.
 Output and per-expert counts bit for bit."""
 import numpy as np
 import pytest

@@ -274,7 +274,6 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
         }
     } else {
         expert_rows(a.gl, a.gl_type, e, lane, row0, row1);
-        if (!expert_in_launch(a, row1 - row0)) return;  // another kernel of this operator call covers the expert
         if (row1 > a.R) row1 = a.R;
         if (row1 <= row0) return;
     }
@@ -593,12 +592,6 @@ static void launch_gemm(KernelT kernel, dim3 grid, hipStream_t st, const GmmArgs
 // tiles (up to 256 rows) that fetch an expert's weights once.  The host only knows the mean, and the histogram may be
 // skewed (real routers are): the 128-row tiles cost a cold expert little more than streaming does (a short tile that
 // is its expert's only one reads its weights once, past the caches) and a hot one a fraction of it, so they start early.
-// products small enough to stream below 1024 rows, large enough to split (see GemmPlan)
-static bool split_size(int64_t weights)
-{
-    return weights >= (1ll << 30) && weights < (9ll << 27);
-}
-
 static int tiled_bm(const GmmArgs& a)
 {
     if (a.K % 64 != 0) return 0;
@@ -615,16 +608,17 @@ static int tiled_bm(const GmmArgs& a)
     //   256 experts, K = 7168 / 2048 (7 and 3.5 GiB): 16 tokens (half a row per expert) 685 against 703 and 253
     //     against 281; 32 tokens 1097 against 1100 and 351 against 328; 64 tokens 1455 against 1449 and 442 against
     //     406; 96 tokens 1584 against 1592 and 508 against 423.  So from one row per expert on: tiles.
-    //   256 experts, K = 4096 / 1024 (2 and 1 GiB), 64 / 128 / 256 / 448 / 640 tokens: 475 / 514 / 539 / 568 / 591 with
-    //     the small product split, 481 / 516 / 535 / 555 / 565 on tiles; Zipf 162 / 201 / 221 / 264 / 305 against 149 /
-    //     193 / 212 / 250 / 290.
+    //   Products of one GiB, 256 experts of 2048 x 2048 (the down product alone), 1 / 2 / 4 / 8 / 14 / 23 rows per
+    //     expert: 123 / 144 / 160 / 167 / 174 / 191 streaming, 116 / 142 / 162 / 166 / 172 / 175 on tiles; Zipf 91 / 117 /
+    //     148 / 202 / 230 / 309 against 74 / 100 / 122 / 154 / 166 / 176; K from 512 to 8192 and 128 experts alike.
+    //     Sending the experts of up to 32 rows to streaming and the others to tiles, in two launches: uniform 115 / 143 /
+    //     164 / 171 / 178 / 207, Zipf 72 / 114 / 137 / 162 / 171 / 184 (never more than 3 % ahead of the tiles, up to
+    //     35 % behind them at K = 8192).
     //   128 experts, K = 2048 / 768 (0.4 and 0.2 GB): 48 / 100 tokens 107 / 112 against 117 / 131 and 81 / 86 against
     //     73 / 81, so decode batches (fewer than 1024 rows) stream; 130 / 190 tokens 120 / 123 against 123 / 126 and
     //     153 / 183 against 80 / 88: tiles.
     if (a.R < a.E) return 0;
     if (avg < 48 && a.R < 1024 && (a.R < 128 || weights < (1ll << 30))) return 0;
-    // at a GiB of weights the experts are split between both families up to 23 rows per expert (gemm_plan)
-    if (avg < 24 && split_size(weights)) return 0;
     // the list of 256-row tiles is built from 16-bit counters (tile_map_kernel, by_length)
     const bool wide_ok = a.R / 256 + a.E < 32768;
     // K = 7168 / 2048, uniform routing, 28 / 40 / 48 / 56 / 64 / 94 rows per expert: the layer takes 1968 / 2028 / 2055 /
@@ -638,47 +632,14 @@ static int tiled_bm(const GmmArgs& a)
     return 128;
 }
 
-// What one operator call launches: the family chosen from the mean rows per expert, restricted to the experts it
-// is good at, and (split > 0) a second family for the experts above that range.
-//   Products of one GiB of weights, mean below 24, decode batches too from one row per expert on: streaming for
-//     experts of at most 32 rows (one pass over their weights, and no request before the group list says that the
-//     expert is theirs), tiles for the others -- a 500-row expert would otherwise stream its weights 16 times while the
-//     units of the cold experts have long finished.  It is the border between the small products, whose decode batches
-//     stream, and the large ones, which run on tiles: 256 experts, K = 4096 / 512, 64 / 128 / 256 tokens, uniform
-//     routing 245 / 283 / 286 us split, 256 / 285 / 285 us on tiles.
-//   The weight-streaming tiles (mean 64..256) keep every expert: sending those above 256 rows to the 128-row
-//     tiles measured the same on a Zipf(1.1) batch of 32,768 rows (2149 against 2180 us for the gate_up product,
-//     1136 against 1119 us for the down product) and would cost the uniform batches an empty launch.
-struct GemmPlan {
-    int bm;        // 0 streaming, 64 / 128 LDS-tiled, 256 weight-streaming tiles
-    int split;     // > 0: experts with more than `split` rows run on another family instead
-    int split_bm;  // that family: 128 LDS-tiled, 256 weight-streaming tiles
-};
-
-static GemmPlan gemm_plan(const GmmArgs& a, bool have_tile_ws)
+// The family of one operator call: 0 streaming, 64 / 128 LDS-tiled, 256 weight-streaming tiles, over all experts.
+// (Sending the experts above 256 rows of a weight-streaming call to the 128-row tiles measured the same on a Zipf(1.1)
+// batch of 32,768 rows, 2149 against 2180 us for the gate_up product, 1136 against 1119 us for the down product, and would
+// cost the uniform batches an empty launch.)
+static int gemm_family(const GmmArgs& a, bool have_tile_ws)
 {
-    GemmPlan p = {have_tile_ws ? tiled_bm(a) : 0, 0, 128};
-    if (a.E == 1 && a.R <= 64) p.bm = 0;  // dense, few rows: the streaming kernel, one workgroup per 64 channels
-    if (!have_tile_ws || a.K % 64 != 0 || a.E == 1) return p;
-#ifdef MOE355_DEV_KNOBS
-    static const char* force = getenv("MOE355_GEMM");
-    if (force && force[0]) return p;
-    static const char* sp = getenv("MOE355_SPLIT");  // "<rows>:<family>", e.g. 32:256
-    if (sp && sp[0] && p.bm == 0 && a.R >= 1024) {  // experiments only
-        p.split = atoi(sp);
-        const char* c = strchr(sp, ':');
-        p.split_bm = c ? atoi(c + 1) : 128;
-        return p;
-    }
-#endif
-    if (p.bm == 0 && a.R >= 128 && a.R >= (int64_t)a.E && split_size((int64_t)a.E * a.N * a.K)) {
-        p.split = 32;
-        // the experts above the border: weight-streaming tiles when K is long (an expert of up to 256 rows fetches
-        // its weights once), 128-row tiles otherwise.  A border of 16 or 64 rows instead of 32 cost 70 / 40 us of
-        // 518 us on 512 tokens of Zipf(1.1) routing at K = 7168.
-        if (a.K >= 4096 && a.R / 256 + a.E < 32768) p.split_bm = 256;
-    }
-    return p;
+    if (!have_tile_ws || (a.E == 1 && a.R <= 64)) return 0;  // dense, few rows: a workgroup per 64 channels streams
+    return tiled_bm(a);
 }
 
 // One expert with enough rows and channels for the 256 x 256 tiles to fill the chip: the dense kernel (measured
@@ -696,8 +657,7 @@ static bool dense_tiles(const GmmArgs& a)
 
 static size_t tiled_ws_max(int64_t rows, int E)
 {
-    // the smallest tile needs the longest tile list; a call that splits the experts over two families builds two
-    return 2 * ((tiled_workspace_bytes(rows, E, 64) + 255) & ~(size_t)255);
+    return (tiled_workspace_bytes(rows, E, 64) + 255) & ~(size_t)255;  // the smallest tile needs the longest tile list
 }
 
 // K slabs of the dense few-row product (one expert, at most 64 rows, a long K, too few pairs of tiles to fill
@@ -712,13 +672,7 @@ static int dense_slabs(int64_t R, int K, int N, int E)
     return slabs < 1 ? 1 : slabs;
 }
 
-// the second family's tile map lies behind the first one's
-static void* second_map(const GmmArgs& a, void* tile_ws)
-{
-    return (char*)tile_ws + ((tiled_workspace_bytes(a.R, a.E, 64) + 255) & ~(size_t)255);
-}
-
-// The tile maps that launch_gemm_auto of this product will look for in tile_ws (at most two).
+// The tile map that launch_gemm_auto of this product will look for in tile_ws: its number, 0 or 1.
 int gemm_tile_specs(int64_t rows, int64_t k, int64_t n, int num_experts, void* tile_ws, TileSpec* specs)
 {
     GmmArgs a = {};
@@ -726,13 +680,9 @@ int gemm_tile_specs(int64_t rows, int64_t k, int64_t n, int num_experts, void* t
     a.K = (int)k;
     a.N = (int)n;
     a.E = num_experts;
-    if (dense_tiles(a)) return 0;
-    const GemmPlan plan = gemm_plan(a, true);
-    int count = 0;
-    if (plan.bm) specs[count++] = tile_spec(rows, num_experts, plan.bm, 0, plan.split, tile_ws);
-    if (plan.split > 0)
-        specs[count++] = tile_spec(rows, num_experts, plan.split_bm, plan.split + 1, 0, second_map(a, tile_ws));
-    return count;
+    const int bm = dense_tiles(a) ? 0 : gemm_family(a, true);
+    if (bm) specs[0] = tile_spec(rows, num_experts, bm, tile_ws);
+    return bm ? 1 : 0;
 }
 
 template <int EPI>
@@ -747,12 +697,9 @@ static int launch_gemm_auto(const GmmArgs& a_in, void* tile_ws, hipStream_t st, 
         launch_dense(EPI, a, st, ev0, ev1);
         return launch_status();
     }
-    const GemmPlan plan = gemm_plan(a, tile_ws != nullptr);
-    void* tile_ws2 = tile_ws ? second_map(a, tile_ws) : nullptr;
-    if (plan.split > 0) a.rows_max = plan.split;
-    hipEvent_t first_stop = plan.split > 0 ? nullptr : ev1;
-    if (plan.bm) {
-        launch_tiled_any(EPI, plan.bm, a, tile_ws, st, ev0, first_stop);
+    const int bm = gemm_family(a, tile_ws != nullptr);
+    if (bm) {
+        launch_tiled_any(EPI, bm, a, tile_ws, st, ev0, ev1);
     } else {
         const int64_t units = (int64_t)a.E * (a.N / 64);
         bool done = false;
@@ -770,7 +717,7 @@ static int launch_gemm_auto(const GmmArgs& a_in, void* tile_ws, hipStream_t st, 
                 if (planes) a.acc_part = (int32_t*)part_ws;
                 else hipLaunchKernelGGL(zero_i32_kernel, cover, dim3(256), 0, st, a.acc, n4);
                 launch_gemm(gmm_stream_kernel<EPI, 4, 4, 3, true>, dim3((unsigned)units, (unsigned)slabs), st, a, ev0,
-                            first_stop);
+                            ev1);
                 if (planes)
                     hipLaunchKernelGGL(slab_sum_kernel, cover, dim3(256), 0, st, a.acc_part, slabs, a.R, a.N, a.gl,
                                        a.acc);
@@ -782,25 +729,18 @@ static int launch_gemm_auto(const GmmArgs& a_in, void* tile_ws, hipStream_t st, 
         // itself (no K split, no LDS reduction); otherwise the four wavefronts of a workgroup split K (from
         // K = 2048 on that measured 1.5 % faster on the whole layer, below it the same or slower).
         if (done) {
-        } else if (plan.split == 0 && a.gl && a.R < (int64_t)a.E) {
+        } else if (a.gl && a.R < (int64_t)a.E) {
             // fewer rows than experts (a decode batch of a few tokens on the sorted path): a slot per row instead
             // of a place per expert, so that the idle experts cost no dispatch; the workgroup looks up the expert
             // of its slot in the group list, so nothing is requested before that
             a.gl_slots = (int)a.R;
             launch_gemm(gmm_stream_kernel<EPI, 4, 4, 3, false, false>, dim3((unsigned)(a.R * (a.N / 64))), st, a, ev0,
-                        first_stop);
-        } else if (plan.split > 0) {
-            launch_gemm(gmm_stream_kernel<EPI, 4, 4, 3, false, false>, dim3((unsigned)units), st, a, ev0, first_stop);
+                        ev1);
         } else if (EPI != EPI_SWIGLU && units >= 2048 && a.K < 2048) {
-            launch_gemm(gmm_stream_kernel<EPI, 1, 4, 2>, dim3((unsigned)((units + 3) / 4)), st, a, ev0, first_stop);
+            launch_gemm(gmm_stream_kernel<EPI, 1, 4, 2>, dim3((unsigned)((units + 3) / 4)), st, a, ev0, ev1);
         } else {
-            launch_gemm(gmm_stream_kernel<EPI, 4, 4, 3>, dim3((unsigned)units), st, a, ev0, first_stop);
+            launch_gemm(gmm_stream_kernel<EPI, 4, 4, 3>, dim3((unsigned)units), st, a, ev0, ev1);
         }
-    }
-    if (plan.split > 0) {
-        a.rows_min = plan.split + 1;
-        a.rows_max = 0;
-        launch_tiled_any(EPI, plan.split_bm, a, tile_ws2, st, nullptr, ev1);
     }
     return launch_status();
 }
@@ -826,12 +766,8 @@ extern "C" const char* moe355_gmm_kernel_name(int epilogue, int64_t rows, int64_
     a.N = (int)n;
     a.E = num_experts;
     if (dense_tiles(a)) return "gmm_dense_kernel";
-    const GemmPlan p = gemm_plan(a, true);  // as launch_gemm_auto decides
-    if (p.bm == 256) return "gmm_wide_kernel";
-    if (p.bm != 0) return "gmm_tiled_kernel";
-    if (!p.split) return "gmm_stream_kernel";
-    return p.split_bm == 256 ? "gmm_stream_kernel + gmm_wide_kernel above 32 rows"
-                             : "gmm_stream_kernel + gmm_tiled_kernel above 32 rows";
+    const int bm = gemm_family(a, true);  // as launch_gemm_auto decides
+    return bm == 256 ? "gmm_wide_kernel" : bm ? "gmm_tiled_kernel" : "gmm_stream_kernel";
 }
 
 extern "C" int moe355_format_cast_nz(const int8_t* w, int layout, int64_t num_experts, int64_t n, int64_t k,

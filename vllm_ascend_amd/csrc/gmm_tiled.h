@@ -10,7 +10,7 @@ namespace moe355 {
 size_t tiled_workspace_bytes(int64_t rows, int E, int BM);
 
 // the tile map of a product over `rows` rows, laid out in a workspace of tiled_workspace_bytes()
-TileSpec tile_spec(int64_t rows, int E, int BM, int rows_min, int rows_max, void* workspace);
+TileSpec tile_spec(int64_t rows, int E, int BM, void* workspace);
 
 // epi: EPI_*; bm: 64 or 128 (LDS-tiled kernel) or 256 (weight-streaming tiles).  ev0/ev1: optional events recorded around the GEMM kernel itself.
 void launch_tiled_any(int epi, int bm, const GmmArgs& a, void* workspace, hipStream_t st, hipEvent_t ev0,

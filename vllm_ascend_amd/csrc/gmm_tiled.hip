@@ -770,13 +770,11 @@ __global__ __launch_bounds__(512, 1) void gmm_dense_kernel(GmmArgs a, int xn, in
 }
 
 // ------------------------------------------------------------------ host side
-TileSpec tile_spec(int64_t rows, int E, int BM, int rows_min, int rows_max, void* workspace)
+TileSpec tile_spec(int64_t rows, int E, int BM, void* workspace)
 {
     TileSpec t;
     t.BM = BM;
     t.by_length = BM == 256;
-    t.rows_min = rows_min;
-    t.rows_max = rows_max;
     t.max_tiles = (int)(rows / BM + E);
     const size_t arr = (size_t)(((size_t)t.max_tiles * 4 + 255) / 256) * 256;
     t.tm.count = (int32_t*)workspace;
@@ -796,7 +794,7 @@ template <int EPI, int BMT, int RING>
 static void launch_tiled(const GmmArgs& a, void* workspace, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1)
 {
     constexpr int BM = 32 * BMT;
-    const TileSpec spec = tile_spec(a.R, a.E, BM, a.rows_min, a.rows_max, workspace);
+    const TileSpec spec = tile_spec(a.R, a.E, BM, workspace);
     const TileMap tm = spec.tm;
     const int max_tiles = spec.max_tiles;
     if (!a.tiles_ready)
@@ -828,7 +826,7 @@ static void launch_wide(const GmmArgs& a, void* workspace, hipStream_t st, hipEv
     static const hipError_t attr = hipFuncSetAttribute((const void*)gmm_wide_kernel<EPI>,
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     (void)attr;
-    const TileSpec spec = tile_spec(a.R, a.E, BM, a.rows_min, a.rows_max, workspace);
+    const TileSpec spec = tile_spec(a.R, a.E, BM, workspace);
     const TileMap tm = spec.tm;
     const int max_tiles = spec.max_tiles;
     if (!a.tiles_ready)

@@ -396,7 +396,7 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
     }
     bool tiles_ready = false;
     if (rc == MOE355_OK && !f.pairs && !f.small) {
-        TileSpec specs[4];
+        TileSpec specs[2];
         int n = 0;
         if (l.weights != W_INT4) {
             n = gemm_tile_specs(R, l.hidden, 2 * l.intermediate, l.num_experts,

@@ -75,7 +75,7 @@ int gmm2_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* wei
               int group_list_type, int64_t rows, int64_t k, int64_t n, int num_experts, void* out, int out_dtype,
               void* workspace, size_t workspace_bytes, void* stream, bool tiles_ready = false);
 void* gmm1_tile_ws(void* workspace, int64_t rows, int64_t n);
-// tile maps (at most two) that a grouped product will look for in its workspace
+// the tile map (0 or 1) that a grouped product will look for in its workspace
 int gemm_tile_specs(int64_t rows, int64_t k, int64_t n, int num_experts, void* tile_ws, TileSpec* specs);
 
 // int4 weights, pair order (gmm_w4.hip)
@@ -88,7 +88,7 @@ int gmm2_w4_pairs(const int8_t* x, const float* x_scale, const int32_t* topk_ids
                   const uint8_t* w, const float* scale, int64_t group, int64_t k, int64_t n, int num_experts, void* out,
                   int out_dtype, hipStream_t st);
 
-// moe355_route_map with the tile maps of the two products (nspecs of them, at most 4) built by the same launch where it
+// moe355_route_map with the tile maps of the two products (nspecs of them, at most 2) built by the same launch where it
 // is one launch (returns 1 in *built then)
 int route_map_impl(const int32_t* expert_idx, int64_t num_tokens, int top_k, int num_experts, int tokens_num_type,
                    int32_t* expanded_row_idx, int32_t* row_token, int64_t* expert_tokens, void* workspace,

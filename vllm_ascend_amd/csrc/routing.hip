@@ -334,7 +334,7 @@ struct RouteMapArgs {
     int32_t* dst;
     int32_t* row_token;
     int64_t* expert_tokens;
-    TileSpec specs[4];
+    TileSpec specs[2];
 };
 constexpr int kMapThreads = 1024;
 constexpr int kMapWaves = kMapThreads / 64;

@@ -21,9 +21,6 @@ struct TileSpec {
     // then the tall ones (more than 192 rows, which become two shorter column items) -- so that the workgroups that
     // start last are the short ones and the compute units finish closer together
     int by_length;
-    // experts whose row count lies outside [rows_min, rows_max] (rows_max 0: no upper bound) get no tiles (another
-    // kernel of the same operator call covers them); their rows still count for the offsets
-    int rows_min, rows_max;
 };
 
 // One workgroup of any size, every thread calls it; rows_of(e) = rows of expert e (not negative).  Thread t owns
@@ -36,9 +33,6 @@ __device__ __forceinline__ void build_tile_map(RowsOf rows_of, int E, const Tile
     const int BM = spec.BM, max_tiles = spec.max_tiles, tid = threadIdx.x;
     const int seg = (E + (int)blockDim.x - 1) / (int)blockDim.x;
     const int e0 = tid * seg;
-    auto tiled_rows = [&](int64_t m) -> int64_t {
-        return (m >= spec.rows_min && (spec.rows_max == 0 || m <= spec.rows_max)) ? m : 0;
-    };
     auto put = [&](int32_t t, int e, int64_t begin, int64_t end) {
         if (t < max_tiles) {
             tm.expert[t] = e;
@@ -55,7 +49,7 @@ __device__ __forceinline__ void build_tile_map(RowsOf rows_of, int E, const Tile
             if (e < E) {
                 const int64_t m = rows_of(e);
                 rows += (int32_t)m;
-                for (int64_t r0 = 0; r0 < tiled_rows(m); r0 += BM) {
+                for (int64_t r0 = 0; r0 < m; r0 += BM) {
                     const int c = cls(m - r0);
                     if (c < 2) n01 += 1 << (16 * c);
                     else n23 += 1 << (16 * (c - 2));
@@ -76,7 +70,7 @@ __device__ __forceinline__ void build_tile_map(RowsOf rows_of, int E, const Tile
             const int e = e0 + j;
             if (e < E) {
                 const int64_t m = rows_of(e);
-                for (int64_t r0 = 0; r0 < tiled_rows(m); r0 += BM) put(next[cls(m - r0)]++, e, row + r0, row + m);
+                for (int64_t r0 = 0; r0 < m; r0 += BM) put(next[cls(m - r0)]++, e, row + r0, row + m);
                 row += m;
             }
         }
@@ -88,7 +82,7 @@ __device__ __forceinline__ void build_tile_map(RowsOf rows_of, int E, const Tile
         if (e < E) {
             const int64_t m = rows_of(e);
             rows += (int32_t)m;
-            tiles += (int32_t)((tiled_rows(m) + BM - 1) / BM);
+            tiles += (int32_t)((m + BM - 1) / BM);
         }
     }
     // exclusive prefix of rows and tiles over the threads (experts in order)
@@ -102,7 +96,7 @@ __device__ __forceinline__ void build_tile_map(RowsOf rows_of, int E, const Tile
         const int e = e0 + j;
         if (e < E) {
             const int64_t m = rows_of(e);
-            for (int64_t r0 = row; r0 < row + tiled_rows(m); r0 += BM) put(t++, e, r0, row + m);
+            for (int64_t r0 = row; r0 < row + m; r0 += BM) put(t++, e, r0, row + m);
             row += m;
         }
     }
