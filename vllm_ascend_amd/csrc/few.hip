@@ -447,9 +447,11 @@ int few_forward(const FewArgs& a, hipStream_t st)
     const bool wide = a.H / 16 <= 256;
 #define MOE355_FEW_DOWN(Q_, N_)                                                                                   \
     do {                                                                                                            \
-        static const hipError_t attr = hipFuncSetAttribute((const void*)few_down_kernel<Q_, N_>,                    \
-                                                           hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);  \
-        if (attr != hipSuccess) return MOE355_E_LAUNCH;                                                             \
+        static OncePerDevice once;                                                                                  \
+        if (!allow_dynamic_lds(once, (const void*)few_down_kernel<Q_, N_>, 80 * 1024)) {                            \
+            (void)hipGetLastError();                                                                                \
+            return MOE355_E_LAUNCH;                                                                                 \
+        }                                                                                                           \
         hipLaunchKernelGGL((few_down_kernel<Q_, N_>), down, dim3(N_), lds, st, a);                                  \
     } while (0)
     if (inside && wide) MOE355_FEW_DOWN(true, 1024);

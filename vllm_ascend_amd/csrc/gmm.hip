@@ -685,6 +685,12 @@ int gemm_tile_specs(int64_t rows, int64_t k, int64_t n, int num_experts, void* t
     return bm ? 1 : 0;
 }
 
+static int launched(bool ok)
+{
+    const int rc = launch_status();  // takes the error of a refused step off the thread too
+    return ok ? rc : MOE355_E_LAUNCH;
+}
+
 template <int EPI>
 static int launch_gemm_auto(const GmmArgs& a_in, void* tile_ws, hipStream_t st, void* part_ws = nullptr,
                             size_t part_bytes = 0)
@@ -694,53 +700,49 @@ static int launch_gemm_auto(const GmmArgs& a_in, void* tile_ws, hipStream_t st, 
     t_ev_start = nullptr;
     t_ev_stop = nullptr;
     if (dense_tiles(a)) {
-        launch_dense(EPI, a, st, ev0, ev1);
-        return launch_status();
+        return launched(launch_dense(EPI, a, st, ev0, ev1));
     }
     const int bm = gemm_family(a, tile_ws != nullptr);
-    if (bm) {
-        launch_tiled_any(EPI, bm, a, tile_ws, st, ev0, ev1);
-    } else {
-        const int64_t units = (int64_t)a.E * (a.N / 64);
-        bool done = false;
-        if constexpr (EPI == EPI_I32) {
-            // One expert with at most 64 rows (the shared expert of a decode batch: a dense product over a few
-            // tokens): too few workgroups for a chip that needs thousands of loads in flight to stream at full rate.
-            // K is cut into slabs, one workgroup per (pair of tiles, slab), partial sums added into the zeroed result.
-            const int slabs = dense_slabs(a.R, a.K, a.N, a.E);
-            if (slabs > 1) {
-                const int64_t n4 = a.R * (int64_t)a.N / 4;  // N % 64 == 0
-                const dim3 cover((unsigned)((n4 + 255) / 256));
-                // with scratch for one plane per slab the partial sums are stored and added up afterwards;
-                // without, they are added into the zeroed result with atomics (32 of 47 us at 8 slabs)
-                const bool planes = part_ws && part_bytes >= (size_t)slabs * a.R * a.N * 4;
-                if (planes) a.acc_part = (int32_t*)part_ws;
-                else hipLaunchKernelGGL(zero_i32_kernel, cover, dim3(256), 0, st, a.acc, n4);
-                launch_gemm(gmm_stream_kernel<EPI, 4, 4, 3, true>, dim3((unsigned)units, (unsigned)slabs), st, a, ev0,
-                            ev1);
-                if (planes)
-                    hipLaunchKernelGGL(slab_sum_kernel, cover, dim3(256), 0, st, a.acc_part, slabs, a.R, a.N, a.gl,
-                                       a.acc);
-                done = true;
-            }
-        }
-        // Occupancy 3 keeps the SwiGLU epilogue out of scratch memory (131 registers).  With enough units to
-        // fill the chip four times over and a short K, the down GEMM lets every wavefront stream a whole unit by
-        // itself (no K split, no LDS reduction); otherwise the four wavefronts of a workgroup split K (from
-        // K = 2048 on that measured 1.5 % faster on the whole layer, below it the same or slower).
-        if (done) {
-        } else if (a.gl && a.R < (int64_t)a.E) {
-            // fewer rows than experts (a decode batch of a few tokens on the sorted path): a slot per row instead
-            // of a place per expert, so that the idle experts cost no dispatch; the workgroup looks up the expert
-            // of its slot in the group list, so nothing is requested before that
-            a.gl_slots = (int)a.R;
-            launch_gemm(gmm_stream_kernel<EPI, 4, 4, 3, false, false>, dim3((unsigned)(a.R * (a.N / 64))), st, a, ev0,
+    if (bm) return launched(launch_tiled_any(EPI, bm, a, tile_ws, st, ev0, ev1));
+    const int64_t units = (int64_t)a.E * (a.N / 64);
+    bool done = false;
+    if constexpr (EPI == EPI_I32) {
+        // One expert with at most 64 rows (the shared expert of a decode batch: a dense product over a few
+        // tokens): too few workgroups for a chip that needs thousands of loads in flight to stream at full rate.
+        // K is cut into slabs, one workgroup per (pair of tiles, slab), partial sums added into the zeroed result.
+        const int slabs = dense_slabs(a.R, a.K, a.N, a.E);
+        if (slabs > 1) {
+            const int64_t n4 = a.R * (int64_t)a.N / 4;  // N % 64 == 0
+            const dim3 cover((unsigned)((n4 + 255) / 256));
+            // with scratch for one plane per slab the partial sums are stored and added up afterwards;
+            // without, they are added into the zeroed result with atomics (32 of 47 us at 8 slabs)
+            const bool planes = part_ws && part_bytes >= (size_t)slabs * a.R * a.N * 4;
+            if (planes) a.acc_part = (int32_t*)part_ws;
+            else hipLaunchKernelGGL(zero_i32_kernel, cover, dim3(256), 0, st, a.acc, n4);
+            launch_gemm(gmm_stream_kernel<EPI, 4, 4, 3, true>, dim3((unsigned)units, (unsigned)slabs), st, a, ev0,
                         ev1);
-        } else if (EPI != EPI_SWIGLU && units >= 2048 && a.K < 2048) {
-            launch_gemm(gmm_stream_kernel<EPI, 1, 4, 2>, dim3((unsigned)((units + 3) / 4)), st, a, ev0, ev1);
-        } else {
-            launch_gemm(gmm_stream_kernel<EPI, 4, 4, 3>, dim3((unsigned)units), st, a, ev0, ev1);
+            if (planes)
+                hipLaunchKernelGGL(slab_sum_kernel, cover, dim3(256), 0, st, a.acc_part, slabs, a.R, a.N, a.gl,
+                                   a.acc);
+            done = true;
         }
+    }
+    // Occupancy 3 keeps the SwiGLU epilogue out of scratch memory (131 registers).  With enough units to
+    // fill the chip four times over and a short K, the down GEMM lets every wavefront stream a whole unit by
+    // itself (no K split, no LDS reduction); otherwise the four wavefronts of a workgroup split K (from
+    // K = 2048 on that measured 1.5 % faster on the whole layer, below it the same or slower).
+    if (done) {
+    } else if (a.gl && a.R < (int64_t)a.E) {
+        // fewer rows than experts (a decode batch of a few tokens on the sorted path): a slot per row instead
+        // of a place per expert, so that the idle experts cost no dispatch; the workgroup looks up the expert
+        // of its slot in the group list, so nothing is requested before that
+        a.gl_slots = (int)a.R;
+        launch_gemm(gmm_stream_kernel<EPI, 4, 4, 3, false, false>, dim3((unsigned)(a.R * (a.N / 64))), st, a, ev0,
+                    ev1);
+    } else if (EPI != EPI_SWIGLU && units >= 2048 && a.K < 2048) {
+        launch_gemm(gmm_stream_kernel<EPI, 1, 4, 2>, dim3((unsigned)((units + 3) / 4)), st, a, ev0, ev1);
+    } else {
+        launch_gemm(gmm_stream_kernel<EPI, 4, 4, 3>, dim3((unsigned)units), st, a, ev0, ev1);
     }
     return launch_status();
 }

@@ -12,11 +12,12 @@ size_t tiled_workspace_bytes(int64_t rows, int E, int BM);
 // the tile map of a product over `rows` rows, laid out in a workspace of tiled_workspace_bytes()
 TileSpec tile_spec(int64_t rows, int E, int BM, void* workspace);
 
-// epi: EPI_*; bm: 64 or 128 (LDS-tiled kernel) or 256 (weight-streaming tiles).  ev0/ev1: optional events recorded around the GEMM kernel itself.
-void launch_tiled_any(int epi, int bm, const GmmArgs& a, void* workspace, hipStream_t st, hipEvent_t ev0,
+// epi: EPI_*; bm: 64 or 128 (LDS-tiled kernel) or 256 (weight-streaming tiles).  ev0/ev1: optional events recorded around
+// the GEMM kernel itself.  false: the device refused the kernel its LDS, nothing was launched.
+bool launch_tiled_any(int epi, int bm, const GmmArgs& a, void* workspace, hipStream_t st, hipEvent_t ev0,
                       hipEvent_t ev1);
 
 // One expert owning every row (a.E == 1): 256 x 256 tiles placed by arithmetic, no tile map, no scratch.
-void launch_dense(int epi, const GmmArgs& a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1);
+bool launch_dense(int epi, const GmmArgs& a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1);
 
 }  // namespace moe355

@@ -819,13 +819,12 @@ static void launch_tiled(const GmmArgs& a, void* workspace, hipStream_t st, hipE
 }
 
 template <int EPI>
-static void launch_wide(const GmmArgs& a, void* workspace, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1)
+static bool launch_wide(const GmmArgs& a, void* workspace, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1)
 {
     constexpr int BM = 256;
     constexpr int lds_bytes = kWideLdsBytes;
-    static const hipError_t attr = hipFuncSetAttribute((const void*)gmm_wide_kernel<EPI>,
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-    (void)attr;
+    static OncePerDevice once;
+    if (!allow_dynamic_lds(once, (const void*)gmm_wide_kernel<EPI>, lds_bytes)) return false;
     const TileSpec spec = tile_spec(a.R, a.E, BM, workspace);
     const TileMap tm = spec.tm;
     const int max_tiles = spec.max_tiles;
@@ -842,15 +841,15 @@ static void launch_wide(const GmmArgs& a, void* workspace, hipStream_t st, hipEv
     else
         hipLaunchKernelGGL((gmm_wide_kernel<EPI>), dim3(grid), dim3(512), lds_bytes, st, a, tm, max_tiles,
                            n_col_blocks, columns);
+    return true;
 }
 
 template <int EPI>
-static void launch_dense_t(const GmmArgs& a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1)
+static bool launch_dense_t(const GmmArgs& a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1)
 {
     constexpr int lds_bytes = kWideLdsBytes;
-    static const hipError_t attr = hipFuncSetAttribute((const void*)gmm_dense_kernel<EPI>,
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-    (void)attr;
+    static OncePerDevice once;
+    if (!allow_dynamic_lds(once, (const void*)gmm_dense_kernel<EPI>, lds_bytes)) return false;
     const int channels = (EPI == EPI_SWIGLU) ? a.N / 2 : a.N;
     const int per_block = (EPI == EPI_SWIGLU) ? kBN / 2 : kBN;
     const int n_col_blocks = (channels + per_block - 1) / per_block;
@@ -872,24 +871,26 @@ static void launch_dense_t(const GmmArgs& a, hipStream_t st, hipEvent_t ev0, hip
                               n_col_blocks);
     else
         hipLaunchKernelGGL((gmm_dense_kernel<EPI>), dim3(grid), dim3(512), lds_bytes, st, a, xn, pm, pn, n_col_blocks);
+    return true;
 }
 
-void launch_dense(int epi, const GmmArgs& a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1)
+bool launch_dense(int epi, const GmmArgs& a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1)
 {
-    if (epi == EPI_I32) launch_dense_t<EPI_I32>(a, st, ev0, ev1);
-    else if (epi == EPI_SWIGLU) launch_dense_t<EPI_SWIGLU>(a, st, ev0, ev1);
-    else launch_dense_t<EPI_DEQUANT>(a, st, ev0, ev1);
+    if (epi == EPI_I32) return launch_dense_t<EPI_I32>(a, st, ev0, ev1);
+    if (epi == EPI_SWIGLU) return launch_dense_t<EPI_SWIGLU>(a, st, ev0, ev1);
+    return launch_dense_t<EPI_DEQUANT>(a, st, ev0, ev1);
 }
 
-void launch_tiled_any(int epi, int bm, const GmmArgs& a, void* workspace, hipStream_t st, hipEvent_t ev0,
+bool launch_tiled_any(int epi, int bm, const GmmArgs& a, void* workspace, hipStream_t st, hipEvent_t ev0,
                       hipEvent_t ev1)
 {
 #define MOE355_TILED(E_, B_) launch_tiled<E_, B_, 3>(a, workspace, st, ev0, ev1)
     if (bm == 256) {
-        if (epi == EPI_I32) launch_wide<EPI_I32>(a, workspace, st, ev0, ev1);
-        else if (epi == EPI_SWIGLU) launch_wide<EPI_SWIGLU>(a, workspace, st, ev0, ev1);
-        else launch_wide<EPI_DEQUANT>(a, workspace, st, ev0, ev1);
-    } else if (bm == 128) {
+        if (epi == EPI_I32) return launch_wide<EPI_I32>(a, workspace, st, ev0, ev1);
+        if (epi == EPI_SWIGLU) return launch_wide<EPI_SWIGLU>(a, workspace, st, ev0, ev1);
+        return launch_wide<EPI_DEQUANT>(a, workspace, st, ev0, ev1);
+    }
+    if (bm == 128) {
         if (epi == EPI_I32) MOE355_TILED(EPI_I32, 4);
         else if (epi == EPI_SWIGLU) MOE355_TILED(EPI_SWIGLU, 4);
         else MOE355_TILED(EPI_DEQUANT, 4);
@@ -899,6 +900,7 @@ void launch_tiled_any(int epi, int bm, const GmmArgs& a, void* workspace, hipStr
         else MOE355_TILED(EPI_DEQUANT, 2);
     }
 #undef MOE355_TILED
+    return true;
 }
 
 }  // namespace moe355

@@ -10,6 +10,7 @@
 #include <stdint.h>
 
 #include "../../include/moe355.h"
+#include "per_device.h"
 
 #define MOE355_WAVE 64
 
@@ -269,6 +270,16 @@ __device__ __forceinline__ void expert_rows(const int64_t* gl, int gl_type, int 
         row0 = s;
         row1 = s + gl[e];
     }
+}
+
+// More dynamic LDS than the 64 KB every kernel may have, on the current device.
+inline bool allow_dynamic_lds(OncePerDevice& once, const void* kernel, int bytes)
+{
+    int device = -1;
+    if (hipGetDevice(&device) != hipSuccess) return false;
+    return once(device, [&] {
+        return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess;
+    });
 }
 
 inline int launch_status()
