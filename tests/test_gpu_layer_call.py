@@ -233,3 +233,17 @@ def test_gating_sort_and_quantisation_in_one_launch(name):
     for _ in range(3):
         assert torch.equal(layer(x, logits), want)
     assert layer._layer_plan is plan and int(counter) == 0
+
+
+# pair order, the sorted path, and a few tokens: the combine counts the pairs of every expert only where loads are kept
+@pytest.mark.parametrize("tokens", [2, 48, 300])
+def test_expert_loads_without_weight_lists(tokens):
+    cfg, layer, x, logits = _pair("c2_small", tokens, collect_expert_load=True)
+    res = layer.forward_impl(x, logits)
+    layer.clear_moe_load()
+    for n in (1, 2):
+        assert torch.equal(layer(x, logits), res.routed_out)
+        assert torch.equal(layer.moe_load, n * res.expert_tokens)
+    layer.eplb_heat_collection_status = False
+    assert torch.equal(layer(x, logits), res.routed_out)
+    assert torch.equal(layer.moe_load, 2 * res.expert_tokens)

@@ -10,9 +10,9 @@ namespace moe355 {
 // DT: bf16 or fp16 (rows, weights, residual and result share it).
 constexpr int kHistMaxExperts = 2048;
 
-// idx == nullptr: the rows lie in pair order (row of token t, slot s = t * top_k + s).  hist_ids != nullptr: one
-// more workgroup (the last of the grid's x range) counts the pairs of every expert into hist_out [hist_experts]
-// (int64), next to the others instead of in a launch of its own.
+// idx == nullptr: the rows lie in pair order (row of token t, slot s = t * top_k + s) and hist_ids holds their ids.
+// hist_out [hist_experts] or load: one more workgroup (the last of the grid's x range) counts the pairs of every expert
+// into the one and adds them to the other, next to the others instead of in a launch of its own.
 template <int TOPK, int DT = MOE355_DT_BF16>
 __global__ __launch_bounds__(256) void token_unpermute_kernel(const uint16_t* __restrict__ permuted,
                                                               const int32_t* __restrict__ idx,
@@ -28,7 +28,7 @@ __global__ __launch_bounds__(256) void token_unpermute_kernel(const uint16_t* __
     __shared__ int32_t srow[64];
     __shared__ float sw[64];
     const int top_k = TOPK > 0 ? TOPK : top_k_rt;
-    if ((hist_ids || load) && blockIdx.x == gridDim.x - 1) {
+    if ((hist_out || load) && blockIdx.x == gridDim.x - 1) {
         __shared__ int32_t hcnt[kHistMaxExperts];
         if (blockIdx.y != 0) return;
         if (!hist_ids) {
@@ -43,7 +43,7 @@ __global__ __launch_bounds__(256) void token_unpermute_kernel(const uint16_t* __
         }
         __syncthreads();
         for (int e = threadIdx.x; e < hist_experts; e += 256) {
-            hist_out[e] = (int64_t)hcnt[e];
+            if (hist_out) hist_out[e] = (int64_t)hcnt[e];
             if (load) load[e] += (int64_t)hcnt[e];
         }
         return;
@@ -133,7 +133,7 @@ int moe355::unpermute_impl(const void* permuted, int dtype, const int32_t* sorte
         if (pieces < 1) pieces = 1;
     }
 #define MOE355_UNPERMUTE(K, D)                                                                                    \
-    hipLaunchKernelGGL((token_unpermute_kernel<K, D>), dim3((unsigned)num_tokens + (hist_ids || load ? 1u : 0u), pieces), dim3(256), 0, (hipStream_t)stream, \
+    hipLaunchKernelGGL((token_unpermute_kernel<K, D>), dim3((unsigned)num_tokens + (hist_out || load ? 1u : 0u), pieces), dim3(256), 0, (hipStream_t)stream, \
                        (const uint16_t*)permuted, sorted_indices, (const uint16_t*)probs, top_k, hidden,             \
                        permuted_rows, (const uint16_t*)residual, (uint16_t*)out, hist_ids, hist_experts, hist_out,  \
                        load_counts, load)

@@ -411,6 +411,5 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
     if (rc != MOE355_OK) return rc;
     const void* residual = l.shared ? b.sh_out : nullptr;
     return unpermute_impl(b.o, l.x_dtype, f.pairs ? nullptr : b.dst, b.topk_weights, T, l.top_k, l.hidden, R, residual,
-                          out, f.pairs ? b.topk_ids : nullptr, l.num_experts, b.expert_tokens, b.expert_tokens, l.load,
-                          stream);
+                          out, f.pairs ? b.topk_ids : nullptr, l.num_experts, nullptr, b.expert_tokens, l.load, stream);
 }

@@ -24,7 +24,7 @@ int gate_quant_impl(bool sort, const GateCall& g, int tokens_num_type, void* top
                     int8_t* xq, float* x_scale, int32_t* expanded_row_idx, int32_t* row_token, int64_t* expert_tokens,
                     int32_t* sync_counter, int64_t* one_group, void* stream);
 
-// sorted_indices null: pair order (hist_ids = the ids, counts to hist_out).  load [hist_experts]: the counts of this
+// sorted_indices null: pair order (hist_ids = the ids, counts to hist_out unless that is null).  load [hist_experts]: the counts of this
 // batch are added to it (from hist_ids, or load_counts where the rows are sorted).
 int unpermute_impl(const void* permuted, int dtype, const int32_t* sorted_indices, const void* probs,
                    int64_t num_tokens, int top_k, int64_t hidden, int64_t permuted_rows, const void* residual,
