@@ -1,9 +1,8 @@
 #!/usr/bin/env python3
 """Benchmark of the W8A8-dynamic fused-MoE layer on one MI355X.
 
-One step = one pass of the whole routed-experts layer (router logits -> final bf16, shared expert included where
-the configuration has one) over one batch of synthetic tokens, through the plugin interface
-(router.select_experts -> quant_method.apply).  Prints ONE JSON line.
+One step = one call of the whole routed-experts layer, `layer(x, logits)` (router logits -> final bf16, shared expert
+included where the configuration has one), over one batch of synthetic tokens.  Prints ONE JSON line.
 
   python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload NAME[,NAME...]] [--mode graph|eager]
 
@@ -15,8 +14,9 @@ Zipf(1.1)-skewed routing at 512 and 4096 tokens; `workloads` carries the same fi
 Inputs are resident in HBM before the timed region (they are drawn on the GPU by a seeded generator).
 Per workload:
   ms_per_step   K timed steps (one HIP-graph replay per step) after W warm-up steps
-  roofline      the dominant kernel (the gate_up grouped GEMM), timed with HIP events that bracket exactly that kernel
-                in every step of a second, eager pass; its name comes from the library
+  roofline      the dominant kernel (the routed experts' gate_up grouped GEMM), timed with HIP events that bracket exactly
+                that kernel in every step of a second, eager pass; its name comes from the library's description of
+                this layer
   parity        the bit-exact gates of the layer against the CPU checker (routing ids and weights, permutation,
                 histogram and the first int8 quantisation on the whole batch; both int32 accumulators, the int8 SwiGLU
                 output, the expert output and the final output on sampled rows / tokens) and the relative error of
@@ -108,7 +108,7 @@ def log(msg: str) -> None:
 
 def capture(step, torch):
     """HIP graph of one step, checked against the eager result; None when capture is not possible."""
-    want = step().routed_out
+    want = step()
     torch.cuda.synchronize()
     try:
         side = torch.cuda.Stream()
@@ -125,7 +125,7 @@ def capture(step, torch):
         for _ in range(3):
             graph.replay()
             torch.cuda.synchronize()
-            if not torch.equal(gres.routed_out, want):
+            if not torch.equal(gres, want):
                 raise RuntimeError("graph replay differs from the eager result")
         return graph
     except Exception as exc:  # capture not possible: measure eager and say so
@@ -186,16 +186,18 @@ def run_workload(name, args, lib, torch, np):
     if args.with_gate:
         from vllm_ascend_amd.fused_moe.gate_linear import AscendGateLinear
 
-        gate = AscendGateLinear(cfg.H, cfg.E, device=dev)
+        gate = layer.gate = AscendGateLinear(cfg.H, cfg.E, device=dev)
         gate.weight.data.copy_(torch.randn(cfg.E, cfg.H, generator=torch.Generator().manual_seed(1)) * 0.05)
 
     def step():
-        if gate is not None:
-            return layer.forward_impl(x, gate(x)[0])
-        return layer.forward_impl(x, logits)
+        return layer(x) if gate is not None else layer(x, logits)
 
-    res = step()
-    torch.cuda.synchronize()
+    # the same layer operator by operator: the rows of every expert, and the output that the one call has to give
+    res = layer.forward_impl(x, logits if gate is None else gate(x)[0])
+    got = step()
+    same = bool(torch.equal(got, res.routed_out))
+    if not same:
+        log(f"{name}: layer(x, logits) differs from the operators")
     counts = res.expert_tokens.cpu().numpy()
     R = int(counts.sum())
 
@@ -214,6 +216,7 @@ def run_workload(name, args, lib, torch, np):
         "ms_per_step": round(ms_per_step, 5),
         "us_per_layer": round(ms_per_step * 1e3, 2),
         "us_per_layer_single_steps": spread,
+        "one_call_equals_the_operators": same,
         "config": {"workload": cfg.name, "tokens": cfg.T, "hidden": cfg.H, "experts": cfg.E, "top_k": cfg.k,
                    "moe_intermediate": cfg.I, "scoring": cfg.scoring, "shared_expert": bool(cfg.shared),
                    "weights": "int4 group %d" % cfg.w4_group if cfg.w4_group >= 0 else "int8 per channel",
@@ -248,45 +251,26 @@ def run_workload(name, args, lib, torch, np):
         for _ in range(min(args.warmup, 10)):
             step()
         torch.cuda.synchronize()
-        hooked = {"i": 0, "fired": 0}
-        # the launchers of the routed gate_up GEMM (batches past a decode batch read their rows through a
-        # row -> token map, decode batches run in pair order)
-        hook_names = (["gmm1_swiglu_quant_w4", "gmm1_swiglu_quant_w4_gather"] if cfg.w4_group >= 0
-                      else ["gmm1_swiglu_quant", "gmm1_swiglu_quant_gather", "gmm1_swiglu_quant_pairs", "gmm1_swiglu_pairs"])
-        origs = {h: getattr(K, h) for h in hook_names}
-
-        def make_timed(orig, routed):
-            def timed_gmm1(x_, *a, **kw):
-                if not routed(x_):  # the shared expert's dense GEMMs go through the same launcher
-                    return orig(x_, *a, **kw)
-                s, e = evs[hooked["i"]]
-                hooked["fired"] += 1
-                # create the underlying hipEvent handles, then let the library record them around the GEMM kernel
-                s.record()
-                e.record()
-                lib.moe355_profile_next_gemm(ctypes.c_void_p(s.cuda_event), ctypes.c_void_p(e.cuda_event))
-                return orig(x_, *a, **kw)
-            return timed_gmm1
-
-        for h in hook_names:
-            setattr(K, h, make_timed(origs[h], (lambda x_: True) if h.endswith(("gather", "pairs"))
-                                     else (lambda x_: x_.shape[0] == R)))
-        try:
-            torch.cuda.synchronize()
-            te0 = time.perf_counter()
-            for i in range(n):
-                hooked["i"] = i
-                step()
-            torch.cuda.synchronize()
-            out["eager_ms_per_step"] = round((time.perf_counter() - te0) * 1e3 / n, 5)
-        finally:
-            for h in hook_names:
-                setattr(K, h, origs[h])
-        if hooked["fired"] == n:
+        te0 = time.perf_counter()
+        for ev0, ev1 in evs:
+            # create the underlying hipEvent handles, then let the library record them around the GEMM kernel
+            ev0.record()
+            ev1.record()
+            lib.moe355_profile_next_gemm(ctypes.c_void_p(ev0.cuda_event), ctypes.c_void_p(ev1.cuda_event))
+            step()
+        torch.cuda.synchronize()
+        out["eager_ms_per_step"] = round((time.perf_counter() - te0) * 1e3 / n, 5)
+        lib.moe355_profile_next_gemm(None, None)
+        plan = layer._layer_plan
+        if plan is not None and plan.desc is not None:
             durs = sorted(s.elapsed_time(e) for s, e in evs)  # ms
             avg_ms = sum(durs) / len(durs)
+            kernel = lib.moe355_layer_kernel_name(plan.ref, cfg.T).decode()
             abytes = algorithmic_bytes_gmm1(cfg, counts)
             ops1 = 2 * R * cfg.H * 2 * cfg.I
+            if "shared" in kernel:  # its product is in the same launch (the same token rows)
+                abytes += int(weight_bytes(cfg, 2 * cfg.I, cfg.H)) + cfg.T * (cfg.I + 4)
+                ops1 += 2 * cfg.T * cfg.H * 2 * cfg.I
             gbs = abytes / (avg_ms * 1e-3) / 1e9
             tops = ops1 / (avg_ms * 1e-3) / 1e12
             # the binding roofline of this kernel: HBM when the weight stream outweighs the MFMA time
@@ -297,16 +281,12 @@ def run_workload(name, args, lib, torch, np):
             else:
                 roofline = {"bound": "mfma", "achieved": round(tops, 1), "peak": INT8_PEAK_TOPS, "unit": "TOP/s",
                             "frac": round(tops / INT8_PEAK_TOPS, 4)}
-            if cfg.w4_group >= 0:
-                kernel = "gmm_w4_stream_kernel"
-            else:
-                kernel = lib.moe355_gmm_kernel_name(1, R, cfg.H, 2 * cfg.I, cfg.E).decode()
             traffic = None if (args.tokens or args.zipf is not None) else TRAFFIC_FROM_PROFILES.get(name)
             roofline.update({
                 "traffic": traffic[0] if traffic else None,
                 "traffic_source": (traffic[1] + " (rocprofv3 --pmc of an earlier run of this command, not measured "
                                                 "in this run)") if traffic else None,
-                "kernel": kernel + "<EPI_SWIGLU> (gate_up grouped GEMM + dequant + SwiGLU)",
+                "kernel": kernel + " (gate_up grouped GEMM + dequant + SwiGLU)",
                 "kernel_avg_us": round(avg_ms * 1e3, 2),
                 "kernel_p50_us": round(durs[len(durs) // 2] * 1e3, 2),
                 "algorithmic_bytes": abytes,
@@ -328,7 +308,7 @@ def run_workload(name, args, lib, torch, np):
         t0 = time.perf_counter()
         r = staged_run(K, cfg, dg)
         big = cfg.H * cfg.I >= 4096 * 2048
-        parity = layer_parity(orc, cfg, dc, r, n_tokens=4 if big else 16, layer_out=res.routed_out,
+        parity = layer_parity(orc, cfg, dc, r, n_tokens=4 if big else 16, layer_out=got,
                               shared=cfg.shared)
         parity["seconds"] = round(time.perf_counter() - t0, 1)
         out["parity"] = parity
@@ -357,7 +337,7 @@ def run_workload(name, args, lib, torch, np):
             passes += 1
         from _inputs import bits
 
-        ok = bool(np.array_equal(bits(res.routed_out[:sample_T]), tr.out))
+        ok = bool(np.array_equal(bits(got[:sample_T]), tr.out))
         c_port = {
             "value": round(sample_T * passes / elapsed, 2), "unit": "tokens/s", "cores": orc.num_threads(),
             "kind": "port", "rendering": "the C checker (oracle/moe_oracle.c) with OpenMP",
@@ -447,7 +427,7 @@ def main() -> int:
     for name in names:
         results[name] = run_workload(name, args, lib, torch, np)
     head = results[head_name]
-    all_ok = all(not w.get("parity", {}).get("failed") for w in results.values())
+    all_ok = all(not w.get("parity", {}).get("failed") and w["one_call_equals_the_operators"] for w in results.values())
     out = {
         "metric": "W8A8 MoE-layer tokens/sec at 1 GPU",
         "value": head["tokens_per_s"],

@@ -490,7 +490,8 @@ int moe355_token_unpermute_pairs(const void *rows, int dtype, const void *probs,
  * state in the library: the armed pair of events is kept in thread-local storage until the next GEMM launch
  * of the same thread takes it.
  * The next grouped-GEMM kernel launched from the calling thread by
- * moe355_gmm1_swiglu_quant / moe355_gmm2_dequant / moe355_gmm_i32 is bracketed
+ * moe355_gmm1_swiglu_quant / moe355_gmm2_dequant / moe355_gmm_i32 and their other
+ * forms, or the routed gate_up product of moe355_layer_forward, is bracketed
  * by the two hipEvent_t handles (recorded immediately before and after that
  * one kernel, not the small helper kernels around it).  One-shot: the pair is
  * consumed by that launch.  Pass two NULLs to cancel.
@@ -542,6 +543,11 @@ size_t moe355_layer_workspace(const moe355_layer *layer /* host */, int64_t num_
 /* logits [T, E] of logits_dtype; ignored with a gate inside the layer.  out [T, H]. */
 int moe355_layer_forward(const moe355_layer *layer /* host */, const void *x, const void *logits, int logits_dtype,
                          int64_t num_tokens, void *out, void *workspace, size_t workspace_bytes, void *stream);
+/* The kernel that such a call launches for the routed experts' gate_up product (of which moe355_profile_next_gemm
+ * brackets one launch, whatever product the call launches first), followed by " with the shared expert" where that
+ * expert's product is in the same launch; "" for arguments no call accepts.  A pure function of its arguments, for
+ * benchmarks and profiles (no counterpart in the reference). */
+const char *moe355_layer_kernel_name(const moe355_layer *layer /* host */, int64_t num_tokens);
 
 #ifdef __cplusplus
 }

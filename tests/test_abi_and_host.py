@@ -363,3 +363,27 @@ def test_expert_load_from_both_group_list_forms():
         assert "should not be None when dynamic_eplb is enabled" in str(e)
     else:
         raise AssertionError("a result without expert_tokens must be refused")
+
+
+def test_layer_kernel_names_follow_the_form():
+    """The kernel of the routed gate_up product, as the whole-layer call launches it (no GPU: a pure function)."""
+    from vllm_ascend_amd import _lib
+
+    lib = _lib.load()
+
+    def name(T, weights=0, hidden=2048, experts=128, inter=768, shared=0, pair_order=1):
+        a = _lib.Layer(hidden=hidden, intermediate=inter, num_experts=experts, top_k=8, k_group=1, group_count=1,
+                       x_dtype=_lib.DT_BF16, weights=weights, pair_order=pair_order, w13=256, s13=256, w2=256, s2=256,
+                       group13=256, group2=256, shared=shared, shared_intermediate=inter, shared_alpha=1.0,
+                       shared_w13=256, shared_s13=256, shared_w2=256, shared_s2=256)
+        return lib.moe355_layer_kernel_name(ctypes.byref(a), T).decode()
+
+    assert name(1) == "few_up_kernel" and name(64) == "gmm_stream_kernel"
+    assert name(1, shared=1) == "few_up_kernel with the shared expert"
+    big = dict(hidden=7168, experts=256, inter=2048)
+    assert name(64, shared=1, **big) == "gmm_stream_kernel with the shared expert"
+    assert name(64, pair_order=0, **big) == "gmm_tiled_kernel" == name(512, **big)
+    assert name(4096, **big) == "gmm_wide_kernel"
+    assert name(16, weights=2, **big) == "gmm_w4_pairs_kernel" and name(512, weights=2, **big) == "gmm_w4_stream_kernel"
+    assert name(0) == "" and name(4, shared=3) == ""
+    assert lib.moe355_layer_kernel_name(None, 4) == b""

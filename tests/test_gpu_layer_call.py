@@ -247,3 +247,29 @@ def test_expert_loads_without_weight_lists(tokens):
     layer.eplb_heat_collection_status = False
     assert torch.equal(layer(x, logits), res.routed_out)
     assert torch.equal(layer.moe_load, 2 * res.expert_tokens)
+
+
+@pytest.mark.parametrize("name, tokens, kw", [("c2_small", 2, {}), ("c2_small", 48, {}), ("c2_small", 300, {}),
+                                              ("c4_small", 96, dict(shared=True)), ("c4_small", 300, dict(shared=True)),
+                                              ("c5_small", 16, {}), ("c5_small", 80, {})])
+def test_measurement_hook_brackets_the_routed_gate_up_product(name, tokens, kw):
+    import ctypes
+
+    from vllm_ascend_amd._lib import load
+
+    cfg, layer, x, logits = _pair(name, tokens, **kw)
+    want = layer(x, logits)
+    ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    ev0.record()
+    ev1.record()  # creates the handles
+    torch.cuda.synchronize()
+    before = ev0.elapsed_time(ev1)
+    load().moe355_profile_next_gemm(ctypes.c_void_p(ev0.cuda_event), ctypes.c_void_p(ev1.cuda_event))
+    assert torch.equal(layer(x, logits), want)
+    torch.cuda.synchronize()
+    first = ev0.elapsed_time(ev1)
+    print(f"hook {name} {tokens}: {before * 1e3:.1f} -> {first * 1e3:.1f} us", flush=True)
+    assert first != before and 5e-4 < first < 5.0
+    layer(x, logits)  # taken by the call before
+    torch.cuda.synchronize()
+    assert ev0.elapsed_time(ev1) == first

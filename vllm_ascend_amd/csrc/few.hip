@@ -11,6 +11,8 @@
 // The ids of at most 64 pairs are one load of one wavefront: every wavefront knows the distinct experts, its expert's
 // rows and its share of the work from ballots, without LDS tables or barriers.  Tokens are the 16-column operand of
 // v_mfma_i32_16x16x64_i8, so an accumulator is four registers and 8 wavefronts cutting K meet in 2 KB of LDS.
+#include <hip/hip_ext.h>
+
 #include "gmm_common.h"
 #include "layer_parts.h"
 
@@ -438,7 +440,10 @@ int few_forward(const FewArgs& a, hipStream_t st)
         return MOE355_E_SHAPE;
     const int places = a.R < a.E ? a.R : a.E;
     const dim3 up((unsigned)(places * (a.I / 16) + (a.sw2 ? a.S / 16 : 0)));
-    hipLaunchKernelGGL(few_up_kernel<4>, up, dim3(kFewThreads), 0, st, a);
+    hipEvent_t ev0, ev1;
+    take_profile_events(ev0, ev1);
+    if (ev0) hipExtLaunchKernelGGL(few_up_kernel<4>, up, dim3(kFewThreads), 0, st, ev0, ev1, 0, a);
+    else hipLaunchKernelGGL(few_up_kernel<4>, up, dim3(kFewThreads), 0, st, a);
     const size_t lds = few_lds_bytes(a);
     const bool inside = few_quant_inside(a);
     if (!inside) hipLaunchKernelGGL(few_quant_kernel, dim3((unsigned)(a.R + (a.sw2 ? a.T : 0))), dim3(256), 0, st, a);

@@ -868,7 +868,12 @@ int moe355::gmm1_w4_pairs(const int8_t* x, const float* x_scale, const int32_t* 
     p.g.pair_gather = 1;
     p.g.limit = swiglu_limit;
     p.g.y = y;
-    hipLaunchKernelGGL((gmm_w4_pairs_kernel<EPI_SWIGLU>), w4_pair_grid(p), dim3(256), 0, st, p);
+    hipEvent_t ev0, ev1;
+    take_profile_events(ev0, ev1);
+    if (ev0)
+        hipExtLaunchKernelGGL((gmm_w4_pairs_kernel<EPI_SWIGLU>), w4_pair_grid(p), dim3(256), 0, st, ev0, ev1, 0, p);
+    else
+        hipLaunchKernelGGL((gmm_w4_pairs_kernel<EPI_SWIGLU>), w4_pair_grid(p), dim3(256), 0, st, p);
     launch_swiglu_requant(y, nullptr, 0, num_experts, p.g.R, (int)(n / 2), out, out_scale, st);
     return launch_status();
 }

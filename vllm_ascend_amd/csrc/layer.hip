@@ -5,6 +5,7 @@
 #include <mutex>
 #include <vector>
 
+#include "gmm_common.h"
 #include "layer_parts.h"
 
 using namespace moe355;
@@ -342,6 +343,17 @@ extern "C" size_t moe355_layer_workspace(const moe355_layer* layer, int64_t num_
     return lay_out(*layer, forms_of(*layer, num_tokens), num_tokens, nullptr).total;
 }
 
+extern "C" const char* moe355_layer_kernel_name(const moe355_layer* layer, int64_t num_tokens)
+{
+    if (check_layer(layer) != MOE355_OK || num_tokens <= 0) return "";
+    const moe355_layer& l = *layer;
+    const Forms f = forms_of(l, num_tokens);
+    if (f.few) return l.shared ? "few_up_kernel with the shared expert" : "few_up_kernel";
+    if (l.weights == W_INT4) return f.pairs ? "gmm_w4_pairs_kernel" : "gmm_w4_stream_kernel";
+    if (f.pairs) return f.merged ? "gmm_stream_kernel with the shared expert" : "gmm_stream_kernel";
+    return moe355_gmm_kernel_name(1, num_tokens * l.top_k, l.hidden, 2 * l.intermediate, l.num_experts);
+}
+
 extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, const void* logits, int logits_dtype,
                                     int64_t num_tokens, void* out, void* workspace, size_t workspace_bytes,
                                     void* stream)
@@ -358,6 +370,9 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
     const Buffers b = lay_out(l, f, T, workspace);
     if (!workspace || ((uintptr_t)workspace & 255) || workspace_bytes < b.total) return MOE355_E_WORKSPACE;
 
+    // measurement hook: the armed events are the routed gate_up product's, whatever is launched in front of it
+    hipEvent_t ev0, ev1;
+    take_profile_events(ev0, ev1);
     GateCall g = {x, logits, l.bias, l.x_dtype, logits_dtype, T, l.hidden, l.num_experts, l.top_k, l.k_group,
                   l.group_count, 1, l.renorm, l.norm_type, l.routed_scaling_factor, l.eps};
     if (l.gate_weight) {
@@ -372,6 +387,7 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
     if (rc != MOE355_OK) return rc;
     if (f.few) {
         // the shared expert rides in the same two launches, whatever stream it was meant for
+        (void)moe355_profile_next_gemm(ev0, ev1);
         FewArgs a = few_args(l, b, T);
         a.out = (uint16_t*)out;
         return few_forward(a, (hipStream_t)stream);
@@ -406,7 +422,10 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
         rc = route_map_impl(b.topk_ids, T, l.top_k, l.num_experts, 1, b.dst, b.row_token, b.expert_tokens, b.map_ws,
                             b.map_bytes, specs, n, &tiles_ready, stream);
     }
-    if (rc == MOE355_OK) rc = f.pairs ? routed_pairs(l, f, b, T, stream) : routed_sorted(l, b, T, tiles_ready, stream);
+    if (rc == MOE355_OK) {
+        (void)moe355_profile_next_gemm(ev0, ev1);
+        rc = f.pairs ? routed_pairs(l, f, b, T, stream) : routed_sorted(l, b, T, tiles_ready, stream);
+    }
     if (!joined && hipStreamWaitEvent((hipStream_t)stream, lease.fj.join, 0) != hipSuccess) return MOE355_E_LAUNCH;
     if (rc != MOE355_OK) return rc;
     const void* residual = l.shared ? b.sh_out : nullptr;
