@@ -10,7 +10,8 @@ Without --workload every configured workload runs in this one process: the DeepS
 (the largest single-GPU configuration and the shape the target is stated on: the top-level `value`, `ms_per_step`,
 `roofline` and `cpu_baseline` are its figures), the Qwen3-30B-A3B-shaped decode and prefill batches, the W4A8
 Zipf-routed batch, the DeepSeek-V3-shaped 64-token decode batch and the same shape with int8 weights under
-Zipf(1.1)-skewed routing at 512 and 4096 tokens; `workloads` carries the same figures for each.
+Zipf(1.1)-skewed routing at 512 and 4096 tokens; `workloads` carries the main figures of each, the whole records go
+to stderr.
 Inputs are resident in HBM before the timed region (they are drawn on the GPU by a seeded generator).
 Per workload:
   ms_per_step   K timed steps (one HIP-graph replay per step) after W warm-up steps
@@ -104,6 +105,24 @@ def layer_bytes(cfg, counts) -> int:
 
 def log(msg: str) -> None:
     print(f"bench.py: {msg}", file=sys.stderr, flush=True)
+
+
+def brief(w: dict) -> dict:
+    """The figures of one workload for the result line; the whole record is on stderr.  A line of all the records is
+    24 KB, and whoever keeps the last 10 KB of an output could not read it."""
+    keep = ("tokens_per_s", "ms_per_step", "us_per_layer", "us_per_layer_single_steps", "eager_ms_per_step",
+            "us_per_layer_single_steps_after_cache_flush", "shared_expert_on_side_stream",
+            "one_call_equals_the_operators")
+    out = {k: w[k] for k in keep if k in w}
+    out["config"] = {k: w["config"][k] for k in ("tokens", "experts_touched", "rows", "launch")}
+    out["layer_frac_of_peak"] = {k: w["layer_frac_of_peak"][k] for k in ("hbm", "mfma")}
+    for part, fields in (("roofline", ("bound", "achieved", "unit", "frac", "traffic", "kernel", "kernel_avg_us",
+                                       "algorithmic_bytes")),
+                         ("parity", ("failed", "output_bit_exact", "rel_err_vs_fp32_dequant_reference")),
+                         ("cpu_baseline", ("value", "unit", "kind"))):
+        if w.get(part):
+            out[part] = {k: w[part][k] for k in fields if k in w[part]}
+    return out
 
 
 def capture(step, torch):
@@ -378,6 +397,7 @@ def run_workload(name, args, lib, torch, np):
         out["cpu_baseline"] = None
     del layer, dg, dc, graph, gpu_expert_rows
     torch.cuda.empty_cache()
+    log(f"{name}: " + json.dumps(out))
     log(f"{name}: {out['us_per_layer']} us per layer, done in {time.perf_counter() - t_start:.1f} s")
     return out
 
@@ -450,7 +470,7 @@ def main() -> int:
         "cpu_baseline": head["cpu_baseline"],
         "parity": head.get("parity"),
         "parity_gates_hold_on_every_workload": all_ok,
-        "workloads": results,
+        "workloads": {name: brief(w) for name, w in results.items()},
     }
     print(json.dumps(out))
     return 0
