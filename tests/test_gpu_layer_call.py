@@ -14,8 +14,8 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-def _pair(name, tokens, **kw):
-    cfg = dataclasses.replace(CONFIGS[name], T=tokens)
+def _pair(name, tokens, shape=None, **kw):
+    cfg = dataclasses.replace(CONFIGS[name], T=tokens, **(shape or {}))
     d = make_layer(cfg, seed=tokens)
     return cfg, build_layer(cfg, d, DEV, **kw), d["x"].to(DEV), d["logits"].to(DEV)
 
@@ -273,3 +273,91 @@ def test_measurement_hook_brackets_the_routed_gate_up_product(name, tokens, kw):
     layer(x, logits)  # taken by the call before
     torch.cuda.synchronize()
     assert ev0.elapsed_time(ev1) == first
+
+
+# every form of the call: a few tokens (their rows quantised in place; by a launch; with the shared expert), pair order
+# (a launch re-quantises; the down GEMM does, rows of one and of several loads; the shared expert in the launches), int4 in pair order and sorted, the sorted path with
+# the shared expert in line and on its side stream, per-expert weight tables
+_REQ = dict(H=1024, E=128, k=8)
+FORMS = [("c2_small", 2, {}), ("c2_small", 2, dict(shape=dict(H=1024, E=128, k=8, I=1408))),
+         ("c4_small", 2, dict(shared=True)), ("c2_small", 24, {}), ("c2_small", 100, {}),
+         ("c2_small", 40, dict(shape=dict(I=320, **_REQ))), ("c2_small", 40, dict(shape=dict(I=1408, **_REQ))),
+         ("c4_small", 40, dict(shared=True)), ("c4_small", 96, dict(shared=True, overlap=True)), ("c5_small", 12, {}),
+         ("c5_small", 80, {}), ("c4_small", 300, dict(shared=True)), ("c4_small", 300, dict(shared=True, overlap=True)),
+         ("c7_small", 40, dict(dynamic_eplb=True)), ("c7_small", 300, dict(dynamic_eplb=True))]
+
+
+def _as_fp16(layer, x):
+    layer.quant_method.in_dtype = torch.float16
+    return x.to(torch.float16)
+
+
+@pytest.mark.parametrize("name, tokens, kw", FORMS)
+@pytest.mark.parametrize("gate", [False, True])
+def test_a_captured_call_replays_on_new_inputs(name, tokens, kw, gate):
+    """Replays with other inputs in the captured buffers, eager work and synchronisations between them."""
+    from vllm_ascend_amd.fused_moe.gate_linear import AscendGateLinear
+
+    print(f"capture {name} {tokens} {kw} gate={gate}", flush=True)
+    cfg, layer, x, logits = _pair(name, tokens, **kw)
+    if gate:
+        layer.gate = AscendGateLinear(cfg.H, cfg.E, device=DEV)
+        layer.gate.weight.data.normal_(0.0, cfg.H ** -0.5)
+    args = (x,) if gate else (x, logits)
+    for _ in range(2):
+        layer(*args)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = layer(*args)
+    first = [a.clone() for a in args]
+    for shift in (0, 1, 5, 0):
+        for a, f in zip(args, first):
+            a.copy_(f.roll(shift, 0) * (1.0 + shift))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = out.clone()
+        assert torch.equal(got, layer(*args))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, got)
+
+
+@pytest.mark.parametrize("name, tokens, kw", FORMS)
+def test_fp16_hidden_states_in_the_call(name, tokens, kw):
+    cfg, layer, x, logits = _pair(name, tokens, **kw)
+    x = _as_fp16(layer, x)
+    got = layer(x, logits)
+    assert got.dtype == torch.float16 and layer._layer_plan.desc is not None
+    assert torch.equal(got, layer.forward_impl(x, logits).routed_out)
+    layer.use_fused_small_batch = False
+    assert torch.equal(got, layer.forward_impl(x, logits).routed_out)
+
+
+def _same_values(a, b):
+    return bool((((a == b) | (a.isnan() & b.isnan()))).all())
+
+
+# an infinity or a NaN in a token's hidden states (the row's maximum, and through the scale its SwiGLU values), a value
+# large enough for the products to overflow: the operators on the sorted order say what comes out, and the other tokens'
+# rows must not notice
+@pytest.mark.parametrize("name, tokens, kw", FORMS)
+def test_infinities_and_nans(name, tokens, kw):
+    print(f"inf and nan {name} {tokens} {kw}", flush=True)
+    cfg, layer, x, logits = _pair(name, tokens, **kw)
+    if "shape" in kw and tokens > 2:
+        from vllm_ascend_amd.kernels import gmm2_requant_pairs_supported
+
+        assert gmm2_requant_pairs_supported(tokens, cfg.k, cfg.H, cfg.I, cfg.E)
+    clean = layer(x, logits)
+    rows = {0: float("inf"), tokens // 2: float("nan"), tokens - 1: -3e38}
+    for t, v in rows.items():
+        x[t, 7 * t % cfg.H] = v
+    got = layer(x, logits)
+    layer.use_fused_small_batch = False
+    want = layer.forward_impl(x, logits).routed_out
+    layer.use_fused_small_batch = True
+    assert _same_values(got, want) and _same_values(layer.forward_impl(x, logits).routed_out, want)
+    others = [t for t in range(tokens) if t not in rows]
+    assert torch.equal(got[others], clean[others])
