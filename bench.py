@@ -49,13 +49,13 @@ WORKLOADS = ["c4_dsv3_prefill", "c2_qwen3_decode", "c3_qwen3_prefill", "c5_w4a8_
 # HBM bytes per launch of the dominant kernel from rocprofv3 --pmc runs (FETCH_SIZE / WRITE_SIZE scaled by a copy
 # kernel of known size), taken from the committed summaries: NOT measured in this run.
 TRAFFIC_FROM_PROFILES = {
-    "c2_qwen3_decode": (401_500_000, "profiles/moe_layer_qwen3_decode_kernel_trace.md"),
-    "c3_qwen3_prefill": (952_400_000, "profiles/moe_layer_qwen3_prefill_kernel_trace.md"),
-    "c4_dsv3_prefill": (8_030_700_000, "profiles/moe_layer_dsv3_prefill_kernel_trace.md"),
-    "c5_w4a8_zipf": (1_662_500_000, "profiles/moe_layer_w4a8_zipf_kernel_trace.md"),
-    "c6_dsv3_decode": (6_600_600_000, "profiles/moe_layer_dsv3_decode_kernel_trace.md"),
-    "c7_w8a8_zipf": (2_892_100_000, "profiles/moe_layer_w8a8_zipf_kernel_trace.md"),
-    "c7_w8a8_zipf_4096": (8_314_400_000, "profiles/moe_layer_w8a8_zipf_4096_kernel_trace.md"),
+    "c2_qwen3_decode": (399_900_000, "profiles/moe_layer_qwen3_decode_kernel_trace.md"),
+    "c3_qwen3_prefill": (950_000_000, "profiles/moe_layer_qwen3_prefill_kernel_trace.md"),
+    "c4_dsv3_prefill": (8_029_100_000, "profiles/moe_layer_dsv3_prefill_kernel_trace.md"),
+    "c5_w4a8_zipf": (1_625_500_000, "profiles/moe_layer_w4a8_zipf_kernel_trace.md"),
+    "c6_dsv3_decode": (6_595_500_000, "profiles/moe_layer_dsv3_decode_kernel_trace.md"),
+    "c7_w8a8_zipf": (3_041_500_000, "profiles/moe_layer_w8a8_zipf_kernel_trace.md"),
+    "c7_w8a8_zipf_4096": (8_322_000_000, "profiles/moe_layer_w8a8_zipf_4096_kernel_trace.md"),
 }
 
 
@@ -196,7 +196,8 @@ def run_workload(name, args, lib, torch, np):
         cfg = dataclasses.replace(cfg, zipf=args.zipf)  # ... with another skew of the expert popularity
     t_start = time.perf_counter()
     dg = make_layer(cfg, seed=0, gen_device=dev)
-    layer = build_layer(cfg, dg, dev, shared=cfg.shared, overlap=False)
+    layer = build_layer(cfg, dg, dev, shared=cfg.shared, overlap=False, dynamic_eplb=args.weight_lists,
+                        collect_expert_load=args.weight_lists)
     x, logits = dg["x"], dg["logits"]
     torch.cuda.synchronize()
     log(f"{name}: layer built in {time.perf_counter() - t_start:.1f} s")
@@ -239,7 +240,7 @@ def run_workload(name, args, lib, torch, np):
         "config": {"workload": cfg.name, "tokens": cfg.T, "hidden": cfg.H, "experts": cfg.E, "top_k": cfg.k,
                    "moe_intermediate": cfg.I, "scoring": cfg.scoring, "shared_expert": bool(cfg.shared),
                    "weights": "int4 group %d" % cfg.w4_group if cfg.w4_group >= 0 else "int8 per channel",
-                   "launch": mode, "router_gate": gate is not None, "experts_touched": int((counts > 0).sum()),
+                   "launch": mode, "router_gate": gate is not None, "weight_lists": args.weight_lists, "experts_touched": int((counts > 0).sum()),
                    "rows": R},
     }
     lbytes, lops = layer_bytes(cfg, counts), algorithmic_ops(cfg, R)
@@ -413,6 +414,8 @@ def main() -> int:
                     help="run the named workload(s) on a batch of this many tokens instead of their own")
     ap.add_argument("--zipf", type=float, default=None,
                     help="expert popularity ~ rank^-S for the named workload(s) instead of their own (0: uniform)")
+    ap.add_argument("--weight-lists", action="store_true",
+                    help="per-expert weight tensors and collected expert loads, as under a dynamic load balancer")
     ap.add_argument("--mode", choices=["graph", "eager"], default="graph")
     ap.add_argument("--with-gate", action="store_true",
                     help="start the step one operator earlier: the fp32 router gate GEMM (hidden states -> logits, "
