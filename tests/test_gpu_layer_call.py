@@ -361,3 +361,29 @@ def test_infinities_and_nans(name, tokens, kw):
     assert _same_values(got, want) and _same_values(layer.forward_impl(x, logits).routed_out, want)
     others = [t for t in range(tokens) if t not in rows]
     assert torch.equal(got[others], clean[others])
+
+
+# scales that start in the middle of a 16-byte line: what the operators refuse, the call refuses in each of its forms
+@pytest.mark.parametrize("name, tokens, kw, where", [
+    ("c2_small", 2, {}, "w13_weight_scale_fp32"), ("c2_small", 2, {}, "w2_weight_scale_fp32"),
+    ("c2_small", 48, {}, "w13_weight_scale_fp32"), ("c2_small", 300, {}, "w2_weight_scale_fp32"),
+    ("c5_small", 12, {}, "w13_weight_scale"), ("c5_small", 12, {}, "w2_weight_scale"), ("c5_small", 80, {}, "w2_weight_scale"),
+    ("c4_small", 2, dict(shared=True), "down_scale_fp32"), ("c4_small", 96, dict(shared=True), "down_scale_fp32"),
+    ("c4_small", 300, dict(shared=True), "down_scale_fp32")])
+def test_misaligned_scales_are_refused(name, tokens, kw, where):
+    from vllm_ascend_amd._lib import Moe355Error
+
+    cfg, layer, x, logits = _pair(name, tokens, **kw)
+    layer(x, logits)
+    owner = layer.shared_experts if where == "down_scale_fp32" else layer
+    t = getattr(owner, where)
+    shifted = torch.empty(t.numel() + 1, device=DEV)[1:].view(t.shape)
+    shifted.copy_(t)
+    if isinstance(t, torch.nn.Parameter):
+        t.data = shifted
+    else:
+        setattr(owner, where, shifted)
+    with pytest.raises(Moe355Error, match="alignment"):
+        layer.forward_impl(x, logits)
+    with pytest.raises(Moe355Error, match="alignment"):
+        layer(x, logits)

@@ -435,9 +435,11 @@ static bool few_quant_inside(const FewArgs& a) { return (int64_t)a.R * a.I + (a.
 int few_forward(const FewArgs& a, hipStream_t st)
 {
     if (!few_supported(a)) return MOE355_E_SHAPE;
-    if (((uintptr_t)a.xq & 15) || ((uintptr_t)a.y & 15) || ((uintptr_t)a.q1 & 15) || ((uintptr_t)a.w13 & 15) ||
-        ((uintptr_t)a.w2 & 15) || ((uintptr_t)a.sw13 & 15) || ((uintptr_t)a.sw2 & 15))
-        return MOE355_E_SHAPE;
+    // the scales are read one by one here, but the operators take none that are not aligned
+    for (const void* p : {(const void*)a.xq, (const void*)a.y, (const void*)a.q1, (const void*)a.w13, (const void*)a.w2,
+                          (const void*)a.sw13, (const void*)a.sw2, (const void*)a.s13, (const void*)a.s2,
+                          (const void*)a.ss13, (const void*)a.ss2})
+        if ((uintptr_t)p & 15) return MOE355_E_SHAPE;
     const int places = a.R < a.E ? a.R : a.E;
     const dim3 up((unsigned)(places * (a.I / 16) + (a.sw2 ? a.S / 16 : 0)));
     hipEvent_t ev0, ev1;

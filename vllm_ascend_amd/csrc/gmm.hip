@@ -1050,6 +1050,7 @@ int moe355::gmm1_pairs_impl(const int8_t* x, const float* x_scale, const int32_t
     if ((int64_t)num_experts * (n / 64) >= 0x7fffffffLL) return MOE355_E_SHAPE;
     if (!x || !x_scale || !topk_ids || !w.complete() || !y) return MOE355_E_ARG;
     if (((uintptr_t)x & 15) || !w.aligned() || ((uintptr_t)y & 15) || ((uintptr_t)out & 3)) return MOE355_E_SHAPE;
+    if (shared && !shared->aligned()) return MOE355_E_SHAPE;
     hipStream_t st = (hipStream_t)stream;
     const int64_t rows = num_tokens * top_k;
     GmmArgs a = {};
@@ -1092,6 +1093,7 @@ int moe355::gmm2_pairs_impl(const int8_t* x, const float* per_token_scale, const
     if ((int64_t)num_experts * (n / 64) >= 0x7fffffffLL) return MOE355_E_SHAPE;
     if (!w.complete() || !topk_ids || !out || (!y && (!x || !per_token_scale))) return MOE355_E_ARG;
     if (((uintptr_t)x & 15) || ((uintptr_t)y & 15) || !w.aligned() || ((uintptr_t)out & 15)) return MOE355_E_SHAPE;
+    if (shared && !shared->aligned()) return MOE355_E_SHAPE;
     hipStream_t st = (hipStream_t)stream;
     GmmArgs a = {};
     a.x = x;

@@ -863,7 +863,7 @@ int moe355::gmm1_w4_pairs(const int8_t* x, const float* x_scale, const int32_t* 
 {
     if (!x || !x_scale || !topk_ids || !w || !scale || !y || !out || !out_scale) return MOE355_E_ARG;
     if (n % 64 != 0 || k % 64 != 0 || group % 64 != 0 || k % group != 0) return MOE355_E_SHAPE;
-    if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)y & 15)) return MOE355_E_SHAPE;
+    if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)scale & 15) || ((uintptr_t)y & 15)) return MOE355_E_SHAPE;
     W4Args p = w4_pair_args(x, x_scale, topk_ids, num_tokens, top_k, w, scale, group, k, n, num_experts);
     p.g.pair_gather = 1;
     p.g.limit = swiglu_limit;
@@ -884,7 +884,7 @@ int moe355::gmm2_w4_pairs(const int8_t* x, const float* x_scale, const int32_t* 
 {
     if (!x || !x_scale || !topk_ids || !w || !scale || !out) return MOE355_E_ARG;
     if (n % 64 != 0 || k % 64 != 0 || group % 64 != 0 || k % group != 0) return MOE355_E_SHAPE;
-    if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)out & 7)) return MOE355_E_SHAPE;
+    if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)scale & 15) || ((uintptr_t)out & 7)) return MOE355_E_SHAPE;
     W4Args p = w4_pair_args(x, x_scale, topk_ids, num_tokens, top_k, w, scale, group, k, n, num_experts);
     p.g.out = (uint16_t*)out;
     p.g.out_f16 = out_dtype == MOE355_DT_F16;

@@ -46,6 +46,7 @@ struct PairShared {
     const int8_t* w;
     const float* scale;
     float limit = 0.0f;
+    bool aligned() const { return !((uintptr_t)w & 15) && !((uintptr_t)scale & 15); }
     template <typename Args>
     void into(Args& a, int num_tokens) const
     {
