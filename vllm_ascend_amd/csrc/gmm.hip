@@ -12,7 +12,6 @@
 // LDS (integer addition: exact, order free).
 #include <hip/hip_ext.h>
 #include <stdlib.h>
-#include <string.h>
 #include <type_traits>
 
 #include "gmm_common.h"

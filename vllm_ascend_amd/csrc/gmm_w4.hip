@@ -205,8 +205,9 @@ __device__ __forceinline__ bool find_chunk(const int64_t* gl, int gl_type, int E
 // Besides HBM the vector ALU bounds it (the fold of 64 sums and the unpacking take longer than the MFMAs), so the fold is
 // conversion, product and sum alone: no shift (the scales in LDS are a sixteenth) and no clearing (the first product of a
 // group starts from the instruction's own zero).  DeepSeek-V3 shape, groups of 256, us a layer call before / after both
-// and the halved barriers: uniform 512 / 1024 / 2048 tokens 1040 / 1236 / 1765 -> 1030 / 1206 / 1707, Zipf(1.1) 128 / 512 /
-// 1024 tokens 334 / 595 / 929 -> 324 / 587 / 883; groups of 128 (scales from memory) 1237 -> 1193 at 512, 771 -> 729 Zipf.
+// and the halved barriers: uniform 512 / 1024 / 2048 tokens 1040 / 1236 / 1765 -> 1030 / 1206 / 1707, Zipf(1.1) 128 /
+// 1024 tokens 334 / 929 -> 324 / 883 (512 skewed tokens: less than runs of one side differ); groups of 128 (scales from
+// memory) 1237 -> 1193 at 512, 771 -> 729 Zipf.
 constexpr int kW4Chunk = 64;
 constexpr int kW4LdsGroups = 32;  // K groups whose scales are kept in LDS (8 KiB per wavefront)
 // LDS_SCALES: the group scales of the wavefront's channels fit LDS (K / group <= kW4LdsGroups)
