@@ -193,9 +193,10 @@ def test_one_layer_on_two_streams(name, tokens, kw, options):
         assert all(torch.equal(o, w) for o in out)
 
 
+@pytest.mark.parametrize("whole", [True, False])
 @pytest.mark.parametrize("name, tokens, kw, options", AT_A_TIME)
-def test_one_layer_on_two_threads(name, tokens, kw, options):
-    print(f"two threads: {name} {tokens} {kw} {options}", flush=True)
+def test_one_layer_on_two_threads(name, tokens, kw, options, whole):
+    print(f"two threads: {name} {tokens} {kw} {options} whole={whole}", flush=True)
     layer, batches, want = _two_batches(name, tokens, kw, options)
     torch.cuda.synchronize()
     got, failed = [[], []], []
@@ -204,7 +205,7 @@ def test_one_layer_on_two_threads(name, tokens, kw, options):
         try:
             with torch.cuda.stream(torch.cuda.Stream()):
                 for _ in range(20):
-                    got[i].append(layer(*batches[i]))
+                    got[i].append(layer(*batches[i]) if whole else layer.forward_impl(*batches[i]).routed_out)
                 torch.cuda.current_stream().synchronize()
         except Exception as exc:  # noqa: BLE001 -- reported by the test's own thread
             failed.append(exc)

@@ -1,5 +1,6 @@
 """Which calls the whole-layer call takes, and when it looks at the layer again: host code, no GPU."""
 import ctypes
+import threading
 import types
 
 import pytest
@@ -300,3 +301,51 @@ def test_no_counter_is_shared_between_calls(told, scheme, pair_order):
     layer.use_pair_order = pair_order
     assert layer_call(layer, X, LOGITS) is not None
     assert not told[-1].sync_counter
+
+
+def test_each_thread_waits_for_its_own_shared_expert(monkeypatch):
+    """Two calls of one layer at a time, the shared expert of both on the side stream: neither takes the other's event."""
+    here = threading.local()
+
+    class Stream:
+        def __init__(self, name):
+            self.name, self.waited = name, []
+
+        def record_event(self):
+            return f"{here.name} on {self.name}"
+
+        def wait_event(self, evt):
+            self.waited.append(evt)
+
+        def __enter__(self):
+            return self
+
+        def __exit__(self, *exc):
+            return None
+
+    side = Stream("side")
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: here.stream)
+    monkeypatch.setattr(torch.cuda, "stream", lambda s: s)
+    monkeypatch.setattr(torch.Tensor, "record_stream", lambda self, s: None)
+    monkeypatch.setattr("vllm_ascend_amd.fused_moe.shared_experts.shared_experts_calculation_stream",
+                        lambda *a: side)
+    monkeypatch.setattr(AscendSharedExperts, "_mlp", lambda self, x, quantized=None: x)
+    shared = AscendSharedExperts.__new__(AscendSharedExperts)
+    torch.nn.Module.__init__(shared)
+    shared.multistream_overlap, shared._done_evts = True, {}
+    both_enqueued, waited = threading.Barrier(2, timeout=30), {}
+
+    def call(name):
+        here.name, here.stream = name, Stream(name)
+        shared.forward(torch.zeros(1))
+        both_enqueued.wait()
+        shared.wait()
+        shared.wait()  # nothing left
+        waited[name] = here.stream.waited
+
+    threads = [threading.Thread(target=call, args=(n,)) for n in ("a", "b")]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert waited == {"a": ["a on side"], "b": ["b on side"]}

@@ -8,6 +8,8 @@ stream (default priority) next to the routed experts, fenced by events like the 
 ``before_routed_experts`` / ``wait_stream`` pair."""
 from __future__ import annotations
 
+import threading
+
 import torch
 
 from .. import npu_ops
@@ -41,6 +43,9 @@ class AscendSharedExperts(torch.nn.Module):
         self.swiglu_alpha = swiglu_alpha
         self.swiglu_beta = swiglu_beta
         self.multistream_overlap = multistream_overlap
+        # thread -> event behind the side-stream MLP that this thread has enqueued and not waited for yet: a layer may be
+        # called by several threads at a time, and each waits for its own
+        self._done_evts = {}
 
     def _mlp(self, hidden_states: torch.Tensor, quantized=None) -> torch.Tensor:
         original_dtype = hidden_states.dtype
@@ -72,11 +77,11 @@ class AscendSharedExperts(torch.nn.Module):
             for t in quantized:
                 t.record_stream(side)
         out.record_stream(main)
-        self._done_evt = done
+        self._done_evts[threading.get_ident()] = done
         return out
 
     def wait(self) -> None:
-        """Make the current stream wait for the side-stream MLP (``wait_stream`` in the reference)."""
-        if self.multistream_overlap and getattr(self, "_done_evt", None) is not None:
-            torch.cuda.current_stream().wait_event(self._done_evt)
-            self._done_evt = None
+        """Make the current stream wait for the side-stream MLP of this thread (``wait_stream`` in the reference)."""
+        done = self._done_evts.pop(threading.get_ident(), None)
+        if done is not None:
+            torch.cuda.current_stream().wait_event(done)
