@@ -349,3 +349,14 @@ def test_each_thread_waits_for_its_own_shared_expert(monkeypatch):
     for t in threads:
         t.join()
     assert waited == {"a": ["a on side"], "b": ["b on side"]}
+
+
+def test_every_device_has_a_side_stream_of_its_own(monkeypatch):
+    from vllm_ascend_amd.fused_moe import shared_experts as module
+
+    monkeypatch.setattr(module, "_SIDE_STREAMS", {})
+    monkeypatch.setattr(torch.cuda, "Stream", lambda device=None: types.SimpleNamespace(device=device))
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    first, second = module.shared_experts_calculation_stream(0), module.shared_experts_calculation_stream(1)
+    assert (first.device, second.device) == (0, 1)
+    assert module.shared_experts_calculation_stream() is second and module.shared_experts_calculation_stream(0) is first

@@ -227,7 +227,7 @@ def _make_plan(layer, x, logits, key) -> _Plan:
         a.shared = 2 if overlap else 1
         a.shared_w13, a.shared_s13, a.shared_w2, a.shared_s2 = up[0], up_scale[0], down[0], down_scale[0]
         if overlap:
-            a.shared_stream = shared_experts_calculation_stream().cuda_stream
+            a.shared_stream = shared_experts_calculation_stream(dev).cuda_stream
     if load is not None:
         if not _is(load, torch.int64, (E,), dev):
             return plan

@@ -15,14 +15,17 @@ import torch
 from .. import npu_ops
 from ..custom_ops import enable_custom_op
 
-_SIDE_STREAM = None
+_SIDE_STREAMS: dict[int, torch.cuda.Stream] = {}
 
 
-def shared_experts_calculation_stream() -> torch.cuda.Stream:
-    global _SIDE_STREAM
-    if _SIDE_STREAM is None:
-        _SIDE_STREAM = torch.cuda.Stream()  # default priority
-    return _SIDE_STREAM
+def shared_experts_calculation_stream(device: int | None = None) -> torch.cuda.Stream:
+    """The side stream of a device (of the current one by default)."""
+    if device is None:
+        device = torch.cuda.current_device()
+    if device not in _SIDE_STREAMS:
+        # default priority; of two threads that come at the same time both get the first one's
+        _SIDE_STREAMS.setdefault(device, torch.cuda.Stream(device))
+    return _SIDE_STREAMS[device]
 
 
 class AscendSharedExperts(torch.nn.Module):
@@ -64,7 +67,7 @@ class AscendSharedExperts(torch.nn.Module):
     def forward(self, hidden_states: torch.Tensor, before_routed_experts_evt=None, quantized=None) -> torch.Tensor:
         if not self.multistream_overlap:
             return self._mlp(hidden_states, quantized)
-        side = shared_experts_calculation_stream()
+        side = shared_experts_calculation_stream(hidden_states.device.index)
         main = torch.cuda.current_stream()
         if before_routed_experts_evt is None:
             before_routed_experts_evt = main.record_event()
