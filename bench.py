@@ -240,8 +240,8 @@ def run_workload(name, args, lib, torch, np):
         "config": {"workload": cfg.name, "tokens": cfg.T, "hidden": cfg.H, "experts": cfg.E, "top_k": cfg.k,
                    "moe_intermediate": cfg.I, "scoring": cfg.scoring, "shared_expert": bool(cfg.shared),
                    "weights": "int4 group %d" % cfg.w4_group if cfg.w4_group >= 0 else "int8 per channel",
-                   "launch": mode, "router_gate": gate is not None, "weight_lists": args.weight_lists, "experts_touched": int((counts > 0).sum()),
-                   "rows": R},
+                   "launch": mode, "router_gate": gate is not None, "weight_lists": args.weight_lists,
+                   "experts_touched": int((counts > 0).sum()), "rows": R},
     }
     lbytes, lops = layer_bytes(cfg, counts), algorithmic_ops(cfg, R)
     out["layer_frac_of_peak"] = {"hbm": round(lbytes / (ms_per_step * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),

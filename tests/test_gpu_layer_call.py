@@ -277,8 +277,9 @@ def test_measurement_hook_brackets_the_routed_gate_up_product(name, tokens, kw):
 
 
 # every form of the call: a few tokens (their rows quantised in place; by a launch; with the shared expert), pair order
-# (a launch re-quantises; the down GEMM does, rows of one and of several loads; the shared expert in the launches), int4 in pair order and sorted, the sorted path with
-# the shared expert in line and on its side stream, per-expert weight tables
+# (a launch re-quantises; the down GEMM does, rows of one and of several loads; the shared expert in the launches), int4
+# in pair order and sorted, the sorted path with the shared expert in line and on its side stream, per-expert weight
+# tables
 _REQ = dict(H=1024, E=128, k=8)
 FORMS = [("c2_small", 2, {}), ("c2_small", 2, dict(shape=dict(H=1024, E=128, k=8, I=1408))),
          ("c4_small", 2, dict(shared=True)), ("c2_small", 24, {}), ("c2_small", 100, {}),
@@ -368,7 +369,8 @@ def test_infinities_and_nans(name, tokens, kw):
 @pytest.mark.parametrize("name, tokens, kw, where", [
     ("c2_small", 2, {}, "w13_weight_scale_fp32"), ("c2_small", 2, {}, "w2_weight_scale_fp32"),
     ("c2_small", 48, {}, "w13_weight_scale_fp32"), ("c2_small", 300, {}, "w2_weight_scale_fp32"),
-    ("c5_small", 12, {}, "w13_weight_scale"), ("c5_small", 12, {}, "w2_weight_scale"), ("c5_small", 80, {}, "w2_weight_scale"),
+    ("c5_small", 12, {}, "w13_weight_scale"), ("c5_small", 12, {}, "w2_weight_scale"),
+    ("c5_small", 80, {}, "w2_weight_scale"),
     ("c4_small", 2, dict(shared=True), "down_scale_fp32"), ("c4_small", 96, dict(shared=True), "down_scale_fp32"),
     ("c4_small", 300, dict(shared=True), "down_scale_fp32")])
 def test_misaligned_scales_are_refused(name, tokens, kw, where):

@@ -80,8 +80,7 @@ def _key(layer, x_dtype, device, logits_dtype):
     option or a part that the library has no whole form for, or a layer that is not put together as
     ``AscendRoutedExperts.__init__`` and the two schemes do it (another scheme, router or shared expert, a gate that is
     any callable, a tensor registered under the name of an attribute), or one with a method or hook of the caller's in
-    it.  Compared on every call, so plain dictionary
-    lookups: types first, then what such types have."""
+    it.  Compared on every call, so plain dictionary lookups: types first, then what such types have."""
     d = layer.__dict__
     try:
         (q, r, cfg, comm, act, on_input, expert_map, redundant, mc2_mask, pertoken, forced, log2phy, fused, pair_order,
