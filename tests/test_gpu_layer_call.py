@@ -97,6 +97,25 @@ def test_a_few_tokens_at_full_size(name, tokens):
     assert torch.equal(layer(x, logits), layer.forward_impl(x, logits).routed_out)
 
 
+# gating and quantisation inside the first launch: 1 to 4 tokens, experts that fill no register or word of four, groups,
+# scores that tie (so the lower index decides) and a row of one score, logits of every type; rows that are no multiple of
+# the 512 values a wavefront takes
+@pytest.mark.parametrize("tokens", [1, 2, 3, 4])
+@pytest.mark.parametrize("experts, k, groups, hidden", [(5, 2, 1, 64), (66, 4, 1, 576), (130, 3, 1, 1088), (256, 4, 8, 512),
+                                                        (36, 4, 4, 1024)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_gating_inside_the_first_launch(tokens, experts, k, groups, hidden, dtype):
+    shape = dict(E=experts, k=k, H=hidden, I=128, n_group=groups, topk_group=max(1, groups // 2),
+                 scoring="sigmoid" if groups > 1 else "softmax", bias=groups > 1)
+    cfg, layer, x, logits = _pair("c2_small", tokens, shape)
+    flat = logits.clone()
+    flat[-1] = 0.25
+    for lg in (logits, (logits * 2).round() / 2, flat):
+        lg = lg.to(dtype)
+        assert torch.equal(layer(x, lg), layer.forward_impl(x, lg).routed_out)
+    assert layer._layer_plan.desc is not None
+
+
 # pair order with experts of several 32-row blocks (workgroups of their own), the others idle or with a few rows
 @pytest.mark.parametrize("tokens", [32, 33, 64, 65, 200])
 @pytest.mark.parametrize("rest", [0, 7])

@@ -37,12 +37,15 @@ __device__ __forceinline__ unsigned wave_max_u32(unsigned v)
 }
 
 // Maximum of a 64-bit key over the wavefront; every lane returns it: the largest high word, and the largest low
-// word among the lanes that hold it.
+// word among the lanes that hold it.  One lane that holds it alone (scores rarely tie) is read instead.
 __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v)
 {
     const unsigned hi = (unsigned)(v >> 32);
     const unsigned m = wave_max_u32(hi);
-    const unsigned lo = wave_max_u32(hi == m ? (unsigned)v : 0u);
+    const unsigned long long holders = __ballot(hi == m);
+    unsigned lo;
+    if ((holders & (holders - 1)) == 0ull) lo = (unsigned)__builtin_amdgcn_readlane((int)v, __builtin_ctzll(holders));
+    else lo = wave_max_u32(hi == m ? (unsigned)v : 0u);
     return ((unsigned long long)m << 32) | lo;
 }
 
@@ -279,150 +282,184 @@ __device__ __forceinline__ void gate_row(const void* __restrict__ x, const void*
     }
 }
 
-// NR token rows by one wavefront at the same time: the arithmetic of gate_row for every row, with the steps of
-// the rows interleaved so that the long dependent chains of one row (wavefront reductions, the k selection
-// rounds) run in the shadow of the others'.  No workgroup barrier: what a row needs from other lanes travels by
-// lane reads, the group scores through grp_lds (NR x E floats private to the wavefront; only touched when G > 1).
-// Weights are written to `weights` in w_dtype after rounding to DT (the cast chain of the reference's caller:
-// gate output in the logits dtype, then .to(hidden dtype)); ids to idx and, when given, to idx_lds.
-template <int DT, int PER, int NR>
-__device__ __forceinline__ void gate_rows(const void* __restrict__ x, const void* __restrict__ bias,
-                                          const int (&row)[NR], const bool (&live)[NR], int E, int k, int k_group,
-                                          int G, int mode, int renorm, int norm_type, float rsf, float eps,
-                                          void* __restrict__ weights, int w_dtype, int32_t* __restrict__ idx,
-                                          float* grp_lds, int32_t* idx_lds, int lane)
+// The order of a selection score as an unsigned integer (the high word of make_key).
+__device__ __forceinline__ unsigned score_order(float score) { return (unsigned)(make_key(score, 0) >> 32); }
+
+// The scores of one token row by one wavefront, the arithmetic of gate_row without a workgroup barrier: p, the values the
+// weights come from, and sel, what the experts are chosen by (groups that are not kept at -inf).  What the row needs from
+// other lanes travels by lane reads, the group scores through grp_lds (E floats private to the wavefront; only touched
+// when G > 1).  logit(e) is the logit as fp32.
+template <int DT, int PER, typename Logit>
+__device__ __forceinline__ void row_scores(Logit logit, const void* __restrict__ bias, int E, int k_group, int G, int mode,
+                                           int norm_type, float* grp_lds, int lane, float (&p)[PER], float (&sel)[PER])
 {
-    float p[NR][PER], sel[NR][PER];
+    float m = -__builtin_inff();
 #pragma unroll
-    for (int r = 0; r < NR; ++r) {
-        float m = -__builtin_inff();
+    for (int i = 0; i < PER; ++i) {
+        const int e = lane + 64 * i;
+        p[i] = (e < E) ? logit(e) : -__builtin_inff();
+        m = p[i] > m ? p[i] : m;
+    }
+    if (norm_type == 0) {
+        m = wave_max_dpp(m);
+        float part = 0.0f;
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
-            const int e = lane + 64 * i;
-            p[r][i] = (e < E) ? load_as_f32<DT>(x, (int64_t)row[r] * E + e) : -__builtin_inff();
-            m = p[r][i] > m ? p[r][i] : m;
-        }
-        if (norm_type == 0) {
-            m = wave_max_dpp(m);
-            float part = 0.0f;
-#pragma unroll
-            for (int i = 0; i < PER; ++i) {
-                if (lane + 64 * i < E) {
-                    p[r][i] = m_expf(p[r][i] - m);
-                    part = part + p[r][i];
-                }
+            if (lane + 64 * i < E) {
+                p[i] = m_expf(p[i] - m);
+                part = part + p[i];
             }
-            const float inv = 1.0f / wave_tree_sum(part);
-#pragma unroll
-            for (int i = 0; i < PER; ++i) p[r][i] = p[r][i] * inv;
-        } else {
-#pragma unroll
-            for (int i = 0; i < PER; ++i) p[r][i] = 1.0f / (1.0f + m_expf(-p[r][i]));
         }
+        const float inv = 1.0f / wave_tree_sum(part);
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int e = lane + 64 * i;
-            if (e < E) sel[r][i] = bias ? p[r][i] + load_as_f32<DT>(bias, e) : p[r][i];
-            else sel[r][i] = -__builtin_inff();
-        }
+        for (int i = 0; i < PER; ++i) p[i] = p[i] * inv;
+    } else {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) p[i] = 1.0f / (1.0f + m_expf(-p[i]));
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int e = lane + 64 * i;
+        if (e < E) sel[i] = bias ? p[i] + load_as_f32<DT>(bias, e) : p[i];
+        else sel[i] = -__builtin_inff();
     }
     if (G > 1) {
         const int gs = E / G;
 #pragma unroll
-        for (int r = 0; r < NR; ++r)
-#pragma unroll
-            for (int i = 0; i < PER; ++i)
-                if (lane + 64 * i < E) grp_lds[r * E + lane + 64 * i] = sel[r][i];
+        for (int i = 0; i < PER; ++i)
+            if (lane + 64 * i < E) grp_lds[lane + 64 * i] = sel[i];
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        unsigned long long gkey[NR];
-#pragma unroll
-        for (int r = 0; r < NR; ++r) {
-            gkey[r] = 0ull;
-            if (butterfly_groups<PER>(sel[r], gs)) {
-                const float sc = group_scores_butterfly<PER>(sel[r], gs, mode, lane);
-                if (lane < G) gkey[r] = make_key(sc, lane);
-            } else if (lane < G) {
-                gkey[r] = make_key(group_score(grp_lds + r * E + lane * gs, gs, mode), lane);
-            }
+        unsigned gu = 0u;
+        if (butterfly_groups<PER>(sel, gs)) gu = score_order(group_scores_butterfly<PER>(sel, gs, mode, lane));
+        else if (lane < G) gu = score_order(group_score(grp_lds + lane * gs, gs, mode));
+        // a group stays if fewer than k_group others come before it
+        int before = 0;
+        for (int g = 0; g < G; ++g) {
+            const unsigned v = (unsigned)__builtin_amdgcn_readlane((int)gu, g);
+            before += (v > gu || (v == gu && g < lane)) ? 1 : 0;
         }
-        unsigned long long keep[NR];
+        const unsigned long long keep = __ballot(lane < G && before < k_group);
 #pragma unroll
-        for (int r = 0; r < NR; ++r) keep[r] = 0ull;
-        for (int c = 0; c < k_group; ++c) {
-#pragma unroll
-            for (int r = 0; r < NR; ++r) {
-                const int g = key_index(wave_max_u64(gkey[r]));
-                keep[r] |= 1ull << g;
-                if (lane == g) gkey[r] = 0ull;
-            }
+        for (int i = 0; i < PER; ++i) {
+            const int e = lane + 64 * i;
+            if (e < E && !((keep >> (e / gs)) & 1ull)) sel[i] = -__builtin_inff();
         }
-#pragma unroll
-        for (int r = 0; r < NR; ++r)
-#pragma unroll
-            for (int i = 0; i < PER; ++i) {
-                const int e = lane + 64 * i;
-                if (e < E && !((keep[r] >> (e / gs)) & 1ull)) sel[r][i] = -__builtin_inff();
-            }
     }
-    // ---- top-k over the (masked) selection scores; the weight of a chosen expert is its unbiased score
-    unsigned long long key[NR][PER];
-#pragma unroll
-    for (int r = 0; r < NR; ++r)
-#pragma unroll
-        for (int i = 0; i < PER; ++i) key[r][i] = (lane + 64 * i < E) ? make_key(sel[r][i], lane + 64 * i) : 0ull;
-    int my_i[NR];
-    float my_p[NR];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-        my_i[r] = 0;
-        my_p[r] = 0.0f;
+}
+
+// The chosen experts of a row, in order, and their weights: lane c (< k) holds the c-th, my_p its unnormalised value.
+// Weights are written to weights[o ..] in w_dtype after rounding to DT (the cast chain of the reference's caller: gate
+// output in the logits dtype, then .to(hidden dtype)) and ids to idx[o ..].
+template <int DT>
+__device__ __forceinline__ void store_choice(int my_i, float my_p, int k, int renorm, int norm_type, float rsf, float eps,
+                                             int64_t o, void* __restrict__ weights, int w_dtype,
+                                             int32_t* __restrict__ idx, int lane)
+{
+    if (norm_type == 1 || renorm == 1) {
+        float wsum = 0.0f;
+        for (int c = 0; c < k; ++c) wsum = wsum + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_p), c));
+        const float d = wsum + eps;
+        my_p = my_p / d;
     }
+    my_p = my_p * rsf;
+    if (lane >= k) return;
+    // a store that is visible to the whole device when it completes (a workgroup on another part of the chip may be the
+    // one that sorts the pairs)
+    __hip_atomic_store(idx + o + lane, my_i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    float stored = my_p;
+    if constexpr (DT == MOE355_DT_BF16) stored = bf16_to_f32(f32_to_bf16(stored));
+    if constexpr (DT == MOE355_DT_F16) stored = f16_to_f32(f32_to_f16(stored));
+    if (w_dtype == MOE355_DT_BF16) ((uint16_t*)weights)[o + lane] = f32_to_bf16(stored);
+    else if (w_dtype == MOE355_DT_F16) ((uint16_t*)weights)[o + lane] = f32_to_f16(stored);
+    else ((float*)weights)[o + lane] = stored;
+}
+
+// One token row by one wavefront.
+template <int DT, int PER, typename Logit>
+__device__ __forceinline__ void gate_row_wave(Logit logit, const void* __restrict__ bias, int E, int k, int k_group,
+                                              int G, int mode, int renorm, int norm_type, float rsf, float eps,
+                                              int64_t o, void* __restrict__ weights, int w_dtype,
+                                              int32_t* __restrict__ idx, float* grp_lds, int lane)
+{
+    float p[PER], sel[PER];
+    row_scores<DT, PER>(logit, bias, E, k_group, G, mode, norm_type, grp_lds, lane, p, sel);
+    unsigned long long key[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) key[i] = (lane + 64 * i < E) ? make_key(sel[i], lane + 64 * i) : 0ull;
+    int my_i = 0;
+    float my_p = 0.0f;
     for (int c = 0; c < k; ++c) {
+        unsigned long long best = 0ull;
 #pragma unroll
-        for (int r = 0; r < NR; ++r) {
-            unsigned long long best = 0ull;
+        for (int i = 0; i < PER; ++i) best = key[i] > best ? key[i] : best;
+        const int win = key_index(wave_max_u64(best));
+        float cand = 0.0f;
 #pragma unroll
-            for (int i = 0; i < PER; ++i) best = key[r][i] > best ? key[r][i] : best;
-            const int win = key_index(wave_max_u64(best));
-            float cand = 0.0f;
+        for (int i = 0; i < PER; ++i) {
+            if (i == (win >> 6)) {
+                cand = p[i];
+                if ((win & 63) == lane) key[i] = 0ull;
+            }
+        }
+        const float pw = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cand), win & 63));
+        if (lane == c) {
+            my_i = win;
+            my_p = pw;
+        }
+    }
+    store_choice<DT>(my_i, my_p, k, renorm, norm_type, rsf, eps, o, weights, w_dtype, idx, lane);
+}
+
+// The ranks of one token row's experts by W wavefronts of a workgroup.  The k rounds of a maximum over the wavefront are a
+// chain of about 430 cycles each: eight of them 1.5 us of one token's call, with everything else waiting (a bound for the
+// k-th best by bisection of the bits takes as long).  Here one wavefront leaves the order of the scores in LDS, and every
+// wavefront counts, for all experts, how many of its share of the experts come before them (larger score, then lower
+// index); the counts add up to the ranks.  orders [E rounded up to 4]: score_order of every expert, at least 1; ranks [E]:
+// zeroes.
+template <int PER>
+__device__ __forceinline__ void rank_row(const unsigned* orders, int E, int w, int W, int* ranks, int lane)
+{
+    unsigned u[PER];
+    int count[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        u[i] = lane + 64 * i < E ? orders[lane + 64 * i] : 0xffffffffu;
+        count[i] = 0;
+    }
+    const int quads = (E + 3) >> 2, q0 = quads * w / W, q1 = quads * (w + 1) / W;
+    for (int qd = q0; qd < q1; ++qd) {
+        const uint4 four = *(const uint4*)(orders + 4 * qd);
+        const unsigned v[4] = {four.x, four.y, four.z, four.w};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int from = 4 * qd + c;
+            if (from >= E) break;
 #pragma unroll
             for (int i = 0; i < PER; ++i) {
-                if (i == (win >> 6)) {
-                    cand = p[r][i];
-                    if ((win & 63) == lane) key[r][i] = 0ull;
-                }
-            }
-            const float pw = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cand), win & 63));
-            if (lane == c) {
-                my_i[r] = win;
-                my_p[r] = pw;
+                // at the same score the lower index comes first: v >= u there, which is v > u - 1 (no order is 0)
+                count[i] += v[c] > u[i] - (from < lane + 64 * i ? 1u : 0u) ? 1 : 0;
             }
         }
     }
 #pragma unroll
-    for (int r = 0; r < NR; ++r) {
-        if (norm_type == 1 || renorm == 1) {
-            float wsum = 0.0f;
-            for (int c = 0; c < k; ++c)
-                wsum = wsum + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_p[r]), c));
-            const float d = wsum + eps;
-            my_p[r] = my_p[r] / d;
-        }
-        my_p[r] = my_p[r] * rsf;
-        if (idx_lds && live[r] && lane < k) idx_lds[row[r] * k + lane] = my_i[r];
-        if (live[r] && lane < k) {
-            // a store that is visible to the whole device when it completes (a workgroup on another part of the
-            // chip may be the one that sorts the pairs)
-            __hip_atomic_store(idx + (int64_t)row[r] * k + lane, my_i[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            float stored = my_p[r];
-            if constexpr (DT == MOE355_DT_BF16) stored = bf16_to_f32(f32_to_bf16(stored));
-            if constexpr (DT == MOE355_DT_F16) stored = f16_to_f32(f32_to_f16(stored));
-            const int64_t o = (int64_t)row[r] * k + lane;
-            if (w_dtype == MOE355_DT_BF16) ((uint16_t*)weights)[o] = f32_to_bf16(stored);
-            else if (w_dtype == MOE355_DT_F16) ((uint16_t*)weights)[o] = f32_to_f16(stored);
-            else ((float*)weights)[o] = stored;
+    for (int i = 0; i < PER; ++i)
+        if (lane + 64 * i < E) atomicAdd(ranks + lane + 64 * i, count[i]);
+}
+
+// the k first of the ranked experts into idx_lds (and their values into p_lds), in order
+template <int PER>
+__device__ __forceinline__ void place_row(const float (&p)[PER], const int* ranks, int E, int k, int* idx_lds, float* p_lds,
+                                          int lane)
+{
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int e = lane + 64 * i;
+        const int r = e < E ? ranks[e] : k;
+        if (r < k) {
+            idx_lds[r] = e;
+            p_lds[r] = p[i];
         }
     }
 }

@@ -264,7 +264,7 @@ struct ForkJoinLease {
 // dense W8A8 MLP over all tokens, on the rows the routed experts quantised
 int shared_expert(const moe355_layer& l, const Forms& f, const Buffers& b, int64_t T, void* st)
 {
-    if (f.shared_few) return few_forward(shared_args(l, b, T), (hipStream_t)st);
+    if (f.shared_few) return few_forward(shared_args(l, b, T), nullptr, (hipStream_t)st);
     const int64_t H = l.hidden, I = l.shared_intermediate;
     int rc = moe355_gmm_i32(b.xq, l.shared_w13, b.one_group, MOE355_GL_CUMSUM, T, H, 2 * I, 1, b.sh_acc, b.sh_ws,
                             b.sh_bytes, st);
@@ -382,15 +382,21 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
         g.logits = b.logits;
         g.logits_dtype = MOE355_DT_F32;
     }
-    rc = gate_quant_impl(f.small, g, 1, b.topk_weights, b.topk_ids, b.xq, b.x_scale, b.dst, b.row_token,
-                         b.expert_tokens, l.sync_counter, l.shared ? b.one_group : nullptr, stream);
-    if (rc != MOE355_OK) return rc;
+    FewArgs few = {};
+    if (f.few) {
+        few = few_args(l, b, T);
+        few.out = (uint16_t*)out;
+    }
+    const bool gates_itself = f.few && few_gates(few, g);
+    if (!gates_itself) {
+        rc = gate_quant_impl(f.small, g, 1, b.topk_weights, b.topk_ids, b.xq, b.x_scale, b.dst, b.row_token,
+                             b.expert_tokens, l.sync_counter, l.shared ? b.one_group : nullptr, stream);
+        if (rc != MOE355_OK) return rc;
+    }
     if (f.few) {
         // the shared expert rides in the same two launches, whatever stream it was meant for
         (void)moe355_profile_next_gemm(ev0, ev1);
-        FewArgs a = few_args(l, b, T);
-        a.out = (uint16_t*)out;
-        return few_forward(a, (hipStream_t)stream);
+        return few_forward(few, gates_itself ? &g : nullptr, (hipStream_t)stream);
     }
 
     ForkJoinLease lease;

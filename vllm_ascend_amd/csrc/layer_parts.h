@@ -18,6 +18,9 @@ struct GateCall {
     float routed_scaling_factor, eps;
 };
 
+// what the gating launches take of such a call, and what they refuse (num_tokens > 0)
+int check_gate(const GateCall& g);
+
 // sort: the whole of moe355_route_quant_small; otherwise gating and quantisation only (any number of tokens).
 // one_group: receives num_tokens on the device, or null.
 int gate_quant_impl(bool sort, const GateCall& g, int tokens_num_type, void* topk_weights, int32_t* topk_ids,
@@ -96,6 +99,14 @@ int route_map_impl(const int32_t* expert_idx, int64_t num_tokens, int top_k, int
                    size_t workspace_bytes, const TileSpec* specs, int nspecs, bool* built, void* stream);
 
 // ------------------------------------------------------------------ a few tokens (few.hip)
+// n / d for n and d below 2^16 in one multiplication (an integer division is about 25 instructions, one after the other)
+struct SmallDivisor {
+    uint32_t m = 0;
+    SmallDivisor() = default;
+    explicit SmallDivisor(uint32_t d) : m(d > 1 ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0) {}
+    __device__ int operator()(int n) const { return m ? (int)__umulhi((uint32_t)n, m) : n; }
+};
+
 struct FewArgs {
     const int8_t* xq;        // [T, H]
     const float* x_scale;    // [T]
@@ -119,9 +130,14 @@ struct FewArgs {
     uint16_t* out;           // [T, H]
     int f16;
     int64_t* load;           // [E] or null: the rows of every expert are added
+    // divisions by k, I / 4, I / 16, S / 4, S / 16 and the items of an expert's K range (few_forward)
+    SmallDivisor by_k, by_i4, by_i16, by_s4, by_s16, by_parts;
 };
 
 bool few_supported(const FewArgs& a);
-int few_forward(const FewArgs& a, hipStream_t st);
+// whether few_forward takes the gating and the token quantisation of such a call as well
+bool few_gates(const FewArgs& a, const GateCall& g);
+// gate: the call that few_forward gates and quantises for itself (ids and weights go to a.ids and a.tw), or null
+int few_forward(const FewArgs& a, const GateCall* gate, hipStream_t st);
 
 }  // namespace moe355

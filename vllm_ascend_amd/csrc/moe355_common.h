@@ -177,12 +177,22 @@ __device__ __forceinline__ float wave_max(float v)
     return v;
 }
 
-// Butterfly sum: after the loop every lane holds the same value; the order of
-// additions is part of the arithmetic contract (partial[l] + partial[l ^ off]).
+// Butterfly sum: every lane receives the same value; the order of additions is part of the arithmetic contract
+// (partial[l] + partial[l ^ off], off = 32 .. 1).  No LDS round trips: halves and rows change places by the lane swaps,
+// lane l ^ 8 is row_ror:8, and for off = 4 row_ror:4 names lane l ^ 4 or l ^ 12, which hold the same value by then.
 __device__ __forceinline__ float wave_tree_sum(float v)
 {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v = v + __shfl_xor(v, off, 64);
+    typedef unsigned v2u __attribute__((ext_vector_type(2)));
+    v2u s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+    s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+#define MOE355_STEP(ctrl) v = v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xf, 0xf, true));
+    MOE355_STEP(0x128)  // row_ror:8
+    MOE355_STEP(0x124)  // row_ror:4
+    MOE355_STEP(0x4e)   // quad_perm 2 3 0 1
+    MOE355_STEP(0xb1)   // quad_perm 1 0 3 2
+#undef MOE355_STEP
     return v;
 }
 

@@ -148,11 +148,11 @@ __global__ __launch_bounds__(kSmallThreads) void route_quant_small_kernel(SmallR
     if (a.one_group && blockIdx.x == 0 && tid == 0) *a.one_group = a.T;
     // ---------------- gating: one row per wavefront
     {
-        int row[1] = {(int)blockIdx.x * kSmallWaves + wave};
-        bool live[1] = {row[0] < a.T};
-        if (!live[0]) row[0] = a.T - 1;
-        gate_rows<LDT, PER, 1>(a.logits, a.bias, row, live, E, k, a.k_group, a.G, a.mode, a.renorm, a.norm_type, a.rsf,
-                               a.eps, a.topk_weights, a.x_dtype, a.topk_ids, lds + (size_t)wave * E, nullptr, lane);
+        const int row = (int)blockIdx.x * kSmallWaves + wave;
+        if (row < a.T)
+            gate_row_wave<LDT, PER>([&](int e) { return load_as_f32<LDT>(a.logits, (int64_t)row * E + e); }, a.bias, E, k,
+                                    a.k_group, a.G, a.mode, a.renorm, a.norm_type, a.rsf, a.eps, (int64_t)row * k,
+                                    a.topk_weights, a.x_dtype, a.topk_ids, lds + (size_t)wave * E, lane);
     }
     if (!a.arrived) return;  // gating and quantisation only (moe355_gate_quant): the maps come from another launch
     // This workgroup's ids have reached memory before it is counted: every thread waits for its own stores, the
@@ -253,6 +253,22 @@ extern "C" int moe355_route_quant_small_supported(int64_t num_tokens, int top_k,
            num_experts <= kSmallMaxExperts && top_k <= num_experts;
 }
 
+int moe355::check_gate(const GateCall& g)
+{
+    if (g.num_tokens < 0 || g.hidden <= 0 || g.num_experts <= 0 || g.top_k <= 0) return MOE355_E_ARG;
+    if (g.norm_type != 0 && g.norm_type != 1) return MOE355_E_ARG;
+    if (g.group_select_mode != 0 && g.group_select_mode != 1) return MOE355_E_ARG;
+    if (g.group_count <= 0 || g.k_group <= 0 || g.k_group > g.group_count) return MOE355_E_ARG;
+    if (g.x_dtype != MOE355_DT_BF16 && g.x_dtype != MOE355_DT_F16) return MOE355_E_UNSUPPORTED;
+    if (g.logits_dtype < MOE355_DT_F32 || g.logits_dtype > MOE355_DT_F16) return MOE355_E_ARG;
+    if (g.num_tokens == 0) return MOE355_OK;
+    if (!moe355_gate_quant_supported(g.num_tokens, g.top_k, g.num_experts)) return MOE355_E_SHAPE;
+    if (g.group_count > 64 || g.num_experts % g.group_count != 0) return MOE355_E_SHAPE;
+    if (g.hidden % 8 != 0 || ((uintptr_t)g.x & 15)) return MOE355_E_SHAPE;
+    if (!g.x || !g.logits) return MOE355_E_ARG;
+    return MOE355_OK;
+}
+
 int moe355::gate_quant_impl(bool sort, const GateCall& g, int tokens_num_type, void* topk_weights, int32_t* topk_ids,
                             int8_t* xq, float* x_scale, int32_t* expanded_row_idx, int32_t* row_token,
                             int64_t* expert_tokens, int32_t* sync_counter, int64_t* one_group, void* stream)
@@ -262,19 +278,12 @@ int moe355::gate_quant_impl(bool sort, const GateCall& g, int tokens_num_type, v
     const int k_group = g.k_group, group_count = g.group_count, group_select_mode = g.group_select_mode;
     const int renorm = g.renorm, norm_type = g.norm_type;
     const int64_t num_tokens = g.num_tokens, hidden = g.hidden;
-    if (num_tokens < 0 || hidden <= 0 || num_experts <= 0 || k <= 0) return MOE355_E_ARG;
-    if (norm_type != 0 && norm_type != 1) return MOE355_E_ARG;
-    if (group_select_mode != 0 && group_select_mode != 1) return MOE355_E_ARG;
-    if (group_count <= 0 || k_group <= 0 || k_group > group_count) return MOE355_E_ARG;
     if (tokens_num_type != 0 && tokens_num_type != 1) return MOE355_E_UNSUPPORTED;
-    if (x_dtype != MOE355_DT_BF16 && x_dtype != MOE355_DT_F16) return MOE355_E_UNSUPPORTED;
-    if (logits_dtype < MOE355_DT_F32 || logits_dtype > MOE355_DT_F16) return MOE355_E_ARG;
-    if (num_tokens == 0) return MOE355_OK;
+    int rc = check_gate(g);
+    if (rc != MOE355_OK || num_tokens == 0) return rc;
     if (sort && !moe355_route_quant_small_supported(num_tokens, k, num_experts)) return MOE355_E_SHAPE;
-    if (!sort && !moe355_gate_quant_supported(num_tokens, k, num_experts)) return MOE355_E_SHAPE;
-    if (group_count > 64 || num_experts % group_count != 0) return MOE355_E_SHAPE;
-    if (hidden % 8 != 0 || ((uintptr_t)x & 15) || ((uintptr_t)xq & 7)) return MOE355_E_SHAPE;
-    if (!x || !logits || !topk_weights || !topk_ids || !xq || !x_scale) return MOE355_E_ARG;
+    if ((uintptr_t)xq & 7) return MOE355_E_SHAPE;
+    if (!topk_weights || !topk_ids || !xq || !x_scale) return MOE355_E_ARG;
     if (sort && (!expanded_row_idx || !row_token || !expert_tokens || !sync_counter)) return MOE355_E_ARG;
     SmallRouteArgs a = {};
     a.x = x;
