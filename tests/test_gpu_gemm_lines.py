@@ -1,4 +1,4 @@
-"""The grouped GEMMs on both sides of the lines between streaming and the tiles: 1023 / 1024 rows for a small product,
+"""The GEMMs on both sides of the lines between their families: streaming and the tiles at 1023 / 1024 rows for a small product,
 fewer rows than experts / one row per expert for one of a GiB and more, 63 / 64 rows per expert at a long K."""
 import numpy as np
 import pytest
@@ -88,3 +88,44 @@ def test_token_rows_quantised_beside_the_gating(T, H, dtype):
     xq, xs = K.dynamic_quant(x)
     torch.cuda.synchronize()
     assert torch.equal(got[2], xq) and torch.equal(got[3].view(torch.int32), xs.view(torch.int32))
+
+# A dense product (one expert) on both sides of the lines around the tiles that cut K over their wavefronts: 64 / 65 rows, as
+# many 128-row tiles as half the compute units, a last tile of one row, a last row of tiles of one and of 64; more K steps
+# than wavefronts, fewer (a wavefront without any), and numbers of them that leave every remainder of the register ring
+SPLIT_LINES = [(64, 256, 256, "stream"), (65, 256, 256, "split"), (128, 64, 64, "split"), (129, 192, 576, "split"),
+               (200, 1408, 320, "split"), (191, 832, 128, "split"), (1000, 512, 3840, "split"), (1024, 128, 4096, "tiled")]
+
+
+@pytest.mark.parametrize("R,Kd,N,family", SPLIT_LINES)
+def test_dense_product_with_k_cut_over_the_wavefronts(R, Kd, N, family):
+    from oracle import oracle as orc
+    from vllm_ascend_amd import kernels as K
+    from vllm_ascend_amd._lib import W_ENK, load
+
+    print(f"dense line R={R} K={Kd} N={N} {family}", flush=True)
+    assert load().moe355_gmm_kernel_name(2, R, Kd, N, 1).decode() == f"gmm_{family}_kernel"
+    g = torch.Generator().manual_seed(R)
+    x = torch.randint(-128, 128, (R, Kd), generator=g, dtype=torch.int8)
+    w = torch.randint(-128, 128, (1, N, Kd), generator=g, dtype=torch.int8)
+    sw = torch.rand(1, N, generator=g) * 0.009 + 0.001
+    sx = torch.rand(R, generator=g) * 0.05 + 0.001
+    wnz = K.format_cast_nz(w.to("cuda"), W_ENK)
+    for rows in (R, R - 1, R // 2):  # the group may hold fewer rows than the buffer
+        cum = torch.tensor([rows], dtype=torch.int64)
+        ref = orc.gmm_i32(x.numpy(), w.numpy(), cum.numpy())
+        acc = K.gmm_i32(x.to("cuda"), wnz, cum.to("cuda"), 0, N, Kd)
+        got = K.gmm2_dequant(x.to("cuda"), wnz, sw.to("cuda"), sx.to("cuda"), cum.to("cuda"), 0, N, Kd)
+        q, s = K.gmm1_swiglu_quant(x.to("cuda"), wnz, sw.to("cuda"), sx.to("cuda"), cum.to("cuda"), 0, N, Kd)
+        torch.cuda.synchronize()
+        assert np.array_equal(acc.cpu().numpy()[:rows], ref[:rows])
+        want = orc.gmm2_dequant(ref, sx.numpy(), sw.numpy(), cum.numpy())
+        assert np.array_equal(got.cpu().contiguous().view(torch.int16).numpy().view(np.uint16)[:rows], want[:rows])
+        q_want, s_want = orc.swiglu_quant(orc.dequant_acc(ref, sx.numpy(), sw.numpy(), cum.numpy()))
+        assert np.array_equal(q.cpu().numpy()[:rows], q_want[:rows])
+        assert np.array_equal(s.cpu().numpy().view(np.uint32)[:rows], s_want.view(np.uint32)[:rows])
+
+
+# few experts: 64-row tiles as long as they do not outnumber the compute units, on both sides of the line
+@pytest.mark.parametrize("R,E,Kd,N", [(1024, 8, 192, 1024), (3904, 8, 64, 1024), (3968, 8, 64, 1024), (1030, 3, 128, 2816)])
+def test_tiles_of_half_the_height_for_few_experts(R, E, Kd, N):
+    test_families_on_both_sides_of_a_line(R, E, Kd, N, "tiled", True)

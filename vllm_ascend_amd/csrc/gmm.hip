@@ -591,6 +591,8 @@ static void launch_gemm(KernelT kernel, dim3 grid, hipStream_t st, const GmmArgs
 // tiles (up to 256 rows) that fetch an expert's weights once.  The host only knows the mean, and the histogram may be
 // skewed (real routers are): the 128-row tiles cost a cold expert little more than streaming does (a short tile that
 // is its expert's only one reads its weights once, past the caches) and a hot one a fraction of it, so they start early.
+constexpr int64_t kComputeUnits = 256;
+
 static int tiled_bm(const GmmArgs& a)
 {
     if (a.K % 64 != 0) return 0;
@@ -618,6 +620,12 @@ static int tiled_bm(const GmmArgs& a)
     //     153 / 183 against 80 / 88: tiles.
     if (a.R < a.E) return 0;
     if (avg < 48 && a.R < 1024 && (a.R < 128 || weights < (1ll << 30))) return 0;
+    // Few experts and few rows: as long as tiles of half the height do not outnumber the compute units they are twice as
+    // many and half as long (rows / 64 and half a tile per expert for its last one).  8 experts of 2816 x 1024 and 1024 x
+    // 1408, the layer at 512 / 768 / 1024 / 1536 tokens of two slots 50.8 / 51.5 / 52.5 / 62.6 us on 128-row tiles, 41.7 /
+    // 46.5 / 49.1 / 59.9 with this rule (2048 tokens, where it would be one tile too many for the down product: 65.8
+    // against 67.2).  Products of up to 512 channels, a handful of workgroups in any family, were not measured and stay.
+    if (a.E > 1 && a.N > 512 && (a.R / 64 + a.E / 2) * ((a.N + 255) / 256) <= kComputeUnits) return 64;
     // the list of 256-row tiles is built from 16-bit counters (tile_map_kernel, by_length)
     const bool wide_ok = a.R / 256 + a.E < 32768;
     // K = 7168 / 2048, uniform routing, 28 / 40 / 48 / 56 / 64 / 94 rows per expert: the layer takes 1968 / 2028 / 2055 /
@@ -625,9 +633,15 @@ static int tiled_bm(const GmmArgs& a)
     // us on 128-row tiles; Zipf(1.1) at 28 / 40 / 64 / 94 / 128 1115 / 1361 / 1703 / 2164 / 2616 against 1069 / 1339 /
     // 1667 / 2155 / 2648.  128 experts at K = 4096, 56 / 69 / 81 rows: 526 / 547 / 567 against 511 / 552 / 576.
     if (avg >= 64 && avg <= 256 && a.K >= 4096 && wide_ok) return 256;
-    // around 128 rows per expert most experts fit one wide tile of 128 or 160 rows and fetch their weights once,
-    // which pays from K = 1024 on (measured: 6 % at K = 2048 and 1024, a loss at K = 768 and at 64 rows)
-    if (avg >= 96 && avg <= 192 && a.K >= 1024 && wide_ok) return 256;
+    // Around 128 rows per expert most experts fit one wide tile of 128 or 160 rows and fetch their weights once, which
+    // pays from K = 1024 on if the experts are about equally popular and there are enough of them to fill the chip.  128
+    // experts, K = 2048 / 768, the layer at 100 / 112 / 128 / 144 / 160 / 192 rows per expert: 201 / 210 / 224 / 241 / 260 /
+    // 280 us with the wide tiles in the first product, 193 / 212 / 232 / 250 / 253 / 264 us on 128-row tiles; Zipf(1.1) at
+    // 96 / 128 / 192 219 / 254 / 322 against 187 / 213 / 268, so no further than they win.
+    // (Products of up to 512 channels keep the range that was measured for them, 96 to 192.)
+    const bool narrow = a.N <= 512;
+    const bool fills = narrow || (int64_t)a.E * ((a.N + 511) / 512) >= kComputeUnits;
+    if (avg >= (narrow ? 96 : 112) && avg <= (narrow ? 192 : 144) && a.K >= 1024 && wide_ok && fills) return 256;
     return 128;
 }
 
@@ -652,6 +666,17 @@ static bool dense_tiles(const GmmArgs& a)
     if (force && force[0]) return false;
 #endif
     return ((a.R + 255) / 256) * ((int64_t)(a.N + 255) / 256) >= 192;
+}
+
+// One expert with more rows than the streaming kernel takes in slabs, and 128-row tiles for less than half of the compute
+// units (the shared expert of a mixed batch): the 64 x 64 tiles that cut K over their wavefronts.  256 experts of the
+// DeepSeek-V3 shape with the shared expert in line, 128 / 192 / 256 / 512 / 1024 tokens 1767 / 1843 / 1882 / 1848 / 1964 us on
+// 128-row tiles, 1660 / 1697 / 1738 / 1828 / 1974 on these.  On a side stream the few workgroups of the 128-row tiles hide
+// behind the routed products and these do not: 100 / 200 / 400 tokens 1609 / 1712 / 1797 against 1620 / 1738 / 1813.
+static bool split_tiles(const GmmArgs& a)
+{
+    if (a.E != 1 || a.beside || a.K % 64 != 0 || a.R <= 64 || a.R * (int64_t)a.K >= (1ll << 31) || dense_tiles(a)) return false;
+    return ((a.R + 127) / 128) * ((a.N + 255) / 256) < kComputeUnits / 2;
 }
 
 static size_t tiled_ws_max(int64_t rows, int E)
@@ -679,7 +704,7 @@ int gemm_tile_specs(int64_t rows, int64_t k, int64_t n, int num_experts, void* t
     a.K = (int)k;
     a.N = (int)n;
     a.E = num_experts;
-    const int bm = dense_tiles(a) ? 0 : gemm_family(a, true);
+    const int bm = dense_tiles(a) || split_tiles(a) ? 0 : gemm_family(a, true);
     if (bm) specs[0] = tile_spec(rows, num_experts, bm, tile_ws);
     return bm ? 1 : 0;
 }
@@ -700,6 +725,10 @@ static int launch_gemm_auto(const GmmArgs& a_in, void* tile_ws, hipStream_t st, 
     t_ev_stop = nullptr;
     if (dense_tiles(a)) {
         return launched(launch_dense(EPI, a, st, ev0, ev1));
+    }
+    if (split_tiles(a)) {
+        launch_split(EPI, a, st, ev0, ev1);
+        return launch_status();
     }
     const int bm = gemm_family(a, tile_ws != nullptr);
     if (bm) return launched(launch_tiled_any(EPI, bm, a, tile_ws, st, ev0, ev1));
@@ -767,6 +796,7 @@ extern "C" const char* moe355_gmm_kernel_name(int epilogue, int64_t rows, int64_
     a.N = (int)n;
     a.E = num_experts;
     if (dense_tiles(a)) return "gmm_dense_kernel";
+    if (split_tiles(a)) return "gmm_split_kernel";
     const int bm = gemm_family(a, true);  // as launch_gemm_auto decides
     return bm == 256 ? "gmm_wide_kernel" : bm ? "gmm_tiled_kernel" : "gmm_stream_kernel";
 }
@@ -791,9 +821,9 @@ extern "C" int moe355_format_cast_nz(const int8_t* w, int layout, int64_t num_ex
     return launch_status();
 }
 
-extern "C" int moe355_gmm_i32(const int8_t* x, const int8_t* weight_nz, const int64_t* group_list,
-                              int group_list_type, int64_t rows, int64_t k, int64_t n, int num_experts, int32_t* acc,
-                              void* workspace, size_t workspace_bytes, void* stream)
+int moe355::gmm_i32_impl(const int8_t* x, const int8_t* weight_nz, const int64_t* group_list, int group_list_type,
+                         int64_t rows, int64_t k, int64_t n, int num_experts, int32_t* acc, void* workspace,
+                         size_t workspace_bytes, void* stream, bool beside)
 {
     int rc = check_gmm(x, weight_nz, group_list, group_list_type, rows, k, n, num_experts);
     if (rc != MOE355_OK) return rc;
@@ -815,7 +845,16 @@ extern "C" int moe355_gmm_i32(const int8_t* x, const int8_t* weight_nz, const in
     a.N = (int)n;
     a.E = num_experts;
     a.acc = acc;
+    a.beside = beside;
     return launch_gemm_auto<EPI_I32>(a, tile_ws, (hipStream_t)stream, part_ws, part_bytes);
+}
+
+extern "C" int moe355_gmm_i32(const int8_t* x, const int8_t* weight_nz, const int64_t* group_list,
+                              int group_list_type, int64_t rows, int64_t k, int64_t n, int num_experts, int32_t* acc,
+                              void* workspace, size_t workspace_bytes, void* stream)
+{
+    return gmm_i32_impl(x, weight_nz, group_list, group_list_type, rows, k, n, num_experts, acc, workspace,
+                        workspace_bytes, stream, false);
 }
 
 extern "C" size_t moe355_gmm_i32_workspace(int64_t rows, int64_t n, int64_t k, int num_experts)
@@ -926,7 +965,7 @@ extern "C" size_t moe355_gmm2_dequant_workspace(int64_t rows, int64_t n, int64_t
 int moe355::gmm2_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list, const float* scale,
                       const float* const* scale_list, const float* per_token_scale, const int64_t* group_list,
                       int group_list_type, int64_t rows, int64_t k, int64_t n, int num_experts, void* out,
-                      int out_dtype, void* workspace, size_t workspace_bytes, void* stream, bool tiles_ready)
+                      int out_dtype, void* workspace, size_t workspace_bytes, void* stream, bool tiles_ready, bool beside)
 {
     const void* wany = weight_list ? (const void*)weight_list : (const void*)weight_nz;
     int rc = check_gmm(x, wany, group_list, group_list_type, rows, k, n, num_experts);
@@ -954,6 +993,7 @@ int moe355::gmm2_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* co
     a.out = (uint16_t*)out;
     a.out_f16 = out_dtype == MOE355_DT_F16;
     a.tiles_ready = tiles_ready;
+    a.beside = beside;
     return launch_gemm_auto<EPI_DEQUANT>(a, workspace, (hipStream_t)stream);
 }
 

@@ -55,6 +55,7 @@ struct GmmArgs {
     // pair order, down GEMM with the re-quantisation inside (REQ): the SwiGLU values [R, K] fp32 that the gate_up
     // GEMM wrote; the workgroup quantises the rows of its expert itself (x and row_scale are not read)
     const float* y_in;
+    int beside;             // dense product on a side stream: few workgroups that hide, not many that finish early
     float limit;            // swiglu clamp
     int tiles_ready;        // the tile maps of this call are in its workspace already (built by the routing launch)
     // outputs

@@ -262,19 +262,19 @@ struct ForkJoinLease {
 };
 
 // dense W8A8 MLP over all tokens, on the rows the routed experts quantised
-int shared_expert(const moe355_layer& l, const Forms& f, const Buffers& b, int64_t T, void* st)
+int shared_expert(const moe355_layer& l, const Forms& f, const Buffers& b, int64_t T, void* st, bool beside)
 {
     if (f.shared_few) return few_forward(shared_args(l, b, T), nullptr, (hipStream_t)st);
     const int64_t H = l.hidden, I = l.shared_intermediate;
-    int rc = moe355_gmm_i32(b.xq, l.shared_w13, b.one_group, MOE355_GL_CUMSUM, T, H, 2 * I, 1, b.sh_acc, b.sh_ws,
-                            b.sh_bytes, st);
+    int rc = gmm_i32_impl(b.xq, l.shared_w13, b.one_group, MOE355_GL_CUMSUM, T, H, 2 * I, 1, b.sh_acc, b.sh_ws, b.sh_bytes,
+                          st, beside);
     if (rc != MOE355_OK) return rc;
     rc = moe355_dequant_swiglu_quant_grouped(b.sh_acc, l.shared_s13, b.x_scale, nullptr, 0, nullptr, 1, T, 2 * I, 1, 1,
                                              l.shared_limit, l.shared_alpha, l.shared_beta, 1, nullptr, 0, nullptr,
                                              b.sh_q, b.sh_q_scale, st);
     if (rc != MOE355_OK) return rc;
-    return moe355_gmm2_dequant(b.sh_q, l.shared_w2, l.shared_s2, b.sh_q_scale, b.one_group, MOE355_GL_CUMSUM, T, I, H, 1,
-                               b.sh_out, l.x_dtype, b.sh_ws2, b.sh2_bytes, st);
+    return gmm2_impl(b.sh_q, l.shared_w2, nullptr, l.shared_s2, nullptr, b.sh_q_scale, b.one_group, MOE355_GL_CUMSUM, T, I, H,
+                     1, b.sh_out, l.x_dtype, b.sh_ws2, b.sh2_bytes, st, false, beside);
 }
 
 int routed_pairs(const moe355_layer& l, const Forms& f, const Buffers& b, int64_t T, void* st)
@@ -409,12 +409,12 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
         if (!lease.take() || hipEventRecord(lease.fj.fork, main) != hipSuccess ||
             hipStreamWaitEvent(side, lease.fj.fork, 0) != hipSuccess)
             return MOE355_E_LAUNCH;
-        rc = shared_expert(l, f, b, T, side);
+        rc = shared_expert(l, f, b, T, side, true);
         // joined below even if a launch was refused: the caller frees the scratch in the order of its own stream
         if (hipEventRecord(lease.fj.join, side) != hipSuccess) return MOE355_E_LAUNCH;
         joined = false;
     } else if (l.shared == 1) {
-        rc = shared_expert(l, f, b, T, stream);
+        rc = shared_expert(l, f, b, T, stream, false);
     }
     bool tiles_ready = false;
     if (rc == MOE355_OK && !f.pairs && !f.small) {

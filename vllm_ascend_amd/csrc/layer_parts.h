@@ -74,10 +74,14 @@ int gmm1_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* wei
               int64_t rows, int64_t k, int64_t n, int num_experts, float swiglu_limit, int8_t* out, float* out_scale,
               void* workspace, size_t workspace_bytes, void* stream, const int32_t* row_src = nullptr,
               bool tiles_ready = false);
+// beside: the launch runs on a side stream, beside the routed experts' products
 int gmm2_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list, const float* scale,
               const float* const* scale_list, const float* per_token_scale, const int64_t* group_list,
               int group_list_type, int64_t rows, int64_t k, int64_t n, int num_experts, void* out, int out_dtype,
-              void* workspace, size_t workspace_bytes, void* stream, bool tiles_ready = false);
+              void* workspace, size_t workspace_bytes, void* stream, bool tiles_ready = false, bool beside = false);
+int gmm_i32_impl(const int8_t* x, const int8_t* weight_nz, const int64_t* group_list, int group_list_type, int64_t rows,
+                 int64_t k, int64_t n, int num_experts, int32_t* acc, void* workspace, size_t workspace_bytes, void* stream,
+                 bool beside);
 void* gmm1_tile_ws(void* workspace, int64_t rows, int64_t n);
 // the tile map (0 or 1) that a grouped product will look for in its workspace
 int gemm_tile_specs(int64_t rows, int64_t k, int64_t n, int num_experts, void* tile_ws, TileSpec* specs);
