@@ -116,6 +116,25 @@ def test_gating_inside_the_first_launch(tokens, experts, k, groups, hidden, dtyp
     assert layer._layer_plan.desc is not None
 
 
+# the router gate's chunk results added up by the launch that gates (up to 16 chunks of 128, the last one whole or half) or
+# by a launch of their own (17), with and without a bias, few and many tokens
+@pytest.mark.parametrize("tokens", [1, 4, 5, 40, 300])
+@pytest.mark.parametrize("hidden, experts", [(64, 8), (960, 66), (1984, 32), (2048, 130), (2112, 32)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_chunk_results_of_the_gate(tokens, hidden, experts, bias):
+    from vllm_ascend_amd.fused_moe.gate_linear import AscendGateLinear
+
+    cfg, layer, x, _ = _pair("c2_small", tokens, dict(H=hidden, E=experts, k=2, I=64))
+    layer.gate = AscendGateLinear(hidden, experts, bias=bias, device=DEV)
+    g = torch.Generator(device=DEV).manual_seed(tokens)
+    layer.gate.weight.data.normal_(0.0, hidden ** -0.5, generator=g)
+    if bias:
+        layer.gate.bias.data.normal_(0.0, 1.0, generator=g)
+    logits, _ = layer.gate(x)
+    assert torch.equal(layer(x), layer.forward_impl(x, logits).routed_out)
+    assert layer._layer_plan.desc is not None
+
+
 # pair order with experts of several 32-row blocks (workgroups of their own), the others idle or with a few rows
 @pytest.mark.parametrize("tokens", [32, 33, 64, 65, 200])
 @pytest.mark.parametrize("rest", [0, 7])

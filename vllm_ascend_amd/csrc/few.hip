@@ -101,7 +101,7 @@ __device__ __forceinline__ void few_gate(const FewArgs& a, const GateCall& g, in
     float amax = 0.0f;
     if (wave < T) {
         float sel[PER];
-        row_scores<DT, PER>([&](int e) { return load_as_f32<DT>(g.logits, (int64_t)wave * a.E + e); }, g.bias, a.E,
+        row_scores<DT, PER>(RowLogits<DT>{g.logits, (int64_t)wave * a.E, (int64_t)T * a.E, g.n_planes, g.plane_bias}, g.bias, a.E,
                             g.k_group, g.group_count, g.group_select_mode, g.norm_type, groups + wave * a.E, lane, p, sel);
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
@@ -628,14 +628,15 @@ static size_t few_lds_bytes(const FewArgs& a)
 
 // At most 64 pairs (a lane each) of at most 16 tokens (the columns of the MFMA), whole 64-wide K steps, and int8 rows
 // that leave room for two workgroups in a compute unit's LDS.  Measured against pair order (us a layer call, 2 GEMM
-// launches of its own, and 4 more for a shared expert; the first two of each row are 17.3 / 25.6 and 68.5 / 130 now): Qwen3
-// shape, 1 / 2 / 4 / 8 tokens 20.6 / 27.5 / 42 / 74 against 27.0 / 32.2 / 39 / 60 (128 workgroups of the down GEMM have to read all touched experts by themselves); small layer
-// of 8 experts, 1 / 4 / 8 / 16 tokens of two slots 17 / 20 / 23 / 26 against 24 / 25 / 27 / 25; DeepSeek-V3 shape with a
-// shared expert on its side stream, 1 / 2 / 3 / 4 tokens 78 / 132 / 186 / 229 against 97 / 150 / 204 / 240, without one
-// 3 tokens 179 against 180.  So: up to 16 pairs, and with a shared expert as many as fit.
+// launches of its own, and 4 more for a shared expert): Qwen3 shape, 3 / 4 / 5 / 6 / 8 tokens 34.1 / 39.4 / 47.7 / 54.0 / 70.0
+// against 38.6 / 41.5 / 46.7 / 50.4 / 57.3 (every workgroup of the down GEMM has to read all touched experts by itself),
+// Zipf(1.1) 27.3 / 32.3 / 36.8 / 40.9 / 53.3 against 34.0 / 35.0 / 36.6 / 37.8 / 40.4; small layer of 8 experts, 10 / 12 / 16
+// tokens of two slots 22.2 / 23.1 / 24.2 against 26.3 / 26.3 / 26.5; DeepSeek-V3 shape without a shared expert, 3 / 4 tokens
+// 162 / 216 against 167 / 217, with one on its side stream, 1 / 2 / 3 / 4 tokens 78 / 132 / 186 / 229 against 97 / 150 / 204 /
+// 240.  So: up to 32 pairs, and with a shared expert as many as fit.
 bool few_supported(const FewArgs& a)
 {
-    return a.T > 0 && a.T <= 16 && a.R <= (a.sw2 ? 64 : 16) && a.H % 64 == 0 && a.I % 64 == 0 && (!a.sw2 || a.S % 64 == 0) &&
+    return a.T > 0 && a.T <= 16 && a.R <= (a.sw2 ? 64 : 32) && a.H % 64 == 0 && a.I % 64 == 0 && (!a.sw2 || a.S % 64 == 0) &&
            few_lds_bytes(a) <= 80 * 1024 - 512;
 }
 

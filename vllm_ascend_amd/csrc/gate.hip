@@ -20,6 +20,7 @@
 
 #include <type_traits>
 
+#include "layer_parts.h"
 #include "moe355_common.h"
 
 namespace moe355 {
@@ -373,10 +374,11 @@ extern "C" size_t moe355_router_gate_workspace(int64_t num_tokens, int hidden, i
     return ((chunks * (size_t)num_tokens * (size_t)num_experts * 4 + 255) / 256) * 256;
 }
 
-extern "C" int moe355_router_gate(const void* x, int x_dtype, const float* weight, const float* bias, int64_t num_tokens,
-                                  int hidden, int num_experts, float* logits, void* workspace, size_t workspace_bytes,
-                                  void* stream)
+int moe355::router_gate_impl(const void* x, int x_dtype, const float* weight, const float* bias, int64_t num_tokens,
+                             int hidden, int num_experts, float* logits, void* workspace, size_t workspace_bytes,
+                             int* n_planes, void* stream)
 {
+    if (n_planes) *n_planes = 0;
     if (num_tokens < 0 || hidden <= 0 || num_experts <= 0) return MOE355_E_ARG;
     if (num_tokens == 0) return MOE355_OK;
     if (!x || !weight || !logits) return MOE355_E_ARG;
@@ -426,10 +428,20 @@ extern "C" int moe355_router_gate(const void* x, int x_dtype, const float* weigh
     if (x_dtype == MOE355_DT_F32 && (first.kw == 4 || rest.kw == 4)) return MOE355_E_UNSUPPORTED;
     launch(first, 0, main_tokens);
     if (main_tokens < num_tokens) launch(rest, main_tokens, num_tokens - main_tokens);
-    if (g.split) {
+    if (g.split && n_planes && n_chunks <= kGatePlanes) {
+        *n_planes = n_chunks;
+    } else if (g.split) {
         const int64_t n = num_tokens * num_experts;
         hipLaunchKernelGGL(router_gate_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
                            (const float*)workspace, bias, logits, n, num_experts, n_chunks);
     }
     return launch_status();
+}
+
+extern "C" int moe355_router_gate(const void* x, int x_dtype, const float* weight, const float* bias, int64_t num_tokens,
+                                  int hidden, int num_experts, float* logits, void* workspace, size_t workspace_bytes,
+                                  void* stream)
+{
+    return router_gate_impl(x, x_dtype, weight, bias, num_tokens, hidden, num_experts, logits, workspace, workspace_bytes,
+                            nullptr, stream);
 }

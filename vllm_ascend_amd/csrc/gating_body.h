@@ -9,6 +9,7 @@
 // wavefront arg-max reductions with the "larger value, then lower index" order.
 #pragma once
 
+#include "layer_parts.h"
 #include "moe355_common.h"
 
 namespace moe355 {
@@ -285,21 +286,62 @@ __device__ __forceinline__ void gate_row(const void* __restrict__ x, const void*
 // The order of a selection score as an unsigned integer (the high word of make_key).
 __device__ __forceinline__ unsigned score_order(float score) { return (unsigned)(make_key(score, 0) >> 32); }
 
+// A row's logits as fp32: read from [T, E], or (fp32 only) added up from the router gate's chunk results, at most
+// kGatePlanes planes of T x E, in ascending order from +0 and the bias last, which is what its own reduction does.
+template <int DT>
+struct RowLogits {
+    const void* logits;
+    int64_t at, plane;  // first value of the row; values of a plane
+    int n_planes;
+    const float* bias;
+    // lane l: the logits of experts l, l + 64, ... (-inf past the last one)
+    template <int PER>
+    __device__ __forceinline__ void load(float (&p)[PER], int E, int lane) const
+    {
+        if constexpr (DT == MOE355_DT_F32) {
+            if (n_planes > 0) {
+                const float* from = (const float*)logits + at + lane;
+                float v[kGatePlanes][PER], sum[PER];
+#pragma unroll
+                for (int c = 0; c < kGatePlanes; ++c)
+#pragma unroll
+                    for (int i = 0; i < PER; ++i)
+                        v[c][i] = c < n_planes && lane + 64 * i < E ? from[c * plane + 64 * i] : 0.0f;
+#pragma unroll
+                for (int i = 0; i < PER; ++i) sum[i] = 0.0f;
+#pragma unroll
+                for (int c = 0; c < kGatePlanes; ++c)
+#pragma unroll
+                    for (int i = 0; i < PER; ++i)
+                        if (c < n_planes) sum[i] = sum[i] + v[c][i];
+#pragma unroll
+                for (int i = 0; i < PER; ++i) {
+                    const int e = lane + 64 * i;
+                    p[i] = e >= E ? -__builtin_inff() : bias ? sum[i] + bias[e] : sum[i];
+                }
+                return;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int e = lane + 64 * i;
+            p[i] = e < E ? load_as_f32<DT>(logits, at + e) : -__builtin_inff();
+        }
+    }
+};
+
 // The scores of one token row by one wavefront, the arithmetic of gate_row without a workgroup barrier: p, the values the
 // weights come from, and sel, what the experts are chosen by (groups that are not kept at -inf).  What the row needs from
 // other lanes travels by lane reads, the group scores through grp_lds (E floats private to the wavefront; only touched
-// when G > 1).  logit(e) is the logit as fp32.
-template <int DT, int PER, typename Logit>
-__device__ __forceinline__ void row_scores(Logit logit, const void* __restrict__ bias, int E, int k_group, int G, int mode,
+// when G > 1).
+template <int DT, int PER>
+__device__ __forceinline__ void row_scores(const RowLogits<DT>& logits, const void* __restrict__ bias, int E, int k_group, int G, int mode,
                                            int norm_type, float* grp_lds, int lane, float (&p)[PER], float (&sel)[PER])
 {
     float m = -__builtin_inff();
+    logits.load(p, E, lane);
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-        const int e = lane + 64 * i;
-        p[i] = (e < E) ? logit(e) : -__builtin_inff();
-        m = p[i] > m ? p[i] : m;
-    }
+    for (int i = 0; i < PER; ++i) m = p[i] > m ? p[i] : m;
     if (norm_type == 0) {
         m = wave_max_dpp(m);
         float part = 0.0f;
@@ -377,14 +419,14 @@ __device__ __forceinline__ void store_choice(int my_i, float my_p, int k, int re
 }
 
 // One token row by one wavefront.
-template <int DT, int PER, typename Logit>
-__device__ __forceinline__ void gate_row_wave(Logit logit, const void* __restrict__ bias, int E, int k, int k_group,
+template <int DT, int PER>
+__device__ __forceinline__ void gate_row_wave(const RowLogits<DT>& logits, const void* __restrict__ bias, int E, int k, int k_group,
                                               int G, int mode, int renorm, int norm_type, float rsf, float eps,
                                               int64_t o, void* __restrict__ weights, int w_dtype,
                                               int32_t* __restrict__ idx, float* grp_lds, int lane)
 {
     float p[PER], sel[PER];
-    row_scores<DT, PER>(logit, bias, E, k_group, G, mode, norm_type, grp_lds, lane, p, sel);
+    row_scores<DT, PER>(logits, bias, E, k_group, G, mode, norm_type, grp_lds, lane, p, sel);
     unsigned long long key[PER];
 #pragma unroll
     for (int i = 0; i < PER; ++i) key[i] = (lane + 64 * i < E) ? make_key(sel[i], lane + 64 * i) : 0ull;

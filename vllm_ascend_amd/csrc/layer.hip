@@ -376,10 +376,11 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
     GateCall g = {x, logits, l.bias, l.x_dtype, logits_dtype, T, l.hidden, l.num_experts, l.top_k, l.k_group,
                   l.group_count, 1, l.renorm, l.norm_type, l.routed_scaling_factor, l.eps};
     if (l.gate_weight) {
-        rc = moe355_router_gate(x, l.x_dtype, l.gate_weight, l.gate_bias, T, (int)l.hidden, l.num_experts, b.logits,
-                                b.gate_ws, b.gate_bytes, stream);
+        rc = router_gate_impl(x, l.x_dtype, l.gate_weight, l.gate_bias, T, (int)l.hidden, l.num_experts, b.logits, b.gate_ws,
+                              b.gate_bytes, &g.n_planes, stream);
         if (rc != MOE355_OK) return rc;
-        g.logits = b.logits;
+        g.logits = g.n_planes ? b.gate_ws : b.logits;
+        g.plane_bias = g.n_planes ? l.gate_bias : nullptr;
         g.logits_dtype = MOE355_DT_F32;
     }
     FewArgs few = {};

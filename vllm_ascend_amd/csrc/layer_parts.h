@@ -7,6 +7,12 @@
 
 namespace moe355 {
 
+// Chunk results of the router gate that the gating launch adds up itself, all of them in flight at once.  With more of them
+// the reduction in a launch of its own is faster: us a call with it / without, 8 planes (H = 1024, 8 experts) 1000 tokens 57 /
+// 53.8; 16 planes (128 experts) 1 / 4 / 60 / 777 tokens 24.9 / 46.9 / 117.4 / 154.3 against 24.1 / 46.2 / 116.8 / 153.7; 56
+// planes (256 experts; eight in flight at a time) one token 79 against 91.
+constexpr int kGatePlanes = 16;
+
 // hidden states and logits of a batch, and how the router scores and groups the experts
 struct GateCall {
     const void* x;       // [T, H] bf16 / fp16
@@ -16,7 +22,16 @@ struct GateCall {
     int64_t num_tokens, hidden;
     int num_experts, top_k, k_group, group_count, group_select_mode, renorm, norm_type;
     float routed_scaling_factor, eps;
+    // (at most kGatePlanes:) fp32 logits that are still the router gate's chunk results: n_planes planes [T, E] at `logits`, to be added in
+    // ascending order from +0, and plane_bias [E] last (or null); 0: `logits` holds the logits
+    int n_planes;
+    const float* plane_bias;
 };
+
+// moe355_router_gate; with n_planes, a launch that leaves the logits as chunk results says how many there are (0: none,
+// `logits` holds them) instead of adding them up: the gating launch behind it does that while it reads them
+int router_gate_impl(const void* x, int x_dtype, const float* weight, const float* bias, int64_t num_tokens, int hidden,
+                     int num_experts, float* logits, void* workspace, size_t workspace_bytes, int* n_planes, void* stream);
 
 // what the gating launches take of such a call, and what they refuse (num_tokens > 0)
 int check_gate(const GateCall& g);

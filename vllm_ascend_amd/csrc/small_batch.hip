@@ -43,6 +43,8 @@ struct SmallRouteArgs {
     int64_t* expert_tokens;  // [E]
     int32_t* arrived;     // one int32, zero between calls
     int64_t* one_group;   // or null: receives T (the group list of a dense product over all tokens)
+    int n_planes;         // GateCall
+    const float* plane_bias;
     int wave_rows;        // the quantising workgroups take four rows each, one per wavefront
 };
 
@@ -150,7 +152,8 @@ __global__ __launch_bounds__(kSmallThreads) void route_quant_small_kernel(SmallR
     {
         const int row = (int)blockIdx.x * kSmallWaves + wave;
         if (row < a.T)
-            gate_row_wave<LDT, PER>([&](int e) { return load_as_f32<LDT>(a.logits, (int64_t)row * E + e); }, a.bias, E, k,
+            gate_row_wave<LDT, PER>(RowLogits<LDT>{a.logits, (int64_t)row * E, (int64_t)a.T * E, a.n_planes, a.plane_bias},
+                                    a.bias, E, k,
                                     a.k_group, a.G, a.mode, a.renorm, a.norm_type, a.rsf, a.eps, (int64_t)row * k,
                                     a.topk_weights, a.x_dtype, a.topk_ids, lds + (size_t)wave * E, lane);
     }
@@ -289,6 +292,8 @@ int moe355::gate_quant_impl(bool sort, const GateCall& g, int tokens_num_type, v
     a.x = x;
     a.logits = logits;
     a.bias = bias;
+    a.n_planes = g.n_planes;
+    a.plane_bias = g.plane_bias;
     a.T = (int)num_tokens;
     a.H = (int)hidden;
     a.E = num_experts;
