@@ -1112,7 +1112,11 @@ int moe355::gmm1_pairs_impl(const int8_t* x, const float* x_scale, const int32_t
     hipEvent_t ev0, ev1;
     take_profile_events(ev0, ev1);
     const int64_t units = (int64_t)pair_places(a, 768) * (n / 64);
-    launch_gemm(gmm_stream_kernel<EPI_SWIGLU, 4, 4, 3, false, true, true>, dim3((unsigned)units), st, a, ev0, ev1);
+    // No more workgroups than two for every compute unit: eight K steps in flight instead of four (the small layer's 64 tokens
+    // 27.4 -> 26.6 us a call; with more workgroups the third one of a compute unit is worth more: 128 tokens 29.8 -> 31.2)
+    if (units <= 2 * kComputeUnits)
+        launch_gemm(gmm_stream_kernel<EPI_SWIGLU, 4, 8, 2, false, true, true>, dim3((unsigned)units), st, a, ev0, ev1);
+    else launch_gemm(gmm_stream_kernel<EPI_SWIGLU, 4, 4, 3, false, true, true>, dim3((unsigned)units), st, a, ev0, ev1);
     if (out)
         launch_swiglu_requant(y, nullptr, 0, num_experts, rows + a.sh_rows, (int)(n / 2), out, out_scale, st, rows);
     return launch_status();
@@ -1166,6 +1170,8 @@ int moe355::gmm2_pairs_impl(const int8_t* x, const float* per_token_scale, const
         else hipLaunchKernelGGL(kernel, by_four, dim3(256), lds, st, a);
     } else if (unsplit && units >= 2048) {
         launch_gemm(gmm_stream_kernel<EPI_DEQUANT, 1, 4, 2, false, true, true>, by_four, st, a, ev0, ev1);
+    } else if (units <= kComputeUnits) {
+        launch_gemm(gmm_stream_kernel<EPI_DEQUANT, 4, 12, 2, false, true, true>, dim3((unsigned)units), st, a, ev0, ev1);
     } else {
         launch_gemm(gmm_stream_kernel<EPI_DEQUANT, 4, 4, 3, false, true, true>, dim3((unsigned)units), st, a, ev0, ev1);
     }
