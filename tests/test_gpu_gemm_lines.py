@@ -129,3 +129,10 @@ def test_dense_product_with_k_cut_over_the_wavefronts(R, Kd, N, family):
 @pytest.mark.parametrize("R,E,Kd,N", [(1024, 8, 192, 1024), (3904, 8, 64, 1024), (3968, 8, 64, 1024), (1030, 3, 128, 2816)])
 def test_tiles_of_half_the_height_for_few_experts(R, E, Kd, N):
     test_families_on_both_sides_of_a_line(R, E, Kd, N, "tiled", True)
+
+
+# ... with three, two and one row at a time in a wavefront's registers: on both sides of 768 and of 1024 values, a last load
+# that is not full, up to eight rows per expert, an expert with a row of every token (several passes of 32 rows)
+@pytest.mark.parametrize("T,E,I", [(128, 128, 768), (128, 128, 736), (33, 128, 544), (56, 128, 800), (56, 128, 1024), (56, 128, 1056)])
+def test_rows_re_quantised_several_at_a_time(T, E, I):
+    test_requantising_down_gemm_gives_the_separate_launches_bits(T, E, I)

@@ -90,12 +90,14 @@ constexpr int kPairExperts = 2048;  // that the lookups of the slots can hold
 // like the non-negative values; then rint(v * (1 / (max / 127))), the arithmetic of swiglu_requant_kernel) and the
 // MFMA operands come from there: the re-quantisation launch and its int8 round trip disappear.  The eight
 // workgroups of an expert each do it again for the expert's few rows, which is nothing next to a launch.
+// REQ_ROWS: rows that a wavefront re-quantises at a time, REQ_VEC: 256 values of each are held (K <= 256 REQ_VEC).
 template <int EPI, int KSPLIT, int UN, int OCC, bool SLABS = false, bool EARLY = true, bool PAIRS = false,
-          bool REQ = false>
+          int REQ_ROWS = 0, int REQ_VEC = 8>
 __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
 {
     static_assert(KSPLIT == 1 || KSPLIT == 4, "workgroup barriers need all four wavefronts on one unit");
     static_assert(!PAIRS || (!SLABS && EARLY && EPI != EPI_I32), "pair order: the two GEMMs of a decode layer");
+    constexpr bool REQ = REQ_ROWS > 0;
     static_assert(!REQ || (PAIRS && EPI == EPI_DEQUANT), "the re-quantisation sits in the pair-order down GEMM");
     extern __shared__ __attribute__((aligned(16))) int8_t qtile[];  // REQ: 32 rows of K + 16 bytes
     __shared__ float qscale[REQ ? 32 : 1];
@@ -325,44 +327,58 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
         float rs = 0.0f;
         if constexpr (!REQ) xo = src * a.K + kh * 16;
         if constexpr (REQ) {
-            // rows r0 .. r0 + 31 of the expert -> int8 in LDS: a wavefront takes every fourth row and holds it in registers
-            // between its maximum and its quantisation (K < 2048).  One row at a time: two would hide the load of the
-            // second one (1 us of 52 at 24 tokens of skewed routing) and cost the fifth wavefront of a SIMD (6 %).
+            // rows r0 .. r0 + 31 of the expert -> int8 in LDS: a wavefront takes every fourth row and holds REQ_ROWS of them in
+            // registers between their maxima and their quantisation
             const int pitch = a.K + 16;  // rows 16 bytes apart in the banks
             const int rows_now = (int)(row1 - r0 < 32 ? row1 - r0 : 32);
             if (r0 != row0) __syncthreads();  // nobody still reads the rows of the pass before
-            for (int rr = wave; rr < rows_now; rr += 4) {
-                const float* y = a.y_in + (int64_t)plist[r0 + rr] * a.K + lane * 4;
-                v4f v[8];
+            for (int rr = wave; rr < rows_now; rr += 4 * REQ_ROWS) {
+                v4f v[REQ_ROWS][REQ_VEC];
+                float amax[REQ_ROWS];
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    v[i] = i * 256 + lane * 4 < a.K ? *(const v4f*)(y + i * 256) : (v4f){0.0f, 0.0f, 0.0f, 0.0f};
-                float amax = 0.0f;
+                for (int t = 0; t < REQ_ROWS; ++t) {
+                    const bool on = rr + 4 * t < rows_now;
+                    const float* y = a.y_in + (int64_t)plist[r0 + (on ? rr + 4 * t : rr)] * a.K + lane * 4;
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
+                    for (int i = 0; i < REQ_VEC; ++i)
+                        v[t][i] = on && i * 256 + lane * 4 < a.K ? *(const v4f*)(y + i * 256) : (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+                }
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const float ab = __builtin_fabsf(v[i][j]);
-                        amax = ab > amax ? ab : amax;
+                for (int t = 0; t < REQ_ROWS; ++t) {
+                    amax[t] = 0.0f;
+#pragma unroll
+                    for (int i = 0; i < REQ_VEC; ++i)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const float ab = __builtin_fabsf(v[t][i][j]);
+                            amax[t] = ab > amax[t] ? ab : amax[t];
+                        }
+                }
+#pragma unroll
+                for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+                    for (int t = 0; t < REQ_ROWS; ++t) {
+                        const float o = __shfl_xor(amax[t], off, 64);
+                        amax[t] = o > amax[t] ? o : amax[t];
                     }
 #pragma unroll
-                for (int off = 32; off > 0; off >>= 1) {
-                    const float o = __shfl_xor(amax, off, 64);
-                    amax = o > amax ? o : amax;
-                }
-                const float inv = 1.0f / (amax / 127.0f);
+                for (int t = 0; t < REQ_ROWS; ++t) {
+                    const int at = rr + 4 * t;
+                    if (at >= rows_now) break;
+                    const float inv = 1.0f / (amax[t] / 127.0f);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    if (i * 256 + lane * 4 >= a.K) break;
-                    uint32_t pk = 0u;
+                    for (int i = 0; i < REQ_VEC; ++i) {
+                        if (i * 256 + lane * 4 >= a.K) break;
+                        uint32_t pk = 0u;
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int8_t q = (amax == 0.0f) ? (int8_t)0 : sat_rint_i8(v[i][j] * inv);
-                        pk |= (uint32_t)(uint8_t)q << (8 * j);
+                        for (int j = 0; j < 4; ++j) {
+                            const int8_t q = (amax[t] == 0.0f) ? (int8_t)0 : sat_rint_i8(v[t][i][j] * inv);
+                            pk |= (uint32_t)(uint8_t)q << (8 * j);
+                        }
+                        *(uint32_t*)(qtile + at * pitch + i * 256 + lane * 4) = pk;
                     }
-                    *(uint32_t*)(qtile + rr * pitch + i * 256 + lane * 4) = pk;
+                    if (lane == 0) qscale[at] = (amax[t] == 0.0f) ? 0.0f : amax[t] / 127.0f;
                 }
-                if (lane == 0) qscale[rr] = (amax == 0.0f) ? 0.0f : amax / 127.0f;
             }
             __syncthreads();
             xo = (valid ? tok : 0) * pitch + kh * 16;
@@ -1165,7 +1181,9 @@ int moe355::gmm2_pairs_impl(const int8_t* x, const float* per_token_scale, const
     const dim3 by_four((unsigned)((units + 3) / 4));
     if (y) {
         const unsigned lds = (unsigned)(32 * (k + 16));
-        auto kernel = gmm_stream_kernel<EPI_DEQUANT, 1, 4, 2, false, true, true, true>;
+        auto kernel = gmm_stream_kernel<EPI_DEQUANT, 1, 4, 2, false, true, true, 1, 8>;
+        if (k <= 768) kernel = gmm_stream_kernel<EPI_DEQUANT, 1, 4, 2, false, true, true, 3, 3>;
+        else if (k <= 1024) kernel = gmm_stream_kernel<EPI_DEQUANT, 1, 4, 2, false, true, true, 2, 4>;
         if (ev0 || ev1) hipExtLaunchKernelGGL(kernel, by_four, dim3(256), lds, st, ev0, ev1, 0, a);
         else hipLaunchKernelGGL(kernel, by_four, dim3(256), lds, st, a);
     } else if (unsplit && units >= 2048) {
@@ -1218,11 +1236,14 @@ extern "C" int moe355_gmm2_requant_pairs_supported(int64_t num_tokens, int top_k
     if (!moe355_gmm_pairs_supported(num_tokens, top_k, n, k) || num_experts <= 0) return 0;
     const int64_t units = (int64_t)num_experts * (n / 64);
     if (!(units >= 2048 && k < 2048 && (n / 64) % 4 == 0 && k % 4 == 0 && 32 * (k + 16) <= 48 * 1024)) return 0;
-    // it pays up to about three and a half rows per expert: every workgroup of an expert quantises all its rows again.
-    // 128 experts of 2048 x 768, the layer in us with the launch of its own / inside: uniform routing 8 / 24 / 48 / 56 / 64
-    // tokens of eight slots 62.5 / 90.9 / 105.4 / 107.0 / 108.4 against 58.9 / 88.4 / 103.6 / 105.8 / 107.4; Zipf(1.1)
-    // 42.8 / 52.0 / 71.4 / 73.0 / 75.0 against 40.2 / 52.3 / 70.4 / 71.9 / 76.6, 96 tokens 85.2 against 87.0
-    return 2 * num_tokens * top_k <= 7 * (int64_t)num_experts;
+    // Every workgroup of an expert quantises all its rows again.  Rows of up to 768 values go three at a time through a
+    // wavefront's registers, and then it pays for all of pair order (eight rows per expert).  128 experts of 2048 x 768, the
+    // layer in us with the launch of its own / one row at a time / three: uniform routing 24 / 48 / 64 / 96 / 127 tokens of eight
+    // slots 92.7 / 108.0 / 109.1 / 111.9 / 114.0 against 91.3 / 105.9 / - / - / - against 91.3 / 105.7 / 106.9 / 109.2 / 111.4;
+    // Zipf(1.1), 16 / 32 / 50 / 64 / 96 / 127 tokens 47.9 / 54.9 / - / 77.4 / 90.3 / 98.2 against 46.2 / 58.5 / 72.4 / - / - / -
+    // against 45.0 / 56.0 / 70.2 / 76.3 / 88.6 / 94.8.  Longer rows: up to three and a half rows per expert (two at a time up to
+    // 1024 values, one beyond).
+    return num_tokens * top_k * 2 <= (k <= 768 ? 16 : 7) * (int64_t)num_experts;
 }
 
 extern "C" int moe355_gmm2_requant_dequant_pairs(const float* y, const int8_t* weight_nz, const float* scale,
