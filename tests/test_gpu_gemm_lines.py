@@ -136,3 +136,9 @@ def test_tiles_of_half_the_height_for_few_experts(R, E, Kd, N):
 @pytest.mark.parametrize("T,E,I", [(128, 128, 768), (128, 128, 736), (33, 128, 544), (56, 128, 800), (56, 128, 1024), (56, 128, 1056)])
 def test_rows_re_quantised_several_at_a_time(T, E, I):
     test_requantising_down_gemm_gives_the_separate_launches_bits(T, E, I)
+
+
+# fewer than 1024 rows: 31 / 32 rows per expert
+@pytest.mark.parametrize("R,family", [(32 * 16 - 1, "stream"), (32 * 16, "tiled")])
+def test_few_rows_on_tiles(R, family):
+    test_families_on_both_sides_of_a_line(R, 16, 192, 320, family, True)

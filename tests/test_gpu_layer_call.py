@@ -151,6 +151,24 @@ def test_hot_experts_in_pair_order(tokens, rest):
     assert torch.equal(layer(x, hot), want)  # against the operators on the sorted order
 
 
+# few experts: the last batch in pair order, and the first whose experts would read 128 MiB again (or have 36 rows each);
+# with a shared expert in the same launches 256 MiB, which neither reaches
+@pytest.mark.parametrize("shape, tokens", [(dict(E=8, k=2, H=1024, I=1408), 497), (dict(E=16, k=2, H=2048, I=1408), 288)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_few_experts_with_many_rows_are_sorted(shape, tokens, shared):
+    from vllm_ascend_amd import kernels as K
+
+    for T, pair_order in ((tokens - 1, True), (tokens, False)):
+        print(f"{shape} {T} tokens shared={shared}", flush=True)
+        assert K.pair_order(T, shape["k"], shape["E"], shape["E"], shape["H"], shape["I"]) is pair_order
+        cfg, layer, x, logits = _pair("c2_small", T, shape, shared=shared)
+        got = layer(x, logits)
+        assert torch.equal(got, layer.forward_impl(x, logits).routed_out)
+        layer.use_pair_order = False
+        assert torch.equal(got, layer(x, logits))
+        assert torch.equal(got, layer.forward_impl(x, logits).routed_out)
+
+
 # int4 weights in pair order (up to 40 tokens): blocks of 16 and 32 rows, further blocks, one scale per channel or per group, hot and idle experts
 @pytest.mark.parametrize("tokens", [1, 16, 17, 32, 33, 40, 41])
 @pytest.mark.parametrize("name", ["c5_small", "c5_small_perchannel"])

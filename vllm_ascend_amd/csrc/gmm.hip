@@ -634,8 +634,12 @@ static int tiled_bm(const GmmArgs& a)
     //   128 experts, K = 2048 / 768 (0.4 and 0.2 GB): 48 / 100 tokens 107 / 112 against 117 / 131 and 81 / 86 against
     //     73 / 81, so decode batches (fewer than 1024 rows) stream; 130 / 190 tokens 120 / 123 against 123 / 126 and
     //     153 / 183 against 80 / 88: tiles.
+    //   From 32 rows per expert on an expert streams its weights more than once, and few rows go on tiles as well: 16
+    //     experts, K = 2048 / 1408, 24 / 32 / 40 rows per expert 57.9 / 68.2 / 73.7 against 54.8 / 56.7 / 58.2 (Zipf 92 / 110
+    //     / 131 against 56 / 57 / 58); 24 experts, K = 4096 / 2048, 27 / 40: 154 / 232 against 133 / 138; 8 experts of that
+    //     shape, 24 / 32: 59.6 / 83.0 against 72.8 / 74.9, so no earlier.
     if (a.R < a.E) return 0;
-    if (avg < 48 && a.R < 1024 && (a.R < 128 || weights < (1ll << 30))) return 0;
+    if (avg < 32 && a.R < 1024 && (a.R < 128 || weights < (1ll << 30))) return 0;
     // Few experts and few rows: as long as tiles of half the height do not outnumber the compute units they are twice as
     // many and half as long (rows / 64 and half a tile per expert for its last one).  8 experts of 2816 x 1024 and 1024 x
     // 1408, the layer at 512 / 768 / 1024 / 1536 tokens of two slots 50.8 / 51.5 / 52.5 / 62.6 us on 128-row tiles, 41.7 /
@@ -1044,16 +1048,34 @@ extern "C" int moe355_gmm_pairs_supported(int64_t num_tokens, int top_k, int64_t
 // a product of a GiB and more has tiles for the hot ones.  DeepSeek-V3 shape, 70 / 80 / 96 tokens with the shared expert
 // in line: uniform routing 1500 / 1541 / 1581 us in pair order, 1575 / 1601 / 1641 us sorted; Zipf(1.1) 506 / 538 / 597
 // against 481 / 514 / 549; 128 tokens without it 742 against 457 us.
-extern "C" int moe355_pair_order(int64_t num_tokens, int top_k, int num_logits, int num_experts, int64_t hidden,
-                                 int64_t intermediate)
+// An expert's weights are read once for every 32 rows.  From 36 rows per expert on (at 32 half of the experts still take one
+// pass) that is what a layer of few experts takes its time for, and beyond 128 MiB of such reads it outweighs the longer
+// chain of launches of the tiles; beyond 256 MiB where the pair-order launches take a shared expert along, which costs the
+// sorted path 30 us of launches more.  us in pair order / sorted, uniform routing (Zipf(1.1)), experts of H / I, two slots:
+//   8 of 1024 / 1408, 440 / 500 tokens 44.5 / 49.1 against 40.5 / 41.0 (44.2 / 48.5 against 46.2 / 46.6);
+//   8 of 4096 / 2048, 128 / 192 / 256 tokens 79 / 91 / 117 against 75 / 78 / 78 (89 / 116 / 141 against 74 / 76 / 76), with a
+//     shared expert 130 / 160 / 200 tokens 91 / 106 / 119 against 102 / 103 / 106;
+//   16 of 2048 / 1408, 256 / 288 / 320 tokens 54.6 / 62.6 / 66.8 against 56.3 / 57.0 / 57.6;
+//   16 of 4096 / 2048, 256 / 511 tokens 130 / 214 against 92 / 109 (190 / 317 against 114 / 128);
+//   8 of 512 / 256, 511 tokens 22 against 36 (22 against 36).
+bool moe355::pair_order_impl(int64_t num_tokens, int top_k, int num_logits, int num_experts, int64_t hidden,
+                             int64_t intermediate, bool with_shared)
 {
     if (!moe355_gmm_pairs_supported(num_tokens, top_k, 2 * intermediate, hidden) ||
         !moe355_gmm_pairs_supported(num_tokens, top_k, hidden, intermediate) ||
         !moe355_gate_quant_supported(num_tokens, top_k, num_logits) || num_experts <= 0 || num_experts > 2048)
-        return 0;
+        return false;
     const int64_t pairs = num_tokens * top_k;
-    if ((int64_t)num_experts * 2 * intermediate * hidden >= (1ll << 30) && pairs > 768) return 0;
+    if ((int64_t)num_experts * 2 * intermediate * hidden >= (1ll << 30) && pairs > 768) return false;
+    const int64_t weight_bytes = 3 * intermediate * hidden;  // of one expert
+    if (pairs >= 36 * (int64_t)num_experts && pairs * weight_bytes / 32 >= (with_shared ? 2ll : 1ll) << 27) return false;
     return pairs < 1024 || pairs / num_experts < 12;
+}
+
+extern "C" int moe355_pair_order(int64_t num_tokens, int top_k, int num_logits, int num_experts, int64_t hidden,
+                                 int64_t intermediate)
+{
+    return pair_order_impl(num_tokens, top_k, num_logits, num_experts, hidden, intermediate, false);
 }
 
 // pair order: the places of the grid.

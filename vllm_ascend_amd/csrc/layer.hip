@@ -127,15 +127,16 @@ Forms forms_of(const moe355_layer& l, int64_t T)
     f.few = l.weights != W_INT4 && l.pair_order && T <= 64 && l.top_k <= 64 &&
             moe355_gate_quant_supported(T, l.top_k, l.num_experts) && few_supported(few_args(l, Buffers{}, T));
     if (f.few) return f;
+    const bool takes_shared = l.weights != W_INT4 && l.shared && l.shared_intermediate == l.intermediate &&
+                              l.shared_alpha == 1.0f && l.shared_beta == 0.0f;
     if (l.weights == W_INT4)
         f.pairs = l.pair_order && moe355_gate_quant_supported(T, l.top_k, l.num_experts) &&
                   w4_pairs_supported(T, l.top_k, l.num_experts, l.hidden, l.intermediate, l.group13, l.group2);
     else
-        f.pairs = l.pair_order && moe355_pair_order(T, l.top_k, l.num_experts, l.num_experts, l.hidden, l.intermediate);
+        f.pairs = l.pair_order && pair_order_impl(T, l.top_k, l.num_experts, l.num_experts, l.hidden, l.intermediate, takes_shared);
     const bool int8_pairs = f.pairs && l.weights != W_INT4;
     f.requant = int8_pairs && moe355_gmm2_requant_pairs_supported(T, l.top_k, l.hidden, l.intermediate, l.num_experts);
-    f.merged = int8_pairs && !f.requant && l.shared && l.shared_intermediate == l.intermediate && l.shared_alpha == 1.0f &&
-               l.shared_beta == 0.0f;
+    f.merged = int8_pairs && !f.requant && takes_shared;
     // Up to 16 tokens the kernels for a few tokens run a shared expert in two or three launches instead of four.  On the
     // side stream that pays from 8 tokens on: below, their many workgroups take more from the routed GEMM beside them
     // than they save.  int4 layer of the DeepSeek-V3 shape, us a call, four launches against these: in line, 2 / 8 / 16
@@ -410,7 +411,11 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
         if (!lease.take() || hipEventRecord(lease.fj.fork, main) != hipSuccess ||
             hipStreamWaitEvent(side, lease.fj.fork, 0) != hipSuccess)
             return MOE355_E_LAUNCH;
-        rc = shared_expert(l, f, b, T, side, true);
+        // Products of the routed experts that end after some 50 us do not cover a dense product that leaves most of the chip
+        // idle.  Experts of 4096 / 2048, two slots, us a call with `beside` / without: 8 experts, 200 / 256 / 320 / 600 tokens
+        // 159 / 174 / 130 / 171 against 100 / 107 / 113 / 166; 16 experts, 700 tokens 156 against 173.
+        const int64_t routed_bytes = 3 * l.num_experts * l.hidden * l.intermediate / (l.weights == W_INT4 ? 2 : 1);
+        rc = shared_expert(l, f, b, T, side, routed_bytes >= (1ll << 28));
         // joined below even if a launch was refused: the caller frees the scratch in the order of its own stream
         if (hipEventRecord(lease.fj.join, side) != hipSuccess) return MOE355_E_LAUNCH;
         joined = false;

@@ -76,6 +76,9 @@ struct PairShared {
     }
 };
 
+// moe355_pair_order; with_shared: the launches take a shared expert of a routed expert's shape along
+bool pair_order_impl(int64_t num_tokens, int top_k, int num_logits, int num_experts, int64_t hidden, int64_t intermediate,
+                     bool with_shared);
 // with `shared`, y, out and out_scale hold num_tokens more rows (the shared expert's, in token order); the same for x,
 // per_token_scale and out of the second
 int gmm1_pairs_impl(const int8_t* x, const float* x_scale, const int32_t* topk_ids, int64_t num_tokens, int top_k,
@@ -89,7 +92,7 @@ int gmm1_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* wei
               int64_t rows, int64_t k, int64_t n, int num_experts, float swiglu_limit, int8_t* out, float* out_scale,
               void* workspace, size_t workspace_bytes, void* stream, const int32_t* row_src = nullptr,
               bool tiles_ready = false);
-// beside: the launch runs on a side stream, beside the routed experts' products
+// beside: the launch runs on a side stream, beside long products of the routed experts
 int gmm2_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list, const float* scale,
               const float* const* scale_list, const float* per_token_scale, const int64_t* group_list,
               int group_list_type, int64_t rows, int64_t k, int64_t n, int num_experts, void* out, int out_dtype,
