@@ -142,3 +142,9 @@ def test_rows_re_quantised_several_at_a_time(T, E, I):
 @pytest.mark.parametrize("R,family", [(32 * 16 - 1, "stream"), (32 * 16, "tiled")])
 def test_few_rows_on_tiles(R, family):
     test_families_on_both_sides_of_a_line(R, 16, 192, 320, family, True)
+
+
+# 64 rows per expert at a long K: as many columns of wide tiles as half of the compute units, and one less
+@pytest.mark.parametrize("E,family", [(63, "tiled"), (64, "wide")])
+def test_columns_of_wide_tiles(E, family):
+    test_families_on_both_sides_of_a_line(64 * E, E, 4096, 576, family, True)

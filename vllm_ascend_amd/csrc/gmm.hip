@@ -652,15 +652,20 @@ static int tiled_bm(const GmmArgs& a)
     // 2091 / 2126 / 2280 us with the weight-streaming tiles in the first product, 1867 / 1975 / 2031 / 2088 / 2162 / 2512
     // us on 128-row tiles; Zipf(1.1) at 28 / 40 / 64 / 94 / 128 1115 / 1361 / 1703 / 2164 / 2616 against 1069 / 1339 /
     // 1667 / 2155 / 2648.  128 experts at K = 4096, 56 / 69 / 81 rows: 526 / 547 / 567 against 511 / 552 / 576.
-    if (avg >= 64 && avg <= 256 && a.K >= 4096 && wide_ok) return 256;
+    // A handful of wide tiles leaves most of the chip idle: 8 experts, K = 4096 / 2048 (64 columns of tiles), 500 / 800 / 1000
+    // tokens of two slots 123 / 159 / 169 us with them, 99 / 102 / 126 on 128-row tiles (Zipf(1.1) 154 / 159 / 172 against 97 /
+    // 104 / 136); 16 experts (128 columns), 600 / 1000 / 1500 tokens 136 / 160 / 193 against 120 / 168 / 160; 32 experts 196 /
+    // 215 / 272 against 196 / 262 / 276.  (One expert: a dense product on a side stream, which should leave the chip idle.)
+    const bool narrow = a.N <= 512;
+    const int64_t columns = (int64_t)a.E * ((a.N + 511) / 512);
+    if (avg >= 64 && avg <= 256 && a.K >= 4096 && wide_ok && (narrow || a.E == 1 || columns >= kComputeUnits / 2)) return 256;
     // Around 128 rows per expert most experts fit one wide tile of 128 or 160 rows and fetch their weights once, which
     // pays from K = 1024 on if the experts are about equally popular and there are enough of them to fill the chip.  128
     // experts, K = 2048 / 768, the layer at 100 / 112 / 128 / 144 / 160 / 192 rows per expert: 201 / 210 / 224 / 241 / 260 /
     // 280 us with the wide tiles in the first product, 193 / 212 / 232 / 250 / 253 / 264 us on 128-row tiles; Zipf(1.1) at
     // 96 / 128 / 192 219 / 254 / 322 against 187 / 213 / 268, so no further than they win.
     // (Products of up to 512 channels keep the range that was measured for them, 96 to 192.)
-    const bool narrow = a.N <= 512;
-    const bool fills = narrow || (int64_t)a.E * ((a.N + 511) / 512) >= kComputeUnits;
+    const bool fills = narrow || columns >= kComputeUnits;
     if (avg >= (narrow ? 96 : 112) && avg <= (narrow ? 192 : 144) && a.K >= 1024 && wide_ok && fills) return 256;
     return 128;
 }
