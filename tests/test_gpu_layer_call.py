@@ -151,6 +151,17 @@ def test_hot_experts_in_pair_order(tokens, rest):
     assert torch.equal(layer(x, hot), want)  # against the operators on the sorted order
 
 
+# ... with further blocks in front of the slots and no places before them (up to two pairs per expert), and behind them as well
+@pytest.mark.parametrize("tokens", [56, 64, 65, 250])
+def test_further_blocks_around_the_slots(tokens):
+    cfg, layer, x, logits = _pair("c2_small", tokens, dict(E=128, k=4))
+    hot = logits[:1].expand(tokens, -1).contiguous()
+    hot[::5] = logits[::5]
+    got = layer(x, hot)
+    layer.use_pair_order = False
+    assert torch.equal(got, layer(x, hot))
+
+
 # few experts: the last batch in pair order, and the first whose experts would read 128 MiB again (or have 36 rows each);
 # with a shared expert in the same launches 256 MiB, which neither reaches
 @pytest.mark.parametrize("shape, tokens", [(dict(E=8, k=2, H=1024, I=1408), 497), (dict(E=16, k=2, H=2048, I=1408), 288)])

@@ -124,6 +124,9 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
         shared = e < a.sh_blocks;
         if (shared) block = e;
         e = shared ? 0 : e - a.sh_blocks;
+        // further blocks are numbered behind the slots, the first pair_early of them run in front of the slots
+        if (e >= a.pair_first && e < a.pair_first + a.pair_early + a.pair_slots)
+            e = e < a.pair_first + a.pair_early ? e + a.pair_slots : e - a.pair_early;
     }
     const int nb0 = (EPI == EPI_SWIGLU) ? p : 2 * p;
     const int nb1 = (EPI == EPI_SWIGLU) ? p + upe : 2 * p + 1;
@@ -1094,14 +1097,20 @@ extern "C" int moe355_pair_order(int64_t num_tokens, int top_k, int num_logits, 
 // uniform 113.3 / 116.7 / 113.6 us.
 // An expert with more than 32 rows takes several passes over its weights, one after the other.  Where an expert has few
 // units (the launch is over after two or three rounds of workgroups) its further blocks of 32 rows become workgroups of
-// their own at the end of the grid: Qwen3 shape, Zipf(1.1), 64 / 100 / 127 tokens 77 / 118 / 135 -> 75 / 86 / 93 us,
+// their own: Qwen3 shape, Zipf(1.1), 64 / 100 / 127 tokens 77 / 118 / 135 -> 75 / 86 / 93 us,
 // uniform routing unchanged.  With 48 units and more the passes hide among the other workgroups, and the repeated
 // fetches at the end do not (DeepSeek-V3 shape, 64 tokens under Zipf(1.1): 444 us in passes, 477 in workgroups).
+// Those are the longest workgroups of the launch, and at the end of the grid the chip waits for them; but there are
+// places for as many as R pairs could need, and in front of the slots an unused one delays them.  So as many as skewed
+// routing usually needs, one for every 56 pairs, run in front and the others at the end.  Qwen3 shape, 40 / 64 / 100 / 127
+// tokens, all at the end / so / one for every 32 pairs in front: Zipf(1.1) 67.3 / 75.3 / 86.8 / 94.5 against 64.4 / 71.0 / 81.5
+// / 90.5 against 63.7 / 70.8 / 82.4 / 88.6 us, uniform routing 103.2 / 108.0 / 110.2 / 111.5 against 103.3 / 108.0 / 110.3 /
+// 111.8 against 103.3 / 108.2 / 110.8 / 112.8.
 // The lookups hold 2048 experts.
 static int pair_places(GmmArgs& a, int resident_units)
 {
     a.pair_first = a.E;
-    a.pair_slots = a.pair_extra = 0;
+    a.pair_slots = a.pair_extra = a.pair_early = 0;
     if (a.E <= kPairExperts) {
         a.pair_first = a.R > 2 * (int64_t)a.E ? resident_units / (a.N / 64) - a.sh_blocks : 0;
         if (a.pair_first > a.E) a.pair_first = a.E;
@@ -1110,6 +1119,7 @@ static int pair_places(GmmArgs& a, int resident_units)
         a.pair_slots = a.R < (int64_t)rest ? (int)a.R : rest;
         // an expert of c rows has (c - 1) / 32 further blocks: over all experts at most (R - 1) / 32
         if (a.N / 64 < 48) a.pair_extra = (int)((a.R - 1) / 32);
+        a.pair_early = a.R / 56 < a.pair_extra ? (int)(a.R / 56) : a.pair_extra;
     }
     return a.sh_blocks + a.pair_first + a.pair_slots + a.pair_extra;
 }

@@ -40,8 +40,9 @@ struct GmmArgs {
     int pair_k, pair_gather;
     // The grid has a place for each of the experts [0, pair_first), and pair_slots places behind them: slot s works on
     // the s-th of the other experts that have pairs (the idle ones cost nothing).  pair_extra > 0: those work on the
-    // first 32 rows of their expert, and as many more places at the end of the grid on further blocks of 32 rows.
-    int pair_first, pair_slots, pair_extra;
+    // first 32 rows of their expert, and as many more places on further blocks of 32 rows: pair_early of them in front of
+    // the slots, the others at the end of the grid.
+    int pair_first, pair_slots, pair_extra, pair_early;
     // Pair order with the shared expert in the same launch: sh_blocks places in front of the others, place b on rows
     // 32 b .. of the sh_rows tokens.  Token t's values lie in row t (pair_gather) or R + t of x, its result goes to row
     // R + t.  Its weights have the shape of a routed expert's.
