@@ -151,10 +151,14 @@ def test_hot_experts_in_pair_order(tokens, rest):
     assert torch.equal(layer(x, hot), want)  # against the operators on the sorted order
 
 
-# ... with further blocks in front of the slots and no places before them (up to two pairs per expert), and behind them as well
-@pytest.mark.parametrize("tokens", [56, 64, 65, 250])
-def test_further_blocks_around_the_slots(tokens):
-    cfg, layer, x, logits = _pair("c2_small", tokens, dict(E=128, k=4))
+# ... with further blocks in front of the slots and no places before them (up to two pairs per expert), and behind them as well;
+# an expert of 50 units on both sides of 384 pairs
+FURTHER = [(t, dict(E=128, k=4)) for t in (56, 64, 65, 250)] + [(t, dict(I=1600)) for t in (95, 96)]
+
+
+@pytest.mark.parametrize("tokens, shape", FURTHER)
+def test_further_blocks_around_the_slots(tokens, shape):
+    cfg, layer, x, logits = _pair("c2_small", tokens, shape)
     hot = logits[:1].expand(tokens, -1).contiguous()
     hot[::5] = logits[::5]
     got = layer(x, hot)

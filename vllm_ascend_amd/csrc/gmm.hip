@@ -1097,9 +1097,11 @@ extern "C" int moe355_pair_order(int64_t num_tokens, int top_k, int num_logits, 
 // uniform 113.3 / 116.7 / 113.6 us.
 // An expert with more than 32 rows takes several passes over its weights, one after the other.  Where an expert has few
 // units (the launch is over after two or three rounds of workgroups) its further blocks of 32 rows become workgroups of
-// their own: Qwen3 shape, Zipf(1.1), 64 / 100 / 127 tokens 77 / 118 / 135 -> 75 / 86 / 93 us,
-// uniform routing unchanged.  With 48 units and more the passes hide among the other workgroups, and the repeated
-// fetches at the end do not (DeepSeek-V3 shape, 64 tokens under Zipf(1.1): 444 us in passes, 477 in workgroups).
+// their own: Qwen3 shape (24 and 32 units), Zipf(1.1), 64 / 100 / 127 tokens 77 / 118 / 135 -> 75 / 86 / 93 us, uniform
+// routing unchanged.  From 48 units on the passes hide among the other workgroups until the hot experts have a few blocks
+// each: DeepSeek-V3 shape, gate_up product (64 units), Zipf(1.1), 33 / 50 / 64 / 90 tokens of eight slots 345 / 417 / 453 / 589 us
+// in passes, 347 / 414 / 448 / 573 in workgroups (uniform 40 / 64 / 96 tokens 1234 / 1467 / 1610 and 1235 / 1468 / 1610); its down
+// product (112 units) is the same either way.
 // Those are the longest workgroups of the launch, and at the end of the grid the chip waits for them; but there are
 // places for as many as R pairs could need, and in front of the slots an unused one delays them.  So as many as skewed
 // routing usually needs, one for every 56 pairs, run in front and the others at the end.  Qwen3 shape, 40 / 64 / 100 / 127
@@ -1118,7 +1120,7 @@ static int pair_places(GmmArgs& a, int resident_units)
         const int rest = a.E - a.pair_first;
         a.pair_slots = a.R < (int64_t)rest ? (int)a.R : rest;
         // an expert of c rows has (c - 1) / 32 further blocks: over all experts at most (R - 1) / 32
-        if (a.N / 64 < 48) a.pair_extra = (int)((a.R - 1) / 32);
+        if (a.N / 64 < (a.R < 384 ? 48 : 96)) a.pair_extra = (int)((a.R - 1) / 32);
         a.pair_early = a.R / 56 < a.pair_extra ? (int)(a.R / 56) : a.pair_extra;
     }
     return a.sh_blocks + a.pair_first + a.pair_slots + a.pair_extra;
