@@ -125,6 +125,31 @@ def test_dense_product_with_k_cut_over_the_wavefronts(R, Kd, N, family):
         assert np.array_equal(s.cpu().numpy().view(np.uint32)[:rows], s_want.view(np.uint32)[:rows])
 
 
+# ... whose rows are gathered from tokens beyond 4 GiB (and, by turns, from tokens in front of them)
+def test_dense_product_gathers_beyond_4_gib():
+    from vllm_ascend_amd import kernels as K
+    from vllm_ascend_amd._lib import W_ENK, load
+
+    R, Kd, N = 70, 1 << 16, 128
+    T = (1 << 32) // Kd + R
+    print(f"dense gather R={R} K={Kd} N={N} from {T} tokens", flush=True)
+    assert load().moe355_gmm_kernel_name(1, R, Kd, N, 1).decode() == "gmm_split_kernel"
+    g = torch.Generator(device="cuda").manual_seed(R)
+    x = torch.zeros(T, Kd, dtype=torch.int8, device="cuda")
+    x[:R], x[-R:] = (torch.randint(-128, 128, (R, Kd), generator=g, dtype=torch.int8, device="cuda") for _ in range(2))
+    rows = torch.arange(R, dtype=torch.int32, device="cuda")
+    rows[::2] += T - R
+    wnz = K.format_cast_nz(torch.randint(-128, 128, (1, N, Kd), generator=g, dtype=torch.int8, device="cuda"), W_ENK)
+    sw = torch.rand(1, N, generator=g, device="cuda") * 0.009 + 0.001
+    sx = torch.rand(T, generator=g, device="cuda") * 0.05 + 0.001
+    cum = torch.tensor([R], dtype=torch.int64, device="cuda")
+    q, s = K.gmm1_swiglu_quant_gather(x, sx, rows, wnz, sw, cum, 0, N, Kd)
+    at = rows.long()
+    q_want, s_want = K.gmm1_swiglu_quant(x[at], wnz, sw, sx[at], cum, 0, N, Kd)
+    torch.cuda.synchronize()
+    assert torch.equal(q, q_want) and torch.equal(s.view(torch.int32), s_want.view(torch.int32))
+
+
 # few experts: 64-row tiles as long as they do not outnumber the compute units, on both sides of the line
 @pytest.mark.parametrize("R,E,Kd,N", [(1024, 8, 192, 1024), (3904, 8, 64, 1024), (3968, 8, 64, 1024), (1030, 3, 128, 2816)])
 def test_tiles_of_half_the_height_for_few_experts(R, E, Kd, N):

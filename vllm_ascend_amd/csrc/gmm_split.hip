@@ -46,13 +46,14 @@ __global__ __launch_bounds__(256, 2) void gmm_split_kernel(GmmArgs a, int units)
     const int8_t* w1 = we + (int64_t)nb1 * KB * 1024;
     const int K64 = a.K >> 6, k0 = K64 * wave / 4, n = K64 * (wave + 1) / 4 - k0;
 
-    // token pieces of this lane: 16 bytes of row 16 i + lane / 4 (rows past the end repeat the last one)
-    uint32_t xo[2 * TB];
+    // token pieces of this lane: 16 bytes of row 16 i + lane / 4 (rows past the end repeat the last one).  64 bits: row_src may
+    // name any token of an x larger than 4 GiB, however few rows there are.
+    int64_t xo[2 * TB];
 #pragma unroll
     for (int i = 0; i < 2 * TB; ++i) {
         int64_t r = row0 + 16 * i + (lane >> 2);
         if (r >= row_end) r = row_end - 1;
-        xo[i] = (uint32_t)((a.row_src ? (int64_t)a.row_src[r] : r) * a.K) + (lane & 3) * 16;
+        xo[i] = (a.row_src ? (int64_t)a.row_src[r] : r) * a.K + (lane & 3) * 16;
     }
     // operands of the epilogue, in front of everything else in the queue of answers: this wavefront finishes the channels
     // of quarter `wave`
@@ -88,7 +89,7 @@ __global__ __launch_bounds__(256, 2) void gmm_split_kernel(GmmArgs a, int units)
             w[slot][1][s] = gload16(w1 + kw + s * 1024 + lo);
         }
 #pragma unroll
-        for (int i = 0; i < 2 * TB; ++i) x[slot][i] = gload16(a.x + kx + (in ? xo[i] : 0u));
+        for (int i = 0; i < 2 * TB; ++i) x[slot][i] = gload16(a.x + kx + (in ? xo[i] : 0));
     };
     // a row's four pieces of a stage lie rotated by half its number: neither the writes (two whole rows at a time) nor the
     // reads (one piece of eight rows) meet in a bank
