@@ -387,3 +387,31 @@ def test_layer_kernel_names_follow_the_form():
     assert name(16, weights=2, **big) == "gmm_w4_pairs_kernel" and name(512, weights=2, **big) == "gmm_w4_stream_kernel"
     assert name(0) == "" and name(4, shared=3) == ""
     assert lib.moe355_layer_kernel_name(None, 4) == b""
+
+
+def test_a_shared_expert_that_the_pair_order_launches_can_take_is_in_them():
+    """Also where the down product could re-quantise inside instead (no GPU: a pure function).  With it the layer stays in
+    pair order up to 256 MiB of repeated weight reads instead of 128."""
+    from vllm_ascend_amd import _lib
+
+    lib = _lib.load()
+
+    def name(T, experts, hidden, inter, top_k, shared, **kw):
+        args = dict(hidden=hidden, intermediate=inter, num_experts=experts, top_k=top_k, k_group=1, group_count=1,
+                    x_dtype=_lib.DT_BF16, pair_order=1, w13=256, s13=256, w2=256, s2=256, shared=shared,
+                    shared_intermediate=inter, shared_alpha=1.0, shared_w13=256, shared_s13=256, shared_w2=256, shared_s2=256)
+        return lib.moe355_layer_kernel_name(ctypes.byref(_lib.Layer(**{**args, **kw})), T).decode()
+
+    merged = "gmm_stream_kernel with the shared expert"
+    for T in (9, 56, 57, 64, 127):
+        for inter in (512, 768, 1024):
+            for shared in (1, 2):
+                assert name(T, 128, 2048, inter, 8, shared) == merged
+                assert name(min(T, 64), 64, 2048, inter, 8, shared) == merged
+            assert name(T, 128, 2048, inter, 8, 1, shared_intermediate=2 * inter) == "gmm_stream_kernel"
+            assert name(T, 128, 2048, inter, 8, 1, shared_alpha=1.5) == "gmm_stream_kernel"
+            assert lib.moe355_gmm2_requant_pairs_supported(T, 8, 2048, inter, 128) == (T <= 56 or inter <= 768)
+    for shared in (1, 2):
+        assert name(170, 8, 4096, 2048, 2, shared) == merged and name(171, 8, 4096, 2048, 2, shared) == "gmm_tiled_kernel"
+    assert name(143, 8, 4096, 2048, 2, 0) == "gmm_stream_kernel" and name(144, 8, 4096, 2048, 2, 0) == "gmm_tiled_kernel"
+    assert not lib.moe355_pair_order(144, 2, 8, 8, 4096, 2048) and lib.moe355_pair_order(143, 2, 8, 8, 4096, 2048)

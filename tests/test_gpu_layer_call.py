@@ -176,12 +176,37 @@ def test_few_experts_with_many_rows_are_sorted(shape, tokens, shared):
     for T, pair_order in ((tokens - 1, True), (tokens, False)):
         print(f"{shape} {T} tokens shared={shared}", flush=True)
         assert K.pair_order(T, shape["k"], shape["E"], shape["E"], shape["H"], shape["I"]) is pair_order
-        cfg, layer, x, logits = _pair("c2_small", T, shape, shared=shared)
+        cfg, layer, x, logits = _pair("c2_small", T, dict(shape, shared=shared), shared=shared)
+        assert (layer.shared_experts is not None) == shared
         got = layer(x, logits)
         assert torch.equal(got, layer.forward_impl(x, logits).routed_out)
         layer.use_pair_order = False
         assert torch.equal(got, layer(x, logits))
         assert torch.equal(got, layer.forward_impl(x, logits).routed_out)
+
+
+# ... the last batch in pair order with a shared expert in the launches, and the first one without
+@pytest.mark.parametrize("overlap", [False, True])
+def test_few_experts_with_a_shared_expert_are_sorted_later(overlap):
+    shape = dict(E=8, k=2, H=4096, I=2048)
+    for T in (170, 171):
+        cfg, layer, x, logits = _pair("c2_small", T, dict(shape, shared=True), shared=True, overlap=overlap)
+        assert layer.shared_experts is not None
+        got = layer(x, logits)
+        assert torch.equal(got, layer.forward_impl(x, logits).routed_out)
+        layer.use_pair_order = False
+        assert torch.equal(got, layer(x, logits))
+
+
+# a shared expert in the launches of a layer whose down product could re-quantise inside
+@pytest.mark.parametrize("tokens", [9, 57, 127])
+@pytest.mark.parametrize("overlap", [False, True])
+def test_shared_expert_instead_of_the_re_quantisation(tokens, overlap):
+    shape = dict(E=128, k=8, H=1024, I=320, shared=True)
+    cfg, layer, x, logits = _pair("c2_small", tokens, shape, shared=True, overlap=overlap)
+    assert layer.shared_experts is not None
+    assert torch.equal(layer(x, logits), layer.forward_impl(x, logits).routed_out)
+    assert layer._layer_plan.desc is not None
 
 
 # int4 weights in pair order (up to 40 tokens): blocks of 16 and 32 rows, further blocks, one scale per channel or per group, hot and idle experts

@@ -135,8 +135,15 @@ Forms forms_of(const moe355_layer& l, int64_t T)
     else
         f.pairs = l.pair_order && pair_order_impl(T, l.top_k, l.num_experts, l.num_experts, l.hidden, l.intermediate, takes_shared);
     const bool int8_pairs = f.pairs && l.weights != W_INT4;
-    f.requant = int8_pairs && moe355_gmm2_requant_pairs_supported(T, l.top_k, l.hidden, l.intermediate, l.num_experts);
-    f.merged = int8_pairs && !f.requant && takes_shared;
+    // A shared expert that the two launches can take along saves more (three or four launches) than the re-quantisation inside
+    // the second one (a launch, and only without a shared expert in it).  us a call with the re-quantisation inside and the
+    // shared expert in launches of its own, in line or on the side stream, against merged: 128 experts of 2048 / 768, eight
+    // slots, 10 / 24 / 57 / 64 tokens 74.9 / 110.5 / 130.7 / 132.0 and 78.0 / 104.7 / 122.2 / 123.8 against 71.1 / 96.3 / 114.3 /
+    // 115.3, Zipf(1.1) 52.9 / 69.0 / 92.7 / 95.5 and 67.6 / 73.4 / 85.6 / 87.3 against 44.6 / 53.3 / 73.1 / 75.8; 64 experts of
+    // 2048 / 512, 64 tokens 71.8 and 73.8 against 57.4.  Nowhere slower between 64 and 128 experts and rows of 512 to 1024 values.
+    f.merged = int8_pairs && takes_shared;
+    f.requant = int8_pairs && !f.merged &&
+                moe355_gmm2_requant_pairs_supported(T, l.top_k, l.hidden, l.intermediate, l.num_experts);
     // Up to 16 tokens the kernels for a few tokens run a shared expert in two or three launches instead of four.  On the
     // side stream that pays from 8 tokens on: below, their many workgroups take more from the routed GEMM beside them
     // than they save.  int4 layer of the DeepSeek-V3 shape, us a call, four launches against these: in line, 2 / 8 / 16
