@@ -548,6 +548,8 @@ int moe355_layer_forward(const moe355_layer *layer /* host */, const void *x, co
  * expert's product is in the same launch; "" for arguments no call accepts.  A pure function of its arguments, for
  * benchmarks and profiles (no counterpart in the reference). */
 const char *moe355_layer_kernel_name(const moe355_layer *layer /* host */, int64_t num_tokens);
+/* 1: that launch gates and quantises the tokens as well; 0: a launch in front of it does. */
+int moe355_layer_gates_inside(const moe355_layer *layer /* host */, int64_t num_tokens);
 
 #ifdef __cplusplus
 }

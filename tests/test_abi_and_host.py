@@ -415,3 +415,20 @@ def test_a_shared_expert_that_the_pair_order_launches_can_take_is_in_them():
         assert name(170, 8, 4096, 2048, 2, shared) == merged and name(171, 8, 4096, 2048, 2, shared) == "gmm_tiled_kernel"
     assert name(143, 8, 4096, 2048, 2, 0) == "gmm_stream_kernel" and name(144, 8, 4096, 2048, 2, 0) == "gmm_tiled_kernel"
     assert not lib.moe355_pair_order(144, 2, 8, 8, 4096, 2048) and lib.moe355_pair_order(143, 2, 8, 8, 4096, 2048)
+
+
+# (experts, slots, hidden, intermediate) and the most tokens that the first launch gates and quantises by itself: the
+# comparisons grow with the experts and the tokens, the rounds over a row's values with the hidden size, and more than 256 or
+# 576 workgroups wait for each other
+@pytest.mark.parametrize("experts, top_k, hidden, inter, most", [
+    (8, 2, 1024, 1408, 3), (32, 4, 1024, 256, 4), (32, 4, 2048, 512, 2), (64, 8, 2048, 512, 2), (64, 2, 1024, 1024, 4),
+    (128, 8, 2048, 768, 1), (128, 4, 2048, 768, 1), (128, 8, 512, 256, 2), (256, 8, 2048, 256, 1), (256, 4, 4096, 384, 0),
+    (256, 8, 7168, 2048, 0), (1, 1, 2048, 1408, 4)])
+def test_gating_inside_the_first_launch_where_it_is_short(experts, top_k, hidden, inter, most):
+    from vllm_ascend_amd import _lib
+
+    lib = _lib.load()
+    a = _lib.Layer(hidden=hidden, intermediate=inter, num_experts=experts, top_k=top_k, k_group=1, group_count=1,
+                   x_dtype=_lib.DT_BF16, pair_order=1, w13=256, s13=256, w2=256, s2=256)
+    assert [lib.moe355_layer_gates_inside(ctypes.byref(a), T) for T in range(6)] == [int(1 <= T <= most) for T in range(6)]
+    assert lib.moe355_layer_gates_inside(None, 1) == 0

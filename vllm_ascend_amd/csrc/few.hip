@@ -647,16 +647,30 @@ static bool few_quant_inside(const FewArgs& a)
     return a.I <= 2048 && (!a.sw2 || a.S <= 2048) && (int64_t)a.R * a.I + (a.sw2 ? a.T * a.S : 0) <= kFewInside;
 }
 
-// Whether the up kernel gates and quantises by itself (few_up_kernel<., PER > 0>).  Every workgroup does, which costs 3.5 us
-// in front of its weights, against a launch of 4 us and its hand-over; so it pays as long as (nearly) all workgroups are
-// resident at once, two in a compute unit.  us a call, in a launch of its own / inside: one token of the Qwen3 shape (384
-// workgroups) 18.6 / 17.3, small layer of 8 experts 1 / 3 / 4 tokens (176, 528, 704 workgroups) 14 / 12.1, 15.4 / 14.9, 17.0 /
-// 17.6; two tokens of the Qwen3 shape (768) 25.6 / 26.5, one of the DeepSeek-V3 shape (1024) 68.6 / 75.7.
-bool few_gates(const FewArgs& a, const GateCall& g)
+// Whether the up kernel gates and quantises by itself (few_up_kernel<., PER > 0>).  Every workgroup does, in front of its
+// weights, against a launch in front of it with its hand-over, 3.2 us.  What it costs is the chain of its slowest wavefront:
+// the experts that it compares (its share of all of them, 64 at a time, about 25 ns each) and its rounds over a row's values
+// (the first of them hides behind the scores, the others take about 30 comparisons each).  Two workgroups of a compute unit
+// take turns at its vector ALUs, so beyond one for every unit all of it counts twice, and beyond (nearly) two the others wait.
+// us a call inside / in a launch of its own (in brackets the workgroups and the sum below):
+//   E =   8, H = 1024, 1 / 2 / 3 / 4 tokens (176 to 704; 1, 4, 68, -)      14.0 / 14.3 / 15.7 / 17.7   17.2 / 16.7 / 16.7 / 17.0
+//   E =  32, H = 2048, 1 / 2 / 3 / 4 tokens (128 to 512; 4, 38, 212, 212)  14.1 / 15.7 / 19.2 / 20.9   17.0 / 16.9 / 18.3 / 20.0
+//   E =  64, H = 2048, 1 / 2 tokens (256, 512; 8, 92)                      14.9 / 19.8                 17.0 / 20.8
+//   E =  64, H = 1024, 3 / 4 tokens of two slots (384, 512; 124)           16.6 / 18.0                 17.1 / 17.4
+//   E = 128, H = 2048, 1 token of eight slots (384; 64)                    18.1                        19.5
+//                      2 / 3 tokens of four (384, 576; 188, 436)           19.1 / 28.5                 18.4 / 22.1
+//   E = 128, H =  512, 2 / 3 tokens (256, 384; 64, 256)                    15.9 / 22.1                 17.1 / 19.4
+//   E = 256, H = 2048, 1 / 2 / 3 / 4 tokens (128 to 512; 128, 286, ..)     17.0 / 21.9 / 38.3 / 42.9   16.6 / 18.0 / 22.0 / 24.9
+//            H = 1024, 1 token of one slot (64; 128)                       14.9                        16.6
+bool few_gates(const FewArgs& a)
 {
-    const int places = a.R < a.E ? a.R : a.E;
-    return a.T <= kFewGateTokens && a.T * (a.H + 16) <= 24 * 1024 && a.E <= 256 && a.R <= 64 &&
-           places * (a.I / 16) + (a.sw2 ? a.S / 16 : 0) <= 576;
+    const int places = a.R < a.E ? a.R : a.E, T = a.T;
+    const int groups = places * (a.I / 16) + (a.sw2 ? a.S / 16 : 0);
+    if (T < 1 || T > kFewGateTokens || T * (a.H + 16) > 24 * 1024 || a.E > 256 || a.R > 64 || groups > 576) return false;
+    const int rankers = T == 1 ? 8 : T == 2 ? 4 : 2, held = a.E <= 64 ? 1 : a.E <= 128 ? 2 : 4;  // few_gate, few_forward
+    const int quantisers = (kFewWaves - T) / T;                                                  // of the row that has fewest
+    const int rounds = (a.H + 512 * quantisers - 1) / (512 * quantisers);
+    return ((a.E + rankers - 1) / rankers * held + 30 * (rounds - 1)) * (groups > 256 ? 2 : 1) <= 128;
 }
 
 int few_forward(const FewArgs& args, const GateCall* gate, hipStream_t st)

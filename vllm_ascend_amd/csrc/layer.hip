@@ -362,6 +362,12 @@ extern "C" const char* moe355_layer_kernel_name(const moe355_layer* layer, int64
     return moe355_gmm_kernel_name(1, num_tokens * l.top_k, l.hidden, 2 * l.intermediate, l.num_experts);
 }
 
+extern "C" int moe355_layer_gates_inside(const moe355_layer* layer, int64_t num_tokens)
+{
+    if (check_layer(layer) != MOE355_OK || num_tokens <= 0) return 0;
+    return forms_of(*layer, num_tokens).few && few_gates(few_args(*layer, Buffers{}, num_tokens));
+}
+
 extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, const void* logits, int logits_dtype,
                                     int64_t num_tokens, void* out, void* workspace, size_t workspace_bytes,
                                     void* stream)
@@ -396,7 +402,7 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
         few = few_args(l, b, T);
         few.out = (uint16_t*)out;
     }
-    const bool gates_itself = f.few && few_gates(few, g);
+    const bool gates_itself = f.few && few_gates(few);
     if (!gates_itself) {
         rc = gate_quant_impl(f.small, g, 1, b.topk_weights, b.topk_ids, b.xq, b.x_scale, b.dst, b.row_token,
                              b.expert_tokens, l.sync_counter, l.shared ? b.one_group : nullptr, stream);

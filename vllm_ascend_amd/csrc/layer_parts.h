@@ -158,7 +158,7 @@ struct FewArgs {
 
 bool few_supported(const FewArgs& a);
 // whether few_forward takes the gating and the token quantisation of such a call as well
-bool few_gates(const FewArgs& a, const GateCall& g);
+bool few_gates(const FewArgs& a);
 // gate: the call that few_forward gates and quantises for itself (ids and weights go to a.ids and a.tw), or null
 int few_forward(const FewArgs& a, const GateCall* gate, hipStream_t st);
 
