@@ -432,3 +432,51 @@ def test_gating_inside_the_first_launch_where_it_is_short(experts, top_k, hidden
                    x_dtype=_lib.DT_BF16, pair_order=1, w13=256, s13=256, w2=256, s2=256)
     assert [lib.moe355_layer_gates_inside(ctypes.byref(a), T) for T in range(6)] == [int(1 <= T <= most) for T in range(6)]
     assert lib.moe355_layer_gates_inside(None, 1) == 0
+
+
+def _code_objects(data):
+    """Where the gfx code objects (ELF files for machine 224) inside a library start."""
+    at = data.find(b"\x7fELF", 4)
+    while at >= 0:
+        if int.from_bytes(data[at + 18:at + 20], "little") == 224:
+            yield at
+        at = data.find(b"\x7fELF", at + 4)
+
+
+def _kernel_metadata(path):
+    """name -> metadata of every kernel of the library, from the notes of its code objects."""
+    import struct
+
+    import msgpack
+
+    data, kernels = open(path, "rb").read(), {}
+    for at in _code_objects(data):
+        (sections,), (size, count) = struct.unpack_from("<Q", data, at + 40), struct.unpack_from("<2H", data, at + 58)
+        for i in range(count):
+            _, kind, _, _, offset, length = struct.unpack_from("<2I4Q", data, at + sections + i * size)
+            if kind != 7:  # SHT_NOTE
+                continue
+            end, p = at + offset + length, at + offset
+            while p < end:
+                name, desc, note = struct.unpack_from("<3I", data, p)
+                body = p + 12 + (name + 3) // 4 * 4
+                if note == 32:  # NT_AMDGPU_METADATA
+                    for k in msgpack.unpackb(data[body:body + desc])["amdhsa.kernels"]:
+                        kernels[k[".name"]] = k
+                p = body + (desc + 3) // 4 * 4
+    return kernels
+
+
+def test_few_token_down_product_leaves_registers_for_the_kernels_beside_it():
+    """96 registers for each of its four wavefronts of a SIMD and 128 for one of the routed gate_up product are the 512 that
+    there are; registers are handed out in eights."""
+    from vllm_ascend_amd import _lib
+
+    kernels = _kernel_metadata(_lib.LIB_PATH)
+    down = {n: k for n, k in kernels.items() if "few_down_kernel" in n}
+    beside = [k for n, k in kernels.items() if "gmm_stream_kernelILi1ELi4ELi4ELi3ELb0ELb1ELb1E" in n]
+    assert len(down) == 6 and len(beside) == 1
+    assert beside[0][".vgpr_count"] <= 128
+    for name, k in down.items():
+        assert k[".vgpr_count"] + k.get(".agpr_count", 0) <= 96, name
+        assert k[".private_segment_fixed_size"] == 0, name  # nothing spilled for it
