@@ -125,6 +125,13 @@ def test_dense_product_with_k_cut_over_the_wavefronts(R, Kd, N, family):
         assert np.array_equal(s.cpu().numpy().view(np.uint32)[:rows], s_want.view(np.uint32)[:rows])
 
 
+# ... narrow products: up to 704 workgroups in rows of eight
+@pytest.mark.parametrize("R,Kd,N,family", [(5632, 64, 64, "split"), (5633, 64, 64, "tiled"), (5632, 64, 512, "split"),
+                                           (5633, 64, 512, "tiled"), (3712, 64, 576, "tiled"), (2816, 64, 576, "split")])
+def test_narrow_dense_products_with_many_rows(R, Kd, N, family):
+    test_dense_product_with_k_cut_over_the_wavefronts(R, Kd, N, family)
+
+
 # ... whose rows are gathered from tokens beyond 4 GiB (and, by turns, from tokens in front of them)
 def test_dense_product_gathers_beyond_4_gib():
     from vllm_ascend_amd import kernels as K

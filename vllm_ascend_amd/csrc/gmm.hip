@@ -701,10 +701,17 @@ static bool dense_tiles(const GmmArgs& a)
 // DeepSeek-V3 shape with the shared expert in line, 128 / 192 / 256 / 512 / 1024 tokens 1767 / 1843 / 1882 / 1848 / 1964 us on
 // 128-row tiles, 1660 / 1697 / 1738 / 1828 / 1974 on these.  On a side stream the few workgroups of the 128-row tiles hide
 // behind the routed products and these do not: 100 / 200 / 400 tokens 1609 / 1712 / 1797 against 1620 / 1738 / 1813.
+// Narrow products reach that with many rows, where 64 x 64 tiles pass them around the chip too often (their grid is rounded up
+// to eight columns, one for every XCD): us on 128-row tiles / on these at N / K, with the workgroups in brackets, 512 / 7168 at
+// 4000 / 6000 rows 52 / 40 (504) and 53 / 57 (752), 512 / 2048 at 6000 / 8000 22.4 / 21.1 (752) and 23.7 / 26.1 (1000), 1024 /
+// 2048 at 3000 / 4000 21.2 / 18.3 (752) and 22.1 / 22.5 (1008), 128 / 8192 at 6000 / 16000 58 / 53 (752) and 66 / 130 (2000), 64 /
+// 2048 at 4000 / 12000 20.7 / 14.2 (504) and 25.2 / 31.3 (1504); but 2048 / 7168 at 2000 63 / 60 (1024), 4096 / 7168 at 1000 66 /
+// 61 (1024).
 static bool split_tiles(const GmmArgs& a)
 {
     if (a.E != 1 || a.beside || a.K % 64 != 0 || a.R <= 64 || a.R * (int64_t)a.K >= (1ll << 31) || dense_tiles(a)) return false;
-    return ((a.R + 127) / 128) * ((a.N + 255) / 256) < kComputeUnits / 2;
+    const int64_t workgroups = (a.R + 63) / 64 * ((a.N / 64 + 7) / 8 * 8);
+    return ((a.R + 127) / 128) * ((a.N + 255) / 256) < kComputeUnits / 2 && (a.N >= 2048 || workgroups <= 704);
 }
 
 static size_t tiled_ws_max(int64_t rows, int E)
