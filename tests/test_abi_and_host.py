@@ -480,3 +480,16 @@ def test_few_token_down_product_leaves_registers_for_the_kernels_beside_it():
     for name, k in down.items():
         assert k[".vgpr_count"] + k.get(".agpr_count", 0) <= 96, name
         assert k[".private_segment_fixed_size"] == 0, name  # nothing spilled for it
+
+
+# a product that streams with workgroups for at most half of the chip (128, of 64 channels) reads its weights twice for
+# nothing: tiles from 48 rows per expert instead of 32, if K is long enough for it to matter
+@pytest.mark.parametrize("experts, k, n, first", [(16, 1024, 512, 48), (16, 960, 512, 32), (16, 1024, 576, 32), (8, 4096, 1024, 48),
+                                                  (8, 4096, 1088, 32), (4, 7168, 2048, 48), (20, 2048, 384, 48)])
+def test_few_streaming_workgroups_keep_streaming(experts, k, n, first):
+    from vllm_ascend_amd import _lib
+
+    name = _lib.load().moe355_gmm_kernel_name
+    for epilogue in (0, 1, 2):
+        assert name(epilogue, first * experts - 1, k, n, experts) == b"gmm_stream_kernel"
+        assert name(epilogue, first * experts, k, n, experts) == b"gmm_tiled_kernel"

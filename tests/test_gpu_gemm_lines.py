@@ -176,6 +176,12 @@ def test_few_rows_on_tiles(R, family):
     test_families_on_both_sides_of_a_line(R, 16, 192, 320, family, True)
 
 
+# ... and 47 / 48 where streaming has workgroups for half of the chip at most
+@pytest.mark.parametrize("R,family", [(48 * 16 - 1, "stream"), (48 * 16, "tiled")])
+def test_few_rows_on_tiles_few_channels(R, family):
+    test_families_on_both_sides_of_a_line(R, 16, 1024, 512, family, True)
+
+
 # 64 rows per expert at a long K: as many columns of wide tiles as half of the compute units, and one less
 @pytest.mark.parametrize("E,family", [(63, "tiled"), (64, "wide")])
 def test_columns_of_wide_tiles(E, family):
