@@ -505,6 +505,8 @@ int moe355_profile_next_gemm(void *start_event, void *stop_event);
  * epilogue: 0 raw int32 (moe355_gmm_i32), 1 SwiGLU (moe355_gmm1_swiglu_quant), 2 dequant (moe355_gmm2_dequant).
  * A pure function of its arguments, for benchmarks and profiles (no counterpart in the reference). */
 const char *moe355_gmm_kernel_name(int epilogue, int64_t rows, int64_t k, int64_t n, int num_experts);
+/* ... and the most rows of one of its tiles: 0 where it streams. */
+int moe355_gmm_tile_rows(int64_t rows, int64_t k, int64_t n, int num_experts);
 
 /* ---------------------------------------------------------------------------
  * The whole layer in one call: (router gate,) gating, dispatch, expert MLPs, shared expert and combine, enqueued

@@ -163,6 +163,18 @@ def test_tiles_of_half_the_height_for_few_experts(R, E, Kd, N):
     test_families_on_both_sides_of_a_line(R, E, Kd, N, "tiled", True)
 
 
+# ... the last row of the line and the first one behind it: half a tile for the last one of up to 16 experts, three quarters
+# of more
+@pytest.mark.parametrize("E,R,Kd,N", [(8, 3903, 64, 1024), (16, 3647, 64, 1024), (17, 3391, 64, 1024), (24, 959, 64, 2048)])
+def test_half_the_height_up_to_a_full_chip(E, R, Kd, N):
+    from vllm_ascend_amd._lib import load
+
+    height = load().moe355_gmm_tile_rows
+    assert height(R, Kd, N, E) == 64 and height(R + 1, Kd, N, E) == 128
+    for rows in (R, R + 1):
+        test_families_on_both_sides_of_a_line(rows, E, Kd, N, "tiled", True)
+
+
 # ... with three, two and one row at a time in a wavefront's registers: on both sides of 768 and of 1024 values, a last load
 # that is not full, up to eight rows per expert, an expert with a row of every token (several passes of 32 rows)
 @pytest.mark.parametrize("T,E,I", [(128, 128, 768), (128, 128, 736), (33, 128, 544), (56, 128, 800), (56, 128, 1024), (56, 128, 1056)])

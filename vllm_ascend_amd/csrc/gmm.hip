@@ -654,8 +654,14 @@ static int tiled_bm(const GmmArgs& a)
     // many and half as long (rows / 64 and half a tile per expert for its last one).  8 experts of 2816 x 1024 and 1024 x
     // 1408, the layer at 512 / 768 / 1024 / 1536 tokens of two slots 50.8 / 51.5 / 52.5 / 62.6 us on 128-row tiles, 41.7 /
     // 46.5 / 49.1 / 59.9 with this rule (2048 tokens, where it would be one tile too many for the down product: 65.8
-    // against 67.2).  Products of up to 512 channels, a handful of workgroups in any family, were not measured and stay.
-    if (a.E > 1 && a.N > 512 && (a.R / 64 + a.E / 2) * ((a.N + 255) / 256) <= kComputeUnits) return 64;
+    // against 67.2).  Half a tile per expert is what a uniform batch needs; under skewed routing nearly every expert has a last
+    // tile of its own, and where that makes one more than the chip holds the launch takes twice as long.  With up to 16
+    // experts it makes few (small layer under Zipf(1.1), 576 / 639 / 1900 tokens 48.4 / 50.9 / 62.4 us with this rule, 51.4 /
+    // 51.6 / 65.0 on 128-row tiles); beyond, three quarters are taken: 24 experts of 7168 x 2048, 48 rows each under Zipf(1.1)
+    // 68 us on 128-row tiles, 111 on 64-row tiles, 64 of 4096 x 768, 40 rows each 42 against 64, while uniform batches lose 3 %
+    // there.  Products of up to 512 channels stay where they were (below).
+    const int64_t last_tiles = a.E <= 16 ? a.E / 2 : 3 * (int64_t)a.E / 4;
+    if (a.E > 1 && a.N > 512 && (a.R / 64 + last_tiles) * ((a.N + 255) / 256) <= kComputeUnits) return 64;
     // the list of 256-row tiles is built from 16-bit counters (tile_map_kernel, by_length)
     const bool wide_ok = a.R / 256 + a.E < 32768;
     // K = 7168 / 2048, uniform routing, 28 / 40 / 48 / 56 / 64 / 94 rows per expert: the layer takes 1968 / 2028 / 2055 /
@@ -841,6 +847,17 @@ extern "C" const char* moe355_gmm_kernel_name(int epilogue, int64_t rows, int64_
     if (split_tiles(a)) return "gmm_split_kernel";
     const int bm = gemm_family(a, true);  // as launch_gemm_auto decides
     return bm == 256 ? "gmm_wide_kernel" : bm ? "gmm_tiled_kernel" : "gmm_stream_kernel";
+}
+
+extern "C" int moe355_gmm_tile_rows(int64_t rows, int64_t k, int64_t n, int num_experts)
+{
+    if (rows <= 0 || k <= 0 || n <= 0 || num_experts <= 0) return 0;
+    GmmArgs a = {};
+    a.R = rows;
+    a.K = (int)k;
+    a.N = (int)n;
+    a.E = num_experts;
+    return dense_tiles(a) ? 256 : split_tiles(a) ? 64 : gemm_family(a, true);
 }
 
 extern "C" int moe355_format_cast_nz(const int8_t* w, int layout, int64_t num_experts, int64_t n, int64_t k,
