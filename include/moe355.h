@@ -460,6 +460,9 @@ int moe355_token_unpermute(const void *permuted, int dtype, const int32_t *sorte
 int moe355_pair_order(int64_t num_tokens, int top_k, int num_logits, int num_experts, int64_t hidden,
                       int64_t intermediate);
 int moe355_gmm_pairs_supported(int64_t num_tokens, int top_k, int64_t n, int64_t k);
+/* How many further 32-row blocks of the hot experts the gate_up product of such a call starts early, in front of the other
+ * experts (the rest runs at the end).  A pure function of its arguments, for profiles (no counterpart in the reference). */
+int moe355_pair_blocks_in_front(int64_t num_pairs, int64_t n, int num_experts);
 size_t moe355_gmm1_swiglu_quant_pairs_workspace(int64_t num_tokens, int top_k, int64_t n);
 int moe355_gmm1_swiglu_quant_pairs(const int8_t *x, const float *x_scale, const int32_t *topk_ids, int64_t num_tokens,
                                    int top_k, const int8_t *weight_nz, const float *weight_scale, int64_t k,

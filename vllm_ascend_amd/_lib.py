@@ -117,6 +117,7 @@ PROTOTYPES = {
                                                   c_int64, c_int, c_void_p, c_int, c_void_p]),
     "moe355_token_unpermute_pairs": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_int64, c_int, c_int64, c_int,
                                              c_void_p, c_void_p, c_void_p, c_void_p]),
+    "moe355_pair_blocks_in_front": (c_int, [c_int64, c_int64, c_int]),
     "moe355_pair_order": (c_int, [c_int64, c_int, c_int, c_int, c_int64, c_int64]),
     "moe355_layer_workspace": (c_size_t, [c_void_p, c_int64]),
     "moe355_layer_forward": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int64, c_void_p, c_void_p, c_size_t,

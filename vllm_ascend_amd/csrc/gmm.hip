@@ -1132,13 +1132,21 @@ extern "C" int moe355_pair_order(int64_t num_tokens, int top_k, int num_logits, 
 // routing unchanged.  From 48 units on the passes hide among the other workgroups until the hot experts have a few blocks
 // each: DeepSeek-V3 shape, gate_up product (64 units), Zipf(1.1), 33 / 50 / 64 / 90 tokens of eight slots 345 / 417 / 453 / 589 us
 // in passes, 347 / 414 / 448 / 573 in workgroups (uniform 40 / 64 / 96 tokens 1234 / 1467 / 1610 and 1235 / 1468 / 1610); its down
-// product (112 units) is the same either way.
+// product (112 units) is the same either way.  32 experts of 2880 / 2880 (90 units), four slots, Zipf(1.1), 96 / 127 / 200 tokens
+// 168 / 204 / 269 in passes, 154 / 181 / 234 in workgroups, uniform 148 / 157 / 193 and 148 / 157 / 194.
 // Those are the longest workgroups of the launch, and at the end of the grid the chip waits for them; but there are
 // places for as many as R pairs could need, and in front of the slots an unused one delays them.  So as many as skewed
 // routing usually needs, one for every 56 pairs, run in front and the others at the end.  Qwen3 shape, 40 / 64 / 100 / 127
 // tokens, all at the end / so / one for every 32 pairs in front: Zipf(1.1) 67.3 / 75.3 / 86.8 / 94.5 against 64.4 / 71.0 / 81.5
 // / 90.5 against 63.7 / 70.8 / 82.4 / 88.6 us, uniform routing 103.2 / 108.0 / 110.2 / 111.5 against 103.3 / 108.0 / 110.3 /
 // 111.8 against 103.3 / 108.2 / 110.8 / 112.8.
+// In front of slots that start behind places of their own, they cost a lookup that the slots of a short launch have to wait for:
+// all at the end / so, 48 / 64 / 127 tokens of eight slots, 128 experts of 512 / 256 (1024 units in both products) uniform 30.0 /
+// 30.2 / 30.9 against 33.2 / 33.4 / 34.0, Zipf(1.1) 28.6 / 28.8 / 30.8 against 28.3 / 28.7 / 31.4, 64 experts of 512 / 512 (1024,
+// 512) uniform 27.9 / 28.4 / 30.5 against 29.2 / 29.8 / 31.8, Zipf 28.9 / 29.8 / 34.9 against 28.6 / 29.9 / 35.2; 128 experts of
+// 1024 / 512 (2048, 2048) uniform 49.1 / 49.9 / 52.3 against 49.6 / 50.4 / 54.3, Zipf 43.2 / 46.2 / 53.6 against 41.1 / 43.6 / 52.2.
+// So from 2048 units on; without places every slot makes that lookup, and nothing waits (256 experts of 1024 / 256, 127 tokens of
+// four slots uniform 47.2 against 46.7, Zipf 33.8 against 30.8).
 // The lookups hold 2048 experts.
 static int pair_places(GmmArgs& a, int resident_units)
 {
@@ -1152,7 +1160,8 @@ static int pair_places(GmmArgs& a, int resident_units)
         a.pair_slots = a.R < (int64_t)rest ? (int)a.R : rest;
         // an expert of c rows has (c - 1) / 32 further blocks: over all experts at most (R - 1) / 32
         if (a.N / 64 < (a.R < 384 ? 48 : 96)) a.pair_extra = (int)((a.R - 1) / 32);
-        a.pair_early = a.R / 56 < a.pair_extra ? (int)(a.R / 56) : a.pair_extra;
+        if (a.pair_first == 0 || (int64_t)a.E * (a.N / 64) >= 2048)
+            a.pair_early = a.R / 56 < a.pair_extra ? (int)(a.R / 56) : a.pair_extra;
     }
     return a.sh_blocks + a.pair_first + a.pair_slots + a.pair_extra;
 }
@@ -1165,6 +1174,17 @@ extern "C" size_t moe355_gmm1_swiglu_quant_pairs_workspace(int64_t num_tokens, i
 
 // gate_up GEMM + SwiGLU in pair order: fp32 values to y, and with `out` the re-quantised rows.  The weights are one
 // tensor (w.one) or per-expert tensors (w.list and w.scale_list).
+extern "C" int moe355_pair_blocks_in_front(int64_t num_pairs, int64_t n, int num_experts)
+{
+    if (num_pairs <= 0 || num_pairs > kPairMax || n <= 0 || n % 64 || num_experts <= 0) return 0;
+    GmmArgs a = {};
+    a.R = num_pairs;
+    a.N = (int)n;
+    a.E = num_experts;
+    pair_places(a, 768);
+    return a.pair_early;
+}
+
 int moe355::gmm1_pairs_impl(const int8_t* x, const float* x_scale, const int32_t* topk_ids, int64_t num_tokens,
                             int top_k, const PairWeights& w, int64_t k, int64_t n, int num_experts, float swiglu_limit,
                             float* y, int8_t* out, float* out_scale, void* stream, const PairShared* shared)
