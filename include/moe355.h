@@ -475,8 +475,9 @@ int moe355_gmm2_dequant_pairs(const int8_t *x, const int8_t *weight_nz, const fl
  * gmm2 takes them as its activation (K = N/2 of gmm1) and every workgroup quantises the rows of its expert itself
  * (the arithmetic of the re-quantisation of moe355_gmm1_swiglu_quant), so that a decode layer is four launches.
  * moe355_gmm2_requant_pairs_supported() != 0: many units of work, a short K (k < 2048, 32 rows of k + 16 bytes
- * in LDS) and at most three and a half pairs per expert on average -- a small decode batch over many small experts, where a
- * launch costs more than the repeated quantisation. */
+ * in LDS) and at most three and a half pairs per expert on average, or eight where k <= 768 and the further 32-row blocks of
+ * a hot expert are workgroups of their own (n < 3072, or n < 6144 from 384 pairs on) -- a decode batch over many small
+ * experts, where a launch costs more than the repeated quantisation. */
 int moe355_gmm1_swiglu_pairs(const int8_t *x, const float *x_scale, const int32_t *topk_ids, int64_t num_tokens,
                              int top_k, const int8_t *weight_nz, const float *weight_scale, int64_t k, int64_t n,
                              int num_experts, float swiglu_limit, float *y, void *stream);

@@ -504,3 +504,17 @@ def test_further_blocks_in_front_of_the_slots(experts, n, pairs, blocks):
     from vllm_ascend_amd import _lib
 
     assert _lib.load().moe355_pair_blocks_in_front(pairs, n, experts) == blocks
+
+
+# the re-quantisation inside the down product: three and a half pairs per expert, eight with short rows if the hot experts'
+# rows are not taken in passes
+@pytest.mark.parametrize("experts, top_k, n, k, most", [(32, 4, 4096, 768, 28), (64, 6, 4096, 640, (37, 64, 85)), (64, 8, 2048, 768, 64),
+                                                        (64, 8, 2048, 800, 28), (128, 8, 2048, 768, 128), (128, 8, 6144, 256, 56),
+                                                        (128, 8, 4096, 256, 128)])
+def test_re_quantisation_inside_the_down_product(experts, top_k, n, k, most):
+    from vllm_ascend_amd import _lib
+
+    supported = _lib.load().moe355_gmm2_requant_pairs_supported
+    first, again, last = most if isinstance(most, tuple) else (most, most, most)
+    for T in range(1, 1024 // top_k + 1):
+        assert bool(supported(T, top_k, n, k, experts)) == (T <= first or again <= T <= last), T

@@ -1117,6 +1117,9 @@ extern "C" int moe355_pair_order(int64_t num_tokens, int top_k, int num_logits, 
     return pair_order_impl(num_tokens, top_k, num_logits, num_experts, hidden, intermediate, false);
 }
 
+// whether a hot expert's further blocks of 32 rows are workgroups of their own (pair_places)
+static bool blocks_of_their_own(int64_t pairs, int64_t n) { return n / 64 < (pairs < 384 ? 48 : 96); }
+
 // pair order: the places of the grid.
 // A place per expert lets a workgroup request its first weight tiles before it has seen a single id, and makes every
 // idle expert cost the dispatch of its workgroups plus 32 KiB of weights requested for nothing.  A slot (the kernel
@@ -1159,7 +1162,7 @@ static int pair_places(GmmArgs& a, int resident_units)
         const int rest = a.E - a.pair_first;
         a.pair_slots = a.R < (int64_t)rest ? (int)a.R : rest;
         // an expert of c rows has (c - 1) / 32 further blocks: over all experts at most (R - 1) / 32
-        if (a.N / 64 < (a.R < 384 ? 48 : 96)) a.pair_extra = (int)((a.R - 1) / 32);
+        if (blocks_of_their_own(a.R, a.N)) a.pair_extra = (int)((a.R - 1) / 32);
         if (a.pair_first == 0 || (int64_t)a.E * (a.N / 64) >= 2048)
             a.pair_early = a.R / 56 < a.pair_extra ? (int)(a.R / 56) : a.pair_extra;
     }
@@ -1327,13 +1330,19 @@ extern "C" int moe355_gmm2_requant_pairs_supported(int64_t num_tokens, int top_k
     const int64_t units = (int64_t)num_experts * (n / 64);
     if (!(units >= 2048 && k < 2048 && (n / 64) % 4 == 0 && k % 4 == 0 && 32 * (k + 16) <= 48 * 1024)) return 0;
     // Every workgroup of an expert quantises all its rows again.  Rows of up to 768 values go three at a time through a
-    // wavefront's registers, and then it pays for all of pair order (eight rows per expert).  128 experts of 2048 x 768, the
-    // layer in us with the launch of its own / one row at a time / three: uniform routing 24 / 48 / 64 / 96 / 127 tokens of eight
-    // slots 92.7 / 108.0 / 109.1 / 111.9 / 114.0 against 91.3 / 105.9 / - / - / - against 91.3 / 105.7 / 106.9 / 109.2 / 111.4;
-    // Zipf(1.1), 16 / 32 / 50 / 64 / 96 / 127 tokens 47.9 / 54.9 / - / 77.4 / 90.3 / 98.2 against 46.2 / 58.5 / 72.4 / - / - / -
-    // against 45.0 / 56.0 / 70.2 / 76.3 / 88.6 / 94.8.  Longer rows: up to three and a half rows per expert (two at a time up to
-    // 1024 values, one beyond).
-    return num_tokens * top_k * 2 <= (k <= 768 ? 16 : 7) * (int64_t)num_experts;
+    // wavefront's registers, and then it pays up to eight rows per expert.  128 experts of 2048 x 768, the layer in us with
+    // the launch of its own / one row at a time / three: uniform routing 24 / 48 / 64 / 96 / 127 tokens of eight slots 92.7 /
+    // 108.0 / 109.1 / 111.9 / 114.0 against 91.3 / 105.9 / - / - / - against 91.3 / 105.7 / 106.9 / 109.2 / 111.4; Zipf(1.1), 16
+    // / 32 / 50 / 64 / 96 / 127 tokens 47.9 / 54.9 / - / 77.4 / 90.3 / 98.2 against 46.2 / 58.5 / 72.4 / - / - / - against 45.0 /
+    // 56.0 / 70.2 / 76.3 / 88.6 / 94.8.  Shorter rows gain less: 128 experts of 2048 x 320, 64 / 127 tokens uniform 60.7 / 63.9
+    // against 59.6 / 62.1, Zipf 48.0 / 58.6 against 50.3 / 59.5; of 1024 x 256, 160 tokens of four slots 36.4 against 34.1, Zipf
+    // 35.2 against 36.7.  Longer rows: up to three and a half rows per expert (two at a time up to 1024 values, one beyond).
+    // So are experts of many channels with few pairs, whose hot ones take their rows in passes: there the re-quantisation
+    // stands in front of every pass.  32 experts of 4096 x 768, four slots, Zipf(1.1), 40 / 64 / 80 tokens 69.4 / 75.3 / 84.3
+    // against 70.9 / 80.6 / 92.0 (uniform 65.6 / 66.2 / 66.7 against 63.0 / 64.1 / 64.8), 112 tokens, which is more than 384
+    // pairs, 80.2 against 78.0.
+    const int64_t pairs = num_tokens * top_k;
+    return pairs * 2 <= (k <= 768 && blocks_of_their_own(pairs, n) ? 16 : 7) * (int64_t)num_experts;
 }
 
 extern "C" int moe355_gmm2_requant_dequant_pairs(const float* y, const int8_t* weight_nz, const float* scale,
