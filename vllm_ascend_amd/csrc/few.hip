@@ -449,6 +449,7 @@ __global__ __launch_bounds__(NT, 5) void few_down_kernel(FewArgs a)
             const float m = few_row_max<false>(a, r, few_row_pieces(a, r, lane), lane);
             if (lane == 0) qdv[r] = m;
         }
+        wave_lds_order();
 #pragma unroll
         for (int j = 0; j < NV; ++j) asm volatile("" : "+v"(yv[j]));
     }

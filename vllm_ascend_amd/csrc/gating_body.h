@@ -370,9 +370,7 @@ __device__ __forceinline__ void row_scores(const RowLogits<DT>& logits, const vo
 #pragma unroll
         for (int i = 0; i < PER; ++i)
             if (lane + 64 * i < E) grp_lds[lane + 64 * i] = sel[i];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_order();
         unsigned gu = 0u;
         if (butterfly_groups<PER>(sel, gs)) gu = score_order(group_scores_butterfly<PER>(sel, gs, mode, lane));
         else if (lane < G) gu = score_order(group_score(grp_lds + lane * gs, gs, mode));

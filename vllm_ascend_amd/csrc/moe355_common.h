@@ -177,6 +177,15 @@ __device__ __forceinline__ float wave_max(float v)
     return v;
 }
 
+// What the lanes of a wavefront wrote to LDS before it, the others read behind it (and write over only behind it): no
+// instruction, the LDS answers a wavefront in order, but the compiler has to keep that order as well.
+__device__ __forceinline__ void wave_lds_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Butterfly sum: every lane receives the same value; the order of additions is part of the arithmetic contract
 // (partial[l] + partial[l ^ off], off = 32 .. 1).  No LDS round trips: halves and rows change places by the lane swaps,
 // lane l ^ 8 is row_ror:8, and for off = 4 row_ror:4 names lane l ^ 4 or l ^ 12, which hold the same value by then.
