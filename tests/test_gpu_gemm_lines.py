@@ -125,9 +125,10 @@ def test_dense_product_with_k_cut_over_the_wavefronts(R, Kd, N, family):
         assert np.array_equal(s.cpu().numpy().view(np.uint32)[:rows], s_want.view(np.uint32)[:rows])
 
 
-# ... narrow products: up to 704 workgroups in rows of eight
-@pytest.mark.parametrize("R,Kd,N,family", [(5632, 64, 64, "split"), (5633, 64, 64, "tiled"), (5632, 64, 512, "split"),
-                                           (5633, 64, 512, "tiled"), (3712, 64, 576, "tiled"), (2816, 64, 576, "split")])
+# ... narrow products: up to 768 workgroups in rows of eight, 1024 if K is short
+@pytest.mark.parametrize("R,Kd,N,family", [(6144, 1088, 64, "split"), (6145, 1088, 64, "tiled"), (3072, 1088, 576, "split"),
+                                           (3073, 1088, 576, "tiled"), (8192, 64, 64, "split"), (8193, 64, 64, "tiled"),
+                                           (4096, 128, 576, "split"), (4097, 128, 576, "tiled")])
 def test_narrow_dense_products_with_many_rows(R, Kd, N, family):
     test_dense_product_with_k_cut_over_the_wavefronts(R, Kd, N, family)
 

@@ -717,14 +717,15 @@ static bool dense_tiles(const GmmArgs& a)
 // Narrow products reach that with many rows, where 64 x 64 tiles pass them around the chip too often (their grid is rounded up
 // to eight columns, one for every XCD): us on 128-row tiles / on these at N / K, with the workgroups in brackets, 512 / 7168 at
 // 4000 / 6000 rows 52 / 40 (504) and 53 / 57 (752), 512 / 2048 at 6000 / 8000 22.4 / 21.1 (752) and 23.7 / 26.1 (1000), 1024 /
-// 2048 at 3000 / 4000 21.2 / 18.3 (752) and 22.1 / 22.5 (1008), 128 / 8192 at 6000 / 16000 58 / 53 (752) and 66 / 130 (2000), 64 /
-// 2048 at 4000 / 12000 20.7 / 14.2 (504) and 25.2 / 31.3 (1504); but 2048 / 7168 at 2000 63 / 60 (1024), 4096 / 7168 at 1000 66 /
-// 61 (1024).
+// 4096 at 3000 / 4000 33.0 / 28.6 (752) and 35.1 / 36.4 (1008), 128 / 8192 at 6000 / 16000 58 / 53 (752) and 66 / 130 (2000),
+// 64 / 2048 at 4000 / 12000 20.7 / 14.2 (504) and 25.2 / 31.3 (1504).  With a short K there is less to pass: 256 / 256 at 8000 /
+// 16000 13.6 / 10.4 (1000) and 16.6 / 18.3 (2000), 512 / 1024 at 8000 17.7 / 18.1 (1000; with SwiGLU 26.7 / 22.4); and with more
+// channels: 2048 / 7168 at 2000 63 / 60 (1024), 4096 / 7168 at 1000 66 / 61 (1024).
 static bool split_tiles(const GmmArgs& a)
 {
     if (a.E != 1 || a.beside || a.K % 64 != 0 || a.R <= 64 || a.R * (int64_t)a.K >= (1ll << 31) || dense_tiles(a)) return false;
     const int64_t workgroups = (a.R + 63) / 64 * ((a.N / 64 + 7) / 8 * 8);
-    return ((a.R + 127) / 128) * ((a.N + 255) / 256) < kComputeUnits / 2 && (a.N >= 2048 || workgroups <= 704);
+    return ((a.R + 127) / 128) * ((a.N + 255) / 256) < kComputeUnits / 2 && (a.N >= 2048 || workgroups <= (a.K <= 1024 ? 1024 : 768));
 }
 
 static size_t tiled_ws_max(int64_t rows, int E)
