@@ -503,9 +503,10 @@ int moe355_token_unpermute_pairs(const void *rows, int dtype, const void *probs,
 int moe355_profile_next_gemm(void *start_event, void *stop_event);
 
 /* Which kernel family the int8 grouped GEMMs above launch for a shape, given a workspace of the size their
- * moe355_*_workspace() asks for: "gmm_stream_kernel" (few rows per expert), "gmm_tiled_kernel" (128-row
- * LDS-tiled), "gmm_wide_kernel" (weight-streaming tiles of up to 256 rows) or "gmm_dense_kernel" (one expert
- * with thousands of rows: 256 x 256 tiles, no tile map); "" for arguments no GEMM accepts.
+ * moe355_*_workspace() asks for: "gmm_stream_kernel" (few rows per expert), "gmm_tiled_kernel" (64- or 128-row
+ * LDS-tiled), "gmm_wide_kernel" (weight-streaming tiles of up to 256 rows), "gmm_split_kernel" (one expert with some
+ * hundreds of rows: 64 x 64 tiles that cut K over their wavefronts, no tile map) or "gmm_dense_kernel" (one expert with
+ * thousands of rows: 256 x 256 tiles, no tile map); "" for arguments no GEMM accepts.
  * epilogue: 0 raw int32 (moe355_gmm_i32), 1 SwiGLU (moe355_gmm1_swiglu_quant), 2 dequant (moe355_gmm2_dequant).
  * A pure function of its arguments, for benchmarks and profiles (no counterpart in the reference). */
 const char *moe355_gmm_kernel_name(int epilogue, int64_t rows, int64_t k, int64_t n, int num_experts);
@@ -527,7 +528,9 @@ typedef struct moe355_layer {
     int32_t x_dtype;          /* of hidden states, result and routing weights */
     const void *bias;         /* [E] in the dtype of the logits, or NULL */
     int32_t weights;          /* 0: int8 tensors; 1: device tables of per-expert int8 tensors; 2: int4 tensors */
-    int32_t pair_order;       /* 0: never; 1: where moe355_pair_order() says so (weights 0 and 1) */
+    int32_t pair_order;       /* 0: never; 1: where moe355_pair_order() says so (weights 0 and 1), and up to 256 MiB of
+                               * repeated weight reads instead of 128 where a shared expert of a routed expert's shape rides in
+                               * the same launches; int4: up to 40 tokens */
     const void *w13, *s13, *w2, *s2;
     int64_t group13, group2;  /* int4: weights along K that share a scale */
     /* of moe355_route_quant_small, for a caller that runs the layer on one stream or graph at a time; NULL: that launch

@@ -158,7 +158,7 @@ def test_dense_product_gathers_beyond_4_gib():
     assert torch.equal(q, q_want) and torch.equal(s.view(torch.int32), s_want.view(torch.int32))
 
 
-# few experts: 64-row tiles as long as they do not outnumber the compute units, on both sides of the line
+# few experts: 64-row tiles as long as they do not outnumber the compute units, and 128-row tiles
 @pytest.mark.parametrize("R,E,Kd,N", [(1024, 8, 192, 1024), (3904, 8, 64, 1024), (3968, 8, 64, 1024), (1030, 3, 128, 2816)])
 def test_tiles_of_half_the_height_for_few_experts(R, E, Kd, N):
     test_families_on_both_sides_of_a_line(R, E, Kd, N, "tiled", True)

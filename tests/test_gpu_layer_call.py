@@ -20,7 +20,7 @@ def _pair(name, tokens, shape=None, **kw):
     return cfg, build_layer(cfg, d, DEV, **kw), d["x"].to(DEV), d["logits"].to(DEV)
 
 
-# one token; the borders of the form for a few tokens (16 pairs, 64 with a shared expert), of pair order (three pairs per expert, 1024
+# one token; the borders of the form for a few tokens (32 pairs, 64 with a shared expert), of pair order (three pairs per expert, 1024
 # pairs) and of the one-launch index maps (4096 pairs); a batch with a ragged end on the sorted path
 @pytest.mark.parametrize("tokens", [1, 4, 5, 8, 9, 24, 25, 127, 128, 129, 512, 513, 1031])
 @pytest.mark.parametrize("name", ["c2_small", "c4_small", "c5_small"])
@@ -166,8 +166,8 @@ def test_further_blocks_around_the_slots(tokens, shape):
     assert torch.equal(got, layer(x, hot))
 
 
-# few experts: the last batch in pair order, and the first whose experts would read 128 MiB again (or have 36 rows each);
-# with a shared expert in the same launches 256 MiB, which neither reaches
+# few experts: the last batch in pair order, and the first whose experts would read 128 MiB again (or have 36 rows each), by
+# the operators' line; with a shared expert in the same launches the layer's lies at 256 MiB, which neither reaches
 @pytest.mark.parametrize("shape, tokens", [(dict(E=8, k=2, H=1024, I=1408), 497), (dict(E=16, k=2, H=2048, I=1408), 288)])
 @pytest.mark.parametrize("shared", [False, True])
 def test_few_experts_with_many_rows_are_sorted(shape, tokens, shared):

@@ -5,7 +5,7 @@
 //
 //   few_up_kernel    gate_up GEMM + SwiGLU of the routed experts AND of the shared expert, and the maxima of every row
 //                    piece (atomics on one maximum per row meet at the memory side: 1536 of them cost 12 us);
-//   few_down_kernel  re-quantisation, down GEMM and the weighted combine: a workgroup owns 16 output channels of ALL
+//   few_down_kernel  re-quantisation, down GEMM and the weighted combine: a workgroup owns 16 (or 8) output channels of ALL
 //                    pairs, so the k rows of a token meet in its LDS and leave as one finished row.
 //
 // From about 12 K SwiGLU values on every workgroup re-quantising all rows costs more than a launch (few_quant_kernel).

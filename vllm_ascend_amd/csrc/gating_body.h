@@ -5,8 +5,10 @@
 // logits row is read with coalesced loads and the softmax sum follows the
 // contract order: strided per-lane partials, then a butterfly.  Group scores
 // go through a per-wavefront LDS copy of the selection scores (a group's
-// experts are spread over lanes); group and expert selection are repeated
-// wavefront arg-max reductions with the "larger value, then lower index" order.
+// experts are spread over lanes).  The order is always "larger value, then lower
+// index".  Groups: repeated arg-max reductions in gate_row, a count of the groups
+// in front of each in row_scores.  Experts: repeated arg-max reductions, or ranks
+// counted by several wavefronts (rank_row) where a launch waits for one row.
 #pragma once
 
 #include "layer_parts.h"

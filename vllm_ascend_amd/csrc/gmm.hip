@@ -86,10 +86,10 @@ constexpr int kPairMax = 1024;
 constexpr int kPairExperts = 2048;  // that the lookups of the slots can hold
 
 // REQ (pair order, down GEMM): the activation is still the fp32 SwiGLU output; the workgroup re-quantises the rows
-// of its expert itself, 32 at a time, into LDS (row maximum through LDS atomics on the bit patterns, which order
-// like the non-negative values; then rint(v * (1 / (max / 127))), the arithmetic of swiglu_requant_kernel) and the
-// MFMA operands come from there: the re-quantisation launch and its int8 round trip disappear.  The eight
-// workgroups of an expert each do it again for the expert's few rows, which is nothing next to a launch.
+// of its expert itself, 32 at a time, into LDS (a wavefront holds whole rows in registers: their maximum by a butterfly, then
+// rint(v * (1 / (max / 127))), the arithmetic of swiglu_requant_kernel) and the MFMA operands come from there: the
+// re-quantisation launch and its int8 round trip disappear.  The workgroups of an expert (one for every 256 channels) each
+// do it again for the expert's rows.
 // REQ_ROWS: rows that a wavefront re-quantises at a time, REQ_VEC: 256 values of each are held (K <= 256 REQ_VEC).
 template <int EPI, int KSPLIT, int UN, int OCC, bool SLABS = false, bool EARLY = true, bool PAIRS = false,
           int REQ_ROWS = 0, int REQ_VEC = 8>
@@ -659,7 +659,7 @@ static int tiled_bm(const GmmArgs& a)
     // experts it makes few (small layer under Zipf(1.1), 576 / 639 / 1900 tokens 48.4 / 50.9 / 62.4 us with this rule, 51.4 /
     // 51.6 / 65.0 on 128-row tiles); beyond, three quarters are taken: 24 experts of 7168 x 2048, 48 rows each under Zipf(1.1)
     // 68 us on 128-row tiles, 111 on 64-row tiles, 64 of 4096 x 768, 40 rows each 42 against 64, while uniform batches lose 3 %
-    // there.  Products of up to 512 channels stay where they were (below).
+    // there.  Not for products of up to 512 channels (below).
     const int64_t last_tiles = a.E <= 16 ? a.E / 2 : 3 * (int64_t)a.E / 4;
     if (a.E > 1 && a.N > 512 && (a.R / 64 + last_tiles) * ((a.N + 255) / 256) <= kComputeUnits) return 64;
     // the list of 256-row tiles is built from 16-bit counters (tile_map_kernel, by_length)
@@ -679,8 +679,14 @@ static int tiled_bm(const GmmArgs& a)
     // pays from K = 1024 on if the experts are about equally popular and there are enough of them to fill the chip.  128
     // experts, K = 2048 / 768, the layer at 100 / 112 / 128 / 144 / 160 / 192 rows per expert: 201 / 210 / 224 / 241 / 260 /
     // 280 us with the wide tiles in the first product, 193 / 212 / 232 / 250 / 253 / 264 us on 128-row tiles; Zipf(1.1) at
-    // 96 / 128 / 192 219 / 254 / 322 against 187 / 213 / 268, so no further than they win.
-    // (Products of up to 512 channels keep the range that was measured for them, 96 to 192.)
+    // 96 / 128 / 192 219 / 254 / 322 against 187 / 213 / 268, so no further than they win.  With 128 to 255 columns they win on
+    // uniform routing (128-row tiles take 0.97 to 1.14 of their time at 128 columns, 1.04 to 1.43 at 192) and lose more under
+    // Zipf(1.1) (0.63 to 0.73, 0.65 to 0.90): 32 experts of 2880 / 2880, 1000 tokens of four slots, a layer with the wide tiles
+    // in both products / in the first 245 / 267, Zipf 312 / 300; 60 of 2048 / 1408, 2100 tokens 193 / 203, Zipf 252 / 231.
+    // (From 256 columns on they win less than they lose as well.  That is left as it is.)
+    // Products of up to 512 channels are on the wide tiles from 96 to 192 rows (from 64 to 256 if K is long) at any number of
+    // columns, and behind the others there: K / N = 1024 / 512, 128 rows, 8 and 128 experts 25 and 29 us against 13 and 31 on
+    // 64-row tiles and 14 and 31 on 128-row tiles (Zipf 34 and 48 against 14 and 34, 14 and 30).  Left as it is as well.
     const bool fills = narrow || columns >= kComputeUnits;
     if (avg >= (narrow ? 96 : 112) && avg <= (narrow ? 192 : 144) && a.K >= 1024 && wide_ok && fills) return 256;
     return 128;

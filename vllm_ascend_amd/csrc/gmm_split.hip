@@ -17,19 +17,16 @@
 
 namespace moe355 {
 
-constexpr int kSplitRing = 3;  // stages of 64 K in registers: one in use, two in flight
+constexpr int kSplitRing = 3;                        // stages of 64 K in registers: one in use, two in flight
+constexpr int TB = 2;                                // blocks of 32 rows of a workgroup
+constexpr int kSplitPatch = TB * 32 * 64;            // LDS: tokens of a stage, one wavefront
+constexpr int kSplitSums = TB * 4 * 3 * 2 * 1024;    // ... what the wavefronts hand each other
+constexpr int kSplitLds = 4 * kSplitPatch > kSplitSums ? 4 * kSplitPatch : kSplitSums;
 
-template <int TB>
-struct SplitLds {
-    static constexpr int PATCH = TB * 32 * 64;                  // tokens of a stage, one wavefront
-    static constexpr int SUMS = TB * 4 * 3 * 2 * 1024;          // what the wavefronts hand each other
-    static constexpr int BYTES = 4 * PATCH > SUMS ? 4 * PATCH : SUMS;
-};
-
-template <int EPI, int TB>
+template <int EPI>
 __global__ __launch_bounds__(256, 2) void gmm_split_kernel(GmmArgs a, int units)
 {
-    __shared__ __attribute__((aligned(16))) int8_t lds[SplitLds<TB>::BYTES];
+    __shared__ __attribute__((aligned(16))) int8_t lds[kSplitLds];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
     // an XCD (workgroup number modulo 8) works on every eighth unit of all tiles: the rows of one expert that share a
@@ -94,7 +91,7 @@ __global__ __launch_bounds__(256, 2) void gmm_split_kernel(GmmArgs a, int units)
     };
     // a row's four pieces of a stage lie rotated by half its number: neither the writes (two whole rows at a time) nor the
     // reads (one piece of eight rows) meet in a bank
-    int8_t* patch = lds + wave * SplitLds<TB>::PATCH;
+    int8_t* patch = lds + wave * kSplitPatch;
     const int wr = (lane >> 2) * 64 + (((lane & 3) + (lane >> 3)) & 3) * 16;
     int rd[2];
 #pragma unroll
@@ -173,22 +170,22 @@ __global__ __launch_bounds__(256, 2) void gmm_split_kernel(GmmArgs a, int units)
     }
 }
 
-template <int EPI, int TB>
+template <int EPI>
 static void launch_split_t(const GmmArgs& a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1)
 {
     const int units = a.N / 64;
     const int64_t tiles = (a.R + 32 * TB - 1) / (32 * TB);
     const dim3 grid((unsigned)(tiles * ((units + 7) / 8) * 8));
-    auto kernel = gmm_split_kernel<EPI, TB>;
+    auto kernel = gmm_split_kernel<EPI>;
     if (ev0 || ev1) hipExtLaunchKernelGGL(kernel, grid, dim3(256), 0, st, ev0, ev1, 0, a, units);
     else hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, a, units);
 }
 
 void launch_split(int epi, const GmmArgs& a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1)
 {
-    if (epi == EPI_I32) launch_split_t<EPI_I32, 2>(a, st, ev0, ev1);
-    else if (epi == EPI_SWIGLU) launch_split_t<EPI_SWIGLU, 2>(a, st, ev0, ev1);
-    else launch_split_t<EPI_DEQUANT, 2>(a, st, ev0, ev1);
+    if (epi == EPI_I32) launch_split_t<EPI_I32>(a, st, ev0, ev1);
+    else if (epi == EPI_SWIGLU) launch_split_t<EPI_SWIGLU>(a, st, ev0, ev1);
+    else launch_split_t<EPI_DEQUANT>(a, st, ev0, ev1);
 }
 
 }  // namespace moe355

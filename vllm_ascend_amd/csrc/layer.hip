@@ -55,7 +55,7 @@ struct Buffers {
 };
 
 struct Forms {
-    bool few;      // a few tokens: two launches behind the gating (few.hip)
+    bool few;      // a few tokens: two or three launches (few.hip), and one in front where few_gates leaves the gating to it
     bool pairs;    // pair order
     bool requant;  // ... with the re-quantisation inside the down GEMM
     bool merged;   // ... and the shared expert in the two GEMM launches
