@@ -495,11 +495,12 @@ def test_few_streaming_workgroups_keep_streaming(experts, k, n, first):
         assert name(epilogue, first * experts, k, n, experts) == b"gmm_tiled_kernel"
 
 
-# one for every 56 pairs, but not where a short launch (fewer than 2048 units of 64 channels) has places in front of its slots:
-# from two pairs per expert on
-@pytest.mark.parametrize("experts, n, pairs, blocks", [(128, 1536, 512, 9), (128, 512, 256, 4), (128, 512, 257, 0), (128, 960, 512, 0),
-                                                       (128, 1024, 512, 9), (64, 1024, 512, 0), (256, 512, 512, 9),
-                                                       (128, 1536, 33, 0), (128, 4096, 383, 0), (128, 4096, 384, 6)])
+# one for every 56 pairs, but not where a short launch (fewer than 1536 units of 64 channels) has places in front of its slots
+# (from two pairs per expert on), nor from twelve pairs per expert on
+@pytest.mark.parametrize("experts, n, pairs, blocks", [(128, 1536, 512, 9), (128, 512, 256, 4), (128, 512, 257, 0), (128, 704, 512, 0),
+                                                       (128, 768, 512, 9), (64, 1024, 512, 0), (256, 512, 512, 9),
+                                                       (128, 1536, 33, 0), (60, 2816, 719, 12), (60, 2816, 720, 0),
+                                                       (128, 4096, 383, 0), (128, 4096, 384, 6)])
 def test_further_blocks_in_front_of_the_slots(experts, n, pairs, blocks):
     from vllm_ascend_amd import _lib
 

@@ -1155,8 +1155,15 @@ static bool blocks_of_their_own(int64_t pairs, int64_t n) { return n / 64 < (pai
 // 30.2 / 30.9 against 33.2 / 33.4 / 34.0, Zipf(1.1) 28.6 / 28.8 / 30.8 against 28.3 / 28.7 / 31.4, 64 experts of 512 / 512 (1024,
 // 512) uniform 27.9 / 28.4 / 30.5 against 29.2 / 29.8 / 31.8, Zipf 28.9 / 29.8 / 34.9 against 28.6 / 29.9 / 35.2; 128 experts of
 // 1024 / 512 (2048, 2048) uniform 49.1 / 49.9 / 52.3 against 49.6 / 50.4 / 54.3, Zipf 43.2 / 46.2 / 53.6 against 41.1 / 43.6 / 52.2.
-// So from 2048 units on; without places every slot makes that lookup, and nothing waits (256 experts of 1024 / 256, 127 tokens of
-// four slots uniform 47.2 against 46.7, Zipf 33.8 against 30.8).
+// 64 of 2048 / 768 (1536, 2048) uniform 65.7 / 66.7 / 72.2 against 65.8 / 67.2 / 73.6, Zipf 60.5 / 67.8 / 84.8 against 59.8 / 66.8 /
+// 83.6; 60 of 2048 / 1408 (2640, 1920), four slots, the down product alone, 40 / 64 / 127 tokens uniform 91.6 / 96.2 / 100.1 against
+// 91.3 / 95.9 / 100.3, Zipf 62.7 / 68.9 / 88.3 against 60.6 / 66.5 / 85.2.
+// So from 1536 units on (two rounds of the gate_up product's workgroups), and with fewer than 12 pairs per expert, beyond which
+// most experts are hot: 60 experts of 2048 / 1408, four slots, 160 / 200 / 250 tokens uniform 102.1 / 105.6 / 110.4 against 102.9 /
+// 107.5 / 112.7, Zipf 100.7 / 107.2 / 114.1 against 96.9 / 108.9 / 119.3; 32 of 2880 / 2880, 130 / 200 / 250 tokens uniform 158.5 /
+// 190.5 / 243.1 against 159.0 / 194.3 / 240.3, Zipf 183.4 / 226.9 / 267.4 against 184.0 / 232.5 / 271.6.  Without places every
+// slot makes that lookup, and nothing waits (256 experts of 1024 / 256, 127 tokens of four slots uniform 47.2 against 46.7, Zipf
+// 33.8 against 30.8).
 // The lookups hold 2048 experts.
 static int pair_places(GmmArgs& a, int resident_units)
 {
@@ -1170,7 +1177,7 @@ static int pair_places(GmmArgs& a, int resident_units)
         a.pair_slots = a.R < (int64_t)rest ? (int)a.R : rest;
         // an expert of c rows has (c - 1) / 32 further blocks: over all experts at most (R - 1) / 32
         if (blocks_of_their_own(a.R, a.N)) a.pair_extra = (int)((a.R - 1) / 32);
-        if (a.pair_first == 0 || (int64_t)a.E * (a.N / 64) >= 2048)
+        if (a.pair_first == 0 || ((int64_t)a.E * (a.N / 64) >= 1536 && a.R < 12 * (int64_t)a.E))
             a.pair_early = a.R / 56 < a.pair_extra ? (int)(a.R / 56) : a.pair_extra;
     }
     return a.sh_blocks + a.pair_first + a.pair_slots + a.pair_extra;
