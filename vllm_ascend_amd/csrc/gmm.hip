@@ -1350,9 +1350,11 @@ extern "C" int moe355_gmm2_requant_pairs_supported(int64_t num_tokens, int top_k
     // / 32 / 50 / 64 / 96 / 127 tokens 47.9 / 54.9 / - / 77.4 / 90.3 / 98.2 against 46.2 / 58.5 / 72.4 / - / - / - against 45.0 /
     // 56.0 / 70.2 / 76.3 / 88.6 / 94.8.  Shorter rows gain less: 128 experts of 2048 x 320, 64 / 127 tokens uniform 60.7 / 63.9
     // against 59.6 / 62.1, Zipf 48.0 / 58.6 against 50.3 / 59.5; of 1024 x 256, 160 tokens of four slots 36.4 against 34.1, Zipf
-    // 35.2 against 36.7.  Longer rows: up to three and a half rows per expert (two at a time up to 1024 values, one beyond).
-    // So are experts of many channels with few pairs, whose hot ones take their rows in passes: there the re-quantisation
-    // stands in front of every pass.  32 experts of 4096 x 768, four slots, Zipf(1.1), 40 / 64 / 80 tokens 69.4 / 75.3 / 84.3
+    // 35.2 against 36.7.  Longer rows: up to three and a half rows per expert (two at a time up to 1024 values, one beyond).  Two at
+    // a time it would pay further: 64 experts of 2048 x 1024, 28 / 64 / 112 tokens 88.2 / 92.1 / 95.8 against 84.1 / 86.9 / 91.4, Zipf
+    // 65.8 / 85.2 / 102.1 against 66.0 / 81.2 / 98.2; left as it is.
+    // Three and a half rows are the limit for experts of many channels with few pairs as well, whose hot ones take their rows
+    // in passes: there the re-quantisation stands in front of every pass.  32 experts of 4096 x 768, four slots, Zipf(1.1), 40 / 64 / 80 tokens 69.4 / 75.3 / 84.3
     // against 70.9 / 80.6 / 92.0 (uniform 65.6 / 66.2 / 66.7 against 63.0 / 64.1 / 64.8), 112 tokens, which is more than 384
     // pairs, 80.2 against 78.0.
     const int64_t pairs = num_tokens * top_k;
