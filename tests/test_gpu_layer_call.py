@@ -97,7 +97,8 @@ def test_a_few_tokens_at_full_size(name, tokens):
     assert torch.equal(layer(x, logits), layer.forward_impl(x, logits).routed_out)
 
 
-# gating and quantisation inside the first launch: 1 to 4 tokens, experts that fill no register or word of four, groups,
+# gating and quantisation inside the first launch: 1 to 4 tokens (130 and 256 experts: one; from two on a launch in front of
+# it), experts that fill no register or word of four, groups,
 # scores that tie (so the lower index decides) and a row of one score, logits of every type; rows that are no multiple of
 # the 512 values a wavefront takes
 @pytest.mark.parametrize("tokens", [1, 2, 3, 4])

@@ -1354,9 +1354,9 @@ extern "C" int moe355_gmm2_requant_pairs_supported(int64_t num_tokens, int top_k
     // a time it would pay further: 64 experts of 2048 x 1024, 28 / 64 / 112 tokens 88.2 / 92.1 / 95.8 against 84.1 / 86.9 / 91.4, Zipf
     // 65.8 / 85.2 / 102.1 against 66.0 / 81.2 / 98.2; left as it is.
     // Three and a half rows are the limit for experts of many channels with few pairs as well, whose hot ones take their rows
-    // in passes: there the re-quantisation stands in front of every pass.  32 experts of 4096 x 768, four slots, Zipf(1.1), 40 / 64 / 80 tokens 69.4 / 75.3 / 84.3
-    // against 70.9 / 80.6 / 92.0 (uniform 65.6 / 66.2 / 66.7 against 63.0 / 64.1 / 64.8), 112 tokens, which is more than 384
-    // pairs, 80.2 against 78.0.
+    // in passes: there the re-quantisation stands in front of every pass.  32 experts of 4096 x 768, four slots, Zipf(1.1), 40 /
+    // 64 / 80 tokens 69.4 / 75.3 / 84.3 against 70.9 / 80.6 / 92.0 (uniform 65.6 / 66.2 / 66.7 against 63.0 / 64.1 / 64.8), 112
+    // tokens, which is more than 384 pairs, 80.2 against 78.0.
     const int64_t pairs = num_tokens * top_k;
     return pairs * 2 <= (k <= 768 && blocks_of_their_own(pairs, n) ? 16 : 7) * (int64_t)num_experts;
 }
