@@ -189,10 +189,10 @@ def test_few_rows_on_tiles(R, family):
     test_families_on_both_sides_of_a_line(R, 16, 192, 320, family, True)
 
 
-# ... and 47 / 48 where streaming has workgroups for half of the chip at most
-@pytest.mark.parametrize("R,family", [(48 * 16 - 1, "stream"), (48 * 16, "tiled")])
+# ... and 47 / 48 where few experts stream with workgroups for half of the chip at most
+@pytest.mark.parametrize("R,family", [(48 * 8 - 1, "stream"), (48 * 8, "tiled")])
 def test_few_rows_on_tiles_few_channels(R, family):
-    test_families_on_both_sides_of_a_line(R, 16, 1024, 512, family, True)
+    test_families_on_both_sides_of_a_line(R, 8, 1024, 512, family, True)
 
 
 # 64 rows per expert at a long K: as many columns of wide tiles as half of the compute units, and one less

@@ -642,13 +642,14 @@ static int tiled_bm(const GmmArgs& a)
     //     / 131 against 56 / 57 / 58); 24 experts, K = 4096 / 2048, 27 / 40: 154 / 232 against 133 / 138; 8 experts of that
     //     shape, 24 / 32: 59.6 / 83.0 against 72.8 / 74.9, so no earlier.
     //     That is so because streaming fills the chip.  With workgroups for half of it the second reading costs nothing, and a
-    //     tile's walk along K alone does: one product, 4 to 32 experts, 32 to 47 rows each, tiles / streaming at up to 128
-    //     workgroups 1.37 to 1.61 for K from 2048, 1.25 to 1.29 for K = 1024 (Zipf 0.4 to 1.3, about even on the whole);
-    //     at 192 and 256 1.04 to 1.38 (Zipf 0.3 to 0.98), at 288 to 512 0.69 to 1.21 (Zipf 0.3 to 0.95).  With K below 1024 it is
-    //     little: layers of 8 to 24 experts of 256 to 768, 26 to 29 us streaming and 28 to 32 on tiles (Zipf 30 to 59 against 28
-    //     to 38).
+    //     tile's walk along K alone does: one product, 32 to 47 rows per expert, tiles / streaming at up to 128 workgroups 1.37
+    //     to 1.61 for K from 2048, 1.25 to 1.29 for K = 1024; at 192 and 256 1.04 to 1.38, at 288 to 512 0.69 to 1.21.  Skewed
+    //     routing pays for the passes of its hot experts, the more the more experts there are: up to 128 workgroups, mean of
+    //     uniform routing and of Zipf(1.1), 4 experts 1.39 and 1.07, 8 experts 1.38 and 0.78, 16 experts 1.40 and 0.57, 24
+    //     experts 1.38 and 0.43.  So up to eight experts.  With K below 1024 it is little: layers of 8 to 24 experts of 256 to
+    //     768, 26 to 29 us streaming and 28 to 32 on tiles (Zipf 30 to 59 against 28 to 38).
     if (a.R < a.E) return 0;
-    const bool few_streams = (int64_t)a.E * (a.N / 64) <= kComputeUnits / 2 && a.K >= 1024;
+    const bool few_streams = a.E <= 8 && (int64_t)a.E * (a.N / 64) <= kComputeUnits / 2 && a.K >= 1024;
     if (avg < (few_streams ? 48 : 32) && a.R < 1024 && (a.R < 128 || weights < (1ll << 30))) return 0;
     // Few experts and few rows: as long as tiles of half the height do not outnumber the compute units they are twice as
     // many and half as long (rows / 64 and half a tile per expert for its last one).  8 experts of 2816 x 1024 and 1024 x
