@@ -1,8 +1,8 @@
 // Pieces shared by the grouped-GEMM kernels: tiled weight addressing, the
 // MFMA accumulator <-> (row, channel) mapping and the three epilogues.
 //
-// MFMA used: v_mfma_i32_32x32x32_i8.  Operand A (4 VGPRs = 16 int8 per lane)
-// carries WEIGHTS: lane l supplies channel l%32, K slice 16*(l/32)..+15 of the
+// MFMA of the streaming kernel: v_mfma_i32_32x32x32_i8 (the tiles of many rows use mfma_i8_16 below).
+// Operand A (4 VGPRs = 16 int8 per lane) carries WEIGHTS: lane l supplies channel l%32, K slice 16*(l/32)..+15 of the
 // 32-wide K step.  Operand B carries TOKENS with the same K mapping.  The
 // 32x32 int32 result sits in 16 VGPRs: lane l, register v holds
 //   token   = l % 32
@@ -98,6 +98,11 @@ __device__ __forceinline__ v4i mfma_i8_16(v4i a, v4i b, v4i c)
 {
     return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
 }
+
+// Weights of 16 channels x 64 K values for it, out of the storage tiles (32 channels x 32 K in 1 KiB: lane l of that tile
+// holds channel l % 32, K half l / 32): this lane's byte offset inside the 2 KiB of 64 K values; the second 16 channels
+// lie 256 bytes further.
+__device__ __forceinline__ int weight_lane(int lane) { return (lane >> 4) * 512 + (lane & 15) * 16; }
 
 // One token row, one run of four consecutive channels starting at c0 (tile 0) and c1 (tile 1).
 // rs: the row's token scale; s0 / s1: the channel scales of the two runs.  The caller loads them before its

@@ -2,10 +2,19 @@
 //
 // Workgroup tile: BM tokens x 256 channels, K consumed 64 at a time.  The four wavefronts own 64
 // channels each (two 32-channel storage tiles: for the gate_up GEMM a gate tile and its up tile,
-// so SwiGLU pairs meet in one lane).  Weights never touch LDS: a storage tile is one MFMA A
-// operand and is loaded straight into registers, two iterations ahead.  Tokens are shared by the
+// so SwiGLU pairs meet in one lane).  Weights never touch LDS: 16 channels x 64 K of a storage tile are one MFMA A
+// operand and are loaded straight into registers, two iterations ahead.  Tokens are shared by the
 // four wavefronts: global -> registers (three iterations ahead) -> LDS in MFMA-operand order
-// (every B operand is one conflict-free 1 KiB ds_read_b128 sweep) -> MFMA.
+// (every B operand, 16 tokens x 64 K, is one conflict-free 1 KiB ds_read_b128 sweep) -> MFMA.
+//
+// All tiles of this file multiply with v_mfma_i32_16x16x64_i8.  v_mfma_i32_32x32x32_i8 takes the same operand bytes and
+// cycles per product but moves four times the accumulators, and these kernels run at the power limit: it only lowers the
+// clock.  Loops on int8 values of a normal distribution of width 32, 32x32x32 against 16x16x64, after the first 2 ms:
+// operands in registers 3.45 POP/s at 1.80 GHz against 4.09 at 2.09; four token operands from LDS per weight pair 3.16 at
+// 1.65 against 3.63 at 1.94; weights from L2 as well 2.67 at 1.59 against 2.97 at 1.88 (zeros: 4.8 at 2.4 GHz for both).
+// The kernels back to back: dense 4096 x 7168 x 4096 127.6 -> 115.6 us; 256 experts of 128 rows, gate_up 7168 / 4096 and
+// its re-quantisation 1550 -> 1488, down 2048 / 7168 805 -> 782; 128 experts of 512 rows, 2048 / 1536 336 -> 329, 768 / 2048
+// 179 -> 174.  Where the weights' way from HBM decides it is the same (128 experts of 48 rows).
 // Tiles are enumerated (expert, row block) by a small map kernel from the group list; the 1-D
 // grid is remapped so that all column blocks of a row block, and the row blocks of one expert,
 // run on the same XCD (workgroup i goes to XCD i % 8) and share its L2.
@@ -42,90 +51,112 @@ struct TiledLds {
     static constexpr int ROWB = 128 + 16;                      // epilogue patch: bytes per token row (padded)
     static constexpr int PATCHES = (EPI == EPI_I32) ? 2 : 1;   // 32-row patches per wavefront in the epilogue
     static constexpr int EPI_BYTES = 4 * PATCHES * 32 * ROWB;
-    static constexpr int BYTES = RING * STAGE_BYTES > EPI_BYTES ? RING * STAGE_BYTES : EPI_BYTES;
+    static constexpr int SCALES = RING * STAGE_BYTES > EPI_BYTES ? RING * STAGE_BYTES : EPI_BYTES;  // token scales, then channel scales
+    static constexpr int BYTES = SCALES + (EPI == EPI_I32 ? 0 : (BM + kBN) * 4);
 };
 
-// Epilogue of one wavefront: BMT token blocks x two 32-channel storage tiles (nb0, nb1) out of the MFMA
-// accumulators.  In the accumulators a lane owns one token and scattered runs of four channels;
-// written like that every store would touch 64 different cache lines.  The wavefront instead
-// turns one 32-token block at a time through a private LDS patch (token-major, 128 data bytes per
+// Epilogue of one wavefront: BMT blocks of 32 tokens x two 32-channel storage tiles (nb0, nb1) out of the MFMA
+// accumulators: acc[t][b] holds channels 16 (t % 2) .. + 15 of storage tile t / 2 for tokens 16 b .. + 15.  There a lane
+// owns one token and runs of four channels; written like that every store would touch 64 different cache lines.  The
+// wavefront instead turns 32 tokens at a time through a private LDS patch (token-major, 128 data bytes per
 // token and tile) and stores whole 128-byte row segments: 8 lanes per token row.
 // FLAG, SwiGLU epilogue: the clamp is compiled in (as compares and selects it costs 8 of about 50 vector
 // instructions per output, and the epilogue is bound by their number); dequant epilogue: the output is fp16
 // instead of bf16.  The caller branches once.
-template <int EPI, int BMT, bool FLAG>
-__device__ __forceinline__ void tiled_epilogue_body(const GmmArgs& a, int e, v16i (&acc)[2][BMT], int64_t row0,
-                                                    int64_t row_end, int nb0, int nb1, int8_t* patch, int lane)
+// IN_LDS: the scales lie in LDS, rs_lds by row of the tile and cs_lds by channel of the wavefront's two storage tiles.
+template <int EPI, int BMT, bool FLAG, bool IN_LDS>
+__device__ __forceinline__ void tiled_epilogue_body(const GmmArgs& a, int e, v4i (&acc)[4][2 * BMT], int64_t row0,
+                                                    int64_t row_end, int nb0, int nb1, int8_t* patch, int lane,
+                                                    const float* rs_lds, const float* cs_lds)
 {
     constexpr int ROWB = TiledLds<EPI, BMT, 3>::ROWB;
-    const int tok = lane & 31;
-    const int hi = lane >> 5;
-    const float* cs = (a.ch_scale || a.s_list) ? expert_scales(a, e) : nullptr;
-    v4f s0[4], s1[4];
-    if constexpr (EPI != EPI_I32) {
+    const int tok = lane & 15;
+    const int run = 4 * (lane >> 4);  // this lane's first channel inside a group of 16
+    v4f s0[2], s1[2];
+    if constexpr (EPI != EPI_I32 && IN_LDS) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            s0[q] = gload4f(cs + nb0 * 32 + 8 * q + 4 * hi);
-            s1[q] = gload4f(cs + nb1 * 32 + 8 * q + 4 * hi);
+        for (int t = 0; t < 2; ++t) {
+            s0[t] = *(const v4f*)(cs_lds + 16 * t + run);
+            s1[t] = *(const v4f*)(cs_lds + 32 + 16 * t + run);
+        }
+    } else if constexpr (EPI != EPI_I32) {
+        const float* cs = expert_scales(a, e);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            s0[t] = gload4f(cs + nb0 * 32 + 16 * t + run);
+            s1[t] = gload4f(cs + nb1 * 32 + 16 * t + run);
         }
     }
     // every token scale is requested before the first store: the memory counter retires in order, so a load
-    // behind a block's stores would wait for their acknowledgement, once per token block
-    float rs_all[BMT];
+    // behind a block's stores would wait for their acknowledgement, once per token block.  The rows' tokens are looked up
+    // in one go: a branch per row would wait for each look-up before it requests the next.
+    float rs_all[2 * BMT];
+    if constexpr (EPI != EPI_I32 && IN_LDS) {
 #pragma unroll
-    for (int b = 0; b < BMT; ++b) {
-        rs_all[b] = 0.0f;
-        if constexpr (EPI != EPI_I32) {
-            const int64_t row = row0 + b * 32 + tok;
-            const int64_t rc = row < row_end ? row : row_end - 1;
-            rs_all[b] = a.row_scale[a.row_src ? (int64_t)a.row_src[rc] : rc];
-            if (row >= row_end) rs_all[b] = 0.0f;
+        for (int b = 0; b < 2 * BMT; ++b) rs_all[b] = rs_lds[b * 16 + tok];
+    } else if constexpr (EPI != EPI_I32) {
+        int32_t at[2 * BMT];  // rows are fewer than 2^31
+#pragma unroll
+        for (int b = 0; b < 2 * BMT; ++b) {
+            const int64_t row = row0 + b * 16 + tok;
+            at[b] = (int32_t)(row < row_end ? row : row_end - 1);
         }
+        if (a.row_src) {
+#pragma unroll
+            for (int b = 0; b < 2 * BMT; ++b) at[b] = a.row_src[at[b]];
+        }
+#pragma unroll
+        for (int b = 0; b < 2 * BMT; ++b) rs_all[b] = a.row_scale[at[b]];
+    } else {
+#pragma unroll
+        for (int b = 0; b < 2 * BMT; ++b) rs_all[b] = 0.0f;
     }
     // ... and has arrived before it: the stores below sit behind "row < row_end" branches, and a wait for a
     // load that is still in flight at that point would have to assume that none of them was issued, which
     // turns it into a wait for every store of the block before
 #pragma unroll
-    for (int b = 0; b < BMT; ++b) asm volatile("" : "+v"(rs_all[b]));
+    for (int b = 0; b < 2 * BMT; ++b) asm volatile("" : "+v"(rs_all[b]));
 #pragma unroll
     for (int b = 0; b < BMT; ++b) {
-        const int64_t row = row0 + b * 32 + tok;
-        const bool valid = row < row_end;
-        const float rs = rs_all[b];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int ch = 8 * q + 4 * hi;  // first of this lane's four channels inside the tile
-            if constexpr (EPI == EPI_I32) {
-                *(v4i*)(patch + tok * ROWB + ch * 4) =
-                    (v4i){acc[0][b][4 * q], acc[0][b][4 * q + 1], acc[0][b][4 * q + 2], acc[0][b][4 * q + 3]};
-                *(v4i*)(patch + 32 * ROWB + tok * ROWB + ch * 4) =
-                    (v4i){acc[1][b][4 * q], acc[1][b][4 * q + 1], acc[1][b][4 * q + 2], acc[1][b][4 * q + 3]};
-            } else if constexpr (EPI == EPI_DEQUANT) {
-                v4u16 o0, o1;
+        for (int h = 0; h < 2; ++h) {
+            const float rs = rs_all[2 * b + h];
+            int8_t* const prow = patch + (16 * h + tok) * ROWB;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    o0[j] = f32_to_half<FLAG ? MOE355_DT_F16 : MOE355_DT_BF16>(((float)acc[0][b][4 * q + j] * rs) * s0[q][j]);
-                    o1[j] = f32_to_half<FLAG ? MOE355_DT_F16 : MOE355_DT_BF16>(((float)acc[1][b][4 * q + j] * rs) * s1[q][j]);
-                }
-                // both tiles are adjacent in the output row: 64 bf16 = 128 bytes per token
-                *(v4u16*)(patch + tok * ROWB + ch * 2) = o0;
-                *(v4u16*)(patch + tok * ROWB + 64 + ch * 2) = o1;
-            } else {
-                v4f yv;
+            for (int t = 0; t < 2; ++t) {
+                const v4i c0 = acc[t][2 * b + h], c1 = acc[2 + t][2 * b + h];
+                const int ch = 16 * t + run;  // first of this lane's four channels inside the storage tile
+                if constexpr (EPI == EPI_I32) {
+                    *(v4i*)(prow + ch * 4) = c0;
+                    *(v4i*)(prow + 32 * ROWB + ch * 4) = c1;
+                } else if constexpr (EPI == EPI_DEQUANT) {
+                    v4u16 o0, o1;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    float gg = ((float)acc[0][b][4 * q + j] * rs) * s0[q][j];
-                    float uu = ((float)acc[1][b][4 * q + j] * rs) * s1[q][j];
-                    if constexpr (FLAG) {
-                        gg = gg > a.limit ? a.limit : gg;
-                        uu = uu > a.limit ? a.limit : uu;
-                        uu = uu < -a.limit ? -a.limit : uu;
+                    for (int j = 0; j < 4; ++j) {
+                        o0[j] = f32_to_half<FLAG ? MOE355_DT_F16 : MOE355_DT_BF16>(((float)c0[j] * rs) * s0[t][j]);
+                        o1[j] = f32_to_half<FLAG ? MOE355_DT_F16 : MOE355_DT_BF16>(((float)c1[j] * rs) * s1[t][j]);
                     }
-                    yv[j] = m_silu(gg) * uu;
+                    // both tiles are adjacent in the output row: 64 bf16 = 128 bytes per token
+                    *(v4u16*)(prow + ch * 2) = o0;
+                    *(v4u16*)(prow + 64 + ch * 2) = o1;
+                } else {
+                    v4f yv;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        float gg = ((float)c0[j] * rs) * s0[t][j];
+                        float uu = ((float)c1[j] * rs) * s1[t][j];
+                        if constexpr (FLAG) {
+                            gg = gg > a.limit ? a.limit : gg;
+                            uu = uu > a.limit ? a.limit : uu;
+                            uu = uu < -a.limit ? -a.limit : uu;
+                        }
+                        yv[j] = m_silu(gg) * uu;
+                    }
+                    *(v4f*)(prow + ch * 4) = yv;
                 }
-                *(v4f*)(patch + tok * ROWB + ch * 4) = yv;
             }
         }
+        wave_lds_order();
         // read back row-major: lane -> (row r8 + 8*p, 16-byte column c16)
         const int c16 = lane & 7, r8 = lane >> 3;
 #pragma unroll
@@ -148,26 +179,28 @@ __device__ __forceinline__ void tiled_epilogue_body(const GmmArgs& a, int e, v16
                 }
             }
         }
+        wave_lds_order();
     }
 }
 
-template <int EPI, int BMT>
-__device__ __forceinline__ void tiled_epilogue(const GmmArgs& a, int e, v16i (&acc)[2][BMT], int64_t row0,
-                                               int64_t row_end, int nb0, int nb1, int8_t* patch, int lane)
+template <int EPI, int BMT, bool IN_LDS = false>
+__device__ __forceinline__ void tiled_epilogue(const GmmArgs& a, int e, v4i (&acc)[4][2 * BMT], int64_t row0,
+                                               int64_t row_end, int nb0, int nb1, int8_t* patch, int lane,
+                                               const float* rs_lds = nullptr, const float* cs_lds = nullptr)
 {
     if constexpr (EPI == EPI_SWIGLU) {
         if (a.limit > 0.0f) {
-            tiled_epilogue_body<EPI, BMT, true>(a, e, acc, row0, row_end, nb0, nb1, patch, lane);
+            tiled_epilogue_body<EPI, BMT, true, IN_LDS>(a, e, acc, row0, row_end, nb0, nb1, patch, lane, rs_lds, cs_lds);
             return;
         }
     }
     if constexpr (EPI == EPI_DEQUANT) {
         if (a.out_f16) {
-            tiled_epilogue_body<EPI, BMT, true>(a, e, acc, row0, row_end, nb0, nb1, patch, lane);
+            tiled_epilogue_body<EPI, BMT, true, IN_LDS>(a, e, acc, row0, row_end, nb0, nb1, patch, lane, rs_lds, cs_lds);
             return;
         }
     }
-    tiled_epilogue_body<EPI, BMT, false>(a, e, acc, row0, row_end, nb0, nb1, patch, lane);
+    tiled_epilogue_body<EPI, BMT, false, IN_LDS>(a, e, acc, row0, row_end, nb0, nb1, patch, lane, rs_lds, cs_lds);
 }
 
 // One tile of BMT token blocks: rows [row0, row_end) of expert e (at most 32 * BMT of them are computed),
@@ -204,12 +237,12 @@ __device__ __forceinline__ void tiled_body(const GmmArgs& a, int e, int64_t row0
     }
     const bool have = (EPI == EPI_SWIGLU) ? (nb0 < half_tiles) : (nb1 < NB);
     const int8_t* we = expert_weights(a, e);
-    const int8_t* w0 = we + ((int64_t)(have ? nb0 : 0) * KB) * 1024 + lane * 16;
-    const int8_t* w1 = we + ((int64_t)(have ? nb1 : 0) * KB) * 1024 + lane * 16;
+    const int8_t* w0 = we + ((int64_t)(have ? nb0 : 0) * KB) * 1024 + weight_lane(lane);
+    const int8_t* w1 = we + ((int64_t)(have ? nb1 : 0) * KB) * 1024 + weight_lane(lane);
 
     const int n_iter = a.K / kBK;
 
-    v4i Areg[RING][2][2];   // [stage][tile][k step]
+    v4i Areg[RING][4];   // [stage][16 channels]
     v4i Breg[RING][CHUNKS];
 
     // Loads past the last K block or the last row are redirected to valid addresses instead of being
@@ -220,13 +253,23 @@ __device__ __forceinline__ void tiled_body(const GmmArgs& a, int e, int64_t row0
     auto load_A = [&](int it, int st) {
         const int itc = it < last_it ? it : last_it;
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            Areg[st][0][s] = weight_tile(w0 + ((int64_t)itc * 2 + s) * 1024);
-            Areg[st][1][s] = weight_tile(w1 + ((int64_t)itc * 2 + s) * 1024);
+        for (int t = 0; t < 2; ++t) {
+            Areg[st][t] = weight_tile(w0 + (int64_t)itc * 2048 + t * 256);
+            Areg[st][2 + t] = weight_tile(w1 + (int64_t)itc * 2048 + t * 256);
         }
     };
     const int8_t* xrow[CHUNKS];
     int lds_off[CHUNKS];
+    int64_t xr[CHUNKS];
+#pragma unroll
+    for (int j = 0; j < CHUNKS; ++j) {
+        xr[j] = row0 + (tid & 15) + 16 * ((tid >> 6) + 4 * j);
+        if (xr[j] > row_end - 1) xr[j] = row_end - 1;  // rows past the expert's end duplicate its last row
+    }
+    if (a.row_src) {  // the rows' values lie in their tokens' rows
+#pragma unroll
+        for (int j = 0; j < CHUNKS; ++j) xr[j] = a.row_src[xr[j]];
+    }
 #pragma unroll
     for (int j = 0; j < CHUNKS; ++j) {
         // 16 consecutive lanes take 16 consecutive token rows at the same K chunk: their 16-byte LDS
@@ -234,12 +277,8 @@ __device__ __forceinline__ void tiled_body(const GmmArgs& a, int e, int64_t row0
         // covers 16 rows x 64 contiguous bytes
         const int row = (tid & 15) + 16 * ((tid >> 6) + 4 * j);
         const int kc = (tid >> 4) & 3;
-        int64_t r = row0 + row;
-        if (r > row_end - 1) r = row_end - 1;  // rows past the expert's end duplicate its last row
-        if (a.row_src) r = a.row_src[r];       // the row's values lie in the token's row
-        xrow[j] = a.x + r * a.K + kc * 16;
-        const int s = kc >> 1, kh = kc & 1;
-        lds_off[j] = (((s * BMT + (row >> 5)) * 64) + kh * 32 + (row & 31)) * 16;
+        xrow[j] = a.x + xr[j] * a.K + kc * 16;
+        lds_off[j] = (row >> 4) * 1024 + kc * 256 + (row & 15) * 16;
     }
     auto load_B = [&](int it, int st) {
         const int itc = it < last_it ? it : last_it;
@@ -251,25 +290,18 @@ __device__ __forceinline__ void tiled_body(const GmmArgs& a, int e, int64_t row0
         for (int j = 0; j < CHUNKS; ++j) *(v4i*)(&Bs[st][lds_off[j]]) = Breg[st][j];
     };
 
-    v16i acc[2][BMT];
+    v4i acc[4][2 * BMT];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int b = 0; b < BMT; ++b) acc[t][b] = (v16i){0};
+        for (int b = 0; b < 2 * BMT; ++b) acc[t][b] = (v4i){0};
 
-    // B operands of one K step (BMT fragments of 1 KiB) live in registers; the two K steps of a stage
-    // are double-buffered so that LDS reads of one step run under the MFMAs of the other.
+    // B operands (fragments of 16 tokens x 64 K, 1 KiB) of half the tokens live in registers; the two halves of a
+    // stage are double-buffered so that LDS reads of one half run under the MFMAs of the other.
     v4i bf0[BMT], bf1[BMT];
-    auto read_frags = [&](v4i* dst, int st, int s) {
+    auto read_frags = [&](v4i* dst, int st) {
 #pragma unroll
-        for (int b = 0; b < BMT; ++b) dst[b] = *(const v4i*)(&Bs[st][((s * BMT + b) * 64 + lane) * 16]);
-    };
-    auto mma_step = [&](const v4i* frags, int st, int s) {
-#pragma unroll
-        for (int b = 0; b < BMT; ++b) {
-            acc[0][b] = mfma_i8(Areg[st][0][s], frags[b], acc[0][b]);
-            acc[1][b] = mfma_i8(Areg[st][1][s], frags[b], acc[1][b]);
-        }
+        for (int b = 0; b < BMT; ++b) dst[b] = *(const v4i*)(&Bs[st][(b * 64 + lane) * 16]);
     };
 
     // ---- prologue.  After it the loads still in flight are, oldest first, A(0) B(1) A(1) B(2) ...: the same
@@ -283,21 +315,38 @@ __device__ __forceinline__ void tiled_body(const GmmArgs& a, int e, int64_t row0
         load_A(r, r);
         load_B(r + 1, r + 1);
     }
+    // the scales of the epilogue too: requested behind the K loop they cost it two or three memory latencies with nothing
+    // else left to do
+    float* const rs_lds = (float*)(lds_raw + TiledLds<EPI, BMT, RING>::SCALES);
+    float* const cs_lds = rs_lds + 32 * BMT + wave * 64;
+    float rs_own = 0.0f, cs_own = 0.0f;
+    if constexpr (EPI != EPI_I32) {
+        if (tid < 32 * BMT) {
+            int64_t r = row0 + tid < row_end ? row0 + tid : row_end - 1;
+            if (a.row_src) r = a.row_src[r];
+            rs_own = a.row_scale[r];
+        }
+        if (have) cs_own = expert_scales(a, e)[(lane < 32 ? nb0 * 32 : nb1 * 32 - 32) + lane];
+    }
     __builtin_amdgcn_sched_barrier(0);
     store_B(0);
+    if constexpr (EPI != EPI_I32) {
+        if (tid < 32 * BMT) rs_lds[tid] = rs_own;
+        cs_lds[lane] = cs_own;
+    }
     __syncthreads();
-    read_frags(bf0, 0, 0);
+    read_frags(bf0, 0);
 
     // One pipeline step on stage U (compile-time ring position) for K block I.  LA / LB: request the weights of
     // K block I + RING - 1 / the tokens of K block I + RING; SB: move the tokens of K block I + 1 to LDS.
 #define MOE355_STEP(U, I, LA, LB, SB)                                                            \
     {                                                                                            \
-        /* first K step: its MFMAs go first; the LDS traffic of the second K step and of the */  \
-        /* next stage is issued in the gaps while the matrix pipe is busy                    */  \
+        /* first half of the tokens: its MFMAs go first; the LDS traffic of the second half and */ \
+        /* of the next stage is issued in the gaps while the matrix pipe is busy             */  \
         _Pragma("unroll") for (int b = 0; b < BMT; ++b)                                          \
         {                                                                                        \
-            acc[0][b] = mfma_i8(Areg[(U)][0][0], bf0[b], acc[0][b]);                             \
-            acc[1][b] = mfma_i8(Areg[(U)][1][0], bf0[b], acc[1][b]);                             \
+            _Pragma("unroll") for (int t = 0; t < 4; ++t)                                        \
+                acc[t][b] = mfma_i8_16(Areg[(U)][t], bf0[b], acc[t][b]);                         \
             bf1[b] = *(const v4i*)(&Bs[(U)][((BMT + b) * 64 + lane) * 16]);                      \
             if ((SB) && b == 0) store_B(((U) + 1) % RING); /* B(I+1): registers -> LDS */        \
             __builtin_amdgcn_sched_barrier(0);                                                   \
@@ -305,8 +354,8 @@ __device__ __forceinline__ void tiled_body(const GmmArgs& a, int e, int64_t row0
         __syncthreads(); /* B(I+1) visible to all wavefronts */                                  \
         _Pragma("unroll") for (int b = 0; b < BMT; ++b)                                          \
         {                                                                                        \
-            acc[0][b] = mfma_i8(Areg[(U)][0][1], bf1[b], acc[0][b]);                             \
-            acc[1][b] = mfma_i8(Areg[(U)][1][1], bf1[b], acc[1][b]);                             \
+            _Pragma("unroll") for (int t = 0; t < 4; ++t)                                        \
+                acc[t][BMT + b] = mfma_i8_16(Areg[(U)][t], bf1[b], acc[t][BMT + b]);             \
             if (SB) bf0[b] = *(const v4i*)(&Bs[((U) + 1) % RING][(b * 64 + lane) * 16]);         \
             if ((LA) && b == 0) load_A((I) + RING - 1, ((U) + RING - 1) % RING);                 \
             if ((LB) && b == (BMT > 1 ? 1 : 0)) load_B((I) + RING, (U));                         \
@@ -349,7 +398,8 @@ __device__ __forceinline__ void tiled_body(const GmmArgs& a, int e, int64_t row0
 
     __syncthreads();  // all wavefronts are done reading the token stages; LDS is reused below
     if (!have) return;
-    tiled_epilogue<EPI, BMT>(a, e, acc, row0, row_end, nb0, nb1, lds_raw + wave * (PATCHES * 32 * ROWB), lane);
+    tiled_epilogue<EPI, BMT, EPI != EPI_I32>(a, e, acc, row0, row_end, nb0, nb1, lds_raw + wave * (PATCHES * 32 * ROWB), lane,
+                                             rs_lds, cs_lds);
 }
 
 // The last tile of an expert is usually short.  Tiles of at most 64 rows run the two-block body (half the
@@ -476,8 +526,9 @@ __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_
     }
     // Tokens: one load covers 16 rows x the 64 K bytes of a stage, four neighbouring lanes on one row (one
     // 64-byte line per lane quad).  LDS slot of (row r, 16-byte chunk c) inside its 16-row KiB:
-    // 4 * (r % 16) + (c + (r % 16) / 4) % 4 -- the rotation spreads the MFMA operand reads (32 rows at one
-    // chunk, 64 bytes apart) over all banks.  Wavefront w copies rows 32 w .. 32 w + 31 (tall: two loads) or
+    // 4 * (r % 16) + (c ^ f(r)), f = 0, 3, 2, 1 for r / 4 % 4 = 0, 1, 2, 3 -- 64 bytes apart, sixteen rows at one chunk
+    // then lie in all sixteen 16-byte bank groups, and so do rows 0..3 and 12..15 at a chunk and rows 4..11 at its
+    // neighbour (c ^ 1), which is how the LDS takes the lanes of a 16-byte read.  Wavefront w copies rows 32 w .. 32 w + 31 (tall: two loads) or
     // 16 w .. 16 w + 15 (wide); 16-row blocks that lie past the expert's last row are not loaded at all
     // (their products are never stored).
     // A wide tile of more than four blocks has more than eight 16-row pieces: wavefront w also copies piece
@@ -485,7 +536,7 @@ __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_
     constexpr int XROWS = WIDE ? 16 : 32;
     constexpr int XSECOND = WIDE ? 8 * 16 : 16;     // rows between the first and the second piece of a wavefront
     constexpr bool X2 = !WIDE || NBLK > 4;
-    const int xchunk = ((lane & 3) - (lane >> 4)) & 3;
+    const int xchunk = (lane & 3) ^ (-(lane >> 4) & 3);
     const int64_t xfirst = row0 + wave * XROWS;
     const bool x2 = X2 && (WIDE ? wave + 8 < 2 * NBLK : true) && xfirst + XSECOND < row_end;
     const int n_xloads = xfirst >= row_end ? 0 : (x2 ? 2 : 1);
@@ -498,12 +549,10 @@ __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_
     }
     const int8_t* xsrc0 = a.x + xr0 * a.K + xchunk * 16;
     const int8_t* xsrc1 = a.x + xr1 * a.K + xchunk * 16;
-    // operand reads of this lane: token l % 32 of a block, K half l / 32, K step s -> chunk 2 s + l / 32
+    // operand reads of this lane: token l % 16 of a block, chunk l / 16
     const int r16 = lane & 15;
-    const int frag_off = XBASE + (h * 8 + ((lane >> 4) & 1)) * 1024 + r16 * 64;
-    const int frag_s0 = frag_off + (((lane >> 5) + (r16 >> 2)) & 3) * 16;
-    const int frag_s1 = frag_off + ((2 + (lane >> 5) + (r16 >> 2)) & 3) * 16;
-    const int a_off = g * 4096 + lane * 16;
+    const int frag_off = XBASE + h * 8192 + r16 * 64 + (((lane >> 4) ^ (-(r16 >> 2) & 3)) * 16);
+    const int a_off = g * 4096 + weight_lane(lane);
 
     const int n_iter = a.K / kBK;
     const int last_it = n_iter - 1;
@@ -542,11 +591,11 @@ __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_
         }
     };
 
-    v16i acc[2][NBLK];
+    v4i acc[4][2 * NBLK];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int b = 0; b < NBLK; ++b) acc[t][b] = (v16i){0};
+        for (int b = 0; b < 2 * NBLK; ++b) acc[t][b] = (v4i){0};
 
     // Every step requests the tokens SX - 1 steps ahead and then the weights SW - 1 steps ahead; the steps before
     // the first one do the same for what lies at or after K block 0, so that the order of the requests, which the
@@ -597,16 +646,14 @@ __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_
             if (active) {
                 const int8_t* wbase = lds + uw * A_BYTES;
                 const int8_t* xbase = lds + ux * X_BYTES;
+                v4i w[4];
 #pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    const v4i a0 = *(const v4i*)(wbase + a_off + s * 1024);
-                    const v4i a1 = *(const v4i*)(wbase + a_off + 2048 + s * 1024);
+                for (int t = 0; t < 4; ++t) w[t] = *(const v4i*)(wbase + a_off + (t >> 1) * 2048 + (t & 1) * 256);
 #pragma unroll
-                    for (int b = 0; b < NBLK; ++b) {
-                        const v4i f = *(const v4i*)(xbase + (s ? frag_s1 : frag_s0) + b * 2048);
-                        acc[0][b] = mfma_i8(a0, f, acc[0][b]);
-                        acc[1][b] = mfma_i8(a1, f, acc[1][b]);
-                    }
+                for (int b = 0; b < 2 * NBLK; ++b) {
+                    const v4i f = *(const v4i*)(xbase + frag_off + b * 1024);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) acc[t][b] = mfma_i8_16(w[t], f, acc[t][b]);
                 }
             }
         };
@@ -623,23 +670,18 @@ __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_
     } else {
         // Tall tiles are bound by the matrix units, and every wavefront meets the others at the barrier of every K
         // block: operand reads that start behind that barrier leave all eight wavefronts, both of each SIMD, without
-        // an MFMA to issue until the first LDS answer is back.  So the operands stay one K step (32 values) ahead in
-        // registers, across the barrier: a block waits for the stage AFTER its own (one stage less of prefetch
-        // distance: the operands of a tall tile are L2 hits), runs its first K step on operands read during the block
-        // before, reads the second K step's under those MFMAs and the next block's first under the second's.  Reads
-        // and MFMAs are placed one by one (sched_barrier): an MFMA that waits for the matrix pipe holds up whatever
-        // is queued behind it in the wavefront.
-        v4i fa[2][2], fb[2][NBLK];  // [register set][tile] / [register set][token block]
-        auto read_operands = [&](int set, int uw, int ux, int s, int part) {
-            const int8_t* wbase = lds + uw * A_BYTES;
-            const int8_t* xbase = lds + ux * X_BYTES;
-            if (part == 0) {
-                fa[set][0] = *(const v4i*)(wbase + a_off + s * 1024);
-                fa[set][1] = *(const v4i*)(wbase + a_off + 2048 + s * 1024);
-                fb[set][0] = *(const v4i*)(xbase + (s ? frag_s1 : frag_s0));
-            } else {
-                fb[set][part] = *(const v4i*)(xbase + (s ? frag_s1 : frag_s0) + part * 2048);
-            }
+        // an MFMA to issue until the first LDS answer is back.  So the operands stay half a K block (64 of the 128
+        // tokens) ahead in registers, across the barrier: a block waits for the stage AFTER its own (one stage less of
+        // prefetch distance: the operands of a tall tile are L2 hits), runs its first half on operands read during the
+        // block before, reads the second half's tokens under those MFMAs and the next block's weights and first tokens
+        // under the second's.  Reads and MFMAs are placed one by one (sched_barrier): an MFMA that waits for the matrix
+        // pipe holds up whatever is queued behind it in the wavefront.
+        v4i fa[4], fb[2][NBLK];  // [16 channels] / [half][16 tokens]
+        auto read_weights = [&](int uw, int t) {
+            fa[t] = *(const v4i*)(lds + uw * A_BYTES + a_off + (t >> 1) * 2048 + (t & 1) * 256);
+        };
+        auto read_tokens = [&](int half, int ux, int b) {
+            fb[half][b] = *(const v4i*)(lds + ux * X_BYTES + frag_off + (half * NBLK + b) * 1024);
         };
         // the stage of K block 0 has landed (for everybody): its first operands
         auto wait_stage = [&]() {
@@ -661,7 +703,9 @@ __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_
         __builtin_amdgcn_s_barrier();
         if (active) {
 #pragma unroll
-            for (int part = 0; part < NBLK; ++part) read_operands(0, 0, 0, 0, part);
+            for (int t = 0; t < 4; ++t) read_weights(0, t);
+#pragma unroll
+            for (int b = 0; b < NBLK; ++b) read_tokens(0, 0, b);
         }
         auto step = [&](auto dtag, int uw, int ux, int it) {
             constexpr int D = decltype(dtag)::value;
@@ -670,20 +714,25 @@ __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_
             if constexpr (D >= SX - 1) load_tokens(it + SX - 1, (ux + SX - 1) % SX);
             if constexpr (D >= SW - 1) load_weights(it + SW - 1, (uw + SW - 1) % SW);
             if (active) {
-                // K step 0 on set 0, reading K step 1 into set 1
+                static_assert(NBLK == 4, "one token read beside every group of channels");
+                // the first half of the tokens, reading the second
 #pragma unroll
-                for (int b = 0; b < NBLK; ++b) {
-                    acc[0][b] = mfma_i8(fa[0][0], fb[0][b], acc[0][b]);
-                    acc[1][b] = mfma_i8(fa[0][1], fb[0][b], acc[1][b]);
-                    read_operands(1, uw, ux, 1, b);
+                for (int t = 0; t < 4; ++t) {
+#pragma unroll
+                    for (int b = 0; b < NBLK; ++b) acc[t][b] = mfma_i8_16(fa[t], fb[0][b], acc[t][b]);
+                    read_tokens(1, ux, t);
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                // K step 1 on set 1, reading the next block's K step 0 into set 0
+                // the second half, reading the next block's first tokens and, where they have just been used for the
+                // last time, its weights
 #pragma unroll
-                for (int b = 0; b < NBLK; ++b) {
-                    acc[0][b] = mfma_i8(fa[1][0], fb[1][b], acc[0][b]);
-                    acc[1][b] = mfma_i8(fa[1][1], fb[1][b], acc[1][b]);
-                    if constexpr (D > 0) read_operands(0, (uw + 1) % SW, (ux + 1) % SX, 0, b);
+                for (int t = 0; t < 4; ++t) {
+#pragma unroll
+                    for (int b = 0; b < NBLK; ++b) acc[t][NBLK + b] = mfma_i8_16(fa[t], fb[1][b], acc[t][NBLK + b]);
+                    if constexpr (D > 0) {
+                        read_tokens(0, (ux + 1) % SX, t);
+                        read_weights((uw + 1) % SW, t);
+                    }
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
