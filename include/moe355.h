@@ -504,7 +504,8 @@ int moe355_profile_next_gemm(void *start_event, void *stop_event);
 
 /* Which kernel family the int8 grouped GEMMs above launch for a shape, given a workspace of the size their
  * moe355_*_workspace() asks for: "gmm_stream_kernel" (few rows per expert), "gmm_tiled_kernel" (64- or 128-row
- * LDS-tiled), "gmm_wide_kernel" (weight-streaming tiles of up to 256 rows), "gmm_split_kernel" (one expert with some
+ * LDS-tiled), "gmm_resident_kernel" (dequant only, many rows per expert and a short K: 128-row tiles whose tokens stay in
+ * LDS), "gmm_wide_kernel" (weight-streaming tiles of up to 256 rows), "gmm_split_kernel" (one expert with some
  * hundreds of rows: 64 x 64 tiles that cut K over their wavefronts, no tile map) or "gmm_dense_kernel" (one expert with
  * thousands of rows: 256 x 256 tiles, no tile map); "" for arguments no GEMM accepts.
  * epilogue: 0 raw int32 (moe355_gmm_i32), 1 SwiGLU (moe355_gmm1_swiglu_quant), 2 dequant (moe355_gmm2_dequant).

@@ -199,3 +199,42 @@ def test_few_rows_on_tiles_few_channels(R, family):
 @pytest.mark.parametrize("E,family", [(63, "tiled"), (64, "wide")])
 def test_columns_of_wide_tiles(E, family):
     test_families_on_both_sides_of_a_line(64 * E, E, 4096, 576, family, True)
+
+
+# The down product with a tile's tokens in LDS: from 288 rows per expert and 512 workgroups of 128 rows x 1024 channels on, rows
+# of 256 to 896 values in steps of 128; experts of no row, of one, at the borders of half and whole tiles; channels that leave
+# every wavefront two groups of 64, some of them one or none
+@pytest.mark.parametrize("avg,E,Kd,N,family", [(287, 16, 256, 14400, "tiled"), (288, 16, 256, 14400, "resident"),
+                                               (512, 15, 384, 9216, "resident"), (400, 12, 896, 14400, "resident"),
+                                               (340, 12, 768, 17408, "resident"), (340, 12, 1024, 17408, "tiled"),
+                                               (340, 12, 704, 17408, "tiled"), (340, 12, 768, 16384, "tiled"),
+                                               (11000, 2, 256, 2112, "resident")])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_tokens_of_a_tile_in_lds(avg, E, Kd, N, family, dtype):
+    from oracle import oracle as orc
+    from vllm_ascend_amd import kernels as K
+    from vllm_ascend_amd._lib import W_ENK, load
+
+    R = avg * E
+    print(f"tokens in LDS R={R} E={E} K={Kd} N={N} {family} {dtype}", flush=True)
+    assert load().moe355_gmm_kernel_name(2, R, Kd, N, E).decode() == f"gmm_{family}_kernel"
+    counts = [0, 1, 63, 64, 65, 127, 128, 129] if E > 8 else []
+    rest = R - sum(counts)
+    counts += [rest // (E - len(counts))] * (E - len(counts) - 1)
+    counts += [R - sum(counts)]
+    cum = torch.tensor(counts).cumsum(0)
+    g = torch.Generator().manual_seed(R)
+    x = torch.randint(-128, 128, (R, Kd), generator=g, dtype=torch.int8)
+    w = torch.randint(-128, 128, (E, N, Kd), generator=g, dtype=torch.int8)
+    sw = torch.rand(E, N, generator=g) * 0.009 + 0.001
+    sx = torch.rand(R, generator=g) * 0.05 + 0.001
+    wnz = K.format_cast_nz(w.to("cuda"), W_ENK)
+    got = K.gmm2_dequant(x.to("cuda"), wnz, sw.to("cuda"), sx.to("cuda"), cum.to("cuda"), 0, N, Kd, out_dtype=dtype)
+    acc = K.gmm_i32(x.to("cuda"), wnz, cum.to("cuda"), 0, N, Kd)  # another kernel; some of its rows against the checker
+    for r in [0, 1, 64, 128, 321, R // 2, R - 129, R - 1]:
+        e = int(torch.searchsorted(cum, r, right=True))
+        want = orc.gmm_i32(x[r:r + 1].numpy(), w[e:e + 1].numpy(), np.array([1]))
+        assert np.array_equal(acc[r].cpu().numpy(), want[0])
+    at = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).to("cuda")
+    want = ((acc.float() * sx.to("cuda")[:, None]) * sw.to("cuda")[at]).to(dtype)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))

@@ -854,6 +854,7 @@ extern "C" const char* moe355_gmm_kernel_name(int epilogue, int64_t rows, int64_
     if (dense_tiles(a)) return "gmm_dense_kernel";
     if (split_tiles(a)) return "gmm_split_kernel";
     const int bm = gemm_family(a, true);  // as launch_gemm_auto decides
+    if (bm == 128 && epilogue == EPI_DEQUANT && resident_supported(a)) return "gmm_resident_kernel";
     return bm == 256 ? "gmm_wide_kernel" : bm ? "gmm_tiled_kernel" : "gmm_stream_kernel";
 }
 

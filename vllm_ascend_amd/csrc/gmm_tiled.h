@@ -17,6 +17,11 @@ TileSpec tile_spec(int64_t rows, int E, int BM, void* workspace);
 bool launch_tiled_any(int epi, int bm, const GmmArgs& a, void* workspace, hipStream_t st, hipEvent_t ev0,
                       hipEvent_t ev1);
 
+// The down product on the list of 128-row tiles (in the workspace) with a tile's tokens in LDS for the whole of K
+// (gmm_resident.hip).
+bool resident_supported(const GmmArgs& a);
+bool launch_resident(const GmmArgs& a, void* workspace, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1);
+
 // One expert owning every row: 64 x 64 tiles with K cut over the wavefronts (gmm_split.hip), no tile map either.
 void launch_split(int epi, const GmmArgs& a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1);
 

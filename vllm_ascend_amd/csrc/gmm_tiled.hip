@@ -942,7 +942,13 @@ bool launch_tiled_any(int epi, int bm, const GmmArgs& a, void* workspace, hipStr
     if (bm == 128) {
         if (epi == EPI_I32) MOE355_TILED(EPI_I32, 4);
         else if (epi == EPI_SWIGLU) MOE355_TILED(EPI_SWIGLU, 4);
-        else MOE355_TILED(EPI_DEQUANT, 4);
+        else if (resident_supported(a)) {
+            if (!a.tiles_ready) {
+                const TileSpec spec = tile_spec(a.R, a.E, bm, workspace);
+                hipLaunchKernelGGL(tile_map_kernel, dim3(1), dim3(256), 0, st, a.gl, a.gl_type, a.E, spec);
+            }
+            return launch_resident(a, workspace, st, ev0, ev1);
+        } else MOE355_TILED(EPI_DEQUANT, 4);
     } else {
         if (epi == EPI_I32) MOE355_TILED(EPI_I32, 2);
         else if (epi == EPI_SWIGLU) MOE355_TILED(EPI_SWIGLU, 2);
