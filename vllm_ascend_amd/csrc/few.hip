@@ -137,14 +137,7 @@ __device__ __forceinline__ void few_gate(const FewArgs& a, const GateCall& g, in
         const int at = part * 64 + lane;
         for (int i = at; i < nv; i += step * 64) {
             const v8u16 v = i == at ? held : xv[i];
-            uint32_t out[2] = {0u, 0u};
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float f = half_to_f32<XDT>(v[j]);
-                const int8_t b = amax == 0.0f ? (int8_t)0 : d.fast ? quantise_by_row<true>(f, d) : quantise_by_row<false>(f, d);
-                out[j >> 2] |= (uint32_t)(uint8_t)b << (8 * (j & 3));
-            }
-            *(uint2*)(q + i * 8) = make_uint2(out[0], out[1]);
+            *(uint2*)(q + i * 8) = d.fast ? quantise_by_row<true, XDT>(v, d) : quantise_by_row<false, XDT>(v, d);
         }
     }
     __syncthreads();
@@ -364,10 +357,8 @@ __device__ __forceinline__ float few_row_max(const FewArgs& a, int row, const Fe
 template <bool SHARED>
 __device__ __forceinline__ uint32_t few_pack(v4f v, float d)
 {
-    uint32_t pk = 0u;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) pk |= (uint32_t)(uint8_t)sat_rint_i8(SHARED ? v[j] / d : v[j] * d) << (8 * j);
-    return pk;
+    if constexpr (SHARED) return pack_low_bytes(sat_rint(v[0] / d), sat_rint(v[1] / d), sat_rint(v[2] / d), sat_rint(v[3] / d));
+    return quantise_times(v, d);
 }
 
 // ... by this.  A row of zeros: 0 * 0, 0 / inf (what else it holds is NaN, which quantises to zero)

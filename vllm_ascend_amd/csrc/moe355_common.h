@@ -121,13 +121,22 @@ __device__ __forceinline__ float m_silu(float g)
     return __builtin_amdgcn_div_fixupf(q1 * c, ds, g);
 }
 
-// clamp(rint(v), -128, 127) as int8
-__device__ __forceinline__ int8_t sat_rint_i8(float v)
+// clamp(rint(v), -128, 127), NaN -> 0.  The conversion saturates and turns NaN into 0, so the clamp is one instruction on
+// integers; and a row of nothing but zeros (and NaN) needs no case of its own where its values are multiplied by 1 / 0 or
+// divided by 0.
+__device__ __forceinline__ int sat_rint(float v)
 {
-    float r = __builtin_rintf(v);
-    r = r > 127.0f ? 127.0f : r;
-    r = r < -128.0f ? -128.0f : r;
-    return (int8_t)(int)r;
+    int i;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(i) : "v"(__builtin_rintf(v)));
+    i = i > 127 ? 127 : i;
+    return i < -128 ? -128 : i;
+}
+__device__ __forceinline__ int8_t sat_rint_i8(float v) { return (int8_t)sat_rint(v); }
+
+// the low bytes of four registers: three instructions, where shifts and masks take nine
+__device__ __forceinline__ uint32_t pack_low_bytes(uint32_t b0, uint32_t b1, uint32_t b2, uint32_t b3)
+{
+    return __builtin_amdgcn_perm(b1, b0, 0x0c0c0400) | __builtin_amdgcn_perm(b3, b2, 0x04000c0c);
 }
 
 // The token quantiser on 16-bit inputs: int8(rint(x / s)) for the values x of a row and the row's s = amax / 127.
@@ -154,17 +163,34 @@ __device__ __forceinline__ RowDivisor row_divisor(float s, bool ieee_only = fals
     return d;
 }
 
+// The int8 is the low byte of the result.
 template <bool FAST>
-__device__ __forceinline__ int8_t quantise_by_row(float x, const RowDivisor& d)
+__device__ __forceinline__ uint32_t quantise_by_row(float x, const RowDivisor& d)
 {
     if constexpr (FAST) {
         const float q0 = x * d.r;
         const float e = __builtin_fmaf(-d.s, q0, x);
-        // |x| <= amax keeps the quotient within +-127.00001: nothing to clamp
-        return (int8_t)(int)__builtin_rintf(__builtin_fmaf(e, d.r, q0));
+        // |x| <= amax keeps the quotient within +-127.00001: nothing to clamp, and 1.5 * 2^23 more rounds it to the integer
+        // (ties to even) that then fills the low bits.  NaN: the low 13 bits of a widened 16-bit value are zero.
+        return __float_as_uint(__builtin_fmaf(e, d.r, q0) + 12582912.0f);
     } else {
-        return sat_rint_i8(x / d.s);
+        return (uint32_t)sat_rint(x / d.s);
     }
+}
+
+template <bool FAST, int DT>
+__device__ __forceinline__ uint2 quantise_by_row(v8u16 v, const RowDivisor& d)
+{
+    uint32_t b[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) b[j] = quantise_by_row<FAST>(half_to_f32<DT>(v[j]), d);
+    return make_uint2(pack_low_bytes(b[0], b[1], b[2], b[3]), pack_low_bytes(b[4], b[5], b[6], b[7]));
+}
+
+// four fp32 values of a row times inv = 1 / scale
+__device__ __forceinline__ uint32_t quantise_times(v4f v, float inv)
+{
+    return pack_low_bytes(sat_rint(v[0] * inv), sat_rint(v[1] * inv), sat_rint(v[2] * inv), sat_rint(v[3] * inv));
 }
 
 __device__ __forceinline__ float wave_max(float v)
@@ -175,6 +201,25 @@ __device__ __forceinline__ float wave_max(float v)
         v = o > v ? o : v;
     }
     return v;
+}
+
+// max(m, |v|) as "v > m ? v : m" has it: NaN is passed over.  v_max3_f32 does two values in one instruction where a
+// comparison and a selection take four; only a signalling NaN (no arithmetic makes one, but memory may hold it) comes
+// through, so a caller whose maximum turns out NaN takes it again with max_abs_any.
+__device__ __forceinline__ float max_abs(float m, v4f v)
+{
+    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(v[0]), "v"(v[1]));
+    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(v[2]), "v"(v[3]));
+    return m;
+}
+__device__ __forceinline__ float max_abs_any(float m, v4f v)
+{
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float a = __builtin_fabsf(v[j]);
+        m = a > m ? a : m;
+    }
+    return m;
 }
 
 // What the lanes of a wavefront wrote to LDS before it, the others read behind it (and write over only behind it): no

@@ -60,14 +60,7 @@ __global__ __launch_bounds__(256) void dynamic_quant_kernel(const uint16_t* __re
 #pragma unroll
             for (int n = 0; n < NV; ++n) {
                 const int64_t i = threadIdx.x + 256 * n;
-                uint32_t w[2] = {0u, 0u};
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    int8_t b = (a == 0.0f) ? (int8_t)0
-                                           : quantise_by_row<decltype(fast)::value>(half_to_f32<DT>(held[n][j]), d);
-                    w[j >> 2] |= (uint32_t)(uint8_t)b << (8 * (j & 3));
-                }
-                if (i < nv) qv[i] = make_uint2(w[0], w[1]);
+                if (i < nv) qv[i] = quantise_by_row<decltype(fast)::value, DT>(held[n], d);
             }
         };
         if (d.fast) emit(std::true_type{});
@@ -102,18 +95,11 @@ __global__ __launch_bounds__(256) void dynamic_quant_kernel(const uint16_t* __re
             const v8u16* xv = (const v8u16*)xr;
             uint2* qv = (uint2*)qr;
             for (int64_t i = threadIdx.x; i < nv; i += 256) {
-                v8u16 v = xv[i];
-                uint32_t w[2] = {0u, 0u};
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    int8_t b = (a == 0.0f) ? (int8_t)0 : quantise_by_row<F>(half_to_f32<DT>(v[j]), d);
-                    w[j >> 2] |= (uint32_t)(uint8_t)b << (8 * (j & 3));
-                }
-                qv[i] = make_uint2(w[0], w[1]);
+                qv[i] = quantise_by_row<F, DT>(xv[i], d);
             }
         } else {
             for (int64_t i = threadIdx.x; i < cols; i += 256)
-                qr[i] = (a == 0.0f) ? (int8_t)0 : quantise_by_row<F>(half_to_f32<DT>(xr[i]), d);
+                qr[i] = (int8_t)quantise_by_row<F>(half_to_f32<DT>(xr[i]), d);
         }
     };
     if (d.fast) emit(std::true_type{});
@@ -174,7 +160,7 @@ __global__ __launch_bounds__(256) void dequant_swiglu_quant_kernel(const int32_t
     const float inv = 1.0f / s;
     if (threadIdx.x == 0) scale[row] = (a == 0.0f) ? 0.0f : s;
     int8_t* yr = y + row * half;
-    auto quantise = [&](float v) { return (a == 0.0f) ? (int8_t)0 : sat_rint_i8(form_b ? v / s : v * inv); };
+    auto quantise = [&](float v) { return sat_rint_i8(form_b ? v / s : v * inv); };
     if constexpr (NH > 0) {
 #pragma unroll
         for (int j = 0; j < NH; ++j) {
@@ -333,7 +319,7 @@ __global__ __launch_bounds__(256) void dequant_swiglu_quant_grouped_kernel(DsqAr
         const float s = amax * (float)(1.0 / 127.0);
         if (threadIdx.x == 0) a.scale[row] = (amax == 0.0f) ? 0.0f : s;
         for (int64_t i = threadIdx.x; i < half; i += 256)
-            yr[i] = (amax == 0.0f) ? (int8_t)0 : sat_rint_i8(value(i) / s);
+            yr[i] = sat_rint_i8(value(i) / s);
     } else {
         for (int64_t i = threadIdx.x; i < half; i += 256) {
             const float v = value(i);
@@ -423,7 +409,7 @@ __global__ __launch_bounds__(256) void act_mul_quant_kernel(const uint16_t* __re
     const float s = a / 127.0f;
     if (threadIdx.x == 0) scale[row] = (a == 0.0f) ? 0.0f : s;
     for (int64_t i = threadIdx.x; i < half; i += 256)
-        q[row * half + i] = (a == 0.0f) ? (int8_t)0 : sat_rint_i8(value(i) / s);
+        q[row * half + i] = sat_rint_i8(value(i) / s);
 }
 
 // out[i] = silu(g[i]) by the kernels' instruction sequence (form 0) or by the IEEE quotient (form 1)

@@ -247,15 +247,7 @@ __device__ __forceinline__ void gather_token_row(const uint16_t* __restrict__ xr
         if (threadIdx.x < top_k && drow[threadIdx.x] >= 0) sx[drow[threadIdx.x]] = (a == 0.0f) ? 0.0f : s;
         auto emit = [&](auto fast) {
             for (int64_t i = threadIdx.x; i < nv; i += 256) {
-                v8u16 v = i < 256 ? held : xv[i];
-                uint32_t w[2] = {0u, 0u};
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    int8_t b = (a == 0.0f) ? (int8_t)0
-                                           : quantise_by_row<decltype(fast)::value>(half_to_f32<DT>(v[j]), d);
-                    w[j >> 2] |= (uint32_t)(uint8_t)b << (8 * (j & 3));
-                }
-                const uint2 pk = make_uint2(w[0], w[1]);
+                const uint2 pk = quantise_by_row<decltype(fast)::value, DT>(i < 256 ? held : xv[i], d);
                 for (int j = 0; j < top_k; ++j)
                     if (drow[j] >= 0) ((uint2*)((int8_t*)xs + (int64_t)drow[j] * H))[i] = pk;
             }

@@ -78,15 +78,7 @@ __device__ __forceinline__ void quantise_token_row(const SmallRouteArgs& a, int 
     uint2* qv = (uint2*)(a.xq + (int64_t)t * a.H);
     auto emit = [&](auto fast) {
         for (int64_t i = tid; i < nv; i += kSmallThreads) {
-            const v8u16 v = i < kSmallThreads ? held : xv[i];
-            uint32_t w[2] = {0u, 0u};
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int8_t b = (amax == 0.0f) ? (int8_t)0
-                                                : quantise_by_row<decltype(fast)::value>(half_to_f32<DT>(v[j]), d);
-                w[j >> 2] |= (uint32_t)(uint8_t)b << (8 * (j & 3));
-            }
-            qv[i] = make_uint2(w[0], w[1]);
+            qv[i] = quantise_by_row<decltype(fast)::value, DT>(i < kSmallThreads ? held : xv[i], d);
         }
     };
     if (d.fast) emit(std::true_type{});
@@ -118,16 +110,8 @@ __device__ __forceinline__ void quantise_token_row_wave(const SmallRouteArgs& a,
     uint2* qv = (uint2*)(a.xq + (int64_t)t * a.H);
     auto emit = [&](auto fast) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            uint32_t w[2] = {0u, 0u};
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int8_t b = (amax == 0.0f) ? (int8_t)0
-                                                : quantise_by_row<decltype(fast)::value>(half_to_f32<DT>(held[i][j]), d);
-                w[j >> 2] |= (uint32_t)(uint8_t)b << (8 * (j & 3));
-            }
-            if (i * 64 + lane < nv) qv[i * 64 + lane] = make_uint2(w[0], w[1]);
-        }
+        for (int i = 0; i < 4; ++i)
+            if (i * 64 + lane < nv) qv[i * 64 + lane] = quantise_by_row<decltype(fast)::value, DT>(held[i], d);
     };
     if (d.fast) emit(std::true_type{});
     else emit(std::false_type{});
