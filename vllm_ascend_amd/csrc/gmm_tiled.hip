@@ -423,10 +423,10 @@ __global__ __launch_bounds__(256, (BMT <= 2 ? 3 : 2)) void gmm_tiled_kernel(GmmA
     int64_t row_end = tm.row_end[mt];
     if (row_end > a.R) row_end = a.R;
     if (row0 >= row_end) return;
-    // Tiles of up to 64 rows that are their expert's only one read its weights once, with non-temporal loads (the tiles
-    // of an expert follow one another in the list).  Qwen3 shape, whole layer, 300 / 777 tokens 146 / 167 -> 138 /
-    // 156 us, 1200 tokens under Zipf(1.1) 198 -> 172 us.  The same for full tiles, a fourth body in the kernel: 1200
-    // tokens uniform 198 -> 192 us, but 180 us under Zipf(1.1), where all four bodies run at once.
+    // Tiles that are their expert's only one read its weights once, with non-temporal loads (the tiles of an expert follow one
+    // another in the list).  Qwen3 shape, whole layer, 300 / 777 tokens 146 / 167 -> 138 / 156 us (short tiles); the products
+    // of 128 experts of 75 rows, 2048 / 1536 and 768 / 2048, 94.5 -> 91.0 and 51.5 -> 48.5, of 256 experts of 80 rows, 2048 /
+    // 7168, 721 -> 697 (full tiles); skewed batches, where all four bodies run at once, + 1 to - 1.4 %.
     const bool once = (mt == 0 || tm.expert[mt - 1] != e) && (mt + 1 == tm.count[0] || tm.expert[mt + 1] != e);
     if (row_end - row0 <= 64) {
         constexpr int SHORT = BMT > 2 ? 2 : BMT;
@@ -434,7 +434,8 @@ __global__ __launch_bounds__(256, (BMT <= 2 ? 3 : 2)) void gmm_tiled_kernel(GmmA
         else tiled_body<EPI, SHORT, RING, REM, false>(a, e, row0, row_end, nt, lds_raw);
         return;
     }
-    tiled_body<EPI, BMT, RING, REM, false>(a, e, row0, row_end, nt, lds_raw);
+    if (once) tiled_body<EPI, BMT, RING, REM, true>(a, e, row0, row_end, nt, lds_raw);
+    else tiled_body<EPI, BMT, RING, REM, false>(a, e, row0, row_end, nt, lds_raw);
 }
 
 // ------------------------------------------------------------------ weight-streaming tiles
@@ -467,9 +468,12 @@ __device__ __forceinline__ void wait_vmcnt()
 
 // NBLK: 32-row token blocks per wavefront (4 in a tall tile; 4, 5 or 6 in a wide one, so that an expert a little
 // above 128 rows keeps the wide shape instead of paying the token traffic of a tall tile).
+// once: the tile is its expert's only one, nobody else reads its weights: non-temporal loads, which stream from HBM at 7.1
+// TB/s where plain ones reach 6.3 (these copies alone, 256 experts of 4096 x 7168).  256 experts, 7168 / 4096, 80 / 128 rows
+// 1328 / 1362 -> 1175 / 1333 us; 2048 / 7168, 128 rows 757 -> 696.
 template <int EPI, bool WIDE, int NBLK = 4>
 __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_t row0, int64_t row_end, int nt,
-                                                 int8_t* lds)
+                                                 bool once, int8_t* lds)
 {
     static_assert(WIDE ? (NBLK >= 1 && NBLK <= 8) : NBLK == 4, "tall tiles have two halves of four blocks");
     constexpr int GROUPS = WIDE ? 8 : 4;            // channel groups (two storage tiles each) per workgroup
@@ -560,21 +564,12 @@ __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_
     // which the hand-written waits rely on, is the same in every step
     auto load_weights = [&](int it, int st) {
         const int itc = it < last_it ? it : last_it;
-        int8_t* base = lds + st * A_BYTES;
-        // plain cache policy: marked non-temporal, the same loads made the kernel 5 % slower
-        if constexpr (WIDE) {
+        int8_t* base = lds + st * A_BYTES + wave * (NA * 1024);
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const int8_t* wp = wsrc[t] + (int64_t)itc * 2048;
-                __builtin_amdgcn_global_load_lds(MOE355_GPTR(wp), MOE355_LPTR(base + wave * 4096 + t * 2048), 16, 0,
-                                                 0);
-                __builtin_amdgcn_global_load_lds(MOE355_GPTR(wp + 1024),
-                                                 MOE355_LPTR(base + wave * 4096 + t * 2048 + 1024), 16, 0, 0);
-            }
-        } else {
-            const int8_t* wp = wsrc[0] + (int64_t)itc * 2048;
-            __builtin_amdgcn_global_load_lds(MOE355_GPTR(wp), MOE355_LPTR(base + wave * 2048), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds(MOE355_GPTR(wp + 1024), MOE355_LPTR(base + wave * 2048 + 1024), 16, 0, 0);
+        for (int j = 0; j < NA; ++j) {
+            const int8_t* wp = wsrc[j / 2] + (int64_t)itc * 2048 + (j & 1) * 1024;
+            if (once) __builtin_amdgcn_global_load_lds(MOE355_GPTR(wp), MOE355_LPTR(base + j * 1024), 16, 0, 2 /* non-temporal */);
+            else __builtin_amdgcn_global_load_lds(MOE355_GPTR(wp), MOE355_LPTR(base + j * 1024), 16, 0, 0);
         }
     };
     auto load_tokens = [&](int it, int st) {
@@ -768,30 +763,32 @@ __global__ __launch_bounds__(512, 1) void gmm_wide_kernel(GmmArgs a, TileMap tm,
     const int col = slot % columns;
     if (mt >= max_tiles) return;
     const int count = tm.count[0];
-    const int e = tm.expert[mt];
+    const int listed = tm.expert[mt];
     const int64_t row0 = tm.row_begin[mt];
     int64_t row_end = tm.row_end[mt];
     if (mt >= count) return;
+    const int e = listed & ~kOnlyTile;
+    const bool once = listed & kOnlyTile;
     if (row_end > a.R) row_end = a.R;
     if (row0 >= row_end) return;
     // An expert of a few rows (the cold ones of a skewed batch) runs the same body with one or two token blocks:
     // the matrix units draw their power whether a block's rows exist or not, and the kernel's clock follows it.
     if (row_end - row0 <= 32) {
-        stream_tile_body<EPI, true, 1>(a, e, row0, row_end, col, wide_lds);
+        stream_tile_body<EPI, true, 1>(a, e, row0, row_end, col, once, wide_lds);
     } else if (row_end - row0 <= 64) {
-        stream_tile_body<EPI, true, 2>(a, e, row0, row_end, col, wide_lds);
+        stream_tile_body<EPI, true, 2>(a, e, row0, row_end, col, once, wide_lds);
     } else if (row_end - row0 <= 128) {
-        stream_tile_body<EPI, true>(a, e, row0, row_end, col, wide_lds);
+        stream_tile_body<EPI, true>(a, e, row0, row_end, col, once, wide_lds);
     } else if (row_end - row0 <= 160) {
-        stream_tile_body<EPI, true, 5>(a, e, row0, row_end, col, wide_lds);
+        stream_tile_body<EPI, true, 5>(a, e, row0, row_end, col, once, wide_lds);
     } else if (row_end - row0 <= 192) {
-        stream_tile_body<EPI, true, 6>(a, e, row0, row_end, col, wide_lds);
+        stream_tile_body<EPI, true, 6>(a, e, row0, row_end, col, once, wide_lds);
     } else {
         // a tall tile is one column block wide: the column's two blocks one after the other
-        stream_tile_body<EPI, false>(a, e, row0, row_end, 2 * col, wide_lds);
+        stream_tile_body<EPI, false>(a, e, row0, row_end, 2 * col, once, wide_lds);
         if (2 * col + 1 < n_col_blocks) {
             __syncthreads();  // the first block's epilogue is out of LDS
-            stream_tile_body<EPI, false>(a, e, row0, row_end, 2 * col + 1, wide_lds);
+            stream_tile_body<EPI, false>(a, e, row0, row_end, 2 * col + 1, once, wide_lds);
         }
     }
 }
@@ -815,7 +812,7 @@ __global__ __launch_bounds__(512, 1) void gmm_dense_kernel(GmmArgs a, int xn, in
     if (rows > a.R) rows = a.R;
     const int64_t row0 = (int64_t)mt * 256;
     if (row0 >= rows) return;
-    stream_tile_body<EPI, false>(a, 0, row0, rows, nt, wide_lds);
+    stream_tile_body<EPI, false>(a, 0, row0, rows, nt, false, wide_lds);
 }
 
 // ------------------------------------------------------------------ host side

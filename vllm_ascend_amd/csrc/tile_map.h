@@ -6,10 +6,13 @@
 
 namespace moe355 {
 
+// in the list by length: the tile is its expert's only one
+constexpr int32_t kOnlyTile = 1 << 30;
+
 // (expert, row block) tiles of one launch
 struct TileMap {
     int32_t* count;      // [1]
-    int32_t* expert;     // [max_tiles]
+    int32_t* expert;     // [max_tiles] (listed by length: and kOnlyTile)
     int32_t* row_begin;  // [max_tiles]
     int32_t* row_end;    // [max_tiles] end of the expert's rows
 };
@@ -70,7 +73,8 @@ __device__ __forceinline__ void build_tile_map(RowsOf rows_of, int E, const Tile
             const int e = e0 + j;
             if (e < E) {
                 const int64_t m = rows_of(e);
-                for (int64_t r0 = 0; r0 < m; r0 += BM) put(next[cls(m - r0)]++, e, row + r0, row + m);
+                for (int64_t r0 = 0; r0 < m; r0 += BM)
+                    put(next[cls(m - r0)]++, m <= BM ? e | kOnlyTile : e, row + r0, row + m);
                 row += m;
             }
         }
