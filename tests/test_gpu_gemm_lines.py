@@ -238,3 +238,10 @@ def test_tokens_of_a_tile_in_lds(avg, E, Kd, N, family, dtype):
     at = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).to("cuda")
     want = ((acc.float() * sx.to("cuda")[:, None]) * sw.to("cuda")[at]).to(dtype)
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+# Weight-streaming tiles for a product with ten columns of them and more per expert, up to 256 rows per expert: tall tiles
+@pytest.mark.parametrize("avg,E,N,family", [(144, 64, 5120, "wide"), (145, 64, 5120, "tiled"), (145, 77, 5120, "wide"),
+                                            (256, 77, 5120, "wide"), (257, 77, 5120, "tiled"), (145, 96, 5056, "tiled")])
+def test_rows_of_weight_streaming_tiles(avg, E, N, family):
+    test_tokens_of_a_tile_in_lds(avg, E, 2048, N, family, torch.bfloat16)

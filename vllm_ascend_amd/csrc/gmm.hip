@@ -656,6 +656,10 @@ static int tiled_bm(const GmmArgs& a)
     // 2091 / 2126 / 2280 us with the weight-streaming tiles in the first product, 1867 / 1975 / 2031 / 2088 / 2162 / 2512
     // us on 128-row tiles; Zipf(1.1) at 28 / 40 / 64 / 94 / 128 1115 / 1361 / 1703 / 2164 / 2616 against 1069 / 1339 /
     // 1667 / 2155 / 2648.  128 experts at K = 4096, 56 / 69 / 81 rows: 526 / 547 / 567 against 511 / 552 / 576.
+    // Since then tiles that are their expert's only one read its weights past the caches, and the wide tiles, bound by that
+    // stream, win a little earlier in uniform routing, not under Zipf(1.1): the same layer, 44 / 50 / 56 rows 1896 / 2020 /
+    // 2032 us on 128-row tiles, 1869 / 1951 / 1895 on wide ones, Zipf 1435 / 1545 / 1654 against 1464 / 1600 / 1633; 128
+    // experts at K = 4096, 40 to 64 rows, 0.96 to 0.99 of the time and 1.04 to 1.10.  So the line stays at 64.
     // A handful of wide tiles leaves most of the chip idle: 8 experts, K = 4096 / 2048 (64 columns of tiles), 500 / 800 / 1000
     // tokens of two slots 123 / 159 / 169 us with them, 99 / 102 / 126 on 128-row tiles (Zipf(1.1) 154 / 159 / 172 against 97 /
     // 104 / 136); 16 experts (128 columns), 600 / 1000 / 1500 tokens 136 / 160 / 193 against 120 / 168 / 160; 32 experts 196 /
@@ -675,8 +679,17 @@ static int tiled_bm(const GmmArgs& a)
     // Products of up to 512 channels are on the wide tiles from 96 to 192 rows (from 64 to 256 if K is long) at any number of
     // columns, and behind the others there: K / N = 1024 / 512, 128 rows, 8 and 128 experts 25 and 29 us against 13 and 31 on
     // 64-row tiles and 14 and 31 on 128-row tiles (Zipf 34 and 48 against 14 and 34, 14 and 30).  Left as it is as well.
+    // From 144 rows on nearly every expert has a second tile, which comes out of the last-level cache.  Uniform routing still
+    // wins there, at any shape; under Zipf(1.1) the hot expert's tall tiles are the end of the launch unless there are many
+    // columns of them for each expert.  One product, wide / 128-row tiles: K = 2048, N = 7168 (14 columns per expert), 256
+    // experts, 144 / 160 / 192 / 224 / 250 rows 0.78 / 0.80 / 0.84 / 0.88 / 0.94 (160 rows 826 against 1035 us), Zipf 1.02
+    // / 1.00 / 0.97 / 0.97 / 0.97; 128 experts, 160 / 192 / 224 rows 0.79 / 0.84 / 0.87, Zipf 1.00 / 0.94 / 0.92; 64 experts,
+    // 160 / 208 rows 0.84 / 0.91, Zipf 1.00 / 1.01; 128 experts of K = 3072, N = 5120 (10 columns), 150 / 200 / 250 rows 0.73 /
+    // 0.83 / 0.91, Zipf 1.04 / 0.98 / 1.00.  With eight columns or fewer (N = 4096, 2048, 1024) 0.79 to 1.07 and 1.01 to
+    // 1.15: 144 rows there.
     const bool fills = narrow || columns >= kComputeUnits;
-    if (avg >= (narrow ? 96 : 112) && avg <= (narrow ? 192 : 144) && a.K >= 1024 && wide_ok && fills) return 256;
+    const int64_t most = narrow ? 192 : a.K >= 2048 && a.N >= 5120 && columns >= 3 * kComputeUnits ? 256 : 144;
+    if (avg >= (narrow ? 96 : 112) && avg <= most && a.K >= 1024 && wide_ok && fills) return 256;
     return 128;
 }
 
