@@ -32,3 +32,12 @@ def test_maps_equal_a_stable_sort(tokens, k, experts, skew):
         assert np.array_equal(dst.cpu().numpy(), want_dst)
         assert np.array_equal(row_token.cpu().numpy()[: order.size], order // k)
         assert np.array_equal(num.cpu().numpy(), counts if kind == 1 else np.cumsum(counts))
+
+
+# from 20480 pairs on, four ids per load: one pair less, remainders of one to three, the last one alone in its 4096; 16 and 8
+# counters per expert (256 / 257 experts, one)
+@pytest.mark.parametrize("skew", ["uniform", "one expert", "dropped"])
+@pytest.mark.parametrize("tokens, k, experts", [(20479, 1, 256), (20480, 1, 256), (20481, 1, 257), (4097, 5, 1), (10241, 2, 512),
+                                                (32767, 1, 64), (32769, 1, 64), (65535, 1, 128)])
+def test_maps_of_many_pairs(tokens, k, experts, skew):
+    test_maps_equal_a_stable_sort(tokens, k, experts, skew)

@@ -322,7 +322,7 @@ __global__ __launch_bounds__(256) void route_gather_small_kernel(const int32_t* 
 // (launches of 4.5 us each otherwise): they do the same counting for their row counts.
 struct RouteMapArgs {
     const int32_t* ids;
-    int R, E, top_k, tokens_num_type, nbits, chunks, nspecs;
+    int R, E, top_k, tokens_num_type, nbits, chunks, nspecs, columns;
     int32_t* dst;
     int32_t* row_token;
     int64_t* expert_tokens;
@@ -332,47 +332,103 @@ constexpr int kMapThreads = 1024;
 constexpr int kMapWaves = kMapThreads / 64;
 constexpr int kMapMaxExperts = 512;
 constexpr int kMapMaxPairs = 65536;
+typedef int32_t v4i_any __attribute__((ext_vector_type(4), aligned(4)));
 
+// MANY (from 20480 pairs on): the counting is the kernel.  Four ids per load, and an expert has 16 counters (8 with
+// more than 256 experts) for the lanes to share: lanes that add to one word take turns, under uniform routing because
+// several of a wavefront's 64 pairs meet in a bank, under skewed routing because they have the same expert.  65536
+// pairs of 128 experts, alone 11.5 -> 9.6 us, Zipf(1.1) 18.6 -> 9.6, behind the gating that writes the ids 16.0 ->
+// 12.4; 32768 pairs of 256 experts 7.9 -> 7.5 and 11.0 -> 7.4; 20480 and 24000 pairs 6.8 -> 6.6 and 6.9 -> 6.8; 16384
+// pairs would take 6.4 instead of 6.1 (Zipf 6.3 instead of 8.0), and fewer are launch, first loads and scan, to which
+// clearing and adding up the counters is 0.3 to 0.8 us of 5 more. (A uniform prefill of 8192 tokens as a whole takes as
+// long as before: at its power limit, what this launch leaves to the others is a rest of 4 us less.  Under Zipf(1.1)
+// 309.4 -> 306.4 us at 4000 tokens.)
+template <bool MANY>
 __global__ __launch_bounds__(kMapThreads) void route_map_kernel(RouteMapArgs a)
 {
     extern __shared__ int32_t map_lds[];
-    int32_t* count = map_lds;          // [E] pairs of every expert: in front of this chunk << 16 | the rest
-    int32_t* part = count + a.E;       // [32] scan scratch
-    int32_t* whist = part + 32;        // [16][E] pairs of every wavefront, then the first row of its pairs
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int E = a.E, R = a.R;
+    const int columns = MANY ? a.columns : 0;
+    int32_t* split = map_lds;             // MANY: [E][columns] what `count` is the sum of
+    int32_t* count = split + E * columns;  // [E] pairs of every expert: in front of this chunk << 16 | the rest
+    int32_t* part = count + E;             // [32] scan scratch
+    int32_t* whist = part + 32;            // [16][E] pairs of every wavefront, then the first row of its pairs
     const bool maps = (int)blockIdx.x >= a.chunks;  // a tile map instead of a chunk
     const int begin = maps ? 0 : (int)blockIdx.x * kMapThreads;
-    for (int i = tid; i < E; i += kMapThreads) count[i] = 0;
+    for (int i = tid; i < (MANY ? E * columns : E); i += kMapThreads) map_lds[i] = 0;
     if (!maps)
         for (int i = tid; i < kMapWaves * E; i += kMapThreads) whist[i] = 0;
     __syncthreads();
     int mine = -1;  // this thread's pair of the chunk
-    int next[8];  // the ids of the next 8192 pairs are requested in front of the counting of these (15.9 -> 14.7 us at 65536)
+    if constexpr (MANY) {
+        // eight loads (32768 pairs) in flight in front of the counting of those before them; the last threads read the
+        // last four pairs and skip those that are their neighbour's
+        auto first_of = [&](int f) { return f < R - 4 ? f : R - 4; };
+        v4i_any next[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) next[j] = j * kMapThreads + tid < R ? a.ids[j * kMapThreads + tid] : -1;
-    for (int base = 0; base < R; base += 8 * kMapThreads) {
-        int id[8];
+        for (int j = 0; j < 8; ++j) next[j] = *(const v4i_any*)(a.ids + first_of((j * kMapThreads + tid) * 4));
+        if (!maps && begin + tid < R) mine = a.ids[begin + tid];
+        int32_t* at = split + (lane & (columns - 1));
+        for (int base = 0; base < R; base += 32 * kMapThreads) {
+            v4i_any id[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) id[j] = next[j];
-        if (base + 8 * kMapThreads < R) {
+            for (int j = 0; j < 8; ++j) id[j] = next[j];
+            if (base + 32 * kMapThreads < R) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    next[j] = *(const v4i_any*)(a.ids + first_of(base + ((8 + j) * kMapThreads + tid) * 4));
+            }
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                const int f = base + (8 + j) * kMapThreads + tid;
-                next[j] = f < R ? a.ids[f] : -1;
+                if (base + j * 4 * kMapThreads >= R) break;
+                const int f = base + (j * kMapThreads + tid) * 4;  // four pairs of one chunk
+                const int skip = f - first_of(f);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int e = id[j][q];
+                    if (q < skip || (uint32_t)e >= (uint32_t)E) continue;
+                    atomicAdd(&at[e * columns], f < begin ? 0x10000 : 1);
+                }
             }
         }
+    } else {
+        int next[8];  // the ids of the next 8192 pairs are requested in front of the counting of these
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int f0 = base + j * kMapThreads;  // a multiple of 1024: a whole chunk
-            const int e = id[j];
-            if (e >= 0 && e < E) atomicAdd(&count[e], f0 < begin ? 0x10000 : 1);
-            if (f0 == begin) mine = e;
+        for (int j = 0; j < 8; ++j) next[j] = j * kMapThreads + tid < R ? a.ids[j * kMapThreads + tid] : -1;
+        for (int base = 0; base < R; base += 8 * kMapThreads) {
+            int id[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) id[j] = next[j];
+            if (base + 8 * kMapThreads < R) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int f = base + (8 + j) * kMapThreads + tid;
+                    next[j] = f < R ? a.ids[f] : -1;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int f0 = base + j * kMapThreads;  // a multiple of 1024: a whole chunk
+                const int e = id[j];
+                if (e >= 0 && e < E) atomicAdd(&count[e], f0 < begin ? 0x10000 : 1);
+                if (f0 == begin) mine = e;
+            }
         }
     }
     if (mine < 0 || mine >= E) mine = -1;
     if (!maps && mine >= 0) atomicAdd(&whist[wave * E + mine], 1);
     __syncthreads();
+    if constexpr (MANY) {  // columns / 4 neighbouring lanes add up an expert
+        const int lanes = columns / 4;
+        for (int i = tid; i < E * lanes; i += kMapThreads) {
+            const v4i v = ((const v4i*)split)[i];
+            int n = v[0] + v[1] + v[2] + v[3];
+            for (int d = 1; d < lanes; d <<= 1) n += __shfl_xor(n, d);
+            if (i % lanes == 0) count[i / lanes] = n;
+        }
+        __syncthreads();
+    }
     // at most 65536 pairs: only in a chunk that has none in front of it may the rest need more than 16 bits
     auto in_front = [&](int e) { return begin == 0 ? 0 : (int)((uint32_t)count[e] >> 16); };
     auto total = [&](int e) { return begin == 0 ? count[e] : (count[e] & 0xffff) + in_front(e); };
@@ -588,9 +644,12 @@ int moe355::route_map_impl(const int32_t* expert_idx, int64_t num_tokens, int to
         a.row_token = row_token;
         a.expert_tokens = expert_tokens;
         for (int i = 0; i < nspecs; ++i) a.specs[i] = specs[i];
-        const size_t lds = ((size_t)(kMapWaves + 1) * num_experts + 32) * 4;  // at most 35 KB
-        hipLaunchKernelGGL(route_map_kernel, dim3((unsigned)(a.chunks + nspecs)), dim3(kMapThreads), lds,
-                           (hipStream_t)stream, a);
+        const bool many = R >= 20480;
+        a.columns = many ? (num_experts <= 256 ? 16 : 8) : 0;
+        const size_t lds = ((size_t)(kMapWaves + 1 + a.columns) * num_experts + 32) * 4;  // at most 51 KB
+        const dim3 grid((unsigned)(a.chunks + nspecs));
+        if (many) hipLaunchKernelGGL(route_map_kernel<true>, grid, dim3(kMapThreads), lds, (hipStream_t)stream, a);
+        else hipLaunchKernelGGL(route_map_kernel<false>, grid, dim3(kMapThreads), lds, (hipStream_t)stream, a);
         if (built) *built = true;
         return launch_status();
     }
