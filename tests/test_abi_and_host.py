@@ -495,6 +495,18 @@ def test_few_streaming_workgroups_keep_streaming(experts, k, n, first):
         assert name(epilogue, first * experts, k, n, experts) == b"gmm_tiled_kernel"
 
 
+# a long K and 2048 columns of weight-streaming tiles: these above 351 rows per expert as well as from 64 to 256
+@pytest.mark.parametrize("experts, k, n, family", [(256, 7168, 4096, "wide"), (255, 7168, 4096, "tiled"), (256, 7104, 4096, "tiled"),
+                                                   (256, 7168, 3584, "tiled")])
+def test_weight_streaming_tiles_of_many_rows(experts, k, n, family):
+    from vllm_ascend_amd import _lib
+
+    name = _lib.load().moe355_gmm_kernel_name
+    for epilogue in (0, 1, 2):
+        for rows, want in ((63, "tiled"), (64, "wide"), (256, "wide"), (257, "tiled"), (351, "tiled"), (352, family), (2000, family)):
+            assert name(epilogue, rows * experts, k, n, experts).decode() == f"gmm_{want}_kernel"
+
+
 # one for every 56 pairs, but not where a short launch (fewer than 1536 units of 64 channels) has places in front of its slots
 # (from two pairs per expert on), nor from twelve pairs per expert on
 @pytest.mark.parametrize("experts, n, pairs, blocks", [(128, 1536, 512, 9), (128, 512, 256, 4), (128, 512, 257, 0), (128, 704, 512, 0),

@@ -666,7 +666,15 @@ static int tiled_bm(const GmmArgs& a)
     // 215 / 272 against 196 / 262 / 276.  (One expert: a dense product on a side stream, which should leave the chip idle.)
     const bool narrow = a.N <= 512;
     const int64_t columns = (int64_t)a.E * ((a.N + 511) / 512);
-    if (avg >= 64 && avg <= 256 && a.K >= 4096 && wide_ok && (narrow || a.E == 1 || columns >= kComputeUnits / 2)) return 256;
+    // Above 256 rows an expert has two tall tiles and more.  They are bound by the matrix units like the 128-row tiles, at half
+    // their weight traffic from L2, and win where a long K leaves that traffic the larger part.  The first product alone, wide /
+    // 128-row tiles, 256 experts, K = 7168, N = 4096 at 264 / 288 / 320 / 384 / 448 / 512 / 640 / 1024 rows: 0.95 / 1.01 / 0.99
+    // / 0.92 / 0.92 / 0.93 / 0.92 / 0.91 (512 rows 4610 against 4980 us), Zipf(1.1) at 288 / 384 / 512 0.97 / 0.94 / 0.95.  With
+    // 256 columns of tiles (32 experts) 384 and 512 rows 0.90 and 0.91, Zipf 1.14 and 1.00; at K = 4096, 288 / 384 / 512 rows,
+    // 1.07 / 1.00 / 1.01, Zipf 1.06 / 1.08 / 1.05: neither.
+    const bool tall = avg >= 352 && a.K >= 7168 && columns >= 8 * kComputeUnits;
+    if (avg >= 64 && (avg <= 256 || tall) && a.K >= 4096 && wide_ok && (narrow || a.E == 1 || columns >= kComputeUnits / 2))
+        return 256;
     // Around 128 rows per expert most experts fit one wide tile of 128 or 160 rows and fetch their weights once, which
     // pays from K = 1024 on if the experts are about equally popular and there are enough of them to fill the chip.  128
     // experts, K = 2048 / 768, the layer at 100 / 112 / 128 / 144 / 160 / 192 rows per expert: 201 / 210 / 224 / 241 / 260 /
