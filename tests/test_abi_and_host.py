@@ -495,15 +495,19 @@ def test_few_streaming_workgroups_keep_streaming(experts, k, n, first):
         assert name(epilogue, first * experts, k, n, experts) == b"gmm_tiled_kernel"
 
 
-# a long K and 2048 columns of weight-streaming tiles: these above 351 rows per expert as well as from 64 to 256
-@pytest.mark.parametrize("experts, k, n, family", [(256, 7168, 4096, "wide"), (255, 7168, 4096, "tiled"), (256, 7104, 4096, "tiled"),
-                                                   (256, 7168, 3584, "tiled")])
-def test_weight_streaming_tiles_of_many_rows(experts, k, n, family):
+# above 256 rows per expert: weight-streaming tiles for weights of 32 MiB an expert, from 384 rows on of 14 MiB (at least 5120
+# channels; fewer at K from 7168 on with 2048 columns of tiles)
+@pytest.mark.parametrize("experts, k, n, first", [(16, 4096, 8192, 257), (15, 4096, 8192, None), (32, 4096, 8128, 384),
+                                                  (64, 2048, 7168, 384), (64, 2048, 7104, None), (64, 3072, 5056, None),
+                                                  (18, 2048, 7168, None), (19, 2048, 7168, 384), (64, 1984, 16384, None),
+                                                  (256, 7168, 4096, 384), (255, 7168, 4096, None), (256, 7104, 4096, None)])
+def test_weight_streaming_tiles_of_many_rows(experts, k, n, first):
     from vllm_ascend_amd import _lib
 
     name = _lib.load().moe355_gmm_kernel_name
     for epilogue in (0, 1, 2):
-        for rows, want in ((63, "tiled"), (64, "wide"), (256, "wide"), (257, "tiled"), (351, "tiled"), (352, family), (2000, family)):
+        for rows in (257, 383, 384, 2000):
+            want = "wide" if first and rows >= first else "tiled"
             assert name(epilogue, rows * experts, k, n, experts).decode() == f"gmm_{want}_kernel"
 
 

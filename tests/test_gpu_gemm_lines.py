@@ -245,3 +245,10 @@ def test_tokens_of_a_tile_in_lds(avg, E, Kd, N, family, dtype):
                                             (256, 77, 5120, "wide"), (257, 77, 5120, "tiled"), (145, 96, 5056, "tiled")])
 def test_rows_of_weight_streaming_tiles(avg, E, N, family):
     test_tokens_of_a_tile_in_lds(avg, E, 2048, N, family, torch.bfloat16)
+
+
+# and of several tall tiles per expert, where an expert's weights are several times an XCD's L2
+@pytest.mark.parametrize("avg,E,Kd,N,family", [(257, 16, 4096, 8192, "wide"), (383, 19, 2048, 7168, "tiled"),
+                                               (384, 19, 2048, 7168, "wide"), (700, 19, 2048, 7232, "wide")])
+def test_several_weight_streaming_tiles_of_an_expert(avg, E, Kd, N, family):
+    test_tokens_of_a_tile_in_lds(avg, E, Kd, N, family, torch.bfloat16)

@@ -666,15 +666,23 @@ static int tiled_bm(const GmmArgs& a)
     // 215 / 272 against 196 / 262 / 276.  (One expert: a dense product on a side stream, which should leave the chip idle.)
     const bool narrow = a.N <= 512;
     const int64_t columns = (int64_t)a.E * ((a.N + 511) / 512);
-    // Above 256 rows an expert has two tall tiles and more.  They are bound by the matrix units like the 128-row tiles, at half
-    // their weight traffic from L2, and win where a long K leaves that traffic the larger part.  The first product alone, wide /
-    // 128-row tiles, 256 experts, K = 7168, N = 4096 at 264 / 288 / 320 / 384 / 448 / 512 / 640 / 1024 rows: 0.95 / 1.01 / 0.99
-    // / 0.92 / 0.92 / 0.93 / 0.92 / 0.91 (512 rows 4610 against 4980 us), Zipf(1.1) at 288 / 384 / 512 0.97 / 0.94 / 0.95.  With
-    // 256 columns of tiles (32 experts) 384 and 512 rows 0.90 and 0.91, Zipf 1.14 and 1.00; at K = 4096, 288 / 384 / 512 rows,
-    // 1.07 / 1.00 / 1.01, Zipf 1.06 / 1.08 / 1.05: neither.
-    const bool tall = avg >= 352 && a.K >= 7168 && columns >= 8 * kComputeUnits;
-    if (avg >= 64 && (avg <= 256 || tall) && a.K >= 4096 && wide_ok && (narrow || a.E == 1 || columns >= kComputeUnits / 2))
-        return 256;
+    if (avg >= 64 && avg <= 256 && a.K >= 4096 && wide_ok && (narrow || a.E == 1 || columns >= kComputeUnits / 2)) return 256;
+    // Above 256 rows an expert has two tall tiles and more, and they fetch its weights half as often as the 128-row tiles.  That
+    // is what counts where an expert's weights are several times the 4 MiB of an XCD's L2.  One product, wide / 128-row tiles:
+    //   32 MiB and more per expert at K >= 4096: 16 experts of 14336 x 4096, 264 / 352 / 512 / 1024 rows 0.79 / 0.78 / 0.69 /
+    //     0.65 (991 against 681 us at 512), Zipf(1.1) 1.00 / 0.83 / 0.80 / 0.78; 64 of 8192 x 5120 0.77 / 0.81 / 0.71 / 0.69, Zipf
+    //     0.91 / 0.87 / 0.82 / 0.75; 32 of 8192 x 4096 0.85 / 0.91 / 0.86 / 0.84, Zipf 0.93 / 0.91 / 0.89 / 0.87.
+    //   14 MiB and more, from 384 rows on (two tiles of 256 are mostly padding before): 256 experts of 7168 x 2048, 352 / 384 /
+    //     512 / 1024 rows 1.05 / 0.95 / 0.93 / 0.89, Zipf 0.94 / 0.90 at 384 / 512; 64 of them 1.05 / 0.96 / 0.93 / 0.89, Zipf
+    //     0.92 / 0.97 / 0.95 / 0.89; 128 of 5120 x 3072 0.97 / 0.95 / 0.93 at 384 / 512 / 1024, Zipf 0.97 / 0.93 / 0.92.  Ten
+    //     MiB (5120 x 2048) 1.05, Zipf 1.00 to 1.04.
+    //   Fewer channels than 5120 only at the longest K and with many columns: 256 experts of 4096 x 7168, 288 / 320 / 384 / 512 /
+    //     1024 rows 1.01 / 0.99 / 0.92 / 0.93 / 0.91 (512 rows 4980 against 4610 us), Zipf 0.94 / 0.95 at 384 / 512; 32 of them
+    //     0.90 / 0.91 but Zipf 1.14 / 1.00; 4096 x 4096 0.97 to 1.01, Zipf 0.99 to 1.08.
+    const int64_t own = (int64_t)a.N * a.K;
+    const bool tall = a.N >= 5120 ? own >= (14 << 20) : a.K >= 7168 && columns >= 8 * kComputeUnits;
+    if (avg > 256 && a.K >= 2048 && wide_ok && columns >= kComputeUnits
+        && ((a.K >= 4096 && own >= (32 << 20)) || (avg >= 384 && tall))) return 256;
     // Around 128 rows per expert most experts fit one wide tile of 128 or 160 rows and fetch their weights once, which
     // pays from K = 1024 on if the experts are about equally popular and there are enough of them to fill the chip.  128
     // experts, K = 2048 / 768, the layer at 100 / 112 / 128 / 144 / 160 / 192 rows per expert: 201 / 210 / 224 / 241 / 260 /
