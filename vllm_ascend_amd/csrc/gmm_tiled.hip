@@ -434,7 +434,10 @@ __global__ __launch_bounds__(256, (BMT <= 2 ? 3 : 2)) void gmm_tiled_kernel(GmmA
         else tiled_body<EPI, SHORT, RING, REM, false>(a, e, row0, row_end, nt, lds_raw);
         return;
     }
-    if (once) tiled_body<EPI, BMT, RING, REM, true>(a, e, row0, row_end, nt, lds_raw);
+    // With a short K full tiles that way only where they are many: a few among short ones are the last to end.  128 experts of
+    // 2048 / 768, the layer with non-temporal / plain full tiles at 49 / 53 / 59 / 66 / 75 rows per expert 1.01 / 1.01 / 0.98 /
+    // 0.97 / 0.97; 256 experts of 7168 / 2048, 47 rows 0.98.
+    if (once && (a.K >= 4096 || a.R >= 56 * (int64_t)a.E)) tiled_body<EPI, BMT, RING, REM, true>(a, e, row0, row_end, nt, lds_raw);
     else tiled_body<EPI, BMT, RING, REM, false>(a, e, row0, row_end, nt, lds_raw);
 }
 
