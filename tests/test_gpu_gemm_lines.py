@@ -230,7 +230,7 @@ def test_tokens_of_a_tile_in_lds(avg, E, Kd, N, family, dtype):
     sx = torch.rand(R, generator=g) * 0.05 + 0.001
     wnz = K.format_cast_nz(w.to("cuda"), W_ENK)
     got = K.gmm2_dequant(x.to("cuda"), wnz, sw.to("cuda"), sx.to("cuda"), cum.to("cuda"), 0, N, Kd, out_dtype=dtype)
-    acc = K.gmm_i32(x.to("cuda"), wnz, cum.to("cuda"), 0, N, Kd)  # another kernel; some of its rows against the checker
+    acc = K.gmm_i32(x.to("cuda"), wnz, cum.to("cuda"), 0, N, Kd)  # some of its rows against the oracle
     for r in [0, 1, 64, 128, 321, R // 2, R - 129, R - 1]:
         e = int(torch.searchsorted(cum, r, right=True))
         want = orc.gmm_i32(x[r:r + 1].numpy(), w[e:e + 1].numpy(), np.array([1]))
