@@ -71,6 +71,35 @@ def test_requantising_down_gemm_gives_the_separate_launches_bits(T, E, I):
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
+# ... y is a caller's: the maximum of a row passes over its NaNs, quiet and signalling, in each of the four places of a load and
+# on either side of the row's largest value
+@pytest.mark.parametrize("bits", [0x7fc00000, 0x7f800001, 0xffa00000], ids=["quiet", "signalling", "negative"])
+@pytest.mark.parametrize("I", [64, 768, 1500 // 32 * 32])
+def test_nan_beside_a_row_s_largest_value(I, bits):
+    from vllm_ascend_amd import kernels as K
+    from vllm_ascend_amd._lib import W_ENK
+
+    T, k, E, H = 8, 4, 128, 1024
+    print(f"nan in y I={I} {bits:#x}", flush=True)
+    assert K.gmm2_requant_pairs_supported(T, k, H, I, E)
+    g = torch.Generator().manual_seed(I)
+    y = torch.randn(T * k, I, generator=g)
+    for r in range(T * k):  # the largest value in place r % 4 of a load, a NaN in r / 4 % 4, one load apart in the last rows
+        at = (r * 20 + 4 * (r // 8)) % (I - 8) // 4 * 4
+        y[r, at + r % 4] = 50.0 + r
+        y.view(torch.int32)[r, at + r // 4 % 4 + (4 if r >= 16 or r % 4 == r // 4 % 4 else 0)] = bits - (bits >> 31 << 32)
+    known = torch.where(y.isnan(), 0.0, y).abs().amax(1)
+    scale = known / 127.0
+    q = torch.where(y.isnan(), 0.0, (y * (1.0 / scale)[:, None]).round().clamp(-128, 127)).to(torch.int8)
+    ids = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)]).to(torch.int32).to("cuda")
+    w2 = K.format_cast_nz(torch.randint(-128, 128, (E, H, I), generator=g, dtype=torch.int8).to("cuda"), W_ENK)
+    s2 = (torch.rand(E, H, generator=g) * 0.009 + 0.001).to("cuda")
+    want = K.gmm2_dequant_pairs(q.to("cuda"), w2, s2, scale.to("cuda"), ids, H, I)
+    got = K.gmm2_requant_dequant_pairs(y.to("cuda"), w2, s2, ids, H, I)
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 # token quantisation with a row per wavefront: from 512 tokens on, rows of up to 2048 values, a last workgroup that is
 # not full
 @pytest.mark.parametrize("T,H", [(511, 2048), (512, 2048), (515, 1032), (513, 8), (777, 2056)])

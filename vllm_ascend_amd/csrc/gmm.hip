@@ -348,10 +348,11 @@ __global__ __launch_bounds__(256, OCC) void gmm_stream_kernel(GmmArgs a)
                 }
 #pragma unroll
                 for (int t = 0; t < REQ_ROWS; ++t) {
+                    bool nan = false;
                     amax[t] = 0.0f;
 #pragma unroll
-                    for (int i = 0; i < REQ_VEC; ++i) amax[t] = max_abs(amax[t], v[t][i]);
-                    if (amax[t] != amax[t]) {
+                    for (int i = 0; i < REQ_VEC; ++i) amax[t] = max_abs(amax[t], v[t][i], nan);
+                    if (nan) {
                         amax[t] = 0.0f;
 #pragma unroll
                         for (int i = 0; i < REQ_VEC; ++i) amax[t] = max_abs_any(amax[t], v[t][i]);
@@ -489,9 +490,10 @@ __global__ __launch_bounds__(256) void swiglu_requant_kernel(const float* __rest
     }
     float amax = 0.0f;
     if constexpr (NV > 0) {
+        bool nan = false;
 #pragma unroll
-        for (int n = 0; n < NV; ++n) amax = max_abs(amax, held[n]);
-        if (amax != amax) {
+        for (int n = 0; n < NV; ++n) amax = max_abs(amax, held[n], nan);
+        if (nan) {
             amax = 0.0f;
 #pragma unroll
             for (int n = 0; n < NV; ++n) amax = max_abs_any(amax, held[n]);

@@ -204,10 +204,12 @@ __device__ __forceinline__ float wave_max(float v)
 }
 
 // max(m, |v|) as "v > m ? v : m" has it: NaN is passed over.  v_max3_f32 does two values in one instruction where a
-// comparison and a selection take four; only a signalling NaN (no arithmetic makes one, but memory may hold it) comes
-// through, so a caller whose maximum turns out NaN takes it again with max_abs_any.
-__device__ __forceinline__ float max_abs(float m, v4f v)
+// comparison and a selection take four, and passes over quiet NaNs; but a signalling NaN (no arithmetic makes one, but a
+// caller's memory may hold it) takes the value it is compared with along, without a trace in the result.  So one more
+// comparison looks at both values: once `nan` is set the caller takes the maximum again with max_abs_any.
+__device__ __forceinline__ float max_abs(float m, v4f v, bool& nan)
 {
+    nan |= __builtin_isunordered(v[0], v[1]) | __builtin_isunordered(v[2], v[3]);
     asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(v[0]), "v"(v[1]));
     asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(v[2]), "v"(v[3]));
     return m;
