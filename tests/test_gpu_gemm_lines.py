@@ -6,6 +6,16 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
+
+def exact_products(x, w, counts):
+    """The int32 sums of the experts' rows, by torch in 64-bit floating point (exact: they are whole and below 2^53)."""
+    out, row = [], 0
+    for e, m in enumerate(counts.tolist()):
+        out.append((x[row:row + m].double() @ w[e].double().t().contiguous()).int())
+        row += m
+    return torch.cat(out)
+
+
 LINES = [(1023, 128, 256, 128, "stream"), (1024, 128, 256, 128, "tiled"), (1100, 1200, 64, 64, "stream"),
          (63 * 8 + 7, 8, 4096, 128, "tiled"), (64 * 8, 8, 4096, 128, "wide"),
          (287, 288, 2048, 2048, "stream"), (288, 288, 2048, 2048, "tiled"),
@@ -267,6 +277,39 @@ def test_tokens_of_a_tile_in_lds(avg, E, Kd, N, family, dtype):
     at = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).to("cuda")
     want = ((acc.float() * sx.to("cuda")[:, None]) * sw.to("cuda")[at]).to(dtype)
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+# ... whose rows end in front of the buffer's, the last ones inside a tile: what lies around the output stays as it is.  Experts of
+# one row, whose tile is 128 rows of the next ones
+@pytest.mark.parametrize("K_, N", [(256, 2048), (768, 1408)])
+@pytest.mark.parametrize("kind", [0, 1])
+def test_nothing_is_written_around_the_rows(K_, N, kind):
+    from vllm_ascend_amd import kernels as K
+    from vllm_ascend_amd._lib import W_ENK, load
+
+    lib, E, R = load(), 16, 33000
+    print(f"around the rows K={K_} N={N} kind={kind}", flush=True)
+    assert lib.moe355_gmm_kernel_name(2, R, K_, N, E) == b"gmm_resident_kernel"
+    counts = torch.tensor([1, 2900, 0, 129, 1, 1, 65, 3000, 128, 1, 4000, 6000, 64, 7000, 8000, 1001])
+    rows = int(counts.sum())
+    assert rows < R - 600 and rows % 128
+    g = torch.Generator(device="cuda").manual_seed(R)
+    x = torch.randint(-128, 128, (R, K_), generator=g, dtype=torch.int8, device="cuda")
+    w = torch.randint(-128, 128, (E, N, K_), generator=g, dtype=torch.int8, device="cuda")
+    sw = torch.rand(E, N, generator=g, device="cuda") * 0.009 + 0.001
+    sx = torch.rand(R, generator=g, device="cuda") * 0.05 + 0.001
+    wnz = K.format_cast_nz(w, W_ENK)
+    gl = (counts if kind else counts.cumsum(0)).to("cuda")
+    around = torch.full((R + 512, N), 0x1234, dtype=torch.int16, device="cuda")
+    ws = torch.empty(lib.moe355_gmm2_dequant_workspace(R, N, K_, E), dtype=torch.uint8, device="cuda")
+    p = lambda t: t.data_ptr()  # noqa: E731
+    assert lib.moe355_gmm2_dequant(p(x), p(wnz), p(sw), p(sx), p(gl), kind, R, K_, N, E, p(around[256]), K._dt(x.bfloat16(), "out"),
+                                   p(ws), ws.numel(), torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert bool((around[:256] == 0x1234).all()) and bool((around[256 + rows:] == 0x1234).all())
+    at = torch.repeat_interleave(torch.arange(E), counts).to("cuda")
+    want = ((exact_products(x, w, counts).float() * sx[:rows, None]) * sw[at]).to(torch.bfloat16)
+    assert torch.equal(around[256:256 + rows], want.view(torch.int16))
 
 
 # Weight-streaming tiles for a product with ten columns of them and more per expert, up to 256 rows per expert: tall tiles

@@ -132,7 +132,10 @@ __device__ __forceinline__ void resident_body(const GmmArgs& a, int e, int64_t r
     const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc((void*)(a.out + row0 * a.N), 0, (int)(n_rows * a.N * 2), 0x00027000);
     // Whole 128-byte row segments through the wavefront's own LDS patch (see tiled_epilogue_body).  The buffer's length cuts
     // the rows past the expert's end: every store is issued, so that the waits for the next group's weights, which are in
-    // flight already, are exact.
+    // flight already, are exact.  Row and column are in the vector offset alone.  That is what the length is
+    // compared with, where the scalar offset need not be; and behind a 16-byte store with a scalar offset the compiler lets the
+    // next vector instruction write over the store's data, which gfx950 then stores (every other row's first four bytes were
+    // the next store's address), while without one it waits for as long as the store takes its data.
     auto epilogue = [&](int g) {
         const float* sg = cs_l + (g - g0) * 64 + 4 * quarter;
         const int c16 = lane & 7, r8 = lane >> 3;
@@ -157,10 +160,11 @@ __device__ __forceinline__ void resident_body(const GmmArgs& a, int e, int64_t r
 #pragma unroll
             for (int i = 0; i < 4; ++i) t[i] = *(const v4i*)(patch + (r8 + 8 * i) * kResRowB + c16 * 16);
             wave_lds_order();
+            int at = r8 * a.N * 2 + g * 128 + c16 * 16;
+            asm volatile("" : "+v"(at));  // the sums below are made here: kept over the K loop they would cost 16 registers
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                __builtin_amdgcn_raw_buffer_store_b128(t[i], out, r8 * a.N * 2 + c16 * 16,
-                                                       (b * 32 + 8 * i) * a.N * 2 + g * 128, 2 /* non-temporal */);
+                __builtin_amdgcn_raw_buffer_store_b128(t[i], out, at + (b * 32 + 8 * i) * a.N * 2, 0, 2 /* non-temporal */);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
