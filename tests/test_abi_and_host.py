@@ -511,6 +511,25 @@ def test_weight_streaming_tiles_of_many_rows(experts, k, n, first):
             assert name(epilogue, rows * experts, k, n, experts).decode() == f"gmm_{want}_kernel"
 
 
+# tokens of a tile in LDS: channels that fill 11 of 16 places of the wavefronts, from 1024 on; rows of fewer than 640 values only
+# from 2048 channels on, 15 of 16 places (all of them below 384) and below 4096 rows; rounds of the chip that are full enough
+@pytest.mark.parametrize("rows, experts, k, n, resident", [
+    (65536, 128, 768, 1024, True), (65536, 128, 768, 960, False), (65535, 128, 768, 1024, False), (65536, 128, 768, 1088, False),
+    (65536, 128, 768, 1280, False), (65536, 128, 768, 1344, False), (65536, 128, 768, 1408, True), (65536, 128, 768, 2112, True),
+    (65536, 128, 896, 2048, True), (65536, 128, 1024, 2048, False), (65536, 128, 704, 2048, False), (65536, 128, 512, 1024, False),
+    (65536, 128, 512, 1984, False), (65536, 128, 512, 2048, True), (65536, 128, 384, 2560, False), (65536, 128, 384, 2880, True),
+    (65536, 128, 256, 2880, False), (65536, 128, 256, 4096, True), (65536, 16, 512, 2048, False), (65520, 16, 512, 2048, True),
+    (65536, 16, 640, 2048, True), (128 * 288 - 1, 128, 768, 2048, False), (128 * 288, 128, 768, 2048, True),
+    (34000, 8, 640, 2048, False), (37759, 8, 640, 2048, False), (37760, 8, 640, 2048, False), (37888, 8, 640, 2048, True),
+    (48640, 8, 640, 2048, True), (48768, 8, 640, 2048, False), (50688, 8, 640, 2048, True), (40000, 1, 640, 2048, False)])
+def test_tokens_of_a_tile_in_lds_lines(rows, experts, k, n, resident):
+    from vllm_ascend_amd import _lib
+
+    name = _lib.load().moe355_gmm_kernel_name
+    assert (name(2, rows, k, n, experts) == b"gmm_resident_kernel") == resident
+    assert name(0, rows, k, n, experts) != b"gmm_resident_kernel" != name(1, rows, k, n, experts)
+
+
 # one for every 56 pairs, but not where a short launch (fewer than 1536 units of 64 channels) has places in front of its slots
 # (from two pairs per expert on), nor from twelve pairs per expert on
 @pytest.mark.parametrize("experts, n, pairs, blocks", [(128, 1536, 512, 9), (128, 512, 256, 4), (128, 512, 257, 0), (128, 704, 512, 0),

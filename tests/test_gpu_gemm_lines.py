@@ -242,12 +242,15 @@ def test_columns_of_wide_tiles(E, family):
 
 # The down product with a tile's tokens in LDS: from 288 rows per expert and 512 workgroups of 128 rows x 1024 channels on, rows
 # of 256 to 896 values in steps of 128; experts of no row, of one, at the borders of half and whole tiles; channels that leave
-# every wavefront two groups of 64, some of them one or none
-@pytest.mark.parametrize("avg,E,Kd,N,family", [(287, 16, 256, 14400, "tiled"), (288, 16, 256, 14400, "resident"),
+# every wavefront two groups of 64 (9216, 4096), some of them one (14400, 17408, 1472, whose last part is a group shorter), and
+# seven of the last part none (15424)
+@pytest.mark.parametrize("avg,E,Kd,N,family", [(287, 16, 384, 14400, "tiled"), (288, 16, 384, 14400, "resident"),
                                                (512, 15, 384, 9216, "resident"), (400, 12, 896, 14400, "resident"),
                                                (340, 12, 768, 17408, "resident"), (340, 12, 1024, 17408, "tiled"),
                                                (340, 12, 704, 17408, "tiled"), (340, 12, 768, 16384, "tiled"),
-                                               (11000, 2, 256, 2112, "resident")])
+                                               (11000, 2, 256, 2112, "tiled"), (13000, 2, 768, 2112, "resident"),
+                                               (1200, 16, 256, 4096, "resident"), (400, 12, 640, 15424, "resident"),
+                                               (1300, 30, 640, 1472, "resident"), (1300, 30, 640, 1344, "tiled")])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_tokens_of_a_tile_in_lds(avg, E, Kd, N, family, dtype):
     from oracle import oracle as orc
@@ -287,10 +290,10 @@ def test_nothing_is_written_around_the_rows(K_, N, kind):
     from vllm_ascend_amd import kernels as K
     from vllm_ascend_amd._lib import W_ENK, load
 
-    lib, E, R = load(), 16, 33000
+    lib, E, R = load(), 16, 38400
     print(f"around the rows K={K_} N={N} kind={kind}", flush=True)
     assert lib.moe355_gmm_kernel_name(2, R, K_, N, E) == b"gmm_resident_kernel"
-    counts = torch.tensor([1, 2900, 0, 129, 1, 1, 65, 3000, 128, 1, 4000, 6000, 64, 7000, 8000, 1001])
+    counts = torch.tensor([1, 2900, 0, 129, 1, 1, 65, 3000, 128, 1, 4000, 6000, 64, 7000, 13400, 1001])
     rows = int(counts.sum())
     assert rows < R - 600 and rows % 128
     g = torch.Generator(device="cuda").manual_seed(R)

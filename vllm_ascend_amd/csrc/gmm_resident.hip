@@ -225,12 +225,37 @@ __global__ __launch_bounds__(512, 1) void gmm_resident_kernel(GmmArgs a, TileMap
 // routing (Zipf(1.1)): 192 rows 267.0 / 264.7, 200 (275.7 / 281.1), 256 330.0 / 331.7, 312 369.8 / 363.6, 344 (398.6 /
 // 399.2), 500 544.7 / 527.9.  One workgroup per compute unit and 32 KiB of weights for 64 channels: an expert's last, short
 // tile costs more than on the smaller tiles.
+//
+// The other lines, by the product alone, back to back, time of 128-row tiles = 1, uniform routing (Zipf(1.1)):
+// - Places: a workgroup's wavefronts take one or two whole groups of 64 channels each, so 1280 channels fill 20 of 32 places.
+//   K = 768, 128 experts of 512 rows, 1088 / 1152 / 1280 channels (0.53 to 0.63 of the places) 1.06 / 1.06 / 1.03 (1.05 / 1.05
+//   / 1.04); 1408 / 1536 / 1792 / 2112 / 2304 / 2560 / 2880 (0.69 to 0.94) 0.93 / 0.94 / 0.94 / 0.90 / 0.90 / 0.92 / 0.87 (0.94
+//   / 0.94 / 0.96 / 0.92 / 0.92 / 0.92 / 0.88); 2048 and 4096 (all) 0.85 and 0.90 (0.89 and 0.87).  K = 896 the same, K = 640
+//   from 1408 on.
+// - Below 1024 channels, one workgroup for a tile either way, nothing is won: 448 / 576 / 768 0.96 / 1.00 / 1.00 (1.05 / 1.04 /
+//   1.02).
+// - A short K has less to keep.  128 experts of 300 rows, 1536 / 2304 / 2560 channels at K = 512 0.95 / 0.98 / 0.96 (1.05 / 1.07
+//   / 1.05), at K = 384 0.94 / 0.95 / 0.97 (1.02 / 1.05 / 1.05), 1024 at K = 512 and 512 rows 0.96 (1.08); 2880 at K = 512 / 384 /
+//   256 0.93 / 0.91 / 0.90 (0.97 / 1.00 / 1.01; K = 256 at 512 rows 1.05); 2048 at K = 512 / 384 / 256 0.88 / 0.89 / 0.88 (1.02 / 1.01 / 0.84) and at 512
+//   rows 0.89 / 0.88 / 0.89 (0.90 / 0.94 / 0.88).  And thousands of rows share an expert's weights in L2 as it is: K = 384, 2048
+//   channels, 65536 rows of 4 / 8 / 16 / 32 experts 1.04 / 1.04 / 1.02 / 0.99 (1.05 / 1.05 / 1.04 / 1.01).
+// - Rounds: workgroups for half a round more than the chip holds leave the rest of it idle.  2048 channels, 34000 rows of 4 / 8 /
+//   16 experts (2.1 rounds) 1.09 / 1.06 / 1.05 at K = 896 and 1.01 / 1.04 / 1.04 at 640, 45000 rows (2.8) 0.89 / 0.88 / 0.90 and
+//   0.88 / 0.86 / 0.87, 65536 (4.0 to 4.1) 0.98 / 0.98 / 0.94 and 0.95 / 0.96 / 0.95, 131072 0.79 / 0.81 / 0.82 and 0.92 / 0.83 /
+//   0.82; 60 experts of 600 rows (2.4) 0.93 and 0.94.  With 1024 channels half as many workgroups do the same: 512 (two rounds
+//   and the experts' short tiles), K = 640 / 768 / 896, 64 experts 0.89 / 0.93 / 0.93, 128 0.92 / 0.94 / 0.95.
 bool resident_supported(const GmmArgs& a)
 {
-    if (a.K % 128 || a.K < 256 || a.N > (1 << 20)) return false;
-    const int64_t parts = (a.N / 64 + 15) / 16;
-    if (a.E < 2 || a.R / a.E < 288 || a.R / 128 * parts < 512) return false;  // two of them for every compute unit
-    return resident_lds(a.K, 16) <= kResLdsBytes;
+    if (a.K % 128 || a.K < 256 || a.N < 1024 || a.N > (1 << 20) || resident_lds(a.K, 16) > kResLdsBytes) return false;
+    if (a.E < 2 || a.R / a.E < 288) return false;
+    const int64_t groups = a.N / 64;
+    const int64_t parts = (groups + 15) / 16;
+    const int64_t places = ((groups + parts - 1) / parts + 7) / 8 * 8 * parts;
+    if (a.K >= 640 ? 16 * groups < 11 * places
+                   : a.N < 2048 || 16 * groups < (a.K >= 384 ? 15 : 16) * places || a.R / a.E >= 4096) return false;
+    if (a.R / 128 * parts < 512) return false;
+    const int64_t workgroups = (a.R / 128 + a.E / 2) * parts;  // half of the experts end in a tile that is hardly begun
+    return parts == 1 || workgroups >= 200 * ((workgroups + 255) / 256);
 }
 
 // (the tile map is in the workspace)
