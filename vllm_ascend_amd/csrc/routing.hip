@@ -422,10 +422,10 @@ __global__ __launch_bounds__(kMapThreads) void route_map_kernel(RouteMapArgs a)
     if constexpr (MANY) {  // columns / 4 neighbouring lanes add up an expert
         const int lanes = columns / 4;
         for (int i = tid; i < E * lanes; i += kMapThreads) {
-            const v4i v = ((const v4i*)split)[i];
-            int n = v[0] + v[1] + v[2] + v[3];
+            const uint4 v = ((const uint4*)split)[i];
+            uint32_t n = v.x + v.y + v.z + v.w;  // above 2^31 from 32768 pairs in front on
             for (int d = 1; d < lanes; d <<= 1) n += __shfl_xor(n, d);
-            if (i % lanes == 0) count[i / lanes] = n;
+            if (i % lanes == 0) count[i / lanes] = (int32_t)n;
         }
         __syncthreads();
     }
