@@ -495,18 +495,21 @@ def test_few_streaming_workgroups_keep_streaming(experts, k, n, first):
         assert name(epilogue, first * experts, k, n, experts) == b"gmm_tiled_kernel"
 
 
-# above 256 rows per expert: weight-streaming tiles for weights of 32 MiB an expert, from 384 rows on of 14 MiB (at least 5120
-# channels; fewer at K from 7168 on with 2048 columns of tiles)
-@pytest.mark.parametrize("experts, k, n, first", [(16, 4096, 8192, 257), (15, 4096, 8192, None), (32, 4096, 8128, 384),
-                                                  (64, 2048, 7168, 384), (64, 2048, 7104, None), (64, 3072, 5056, None),
-                                                  (18, 2048, 7168, None), (19, 2048, 7168, 384), (64, 1984, 16384, None),
-                                                  (256, 7168, 4096, 384), (255, 7168, 4096, None), (256, 7104, 4096, None)])
+# above 256 rows per expert: weight-streaming tiles for weights of 32 MiB an expert, from 384 rows on (512 below 768 columns of
+# tiles) of 14 MiB with at least 5120 channels, of 20 MiB with fewer, from 3072 on, at K from 5120 on with 768 columns
+@pytest.mark.parametrize("experts, k, n, first", [(16, 4096, 8192, 257), (15, 4096, 8192, None), (32, 4096, 8128, 512),
+                                                  (48, 4096, 8128, 384), (55, 2048, 7168, 384), (54, 2048, 7168, 512),
+                                                  (64, 2048, 7104, None), (64, 3072, 5056, None), (18, 2048, 7168, None),
+                                                  (19, 2048, 7168, 512), (64, 1984, 16384, None), (256, 7168, 4096, 384),
+                                                  (96, 7168, 4096, 384), (95, 7168, 4096, None), (256, 5120, 4096, 384),
+                                                  (256, 5120, 4032, None), (160, 5056, 4608, None), (160, 7168, 3072, 384),
+                                                  (160, 7168, 3008, None)])
 def test_weight_streaming_tiles_of_many_rows(experts, k, n, first):
     from vllm_ascend_amd import _lib
 
     name = _lib.load().moe355_gmm_kernel_name
     for epilogue in (0, 1, 2):
-        for rows in (257, 383, 384, 2000):
+        for rows in (257, 383, 384, 511, 512, 2000):
             want = "wide" if first and rows >= first else "tiled"
             assert name(epilogue, rows * experts, k, n, experts).decode() == f"gmm_{want}_kernel"
 

@@ -315,15 +315,15 @@ def test_nothing_is_written_around_the_rows(K_, N, kind):
     assert torch.equal(around[256:256 + rows], want.view(torch.int16))
 
 
-# Weight-streaming tiles for a product with ten columns of them and more per expert, up to 256 rows per expert: tall tiles
-@pytest.mark.parametrize("avg,E,N,family", [(144, 64, 5120, "wide"), (145, 64, 5120, "tiled"), (145, 77, 5120, "wide"),
-                                            (256, 77, 5120, "wide"), (257, 77, 5120, "tiled"), (145, 96, 5056, "tiled")])
+# Weight-streaming tiles for a product of 14 MiB per expert and 896 columns of them, up to 256 rows per expert: tall tiles
+@pytest.mark.parametrize("avg,E,N,family", [(144, 63, 7168, "wide"), (145, 63, 7168, "tiled"), (145, 64, 7168, "wide"),
+                                            (256, 64, 7168, "wide"), (257, 64, 7168, "tiled"), (145, 80, 7104, "tiled")])
 def test_rows_of_weight_streaming_tiles(avg, E, N, family):
     test_tokens_of_a_tile_in_lds(avg, E, 2048, N, family, torch.bfloat16)
 
 
 # and of several tall tiles per expert, where an expert's weights are several times an XCD's L2
-@pytest.mark.parametrize("avg,E,Kd,N,family", [(257, 16, 4096, 8192, "wide"), (383, 19, 2048, 7168, "tiled"),
-                                               (384, 19, 2048, 7168, "wide"), (700, 19, 2048, 7232, "wide")])
+@pytest.mark.parametrize("avg,E,Kd,N,family", [(257, 16, 4096, 8192, "wide"), (511, 19, 2048, 7168, "tiled"),
+                                               (512, 19, 2048, 7168, "wide"), (700, 19, 2048, 7232, "wide")])
 def test_several_weight_streaming_tiles_of_an_expert(avg, E, Kd, N, family):
     test_tokens_of_a_tile_in_lds(avg, E, Kd, N, family, torch.bfloat16)

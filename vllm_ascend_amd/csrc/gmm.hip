@@ -676,15 +676,23 @@ static int tiled_bm(const GmmArgs& a)
     //     0.91 / 0.87 / 0.82 / 0.75; 32 of 8192 x 4096 0.85 / 0.91 / 0.86 / 0.84, Zipf 0.93 / 0.91 / 0.89 / 0.87.
     //   14 MiB and more, from 384 rows on (two tiles of 256 are mostly padding before): 256 experts of 7168 x 2048, 352 / 384 /
     //     512 / 1024 rows 1.05 / 0.95 / 0.93 / 0.89, Zipf 0.94 / 0.90 at 384 / 512; 64 of them 1.05 / 0.96 / 0.93 / 0.89, Zipf
-    //     0.92 / 0.97 / 0.95 / 0.89; 128 of 5120 x 3072 0.97 / 0.95 / 0.93 at 384 / 512 / 1024, Zipf 0.97 / 0.93 / 0.92.  Ten
-    //     MiB (5120 x 2048) 1.05, Zipf 1.00 to 1.04.
-    //   Fewer channels than 5120 only at the longest K and with many columns: 256 experts of 4096 x 7168, 288 / 320 / 384 / 512 /
-    //     1024 rows 1.01 / 0.99 / 0.92 / 0.93 / 0.91 (512 rows 4980 against 4610 us), Zipf 0.94 / 0.95 at 384 / 512; 32 of them
-    //     0.90 / 0.91 but Zipf 1.14 / 1.00; 4096 x 4096 0.97 to 1.01, Zipf 0.99 to 1.08.
+    //     0.92 / 0.97 / 0.95 / 0.89; 128 of 5120 x 3072 0.97 / 0.95 / 0.93 at 384 / 512 / 1024, Zipf 0.97 / 0.93 / 0.92.  With
+    //     fewer columns of tiles the last tall ones weigh more: 384 / 512 / 1024 rows, 266 columns (19 experts of 7168 x 2048)
+    //     1.06 / 1.01 / 0.92, Zipf 1.07 / 0.90 / 0.89, 260 (26 of 5120 x 3072) 1.14 / 1.00 / 0.94, Zipf 1.09 / 0.95 / 0.98, 520 (52
+    //     of them) 1.05 / 1.01 / 0.95, Zipf 0.98 / 0.97 / 0.93; so from 512 rows on below 768 columns.  Ten MiB (5120 x 2048)
+    //     1.05, Zipf 1.00 to 1.04.
+    //   Fewer channels than 5120 from 3072 on, for 20 MiB, K >= 5120 and 768 columns: 384 / 512 / 1024 rows, 256 experts of 4096 x
+    //     7168 0.91 / 0.92 / 0.90 (512 rows 4961 against 4565 us), Zipf 0.94 / 0.94 / 0.91; 128 of them 0.89 / 0.91 / 0.89, Zipf
+    //     0.97 / 0.95 / 0.91; 160 of 4608 x 7168 0.90 / 0.90 / 0.89, Zipf 0.94 / 0.93 / 0.87; 128 of 4096 x 6144 0.94 / 0.95 /
+    //     0.92, Zipf 0.98 / 0.98 / 0.93; 256 of 4096 x 5120 0.98 / 0.98 / 0.96, Zipf 0.96 / 0.97 / 0.94; 160 of 3072 x 7168 0.98 /
+    //     0.99 / 0.96, Zipf 0.97 / 0.97 / 0.93.  300 rows 0.97 to 1.12.  256 columns (32 of 4096 x 7168) 0.89 / 0.91 / 0.92, Zipf
+    //     1.12 / 0.99 / 0.95, 258 (43 of 3072 x 7168) 1.11 / 1.03 / 0.98, Zipf 1.13 / 0.97 / 0.96.  2048 x 7168 0.97 to 1.01; 4096 x
+    //     4096 0.97 to 1.01, Zipf 0.99 to 1.08.
     const int64_t own = (int64_t)a.N * a.K;
-    const bool tall = a.N >= 5120 ? own >= (14 << 20) : a.K >= 7168 && columns >= 8 * kComputeUnits;
+    const bool many_columns = columns >= 3 * kComputeUnits;
+    const bool tall = a.N >= 5120 ? own >= (14 << 20) : many_columns && a.N >= 3072 && a.K >= 5120 && own >= (20 << 20);
     if (avg > 256 && a.K >= 2048 && wide_ok && columns >= kComputeUnits
-        && ((a.K >= 4096 && own >= (32 << 20)) || (avg >= 384 && tall))) return 256;
+        && ((a.K >= 4096 && own >= (32 << 20)) || (avg >= (many_columns ? 384 : 512) && tall))) return 256;
     // Around 128 rows per expert most experts fit one wide tile of 128 or 160 rows and fetch their weights once, which
     // pays from K = 1024 on if the experts are about equally popular and there are enough of them to fill the chip.  128
     // experts, K = 2048 / 768, the layer at 100 / 112 / 128 / 144 / 160 / 192 rows per expert: 201 / 210 / 224 / 241 / 260 /
@@ -698,15 +706,20 @@ static int tiled_bm(const GmmArgs& a)
     // columns, and behind the others there: K / N = 1024 / 512, 128 rows, 8 and 128 experts 25 and 29 us against 13 and 31 on
     // 64-row tiles and 14 and 31 on 128-row tiles (Zipf 34 and 48 against 14 and 34, 14 and 30).  Left as it is as well.
     // From 144 rows on nearly every expert has a second tile, which comes out of the last-level cache.  Uniform routing still
-    // wins there, at any shape; under Zipf(1.1) the hot expert's tall tiles are the end of the launch unless there are many
-    // columns of them for each expert.  One product, wide / 128-row tiles: K = 2048, N = 7168 (14 columns per expert), 256
-    // experts, 144 / 160 / 192 / 224 / 250 rows 0.78 / 0.80 / 0.84 / 0.88 / 0.94 (160 rows 826 against 1035 us), Zipf 1.02
-    // / 1.00 / 0.97 / 0.97 / 0.97; 128 experts, 160 / 192 / 224 rows 0.79 / 0.84 / 0.87, Zipf 1.00 / 0.94 / 0.92; 64 experts,
-    // 160 / 208 rows 0.84 / 0.91, Zipf 1.00 / 1.01; 128 experts of K = 3072, N = 5120 (10 columns), 150 / 200 / 250 rows 0.73 /
-    // 0.83 / 0.91, Zipf 1.04 / 0.98 / 1.00.  With eight columns or fewer (N = 4096, 2048, 1024) 0.79 to 1.07 and 1.01 to
-    // 1.15: 144 rows there.
+    // wins there, at any shape; under Zipf(1.1) the hot expert's tall tiles are the end of the launch unless an expert's weights
+    // are several times an XCD's L2 and there are many columns of tiles.  One product, wide / 128-row tiles: K = 2048, N = 7168
+    // (14 MiB and 14 columns per expert), 256 experts, 144 / 160 / 192 / 224 / 250 rows 0.78 / 0.80 / 0.84 / 0.88 / 0.94 (160 rows
+    // 826 against 1035 us), Zipf 1.02 / 1.00 / 0.97 / 0.97 / 0.97; 128 experts, 160 / 192 / 224 rows 0.79 / 0.84 / 0.87, Zipf 1.00
+    // / 0.94 / 0.92; 64 experts, 160 / 208 rows 0.84 / 0.91, Zipf 1.00 / 1.01.  K = 3072, N = 5120 (15 MiB), 150 / 200 / 250 rows,
+    // 128 experts 0.71 / 0.82 / 0.90, Zipf 1.04 / 0.97 / 1.00, 90 experts 0.73 / 0.85 / 0.95, Zipf 1.01 / 1.00 / 0.98.  70 experts
+    // of K = 3072, N = 6144 (840 columns) 0.72 / 0.87 / 0.96, Zipf 1.08 / 0.97 / 1.00, so from 896 on, where 56 experts of K = 2048,
+    // N = 8192 have 0.71 / 0.86 / 0.92, Zipf 0.99 / 0.95 / 0.91.  Ten MiB (K = 2048, N = 5120) win less and lose more: 128 experts
+    // 0.75 / 0.88 / 0.95, Zipf 1.09 / 1.00 / 1.02, 96 experts 0.78 / 0.89 / 0.97, Zipf 1.03 / 1.09 / 1.00, 80 experts 0.82 / 0.99 /
+    // 1.05, Zipf 1.13 / 1.01 / 1.03.  With eight columns or fewer per expert (N = 4096, 2048, 1024) 0.79 to 1.07 and 1.01 to
+    // 1.15.  144 rows for those.
     const bool fills = narrow || columns >= kComputeUnits;
-    const int64_t most = narrow ? 192 : a.K >= 2048 && a.N >= 5120 && columns >= 3 * kComputeUnits ? 256 : 144;
+    const bool beyond = a.K >= 2048 && a.N >= 5120 && own >= (14 << 20) && 2 * columns >= 7 * kComputeUnits;
+    const int64_t most = narrow ? 192 : beyond ? 256 : 144;
     if (avg >= (narrow ? 96 : 112) && avg <= most && a.K >= 1024 && wide_ok && fills) return 256;
     return 128;
 }
