@@ -261,25 +261,36 @@ def test_tokens_of_a_tile_in_lds(avg, E, Kd, N, family, dtype):
     print(f"tokens in LDS R={R} E={E} K={Kd} N={N} {family} {dtype}", flush=True)
     assert load().moe355_gmm_kernel_name(2, R, Kd, N, E).decode() == f"gmm_{family}_kernel"
     counts = [0, 1, 63, 64, 65, 127, 128, 129] if E > 8 else []
+    counts += [160, 161, 192, 193, 256, 257] if E > 24 else []  # the heights of the weight-streaming tiles
     rest = R - sum(counts)
     counts += [rest // (E - len(counts))] * (E - len(counts) - 1)
     counts += [R - sum(counts)]
-    cum = torch.tensor(counts).cumsum(0)
-    g = torch.Generator().manual_seed(R)
-    x = torch.randint(-128, 128, (R, Kd), generator=g, dtype=torch.int8)
-    w = torch.randint(-128, 128, (E, N, Kd), generator=g, dtype=torch.int8)
-    sw = torch.rand(E, N, generator=g) * 0.009 + 0.001
-    sx = torch.rand(R, generator=g) * 0.05 + 0.001
-    wnz = K.format_cast_nz(w.to("cuda"), W_ENK)
-    got = K.gmm2_dequant(x.to("cuda"), wnz, sw.to("cuda"), sx.to("cuda"), cum.to("cuda"), 0, N, Kd, out_dtype=dtype)
-    acc = K.gmm_i32(x.to("cuda"), wnz, cum.to("cuda"), 0, N, Kd)  # some of its rows against the oracle
-    for r in [0, 1, 64, 128, 321, R // 2, R - 129, R - 1]:
-        e = int(torch.searchsorted(cum, r, right=True))
-        want = orc.gmm_i32(x[r:r + 1].numpy(), w[e:e + 1].numpy(), np.array([1]))
-        assert np.array_equal(acc[r].cpu().numpy(), want[0])
-    at = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).to("cuda")
-    want = ((acc.float() * sx.to("cuda")[:, None]) * sw.to("cuda")[at]).to(dtype)
+    counts = torch.tensor(counts)
+    cum = counts.cumsum(0)
+    g = torch.Generator(device="cuda").manual_seed(R)
+    x = torch.randint(-128, 128, (R, Kd), generator=g, dtype=torch.int8, device="cuda")
+    w = torch.randint(-128, 128, (E, N, Kd), generator=g, dtype=torch.int8, device="cuda")
+    sw = torch.rand(E, N, generator=g, device="cuda") * 0.009 + 0.001
+    sx = torch.rand(R, generator=g, device="cuda") * 0.05 + 0.001
+    wnz = K.format_cast_nz(w, W_ENK)
+    acc = exact_products(x, w, counts)
+    assert torch.equal(K.gmm_i32(x, wnz, cum.to("cuda"), 0, N, Kd), acc)
+    got = K.gmm2_dequant(x, wnz, sw, sx, cum.to("cuda"), 0, N, Kd, out_dtype=dtype)
+    at = torch.repeat_interleave(torch.arange(E), counts).to("cuda")
+    want = ((acc.float() * sx[:, None]) * sw[at]).to(dtype)
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    if family != "wide":
+        return
+    # the gate_up product of the same line: the first, a middle and the last rows of every expert against the oracle
+    assert load().moe355_gmm_kernel_name(1, R, Kd, N, E) == b"gmm_wide_kernel"
+    q, qs = K.gmm1_swiglu_quant(x, wnz, sw, sx, cum.to("cuda"), 0, N, Kd)
+    rows = [sorted({int(c) - int(m), int(c) - int(m) // 2 - 1, int(c) - 1}) for c, m in zip(cum, counts) if m]
+    picked = torch.tensor(sum(rows, []))
+    ends = np.searchsorted(picked.numpy(), cum.numpy())
+    q_want, s_want = orc.swiglu_quant(orc.dequant_acc(acc[picked.to("cuda")].cpu().numpy(), sx.cpu()[picked].numpy(),
+                                                      sw.cpu().numpy(), ends))
+    assert np.array_equal(q.cpu()[picked].numpy(), q_want)
+    assert np.array_equal(qs.cpu()[picked].numpy().view(np.uint32), s_want.view(np.uint32))
 
 
 # ... whose rows end in front of the buffer's, the last ones inside a tile: what lies around the output stays as it is.  Experts of
@@ -324,6 +335,7 @@ def test_rows_of_weight_streaming_tiles(avg, E, N, family):
 
 # and of several tall tiles per expert, where an expert's weights are several times an XCD's L2
 @pytest.mark.parametrize("avg,E,Kd,N,family", [(257, 16, 4096, 8192, "wide"), (511, 19, 2048, 7168, "tiled"),
-                                               (512, 19, 2048, 7168, "wide"), (700, 19, 2048, 7232, "wide")])
+                                               (512, 19, 2048, 7168, "wide"), (700, 19, 2048, 7232, "wide"),
+                                               (384, 96, 5120, 4096, "wide")])
 def test_several_weight_streaming_tiles_of_an_expert(avg, E, Kd, N, family):
     test_tokens_of_a_tile_in_lds(avg, E, Kd, N, family, torch.bfloat16)
