@@ -31,8 +31,8 @@ static int resident_lds(int64_t K, int group_span) { return (int)(128 * K) + kRe
 #define MOE355_LPTR(p) ((__attribute__((address_space(3))) void*)(p))
 
 // Rows [row0, row_end) of expert e (at most 32 * NBLK) x the channel groups (64 channels) g0 .. g0 + span - 1: wavefront w
-// takes groups g0 + w, g0 + w + 8 (at most two).  S: K blocks of 64 values whose weights are in flight per wavefront; K is a
-// multiple of 64 * S and holds at least two such pieces.
+// takes groups g0 + w, g0 + w + 8 (at most two).  The rows of a down product lie in x one after the other.  S: K blocks of
+// 64 values whose weights are in flight per wavefront; K is a multiple of 64 * S and holds at least two such pieces.
 // EVEN: every wavefront has two groups.
 template <int NBLK, int S, bool F16, bool EVEN>
 __device__ __forceinline__ void resident_body(const GmmArgs& a, int e, int64_t row0, int64_t row_end, int g0, int span,
@@ -62,7 +62,6 @@ __device__ __forceinline__ void resident_body(const GmmArgs& a, int e, int64_t r
             const int c = (lane & 7) ^ ((r8 >> 1) | ((rp & 1) << 2));
             int64_t r = row0 + rp * 8 + r8;
             if (r > row_end - 1) r = row_end - 1;  // rows past the expert's end repeat its last row (never stored)
-            if (a.row_src) r = a.row_src[r];
             __builtin_amdgcn_global_load_lds(MOE355_GPTR(a.x + r * K + seg * 128 + c * 16), MOE355_LPTR(lds + u * 1024), 16, 0, 0);
         }
     }
@@ -82,7 +81,7 @@ __device__ __forceinline__ void resident_body(const GmmArgs& a, int e, int64_t r
     if (threadIdx.x < 128) {
         int64_t r = row0 + threadIdx.x;
         if (r > row_end - 1) r = row_end - 1;
-        rs_l[threadIdx.x] = a.row_scale[a.row_src ? (int64_t)a.row_src[r] : r];
+        rs_l[threadIdx.x] = a.row_scale[r];
     }
     for (int i = threadIdx.x; i < span * 64; i += 64 * kResWaves)
         cs_l[i] = g0 * 64 + i < a.N ? cs[g0 * 64 + i] : 0.0f;
