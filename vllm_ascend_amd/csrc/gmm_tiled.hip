@@ -41,7 +41,7 @@ __global__ __launch_bounds__(256) void tile_map_kernel(const int64_t* __restrict
 }
 
 constexpr int kBN = 256;  // channels per workgroup (4 wavefronts x 2 storage tiles)
-constexpr int kBK = 64;   // K per pipeline stage (2 MFMA K steps)
+constexpr int kBK = 64;   // K per pipeline stage (one MFMA K step)
 
 // LDS of one workgroup: RING token stages of the tallest tile, reused by the epilogue patches
 template <int EPI, int BMT, int RING>
@@ -451,9 +451,9 @@ __global__ __launch_bounds__(256, (BMT <= 2 ? 3 : 2)) void gmm_tiled_kernel(GmmA
 //   tall tile (193..256 rows left): wavefront (h, g) = token half h x channel group g of 4 -> 256 x 256, twice
 //   the token traffic per weight byte (tokens come from L2, and that traffic costs weight bandwidth).
 // Both operands reach LDS by LDS-direct loads (no register staging, so the prefetch depth costs no registers),
-// each into a ring of its own.  A weight stage holds the weights of 64 K values (every storage tile x 2 K steps
-// is a contiguous 1 KiB MFMA operand that is copied as it lies), a token stage the tokens' 64 bytes (row-major,
-// with a rotation of the 16-byte chunks).
+// each into a ring of its own.  A weight stage holds the weights of 64 K values (2 KiB of every storage tile,
+// copied as they lie; an MFMA operand of 16 channels is four pieces of 256 bytes of them, 512 apart), a token stage the
+// tokens' 64 bytes (row-major, the 16-byte chunks exchanged by row).
 // The compiler does not count LDS-direct loads against the LDS reads that consume them: the wait for a stage
 // is written by hand, before the barrier that publishes the stage.
 constexpr int kWideLdsBytes = 163840;
@@ -520,7 +520,7 @@ __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_
     const bool active = have && hrow0 < row_end;
 
     // what this wavefront copies.  Weights: tall -- storage tile wave % 2 of group wave / 2; wide -- both
-    // storage tiles of group wave; always both K steps of the stage (2 KiB contiguous per tile).
+    // storage tiles of group wave; always the stage's 64 K values (2 KiB contiguous per tile).
     const int8_t* we = expert_weights(a, e);
     const int8_t* wsrc[WIDE ? 2 : 1];
     if constexpr (WIDE) {
