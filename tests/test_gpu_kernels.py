@@ -714,7 +714,10 @@ W4_COUNTS = [0, 1, 31, 32, 33, 63, 64, 65, 0, 130, 200, 7]
                                         # more than 32 scale groups: the scales no longer fit LDS and are read
                                         # from memory group by group (40 K blocks: whole passes of that
                                         # variant's ring; 36: a remainder)
-                                        (2560, 64, 64), (2304, 128, 64)])
+                                        (2560, 64, 64), (2304, 128, 64),
+                                        # odd numbers of K blocks and of stages; the most groups whose scales LDS
+                                        # holds, and one more (read from memory)
+                                        (64, 64, 64), (192, 64, 64), (704, 192, 64), (17408, 64, 64), (17472, 64, 64)])
 @pytest.mark.parametrize("gl_type", [0, 1])
 def test_w4_gemms_at_chunk_boundaries(K, orc, Kd, N, group, gl_type):
     print(f"w4 gemms K={Kd} N={N} group={group} gl_type={gl_type}", flush=True)
@@ -759,6 +762,27 @@ def test_w4_gemms_at_chunk_boundaries(K, orc, Kd, N, group, gl_type):
     got_b = K.gmm2_dequant_w4(x.to(DEV), w4, sg.to(DEV), gsz, sx.to(DEV), gl, gl_type, N, Kd, bias=bias.to(DEV))
     torch.cuda.synchronize()
     assert np.array_equal(bits(got_b.cpu()), orc.w4_rows_to_bf16(fb, sx.numpy()))
+
+
+def test_w4_rows_more_than_4_gib_apart(K):
+    """Gathered token rows beyond what a 32-bit offset reaches: the same values as the rows copied together."""
+    g = torch.Generator().manual_seed(5)
+    Kd, N, group, cnt = 4096, 64, 256, [40, 64, 7]
+    E, R = len(cnt), sum(cnt)
+    T = 2 ** 32 // Kd + 64
+    print(f"w4 gather from {T} rows of {Kd}", flush=True)
+    rows = torch.cat([torch.arange(56), torch.arange(T - 55, T)])[torch.randperm(R, generator=g)].to(torch.int32)
+    vals = torch.randint(-128, 128, (R, Kd), generator=g, dtype=torch.int8).to(DEV)
+    xs = (torch.rand(R, generator=g) * 0.05 + 0.001).to(DEV)
+    x, ts = torch.zeros(T, Kd, dtype=torch.int8, device=DEV), torch.zeros(T, device=DEV)
+    x[rows.long().to(DEV)], ts[rows.long().to(DEV)] = vals, xs
+    w4 = K.format_cast_nz_int4(torch.randint(-8, 8, (E, N, Kd), generator=g, dtype=torch.int8).to(DEV), 0, N, Kd)
+    sg = (torch.rand(E, Kd // group, N, generator=g) * 0.09 + 0.01).to(DEV)
+    gl = torch.tensor(cnt, dtype=torch.int64, device=DEV)
+    q, s = K.gmm1_swiglu_quant_w4_gather(x, ts, rows.to(DEV), w4, sg, group, gl, 1, N, Kd)
+    q_near, s_near = K.gmm1_swiglu_quant_w4(vals, w4, sg, group, xs, gl, 1, N, Kd)
+    torch.cuda.synchronize()
+    assert torch.equal(q, q_near) and torch.equal(s, s_near)
 
 
 # rows per expert around the 128-row tile of the LDS-tiled kernel and its 64-row short-tile path, and around the

@@ -824,6 +824,7 @@ TileSpec tile_spec(int64_t rows, int E, int BM, void* workspace)
     TileSpec t;
     t.BM = BM;
     t.by_length = BM == 256;
+    t.flag_only = 0;
     t.max_tiles = (int)(rows / BM + E);
     const size_t arr = (size_t)(((size_t)t.max_tiles * 4 + 255) / 256) * 256;
     t.tm.count = (int32_t*)workspace;

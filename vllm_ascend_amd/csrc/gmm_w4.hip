@@ -14,6 +14,7 @@
 #include <type_traits>
 
 #include "gmm_common.h"
+#include "gmm_tiled.h"
 #include "layer_parts.h"
 
 namespace moe355 {
@@ -94,6 +95,7 @@ struct W4Args {
     const float* gscale;  // [E, K/group, N]
     const float* bias;    // [E, N] or null, added before the token scale
     int group;            // K values per scale group (multiple of 64)
+    TileMap tm;           // sorted rows: the list of chunks, built by the routing launch, or null (found from the group list)
 };
 
 __device__ __forceinline__ v4i nib_lo(v4i v)
@@ -194,255 +196,319 @@ __device__ __forceinline__ bool find_chunk(const int64_t* gl, int gl_type, int E
     return false;
 }
 
-// One wavefront per unit (chunk of up to 64 rows of one expert, pair of 32-channel tiles), whole K range in
-// ascending order (the fp32 sum over scale groups has one fixed order).  An expert with many rows becomes
-// many units that run side by side on different CUs and find the expert's weights in L2 / Infinity Cache,
-// instead of one wavefront streaming the same weights once per 32 rows.
-// The four wavefronts of a workgroup work on the same chunk (four neighbouring tile pairs), so the chunk's
-// tokens go through LDS once per workgroup: every thread loads one 16-byte piece of the 64 x 64-byte K block
-// (rows are read in 64-byte runs instead of 16-byte crumbs per lane), writes it in MFMA-operand order, and
-// each wavefront reads its four B operands back with conflict-free 1 KiB sweeps; one barrier per two K blocks.
-// Besides HBM the vector ALU bounds it (the fold of 64 sums and the unpacking take longer than the MFMAs), so the fold is
-// conversion, product and sum alone: no shift (the scales in LDS are a sixteenth) and no clearing (the first product of a
-// group starts from the instruction's own zero).  DeepSeek-V3 shape, groups of 256, us a layer call before / after both
-// and the halved barriers: uniform 512 / 1024 / 2048 tokens 1040 / 1236 / 1765 -> 1030 / 1206 / 1707, Zipf(1.1) 128 /
-// 1024 tokens 334 / 929 -> 324 / 883 (512 skewed tokens: less than runs of one side differ); groups of 128 (scales from
-// memory) 1237 -> 1193 at 512, 771 -> 729 Zipf.
+// One wavefront per unit (chunk of up to 64 rows of one expert, 32 channels), whole K range in ascending order (the fp32
+// sum over scale groups has one fixed order).  An expert with many rows becomes many units that run side by side on
+// different CUs and find the expert's weights in L2 / Infinity Cache, instead of one wavefront streaming the same weights
+// once per 32 rows.
+// 32 channels instead of a pair of 32-channel tiles: accumulators and fp32 sums are 64 registers, four wavefronts fit a SIMD.
+// The vector instructions of the fold and of the unpacking, the MFMAs, the LDS reads and the wait for memory follow each
+// other in a wavefront, so what runs beside them is other wavefronts.  For the gate_up product the 32 channels are 16 of the
+// gate and the 16 of the up projection that belong to them, out of half a storage tile each: they meet in one lane.
+// The four wavefronts of a workgroup share the chunk's tokens: stages of 8 KiB (two K blocks of 64 rows, or four of 32 for a
+// chunk of at most 32 rows) in a ring of three, copied by LDS-direct loads (no registers) two stages ahead, and one barrier
+// per stage.  A wavefront requests its weights two stages ahead as well, between the tokens of the same stages: the memory
+// counter retires loads in order, so that the wait for a stage is a count.
+// The fold is conversion, product and sum alone: no shift (the scales in LDS are a sixteenth) and no clearing (the first
+// product of a group starts from the instruction's own zero).
+// What bounds it: the weight stream where the experts have one chunk each (6.1 to 6.4 TB/s), the vector unit and the MFMAs,
+// which share its issue, where a hot expert's chunks find their weights in L2.  DeepSeek-V3 shape, groups of 256, us a layer
+// call on 64 channels per wavefront with two of them on a SIMD, tokens through registers and a barrier every two K blocks
+// of 64 / on this: uniform 100 / 600 / 1024 tokens 928 / 1047 / 1164 -> 876 / 983 / 1085, Zipf(1.1) 256 / 512 / 1024 tokens
+// 428 / 606 / 890 -> 391 / 563 / 838.  More loads in flight (three or four stages of weights, three of tokens, then three
+// wavefronts on a SIMD) 2 to 4 % slower; the chunks of hot experts first, or spread among the others, 0 to 2 % slower than in
+// the order of the experts; all weights through the caches 1037 -> 1126 at 600 tokens.
 constexpr int kW4Chunk = 64;
-constexpr int kW4LdsGroups = 32;  // K groups whose scales are kept in LDS (8 KiB per wavefront)
-// LDS_SCALES: the group scales of the wavefront's channels fit LDS (K / group <= kW4LdsGroups)
-template <int EPI, bool LDS_SCALES>
-__global__ __launch_bounds__(256, 2) void gmm_w4_stream_kernel(W4Args p)
+constexpr int kW4LdsGroups = 32;     // K groups whose scales the pair-order kernel keeps in LDS (8 KiB per wavefront)
+constexpr int kW4StageBytes = 8192;  // LDS bytes of the tokens of one stage
+constexpr int kW4Ring = 3 * kW4StageBytes;
+
+// LDS: the ring of token stages, the group scales of four times 32 channels
+static int w4_lds_bytes(int64_t n_groups) { return kW4Ring + (int)n_groups * 512; }
+constexpr int kW4LdsMax = 163840;
+constexpr int kW4ScaleGroups = (kW4LdsMax - kW4Ring) / 512;
+
+#define MOE355_LPTR(p) ((__attribute__((address_space(3))) void*)(p))
+
+// what the bodies of a chunk share: everything but the lane's own offsets is the same in all lanes of a wavefront
+struct W4Unit {
+    int8_t* lds;
+    const float* scales;   // LDS: scale / 16 (shift: scale) of the unit's channels, [group][32]
+    const float* gscale;   // scales of the expert, [group][N]
+    const uint8_t* w;      // the lane's 16 bytes of the unit's first K block
+    int e, u, row0, row1;  // row1: the end of the expert's rows
+    bool have, shift;
+};
+
+// NB: blocks of 32 rows.  STREAM: the expert has a single chunk, nobody else reads these weights: non-temporal loads (the
+// faster pure stream).  Otherwise the sibling chunks of the expert run at the same time on the same XCD (their workgroup
+// numbers differ by a multiple of 8) and ordinary loads let them share one fetch in L2.
+template <int EPI, bool LDS_SCALES, int NB, bool STREAM, bool FAR>
+__device__ __forceinline__ void w4_chunk_body(const W4Args& p, const W4Unit& t, const __amdgpu_buffer_rsrc_t xr, const int8_t* xb,
+                                              const int64_t* xo)
 {
+    constexpr int BLOCKS = 4 / NB;            // K blocks of a stage
+    constexpr int BLOCK_BYTES = NB * 2048;
     const GmmArgs& a = p.g;
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
-    const int NB = a.N >> 5, KB64 = a.K >> 6;
-    const int upe = NB >> 1;
-    // workgroup = (chunk, four neighbouring tile pairs); a wavefront past the last pair still stages tokens
-    const int quads = (upe + 3) >> 2;
-    const int chunk = (int)(blockIdx.x / quads);
-    const int pi_raw = (int)(blockIdx.x % quads) * 4 + wave;
-    const bool have = pi_raw < upe;
-    const int pi = have ? pi_raw : 0;
-    int e = 0;
-    int64_t row0 = 0, row1 = 0;
-    bool single_chunk = false;
-    if (!find_chunk(a.gl, a.gl_type, a.E, chunk, kW4Chunk, lane, e, row0, row1, single_chunk)) return;
-    if (row1 > a.R) row1 = a.R;
-    if (row1 <= row0) return;
-    const int nb0 = (EPI == EPI_SWIGLU) ? pi : 2 * pi;
-    const int nb1 = (EPI == EPI_SWIGLU) ? pi + upe : 2 * pi + 1;
-
-    const uint8_t* w0 = p.w4 + (((int64_t)e * NB + nb0) * KB64) * 1024 + lane * 16;
-    const uint8_t* w1 = p.w4 + (((int64_t)e * NB + nb1) * KB64) * 1024 + lane * 16;
-    // weights and tokens: rings of RW single K blocks, requested RW - 1 blocks ahead of their MFMAs.  Both
-    // rings have the same depth on purpose: the memory counter retires loads in order, so waiting for a
-    // token block that was requested late would also wait for every weight block requested before it.
-    constexpr int RW = LDS_SCALES ? 6 : 4;  // even; scales read from memory inside the fold need the registers of a slot
-    v4i a0[RW], a1[RW];
-    // STREAM: the expert has a single chunk, nobody else reads these weights: non-temporal loads (the faster
-    // pure stream).  Otherwise the sibling chunks of the expert run at the same time on the same XCD (their
-    // workgroup numbers differ by a multiple of 16) and ordinary loads let them share one fetch in L2.
-    auto load_weights = [&](auto stream, int slot, int kb) {
-        const int k = kb < KB64 ? kb : KB64 - 1;  // past the end: a valid block that is never used
-        if constexpr (decltype(stream)::value) {
-            a0[slot] = __builtin_nontemporal_load((const v4i*)(w0 + (int64_t)k * 1024));
-            a1[slot] = __builtin_nontemporal_load((const v4i*)(w1 + (int64_t)k * 1024));
-        } else {
-            a0[slot] = *(const v4i*)(w0 + (int64_t)k * 1024);
-            a1[slot] = *(const v4i*)(w1 + (int64_t)k * 1024);
-        }
+    const int c32 = lane & 31, hi = lane >> 5;
+    const int KB64 = a.K >> 6;
+    const int steps_per_group = p.group >> 6;  // K blocks per scale group
+    // channel of the lane's run q (0..3) of four results: 8 q + 4 hi + 0..3 of the unit
+    auto run_channel = [&](int q) {
+        return EPI == EPI_SWIGLU ? (q >= 2 ? a.N >> 1 : 0) + t.u * 16 + 8 * (q & 1) + 4 * hi : t.u * 32 + 8 * q + 4 * hi;
     };
+    int frag[2];  // where this lane's operand bytes of K 0..31 and 32..63 of a block lie; rows 32.. are 2048 bytes further
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) frag[kk] = c32 * 64 + (((2 * kk + hi) ^ ((c32 >> 2) & 3)) * 16);
 
-    const int tok = lane & 31;
-    const int hi = lane >> 5;
-    const int steps_per_group = p.group >> 6;  // 64-wide K blocks per scale group
-    const int n_groups = a.K / p.group;
-    const float* gs = p.gscale + (int64_t)e * n_groups * a.N;
-
-    __shared__ __attribute__((aligned(16))) int8_t Bs[2][2][kW4Chunk * 64];  // two stages of two blocks of 64 rows x 64 K bytes
-    int64_t row[2];
-    bool valid[2];
+    v16i c[NB];
+    float f[NB][16];
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-        row[b] = row0 + 32 * b + tok;
-        valid[b] = row[b] < row1;
-    }
-    // staging: thread t carries row (t % 16) + 16 * (t / 64), 16-byte piece (t / 16) % 4 of the K block
-    const int srow = (threadIdx.x & 15) + 16 * wave;
-    const int skc = (threadIdx.x >> 4) & 3;
-    int64_t sr = row0 + srow;
-    if (sr > row1 - 1) sr = row1 - 1;  // rows past the chunk's end repeat its last row (never stored)
-    if (a.row_src) sr = a.row_src[sr];  // the row's values lie in its token's row
-    const int8_t* xs = a.x + sr * a.K + skc * 16;
-    const int lds_off = ((((skc >> 1) * 2 + (srow >> 5)) * 64) + (skc & 1) * 32 + (srow & 31)) * 16;
-    const bool two = row0 + 32 < row1;  // the second token block holds rows (wavefront-uniform)
-
-    v16i c0[2], c1[2];
-    float f0[2][16], f1[2][16];
+    for (int b = 0; b < NB; ++b) {
+        c[b] = (v16i){0};
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-        c0[b] = (v16i){0};
-        c1[b] = (v16i){0};
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            f0[b][v] = 0.0f;
-            f1[b][v] = 0.0f;
-        }
-    }
-    // The scales of this wavefront's 64 channels for every K group sit in LDS (when they fit: up to 32
-    // groups), loaded once up front: the K loop then has no load whose result is needed at once, and its
-    // waits for weights and tokens stay partial.
-    // Kept there as scale / 16: the sixteen of the accumulators then cancels in the product, bit for bit as long as the
-    // quotient is exact; a wavefront with a scale so small that it is not shifts its accumulators instead.
-    __shared__ float Ss[4][LDS_SCALES ? kW4LdsGroups * 64 : 1];
-    bool shift = !LDS_SCALES;
-    if constexpr (LDS_SCALES) {
-        const int ch = lane < 32 ? nb0 * 32 + lane : nb1 * 32 + (lane - 32);
-        for (int g0 = 0; g0 < n_groups; g0 += 8) {  // eight loads in flight at a time
-            float t[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) t[j] = gs[(int64_t)(g0 + j < n_groups ? g0 + j : n_groups - 1) * a.N + ch];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                if (g0 + j < n_groups) Ss[wave][(g0 + j) * 64 + lane] = t[j] * 0.0625f;
-                shift |= (t[j] * 0.0625f) * 16.0f != t[j];
-            }
-        }
-        shift = __ballot(shift) != 0;
-        if (shift)
-            for (int i = lane; i < n_groups * 64; i += 64) Ss[wave][i] = gs[(int64_t)(i >> 6) * a.N + ch];
+        for (int v = 0; v < 16; ++v) f[b][v] = 0.0f;
     }
     int in_group = 0, grp = 0;
     // f += float(acc / 16) * scale[e, grp, channel]
-    auto fold_with = [&](const v4f* s0, const v4f* s1) {
+    auto fold = [&]() {
+        if (t.shift) {
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            if (b == 1 && !two) break;  // no rows in the second token block
-            if (shift) {
-                c0[b] = c0[b] >> 4;
-                c1[b] = c1[b] >> 4;
-            }
+            for (int b = 0; b < NB; ++b) c[b] = c[b] >> 4;
+        }
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
+        for (int q = 0; q < 4; ++q) {
+            v4f s;
+            if constexpr (LDS_SCALES) s = *(const v4f*)(t.scales + grp * 32 + 8 * q + 4 * hi);
+            else s = *(const v4f*)(t.gscale + (int64_t)grp * a.N + run_channel(q));
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    f0[b][4 * q + j] = f0[b][4 * q + j] + (float)c0[b][4 * q + j] * s0[q][j];
-                    f1[b][4 * q + j] = f1[b][4 * q + j] + (float)c1[b][4 * q + j] * s1[q][j];
-                }
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) f[b][4 * q + j] = f[b][4 * q + j] + (float)c[b][4 * q + j] * s[j];
         }
         in_group = 0;
         ++grp;
     };
-    auto fold = [&]() {
-        v4f s0[4], s1[4];
-        if constexpr (LDS_SCALES) {
-            const float* sl = &Ss[wave][grp * 64 + 4 * hi];
+
+    // A wavefront copies 16 rows x 64 values by one load.  NB == 2: rows 16 w .. of both blocks of a stage, else both halves of
+    // the rows of block w.
+    auto load_tokens = [&](int8_t* stage, int kb) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                s0[q] = *(const v4f*)(sl + 8 * q);
-                s1[q] = *(const v4f*)(sl + 32 + 8 * q);
-            }
-            fold_with(s0, s1);
-        } else {
-            const float* s = gs + (int64_t)grp * a.N + 4 * hi;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                s0[q] = *(const v4f*)(s + nb0 * 32 + 8 * q);
-                s1[q] = *(const v4f*)(s + nb1 * 32 + 8 * q);
-            }
-            fold_with(s0, s1);
+        for (int i = 0; i < 2; ++i) {
+            const int kw = kb + (NB == 2 ? i : wave);
+            const int k = kw < KB64 ? kw : KB64 - 1;  // past the end: the last block again, never used
+            int8_t* to = stage + (NB == 2 ? i * BLOCK_BYTES + wave * 1024 : wave * BLOCK_BYTES + i * 1024);
+            const int64_t from = xo[NB == 2 ? 0 : i];
+            if constexpr (FAR) *(v4i*)(to + lane * 16) = *(const v4i*)(xb + from + (int64_t)k * 64);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, MOE355_LPTR(to), 16, (int)from, k * 64, 0, 0);
         }
     };
-    // tokens: K blocks kb and kb + 1 (kb even) live in LDS stage (kb / 2) & 1; treg[kb % RW] carries block kb from its load
-    // until it is written to LDS two steps before it is used
-    auto load_tokens = [&](int kb) { return *(const v4i*)(xs + (int64_t)(kb < KB64 ? kb : KB64 - 1) * 64); };
-    v4i treg[RW];
-    treg[0] = load_tokens(0);
-    treg[1] = load_tokens(1);
-    *(v4i*)(&Bs[0][0][lds_off]) = treg[0];
-    *(v4i*)(&Bs[0][1][lds_off]) = treg[1];
+    v4i w[2 * BLOCKS];  // weights of the two stages in flight
+    auto load_weights = [&](int slot, int kb) {
+        const int k = kb < KB64 ? kb : KB64 - 1;
+        if constexpr (STREAM) w[slot] = __builtin_nontemporal_load((const v4i*)(t.w + (int64_t)k * 1024));
+        else w[slot] = *(const v4i*)(t.w + (int64_t)k * 1024);
+    };
+    // one K block of a stage
+    auto block = [&](const int8_t* st, v4i wv) {
+        v4i x[2][NB];  // [K half][rows]
 #pragma unroll
-    for (int i = 2; i < RW + 2; ++i) treg[i % RW] = load_tokens(i);
-    __syncthreads();
-    auto step = [&](auto stream, int slot, int kb) {  // one 64-wide K block; slot = kb % RW (compile time)
-        v4i bl[2], bh[2];  // [token block]: K 0..31 / 32..63 of the block
-        const int8_t* st = Bs[(kb >> 1) & 1][kb & 1];
+        for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            bl[b] = *(const v4i*)(st + ((0 * 2 + b) * 64 + lane) * 16);
-            bh[b] = *(const v4i*)(st + ((1 * 2 + b) * 64 + lane) * 16);
-        }
-        *(v4i*)(&Bs[((kb >> 1) & 1) ^ 1][kb & 1][lds_off]) = treg[(slot + 2) % RW];  // block kb + 2; its stage was last read before the last barrier
-        treg[(slot + 2) % RW] = load_tokens(kb + 2 + RW);
-        const v4i l0 = nib_lo(a0[slot]), h0 = nib_hi(a0[slot]);
-        const v4i l1 = nib_lo(a1[slot]), h1 = nib_hi(a1[slot]);
-        load_weights(stream, (slot + RW - 1) % RW, kb + RW - 1);  // the slot block kb - 1 has just left
+            for (int b = 0; b < NB; ++b) x[kk][b] = *(const v4i*)(st + b * 2048 + frag[kk]);
+        const v4i lo = nib_lo(wv), up = nib_hi(wv);
         const bool first = in_group == 0;  // of its scale group: the accumulators start from the instruction's own zero
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            if (b == 1 && !two) break;
-            if (first) {
-                c0[b] = mfma_i8(l0, bl[b], (v16i){0});
-                c1[b] = mfma_i8(l1, bl[b], (v16i){0});
-            } else {
-                c0[b] = mfma_i8(l0, bl[b], c0[b]);
-                c1[b] = mfma_i8(l1, bl[b], c1[b]);
-            }
-            c0[b] = mfma_i8(h0, bh[b], c0[b]);
-            c1[b] = mfma_i8(h1, bh[b], c1[b]);
+        for (int b = 0; b < NB; ++b) {
+            if (first) c[b] = mfma_i8(lo, x[0][b], (v16i){0});
+            else c[b] = mfma_i8(lo, x[0][b], c[b]);
         }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) c[b] = mfma_i8(up, x[1][b], c[b]);
         if (++in_group == steps_per_group) fold();
-        if (slot & 1) __syncthreads();  // blocks kb + 1 and kb + 2 are visible; nobody still reads kb - 1 and kb
     };
-    // whole passes through the ring without a condition on kb; the remainder is peeled
-    const int kb_full = (KB64 / RW) * RW;
-    auto k_loop = [&](auto stream) {
+    const int n_stages = (KB64 + 2 * BLOCKS - 1) / (2 * BLOCKS) * 2;  // the registers go by pairs of stages: the last ones may hold nothing
+    int8_t* st_now = t.lds;  // stage s, and where stage s + 2 goes
+    int8_t* st_load = t.lds + 2 * kW4StageBytes;
+    auto next_stage = [&](int8_t* st) { return st == t.lds + 2 * kW4StageBytes ? t.lds : st + kW4StageBytes; };
+    // Stage s.  PAR: which half of the weight registers; LOAD: stage s + 2 is requested; LAST: the last stage.
+    // Behind the tokens of a stage there are its weights, the tokens and the weights of the next stage when its turn comes;
+    // in front of the last one the next stage's are missing.
+    auto run_stage = [&](auto par, auto load, auto last, int s) {
+        constexpr int PAR = decltype(par)::value;
+        constexpr bool LOAD = decltype(load)::value, LAST = decltype(last)::value;
+        constexpr int BEHIND = LAST ? 0 : 2 * BLOCKS + 2;
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(BEHIND) : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (LOAD) load_tokens(st_load, (s + 2) * BLOCKS);
 #pragma unroll
-        for (int i = 0; i < RW - 1; ++i) load_weights(stream, i, i);
-        for (int kb = 0; kb < kb_full; kb += RW) {
-#pragma unroll
-            for (int i = 0; i < RW; ++i) step(stream, i, kb + i);
+        for (int i = 0; i < BLOCKS; ++i) {
+            if (!LOAD && s * BLOCKS + i >= KB64) break;
+            block(st_now + i * BLOCK_BYTES, w[PAR * BLOCKS + i]);
+            if constexpr (LOAD) load_weights(PAR * BLOCKS + i, (s + 2) * BLOCKS + i);
         }
-#pragma unroll
-        for (int i = 0; i < RW - 1; ++i)
-            if (kb_full + i < KB64) step(stream, i, kb_full + i);
+        __builtin_amdgcn_sched_barrier(0);
+        st_now = next_stage(st_now);
+        st_load = next_stage(st_load);
     };
-    if (single_chunk) k_loop(std::true_type{});
-    else k_loop(std::false_type{});
-    if (!have) return;  // (after the last barrier)
-    // both token scales are requested before the first store of the epilogue (a load placed behind a store
-    // would wait for it: the memory counter retires in order)
-    float rs_pre[2];
+    {
+        const std::integral_constant<int, 0> p0;
+        const std::integral_constant<int, 1> p1;
+        const std::true_type yes;
+        const std::false_type no;
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-        const int64_t r = valid[b] ? row[b] : row0;
-        rs_pre[b] = a.row_scale[a.row_src ? (int64_t)a.row_src[r] : r];
+        for (int s = 0; s < 2; ++s) {
+            load_tokens(t.lds + s * kW4StageBytes, s * BLOCKS);
+#pragma unroll
+            for (int i = 0; i < BLOCKS; ++i) load_weights(s * BLOCKS + i, s * BLOCKS + i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        int s = 0;
+        for (; s + 2 < n_stages; s += 2) {
+            run_stage(p0, yes, no, s);
+            run_stage(p1, yes, no, s + 1);
+        }
+        run_stage(p0, no, no, s);
+        run_stage(p1, no, yes, s + 1);
+    }
+    if (!t.have) return;  // (after the last barrier)
+    int row[NB];
+    bool valid[NB];
+    // the token scales are requested before the first store of the epilogue (a load placed behind a store
+    // would wait for it: the memory counter retires in order)
+    float rs_pre[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        row[b] = t.row0 + 32 * b + c32;
+        valid[b] = row[b] < t.row1;
+        const int r = valid[b] ? row[b] : t.row0;
+        rs_pre[b] = a.row_scale[a.row_src ? a.row_src[r] : r];
     }
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-        if (b == 1 && !two) break;
+    for (int b = 0; b < NB; ++b) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int ch = 8 * q + 4 * hi;
-            float g[4], u[4];
+        for (int q = 0; q < 2; ++q) {  // runs q and q + 2: a gate run and its up run, or any two
+            const int ch0 = run_channel(q), ch1 = run_channel(q + 2);
+            float g[4], up[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                g[j] = f0[b][4 * q + j];
-                u[j] = f1[b][4 * q + j];
+                g[j] = f[b][4 * q + j];
+                up[j] = f[b][8 + 4 * q + j];
             }
             if (p.bias) {
-                const v4f bg = *(const v4f*)(p.bias + (int64_t)e * a.N + nb0 * 32 + ch);
-                const v4f bu = *(const v4f*)(p.bias + (int64_t)e * a.N + nb1 * 32 + ch);
+                const v4f bg = *(const v4f*)(p.bias + (int64_t)t.e * a.N + ch0);
+                const v4f bu = *(const v4f*)(p.bias + (int64_t)t.e * a.N + ch1);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     g[j] = g[j] + bg[j];
-                    u[j] = u[j] + bu[j];
+                    up[j] = up[j] + bu[j];
                 }
             }
-            epilogue_run_w4<EPI>(a, row[b], valid[b], nb0 * 32 + ch, nb1 * 32 + ch, g, u, rs_pre[b]);
+            epilogue_run_w4<EPI>(a, row[b], valid[b], ch0, ch1, g, up, rs_pre[b]);
         }
+    }
+}
+
+// LDS_SCALES: the group scales of the wavefront's channels are in LDS
+template <int EPI, bool LDS_SCALES>
+__global__ __launch_bounds__(256, LDS_SCALES ? 4 : 3) void gmm_w4_stream_kernel(W4Args p)
+{
+    const GmmArgs& a = p.g;
+    extern __shared__ __attribute__((aligned(16))) int8_t w4_lds[];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63;
+    const int NB = a.N >> 5, KB64 = a.K >> 6;
+    // workgroup = (chunk, four neighbouring units of 32 channels); a wavefront past the last unit still stages tokens
+    const int quads = (NB + 3) >> 2;
+    const int chunk = (int)(blockIdx.x / quads);
+    const int u_raw = (int)(blockIdx.x % quads) * 4 + wave;
+    W4Unit t;
+    t.lds = w4_lds;
+    t.have = u_raw < NB;
+    t.u = t.have ? u_raw : 0;
+    int e, row0, row1;  // (rows are fewer than 2^31)
+    bool single;
+    if (p.tm.count) {
+        if (chunk >= p.tm.count[0]) return;
+        e = p.tm.expert[chunk];
+        row0 = p.tm.row_begin[chunk];
+        row1 = p.tm.row_end[chunk];
+        single = (e & kOnlyTile) != 0;
+        e &= ~kOnlyTile;
+    } else {
+        int64_t first_row, end_row;
+        if (!find_chunk(a.gl, a.gl_type, a.E, chunk, kW4Chunk, lane, e, first_row, end_row, single)) return;
+        row0 = (int)first_row;
+        row1 = (int)(end_row < a.R ? end_row : a.R);
+    }
+    t.e = __builtin_amdgcn_readfirstlane(e);
+    t.row0 = __builtin_amdgcn_readfirstlane(row0);
+    row1 = __builtin_amdgcn_readfirstlane(row1);
+    single = __builtin_amdgcn_readfirstlane((int)single);
+    t.row1 = row1 < a.R ? row1 : (int)a.R;
+    if (t.row1 <= t.row0) return;
+
+    // lane l of an MFMA operand: channel l % 32 of the unit, K half l / 32
+    const int c32 = lane & 31, hi = lane >> 5;
+    const int tile = EPI == EPI_SWIGLU ? (t.u >> 1) + (c32 >= 16 ? NB >> 1 : 0) : t.u;
+    const int chunk16 = EPI == EPI_SWIGLU ? hi * 32 + (t.u & 1) * 16 + (c32 & 15) : lane;
+    t.w = p.w4 + (((int64_t)t.e * NB + tile) * KB64) * 1024 + chunk16 * 16;
+
+    // The scales sit in LDS, loaded once up front: the K loop then has no load whose result is needed at once.
+    // Kept there as scale / 16: the sixteen of the accumulators then cancels in the product, bit for bit as long as the
+    // quotient is exact; a wavefront with a scale so small that it is not shifts its accumulators instead.
+    const int n_groups = a.K / p.group;
+    t.gscale = p.gscale + (int64_t)t.e * n_groups * a.N;
+    float* ss = (float*)(w4_lds + kW4Ring) + wave * n_groups * 32;
+    t.scales = ss;
+    t.shift = !LDS_SCALES;
+    if constexpr (LDS_SCALES) {
+        const float* gs = t.gscale + (EPI == EPI_SWIGLU ? (c32 >= 16 ? a.N >> 1 : 0) + t.u * 16 + (c32 & 15) : t.u * 32 + c32);
+        bool inexact = false;
+        for (int g0 = 0; g0 < n_groups; g0 += 16) {  // eight loads in flight at a time
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int g = g0 + 2 * j + hi;
+                v[j] = gs[(int64_t)(g < n_groups ? g : n_groups - 1) * a.N];
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int g = g0 + 2 * j + hi;
+                if (g < n_groups) ss[g * 32 + c32] = v[j] * 0.0625f;
+                inexact |= (v[j] * 0.0625f) * 16.0f != v[j];
+            }
+        }
+        t.shift = __ballot(inexact) != 0;
+        if (t.shift)
+            for (int g = hi; g < n_groups; g += 2) ss[g * 32 + c32] = gs[(int64_t)g * a.N];
+    }
+
+    // Tokens: a load copies 16 rows x 64 values of a K block, the 16-byte piece c of row r to place c ^ (r / 4) % 4 of the
+    // row's 64 bytes: sixteen rows at one piece fall into sixteen different bank groups.
+    const bool two = t.row0 + 32 < t.row1;  // the second block of 32 rows holds some
+    const int rows = t.row1 - t.row0;
+    int64_t xo[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int r = (two ? wave : i) * 16 + (lane >> 2);
+        const int lrow = r < rows ? r : rows - 1;  // rows past the chunk's end repeat its last row (never stored)
+        // the row's values lie in its token's row, or in the row itself
+        xo[i] = (int64_t)(a.row_src ? a.row_src[t.row0 + lrow] : lrow) * a.K + (((lane & 3) ^ ((r >> 2) & 3)) * 16);
+    }
+    const int8_t* xb = a.row_src ? a.x : a.x + (int64_t)t.row0 * a.K;
+    // Buffer loads, whose offsets have 32 bits: a global load to LDS counts as a flat access, behind which the compiler waits
+    // for every load in flight.  A chunk with rows further away than that copies them through registers.
+    const bool far = __ballot((xo[0] > xo[1] ? xo[0] : xo[1]) + a.K > 0xffffffffll) != 0;
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)xb, 0, -1, 0x00027000);
+    if (two) {
+        if (far) w4_chunk_body<EPI, LDS_SCALES, 2, false, true>(p, t, xr, xb, xo);
+        else if (single) w4_chunk_body<EPI, LDS_SCALES, 2, true, false>(p, t, xr, xb, xo);
+        else w4_chunk_body<EPI, LDS_SCALES, 2, false, false>(p, t, xr, xb, xo);
+    } else {
+        if (far) w4_chunk_body<EPI, LDS_SCALES, 1, false, true>(p, t, xr, xb, xo);
+        else w4_chunk_body<EPI, LDS_SCALES, 1, true, false>(p, t, xr, xb, xo);
     }
 }
 
@@ -698,18 +764,23 @@ static int64_t w4_blocks(int64_t rows, int num_experts, int64_t n)
     // a chunk has at least one row: a decode batch of a few rows has a few chunks, not one per expert (a workgroup
     // that only finds its chunk missing still costs its dispatch)
     const int64_t by_experts = rows / kW4Chunk + num_experts;
-    return (rows < by_experts ? rows : by_experts) * ((n / 64 + 3) / 4);
+    return (rows < by_experts ? rows : by_experts) * ((n / 32 + 3) / 4);
 }
 
 template <int EPI>
-static void launch_w4(const W4Args& p, int64_t blocks, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1)
+static bool launch_w4(const W4Args& p, int64_t blocks, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1)
 {
-    const bool lds_scales = p.g.K / p.group <= kW4LdsGroups;
+    const int64_t n_groups = p.g.K / p.group;
+    const bool lds_scales = n_groups <= kW4ScaleGroups;
+    const int lds = lds_scales ? w4_lds_bytes(n_groups) : kW4Ring;
     auto kernel = lds_scales ? gmm_w4_stream_kernel<EPI, true> : gmm_w4_stream_kernel<EPI, false>;
+    static OncePerDevice once;
+    if (lds_scales && !allow_dynamic_lds(once, (const void*)gmm_w4_stream_kernel<EPI, true>, kW4LdsMax)) return false;
     if (ev0 && ev1)
-        hipExtLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, st, ev0, ev1, 0, p);
+        hipExtLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), lds, st, ev0, ev1, 0, p);
     else
-        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, st, p);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), lds, st, p);
+    return true;
 }
 
 static int check_w4(const void* x, const void* w, const float* scale, const int64_t* gl, int gl_type, int64_t rows,
@@ -762,11 +833,18 @@ extern "C" int moe355_w4_offset_correction(const uint8_t* weight_nz4, const floa
     return launch_status();
 }
 
-static int gmm1_w4_impl(const int8_t* x, const uint8_t* weight_nz4, const float* weight_scale, int64_t group_size,
-                        const float* bias, const float* x_scale, const int64_t* group_list, int group_list_type,
-                        int64_t rows, int64_t k, int64_t n, int num_experts, float swiglu_limit, int8_t* out,
-                        float* out_scale, void* workspace, size_t workspace_bytes, void* stream,
-                        const int32_t* row_src)
+TileSpec moe355::w4_chunk_spec(int64_t rows, int num_experts, void* workspace)
+{
+    TileSpec t = tile_spec(rows, num_experts, kW4Chunk, workspace);
+    t.flag_only = 1;
+    return t;
+}
+
+int moe355::gmm1_w4_impl(const int8_t* x, const uint8_t* weight_nz4, const float* weight_scale, int64_t group_size,
+                         const float* bias, const float* x_scale, const int64_t* group_list, int group_list_type,
+                         int64_t rows, int64_t k, int64_t n, int num_experts, float swiglu_limit, int8_t* out,
+                         float* out_scale, void* workspace, size_t workspace_bytes, void* stream,
+                         const int32_t* row_src, const TileMap* chunks)
 {
     int rc = check_w4(x, weight_nz4, weight_scale, group_list, group_list_type, rows, k, n, num_experts, group_size);
     if (rc != MOE355_OK) return rc;
@@ -792,10 +870,11 @@ static int gmm1_w4_impl(const int8_t* x, const uint8_t* weight_nz4, const float*
     p.gscale = weight_scale;
     p.bias = bias;
     p.group = (int)group_size;
+    if (chunks) p.tm = *chunks;
     const int64_t blocks = w4_blocks(rows, num_experts, n);
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     take_profile_events(ev0, ev1);
-    launch_w4<EPI_SWIGLU>(p, blocks, st, ev0, ev1);
+    if (!launch_w4<EPI_SWIGLU>(p, blocks, st, ev0, ev1)) return MOE355_E_LAUNCH;
     launch_swiglu_requant(p.g.y, group_list, group_list_type, num_experts, rows, (int)(n / 2), out, out_scale, st);
     return launch_status();
 }
@@ -807,7 +886,7 @@ extern "C" int moe355_gmm1_swiglu_quant_w4(const int8_t* x, const uint8_t* weigh
                                            float* out_scale, void* workspace, size_t workspace_bytes, void* stream)
 {
     return gmm1_w4_impl(x, weight_nz4, weight_scale, group_size, bias, x_scale, group_list, group_list_type, rows, k,
-                        n, num_experts, swiglu_limit, out, out_scale, workspace, workspace_bytes, stream, nullptr);
+                        n, num_experts, swiglu_limit, out, out_scale, workspace, workspace_bytes, stream, nullptr, nullptr);
 }
 
 extern "C" int moe355_gmm1_swiglu_quant_w4_gather(const int8_t* x, const float* x_scale, const int32_t* row_token,
@@ -819,7 +898,7 @@ extern "C" int moe355_gmm1_swiglu_quant_w4_gather(const int8_t* x, const float* 
 {
     if (rows > 0 && !row_token) return MOE355_E_ARG;
     return gmm1_w4_impl(x, weight_nz4, weight_scale, group_size, bias, x_scale, group_list, group_list_type, rows, k,
-                        n, num_experts, swiglu_limit, out, out_scale, workspace, workspace_bytes, stream, row_token);
+                        n, num_experts, swiglu_limit, out, out_scale, workspace, workspace_bytes, stream, row_token, nullptr);
 }
 
 // Up to 40 tokens.  Uniform routing would gain beyond (47 tokens 750 -> 710 us, 64 844 -> 795 us), but skewed routing loses by
@@ -893,10 +972,10 @@ int moe355::gmm2_w4_pairs(const int8_t* x, const float* x_scale, const int32_t* 
     return launch_status();
 }
 
-extern "C" int moe355_gmm2_dequant_w4(const int8_t* x, const uint8_t* weight_nz4, const float* scale,
-                                      int64_t group_size, const float* bias, const float* per_token_scale,
-                                      const int64_t* group_list, int group_list_type, int64_t rows, int64_t k,
-                                      int64_t n, int num_experts, void* out, int out_dtype, void* stream)
+int moe355::gmm2_w4_impl(const int8_t* x, const uint8_t* weight_nz4, const float* scale, int64_t group_size,
+                         const float* bias, const float* per_token_scale, const int64_t* group_list, int group_list_type,
+                         int64_t rows, int64_t k, int64_t n, int num_experts, void* out, int out_dtype, void* stream,
+                         const TileMap* chunks)
 {
     int rc = check_w4(x, weight_nz4, scale, group_list, group_list_type, rows, k, n, num_experts, group_size);
     if (rc != MOE355_OK) return rc;
@@ -919,7 +998,17 @@ extern "C" int moe355_gmm2_dequant_w4(const int8_t* x, const uint8_t* weight_nz4
     p.gscale = scale;
     p.bias = bias;
     p.group = (int)group_size;
+    if (chunks) p.tm = *chunks;
     const int64_t blocks = w4_blocks(rows, num_experts, n);
-    launch_w4<EPI_DEQUANT>(p, blocks, (hipStream_t)stream, nullptr, nullptr);
+    if (!launch_w4<EPI_DEQUANT>(p, blocks, (hipStream_t)stream, nullptr, nullptr)) return MOE355_E_LAUNCH;
     return launch_status();
+}
+
+extern "C" int moe355_gmm2_dequant_w4(const int8_t* x, const uint8_t* weight_nz4, const float* scale,
+                                      int64_t group_size, const float* bias, const float* per_token_scale,
+                                      const int64_t* group_list, int group_list_type, int64_t rows, int64_t k,
+                                      int64_t n, int num_experts, void* out, int out_dtype, void* stream)
+{
+    return gmm2_w4_impl(x, weight_nz4, scale, group_size, bias, per_token_scale, group_list, group_list_type, rows, k, n,
+                        num_experts, out, out_dtype, stream, nullptr);
 }

@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "gmm_common.h"
+#include "gmm_tiled.h"
 #include "layer_parts.h"
 
 using namespace moe355;
@@ -195,7 +196,7 @@ Buffers lay_out(const moe355_layer& l, const Forms& f, int64_t T, void* base)
         b.mlp_bytes = l.weights == W_INT4 ? y : moe355_gmm1_swiglu_quant_workspace(R, 2 * I, H, E);
         b.mlp_ws = a.take<void>(b.mlp_bytes > o ? b.mlp_bytes : o);
         b.o = b.mlp_ws;
-        b.gmm2_bytes = l.weights == W_INT4 ? 0 : moe355_gmm2_dequant_workspace(R, H, I, E);
+        b.gmm2_bytes = l.weights == W_INT4 ? tiled_workspace_bytes(R, E, 64) : moe355_gmm2_dequant_workspace(R, H, I, E);
         b.gmm2_ws = a.take<void>(b.gmm2_bytes);
     }
     if (f.merged) {
@@ -323,13 +324,14 @@ int routed_sorted(const moe355_layer& l, const Buffers& b, int64_t T, bool tiles
     const int E = l.num_experts;
     int rc;
     if (l.weights == W_INT4) {
-        rc = moe355_gmm1_swiglu_quant_w4_gather(b.xq, b.x_scale, b.row_token, (const uint8_t*)l.w13,
-                                                (const float*)l.s13, l.group13, nullptr, b.expert_tokens,
-                                                MOE355_GL_COUNT, R, H, 2 * I, E, l.swiglu_limit, b.q1, b.q1_scale,
-                                                b.mlp_ws, b.mlp_bytes, st);
+        const TileMap chunks = w4_chunk_spec(R, E, b.gmm2_ws).tm;
+        const TileMap* tm = tiles_ready ? &chunks : nullptr;
+        rc = gmm1_w4_impl(b.xq, (const uint8_t*)l.w13, (const float*)l.s13, l.group13, nullptr, b.x_scale, b.expert_tokens,
+                          MOE355_GL_COUNT, R, H, 2 * I, E, l.swiglu_limit, b.q1, b.q1_scale, b.mlp_ws, b.mlp_bytes, st,
+                          b.row_token, tm);
         if (rc != MOE355_OK) return rc;
-        return moe355_gmm2_dequant_w4(b.q1, (const uint8_t*)l.w2, (const float*)l.s2, l.group2, nullptr, b.q1_scale,
-                                      b.expert_tokens, MOE355_GL_COUNT, R, I, H, E, b.o, l.x_dtype, st);
+        return gmm2_w4_impl(b.q1, (const uint8_t*)l.w2, (const float*)l.s2, l.group2, nullptr, b.q1_scale, b.expert_tokens,
+                            MOE355_GL_COUNT, R, I, H, E, b.o, l.x_dtype, st, tm);
     }
     const bool list = l.weights == W_INT8_LIST;
     rc = gmm1_impl(b.xq, list ? nullptr : (const int8_t*)l.w13, list ? (const int8_t* const*)l.w13 : nullptr,
@@ -439,7 +441,9 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
     if (rc == MOE355_OK && !f.pairs && !f.small) {
         TileSpec specs[2];
         int n = 0;
-        if (l.weights != W_INT4) {
+        if (l.weights == W_INT4) {
+            specs[n++] = w4_chunk_spec(R, l.num_experts, b.gmm2_ws);
+        } else {
             n = gemm_tile_specs(R, l.hidden, 2 * l.intermediate, l.num_experts,
                                 gmm1_tile_ws(b.mlp_ws, R, 2 * l.intermediate), specs);
             n += gemm_tile_specs(R, l.intermediate, l.hidden, l.num_experts, b.gmm2_ws, specs + n);

@@ -104,6 +104,17 @@ void* gmm1_tile_ws(void* workspace, int64_t rows, int64_t n);
 // the tile map (0 or 1) that a grouped product will look for in its workspace
 int gemm_tile_specs(int64_t rows, int64_t k, int64_t n, int num_experts, void* tile_ws, TileSpec* specs);
 
+// int4 weights, sorted rows (gmm_w4.hip): the chunks of both products in the order they run in, for the routing launch to build
+// in a workspace of tiled_workspace_bytes(rows, E, 64); without it (null) every workgroup finds its chunk from the group list
+TileSpec w4_chunk_spec(int64_t rows, int num_experts, void* workspace);
+int gmm1_w4_impl(const int8_t* x, const uint8_t* weight_nz4, const float* weight_scale, int64_t group_size,
+                 const float* bias, const float* x_scale, const int64_t* group_list, int group_list_type, int64_t rows,
+                 int64_t k, int64_t n, int num_experts, float swiglu_limit, int8_t* out, float* out_scale, void* workspace,
+                 size_t workspace_bytes, void* stream, const int32_t* row_src, const TileMap* chunks);
+int gmm2_w4_impl(const int8_t* x, const uint8_t* weight_nz4, const float* scale, int64_t group_size, const float* bias,
+                 const float* per_token_scale, const int64_t* group_list, int group_list_type, int64_t rows, int64_t k,
+                 int64_t n, int num_experts, void* out, int out_dtype, void* stream, const TileMap* chunks);
+
 // int4 weights, pair order (gmm_w4.hip)
 bool w4_pairs_supported(int64_t num_tokens, int top_k, int num_experts, int64_t hidden, int64_t intermediate,
                         int64_t group13, int64_t group2);

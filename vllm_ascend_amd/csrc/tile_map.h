@@ -6,13 +6,13 @@
 
 namespace moe355 {
 
-// in the list by length: the tile is its expert's only one
+// in the list by length and where it is asked for: the tile is its expert's only one
 constexpr int32_t kOnlyTile = 1 << 30;
 
 // (expert, row block) tiles of one launch
 struct TileMap {
     int32_t* count;      // [1]
-    int32_t* expert;     // [max_tiles] (listed by length: and kOnlyTile)
+    int32_t* expert;     // [max_tiles] (and kOnlyTile)
     int32_t* row_begin;  // [max_tiles]
     int32_t* row_end;    // [max_tiles] end of the expert's rows
 };
@@ -24,6 +24,7 @@ struct TileSpec {
     // then the tall ones (more than 192 rows, which become two shorter column items) -- so that the workgroups that
     // start last are the short ones and the compute units finish closer together
     int by_length;
+    int flag_only;  // kOnlyTile also in a list in the order of the experts
 };
 
 // One workgroup of any size, every thread calls it; rows_of(e) = rows of expert e (not negative).  Thread t owns
@@ -100,7 +101,7 @@ __device__ __forceinline__ void build_tile_map(RowsOf rows_of, int E, const Tile
         const int e = e0 + j;
         if (e < E) {
             const int64_t m = rows_of(e);
-            for (int64_t r0 = row; r0 < row + m; r0 += BM) put(t++, e, r0, row + m);
+            for (int64_t r0 = row; r0 < row + m; r0 += BM) put(t++, spec.flag_only && m <= BM ? e | kOnlyTile : e, r0, row + m);
             row += m;
         }
     }
