@@ -15,26 +15,38 @@ constexpr int kHistMaxExperts = 2048;
 // idx == nullptr: the rows lie in pair order (row of token t, slot s = t * top_k + s) and hist_ids holds their ids.
 // hist_out [hist_experts] or load: one more workgroup (the last of the grid's x range) counts the pairs of every expert
 // into the one and adds them to the other, next to the others instead of in a launch of its own.
+struct UnpermuteArgs {
+    int T, top_k, pieces, hist_experts;  // (gridDim would be a load of its own in front of everything else)
+    const uint16_t* permuted;
+    const int32_t* idx;
+    const uint16_t* probs;
+    const uint16_t* residual;
+    uint16_t* out;
+    const int32_t* hist_ids;
+    int64_t H, permuted_rows;
+    int64_t* hist_out;
+    const int64_t* load_counts;
+    int64_t* load;
+};
+
 template <int TOPK, int DT = MOE355_DT_BF16>
-__global__ __launch_bounds__(256) void token_unpermute_kernel(const uint16_t* __restrict__ permuted,
-                                                              const int32_t* __restrict__ idx,
-                                                              const uint16_t* __restrict__ probs, int top_k_rt,
-                                                              int64_t H, int64_t permuted_rows,
-                                                              const uint16_t* __restrict__ residual,
-                                                              uint16_t* __restrict__ out,
-                                                              const int32_t* __restrict__ hist_ids, int hist_experts,
-                                                              int64_t* __restrict__ hist_out,
-                                                              const int64_t* __restrict__ load_counts,
-                                                              int64_t* __restrict__ load)
+__global__ __launch_bounds__(256) void token_unpermute_kernel(UnpermuteArgs a)
 {
-    __shared__ int32_t srow[64];
-    __shared__ float sw[64];
-    const int top_k = TOPK > 0 ? TOPK : top_k_rt;
-    if ((hist_out || load) && blockIdx.x == gridDim.x - 1) {
+    const uint16_t* __restrict__ permuted = a.permuted;
+    const int32_t* __restrict__ idx = a.idx;
+    const uint16_t* __restrict__ probs = a.probs;
+    const uint16_t* __restrict__ residual = a.residual;
+    uint16_t* __restrict__ out = a.out;
+    const int32_t* __restrict__ hist_ids = a.hist_ids;
+    const int64_t H = a.H, permuted_rows = a.permuted_rows;
+    const int hist_experts = a.hist_experts;
+    if ((int)blockIdx.x == a.T) {
+        int64_t* hist_out = a.hist_out;
+        int64_t* load = a.load;
         __shared__ int32_t hcnt[kHistMaxExperts];
         if (blockIdx.y != 0) return;
         if (!hist_ids) {
-            for (int e = threadIdx.x; e < hist_experts; e += 256) load[e] += load_counts[e];
+            for (int e = threadIdx.x; e < hist_experts; e += 256) load[e] += a.load_counts[e];
             return;
         }
         for (int e = threadIdx.x; e < hist_experts; e += 256) hcnt[e] = 0;
@@ -51,41 +63,87 @@ __global__ __launch_bounds__(256) void token_unpermute_kernel(const uint16_t* __
         return;
     }
     const int64_t t = blockIdx.x;
-    if (threadIdx.x < top_k) {
-        int32_t d = idx ? idx[t * top_k + threadIdx.x] : (int32_t)(t * top_k + threadIdx.x);
-        d = d < 0 ? -d : d;
-        if (!idx && hist_ids) {  // pair order: a pair whose expert id is out of range was computed by nobody
-            const int32_t e = hist_ids[t * top_k + threadIdx.x];
-            if (e < 0 || e >= hist_experts) d = 0x7fffffff;
-        }
-        srow[threadIdx.x] = ((int64_t)d < permuted_rows) ? d : -1;
-        sw[threadIdx.x] = probs ? half_to_f32<DT>(probs[t * top_k + threadIdx.x]) : 1.0f;
-    }
-    __syncthreads();
     const int64_t nv = H >> 3;
-    // few tokens: a row is cut into gridDim.y pieces, one workgroup each
-    for (int64_t i = (int64_t)blockIdx.y * 256 + threadIdx.x; i < nv; i += 256 * (int64_t)gridDim.y) {
-        float acc[8];
+    // few tokens: a row is cut into pieces, one workgroup each
+    const int64_t first = (int64_t)blockIdx.y * 256 + threadIdx.x, step = 256 * (int64_t)a.pieces;
+    auto load_residual = [&](int64_t i) {
+        return residual ? ((const v8u16*)(residual + t * H))[i] : (v8u16){0, 0, 0, 0, 0, 0, 0, 0};
+    };
+    auto finish = [&](int64_t i, float (&acc)[8], v8u16 r) {
+        if (residual) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
-        if constexpr (TOPK > 0) {
+            for (int j = 0; j < 8; ++j) acc[j] = acc[j] + half_to_f32<DT>(r[j]);
+        }
+        v8u16 o;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o[j] = f32_to_half<DT>(acc[j]);
+        ((v8u16*)(out + t * H))[i] = o;
+    };
+    if constexpr (TOPK > 0) {
+        // Rows, weights and ids of the slots are the same for the whole workgroup: every wavefront reads them into lanes, one load
+        // each, in front of the rows.  In pair order the rows' addresses wait for nothing (a row that nobody computed is read
+        // and left out).  With a barrier and LDS between the two, 64 tokens of 2 x 1024 values took 2.9 us and take 1.7 (the small
+        // layer 26.3 -> 24.9 us a call); of 8 x 2048 values 109.9 -> 109.4 us a call.
+        const int lane = threadIdx.x & 63;
+        const int64_t mine = t * TOPK + (lane < TOPK ? lane : TOPK - 1);
+        int32_t d = idx ? idx[mine] : (int32_t)mine;
+        int32_t e = !idx && hist_ids ? hist_ids[mine] : -1;
+        uint32_t p16 = probs ? probs[mine] : 0u;
+        int32_t row[TOPK];
+        if (idx) {
+            d = d < 0 ? -d : d;
+            const int32_t r = (int64_t)d < permuted_rows ? d : 0;
+#pragma unroll
+            for (int s = 0; s < TOPK; ++s) row[s] = __builtin_amdgcn_readlane(r, s);
+        } else {
+#pragma unroll
+            for (int s = 0; s < TOPK; ++s) row[s] = t * TOPK + s < permuted_rows ? (int32_t)(t * TOPK + s) : 0;
+        }
+        for (int64_t i = first; i < nv; i += step) {
             v8u16 v[TOPK];
+            if (permuted_rows > 0) {
 #pragma unroll
-            for (int s = 0; s < TOPK; ++s) {
-                const int32_t d = srow[s];
-                v[s] = (d >= 0) ? __builtin_nontemporal_load((const v8u16*)(permuted + (int64_t)d * H) + i) : (v8u16){0, 0, 0, 0, 0, 0, 0, 0};
+                for (int s = 0; s < TOPK; ++s) v[s] = __builtin_nontemporal_load((const v8u16*)(permuted + (int64_t)row[s] * H) + i);
             }
+            const v8u16 r = load_residual(i);
+            asm volatile("" : "+v"(d), "+v"(e), "+v"(p16));  // used from here on: what is made of them stays behind the rows' loads
+            // pair order: a pair whose expert id is out of range was computed by nobody
+            const unsigned long long use = __ballot((int64_t)d < permuted_rows && (idx || !hist_ids || (e >= 0 && e < hist_experts)));
+            const float w_lane = probs ? half_to_f32<DT>((uint16_t)p16) : 1.0f;
+            float acc[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
 #pragma unroll
             for (int s = 0; s < TOPK; ++s) {
-                if (srow[s] < 0) continue;
-                const float w = sw[s];
+                if (!((use >> s) & 1)) continue;
+                const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w_lane), s));
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     float pr = w * half_to_f32<DT>(v[s][j]);
                     acc[j] = acc[j] + pr;
                 }
             }
-        } else {
+            finish(i, acc, r);
+        }
+    } else {
+        __shared__ int32_t srow[64];
+        __shared__ float sw[64];
+        const int top_k = a.top_k;
+        if (threadIdx.x < top_k) {
+            int32_t d = idx ? idx[t * top_k + threadIdx.x] : (int32_t)(t * top_k + threadIdx.x);
+            d = d < 0 ? -d : d;
+            if (!idx && hist_ids) {
+                const int32_t e = hist_ids[t * top_k + threadIdx.x];
+                if (e < 0 || e >= hist_experts) d = 0x7fffffff;
+            }
+            srow[threadIdx.x] = ((int64_t)d < permuted_rows) ? d : -1;
+            sw[threadIdx.x] = probs ? half_to_f32<DT>(probs[t * top_k + threadIdx.x]) : 1.0f;
+        }
+        __syncthreads();
+        for (int64_t i = first; i < nv; i += step) {
+            float acc[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
             for (int s = 0; s < top_k; ++s) {
                 const int32_t d = srow[s];
                 if (d < 0) continue;
@@ -97,16 +155,8 @@ __global__ __launch_bounds__(256) void token_unpermute_kernel(const uint16_t* __
                     acc[j] = acc[j] + pr;
                 }
             }
+            finish(i, acc, load_residual(i));
         }
-        if (residual) {
-            const v8u16 r = ((const v8u16*)(residual + t * H))[i];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) acc[j] = acc[j] + half_to_f32<DT>(r[j]);
-        }
-        v8u16 o;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) o[j] = f32_to_half<DT>(acc[j]);
-        ((v8u16*)(out + t * H))[i] = o;
     }
 }
 
@@ -134,11 +184,11 @@ int moe355::unpermute_impl(const void* permuted, int dtype, const int32_t* sorte
         pieces = (unsigned)(per_row < want ? per_row : want);
         if (pieces < 1) pieces = 1;
     }
-#define MOE355_UNPERMUTE(K, D)                                                                                    \
-    hipLaunchKernelGGL((token_unpermute_kernel<K, D>), dim3((unsigned)num_tokens + (hist_out || load ? 1u : 0u), pieces), dim3(256), 0, (hipStream_t)stream, \
-                       (const uint16_t*)permuted, sorted_indices, (const uint16_t*)probs, top_k, hidden,             \
-                       permuted_rows, (const uint16_t*)residual, (uint16_t*)out, hist_ids, hist_experts, hist_out,  \
-                       load_counts, load)
+    const UnpermuteArgs a = {(int)num_tokens, top_k, (int)pieces, hist_experts, (const uint16_t*)permuted, sorted_indices,
+                             (const uint16_t*)probs, (const uint16_t*)residual, (uint16_t*)out, hist_ids, hidden, permuted_rows,
+                             hist_out, load_counts, load};
+    const dim3 grid((unsigned)num_tokens + (hist_out || load ? 1u : 0u), pieces);
+#define MOE355_UNPERMUTE(K, D) hipLaunchKernelGGL((token_unpermute_kernel<K, D>), grid, dim3(256), 0, (hipStream_t)stream, a)
     if (dtype == MOE355_DT_F16) {
         // fp16 models: the common fan-outs unrolled, the rest through the generic loop
         if (top_k == 8) MOE355_UNPERMUTE(8, MOE355_DT_F16);
