@@ -339,3 +339,34 @@ def test_rows_of_weight_streaming_tiles(avg, E, N, family):
                                                (384, 96, 5120, 4096, "wide")])
 def test_several_weight_streaming_tiles_of_an_expert(avg, E, Kd, N, family):
     test_tokens_of_a_tile_in_lds(avg, E, Kd, N, family, torch.bfloat16)
+
+
+# Tall tiles of the weight-streaming family (193 to 256 rows), whose two halves of columns are entries of their own as long as
+# the list has room: all of them, some of them; an even and an odd number of column blocks (the second half of the last column
+# does not exist); beside tiles of every other height
+@pytest.mark.parametrize("Kd,N", [(4096, 192), (4096, 448)])
+@pytest.mark.parametrize("counts", [[193] * 8, [256, 193, 255, 194, 200, 220, 193, 256], [512, 0, 3, 509, 40, 0], [700, 192, 161, 129, 1, 0, 64, 33]],
+                         ids=["no room", "some room", "room", "all heights"])
+def test_halves_of_tall_tiles(counts, Kd, N):
+    from oracle import oracle as orc
+    from vllm_ascend_amd import kernels as K
+    from vllm_ascend_amd._lib import W_ENK, load
+
+    E, R = len(counts), sum(counts)
+    print(f"tall tiles {counts} K={Kd} N={N}", flush=True)
+    assert load().moe355_gmm_kernel_name(2, R, Kd, N, E).decode() == "gmm_wide_kernel"
+    g = torch.Generator().manual_seed(R + N)
+    cum = torch.cumsum(torch.tensor(counts, dtype=torch.int64), 0)
+    x = torch.randint(-128, 128, (R, Kd), generator=g, dtype=torch.int8)
+    w = torch.randint(-128, 128, (E, N, Kd), generator=g, dtype=torch.int8)
+    sw = torch.rand(E, N, generator=g) * 0.009 + 0.001
+    sx = torch.rand(R, generator=g) * 0.05 + 0.001
+    wnz = K.format_cast_nz(w.to("cuda"), W_ENK)
+    ref = orc.gmm_i32(x.numpy(), w.numpy(), cum.numpy())
+    got = K.gmm2_dequant(x.to("cuda"), wnz, sw.to("cuda"), sx.to("cuda"), cum.to("cuda"), 0, N, Kd)
+    q, s = K.gmm1_swiglu_quant(x.to("cuda"), wnz, sw.to("cuda"), sx.to("cuda"), cum.to("cuda"), 0, N, Kd)
+    torch.cuda.synchronize()
+    assert np.array_equal(got.cpu().contiguous().view(torch.int16).numpy().view(np.uint16), orc.gmm2_dequant(ref, sx.numpy(), sw.numpy(), cum.numpy()))
+    q_want, s_want = orc.swiglu_quant(orc.dequant_acc(ref, sx.numpy(), sw.numpy(), cum.numpy()))
+    assert np.array_equal(q.cpu().numpy(), q_want)
+    assert np.array_equal(s.cpu().numpy().view(np.uint32), s_want.view(np.uint32))

@@ -770,7 +770,7 @@ __global__ __launch_bounds__(512, 1) void gmm_wide_kernel(GmmArgs a, TileMap tm,
     const int64_t row0 = tm.row_begin[mt];
     int64_t row_end = tm.row_end[mt];
     if (mt >= count) return;
-    const int e = listed & ~kOnlyTile;
+    const int e = listed & ~(kOnlyTile | kFirstHalf | kSecondHalf);
     const bool once = listed & kOnlyTile;
     if (row_end > a.R) row_end = a.R;
     if (row0 >= row_end) return;
@@ -787,9 +787,11 @@ __global__ __launch_bounds__(512, 1) void gmm_wide_kernel(GmmArgs a, TileMap tm,
     } else if (row_end - row0 <= 192) {
         stream_tile_body<EPI, true, 6>(a, e, row0, row_end, col, once, wide_lds);
     } else {
-        // a tall tile is one column block wide: the column's two blocks one after the other
-        stream_tile_body<EPI, false>(a, e, row0, row_end, 2 * col, once, wide_lds);
-        if (2 * col + 1 < n_col_blocks) {
+        // a tall tile is one column block wide: the column's two blocks have an entry each, or are done one after the other
+        const bool second = listed & kSecondHalf;
+        if (second && 2 * col + 1 >= n_col_blocks) return;
+        stream_tile_body<EPI, false>(a, e, row0, row_end, second ? 2 * col + 1 : 2 * col, once, wide_lds);
+        if (!(listed & (kFirstHalf | kSecondHalf)) && 2 * col + 1 < n_col_blocks) {
             __syncthreads();  // the first block's epilogue is out of LDS
             stream_tile_body<EPI, false>(a, e, row0, row_end, 2 * col + 1, once, wide_lds);
         }

@@ -8,11 +8,13 @@ namespace moe355 {
 
 // in the list by length and where it is asked for: the tile is its expert's only one
 constexpr int32_t kOnlyTile = 1 << 30;
+// in the list by length: an entry of one half of a tall tile's columns (neither: both of them)
+constexpr int32_t kFirstHalf = 1 << 29, kSecondHalf = 1 << 28;
 
 // (expert, row block) tiles of one launch
 struct TileMap {
     int32_t* count;      // [1]
-    int32_t* expert;     // [max_tiles] (and kOnlyTile)
+    int32_t* expert;     // [max_tiles] (and kOnlyTile, kFirstHalf, kSecondHalf)
     int32_t* row_begin;  // [max_tiles]
     int32_t* row_end;    // [max_tiles] end of the expert's rows
 };
@@ -20,9 +22,16 @@ struct TileMap {
 struct TileSpec {
     TileMap tm;
     int BM, max_tiles;
-    // the 256-row weight-streaming tiles: the tiles are listed longest first -- 161..192 rows, 129..160, up to 128,
-    // then the tall ones (more than 192 rows, which become two shorter column items) -- so that the workgroups that
-    // start last are the short ones and the compute units finish closer together
+    // the 256-row weight-streaming tiles, listed longest first -- 161..192 rows, 129..160, up to 128 -- so that the workgroups
+    // that start last are the short ones and the compute units finish closer together, and the tall ones (more than 192 rows)
+    // spread evenly among them: the tall tiles of a hot expert find their weights in the caches and wait for the matrix units,
+    // the cold experts' tiles for their weights from HBM, and so both are busy all the time.  In eights, because entry t
+    // runs on XCD t % 8.  A tall tile has an entry for either half of its columns as long as the list has room for that (a
+    // workgroup per entry and column is launched for as many tiles as the rows can make), beyond it one for both.
+    // Layers under Zipf(1.1), 256 experts of 7168 / 2048, 2048 / 3000 / 4096 tokens: tall ones whole and last 1662 / 2165 / 2520 us,
+    // halves last 1631 / 2108 / 2510, halves first 1617 / 2075 / 2443, spread 1567 / 1998 / 2254; 128 experts of 2048 / 768, 1900
+    // tokens 223 whole and last, 214 spread.  4096 tokens of uniform routing, a few of whose experts are tall because of the
+    // router's bias, gate_up alone 1295 whole and last, 1325 halves first, the same spread.
     int by_length;
     int flag_only;  // kOnlyTile also in a list in the order of the experts
 };
@@ -66,16 +75,48 @@ __device__ __forceinline__ void build_tile_map(RowsOf rows_of, int E, const Tile
         const int32_t b23 = block_scan_exclusive_i32(n23, part_b, all23);
         const int32_t total[4] = {all01 & 0xffff, all01 >> 16, all23 & 0xffff, all23 >> 16};
         const int32_t all_tiles = total[0] + total[1] + total[2] + total[3];
-        if (tid == 0) tm.count[0] = all_tiles < max_tiles ? all_tiles : max_tiles;
-        int32_t next[4] = {b01 & 0xffff, total[0] + (b01 >> 16), total[0] + total[1] + (b23 & 0xffff),
-                           total[0] + total[1] + total[2] + (b23 >> 16)};
+        const int32_t room = max_tiles > all_tiles ? max_tiles - all_tiles : 0;
+        const int32_t whole = total[3] > room ? total[3] - room : 0;  // tall tiles with one entry, the first ones
+        const int32_t tall = 2 * total[3] - whole;
+        if (tid == 0) tm.count[0] = all_tiles < max_tiles ? all_tiles - total[3] + tall : max_tiles;
+        // eight entries, one for every XCD, are a block; the blocks of tall entries lie at ((2 b + 1) n / 2 a) of the a of them among
+        // n blocks, and what fills no block at the end
+        const int64_t a8 = tall >> 3, n8 = a8 + ((all_tiles - total[3]) >> 3);
+        auto tall_at = [&](int32_t i) {
+            return (i >> 3) < a8 ? (int32_t)((2 * (i >> 3) + 1) * n8 / (2 * a8)) * 8 + (i & 7) : all_tiles - total[3] + i;
+        };
+        auto other_at = [&](int32_t i) {
+            int64_t at = i >> 3, before = 0;
+            if (at >= n8 - a8) return (int32_t)(a8 * 8 + i);
+            for (int64_t next = -1; next != before;) {  // the tall blocks in front of it: those at `at` or before
+                next = before;
+                const int64_t reach = 2 * (at + before + 1) * a8 - n8;
+                before = reach <= 0 ? 0 : (reach + 2 * n8 - 1) / (2 * n8);
+                if (before > a8) before = a8;
+            }
+            return (int32_t)(at + before) * 8 + (i & 7);
+        };
+        int32_t next[3] = {b01 & 0xffff, total[0] + (b01 >> 16), total[0] + total[1] + (b23 & 0xffff)};
+        int32_t next_tall = b23 >> 16;
         int64_t row = rows_before;
         for (int j = 0; j < seg; ++j) {
             const int e = e0 + j;
             if (e < E) {
                 const int64_t m = rows_of(e);
-                for (int64_t r0 = 0; r0 < m; r0 += BM)
-                    put(next[cls(m - r0)]++, m <= BM ? e | kOnlyTile : e, row + r0, row + m);
+                for (int64_t r0 = 0; r0 < m; r0 += BM) {
+                    const int c = cls(m - r0), listed = m <= BM ? e | kOnlyTile : e;
+                    if (c < 3) {
+                        put(other_at(next[c]++), listed, row + r0, row + m);
+                        continue;
+                    }
+                    const int32_t i = next_tall++;
+                    if (i < whole) {
+                        put(tall_at(i), listed, row + r0, row + m);
+                    } else {
+                        put(tall_at(2 * i - whole), listed | kFirstHalf, row + r0, row + m);
+                        put(tall_at(2 * i - whole + 1), listed | kSecondHalf, row + r0, row + m);
+                    }
+                }
                 row += m;
             }
         }
