@@ -341,6 +341,15 @@ def test_several_weight_streaming_tiles_of_an_expert(avg, E, Kd, N, family):
     test_tokens_of_a_tile_in_lds(avg, E, Kd, N, family, torch.bfloat16)
 
 
+# and where they begin when there are columns for several rounds of the chip
+@pytest.mark.parametrize("avg,E,Kd,N,family", [(39, 512, 4096, 576, "tiled"), (40, 512, 4096, 576, "wide"), (40, 511, 4096, 576, "tiled"),
+                                               (11, 1024, 7168, 576, "tiled"), (12, 1024, 7168, 576, "wide"),
+                                               (71, 128, 2048, 7168, "tiled"), (72, 128, 2048, 7168, "wide"),
+                                               (39, 179, 3072, 5184, "tiled"), (40, 179, 3072, 5184, "wide")])
+def test_few_rows_on_weight_streaming_tiles(avg, E, Kd, N, family):
+    test_tokens_of_a_tile_in_lds(avg, E, Kd, N, family, torch.bfloat16)
+
+
 # Tall tiles of the weight-streaming family (193 to 256 rows), whose two halves of columns are entries of their own as long as
 # the list has room: all of them, some of them; an even and an odd number of column blocks (the second half of the last column
 # does not exist); beside tiles of every other height

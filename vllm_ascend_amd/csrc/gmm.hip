@@ -668,7 +668,19 @@ static int tiled_bm(const GmmArgs& a)
     // 215 / 272 against 196 / 262 / 276.  (One expert: a dense product on a side stream, which should leave the chip idle.)
     const bool narrow = a.N <= 512;
     const int64_t columns = (int64_t)a.E * ((a.N + 511) / 512);
-    if (avg >= 64 && avg <= 256 && a.K >= 4096 && wide_ok && (narrow || a.E == 1 || columns >= kComputeUnits / 2)) return 256;
+    // Since their tall tiles are spread among the others they win earlier under Zipf(1.1) too where there are columns for four
+    // rounds of the chip and more.  One product, wide / 128-row tiles, uniform (Zipf(1.1)), at 24 / 40 / 60 rows: 1024 columns, 128
+    // experts of 7168 / 4096 0.98 / 0.95 / 0.94 (1.01 / 0.94 / 0.92); 1280 and 1536 columns of them 0.98 / 0.96 / 0.91 (0.99 to 1.01 /
+    // 0.92 to 0.95 / 0.94 to 0.96); 256 of 5120 / 4096 0.96 / 0.94 / 0.90 (1.00 / 0.92 / 0.92), of 4096 / 4096 0.99 / 0.98 / 0.97
+    // (1.03 / 0.98 / 0.96), of 7168 / 3072 0.97 / 0.96 / 0.90 (1.02 / 0.93 / 0.91); 160 of 6144 / 6144 0.99 / 0.97 / 0.92 (0.99 /
+    // 0.95 / 0.92): from 40 rows on.  Below 1024 columns uniform routing wins and Zipf does not: 512 and 256 columns of 7168 / 4096
+    // at 48 rows 0.98 and 0.99 (1.03 and 1.18), 768 of 128 experts of 4096 / 3072 0.94 (1.03).  From 2048 columns on and K = 7168
+    // earlier still: 256 experts of 7168 / 4096 at 8 / 16 / 32 / 48 rows 0.99 / 0.98 / 0.96 / 0.93 (0.98 / 0.99 / 0.94 / 0.94), 128 of
+    // 7168 / 8192 at 8 / 12 / 24 0.99 / 0.99 / 0.98 (1.02 / 0.99 / 0.98); in the layer, whose router leaves more experts idle, 9 /
+    // 12 / 16 / 22 / 31 rows 0.99 / 0.98 / 0.98 / 0.96 / 0.96 (0.99 / 0.95 / 0.89 / 0.93 / 0.91): 512 tokens under Zipf(1.1) 599 ->
+    // 536 us.
+    const int64_t from = columns < 4 * kComputeUnits || narrow ? 64 : columns >= 8 * kComputeUnits && a.K >= 7168 ? 12 : 40;
+    if (avg >= from && avg <= 256 && a.K >= 4096 && wide_ok && (narrow || a.E == 1 || columns >= kComputeUnits / 2)) return 256;
     // Above 256 rows an expert has two tall tiles and more, and they fetch its weights half as often as the 128-row tiles.  That
     // is what counts where an expert's weights are several times the 4 MiB of an XCD's L2.  One product, wide / 128-row tiles:
     //   32 MiB and more per expert at K >= 4096: 16 experts of 14336 x 4096, 264 / 352 / 512 / 1024 rows 0.79 / 0.78 / 0.69 /
@@ -720,7 +732,14 @@ static int tiled_bm(const GmmArgs& a)
     const bool fills = narrow || columns >= kComputeUnits;
     const bool beyond = a.K >= 2048 && a.N >= 5120 && own >= (14 << 20) && 2 * columns >= 7 * kComputeUnits;
     const int64_t most = narrow ? 192 : beyond ? 256 : 144;
-    if (avg >= (narrow ? 96 : 112) && avg <= most && a.K >= 1024 && wide_ok && fills) return 256;
+    // With columns for seven rounds such products are on the wide tiles earlier, since the tall ones are spread among the others:
+    // at 40 / 64 / 80 / 100 rows 256 experts of K = 3072, N = 5120 0.96 / 0.90 / 0.88 / 0.86 (Zipf 0.97 / 0.95 / 0.95 / 0.94); of K =
+    // 2048, N = 7168 1.00 / 1.02 / 0.95 / 0.94 (0.99 / 0.97 / 0.96 / 0.94), in the layer at 62 / 72 rows 0.99 / 0.97 (0.90 / 0.87);
+    // 192 of them 1.00 / 1.01 / 1.01 / 0.97 (1.02 / 0.99 / 0.97 / 0.95), 128 1.00 / 0.99 / 0.98 / 0.96 (1.03 / 0.97 / 0.95 / 0.96);
+    // 256 and 160 of K = 2048, N = 8192 1.01 and 1.02 / 1.01 and 1.00 / 1.01 and 1.00 / 0.97 and 0.96 (0.96 and 1.02 / 0.94 and 0.97 /
+    // 0.94 and 0.92 / 0.91 and 0.90).
+    const int64_t least = narrow ? 96 : beyond && columns >= 7 * kComputeUnits ? (a.K >= 3072 ? 40 : 72) : 112;
+    if (avg >= least && avg <= most && a.K >= 1024 && wide_ok && fills) return 256;
     return 128;
 }
 
