@@ -210,7 +210,7 @@ def test_shared_expert_instead_of_the_re_quantisation(tokens, overlap):
     assert layer._layer_plan.desc is not None
 
 
-# int4 weights in pair order (up to 40 tokens): blocks of 16 and 32 rows, further blocks, one scale per channel or per group, hot and idle experts
+# int4 weights in pair order (up to 32 tokens): blocks of 16 and 32 rows, one scale per channel or per group, hot and idle experts
 @pytest.mark.parametrize("tokens", [1, 16, 17, 32, 33, 40, 41])
 @pytest.mark.parametrize("name", ["c5_small", "c5_small_perchannel"])
 def test_int4_pair_order(name, tokens):
@@ -219,6 +219,26 @@ def test_int4_pair_order(name, tokens):
     hot[::9] = logits[::9]
     for lg in (logits, hot):
         assert torch.equal(layer(x, lg), layer.forward_impl(x, lg).routed_out)
+
+
+# the same: fewer K blocks than the ring holds, no multiple of it, channels that leave wavefronts of a workgroup idle; an
+# expert named more than once by a token (more rows than tokens: further passes over its weights)
+@pytest.mark.parametrize("H,I,tokens", [(64, 64, 1), (192, 64, 16), (448, 320, 17), (832, 448, 32)])
+def test_int4_pair_order_edges(H, I, tokens):
+    cfg, layer, x, logits = _pair("c5_small_perchannel", tokens, dict(H=H, I=I))
+    assert torch.equal(layer(x, logits), layer.forward_impl(x, logits).routed_out)
+    select = layer.router.select_experts
+
+    def repeated(*a, **kw):
+        weights, ids = select(*a, **kw)
+        ids = ids.clone()
+        ids[:, 1:3] = 3
+        return weights, ids
+
+    layer.router.select_experts = repeated
+    weights, ids = repeated(x, logits)
+    want = layer.quant_method.apply(layer, x, weights, ids, None, None).routed_out
+    assert torch.equal(layer(x, logits), want)
 
 
 def test_the_call_follows_the_layer():

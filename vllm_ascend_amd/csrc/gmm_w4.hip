@@ -513,23 +513,25 @@ __global__ __launch_bounds__(256, LDS_SCALES ? 4 : 3) void gmm_w4_stream_kernel(
 }
 
 // ------------------------------------------------------------------ decode batches, pair order
-// The same product for at most kW4PairMax (token, slot) pairs whose ids come straight from the gate: an expert has one to
-// a few rows, so nothing is sorted (a row belongs to its pair throughout, as in gmm_stream_kernel's pair order), nothing
-// is staged and no wavefront waits for another one inside the K loop.  One wavefront per pair of 32-channel tiles over
-// the whole K range (the fp32 sum over the scale groups has one fixed order); tokens are the 16 columns of
-// v_mfma_i32_16x16x64_i8 (one or two times, for experts of more than 16 rows), so accumulators and fp32 sums are 16
-// registers each instead of 64 and the fold is a quarter of the work.  HBM-bound: DeepSeek-V3 shape, us a layer call
-// against the sorted chunks, uniform routing, 1 / 4 / 16 / 32 tokens 59 / 136 / 382 / 557 against 86 / 157 / 412 / 593
-// (16 tokens: 2.3 GB at 6.4 TB/s), Zipf(1.1), 24 / 32 tokens 148 / 178 against 163 / 203.  A ring of
-// 8, 10 or 12 blocks 389 to 393 us at 16 tokens, three wavefronts per SIMD the same as two and 191 us at 32 under Zipf.
+// The same product for at most 32 tokens (see w4_pairs_supported) whose ids come straight from the gate: an expert has
+// one to a few rows, so nothing is sorted (a row belongs to its pair throughout, as in gmm_stream_kernel's pair order),
+// nothing is staged and no wavefront waits for another one inside the K loop.  One wavefront per 32 channels (SwiGLU: 16 of the gate
+// and the 16 of the up projection that belong to them) over the whole K range (the fp32 sum over the scale groups has one
+// fixed order); tokens are the 16 columns of v_mfma_i32_16x16x64_i8, one or two times.  HBM-bound.
+// DeepSeek-V3 shape, us a layer call with 64 channels per wavefront, two wavefronts per SIMD / with 32, four: uniform
+// routing, 1 / 4 / 8 / 16 / 24 tokens 57 / 136 / 230 / 385 / 501 against 50 / 127 / 217 / 362 / 468 (16 tokens: 2.2 GB at
+// 6.1 TB/s); Zipf(1.1), 16 / 20 / 24 tokens 148 / 171 / 178 against 137 / 155 / 169.  A ring of 3 (six wavefronts), 4 (five),
+// 5, 6, 7, 8, 10 or 14 (two) blocks, 1 and 16 tokens: 56 and 366, 53 and 362, 50 and 359, 50 and 360, 50 and 367, 51 and
+// 367, 50 and 371, 54 and 391.  More than 16 rows under Zipf(1.1), 24 / 32 tokens: two blocks at a time 169 / 194, one
+// after the other 183 / 213, the second block in workgroups of its own 185 / 207.
 // An int4 tile (lane = channel l % 32, K half l / 32; low nibbles K 0..31, high nibbles K 32..63) becomes the operands of
 // its two groups of 16 channels by one exchange: rows of 16 lanes 1 and 3 of the low-nibble register against rows 0 and 2
 // of the high-nibble register (v_permlane16_swap) leave channels 0..15 in one register and 16..31 in the other, row r of
 // either holding the K slice 0, 32, 16 or 48 + 0..15 for r = 0, 1, 2, 3.  The tokens are read in that order.
 constexpr int kW4PairMax = 1024;
-constexpr int kW4PairTokens = 40;  // see w4_pairs_supported
 constexpr int kW4PairExperts = 2048;
-constexpr int kW4PairRing = 6;     // K blocks of weights and tokens in flight per wavefront
+constexpr int kW4PairRing = 6;     // K blocks of weights and tokens in flight per wavefront,
+constexpr int kW4PairRing2 = 4;    // with two blocks of 16 rows: what 128 registers hold
 
 __device__ __forceinline__ void w4_operands(v4i v, v4i& first, v4i& second)
 {
@@ -542,24 +544,11 @@ __device__ __forceinline__ void w4_operands(v4i v, v4i& first, v4i& second)
     }
 }
 
-template <int EPI>
-__global__ __launch_bounds__(256, 2) void gmm_w4_pairs_kernel(W4Args p)
+// The expert of a slot (the slot-th one that has pairs) and, in plist, its pairs in ascending order; every thread of the
+// workgroup calls it and gets the same answer, -1 where there are fewer such experts.  See gmm_stream_kernel.
+__device__ __forceinline__ int w4_slot_pairs(const GmmArgs& a, int slot, int wave, int lane, uint32_t* pmap,
+                                             int32_t* pcount, uint16_t* plist, int& rows)
 {
-    const GmmArgs& a = p.g;
-    __shared__ uint16_t plist[kW4PairMax];       // the expert's pairs, ascending
-    __shared__ int32_t pcount[4];
-    __shared__ uint32_t pmap[kW4PairExperts / 32];  // one bit per expert that has pairs
-    __shared__ float Ss[4][kW4LdsGroups * 64];      // group scales of every wavefront's 64 channels
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    const int NB = a.N >> 5, KB64 = a.K >> 6;
-    const int upe = NB >> 1, quads = (upe + 3) >> 2;
-    const int slot = (int)(blockIdx.x / quads) - a.pair_extra;
-    const int pi_raw = (int)(blockIdx.x % quads) * 4 + wave;
-    const bool have = pi_raw < upe;
-    const int pi = have ? pi_raw : 0;
-
-    // the slot's expert: the slot-th one that has pairs (see gmm_stream_kernel)
     const int Q = (((int)a.R + 255) >> 8) << 6;
     int pid[4];
 #pragma unroll
@@ -578,161 +567,140 @@ __global__ __launch_bounds__(256, 2) void gmm_w4_pairs_kernel(W4Args p)
     const int incl = wave_scan_inclusive_i32(cnt);
     const bool has = slot >= incl - cnt && slot < incl;
     const unsigned long long holder = __ballot(has);
-    int e, first = 0;
-    if (holder != 0ull) {  // the same answer in all four wavefronts
-        uint32_t t = bits;
-        for (int i = has ? slot - (incl - cnt) : 0; i > 0; --i) t &= t - 1;
-        e = __builtin_amdgcn_readlane(lane * 32 + (t ? __builtin_ctz(t) : 0), __builtin_ctzll(holder));
-    } else {
-        // the slots in front (and those past the last expert with pairs, which leave): the experts of more than 32 rows, for
-        // the rows from 32 on.  In the same workgroup one after the other they held up the launch: 40 tokens 212 / 252 /
-        // 262 us -> 216 / 214 / 262, slots behind all others instead 222 / 217 / 271.  The pairs are counted where the scales
-        // will lie.
-        if (slot >= 0) return;
-        const int j = slot + a.pair_extra;
-        int* count = (int*)&Ss[0][0];
-        for (int i = threadIdx.x; i < kW4PairExperts; i += 256) count[i] = 0;
-        __syncthreads();
+    if (holder == 0ull) return -1;
+    uint32_t t = bits;
+    for (int i = has ? slot - (incl - cnt) : 0; i > 0; --i) t &= t - 1;
+    const int e = __builtin_amdgcn_readlane(lane * 32 + (t ? __builtin_ctz(t) : 0), __builtin_ctzll(holder));
+    const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    bool mine[4];
+    int n = 0;
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (pid[c] >= 0 && pid[c] < a.E) atomicAdd(&count[pid[c]], 1);
-        __syncthreads();
-        int hot = -1, seen = 0;  // the j-th of them, experts lane, lane + 64, ... in rounds of 64
-        for (int i = 0; i < (a.E + 63) >> 6 && hot < 0; ++i) {
-            unsigned long long m = __ballot(i * 64 + lane < a.E && count[i * 64 + lane] > 32);
-            const int n = __popcll(m);
-            if (j < seen + n) {
-                for (int q = j - seen; q > 0; --q) m &= m - 1;
-                hot = i * 64 + __builtin_ctzll(m);
-            }
-            seen += n;
-        }
-        if (hot < 0) return;
-        __syncthreads();
-        e = hot;
-        first = 32;
+    for (int c = 0; c < 4; ++c) {
+        mine[c] = pid[c] == e;
+        n += __popcll(__ballot(mine[c]));
     }
+    if (lane == 0) pcount[wave] = n;
+    __syncthreads();
+    int base = 0;
+    rows = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        if (w < wave) base += pcount[w];
+        rows += pcount[w];
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const unsigned long long m = __ballot(mine[c]);
+        if (mine[c]) plist[base + __popcll(m & below)] = (uint16_t)(wave * Q + c * 64 + lane);
+        base += __popcll(m);
+    }
+    __syncthreads();
+    return e;
+}
 
-    const int nb0 = (EPI == EPI_SWIGLU) ? pi : 2 * pi;
-    const int nb1 = (EPI == EPI_SWIGLU) ? pi + upe : 2 * pi + 1;
-    const uint8_t* we = p.w4 + (int64_t)e * NB * KB64 * 1024;
-    const uint8_t* w0 = we + (int64_t)nb0 * KB64 * 1024 + lane * 16;
-    const uint8_t* w1 = we + (int64_t)nb1 * KB64 * 1024 + lane * 16;
+// Workgroup = (slot, four groups of 32 channels).
+template <int EPI>
+__global__ __launch_bounds__(256, 4) void gmm_w4_pairs_kernel(W4Args p)
+{
+    const GmmArgs& a = p.g;
+    __shared__ uint16_t plist[kW4PairMax];       // the expert's pairs, ascending
+    __shared__ int32_t pcount[4];
+    __shared__ uint32_t pmap[kW4PairExperts / 32];  // one bit per expert that has pairs
+    __shared__ float Ss[4][kW4LdsGroups * 32];      // group scales of every wavefront's channels
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63;
+    const int NB = a.N >> 5, KB64 = a.K >> 6;
+    const int quads = (NB + 3) >> 2;
+    const int u_raw = (int)(blockIdx.x % quads) * 4 + wave;
+    const bool have = u_raw < NB;
+    const int u = have ? u_raw : 0;
+    int rows;
+    const int e = w4_slot_pairs(a, (int)(blockIdx.x / quads), wave, lane, pmap, pcount, plist, rows);
+    if (e < 0 || !have) return;  // no barrier behind this one
+
+    const int c32 = lane & 31, hi = lane >> 5;
+    const int tile = EPI == EPI_SWIGLU ? (u >> 1) + (c32 >= 16 ? NB >> 1 : 0) : u;
+    const int chunk16 = EPI == EPI_SWIGLU ? hi * 32 + (u & 1) * 16 + (c32 & 15) : lane;
+    const uint8_t* wp = p.w4 + (((int64_t)e * NB + tile) * KB64) * 1024 + chunk16 * 16;
     const int n_groups = a.K / p.group, steps_per_group = p.group >> 6;
-    {
-        const float* gs = p.gscale + (int64_t)e * n_groups * a.N;
-        const int ch = lane < 32 ? nb0 * 32 + lane : nb1 * 32 + (lane - 32);
-        for (int g0 = 0; g0 < n_groups; g0 += 8) {  // eight loads in flight at a time
-            float v[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = gs[(int64_t)(g0 + j < n_groups ? g0 + j : n_groups - 1) * a.N + ch];
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (g0 + j < n_groups) Ss[wave][(g0 + j) * 64 + lane] = v[j];
-        }
-    }
-    // the expert's pairs
-    int rows = 0;
-    {
-        const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-        bool mine[4];
-        int n = 0;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            mine[c] = pid[c] == e;
-            n += __popcll(__ballot(mine[c]));
-        }
-        if (lane == 0) pcount[wave] = n;
-        __syncthreads();
-        int base = 0;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            if (w < wave) base += pcount[w];
-            rows += pcount[w];
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const unsigned long long m = __ballot(mine[c]);
-            if (mine[c]) plist[base + __popcll(m & below)] = (uint16_t)(wave * Q + c * 64 + lane);
-            base += __popcll(m);
-        }
-        __syncthreads();  // the last barrier
-    }
-    if (!have) return;
-
     const int tok = lane & 15, r16 = lane >> 4;
     const int slice = 16 * ((r16 >> 1) + 2 * (r16 & 1));  // K 0, 32, 16, 48 for rows 0..3
-    constexpr int D = kW4PairRing;
-    // one pass over the weights for NT blocks of 16 rows
-    auto pass = [&](auto blocks, int first) {
-        constexpr int NT = decltype(blocks)::value;
-        v4i a0[D], a1[D], tk[D][NT];
+    // one pass over the weights for NT blocks of 16 rows, D blocks of K in flight
+    auto pass = [&](auto blocks, auto depth, int first) {
+        constexpr int NT = decltype(blocks)::value, D = decltype(depth)::value;
+        v4i w[D], x[D][NT];
         bool valid[NT];
         int row[NT];  // where the row's result goes
-        uint32_t xo[NT];
+        const int8_t* xp[NT];
         float rs[NT];
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
             valid[n] = first + 16 * n + tok < rows;
             row[n] = plist[valid[n] ? first + 16 * n + tok : 0];
             const int src = a.pair_gather ? row[n] / a.pair_k : row[n];
-            xo[n] = (uint32_t)src * (uint32_t)a.K + slice;
+            xp[n] = a.x + (int64_t)src * a.K + slice;
             rs[n] = a.row_scale[src];
         }
         auto request = [&](int s, int kb) {
             const int k = kb < KB64 ? kb : KB64 - 1;  // past the end: a valid block that is never used
-            a0[s] = gload16_nt(w0 + (int64_t)k * 1024);
-            a1[s] = gload16_nt(w1 + (int64_t)k * 1024);
+            w[s] = gload16_nt(wp + (int64_t)k * 1024);
 #pragma unroll
-            for (int n = 0; n < NT; ++n)
-                tk[s][n] = valid[n] ? *(const v4i*)(a.x + (xo[n] + k * 64)) : (v4i){0, 0, 0, 0};
+            for (int n = 0; n < NT; ++n) x[s][n] = *(const v4i*)(xp[n] + k * 64);
         };
-        v4i c[NT][2][2];  // [token block][tile][16 channels]
-        float f[NT][2][2][4];
+#pragma unroll
+        for (int i = 0; i < D; ++i) request(i, i);
+        if (first == 0) {
+            const float* gs = p.gscale + (int64_t)e * n_groups * a.N +
+                              (EPI == EPI_SWIGLU ? (c32 >= 16 ? a.N >> 1 : 0) + u * 16 + (c32 & 15) : u * 32 + c32);
+            for (int g0 = 0; g0 < n_groups; g0 += 16) {  // eight loads in flight at a time
+                float v[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int g = g0 + 2 * j + hi;
+                    v[j] = gs[(int64_t)(g < n_groups ? g : n_groups - 1) * a.N];
+                }
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (g0 + 2 * j + hi < n_groups) Ss[wave][(g0 + 2 * j + hi) * 32 + c32] = v[j];
+            }
+            wave_lds_order();
+        }
+        v4i c[NT][2];  // 16 channels each
+        float f[NT][2][4];
 #pragma unroll
         for (int n = 0; n < NT; ++n)
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int h = 0; h < 2; ++h) {
+                c[n][h] = (v4i){0, 0, 0, 0};
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    c[n][i][h] = (v4i){0, 0, 0, 0};
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) f[n][i][h][j] = 0.0f;
-                }
+                for (int j = 0; j < 4; ++j) f[n][h][j] = 0.0f;
+            }
         int in_group = 0, grp = 0;
         auto step = [&](int s, int kb) {  // s = kb % D, compile time
-            v4i l0, h0, l1, h1;
-            w4_operands(a0[s], l0, h0);
-            w4_operands(a1[s], l1, h1);
+            v4i lo, up;
+            w4_operands(w[s], lo, up);
 #pragma unroll
             for (int n = 0; n < NT; ++n) {
-                c[n][0][0] = mfma_i8_16(l0, tk[s][n], c[n][0][0]);
-                c[n][0][1] = mfma_i8_16(h0, tk[s][n], c[n][0][1]);
-                c[n][1][0] = mfma_i8_16(l1, tk[s][n], c[n][1][0]);
-                c[n][1][1] = mfma_i8_16(h1, tk[s][n], c[n][1][1]);
+                c[n][0] = mfma_i8_16(lo, x[s][n], c[n][0]);
+                c[n][1] = mfma_i8_16(up, x[s][n], c[n][1]);
             }
             request(s, kb + D);
             if (++in_group == steps_per_group) {  // f += float(acc / 16) * scale[e, grp, channel]
-                const float* sl = &Ss[wave][grp * 64 + 4 * r16];
+                const float* sl = &Ss[wave][grp * 32 + 4 * r16];
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
+                for (int h = 0; h < 2; ++h) {
+                    const v4f sc = *(const v4f*)(sl + 16 * h);
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        const v4f sc = *(const v4f*)(sl + 32 * i + 16 * h);
+                    for (int n = 0; n < NT; ++n) {
 #pragma unroll
-                        for (int n = 0; n < NT; ++n) {
-#pragma unroll
-                            for (int j = 0; j < 4; ++j)
-                                f[n][i][h][j] = f[n][i][h][j] + (float)(c[n][i][h][j] >> 4) * sc[j];
-                            c[n][i][h] = (v4i){0, 0, 0, 0};
-                        }
+                        for (int j = 0; j < 4; ++j) f[n][h][j] = f[n][h][j] + (float)(c[n][h][j] >> 4) * sc[j];
+                        c[n][h] = (v4i){0, 0, 0, 0};
                     }
+                }
                 in_group = 0;
                 ++grp;
             }
         };
-#pragma unroll
-        for (int i = 0; i < D; ++i) request(i, i);
         const int kb_full = (KB64 / D) * D;
         for (int kb = 0; kb < kb_full; kb += D) {
 #pragma unroll
@@ -741,20 +709,16 @@ __global__ __launch_bounds__(256, 2) void gmm_w4_pairs_kernel(W4Args p)
 #pragma unroll
         for (int i = 0; i < D - 1; ++i)
             if (kb_full + i < KB64) step(i, kb_full + i);
+        const int c0 = EPI == EPI_SWIGLU ? u * 16 + 4 * r16 : u * 32 + 4 * r16;
 #pragma unroll
         for (int n = 0; n < NT; ++n)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int ch = 16 * h + 4 * r16;
-                epilogue_run_w4<EPI>(a, row[n], valid[n], nb0 * 32 + ch, nb1 * 32 + ch, f[n][0][h], f[n][1][h], rs[n]);
-            }
+            epilogue_run_w4<EPI>(a, row[n], valid[n], c0, EPI == EPI_SWIGLU ? c0 + (a.N >> 1) : c0 + 16, f[n][0], f[n][1],
+                                 rs[n]);
     };
-    if (first == 0 && a.pair_extra > 0 && rows > 32) rows = 32;  // another workgroup has the others
-    if (rows - first <= 16) {
-        pass(std::integral_constant<int, 1>{}, first);
-    } else {
-        for (; first < rows; first += 32) pass(std::integral_constant<int, 2>{}, first);
-    }
+    int first = 0;
+    for (; rows - first > 16; first += 32)
+        pass(std::integral_constant<int, 2>{}, std::integral_constant<int, kW4PairRing2>{}, first);
+    if (first < rows) pass(std::integral_constant<int, 1>{}, std::integral_constant<int, kW4PairRing>{}, first);
 }
 
 // workgroups: an upper bound of the number of 64-row chunks (known on the host without reading the group
@@ -901,14 +865,19 @@ extern "C" int moe355_gmm1_swiglu_quant_w4_gather(const int8_t* x, const float* 
                         n, num_experts, swiglu_limit, out, out_scale, workspace, workspace_bytes, stream, row_token, nullptr);
 }
 
-// Up to 40 tokens.  Uniform routing would gain beyond (47 tokens 750 -> 710 us, 64 844 -> 795 us), but skewed routing loses by
-// the second reading of its hot experts' weights: Zipf(1.1), three draws, 40 tokens 216 / 214 / 262 us against 220 / 232 /
-// 271 sorted, 47 tokens 232 / 251 / 274 against 235 / 237 / 274, 128 tokens 479 against 327; the host cannot know.
+// Up to 24 tokens; 32, two blocks of 16 rows, with experts under 16 MiB, where the launches of a sorted layer cost as much
+// as a few more bytes.  Beyond, a skewed batch waits for its hot experts; the host cannot know.  Pair order / sorted, us a
+// call.  DeepSeek-V3 shape (22 MB), 20 / 24 / 32 / 48 tokens: uniform routing 423 / 468 / 548 / 685 against 442 / 493 / 571
+// / 709, Zipf(0.8) 205 / 219 / 244 / 308 against 216 / 231 / 248 / 291, Zipf(1.1) 155 / 169 / 194 / 241 against 162 / 172 /
+// 190 / 207, Zipf(1.4) 127 / 140 / 159 / 225 against 134 / 141 / 148 / 171.  128 experts of 2.4 MB, 28 / 32 / 40 tokens:
+// uniform 63 / 65 / 68 against 70 / 72 / 77, Zipf(1.1) 41 / 43 / 54 against 43 / 44 / 49; of 9.4 MB 173 / 182 / 193
+// against 183 / 195 / 205, 91 / 100 / 118 against 93 / 98 / 104.
 bool moe355::w4_pairs_supported(int64_t num_tokens, int top_k, int num_experts, int64_t hidden, int64_t intermediate,
                                 int64_t group13, int64_t group2)
 {
-    return num_tokens > 0 && num_tokens <= kW4PairTokens && num_tokens * top_k <= kW4PairMax && num_experts <= kW4PairExperts && group13 > 0 && group2 > 0 &&
-           hidden / group13 <= kW4LdsGroups && intermediate / group2 <= kW4LdsGroups;
+    const int64_t most = hidden * intermediate * 3 / 2 < (16 << 20) ? 32 : 24;
+    return num_tokens > 0 && num_tokens <= most && num_tokens * top_k <= kW4PairMax && num_experts <= kW4PairExperts &&
+           group13 > 0 && group2 > 0 && hidden / group13 <= kW4LdsGroups && intermediate / group2 <= kW4LdsGroups;
 }
 
 // one GEMM in pair order: the gate_up one (y set: fp32 SwiGLU values, rows re-quantised into out) or the down one
@@ -927,14 +896,19 @@ static W4Args w4_pair_args(const int8_t* x, const float* x_scale, const int32_t*
     p.w4 = w;
     p.gscale = scale;
     p.group = (int)group;
-    p.g.pair_extra = num_tokens > 32 ? (int)(p.g.R / 33) : 0;  // a row of an expert per token
     return p;
 }
 
-static dim3 w4_pair_grid(const W4Args& p)
+template <int EPI>
+static void launch_w4_pairs(const W4Args& p, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1)
 {
     const int64_t slots = p.g.R < (int64_t)p.g.E ? p.g.R : (int64_t)p.g.E;
-    return dim3((unsigned)((slots + p.g.pair_extra) * ((p.g.N / 64 + 3) / 4)));
+    auto kernel = gmm_w4_pairs_kernel<EPI>;
+    const dim3 grid((unsigned)(slots * ((p.g.N / 32 + 3) / 4)));
+    if (ev0 || ev1)
+        hipExtLaunchKernelGGL(kernel, grid, dim3(256), 0, st, ev0, ev1, 0, p);
+    else
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, p);
 }
 
 int moe355::gmm1_w4_pairs(const int8_t* x, const float* x_scale, const int32_t* topk_ids, int64_t num_tokens, int top_k,
@@ -950,10 +924,7 @@ int moe355::gmm1_w4_pairs(const int8_t* x, const float* x_scale, const int32_t* 
     p.g.y = y;
     hipEvent_t ev0, ev1;
     take_profile_events(ev0, ev1);
-    if (ev0)
-        hipExtLaunchKernelGGL((gmm_w4_pairs_kernel<EPI_SWIGLU>), w4_pair_grid(p), dim3(256), 0, st, ev0, ev1, 0, p);
-    else
-        hipLaunchKernelGGL((gmm_w4_pairs_kernel<EPI_SWIGLU>), w4_pair_grid(p), dim3(256), 0, st, p);
+    launch_w4_pairs<EPI_SWIGLU>(p, st, ev0, ev1);
     launch_swiglu_requant(y, nullptr, 0, num_experts, p.g.R, (int)(n / 2), out, out_scale, st);
     return launch_status();
 }
@@ -968,7 +939,7 @@ int moe355::gmm2_w4_pairs(const int8_t* x, const float* x_scale, const int32_t* 
     W4Args p = w4_pair_args(x, x_scale, topk_ids, num_tokens, top_k, w, scale, group, k, n, num_experts);
     p.g.out = (uint16_t*)out;
     p.g.out_f16 = out_dtype == MOE355_DT_F16;
-    hipLaunchKernelGGL((gmm_w4_pairs_kernel<EPI_DEQUANT>), w4_pair_grid(p), dim3(256), 0, st, p);
+    launch_w4_pairs<EPI_DEQUANT>(p, st, nullptr, nullptr);
     return launch_status();
 }
 
