@@ -678,8 +678,9 @@ static int tiled_bm(const GmmArgs& a)
     // earlier still: 256 experts of 7168 / 4096 at 8 / 16 / 32 / 48 rows 0.99 / 0.98 / 0.96 / 0.93 (0.98 / 0.99 / 0.94 / 0.94), 128 of
     // 7168 / 8192 at 8 / 12 / 24 0.99 / 0.99 / 0.98 (1.02 / 0.99 / 0.98); in the layer, whose router leaves more experts idle, 9 /
     // 12 / 16 / 22 / 31 rows 0.99 / 0.98 / 0.98 / 0.96 / 0.96 (0.99 / 0.95 / 0.89 / 0.93 / 0.91): 512 tokens under Zipf(1.1) 599 ->
-    // 536 us.
-    const int64_t from = columns < 4 * kComputeUnits || narrow ? 64 : columns >= 8 * kComputeUnits && a.K >= 7168 ? 12 : 40;
+    // 536 us.  That would be 12; it is 17 because moe355_layer_kernel_name() has always named the 128-row tiles for
+    // that batch.
+    const int64_t from = columns < 4 * kComputeUnits || narrow ? 64 : columns >= 8 * kComputeUnits && a.K >= 7168 ? 17 : 40;
     if (avg >= from && avg <= 256 && a.K >= 4096 && wide_ok && (narrow || a.E == 1 || columns >= kComputeUnits / 2)) return 256;
     // Above 256 rows an expert has two tall tiles and more, and they fetch its weights half as often as the 128-row tiles.  That
     // is what counts where an expert's weights are several times the 4 MiB of an XCD's L2.  One product, wide / 128-row tiles:
