@@ -267,6 +267,34 @@ def test_gate_quant_equals_gating_plus_dynamic_quant(K, orc, case):
     assert torch.equal(xq, xq_want) and torch.equal(xs.view(torch.int32), xs_want.view(torch.int32))
 
 
+# the choice of the experts by counting: below and from where it starts, more candidates than lanes, experts that fill no
+# whole register, groups, and scores that tie in part, nearly all or all of them; NaN and infinities among them
+@pytest.mark.parametrize("k,E,G,k_group", [(5, 128, 1, 1), (6, 128, 1, 1), (8, 128, 1, 1), (8, 256, 8, 4), (8, 256, 1, 1), (8, 8, 1, 1),
+                                           (8, 60, 1, 1), (8, 65, 1, 1), (6, 200, 4, 2), (6, 96, 3, 2), (16, 256, 1, 1), (17, 256, 1, 1),
+                                           (32, 128, 1, 1), (33, 128, 1, 1), (64, 64, 1, 1), (64, 130, 1, 1)])
+@pytest.mark.parametrize("levels", [0, 40, 3, 1])
+def test_experts_chosen_by_counting(K, k, E, G, k_group, levels):
+    g = torch.Generator().manual_seed(k * E + levels)
+    T = 70
+    logits = torch.randn(T, E, generator=g) if levels == 0 else torch.randint(0, levels, (T, E), generator=g).float() / 8
+    for i in range(3):  # few large scores that share their lanes
+        logits[i, i::64] += 9.0
+    x = torch.randn(T, 64, generator=g).to(torch.bfloat16).to(DEV)
+    rows = [logits]
+    if levels == 0:
+        odd = logits.clone()
+        odd[::3, ::7], odd[1::3, 5], odd[2::3, -1] = -float("inf"), float("inf"), float("nan")
+        rows.append(odd)
+    for lg in rows:
+        for norm_type in (0, 1):
+            tw, ids, _, _ = K.gate_quant(x, lg.to(DEV), k, k_group, G, 1, 1, norm_type, 1.0, 1e-20, None)
+            _, want, _, y_alt = K.gating_top_k(lg.to(DEV), k, k_group, G, 1, 1, norm_type, False, 1.0, 1e-20, None,
+                                               alt_dtype=torch.bfloat16)
+            torch.cuda.synchronize()
+            assert torch.equal(ids, want)
+            assert torch.equal(tw.view(torch.int16), y_alt.view(torch.int16))
+
+
 @pytest.mark.parametrize("R,E,Kd,N,T", [(512, 128, 2048, 1536, 64), (40, 4, 64, 128, 40), (300, 16, 768, 256, 75),
                                         (512, 256, 1024, 4096, 64), (100, 8, 64, 4160, 25),
                                         # many rows per expert: the LDS-tiled kernel (128- and 64-row tiles) and the

@@ -48,6 +48,9 @@ struct SmallRouteArgs {
     int wave_rows;        // the quantising workgroups take four rows each, one per wavefront
 };
 
+// LDS of a gating wavefront (gate_row_wave)
+__host__ __device__ constexpr int gate_row_floats(int E) { return E <= 192 ? 192 : (E + 3) & ~3; }
+
 // the quantiser of the layer on one row, by the whole workgroup
 template <int DT>
 __device__ __forceinline__ void quantise_token_row(const SmallRouteArgs& a, int t, float* lds16)
@@ -121,7 +124,7 @@ __device__ __forceinline__ void quantise_token_row_wave(const SmallRouteArgs& a,
 template <int LDT, int PER, int XDT>
 __global__ __launch_bounds__(kSmallThreads) void route_quant_small_kernel(SmallRouteArgs a)
 {
-    extern __shared__ float lds[];
+    extern __shared__ __attribute__((aligned(16))) float lds[];
     const int gate_wgs = (a.T + kSmallWaves - 1) / kSmallWaves;
     if ((int)blockIdx.x >= gate_wgs) {
         const int wg = (int)blockIdx.x - gate_wgs;
@@ -139,7 +142,7 @@ __global__ __launch_bounds__(kSmallThreads) void route_quant_small_kernel(SmallR
             gate_row_wave<LDT, PER>(RowLogits<LDT>{a.logits, (int64_t)row * E, (int64_t)a.T * E, a.n_planes, a.plane_bias},
                                     a.bias, E, k,
                                     a.k_group, a.G, a.mode, a.renorm, a.norm_type, a.rsf, a.eps, (int64_t)row * k,
-                                    a.topk_weights, a.x_dtype, a.topk_ids, lds + (size_t)wave * E, lane);
+                                    a.topk_weights, a.x_dtype, a.topk_ids, lds + wave * gate_row_floats(E), lane);
     }
     if (!a.arrived) return;  // gating and quantisation only (moe355_gate_quant): the maps come from another launch
     // This workgroup's ids have reached memory before it is counted: every thread waits for its own stores, the
@@ -303,9 +306,9 @@ int moe355::gate_quant_impl(bool sort, const GateCall& g, int tokens_num_type, v
     const int E = num_experts;
     int per = 1;
     while (64 * per < E) per *= 2;
-    // LDS: the sorting tables; the gating rows need E floats per wavefront and the quantiser 4 floats (less)
+    // LDS: the sorting tables; the gating rows need gate_row_floats(E) per wavefront and the quantiser 4 floats (less)
     const size_t lds_bytes = sort ? ((size_t)kSmallMaxPairs + (size_t)kSmallChunks * E + E + 16) * 4
-                                  : ((size_t)kSmallWaves * E + 16) * 4;
+                                  : ((size_t)kSmallWaves * gate_row_floats(E) + 16) * 4;
     const int64_t quads = (num_tokens + kSmallWaves - 1) / kSmallWaves;
     // A workgroup per row has 16 bytes per thread in flight and a barrier in the middle; at 8192 tokens the launch takes 25.0 us
     // against 19.8 with a row per wavefront (H = 2048; H = 1024 14.7 against 10.9), at 2048 9.3 against 8.3, the same at 512
