@@ -110,10 +110,10 @@ __device__ __forceinline__ float group_score(const float* s, int gs, int mode)
 // group_score (a tie is two equal values either way; the order of a +0 and a -0 does not change their sum), the
 // same sum; a row that holds a NaN takes group_score instead, whose treatment of it depends on the position.
 // Lane g (< G) returns the score of group g, the other lanes anything.
-// The exchanges are register permutations (a step of lane reads through LDS is a chain of some 150 cycles): behind the steps
-// of 1 and 2 the lanes of a quad agree, so a mirrored half row or row names a lane of the partner as well as lane ^ 4 or ^ 8.  With the divisions of
-// row_scores by shifts, the routing launch of 256 experts in 8 groups and rows of 7168 values, 1 / 64 / 512 / 4096 tokens 4.93 / 5.96 /
-// 6.42 / 19.95 -> 4.76 / 5.35 / 5.85 / 18.93 us.
+// The exchanges are register permutations (a step of lane reads through LDS is a chain of some 150 cycles): behind the
+// steps of 1 and 2 the lanes of a quad agree, so a mirrored half row or row names a lane of the partner as well as lane
+// ^ 4 or ^ 8.  With the divisions of row_scores by shifts, the routing launch of 256 experts in 8 groups and rows of
+// 7168 values, 1 / 64 / 512 / 4096 tokens 4.93 / 5.96 / 6.42 / 19.95 -> 4.76 / 5.35 / 5.85 / 18.93 us.
 template <int PER>
 __device__ __forceinline__ float group_scores_butterfly(const float (&sel)[PER], int gs, int mode, int lane)
 {
@@ -386,7 +386,8 @@ __device__ __forceinline__ void row_scores(const RowLogits<DT>& logits, const vo
         else sel[i] = -__builtin_inff();
     }
     if (G > 1) {
-        const bool powers = (G & (G - 1)) == 0 && (E & (E - 1)) == 0;  // a division by a number of the call is some 150 cycles
+        // a division by a number of the call is some 150 cycles
+        const bool powers = (G & (G - 1)) == 0 && (E & (E - 1)) == 0;
         const int gs = powers ? E >> __builtin_ctz(G) : E / G;
 #pragma unroll
         for (int i = 0; i < PER; ++i)

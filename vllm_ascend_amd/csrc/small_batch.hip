@@ -48,9 +48,9 @@ struct SmallRouteArgs {
     int wave_rows;        // the quantising workgroups take four rows each, one per wavefront
 };
 
-// 16-byte pieces of a row that a thread of its workgroup requests at once and holds: rows of up to 8192 values are read once.  The
-// launch of rows of 7168 values, 256 experts without groups, 1 / 64 / 512 / 4096 tokens, us with one piece held and the others read
-// twice / so: 3.78 / 4.15 / 5.20 / 20.24 against 3.29 / 3.92 / 4.43 / 17.24.
+// 16-byte pieces of a row that a thread of its workgroup requests at once and holds: rows of up to 8192 values are read
+// once.  The launch of rows of 7168 values, 256 experts without groups, 1 / 64 / 512 / 4096 tokens, us with one piece
+// held and the others read twice / so: 3.78 / 4.15 / 5.20 / 20.24 against 3.29 / 3.92 / 4.43 / 17.24.
 constexpr int kHeld = 4;
 
 // LDS of a gating wavefront (gate_row_wave)
