@@ -31,7 +31,7 @@ struct TileSpec {
     // Layers under Zipf(1.1), 256 experts of 7168 / 2048, 2048 / 3000 / 4096 tokens: tall ones whole and last 1662 / 2165 / 2520 us,
     // halves last 1631 / 2108 / 2510, halves first 1617 / 2075 / 2443, spread 1567 / 1998 / 2254; 128 experts of 2048 / 768, 1900
     // tokens 223 whole and last, 214 spread.  4096 tokens of uniform routing, a few of whose experts are tall because of the
-    // router's bias, gate_up alone 1295 whole and last, 1325 halves first, the same spread.
+    // router's bias, gate_up alone 1295 whole and last, 1325 halves first.
     int by_length;
     int flag_only;  // kOnlyTile also in a list in the order of the experts
 };
@@ -79,12 +79,16 @@ __device__ __forceinline__ void build_tile_map(RowsOf rows_of, int E, const Tile
         const int32_t total[4] = {all01 & 0xffff, all01 >> 16, all23 & 0xffff, all23 >> 16};
         const int32_t all_tiles = total[0] + total[1] + total[2] + total[3];
         const int32_t room = max_tiles > all_tiles ? max_tiles - all_tiles : 0;
-        const int32_t whole = total[3] > room ? total[3] - room : 0;  // tall tiles with one entry, the first ones
+        // Fewer than one tall tile in 16 has no phase of its own to mix, and halves only read their tokens twice: whole and last.
+        // 4096 tokens of uniform routing, gate_up / down 1344 / 792 us spread, 1318 / 778 so; under Zipf(0.6), where one in 8 to 16
+        // is tall, the layer at 2048 tokens 2175 spread, 2261 so.
+        const bool few = 16 * total[3] < all_tiles;
+        const int32_t whole = few ? total[3] : total[3] > room ? total[3] - room : 0;  // tall tiles with one entry, the first ones
         const int32_t tall = 2 * total[3] - whole;
         if (tid == 0) tm.count[0] = all_tiles < max_tiles ? all_tiles - total[3] + tall : max_tiles;
         // eight entries, one for every XCD, are a block; the blocks of tall entries lie at ((2 b + 1) n / 2 a) of the a of them among
         // n blocks, and what fills no block at the end
-        const int32_t a8 = tall >> 3, n8 = a8 + ((all_tiles - total[3]) >> 3);  // at most 8192 and 12288
+        const int32_t a8 = few ? 0 : tall >> 3, n8 = a8 + ((all_tiles - total[3]) >> 3);  // at most 8192 and 12288
         // x / d where the quotient is at most 12288: by the reciprocal it is off by one at most.  One lane walks the tiles
         // of a hot expert, and 64-bit divisions for each of them made the launch of 4096 tokens under Zipf(1.1) 30 us
         // instead of 16.
