@@ -539,6 +539,37 @@ def test_token_unpermute(K, orc, T, k, H, residual):
     assert np.array_equal(bits(out), ref)
 
 
+# Rows that end inside a wavefront: fewer 8-value pieces than slots in the last one, as many, more (every slot still counts), and
+# a whole row shorter than the slots; sorted rows and rows in pair order, dropped pairs among them
+@pytest.mark.parametrize("dtype,k", [("bf16", 1), ("bf16", 2), ("bf16", 4), ("bf16", 6), ("bf16", 8), ("bf16", 3), ("f16", 2), ("f16", 8), ("f16", 4)])
+@pytest.mark.parametrize("H", [8, 32, 56, 64, 72, 520, 2056, 2080, 6152])
+def test_combine_of_rows_that_end_inside_a_wavefront(K, orc, dtype, k, H):
+    T, E = 5, 16
+    print(f"combine {dtype} k={k} H={H}", flush=True)
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    g = torch.Generator().manual_seed(k * 10000 + H)
+    R = T * k
+    o, p, res = (torch.randn(s, generator=g).to(dt) for s in ((R, H), (T, k), (T, H)))
+    idx = torch.randperm(R, generator=g).to(torch.int32)
+    idx[1] = R  # no such row: left out
+    idx[R - 1] = -idx[R - 1]  # by its magnitude
+    ids = torch.randint(0, E, (T, k), generator=g, dtype=torch.int32)
+    ids[0, k - 1], ids[2, 0] = E, -1
+    here = ((ids >= 0) & (ids < E)).view(-1)
+    pair = torch.where(here, torch.arange(R), R).to(torch.int32)
+    for r in (None, res):
+        rd = None if r is None else r.to(DEV)
+        got = K.token_unpermute(o.to(DEV), idx.to(DEV), p.to(DEV), rd)
+        got_pairs, cnt = K.token_unpermute_pairs(o.to(DEV), p.to(DEV), ids.to(DEV), E, rd)
+        torch.cuda.synchronize()
+        with orc.half_kind(dtype):
+            want = orc.unpermute(bits(o), idx.numpy(), bits(p), None if r is None else bits(r))
+            want_pairs = orc.unpermute(bits(o), pair.numpy(), bits(p), None if r is None else bits(r))
+        assert np.array_equal(bits(got.cpu()), want)
+        assert np.array_equal(bits(got_pairs.cpu()), want_pairs)
+        assert np.array_equal(cnt.cpu().numpy(), np.bincount(ids.view(-1)[here].numpy(), minlength=E))
+
+
 # n / 2 up to 1024 and up to 4096 are held in registers between the passes, longer rows are computed twice
 @pytest.mark.parametrize("rows,n", [(2, 192), (4, 192), (8, 384), (1, 256), (300, 2048), (3, 4096), (2, 8448)])
 @pytest.mark.parametrize("left", [True, False])

@@ -99,7 +99,9 @@ __global__ __launch_bounds__(256) void token_unpermute_kernel(UnpermuteArgs a)
 #pragma unroll
             for (int s = 0; s < TOPK; ++s) row[s] = t * TOPK + s < permuted_rows ? (int32_t)(t * TOPK + s) : 0;
         }
-        for (int64_t i = first; i < nv; i += step) {
+        // Whole wavefronts go round: lane s holds slot s, also where the row ends in front of that lane.
+        for (int64_t at = first; at - lane < nv; at += step) {
+            const int64_t i = at < nv ? at : nv - 1;
             v8u16 v[TOPK];
             if (permuted_rows > 0) {
 #pragma unroll
@@ -123,7 +125,7 @@ __global__ __launch_bounds__(256) void token_unpermute_kernel(UnpermuteArgs a)
                     acc[j] = acc[j] + pr;
                 }
             }
-            finish(i, acc, r);
+            if (at < nv) finish(i, acc, r);
         }
     } else {
         __shared__ int32_t srow[64];
