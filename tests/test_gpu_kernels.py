@@ -570,6 +570,22 @@ def test_combine_of_rows_that_end_inside_a_wavefront(K, orc, dtype, k, H):
         assert np.array_equal(cnt.cpu().numpy(), np.bincount(ids.view(-1)[here].numpy(), minlength=E))
 
 
+# indices at the ends of their type: no such row, in the forms with a compiled-in number of slots and in the general one
+@pytest.mark.parametrize("dtype,k", [("bf16", 1), ("bf16", 2), ("bf16", 4), ("bf16", 6), ("bf16", 8), ("bf16", 3), ("f16", 2), ("f16", 8), ("f16", 3)])
+def test_combine_leaves_out_the_ends_of_the_index_type(K, orc, dtype, k):
+    T, H = 7, 128
+    print(f"combine, ends of the index type, {dtype} k={k}", flush=True)
+    g = torch.Generator().manual_seed(k)
+    R, lo, hi = T * k, -2 ** 31, 2 ** 31 - 1
+    o, p = (torch.randn(s, generator=g).to(torch.bfloat16 if dtype == "bf16" else torch.float16) for s in ((R, H), (T, k)))
+    idx = torch.randperm(R, generator=g).to(torch.int32)
+    idx[0], idx[R // 2], idx[R - 1], idx[R // 3] = lo, lo, hi, -hi
+    got = K.token_unpermute(o.to(DEV), idx.to(DEV), p.to(DEV))
+    torch.cuda.synchronize()
+    with orc.half_kind(dtype):
+        assert np.array_equal(bits(got.cpu()), orc.unpermute(bits(o), idx.numpy(), bits(p)))
+
+
 # n / 2 up to 1024 and up to 4096 are held in registers between the passes, longer rows are computed twice
 @pytest.mark.parametrize("rows,n", [(2, 192), (4, 192), (8, 384), (1, 256), (300, 2048), (3, 4096), (2, 8448)])
 @pytest.mark.parametrize("left", [True, False])

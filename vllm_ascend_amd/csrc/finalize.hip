@@ -29,6 +29,9 @@ struct UnpermuteArgs {
     int64_t* load;
 };
 
+// |index| as a row; INT32_MIN stays negative (no overflow that the compiler may build on), and a negative row is none
+__device__ __forceinline__ int32_t row_of(int32_t index) { return index < 0 ? (int32_t)(0u - (uint32_t)index) : index; }
+
 template <int TOPK, int DT = MOE355_DT_BF16>
 __global__ __launch_bounds__(256) void token_unpermute_kernel(UnpermuteArgs a)
 {
@@ -91,8 +94,8 @@ __global__ __launch_bounds__(256) void token_unpermute_kernel(UnpermuteArgs a)
         uint32_t p16 = probs ? probs[mine] : 0u;
         int32_t row[TOPK];
         if (idx) {
-            d = d < 0 ? -d : d;
-            const int32_t r = (int64_t)d < permuted_rows ? d : 0;
+            d = row_of(d);
+            const int32_t r = d >= 0 && (int64_t)d < permuted_rows ? d : 0;
 #pragma unroll
             for (int s = 0; s < TOPK; ++s) row[s] = __builtin_amdgcn_readlane(r, s);
         } else {
@@ -110,7 +113,7 @@ __global__ __launch_bounds__(256) void token_unpermute_kernel(UnpermuteArgs a)
             const v8u16 r = load_residual(i);
             asm volatile("" : "+v"(d), "+v"(e), "+v"(p16));  // used from here on: what is made of them stays behind the rows' loads
             // pair order: a pair whose expert id is out of range was computed by nobody
-            const unsigned long long use = __ballot((int64_t)d < permuted_rows && (idx || !hist_ids || (e >= 0 && e < hist_experts)));
+            const unsigned long long use = __ballot(d >= 0 && (int64_t)d < permuted_rows && (idx || !hist_ids || (e >= 0 && e < hist_experts)));
             const float w_lane = probs ? half_to_f32<DT>((uint16_t)p16) : 1.0f;
             float acc[8];
 #pragma unroll
@@ -133,7 +136,7 @@ __global__ __launch_bounds__(256) void token_unpermute_kernel(UnpermuteArgs a)
         const int top_k = a.top_k;
         if (threadIdx.x < top_k) {
             int32_t d = idx ? idx[t * top_k + threadIdx.x] : (int32_t)(t * top_k + threadIdx.x);
-            d = d < 0 ? -d : d;
+            d = row_of(d);
             if (!idx && hist_ids) {
                 const int32_t e = hist_ids[t * top_k + threadIdx.x];
                 if (e < 0 || e >= hist_experts) d = 0x7fffffff;
