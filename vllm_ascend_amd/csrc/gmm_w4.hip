@@ -240,7 +240,9 @@ struct W4Unit {
 };
 
 // NB: blocks of 32 rows.  STREAM: the expert has a single chunk, nobody else reads these weights: non-temporal loads (the
-// faster pure stream).  Otherwise the sibling chunks of the expert run at the same time on the same XCD (their workgroup
+// faster pure stream).  That goes for the number of chunks, not of rows: with the last 32 rows and fewer of a hot expert past
+// the caches too, Zipf(1.1), 128 / 256 / 512 / 1024 tokens took 322 / 413 / 623 / 896 us a layer call and take 314 / 406 / 615 /
+// 884 (512 tokens: 1766 and 802 MB read from HBM by the two products, 1708 and 770 so).  Otherwise the sibling chunks of the expert run at the same time on the same XCD (their workgroup
 // numbers differ by a multiple of 8) and ordinary loads let them share one fetch in L2.
 template <int EPI, bool LDS_SCALES, int NB, bool STREAM, bool FAR>
 __device__ __forceinline__ void w4_chunk_body(const W4Args& p, const W4Unit& t, const __amdgpu_buffer_rsrc_t xr, const int8_t* xb,
@@ -508,7 +510,8 @@ __global__ __launch_bounds__(256, LDS_SCALES ? 4 : 3) void gmm_w4_stream_kernel(
         else w4_chunk_body<EPI, LDS_SCALES, 2, false, false>(p, t, xr, xb, xo);
     } else {
         if (far) w4_chunk_body<EPI, LDS_SCALES, 1, false, true>(p, t, xr, xb, xo);
-        else w4_chunk_body<EPI, LDS_SCALES, 1, true, false>(p, t, xr, xb, xo);
+        else if (single) w4_chunk_body<EPI, LDS_SCALES, 1, true, false>(p, t, xr, xb, xo);
+        else w4_chunk_body<EPI, LDS_SCALES, 1, false, false>(p, t, xr, xb, xo);
     }
 }
 
