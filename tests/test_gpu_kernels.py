@@ -839,6 +839,27 @@ def test_w4_gemms_at_chunk_boundaries(K, orc, Kd, N, group, gl_type):
     assert np.array_equal(bits(got_b.cpu()), orc.w4_rows_to_bf16(fb, sx.numpy()))
 
 
+# The group scales lie in LDS as long as two workgroups fit a compute unit with them (112 groups), beyond only in a launch of
+# few workgroups: the channels of a wide product against the same channels in a narrow one
+@pytest.mark.parametrize("Kd", [7168, 7232, 17408])
+def test_w4_scales_in_lds_or_from_memory(K, Kd):
+    g = torch.Generator(device=DEV).manual_seed(Kd)
+    cnt = [0, 1, 33, 64, 130, 7]
+    E, R, N, part, group = len(cnt), sum(cnt), 9216, 192, 64
+    chunks = R // 64 + E
+    assert chunks * ((N // 32 + 3) // 4) >= 640 > chunks * ((part // 32 + 3) // 4)
+    print(f"w4 scales K={Kd} groups={Kd // group}", flush=True)
+    x = torch.randint(-128, 128, (R, Kd), generator=g, dtype=torch.int8, device=DEV)
+    xs = torch.rand(R, generator=g, device=DEV) * 0.05 + 0.001
+    w = torch.randint(-8, 8, (E, N, Kd), generator=g, dtype=torch.int8, device=DEV)
+    sg = torch.rand(E, Kd // group, N, generator=g, device=DEV) * 0.09 + 0.01
+    gl = torch.tensor(cnt, dtype=torch.int64, device=DEV)
+    want = K.gmm2_dequant_w4(x, K.format_cast_nz_int4(w, 0, N, Kd), sg, group, xs, gl, 1, N, Kd)
+    got = K.gmm2_dequant_w4(x, K.format_cast_nz_int4(w[:, :part].contiguous(), 0, part, Kd), sg[:, :, :part].contiguous(), group, xs, gl, 1, part, Kd)
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), want[:, :part].contiguous().view(torch.int16))
+
+
 def test_w4_rows_more_than_4_gib_apart(K):
     """Gathered token rows beyond what a 32-bit offset reaches: the same values as the rows copied together."""
     g = torch.Generator().manual_seed(5)

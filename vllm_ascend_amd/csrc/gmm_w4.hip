@@ -200,7 +200,8 @@ __device__ __forceinline__ bool find_chunk(const int64_t* gl, int gl_type, int E
 // sum over scale groups has one fixed order).  An expert with many rows becomes many units that run side by side on
 // different CUs and find the expert's weights in L2 / Infinity Cache, instead of one wavefront streaming the same weights
 // once per 32 rows.
-// 32 channels instead of a pair of 32-channel tiles: accumulators and fp32 sums are 64 registers, four wavefronts fit a SIMD.
+// 32 channels instead of a pair of 32-channel tiles: accumulators and fp32 sums are 64 registers, four wavefronts fit a SIMD
+// (with up to 32 scale groups, see w4_scales_in_lds).
 // The vector instructions of the fold and of the unpacking, the MFMAs, the LDS reads and the wait for memory follow each
 // other in a wavefront, so what runs beside them is other wavefronts.  For the gate_up product the 32 channels are 16 of the
 // gate and the 16 of the up projection that belong to them, out of half a storage tile each: they meet in one lane.
@@ -223,9 +224,31 @@ constexpr int kW4StageBytes = 8192;  // LDS bytes of the tokens of one stage
 constexpr int kW4Ring = 3 * kW4StageBytes;
 
 // LDS: the ring of token stages, the group scales of four times 32 channels
-static int w4_lds_bytes(int64_t n_groups) { return kW4Ring + (int)n_groups * 512; }
+static int64_t w4_lds_bytes(int64_t n_groups) { return kW4Ring + n_groups * 512; }
 constexpr int kW4LdsMax = 163840;
-constexpr int kW4ScaleGroups = (kW4LdsMax - kW4Ring) / 512;
+// With the scales in LDS four workgroups fit a compute unit up to 32 groups, three up to 58, two up to 112 and one up to 272;
+// with the scales read from memory in every fold four always do.  Two or more of them win at any size; a single one wins as long
+// as the launch is about two rounds of the chip (`blocks`, an upper bound of the workgroups that have rows, below two and a
+// half).  Layers, us a call with the scales in LDS / from memory, uniform (Zipf(1.1)):
+//   48 groups: 128 experts of 3072 / 1024, 64 / 400 / 1200 tokens 154 / 178 / 335 against 174 / 203 / 383 (89 / 165 / 317 against
+//     103 / 187 / 360); 56: 256 of 7168 / 2048, 50 / 600 / 1024 tokens 758 / 1086 / 1237 against 848 / 1195 / 1365 (512 tokens 674
+//     against 733)
+//   80 groups: 64 of 5120 / 1536, 50 / 200 / 800 tokens 192 / 206 / 416 against 223 / 234 / 449 (123 / 203 / 408 against 146 / 247
+//     / 435); 112: 256 of 7168 / 2048, 50 / 600 / 1024 tokens 1010 / 1385 / 1555 against 1107 / 1484 / 1694 (512 tokens 889
+//     against 951)
+//   128 groups, by blocks: 8 of 8192 / 1024, 224 / 320 / 416 95 / 104 / 175 against 129 / 129 / 160 (99 / 105 / 177 against 131 /
+//     138 / 163); 16 of 2048 / 8192, 352 / 448 / 544 / 656 / 848 153 / 204 / 286 / 300 / 419 against 205 / 243 / 314 / 291 / 370
+//     (202 / 237 / 276 / 334 at 352 / 448 / 544 / 656 against 232 / 279 / 305 / 334); 16 of 8192 / 2048, 576 / 640 / 704 144 / 145 /
+//     155 against 147 / 148 / 167 (150 / 163 / 205 against 175 / 180 / 195); 32 of 8192 / 1024, 544 / 608 143 / 145 against 147 / 149
+//     (136 / 158 against 138 / 174); 18 of 8192 / 2048, 640 195 against 162 (196 against 188); 32 of them, 1184 / 1408 258 / 330
+//     against 213 / 275 (264 / 407 against 227 / 349)
+//   224 groups, 8 of 4096 / 14336, 320 / 512 / 576 / 640 / 704 / 896 235 / 449 / 510 / 525 / 579 / 755 against 306 / 508 / 467 / 510 /
+//     538 / 679 (268 / 440 / 496 / 526 / 635 against 360 / 487 / 536 / 583 / 627, 899 against 808 at 1024); 272 groups, 8 of 2048 /
+//     17408, 224 / 320 / 416 / 528 262 / 342 / 526 / 583 against 373 / 427 / 490 / 553 (276 / 331 / 522 / 573 against 395 / 450 / 533 / 608)
+static bool w4_scales_in_lds(int64_t n_groups, int64_t blocks)
+{
+    return w4_lds_bytes(n_groups) <= (2 * blocks < 5 * 256 ? kW4LdsMax : kW4LdsMax / 2);
+}
 
 #define MOE355_LPTR(p) ((__attribute__((address_space(3))) void*)(p))
 
@@ -738,8 +761,8 @@ template <int EPI>
 static bool launch_w4(const W4Args& p, int64_t blocks, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1)
 {
     const int64_t n_groups = p.g.K / p.group;
-    const bool lds_scales = n_groups <= kW4ScaleGroups;
-    const int lds = lds_scales ? w4_lds_bytes(n_groups) : kW4Ring;
+    const bool lds_scales = w4_scales_in_lds(n_groups, blocks);
+    const int lds = lds_scales ? (int)w4_lds_bytes(n_groups) : kW4Ring;
     auto kernel = lds_scales ? gmm_w4_stream_kernel<EPI, true> : gmm_w4_stream_kernel<EPI, false>;
     static OncePerDevice once;
     if (lds_scales && !allow_dynamic_lds(once, (const void*)gmm_w4_stream_kernel<EPI, true>, kW4LdsMax)) return false;
