@@ -531,7 +531,7 @@ typedef struct moe355_layer {
     int32_t weights;          /* 0: int8 tensors; 1: device tables of per-expert int8 tensors; 2: int4 tensors */
     int32_t pair_order;       /* 0: never; 1: where moe355_pair_order() says so (weights 0 and 1), and up to 256 MiB of
                                * repeated weight reads instead of 128 where a shared expert of a routed expert's shape rides in
-                               * the same launches; int4: up to 40 tokens */
+                               * the same launches; int4: up to 24 tokens, 32 with experts under 16 MiB, 40 under 5 MiB */
     const void *w13, *s13, *w2, *s2;
     int64_t group13, group2;  /* int4: weights along K that share a scale */
     /* of moe355_route_quant_small, for a caller that runs the layer on one stream or graph at a time; NULL: that launch

@@ -210,7 +210,7 @@ def test_shared_expert_instead_of_the_re_quantisation(tokens, overlap):
     assert layer._layer_plan.desc is not None
 
 
-# int4 weights in pair order (up to 32 tokens): blocks of 16 and 32 rows, one scale per channel or per group, hot and idle experts
+# int4 weights in pair order (up to 40 tokens of experts this small): one block of 16 or 32 rows and several, one scale per channel or per group, hot and idle experts
 @pytest.mark.parametrize("tokens", [1, 16, 17, 32, 33, 40, 41])
 @pytest.mark.parametrize("name", ["c5_small", "c5_small_perchannel"])
 def test_int4_pair_order(name, tokens):

@@ -539,7 +539,7 @@ __global__ __launch_bounds__(256, LDS_SCALES ? 4 : 3) void gmm_w4_stream_kernel(
 }
 
 // ------------------------------------------------------------------ decode batches, pair order
-// The same product for at most 32 tokens (see w4_pairs_supported) whose ids come straight from the gate: an expert has
+// The same product for at most 40 tokens (see w4_pairs_supported) whose ids come straight from the gate: an expert has
 // one to a few rows, so nothing is sorted (a row belongs to its pair throughout, as in gmm_stream_kernel's pair order),
 // nothing is staged and no wavefront waits for another one inside the K loop.  One wavefront per 32 channels (SwiGLU: 16 of the gate
 // and the 16 of the up projection that belong to them) over the whole K range (the fp32 sum over the scale groups has one
@@ -892,16 +892,24 @@ extern "C" int moe355_gmm1_swiglu_quant_w4_gather(const int8_t* x, const float* 
 }
 
 // Up to 24 tokens; 32, two blocks of 16 rows, with experts under 16 MiB, where the launches of a sorted layer cost as much
-// as a few more bytes.  Beyond, a skewed batch waits for its hot experts; the host cannot know.  Pair order / sorted, us a
-// call.  DeepSeek-V3 shape (22 MB), 20 / 24 / 32 / 48 tokens: uniform routing 423 / 468 / 548 / 685 against 442 / 493 / 571
-// / 709, Zipf(0.8) 205 / 219 / 244 / 308 against 216 / 231 / 248 / 291, Zipf(1.1) 155 / 169 / 194 / 241 against 162 / 172 /
-// 190 / 207, Zipf(1.4) 127 / 140 / 159 / 225 against 134 / 141 / 148 / 171.  128 experts of 2.4 MB, 28 / 32 / 40 tokens:
-// uniform 63 / 65 / 68 against 70 / 72 / 77, Zipf(1.1) 41 / 43 / 54 against 43 / 44 / 49; of 9.4 MB 173 / 182 / 193
-// against 183 / 195 / 205, 91 / 100 / 118 against 93 / 98 / 104.
+// as a few more bytes; 40 under 5 MiB, where they cost more than a second reading of the experts with more than 32 rows.  Beyond,
+// a skewed batch waits for its hot experts; the host cannot know.  Pair order / sorted, us a call.  DeepSeek-V3 shape (22 MB),
+// 20 / 24 / 32 / 48 tokens: uniform routing 423 / 468 / 548 / 685 against 442 / 493 / 571 / 709, Zipf(0.8) 205 / 219 / 244 / 308
+// against 216 / 231 / 248 / 291, Zipf(1.1) 155 / 169 / 194 / 241 against 162 / 172 / 190 / 207, Zipf(1.4) 127 / 140 / 159 / 225
+// against 134 / 141 / 148 / 171.  28 / 32 tokens: 128 experts of 2.4 MB uniform 63 / 65 against 70 / 72, Zipf(1.1) 41 / 43
+// against 43 / 44; of 9.4 MB 173 / 182 against 183 / 195, 91 / 100 against 93 / 98.  33 / 36 / 40 tokens, uniform (Zipf(1.1)):
+//   0.8 MB (256 of 1024 / 512)   45 / 46 / 47    (30 / 34 / 36) against    53 / 55 / 56    (35 / 37 / 37)
+//   2.2 MB (8 of 1024 / 1408)    25 / 26 / 27    (30 / 31 / 35) against    34 / 33 / 33    (33 / 34 / 36)
+//   2.4 MB (128 of 2048 / 768)   65 / 66 / 66    (46 / 51 / 52) against    73 / 74 / 75    (46 / 48 / 49)
+//   4.3 MB (64 of 2048 / 1408)   62 / 63 / 63    (48 / 59 / 60) against    73 / 73 / 73    (51 / 56 / 56)
+//   4.7 MB (64 of 2048 / 1536)   65 / 66 / 67    (58 / 65 / 68) against    74 / 75 / 75    (57 / 60 / 60)
+//   6.3 MB (128 of 4096 / 1024) 134 / 136 / 138  (80 / 92 / 93) against   144 / 146 / 147  (75 / 78 / 79)
+//   7.9 MB (64 of 5120 / 1024)   96 / 97 / 98    (73 / 92 / 94) against   103 / 105 / 105  (65 / 73 / 75)
 bool moe355::w4_pairs_supported(int64_t num_tokens, int top_k, int num_experts, int64_t hidden, int64_t intermediate,
                                 int64_t group13, int64_t group2)
 {
-    const int64_t most = hidden * intermediate * 3 / 2 < (16 << 20) ? 32 : 24;
+    const int64_t expert = hidden * intermediate * 3 / 2;
+    const int64_t most = expert < (5 << 20) ? 40 : expert < (16 << 20) ? 32 : 24;
     return num_tokens > 0 && num_tokens <= most && num_tokens * top_k <= kW4PairMax && num_experts <= kW4PairExperts &&
            group13 > 0 && group2 > 0 && hidden / group13 <= kW4LdsGroups && intermediate / group2 <= kW4LdsGroups;
 }
