@@ -495,6 +495,21 @@ def test_few_streaming_workgroups_keep_streaming(experts, k, n, first):
         assert name(epilogue, first * experts, k, n, experts) == b"gmm_tiled_kernel"
 
 
+# where the weight-streaming tiles begin, by columns of 512 channels over all experts, and by experts and K from 2048 columns on
+@pytest.mark.parametrize("experts, k, n, first", [(127, 7168, 4096, 64), (128, 7168, 4096, 40), (255, 4096, 4096, 40), (256, 4096, 4096, 28),
+                                                  (256, 5120, 4096, 17), (256, 5056, 4096, 28), (256, 7168, 4096, 17), (512, 4096, 2048, 28),
+                                                  (256, 4032, 4096, None), (192, 7168, 5632, 28), (228, 4096, 4160, 28),
+                                                  (227, 4096, 4160, 40), (128, 8192, 8192, 28), (64, 6144, 16384, 28)])
+def test_where_weight_streaming_tiles_begin(experts, k, n, first):
+    from vllm_ascend_amd import _lib
+
+    name = _lib.load().moe355_gmm_kernel_name
+    for epilogue in (0, 1, 2):
+        for rows in (16, 17, 27, 28, 39, 40, 63, 64):
+            want = "wide" if first and rows >= first else "tiled"
+            assert name(epilogue, rows * experts, k, n, experts).decode() == f"gmm_{want}_kernel", rows
+
+
 # above 256 rows per expert: weight-streaming tiles for weights of 32 MiB an expert, from 384 rows on (512 below 768 columns of
 # tiles) of 14 MiB with at least 5120 channels, of 20 MiB with fewer, from 3072 on, at K from 5120 on with 768 columns
 @pytest.mark.parametrize("experts, k, n, first", [(16, 4096, 8192, 257), (15, 4096, 8192, None), (32, 4096, 8128, 512),

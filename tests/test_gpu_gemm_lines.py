@@ -344,6 +344,8 @@ def test_several_weight_streaming_tiles_of_an_expert(avg, E, Kd, N, family):
 # and where they begin when there are columns for several rounds of the chip
 @pytest.mark.parametrize("avg,E,Kd,N,family", [(39, 512, 4096, 576, "tiled"), (40, 512, 4096, 576, "wide"), (40, 511, 4096, 576, "tiled"),
                                                (16, 1024, 7168, 576, "tiled"), (17, 1024, 7168, 576, "wide"),
+                                               (16, 1024, 5120, 576, "tiled"), (17, 1024, 5120, 576, "wide"),
+                                               (27, 228, 4096, 4160, "tiled"), (28, 228, 4096, 4160, "wide"),
                                                (71, 128, 2048, 7168, "tiled"), (72, 128, 2048, 7168, "wide"),
                                                (39, 179, 3072, 5184, "tiled"), (40, 179, 3072, 5184, "wide")])
 def test_few_rows_on_weight_streaming_tiles(avg, E, Kd, N, family):

@@ -674,13 +674,19 @@ static int tiled_bm(const GmmArgs& a)
     // 0.92 to 0.95 / 0.94 to 0.96); 256 of 5120 / 4096 0.96 / 0.94 / 0.90 (1.00 / 0.92 / 0.92), of 4096 / 4096 0.99 / 0.98 / 0.97
     // (1.03 / 0.98 / 0.96), of 7168 / 3072 0.97 / 0.96 / 0.90 (1.02 / 0.93 / 0.91); 160 of 6144 / 6144 0.99 / 0.97 / 0.92 (0.99 /
     // 0.95 / 0.92): from 40 rows on.  Below 1024 columns uniform routing wins and Zipf does not: 512 and 256 columns of 7168 / 4096
-    // at 48 rows 0.98 and 0.99 (1.03 and 1.18), 768 of 128 experts of 4096 / 3072 0.94 (1.03).  From 2048 columns on and K = 7168
-    // earlier still: 256 experts of 7168 / 4096 at 8 / 16 / 32 / 48 rows 0.99 / 0.98 / 0.96 / 0.93 (0.98 / 0.99 / 0.94 / 0.94), 128 of
-    // 7168 / 8192 at 8 / 12 / 24 0.99 / 0.99 / 0.98 (1.02 / 0.99 / 0.98); in the layer, whose router leaves more experts idle, 9 /
-    // 12 / 16 / 22 / 31 rows 0.99 / 0.98 / 0.98 / 0.96 / 0.96 (0.99 / 0.95 / 0.89 / 0.93 / 0.91): 512 tokens under Zipf(1.1) 599 ->
-    // 536 us.  That would be 12; it is 17 because moe355_layer_kernel_name() has always named the 128-row tiles for
-    // that batch.
-    const int64_t from = columns < 4 * kComputeUnits || narrow ? 64 : columns >= 8 * kComputeUnits && a.K >= 7168 ? 17 : 40;
+    // at 48 rows 0.98 and 0.99 (1.03 and 1.18), 768 of 128 experts of 4096 / 3072 0.94 (1.03).
+    // From 2048 columns on earlier still, and with many experts and a long K, where more of the time is the weight stream, before
+    // that.  Layers, the mean over uniform routing, Zipf(0.8) and Zipf(1.1), ten draws each, wide / 128-row tiles at 12 / 16 / 18 /
+    // 20 / 24 / 28 / 36 rows:
+    //   256 experts of 7168 / 2048 1.02 / 0.99 / 0.98 / 0.98 / 0.99 / 0.96 / 0.96, of 5120 / 2048 1.04 / 0.99 / 0.98 / 0.98 / 0.98 /
+    //     0.96 / 0.95: from 17 on, though mildly skewed batches lose until 24 (at 18 rows uniform 0.98 and 0.97, Zipf(0.8) 1.02 and
+    //     1.02, Zipf(1.1) 0.95 and 0.94)
+    //   256 of 4096 / 2048 1.05 / 1.01 / 1.00 / 1.00 / 1.00 / 0.98 / 0.97 (Zipf(0.8) 1.04 at 18 and 20, 0.99 at 28), 512 of 4096 / 1024
+    //     1.03 / 1.01 / 0.99 / 0.99 / 1.00 / 0.99 / 0.99, 192 of 7168 / 2816 1.03 / 1.02 / 1.01 / 1.00 / 0.99 / 0.98 / 0.97, 128 of 7168 /
+    //     4096 0.99 / 1.01 / 1.00 / 1.00 / 1.00 / 0.98 / 0.96, of 8192 / 4096 0.98 / 1.02 / 1.01 / 1.02 / 1.02 / 0.98 / 0.95, of 5120 / 4096
+    //     0.98 / 1.01 / 0.99 / 1.01 / 1.00 / 0.97 / 0.96, 64 of 6144 / 8192 1.00 / 0.99 / 0.99 / 0.98 / 0.98 / 0.96 / 0.95: from 28 on
+    const int64_t early = a.E >= 256 && a.K >= 5120 ? 17 : 28;
+    const int64_t from = columns < 4 * kComputeUnits || narrow ? 64 : columns < 8 * kComputeUnits ? 40 : early;
     if (avg >= from && avg <= 256 && a.K >= 4096 && wide_ok && (narrow || a.E == 1 || columns >= kComputeUnits / 2)) return 256;
     // Above 256 rows an expert has two tall tiles and more, and they fetch its weights half as often as the 128-row tiles.  That
     // is what counts where an expert's weights are several times the 4 MiB of an XCD's L2.  One product, wide / 128-row tiles:
