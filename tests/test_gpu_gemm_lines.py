@@ -359,6 +359,36 @@ def test_few_rows_on_weight_streaming_tiles(avg, E, Kd, N, family):
 @pytest.mark.parametrize("counts", [[193] * 8, [256, 193, 255, 194, 200, 220, 193, 256], [512, 0, 3, 509, 40, 0], [700, 192, 161, 129, 1, 0, 64, 33]],
                          ids=["no room", "some room", "room", "all heights"])
 def test_halves_of_tall_tiles(counts, Kd, N):
+    _check_tall_tiles(counts, Kd, N)
+
+
+# ... which are those of experts with several tiles; tall ones that are their expert's only tile have one entry.  The number of
+# entries of the list (the first word of the workspace), with no room for halves, some, enough
+@pytest.mark.parametrize("counts,entries", [([200] * 8, 8), ([256, 193, 255, 194, 200, 220, 193, 256], 8), ([449, 1, 1, 1], 5),
+                                            ([449, 500, 40, 0], 7), ([449] * 4 + [1] * 4, 15), ([512, 0, 3, 509, 40, 0], 10),
+                                            ([240] * 23 + [257], 25), ([240] * 22 + [257, 0], 45)])
+def test_entries_of_tall_tiles(counts, entries):
+    from vllm_ascend_amd import kernels as K
+    from vllm_ascend_amd._lib import load
+
+    lib, E, R, Kd, N = load(), len(counts), sum(counts), 4096, 192
+    print(f"entries of {counts}", flush=True)
+    assert lib.moe355_gmm_kernel_name(2, R, Kd, N, E).decode() == "gmm_wide_kernel"
+    x = torch.zeros(R, Kd, dtype=torch.int8, device="cuda")
+    w = torch.zeros(E, N * Kd, dtype=torch.int8, device="cuda")
+    sw, sx = torch.ones(E, N, device="cuda"), torch.ones(R, device="cuda")
+    gl = torch.tensor(counts, dtype=torch.int64, device="cuda")
+    out = torch.empty(R, N, dtype=torch.bfloat16, device="cuda")
+    ws = torch.zeros(lib.moe355_gmm2_dequant_workspace(R, N, Kd, E), dtype=torch.uint8, device="cuda")
+    p = lambda t: t.data_ptr()  # noqa: E731
+    assert lib.moe355_gmm2_dequant(p(x), p(w), p(sw), p(sx), p(gl), 1, R, Kd, N, E, p(out), K._dt(out, "out"), p(ws), ws.numel(),
+                                   torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert int(ws[:4].view(torch.int32)) == entries
+    _check_tall_tiles(counts, Kd, N)
+
+
+def _check_tall_tiles(counts, Kd, N):
     from oracle import oracle as orc
     from vllm_ascend_amd import kernels as K
     from vllm_ascend_amd._lib import W_ENK, load

@@ -23,8 +23,8 @@ struct TileSpec {
     TileMap tm;
     int BM, max_tiles;
     // the 256-row weight-streaming tiles, listed longest first -- 161..192 rows, 129..160, up to 128 -- so that the workgroups
-    // that start last are the short ones and the compute units finish closer together, and the tall ones (more than 192 rows)
-    // spread evenly among them: the tall tiles of a hot expert find their weights in the caches and wait for the matrix units,
+    // that start last are the short ones and the compute units finish closer together, and the tall ones (more than 192 rows),
+    // where enough of them share their weights with another tile, spread evenly among them: the tall tiles of a hot expert find their weights in the caches and wait for the matrix units,
     // the cold experts' tiles for their weights from HBM, and so both are busy all the time.  In eights, because entry t
     // runs on XCD t % 8.  A tall tile has an entry for either half of its columns as long as the list has room for that (a
     // workgroup per entry and column is launched for as many tiles as the rows can make), beyond it one for both.
@@ -59,6 +59,7 @@ __device__ __forceinline__ void build_tile_map(RowsOf rows_of, int E, const Tile
         // tiles in front of an expert's last one, all of them tall
         auto full_tiles = [](int64_t m) -> int32_t { return (int32_t)((uint32_t)(m - 1) >> 8); };
         int32_t rows = 0, n01 = 0, n23 = 0;  // counts packed 16 + 16 bits (at most max_tiles < 32768 tiles)
+        int32_t shared = 0;                  // tall tiles whose weights another tile of the expert reads too
         for (int j = 0; j < seg; ++j) {
             const int e = e0 + j;
             if (e < E) {
@@ -68,21 +69,33 @@ __device__ __forceinline__ void build_tile_map(RowsOf rows_of, int E, const Tile
                 const int32_t full = full_tiles(m);
                 const int c = cls(m - (int64_t)full * 256);
                 n23 += full << 16;
+                shared += full + (full > 0 && c == 3 ? 1 : 0);
                 if (c < 2) n01 += 1 << (16 * c);
                 else n23 += 1 << (16 * (c - 2));
             }
         }
         int32_t all_rows, all01, all23;
         const int32_t rows_before = block_scan_exclusive_i32(rows, part_a, all_rows);
+        // part_a is free behind the first scan; its sums are visible behind the second one and read before the third one is over
+        const int32_t shared_wave = wave_scan_inclusive_i32(shared);
+        if ((tid & 63) == 63) part_a[tid >> 6] = shared_wave;
         const int32_t b01 = block_scan_exclusive_i32(n01, part_b, all01);
+        int32_t all_shared = 0;
+        for (int w = 0; w < (int)(blockDim.x + 63) >> 6; ++w) all_shared += part_a[w];
         const int32_t b23 = block_scan_exclusive_i32(n23, part_b, all23);
         const int32_t total[4] = {all01 & 0xffff, all01 >> 16, all23 & 0xffff, all23 >> 16};
         const int32_t all_tiles = total[0] + total[1] + total[2] + total[3];
         const int32_t room = max_tiles > all_tiles ? max_tiles - all_tiles : 0;
-        // Fewer than one tall tile in 16 has no phase of its own to mix, and halves only read their tokens twice: whole and last.
-        // 4096 tokens of uniform routing, gate_up / down 1344 / 792 us spread, 1318 / 778 so; under Zipf(0.6), where one in 8 to 16
-        // is tall, the layer at 2048 tokens 2175 spread, 2261 so.
-        const bool few = 16 * total[3] < all_tiles;
+        // Whole and last: fewer than one tall tile in 16, which has no phase of its own to mix, and tall tiles that are their
+        // experts' only ones, which wait for HBM as the others do; halves would only read their tokens twice.  Few of the first
+        // kind, 4096 tokens of uniform routing, gate_up / down 1344 / 792 us spread, 1318 / 778 so; under Zipf(0.6), where one in 8 to
+        // 16 is tall, the layer at 2048 tokens 2175 spread, 2261 so.  Of the second kind, uniform routing, layers as they were
+        // before there were halves / spread / so: 8 experts of 4096 / 14336, 187 / 200 / 220 rows each 471 / 525 / 469, 473 / 634 / 473, 484 /
+        // 600 / 484; 128 of 4096 / 1536, 210 rows 777 / 803 / 778; 96 of 8192 / 2048, 200 rows 1301 / 1361 / 1304.  With 240 to 256 rows,
+        // where some experts spill over into a second tile, spreading wins: 256 of 7168 / 2048 3580 / 3475 at 240, 64 of 8192 /
+        // 2560 1453 / 1340 at 250, 96 of 8192 / 2048 1562 / 1505 under Zipf(0.1) at 220, where one tile in eight is tall and shared.
+        // Between (one in 33, 24, 22, 21, 17): 1.01, 0.98, 0.95, 1.01, 0.97 of the time.
+        const bool few = 16 * total[3] < all_tiles || 24 * all_shared < all_tiles;
         const int32_t whole = few ? total[3] : total[3] > room ? total[3] - room : 0;  // tall tiles with one entry, the first ones
         const int32_t tall = 2 * total[3] - whole;
         if (tid == 0) tm.count[0] = all_tiles < max_tiles ? all_tiles - total[3] + tall : max_tiles;
