@@ -52,7 +52,7 @@ TRAFFIC_FROM_PROFILES = {
     "c2_qwen3_decode": (399_900_000, "profiles/moe_layer_qwen3_decode_kernel_trace.md"),
     "c3_qwen3_prefill": (960_000_000, "profiles/moe_layer_qwen3_prefill_kernel_trace.md"),
     "c4_dsv3_prefill": (8_014_000_000, "profiles/moe_layer_dsv3_prefill_kernel_trace.md"),
-    "c5_w4a8_zipf": (1_799_700_000, "profiles/moe_layer_w4a8_zipf_kernel_trace.md"),
+    "c5_w4a8_zipf": (1_742_000_000, "profiles/moe_layer_w4a8_zipf_kernel_trace.md"),
     "c6_dsv3_decode": (6_596_100_000, "profiles/moe_layer_dsv3_decode_kernel_trace.md"),
     "c7_w8a8_zipf": (3_031_500_000, "profiles/moe_layer_w8a8_zipf_kernel_trace.md"),
     "c7_w8a8_zipf_4096": (8_188_300_000, "profiles/moe_layer_w8a8_zipf_4096_kernel_trace.md"),

@@ -85,8 +85,8 @@ __global__ __launch_bounds__(256) void token_unpermute_kernel(UnpermuteArgs a)
     if constexpr (TOPK > 0) {
         // Rows, weights and ids of the slots are the same for the whole workgroup: every wavefront reads them into lanes, one load
         // each, in front of the rows.  In pair order the rows' addresses wait for nothing (a row that nobody computed is read
-        // and left out).  With a barrier and LDS between the two, 64 tokens of 2 x 1024 values took 2.9 us and take 1.7 (the small
-        // layer 26.3 -> 24.9 us a call); of 8 x 2048 values 109.9 -> 109.4 us a call.
+        // and left out).  With a barrier and LDS between the two, 64 tokens of 2 x 1024 values took 2.9 us and take 1.7; calls of
+        // both in turn: the small layer, 64 tokens, 24.7 and 24.4 us, others the same within noise.
         const int lane = threadIdx.x & 63;
         const int64_t mine = t * TOPK + (lane < TOPK ? lane : TOPK - 1);
         int32_t d = idx ? idx[mine] : (int32_t)mine;

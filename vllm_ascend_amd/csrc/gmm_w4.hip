@@ -265,8 +265,9 @@ struct W4Unit {
 // NB: blocks of 32 rows.  STREAM: the expert has a single chunk, nobody else reads these weights: non-temporal loads (the
 // faster pure stream).  That goes for the number of chunks, not of rows: with the last 32 rows and fewer of a hot expert past
 // the caches too, Zipf(1.1), 128 / 256 / 512 / 1024 tokens took 322 / 413 / 623 / 896 us a layer call and take 314 / 406 / 615 /
-// 884 (512 tokens: 1766 and 802 MB read from HBM by the two products, 1708 and 770 so).  Otherwise the sibling chunks of the expert run at the same time on the same XCD (their workgroup
-// numbers differ by a multiple of 8) and ordinary loads let them share one fetch in L2.
+// 884 (512 tokens: 1766 and 802 MB read from HBM by the two products, 1708 and 770 so).  Otherwise the sibling chunks of the expert run
+// at the same time and ordinary loads let them share a fetch: in L2 where a chunk has a multiple of eight workgroups (N of about
+// a multiple of 1024), so that the same channels of all chunks are on one XCD, else in the last-level cache.
 template <int EPI, bool LDS_SCALES, int NB, bool STREAM, bool FAR>
 __device__ __forceinline__ void w4_chunk_body(const W4Args& p, const W4Unit& t, const __amdgpu_buffer_rsrc_t xr, const int8_t* xb,
                                               const int64_t* xo)
@@ -748,7 +749,7 @@ __global__ __launch_bounds__(256, 4) void gmm_w4_pairs_kernel(W4Args p)
 }
 
 // workgroups: an upper bound of the number of 64-row chunks (known on the host without reading the group
-// list) times the groups of four tile pairs
+// list) times the groups of four units of 32 channels
 static int64_t w4_blocks(int64_t rows, int num_experts, int64_t n)
 {
     // a chunk has at least one row: a decode batch of a few rows has a few chunks, not one per expert (a workgroup
