@@ -87,6 +87,16 @@ __device__ __forceinline__ v4i gload16(const void* p) { return *(gv4i_ptr)(uintp
 __device__ __forceinline__ v4i gload16_nt(const void* p) { return __builtin_nontemporal_load((gv4i_ptr)(uintptr_t)p); }
 __device__ __forceinline__ v4f gload4f(const float* p) { return *(gv4f_ptr)(uintptr_t)p; }
 
+// 16 bytes written through the L2, for the outputs of the large products.  A read stream of weights with 128-byte row pieces
+// written beside it, non-temporal / plain / written through, us: 1611 + 75 MB 292 / 296 / 282, 805 + 101 MB 156 / 155 / 148, 201 +
+// 25 MB 37.7 / 39.1 / 34.7, 1611 + 200 MB 324 / 316 / 304 (sc0 sc1 as sc1; with nt beside either as non-temporal; pieces of 128
+// bytes to 1 KiB the same).  The down products 2 to 5 % faster than with non-temporal stores.
+__device__ __forceinline__ void store16_through(void* p, v4i v)
+{
+    // (behind a store of 16 bytes the next two wait states may not write its data)
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+}
+
 __device__ __forceinline__ v16i mfma_i8(v4i a, v4i b, v16i c)
 {
     return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);

@@ -163,7 +163,7 @@ __device__ __forceinline__ void resident_body(const GmmArgs& a, int e, int64_t r
             asm volatile("" : "+v"(at));  // the sums below are made here: kept over the K loop they would cost 16 registers
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                __builtin_amdgcn_raw_buffer_store_b128(t[i], out, at + (b * 32 + 8 * i) * a.N * 2, 0, 2 /* non-temporal */);
+                __builtin_amdgcn_raw_buffer_store_b128(t[i], out, at + (b * 32 + 8 * i) * a.N * 2, 0, 16 /* sc1: see store16_through */);
             __builtin_amdgcn_sched_barrier(0);
         }
     };

@@ -169,13 +169,11 @@ __device__ __forceinline__ void tiled_epilogue_body(const GmmArgs& a, int e, v4i
                     *(v4i*)(a.acc + orow * a.N + nb1 * 32 + c16 * 4) =
                         *(const v4i*)(patch + 32 * ROWB + r * ROWB + c16 * 16);
                 } else if constexpr (EPI == EPI_DEQUANT) {
-                    // Non-temporal stores for the two large outputs: written back through the L2 in the ordinary
-                    // way they slowed the weight streams of every other workgroup (K loops 8 % longer).
-                    __builtin_nontemporal_store(*(const v4i*)(patch + r * ROWB + c16 * 16),
-                                                (v4i*)(a.out + orow * a.N + nb0 * 32 + c16 * 8));
+                    // Written through the L2: written back by it in the ordinary way they slowed the weight streams of every
+                    // other workgroup (K loops 8 % longer), and store16_through has the rest.
+                    store16_through(a.out + orow * a.N + nb0 * 32 + c16 * 8, *(const v4i*)(patch + r * ROWB + c16 * 16));
                 } else {
-                    __builtin_nontemporal_store(*(const v4i*)(patch + r * ROWB + c16 * 16),
-                                                (v4i*)(a.y + orow * (a.N >> 1) + nb0 * 32 + c16 * 4));
+                    store16_through(a.y + orow * (a.N >> 1) + nb0 * 32 + c16 * 4, *(const v4i*)(patch + r * ROWB + c16 * 16));
                 }
             }
         }
