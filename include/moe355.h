@@ -502,6 +502,14 @@ int moe355_token_unpermute_pairs(const void *rows, int dtype, const void *probs,
  */
 int moe355_profile_next_gemm(void *start_event, void *stop_event);
 
+/* On the sorted path of moe355_layer_forward the workgroups of a tile of the gate_up product can exchange the maxima of its rows
+ * and quantise them in place: the rows of those tiles, or 0 where the fp32 values go through memory and a launch of their own.
+ * A workgroup that has looked for the others' maxima some thousand times computes them itself; the next such product that the
+ * calling thread launches gives up after `looks` instead (0: at once).  The results are the same either way.
+ */
+int moe355_meeting_tile_rows(int64_t rows, int64_t k, int64_t n, int num_experts);
+int moe355_next_meeting_looks(int looks);
+
 /* Which kernel family the int8 grouped GEMMs above launch for a shape, given a workspace of the size their
  * moe355_*_workspace() asks for: "gmm_stream_kernel" (few rows per expert), "gmm_tiled_kernel" (64- or 128-row
  * LDS-tiled), "gmm_resident_kernel" (dequant only, many rows per expert and a short K: 128-row tiles whose tokens stay in

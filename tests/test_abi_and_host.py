@@ -548,6 +548,18 @@ def test_tokens_of_a_tile_in_lds_lines(rows, experts, k, n, resident):
     assert name(0, rows, k, n, experts) != b"gmm_resident_kernel" != name(1, rows, k, n, experts)
 
 
+# where the column workgroups of a gate_up tile exchange the rows' maxima: rows of their tiles
+@pytest.mark.parametrize("experts, k, n, rows, tile_rows", [
+    (256, 7168, 4096, 4096, 128), (256, 7168, 4096, 256 * 144, 256), (256, 7168, 4096, 256 * 145, 0), (128, 2048, 2048, 1152, 128),
+    (128, 2048, 1536, 1024, 64), (128, 2048, 1536, 128 * 64 - 1, 64), (128, 2048, 1536, 128 * 64, 128), (128, 2048, 1536, 65536, 128),
+    (256, 2048, 1536, 256 * 48 - 1, 0), (256, 2048, 1536, 256 * 48, 128), (64, 4096, 3072, 1152, 0), (128, 4096, 3072, 10240, 0),
+    (32, 2880, 5760, 9600, 0), (8, 1024, 2816, 1040, 64), (8, 1024, 2816, 16000, 128), (128, 2048, 1536, 512, 0), (1, 2048, 4096, 4096, 0)])
+def test_where_gate_up_tiles_quantise_their_rows(experts, k, n, rows, tile_rows):
+    from vllm_ascend_amd import _lib
+
+    assert _lib.load().moe355_meeting_tile_rows(rows, k, n, experts) == tile_rows
+
+
 # one for every 56 pairs, but not where a short launch (fewer than 1536 units of 64 channels) has places in front of its slots
 # (from two pairs per expert on), nor from twelve pairs per expert on
 @pytest.mark.parametrize("experts, n, pairs, blocks", [(128, 1536, 512, 9), (128, 512, 256, 4), (128, 512, 257, 0), (128, 704, 512, 0),

@@ -1,0 +1,115 @@
+"""The gate_up product whose tiles' workgroups exchange the maxima of their rows and store int8, against the operators (fp32
+values in memory, a launch that quantises them): the same bits, also where a workgroup gives up looking for the others'."""
+import dataclasses
+
+import pytest
+import torch
+
+from _inputs import CONFIGS, make_layer
+from _layer_utils import build_layer
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _lib():
+    from vllm_ascend_amd._lib import load
+
+    return load()
+
+
+def _layer(tokens, **shape):
+    cfg = dataclasses.replace(CONFIGS["c2_small"], T=tokens, **shape)
+    d = make_layer(cfg, seed=tokens)
+    return cfg, build_layer(cfg, d, DEV), d["x"].to(DEV), d["logits"].to(DEV)
+
+
+def _random_layer(tokens, E, k, H, I):
+    """Weights made on the GPU: the shapes that reach the weight-streaming tiles are too large for the host's generator."""
+    cfg = dataclasses.replace(CONFIGS["c2_small"], T=8, E=E, k=k, H=64, I=32)
+    d = make_layer(cfg, seed=tokens)
+    g = torch.Generator(device=DEV).manual_seed(tokens)
+    for name, shape in (("w13", (E, 2 * I, H)), ("w2", (E, H, I))):
+        d[name] = torch.randint(-128, 128, shape, generator=g, device=DEV, dtype=torch.int8)
+    d["s13"], d["s2"] = (torch.rand(E, n, generator=g, device=DEV) * 0.009 + 0.001 for n in (2 * I, H))
+    layer = build_layer(dataclasses.replace(cfg, T=tokens, H=H, I=I), d, DEV)
+    x = torch.randn(tokens, H, generator=g, device=DEV).to(torch.bfloat16)
+    return layer, x, torch.randn(tokens, E, generator=g, device=DEV)
+
+
+def _check(layer, x, logits, looks=(None,)):
+    want = layer.forward_impl(x, logits).routed_out
+    for n in looks:
+        if n is not None:
+            assert _lib().moe355_next_meeting_looks(n) == 0
+        got = layer(x, logits)
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), n
+    assert layer._layer_plan.desc is not None
+
+
+# one column block and several, whole and partial ones (128 values each), 64- and 128-row tiles, a list whose tiles two XCDs
+# share, K of one step and of every remainder modulo the ring
+@pytest.mark.parametrize("E, k, T, H, I, tile_rows", [
+    (8, 2, 512, 64, 32, 128), (8, 2, 513, 128, 160, 128), (8, 2, 515, 192, 288, 64), (8, 2, 521, 256, 512, 64), (6, 2, 600, 320, 1408, 64),
+    (32, 4, 517, 512, 512, 64), (16, 4, 2049, 256, 1024, 128), (64, 8, 300, 448, 640, 128), (96, 8, 257, 256, 1024, 64)])
+@pytest.mark.parametrize("skew", [0.0, 3.0])
+def test_layers_on_tiles(E, k, T, H, I, tile_rows, skew):
+    print(f"E={E} k={k} T={T} H={H} I={I} skew={skew} tiles of {_lib().moe355_meeting_tile_rows(T * k, H, 2 * I, E)}", flush=True)
+    cfg, layer, x, logits = _layer(T, E=E, k=k, H=H, I=I)
+    logits = logits - skew * torch.arange(E, device=DEV).float().log1p()
+    _check(layer, x, logits, looks=(None, 0, 1))
+
+
+# rows at the edges of a tile and of a wavefront's groups of 16
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 31, 33, 63, 64, 65, 127, 128, 129, 192, 193])
+def test_rows_of_an_expert(rows):
+    T, E = 1024, 8
+    cfg, layer, x, logits = _layer(T, E=E, k=1, H=128, I=256)
+    assert _lib().moe355_meeting_tile_rows(T, 128, 512, E)
+    logits = torch.full((T, E), -9.0, device=DEV)
+    logits[torch.arange(T), torch.where(torch.arange(T) < rows, 0, 1 + torch.arange(T) % (E - 1))] = 9.0
+    _check(layer, x, logits, looks=(None, 0))
+
+
+@pytest.mark.parametrize("limit", [0.0, 0.7])
+def test_clamp_infinities_and_zeros(limit):
+    cfg, layer, x, logits = _layer(640, E=8, k=2, H=256, I=512)
+    layer.moe_config = dataclasses.replace(layer.moe_config, swiglu_limit=limit)
+    x = x.clone()
+    x[3] = 0
+    x[70] = float("inf")
+    x[200, 5] = float("nan")
+    x[300] *= 1e30
+    _check(layer, x, logits, looks=(None, 0))
+
+
+# weight-streaming tiles: one to six blocks of 32 rows, tall ones with an entry for every half and with one for both, alone and
+# beside short ones; the last column block of 512 channels a half one, an odd number of them
+@pytest.mark.parametrize("E, k, H, I, T, skew", [
+    (64, 8, 1024, 1024, 1000, 0.0), (64, 8, 1024, 1024, 1100, 0.3), (64, 8, 1024, 1024, 1100, 1.1), (128, 8, 1024, 640, 2000, 0.0),
+    (128, 8, 1024, 640, 1900, 1.1), (128, 8, 1088, 672, 2000, 0.5), (4, 1, 1024, 256, 500, 0.2)])
+def test_layers_on_weight_streaming_tiles(E, k, H, I, T, skew):
+    rows = _lib().moe355_meeting_tile_rows(T * k, H, 2 * I, E)
+    print(f"E={E} k={k} T={T} H={H} I={I} skew={skew} tiles of {rows}", flush=True)
+    assert rows == 256
+    layer, x, logits = _random_layer(T, E, k, H, I)
+    _check(layer, x, logits - skew * torch.arange(E, device=DEV).float().log1p(), looks=(None, 0))
+
+
+def test_captured_and_from_two_streams():
+    cfg, layer, x, logits = _layer(700, E=8, k=2, H=256, I=640)
+    want = layer.forward_impl(x, logits).routed_out
+    layer(x, logits)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = layer(x, logits)
+    side = torch.cuda.Stream()
+    for _ in range(5):
+        out.zero_()
+        graph.replay()
+        with torch.cuda.stream(side):
+            beside = [layer(x, logits) for _ in range(3)]
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and all(torch.equal(b, want) for b in beside)

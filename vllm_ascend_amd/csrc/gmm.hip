@@ -810,14 +810,14 @@ static int dense_slabs(int64_t R, int K, int N, int E)
 }
 
 // The tile map that launch_gemm_auto of this product will look for in tile_ws: its number, 0 or 1.
-int gemm_tile_specs(int64_t rows, int64_t k, int64_t n, int num_experts, void* tile_ws, TileSpec* specs)
+int gemm_tile_specs(int64_t rows, int64_t k, int64_t n, int num_experts, void* tile_ws, TileSpec* specs, int tile_rows)
 {
     GmmArgs a = {};
     a.R = rows;
     a.K = (int)k;
     a.N = (int)n;
     a.E = num_experts;
-    const int bm = dense_tiles(a) || split_tiles(a) ? 0 : gemm_family(a, true);
+    const int bm = tile_rows ? tile_rows : dense_tiles(a) || split_tiles(a) ? 0 : gemm_family(a, true);
     if (bm) specs[0] = tile_spec(rows, num_experts, bm, tile_ws);
     return bm ? 1 : 0;
 }
@@ -1005,11 +1005,75 @@ extern "C" size_t moe355_gmm1_swiglu_quant_workspace(int64_t rows, int64_t n, in
     return (((size_t)rows * (size_t)(n / 2) * 4 + 255) & ~(size_t)255) + tiled_ws_max(rows, num_experts);
 }
 
+// a few milliseconds
+constexpr int kMeetLooks = 4096;
+static thread_local int t_meet_looks = kMeetLooks;
+
+extern "C" int moe355_next_meeting_looks(int looks)
+{
+    if (looks < 0) return MOE355_E_ARG;
+    t_meet_looks = looks;
+    return MOE355_OK;
+}
+
+// Whether the column workgroups of the gate_up product's tiles meet.  A tile whose columns do not all start in the same round of
+// workgroups makes the first of them wait for the rest, holding their place: so a number of columns that divides the places of an
+// XCD (64 of the 128-row tiles, 32 of the wide ones) is what matters.  The layer with / without, uniform routing (Zipf(1.1)),
+// rows per expert in brackets:
+//   - dividing: 8 columns, 64 and 128 experts of 2048 / 1024 (18 to 160) 0.99 .. 0.94 (1.01 .. 0.95); 4 columns, 256 of 2048 / 512 (9 to
+//     160) 1.00 .. 0.92 (0.97 .. 0.93), 64 of 1024 / 512 0.99 .. 0.94 (0.97 .. 0.92); 16 columns, 256 of 7168 / 2048 (6 and 16) 0.98 and
+//     0.96 (0.97 at 16);
+//   - others: 6 columns, 128 of 2048 / 768 (54 / 100 / 200 / 300) 0.98 / 0.99 / 0.96 / 0.94 (0.97 / 0.99 / 0.96 / 0.96), 256 of them (18 / 48 /
+//     100 / 300) 1.03 / 0.97 / 0.98 / 1.00 (1.00 / 0.99 / 0.96 / 0.99); 11 columns, 60 of 2048 / 1408 (30 / 64 / 128 / 300) 0.98 / 0.96 /
+//     0.97 / 0.95 (1.03 / 0.98 / 1.01 / 0.98), 8 of 1024 / 1408 (250 to 2000) 0.96 .. 0.92; 12 columns of 12 and 16 MB an expert, 64 of
+//     4096 / 1536 (18 / 36 / 300 / 600) 1.07 / 1.07 / 1.00 / 0.98 (1.00 / 0.99 / 0.99 / 1.00), 128 of them (9 / 36 / 300) 1.02 / 1.02 / 1.00
+//     (1.03 / 0.98 / 0.99); 23 columns, 32 of 2880 / 2880 (36 / 60 / 300 / 600) 0.98 / 1.00 / 1.05 / 1.15 (1.04 / 0.99 / 1.00 / 1.12).  So from
+//     48 rows on, up to 12 columns and 8 MB.
+//   - a launch with workgroups for more than two and up to three per compute unit (128 of 2048 / 768: 768) loses on 128-row tiles, which
+//     fill a round and a half (9 / 18 / 27 / 36 rows 1.06 / 1.04 / 1.02 / 1.01, Zipf(1.1) 0.98 / 0.99 / 1.01 / 0.99), and wins on tiles of
+//     64 rows, three of which fit a compute unit: 0.99 / 0.97 / 0.95 / 0.94 (0.96 / 0.94 / 0.95 / 0.98; Zipf(0.8) 0.98 / 1.01 / 0.96 / 0.97),
+//     at 48 and 60 rows 0.99 and 0.94 (0.99 and 0.97; 1.00 and 1.00).  Not with 12 MB an expert, whose hot ones read them again for every
+//     tile (64 of 4096 / 1536, 36 / 48 / 60 rows under Zipf(1.1) 1.06 / 1.08 / 1.09).
+//   - wide tiles, 8 columns of 512 channels, 64 experts of 7168 / 2048 (40 / 64 / 96 / 128 / 160 / 200) 0.98 / 0.98 / 0.97 / 0.96 / 0.98 / 1.00
+//     (0.98 / 0.97 / 0.98 / 0.98 / 1.04 / 0.99), 256 of them (47 / 94 / 128) 0.94 / 0.95 / 1.00; 4 columns, 64 of 4096 / 1024 (64 / 128 / 200)
+//     0.97 / 0.95 / 0.99 (0.99 / 0.97 / 0.98); 3 columns, 128 of 2048 / 768 (125) 0.95 (0.98), 160 of 4096 / 768 (40 / 100 / 160) 0.94 / 0.96
+//     / 1.00 (0.99 / 0.97 / 0.98); 6 columns, 128 of 4096 / 1536 (64 / 80 / 112 / 160) 1.03 / 1.04 / 1.03 / 1.08 (1.00 / 0.99 / 1.00 / 1.02);
+//     10 columns, 128 of 5120 / 2560 (40 / 96 / 128 / 160) 1.00 / 1.02 / 1.02 / 1.05 (0.98 / 1.01 / 1.02 / 1.00).  So up to 4 columns and
+//     with 8, to 144 rows.
+MeetingPlan moe355::meeting_plan(int64_t rows, int64_t k, int64_t n, int num_experts)
+{
+    GmmArgs a = {};
+    a.R = rows;
+    a.K = (int)k;
+    a.N = (int)n;
+    a.E = num_experts;
+    if (dense_tiles(a) || split_tiles(a)) return {};
+    const int bm = gemm_family(a, true), columns = (a.N / 2 + 127) / 128;
+    const int64_t avg = rows / num_experts, own = n * k;
+    const MeetingPlan yes = {bm, columns};
+    if (bm == 256) {
+        const int wide = (columns + 1) / 2;
+        return (wide <= 4 || wide == 8) && avg <= 144 ? yes : MeetingPlan{};
+    }
+    if (bm == 0) return {};
+    if (columns <= 16 && (columns & (columns - 1)) == 0) return yes;
+    const int64_t least = (int64_t)num_experts * columns;
+    if (bm == 128 && least > 2 * kComputeUnits && least <= 3 * kComputeUnits && own <= (4 << 20) && avg < 64) return {64, columns};
+    return columns <= 12 && own <= (8 << 20) && avg >= 48 ? yes : MeetingPlan{};
+}
+
+extern "C" int moe355_meeting_tile_rows(int64_t rows, int64_t k, int64_t n, int num_experts)
+{
+    if (rows <= 0 || k <= 0 || n <= 0 || num_experts <= 0) return 0;
+    return moe355::meeting_plan(rows, k, n, num_experts).tile_rows;
+}
+
 int moe355::gmm1_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list,
                       const float* weight_scale, const float* const* scale_list, const float* x_scale,
                       const int64_t* group_list, int group_list_type, int64_t rows, int64_t k, int64_t n,
                       int num_experts, float swiglu_limit, int8_t* out, float* out_scale, void* workspace,
-                      size_t workspace_bytes, void* stream, const int32_t* row_src, bool tiles_ready)
+                      size_t workspace_bytes, void* stream, const int32_t* row_src, bool tiles_ready, const MeetingPlan& plan,
+                      uint32_t* meet)
 {
     const void* wany = weight_list ? (const void*)weight_list : (const void*)weight_nz;
     int rc = check_gmm(x, wany, group_list, group_list_type, rows, k, n, num_experts);
@@ -1041,6 +1105,16 @@ int moe355::gmm1_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* co
     a.row_src = row_src;
     a.tiles_ready = tiles_ready;
     void* tile_ws = gmm1_tile_ws(workspace, rows, n);
+    if (tiles_ready && plan.columns) {
+        a.meet = meet;
+        a.meet_looks = t_meet_looks;
+        t_meet_looks = kMeetLooks;
+        a.q = out;
+        a.q_scale = out_scale;
+        hipEvent_t ev0, ev1;
+        take_profile_events(ev0, ev1);
+        return launched(launch_tiled_any(EPI_MEET, plan.tile_rows, a, tile_ws, st, ev0, ev1));
+    }
     rc = launch_gemm_auto<EPI_SWIGLU>(a, tile_ws, st);
     if (rc != MOE355_OK) return rc;
     launch_swiglu_requant(y, group_list, group_list_type, num_experts, rows, I, out, out_scale, st);

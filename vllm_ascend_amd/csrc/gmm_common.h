@@ -14,7 +14,10 @@
 
 namespace moe355 {
 
-enum { EPI_I32 = 0, EPI_SWIGLU = 1, EPI_DEQUANT = 2 };
+enum { EPI_I32 = 0, EPI_SWIGLU = 1, EPI_DEQUANT = 2, EPI_MEET = 3 };
+
+// EPI_MEET: SwiGLU and the rows' quantisation; the workgroups of a tile exchange the maxima of its rows (gmm_tiled.hip)
+constexpr bool gated(int epi) { return epi == EPI_SWIGLU || epi == EPI_MEET; }
 
 struct GmmArgs {
     const int8_t* x;        // [R, K]
@@ -59,6 +62,11 @@ struct GmmArgs {
     int beside;             // dense product on a side stream: few workgroups that hide, not many that finish early
     float limit;            // swiglu clamp
     int tiles_ready;        // the tile maps of this call are in its workspace already (built by the routing launch)
+    // EPI_MEET: [columns][R] the maximum of a row over a column block, its bits with the sign set; zero before the launch
+    uint32_t* meet;
+    int meet_looks;         // at the others' maxima before a workgroup computes them itself
+    int8_t* q;              // [R, N/2]
+    float* q_scale;         // [R]
     // outputs
     int32_t* acc;           // EPI_I32   [R, N]
     int32_t* acc_part;      // EPI_I32 with K cut into slabs: [slabs][R, N] partial sums (or null: atomics into acc)

@@ -181,6 +181,251 @@ __device__ __forceinline__ void tiled_epilogue_body(const GmmArgs& a, int e, v4i
     }
 }
 
+// ------------------------------------------------------------------ where the column workgroups of a tile meet
+// A row of SwiGLU values is quantised with its maximum, and its columns are in several workgroups.  Written as fp32 and quantised by
+// a launch of its own, the values of a prefill batch pass through HBM twice, and what a product writes costs it more than what
+// it reads: beside a stream of weights at 7 TB/s the writes go at 1.7 to 2.6 (128 experts of 49 rows, 2048 / 1536: 72.8 us, 64.5
+// without the stores).  So (EPI_MEET) the workgroups of a tile exchange the maxima of their columns, keep the values in registers
+// until the others' are there, and store int8.
+// - Every workgroup stores the maxima of its rows over its columns into a word of its own per row (with the sign set: a word of
+//   zero is not there yet) and looks at the others' until none is missing: no counter, no order, no fence, since a word is all that
+//   is handed over.  The routing launch clears the words.
+// - They run at the same time, because a launch starts its workgroups in order and those of a tile are neighbours.  Nothing rests on
+//   that: a workgroup that has looked meet_looks times (a few milliseconds) computes the missing maxima itself.
+// What it costs is that they wait for the slowest, which is why the number of columns matters (meeting_plan in gmm.hip).  us a layer
+// with / without, 128 experts of 2048 / 768, 777 / 2000 / 4000 / 8192 tokens 138 / 184 / 292 / 496 against 143 / 194 / 313 / 531; 256 of
+// 7168 / 2048, 500 / 1500 / 3000 tokens 1712 / 1831 / 2049 against 1770 / 1956 / 2157; 8 of 1024 / 1408, 6000 tokens 105 against 115.
+// Exchanged by atomic maxima and a counter per tile it took 2 us a tile more, with atomics inside the XCD's L2 the same
+// (4096 / 7168: 6 % more).
+//
+// a look at a word that another workgroup writes
+__device__ __forceinline__ uint32_t look(const uint32_t* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The maxima of the tile's rows over column block c, by the workgroup itself and one product after the other: only where the
+// workgroup that is meant for that block has not come.  sum: rows words of LDS
+template <bool LIMIT>
+__device__ __forceinline__ void maxima_of_column(const GmmArgs& a, int e, int64_t row0, int rows, int c, int channels, uint32_t* sum)
+{
+    for (int i = threadIdx.x; i < rows; i += (int)blockDim.x) sum[i] = 0u;
+    __syncthreads();
+    const int I = a.N >> 1, first = c * channels, n = I - first < channels ? I - first : channels;
+    const int8_t* we = expert_weights(a, e);
+    const float* cs = expert_scales(a, e);
+    for (int i = threadIdx.x; i < rows * n; i += (int)blockDim.x) {
+        const int r = i / n, ch = first + i % n;
+        const int64_t src = a.row_src ? (int64_t)a.row_src[row0 + r] : row0 + r;
+        int g = 0, u = 0;
+        for (int k = 0; k < a.K; k += 16) {
+            const v4i x = gload16(a.x + src * a.K + k);
+            auto add = [&](int ch, int s) {
+                const v4i w = gload16(we + ((int64_t)(ch >> 5) * (a.K >> 5) + (k >> 5)) * 1024 + (k >> 4 & 1) * 512 + (ch & 31) * 16);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) s = __builtin_amdgcn_sdot4(x[j], w[j], s, false);
+                return s;
+            };
+            g = add(ch, g);
+            u = add(ch + I, u);
+        }
+        float gg = ((float)g * a.row_scale[src]) * cs[ch], uu = ((float)u * a.row_scale[src]) * cs[ch + I];
+        if constexpr (LIMIT) {
+            gg = gg > a.limit ? a.limit : gg;
+            uu = uu > a.limit ? a.limit : uu;
+            uu = uu < -a.limit ? -a.limit : uu;
+        }
+        const float y = __builtin_fabsf(m_silu(gg) * uu);
+        if (y > 0.0f) atomicMax(sum + r, __float_as_uint(y));  // (not where it is NaN)
+    }
+    __syncthreads();
+}
+
+// What one workgroup has of a tile.  nt: its column block, of `columns`; g: this wavefront's channel group (a gate tile nb0 and
+// its up tile); lrow: its first row behind row0.  Tall tiles whose two column blocks are done by one workgroup, one after the
+// other: `first` leaves its values in y and goes on, `second` stores both.
+struct TilePart {
+    int e, lrow, g, nb0, nt, columns;
+    int64_t row0, row_end;
+    bool active, first, second;
+};
+
+// acc: the wavefront's 16 NB2 rows.  lds: ROWS * (32 GROUPS + 16) bytes (the maxima of every quarter of a wavefront, then the int8
+// rows), behind them 64 KiB for the values of the widest tiles.  scales: those of the rows (ROWS of them), then 64 of the channels for
+// each group.
+template <int NB2, int GROUPS, int ROWS, bool LIMIT>
+__device__ __forceinline__ void meet_body(const GmmArgs& a, const TilePart& p, v4i (&acc)[4][NB2], int8_t* lds, float* scales)
+{
+    constexpr int PITCH = 32 * GROUPS + 16;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, tok = lane & 15, quarter = lane >> 4, run = 4 * quarter;
+    const int64_t row0 = p.row0, row_end = p.row_end;
+    const int nt = p.nt, columns = p.columns, lrow = p.lrow, g = p.g;
+    const int rows = (int)(row_end - row0 < ROWS ? row_end - row0 : ROWS);
+    float* const part = (float*)lds + (g * 4 + quarter) * ROWS + lrow + tok;
+    int* const met = (int*)(scales + ROWS);  // (in the place of channel scales that have been read by then)
+    const float* const cs = scales + ROWS + g * 64;
+    // With ten groups of 16 rows and more there is no room for all values beside the sums: those of the first four go to LDS.
+    constexpr int STASH = NB2 > 8 ? 4 : 0;
+    constexpr int STASH_AT = (ROWS * PITCH + (ROWS + 64 * GROUPS) * 4 + 15) / 16 * 16;  // behind the scales
+    v4f* const stash = (v4f*)(lds + STASH_AT) + g * (STASH * 2 * 64) + lane;
+    v4f y[2][NB2 - STASH];  // (a wavefront without channels has sums of zero and scales of zero)
+#pragma unroll
+    for (int b = 0; b < NB2; ++b) {
+        const float rs = scales[lrow + b * 16 + tok];
+        float m = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            // (read again for every 16 rows: with six blocks there is no room for them beside the sums)
+            const v4f s0 = *(const v4f*)(cs + 16 * t + run), s1 = *(const v4f*)(cs + 32 + 16 * t + run);
+            v4f yv;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                float gg = ((float)acc[t][b][j] * rs) * s0[j];
+                float uu = ((float)acc[2 + t][b][j] * rs) * s1[j];
+                if constexpr (LIMIT) {
+                    gg = gg > a.limit ? a.limit : gg;
+                    uu = uu > a.limit ? a.limit : uu;
+                    uu = uu < -a.limit ? -a.limit : uu;
+                }
+                yv[j] = m_silu(gg) * uu;
+            }
+            bool nan = false;  // (arithmetic makes no signalling NaNs)
+            m = max_abs(m, yv, nan);
+            if (b < STASH) stash[(b * 2 + t) * 64] = yv;
+            else y[t][b < STASH ? 0 : b - STASH] = yv;
+        }
+        part[b * 16] = m;
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+    if (tid == 0) *met = 1;
+    float amax = 0.0f;
+    if (tid < rows) {
+#pragma unroll
+        for (int i = 0; i < 4 * GROUPS; ++i) {
+            const float o = ((const float*)lds)[i * ROWS + tid];
+            amax = o > amax ? o : amax;
+        }
+    }
+    if (columns > 1) {
+        __syncthreads();  // (and the note below is reset)
+        uint32_t* const word = a.meet + row0;
+        if (tid < rows)
+            __hip_atomic_store(word + nt * a.R + tid, __float_as_uint(amax) | 1u << 31, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (p.first && p.active) {
+#pragma unroll
+            for (int b = 0; b < NB2; ++b) {
+                const int64_t row = row0 + lrow + b * 16 + tok;
+                if (row >= row_end) continue;
+#pragma unroll
+                for (int t = 0; t < 2; ++t) *(v4f*)(a.y + row * (a.N >> 1) + p.nb0 * 32 + 16 * t + run) = y[t][b < STASH ? 0 : b - STASH];
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+        if (p.first) return;
+        // A look takes what every column has left for one row, until nothing is missing there; what the others have left for the
+        // other rows of the tile came with it or follows at once.
+        const int last = rows > 64 ? rows - 1 : 0;
+        if (tid < 64) {
+            int looks = a.meet_looks;
+            for (; looks > 0; --looks) {
+                const uint32_t w = lane < columns ? look(word + lane * a.R + last) : 1u;
+                if (!__any(w == 0u)) break;
+                __builtin_amdgcn_s_sleep(4);
+            }
+            if (tid == 0 && looks <= 0) *met = 0;
+        }
+        __syncthreads();
+        if (*met && tid < rows) {
+            for (int c = 0, looks = a.meet_looks;;) {
+                uint32_t w[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) w[i] = c + i < columns ? look(word + (c + i) * a.R + tid) : 1u << 31;
+                int here = 0;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    if (here < i || w[i] == 0u) continue;
+                    const float o = __uint_as_float(w[i] & ~(1u << 31));
+                    amax = o > amax ? o : amax;
+                    ++here;
+                }
+                c += here;
+                if (c >= columns) break;
+                if (here < 8 && looks-- <= 0) {
+                    *met = 0;
+                    break;
+                }
+            }
+        }
+        __syncthreads();
+        if (!*met) {
+            for (int c = 0; c < columns; ++c) {
+                if (c == nt) continue;
+                maxima_of_column<LIMIT>(a, p.e, row0, rows, c, 32 * GROUPS, (uint32_t*)lds);
+                if (tid < rows) {
+                    const float o = __uint_as_float(((const uint32_t*)lds)[tid]);
+                    amax = o > amax ? o : amax;
+                }
+                __syncthreads();
+            }
+        }
+    }
+    const int I = a.N >> 1;
+    if (tid < rows) {
+        const float s = amax / 127.0f;
+        scales[tid] = 1.0f / s;
+        if (nt == 0) a.q_scale[row0 + tid] = amax == 0.0f ? 0.0f : s;
+    }
+    __syncthreads();
+    auto quantise_block = [&](bool mine, int block) __attribute__((always_inline)) {
+        if (mine) {
+#pragma unroll
+            for (int b = 0; b < NB2; ++b) {
+                const float by = scales[lrow + b * 16 + tok];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const v4f v = b < STASH ? stash[(b * 2 + t) * 64] : y[t][b < STASH ? 0 : b - STASH];
+                    *(uint32_t*)(lds + (lrow + b * 16 + tok) * PITCH + g * 32 + 16 * t + run) = quantise_times(v, by);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __syncthreads();
+        constexpr int PIECES = 2 * GROUPS;  // of 16 bytes in a row
+        for (int i = tid; i < rows * PIECES; i += (int)blockDim.x) {
+            const int r = i / PIECES, ch = block * 32 * GROUPS + i % PIECES * 16;
+            if (ch < I) store16_through(a.q + (row0 + r) * I + ch, *(const v4i*)(lds + r * PITCH + i % PIECES * 16));
+        }
+    };
+    quantise_block(p.active, nt);
+    if (p.second) {
+        // the column block in front of this one, whose values this wavefront has left in y
+        const bool rows_here = row0 + lrow < row_end;
+        if (rows_here) {
+#pragma unroll
+            for (int b = 0; b < NB2; ++b) {
+                const int64_t row = row0 + lrow + b * 16 + tok;
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const float* from = a.y + (row < row_end ? row : row_end - 1) * I + ((nt - 1) * GROUPS + g) * 32;
+                    y[t][b < STASH ? 0 : b - STASH] = *(const v4f*)(from + 16 * t + run);
+                }
+            }
+        }
+        __syncthreads();  // the pieces of the block before are out of LDS
+        quantise_block(rows_here, nt - 1);
+        if (nt == 1 && tid < rows) a.q_scale[row0 + tid] = amax == 0.0f ? 0.0f : amax / 127.0f;
+    }
+}
+
+template <int NB2, int GROUPS, int ROWS>
+__device__ __forceinline__ void meet_epilogue(const GmmArgs& a, const TilePart& p, v4i (&acc)[4][NB2], int8_t* lds, float* scales)
+{
+    if (a.limit > 0.0f) meet_body<NB2, GROUPS, ROWS, true>(a, p, acc, lds, scales);
+    else meet_body<NB2, GROUPS, ROWS, false>(a, p, acc, lds, scales);
+}
+
 template <int EPI, int BMT, bool IN_LDS = false>
 __device__ __forceinline__ void tiled_epilogue(const GmmArgs& a, int e, v4i (&acc)[4][2 * BMT], int64_t row0,
                                                int64_t row_end, int nb0, int nb1, int8_t* patch, int lane,
@@ -209,7 +454,7 @@ __device__ __forceinline__ void tiled_epilogue(const GmmArgs& a, int e, v4i (&ac
 // streaming kernel uses them.  With several row blocks the others find the weights in L2, and must.
 template <int EPI, int BMT, int RING, int REM, bool ONCE>  // BMT = token blocks of 32 per tile (BM = 32 * BMT)
 __device__ __forceinline__ void tiled_body(const GmmArgs& a, int e, int64_t row0, int64_t row_end, int nt,
-                                           int8_t* lds_raw)
+                                           int8_t* lds_raw, int columns)
 {
     constexpr int STAGE_BYTES = TiledLds<EPI, BMT, RING>::STAGE_BYTES;
     constexpr int CHUNKS = STAGE_BYTES / 16 / 256;        // 16-byte chunks per thread per stage
@@ -226,14 +471,14 @@ __device__ __forceinline__ void tiled_body(const GmmArgs& a, int e, int64_t row0
     const int half_tiles = NB >> 1;
     // storage tiles of this wavefront
     int nb0, nb1;
-    if constexpr (EPI == EPI_SWIGLU) {
+    if constexpr (gated(EPI)) {
         nb0 = nt * 4 + wave;          // gate tile
         nb1 = nb0 + half_tiles;       // its up tile
     } else {
         nb0 = nt * 8 + 2 * wave;
         nb1 = nb0 + 1;
     }
-    const bool have = (EPI == EPI_SWIGLU) ? (nb0 < half_tiles) : (nb1 < NB);
+    const bool have = gated(EPI) ? (nb0 < half_tiles) : (nb1 < NB);
     const int8_t* we = expert_weights(a, e);
     const int8_t* w0 = we + ((int64_t)(have ? nb0 : 0) * KB) * 1024 + weight_lane(lane);
     const int8_t* w1 = we + ((int64_t)(have ? nb1 : 0) * KB) * 1024 + weight_lane(lane);
@@ -395,9 +640,14 @@ __device__ __forceinline__ void tiled_body(const GmmArgs& a, int e, int64_t row0
 #undef MOE355_STEP
 
     __syncthreads();  // all wavefronts are done reading the token stages; LDS is reused below
-    if (!have) return;
-    tiled_epilogue<EPI, BMT, EPI != EPI_I32>(a, e, acc, row0, row_end, nb0, nb1, lds_raw + wave * (PATCHES * 32 * ROWB), lane,
-                                             rs_lds, cs_lds);
+    if constexpr (EPI == EPI_MEET) {
+        meet_epilogue<2 * BMT, 4, 32 * BMT>(a, TilePart{e, 0, wave, nb0, nt, columns, row0, row_end, have, false, false}, acc, lds_raw,
+                                            rs_lds);
+    } else {
+        if (have)
+            tiled_epilogue<EPI, BMT, EPI != EPI_I32>(a, e, acc, row0, row_end, nb0, nb1, lds_raw + wave * (PATCHES * 32 * ROWB), lane,
+                                                     rs_lds, cs_lds);
+    }
 }
 
 // The last tile of an expert is usually short.  Tiles of at most 64 rows run the two-block body (half the
@@ -412,8 +662,10 @@ __global__ __launch_bounds__(256, (BMT <= 2 ? 3 : 2)) void gmm_tiled_kernel(GmmA
     const int total = tm.count[0] * n_col_blocks;
     const int per_xcd = (total + 7) / 8;
     const int slot = (int)(blockIdx.x / 8);
-    const int item = (int)(blockIdx.x % 8) * per_xcd + slot;
-    if (slot >= per_xcd || item >= total) return;
+    const int first = (int)(blockIdx.x % 8) * per_xcd, end = first + per_xcd < total ? first + per_xcd : total;
+    // EPI_MEET: every other XCD takes its share from the end, so that a tile that two XCDs share is worked on by both at once
+    const int item = EPI == EPI_MEET && (blockIdx.x & 1) ? end - 1 - slot : first + slot;
+    if (item < first || item >= end) return;
     const int mt = item / n_col_blocks;
     const int nt = item % n_col_blocks;
     const int e = tm.expert[mt];
@@ -428,15 +680,15 @@ __global__ __launch_bounds__(256, (BMT <= 2 ? 3 : 2)) void gmm_tiled_kernel(GmmA
     const bool once = (mt == 0 || tm.expert[mt - 1] != e) && (mt + 1 == tm.count[0] || tm.expert[mt + 1] != e);
     if (row_end - row0 <= 64) {
         constexpr int SHORT = BMT > 2 ? 2 : BMT;
-        if (once) tiled_body<EPI, SHORT, RING, REM, true>(a, e, row0, row_end, nt, lds_raw);
-        else tiled_body<EPI, SHORT, RING, REM, false>(a, e, row0, row_end, nt, lds_raw);
+        if (once) tiled_body<EPI, SHORT, RING, REM, true>(a, e, row0, row_end, nt, lds_raw, n_col_blocks);
+        else tiled_body<EPI, SHORT, RING, REM, false>(a, e, row0, row_end, nt, lds_raw, n_col_blocks);
         return;
     }
     // With a short K full tiles that way only where they are many: a few among short ones are the last to end.  128 experts of
     // 2048 / 768, the layer with non-temporal / plain full tiles at 49 / 53 / 59 / 66 / 75 rows per expert 1.01 / 1.01 / 0.98 /
     // 0.97 / 0.97; 256 experts of 7168 / 2048, 47 rows 0.98.
-    if (once && (a.K >= 4096 || a.R >= 56 * (int64_t)a.E)) tiled_body<EPI, BMT, RING, REM, true>(a, e, row0, row_end, nt, lds_raw);
-    else tiled_body<EPI, BMT, RING, REM, false>(a, e, row0, row_end, nt, lds_raw);
+    if (once && (a.K >= 4096 || a.R >= 56 * (int64_t)a.E)) tiled_body<EPI, BMT, RING, REM, true>(a, e, row0, row_end, nt, lds_raw, n_col_blocks);
+    else tiled_body<EPI, BMT, RING, REM, false>(a, e, row0, row_end, nt, lds_raw, n_col_blocks);
 }
 
 // ------------------------------------------------------------------ weight-streaming tiles
@@ -474,7 +726,8 @@ __device__ __forceinline__ void wait_vmcnt()
 // 1328 / 1362 -> 1175 / 1333 us; 2048 / 7168, 128 rows 757 -> 696.
 template <int EPI, bool WIDE, int NBLK = 4>
 __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_t row0, int64_t row_end, int nt,
-                                                 bool once, int8_t* lds)
+                                                 bool once, int8_t* lds, int columns = 0, bool first = false,
+                                                 bool second = false)
 {
     static_assert(WIDE ? (NBLK >= 1 && NBLK <= 8) : NBLK == 4, "tall tiles have two halves of four blocks");
     constexpr int GROUPS = WIDE ? 8 : 4;            // channel groups (two storage tiles each) per workgroup
@@ -501,7 +754,7 @@ __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_
     const int NB = a.N >> 5, KB = a.K >> 5;
     const int half_tiles = NB >> 1;
     auto tiles_of = [&](int cg, int& t0, int& t1) -> bool {
-        if constexpr (EPI == EPI_SWIGLU) {
+        if constexpr (gated(EPI)) {
             t0 = cg;
             t1 = cg + half_tiles;
             return cg < half_tiles;
@@ -592,6 +845,19 @@ __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_
     for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int b = 0; b < 2 * NBLK; ++b) acc[t][b] = (v4i){0};
+
+    // the scales of the epilogue, in front of everything else in the queue of answers
+    constexpr int ROWS = WIDE ? 32 * NBLK : 256;
+    float rs_own = 0.0f, cs_own = 0.0f;
+    if constexpr (EPI == EPI_MEET) {
+        if ((int)threadIdx.x < ROWS) {
+            int64_t r = row0 + threadIdx.x < row_end ? row0 + threadIdx.x : row_end - 1;
+            if (a.row_src) r = a.row_src[r];
+            rs_own = a.row_scale[r];
+        }
+        if (have) cs_own = expert_scales(a, e)[(lane < 32 ? nb0 * 32 : nb1 * 32 - 32) + lane];
+        asm volatile("" : "+v"(rs_own), "+v"(cs_own));  // (here: the waits below count what is requested behind it)
+    }
 
     // Every step requests the tokens SX - 1 steps ahead and then the weights SW - 1 steps ahead; the steps before
     // the first one do the same for what lies at or after K block 0, so that the order of the requests, which the
@@ -746,8 +1012,19 @@ __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_
 
     wait_vmcnt<0>();  // the redirected loads past the end still write LDS
     __builtin_amdgcn_s_barrier();
-    if (!active) return;
-    tiled_epilogue<EPI, NBLK>(a, e, acc, hrow0, row_end, nb0, nb1, lds + wave * (PATCHES * 32 * ROWB), lane);
+    if constexpr (EPI == EPI_MEET) {
+        constexpr int SCALES = ROWS * (32 * GROUPS + 16);
+        static_assert(16 * GROUPS * ROWS <= SCALES && SCALES + (ROWS + GROUPS * 64) * 4 + 16 + (NBLK > 4 ? 65536 : 0) <= kWideLdsBytes &&
+                      ROWS <= 512, "maxima, rows, scales and values fit LDS; a thread for every row");
+        float* const scales = (float*)(lds + SCALES);
+        if ((int)threadIdx.x < ROWS) scales[threadIdx.x] = rs_own;
+        if (WIDE || h == 0) scales[ROWS + g * 64 + lane] = cs_own;
+        __syncthreads();
+        meet_epilogue<2 * NBLK, GROUPS, ROWS>(a, TilePart{e, 128 * h, g, nb0, nt, columns, row0, row_end, active, first, second}, acc,
+                                              lds, scales);
+    } else {
+        if (active) tiled_epilogue<EPI, NBLK>(a, e, acc, hrow0, row_end, nb0, nb1, lds + wave * (PATCHES * 32 * ROWB), lane);
+    }
 }
 
 template <int EPI>
@@ -775,23 +1052,24 @@ __global__ __launch_bounds__(512, 1) void gmm_wide_kernel(GmmArgs a, TileMap tm,
     // An expert of a few rows (the cold ones of a skewed batch) runs the same body with one or two token blocks:
     // the matrix units draw their power whether a block's rows exist or not, and the kernel's clock follows it.
     if (row_end - row0 <= 32) {
-        stream_tile_body<EPI, true, 1>(a, e, row0, row_end, col, once, wide_lds);
+        stream_tile_body<EPI, true, 1>(a, e, row0, row_end, col, once, wide_lds, columns);
     } else if (row_end - row0 <= 64) {
-        stream_tile_body<EPI, true, 2>(a, e, row0, row_end, col, once, wide_lds);
+        stream_tile_body<EPI, true, 2>(a, e, row0, row_end, col, once, wide_lds, columns);
     } else if (row_end - row0 <= 128) {
-        stream_tile_body<EPI, true>(a, e, row0, row_end, col, once, wide_lds);
+        stream_tile_body<EPI, true>(a, e, row0, row_end, col, once, wide_lds, columns);
     } else if (row_end - row0 <= 160) {
-        stream_tile_body<EPI, true, 5>(a, e, row0, row_end, col, once, wide_lds);
+        stream_tile_body<EPI, true, 5>(a, e, row0, row_end, col, once, wide_lds, columns);
     } else if (row_end - row0 <= 192) {
-        stream_tile_body<EPI, true, 6>(a, e, row0, row_end, col, once, wide_lds);
+        stream_tile_body<EPI, true, 6>(a, e, row0, row_end, col, once, wide_lds, columns);
     } else {
         // a tall tile is one column block wide: the column's two blocks have an entry each, or are done one after the other
         const bool second = listed & kSecondHalf;
         if (second && 2 * col + 1 >= n_col_blocks) return;
-        stream_tile_body<EPI, false>(a, e, row0, row_end, second ? 2 * col + 1 : 2 * col, once, wide_lds);
-        if (!(listed & (kFirstHalf | kSecondHalf)) && 2 * col + 1 < n_col_blocks) {
+        const bool two = !(listed & (kFirstHalf | kSecondHalf)) && 2 * col + 1 < n_col_blocks;
+        stream_tile_body<EPI, false>(a, e, row0, row_end, second ? 2 * col + 1 : 2 * col, once, wide_lds, n_col_blocks, two);
+        if (two) {
             __syncthreads();  // the first block's epilogue is out of LDS
-            stream_tile_body<EPI, false>(a, e, row0, row_end, 2 * col + 1, once, wide_lds);
+            stream_tile_body<EPI, false>(a, e, row0, row_end, 2 * col + 1, once, wide_lds, n_col_blocks, false, true);
         }
     }
 }
@@ -849,8 +1127,8 @@ static void launch_tiled(const GmmArgs& a, void* workspace, hipStream_t st, hipE
     const int max_tiles = spec.max_tiles;
     if (!a.tiles_ready)
         hipLaunchKernelGGL(tile_map_kernel, dim3(1), dim3(256), 0, st, a.gl, a.gl_type, a.E, spec);
-    const int channels = (EPI == EPI_SWIGLU) ? a.N / 2 : a.N;
-    const int per_block = (EPI == EPI_SWIGLU) ? kBN / 2 : kBN;
+    const int channels = gated(EPI) ? a.N / 2 : a.N;
+    const int per_block = gated(EPI) ? kBN / 2 : kBN;
     const int n_col_blocks = (channels + per_block - 1) / per_block;
     const int total = max_tiles * n_col_blocks;
     const int grid = ((total + 7) / 8) * 8;
@@ -880,8 +1158,8 @@ static bool launch_wide(const GmmArgs& a, void* workspace, hipStream_t st, hipEv
     const int max_tiles = spec.max_tiles;
     if (!a.tiles_ready)
         hipLaunchKernelGGL(tile_map_kernel, dim3(1), dim3(256), 0, st, a.gl, a.gl_type, a.E, spec);
-    const int channels = (EPI == EPI_SWIGLU) ? a.N / 2 : a.N;
-    const int per_block = (EPI == EPI_SWIGLU) ? kBN / 2 : kBN;
+    const int channels = gated(EPI) ? a.N / 2 : a.N;
+    const int per_block = gated(EPI) ? kBN / 2 : kBN;
     const int n_col_blocks = (channels + per_block - 1) / per_block;
     const int columns = (n_col_blocks + 1) / 2;
     const int grid = 8 * ((max_tiles + 7) / 8) * columns;  // one workgroup per (tile, column), no idle ones
@@ -938,11 +1216,13 @@ bool launch_tiled_any(int epi, int bm, const GmmArgs& a, void* workspace, hipStr
     if (bm == 256) {
         if (epi == EPI_I32) return launch_wide<EPI_I32>(a, workspace, st, ev0, ev1);
         if (epi == EPI_SWIGLU) return launch_wide<EPI_SWIGLU>(a, workspace, st, ev0, ev1);
+        if (epi == EPI_MEET) return launch_wide<EPI_MEET>(a, workspace, st, ev0, ev1);
         return launch_wide<EPI_DEQUANT>(a, workspace, st, ev0, ev1);
     }
     if (bm == 128) {
         if (epi == EPI_I32) MOE355_TILED(EPI_I32, 4);
         else if (epi == EPI_SWIGLU) MOE355_TILED(EPI_SWIGLU, 4);
+        else if (epi == EPI_MEET) MOE355_TILED(EPI_MEET, 4);
         else if (resident_supported(a)) {
             if (!a.tiles_ready) {
                 const TileSpec spec = tile_spec(a.R, a.E, bm, workspace);
@@ -953,6 +1233,7 @@ bool launch_tiled_any(int epi, int bm, const GmmArgs& a, void* workspace, hipStr
     } else {
         if (epi == EPI_I32) MOE355_TILED(EPI_I32, 2);
         else if (epi == EPI_SWIGLU) MOE355_TILED(EPI_SWIGLU, 2);
+        else if (epi == EPI_MEET) MOE355_TILED(EPI_MEET, 2);
         else MOE355_TILED(EPI_DEQUANT, 2);
     }
 #undef MOE355_TILED

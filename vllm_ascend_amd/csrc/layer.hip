@@ -38,6 +38,8 @@ struct Buffers {
     float* ymax;  // a few tokens: maxima of the SwiGLU values, 16 at a time
     int32_t* dst;
     int32_t* row_token;
+    MeetingPlan plan;
+    uint32_t* meet;  // [plan.columns][R]
     void* map_ws;
     float* logits;
     void* gate_ws;
@@ -189,6 +191,8 @@ Buffers lay_out(const moe355_layer& l, const Forms& f, int64_t T, void* base)
     } else {
         b.dst = a.take<int32_t>((size_t)R * 4);
         b.row_token = a.take<int32_t>((size_t)R * 4);
+        if (l.weights != W_INT4) b.plan = meeting_plan(R, H, 2 * I, E);
+        b.meet = a.take<uint32_t>((size_t)R * 4 * b.plan.columns);
         b.map_bytes = moe355_init_routing_workspace(T, l.top_k, E);
         b.map_ws = a.take<void>(b.map_bytes);
         // the down GEMM writes its rows where the SwiGLU values were: those are dead once re-quantised
@@ -337,7 +341,7 @@ int routed_sorted(const moe355_layer& l, const Buffers& b, int64_t T, bool tiles
     rc = gmm1_impl(b.xq, list ? nullptr : (const int8_t*)l.w13, list ? (const int8_t* const*)l.w13 : nullptr,
                    list ? nullptr : (const float*)l.s13, list ? (const float* const*)l.s13 : nullptr, b.x_scale,
                    b.expert_tokens, MOE355_GL_COUNT, R, H, 2 * I, E, l.swiglu_limit, b.q1, b.q1_scale, b.mlp_ws,
-                   b.mlp_bytes, st, b.row_token, tiles_ready);
+                   b.mlp_bytes, st, b.row_token, tiles_ready, b.plan, b.meet);
     if (rc != MOE355_OK) return rc;
     return gmm2_impl(b.q1, list ? nullptr : (const int8_t*)l.w2, list ? (const int8_t* const*)l.w2 : nullptr,
                      list ? nullptr : (const float*)l.s2, list ? (const float* const*)l.s2 : nullptr, b.q1_scale,
@@ -445,11 +449,11 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
             specs[n++] = w4_chunk_spec(R, l.num_experts, b.gmm2_ws);
         } else {
             n = gemm_tile_specs(R, l.hidden, 2 * l.intermediate, l.num_experts,
-                                gmm1_tile_ws(b.mlp_ws, R, 2 * l.intermediate), specs);
+                                gmm1_tile_ws(b.mlp_ws, R, 2 * l.intermediate), specs, b.plan.tile_rows);
             n += gemm_tile_specs(R, l.intermediate, l.hidden, l.num_experts, b.gmm2_ws, specs + n);
         }
         rc = route_map_impl(b.topk_ids, T, l.top_k, l.num_experts, 1, b.dst, b.row_token, b.expert_tokens, b.map_ws,
-                            b.map_bytes, specs, n, &tiles_ready, stream);
+                            b.map_bytes, specs, n, &tiles_ready, stream, b.meet, b.plan.columns);
     }
     if (rc == MOE355_OK) {
         (void)moe355_profile_next_gemm(ev0, ev1);

@@ -87,11 +87,18 @@ int gmm1_pairs_impl(const int8_t* x, const float* x_scale, const int32_t* topk_i
 int gmm2_pairs_impl(const int8_t* x, const float* per_token_scale, const float* y, const PairWeights& w,
                     const int32_t* topk_ids, int64_t num_tokens, int top_k, int64_t k, int64_t n, int num_experts,
                     void* out, int out_dtype, void* stream, const PairShared* shared = nullptr);
+// the gate_up product whose tiles' workgroups exchange the rows' maxima: rows of its tiles and workgroups of a tile (0: they do not),
+// a word for each of them and every row in `meet`, cleared before the launch
+struct MeetingPlan {
+    int tile_rows = 0, columns = 0;
+};
+MeetingPlan meeting_plan(int64_t rows, int64_t k, int64_t n, int num_experts);
+// plan, meet: used where the tile map is ready
 int gmm1_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list, const float* weight_scale,
               const float* const* scale_list, const float* x_scale, const int64_t* group_list, int group_list_type,
               int64_t rows, int64_t k, int64_t n, int num_experts, float swiglu_limit, int8_t* out, float* out_scale,
               void* workspace, size_t workspace_bytes, void* stream, const int32_t* row_src = nullptr,
-              bool tiles_ready = false);
+              bool tiles_ready = false, const MeetingPlan& plan = {}, uint32_t* meet = nullptr);
 // beside: the launch runs on a side stream, beside long products of the routed experts
 int gmm2_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list, const float* scale,
               const float* const* scale_list, const float* per_token_scale, const int64_t* group_list,
@@ -102,7 +109,7 @@ int gmm_i32_impl(const int8_t* x, const int8_t* weight_nz, const int64_t* group_
                  bool beside);
 void* gmm1_tile_ws(void* workspace, int64_t rows, int64_t n);
 // the tile map (0 or 1) that a grouped product will look for in its workspace
-int gemm_tile_specs(int64_t rows, int64_t k, int64_t n, int num_experts, void* tile_ws, TileSpec* specs);
+int gemm_tile_specs(int64_t rows, int64_t k, int64_t n, int num_experts, void* tile_ws, TileSpec* specs, int tile_rows = 0);
 
 // int4 weights, sorted rows (gmm_w4.hip): the chunks of both products in the order they run in, for the routing launch to build
 // in a workspace of tiled_workspace_bytes(rows, E, 64); without it (null) every workgroup finds its chunk from the group list
@@ -126,10 +133,11 @@ int gmm2_w4_pairs(const int8_t* x, const float* x_scale, const int32_t* topk_ids
                   int out_dtype, hipStream_t st);
 
 // moe355_route_map with the tile maps of the two products (nspecs of them, at most 2) built by the same launch where it
-// is one launch (returns 1 in *built then)
+// is one launch (returns 1 in *built then), which also clears zeros_per_pair words for every pair
 int route_map_impl(const int32_t* expert_idx, int64_t num_tokens, int top_k, int num_experts, int tokens_num_type,
                    int32_t* expanded_row_idx, int32_t* row_token, int64_t* expert_tokens, void* workspace,
-                   size_t workspace_bytes, const TileSpec* specs, int nspecs, bool* built, void* stream);
+                   size_t workspace_bytes, const TileSpec* specs, int nspecs, bool* built, void* stream, uint32_t* zeros = nullptr,
+                   int zeros_per_pair = 0);
 
 // ------------------------------------------------------------------ a few tokens (few.hip)
 // n / d for n and d below 2^16 in one multiplication (an integer division is about 25 instructions, one after the other)

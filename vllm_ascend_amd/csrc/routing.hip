@@ -321,6 +321,8 @@ __global__ __launch_bounds__(256) void route_gather_small_kernel(const int32_t* 
 // come from per-wavefront counts and ballots.  Further workgroups build the tile maps of the grouped GEMMs behind it
 // (launches of 4.5 us each otherwise): they do the same counting for their row counts.
 struct RouteMapArgs {
+    uint32_t* zeros;      // [zeros_per_pair][R] cleared for the launches behind this one
+    int zeros_per_pair;
     const int32_t* ids;
     int R, E, top_k, tokens_num_type, nbits, chunks, nspecs, columns;
     int32_t* dst;
@@ -356,6 +358,8 @@ __global__ __launch_bounds__(kMapThreads) void route_map_kernel(RouteMapArgs a)
     int32_t* whist = part + 32;            // [16][E] pairs of every wavefront, then the first row of its pairs
     const bool maps = (int)blockIdx.x >= a.chunks;  // a tile map instead of a chunk
     const int begin = maps ? 0 : (int)blockIdx.x * kMapThreads;
+    if (!maps && begin + tid < R)  // (zeros is null where there are none)
+        for (int c = 0; c < a.zeros_per_pair; ++c) a.zeros[(int64_t)c * R + begin + tid] = 0u;
     for (int i = tid; i < (MANY ? E * columns : E); i += kMapThreads) map_lds[i] = 0;
     if (!maps)
         for (int i = tid; i < kMapWaves * E; i += kMapThreads) whist[i] = 0;
@@ -615,7 +619,7 @@ extern "C" int moe355_init_routing(const void* x, int x_dtype, int64_t num_token
 int moe355::route_map_impl(const int32_t* expert_idx, int64_t num_tokens, int top_k, int num_experts,
                            int tokens_num_type, int32_t* expanded_row_idx, int32_t* row_token, int64_t* expert_tokens,
                            void* workspace, size_t workspace_bytes, const TileSpec* specs, int nspecs, bool* built,
-                           void* stream)
+                           void* stream, uint32_t* zeros, int zeros_per_pair)
 {
     if (built) *built = false;
     if (num_tokens < 0 || top_k <= 0 || num_experts <= 0) return MOE355_E_ARG;
@@ -643,6 +647,8 @@ int moe355::route_map_impl(const int32_t* expert_idx, int64_t num_tokens, int to
         a.dst = expanded_row_idx;
         a.row_token = row_token;
         a.expert_tokens = expert_tokens;
+        a.zeros = zeros;
+        a.zeros_per_pair = zeros_per_pair;
         for (int i = 0; i < nspecs; ++i) a.specs[i] = specs[i];
         const bool many = R >= 20480;
         a.columns = many ? (num_experts <= 256 ? 16 : 8) : 0;
