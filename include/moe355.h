@@ -504,8 +504,8 @@ int moe355_profile_next_gemm(void *start_event, void *stop_event);
 
 /* On the sorted path of moe355_layer_forward the workgroups of a tile of the gate_up product can exchange the maxima of its rows
  * and quantise them in place: the rows of those tiles, or 0 where the fp32 values go through memory and a launch of their own.
- * A workgroup that has looked for the others' maxima some thousand times computes them itself; the next such product that the
- * calling thread launches gives up after `looks` instead (0: at once).  The results are the same either way.
+ * A workgroup that has looked for the others' maxima some thousand times computes them itself; in the next layer call of the
+ * calling thread it gives up after `looks` instead (0: at once).  The results are the same either way.
  */
 int moe355_meeting_tile_rows(int64_t rows, int64_t k, int64_t n, int num_experts);
 int moe355_next_meeting_looks(int looks);

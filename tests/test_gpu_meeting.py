@@ -113,3 +113,28 @@ def test_captured_and_from_two_streams():
             beside = [layer(x, logits) for _ in range(3)]
         torch.cuda.synchronize()
         assert torch.equal(out, want) and all(torch.equal(b, want) for b in beside)
+
+
+# the shared expert of a prefill batch, 256 x 256 tiles: whole and partial row tiles and column blocks, one round of workgroups
+# and several, as many columns as meet and one more, words of the meeting that do and do not fill whole rows of the routed experts' pairs, beside int4 experts
+@pytest.mark.parametrize("T, S, H, k, w4", [
+    (3072, 2048, 64, 2, False), (3007, 2016, 192, 3, False), (12200, 512, 128, 1, False), (6001, 1984, 256, 8, False), (3009, 2048, 128, 2, True),
+    (700, 8192, 64, 2, False), (700, 8224, 64, 2, False)])
+@pytest.mark.parametrize("limit", [0.0, 0.7])
+def test_shared_expert_on_dense_tiles(T, S, H, k, w4, limit):
+    from vllm_ascend_amd.fused_moe.shared_experts import AscendSharedExperts
+
+    print(f"T={T} S={S} H={H} k={k} w4={w4} limit={limit}", flush=True)
+    assert -(-T // 256) * -(-2 * S // 256) >= 192
+    cfg = dataclasses.replace(CONFIGS["c5_small_perchannel" if w4 else "c2_small"], T=T, E=8, k=k, H=H, I=64)
+    d = make_layer(cfg, seed=T)
+    layer = build_layer(cfg, d, DEV)
+    g = torch.Generator(device=DEV).manual_seed(T)
+    up, down = (torch.randint(-128, 128, shape, generator=g, device=DEV, dtype=torch.int8) for shape in ((2 * S, H), (H, S)))
+    up_scale, down_scale = (torch.rand(n, generator=g, device=DEV) * 0.009 + 0.001 for n in (2 * S, H))
+    layer.shared_experts = AscendSharedExperts(up, up_scale, down, down_scale, swiglu_limit=limit)
+    x = d["x"].to(DEV).clone()
+    x[3] = 0
+    x[70] = float("inf")
+    x[300] *= 1e30
+    _check(layer, x, d["logits"].to(DEV), looks=(None, 0, 1))

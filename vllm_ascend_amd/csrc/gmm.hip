@@ -508,7 +508,7 @@ __global__ __launch_bounds__(256) void swiglu_requant_kernel(const float* __rest
     if (lane == 0) qs[row] = (amax == 0.0f) ? 0.0f : s;
     uint32_t* qr = (uint32_t*)(q + row * I);
     auto pack = [&](v4f v) {
-        if (shared) return pack_low_bytes(sat_rint(v[0] / s), sat_rint(v[1] / s), sat_rint(v[2] / s), sat_rint(v[3] / s));
+        if (shared) return quantise_over(v, s);
         return quantise_times(v, inv);
     };
     if constexpr (NV > 0) {
@@ -1009,6 +1009,13 @@ extern "C" size_t moe355_gmm1_swiglu_quant_workspace(int64_t rows, int64_t n, in
 constexpr int kMeetLooks = 4096;
 static thread_local int t_meet_looks = kMeetLooks;
 
+int moe355::take_meeting_looks()
+{
+    const int looks = t_meet_looks;
+    t_meet_looks = kMeetLooks;
+    return looks;
+}
+
 extern "C" int moe355_next_meeting_looks(int looks)
 {
     if (looks < 0) return MOE355_E_ARG;
@@ -1068,6 +1075,50 @@ extern "C" int moe355_meeting_tile_rows(int64_t rows, int64_t k, int64_t n, int 
     return moe355::meeting_plan(rows, k, n, num_experts).tile_rows;
 }
 
+// The shared expert's gate_up product in line, on the dense tiles.  Without the meeting its int32 sums pass through memory (67 MB each
+// way for 4096 rows of 4096 channels; the product and the launch that quantises 109 + 25 us, together 117).  The layer without / with,
+// us: 256 experts of 7168 / 2048, 4096 / 5000 / 6000 / 7000 / 8192 tokens 2641 / 2855 / 3328 / 3828 / 4519 and 2617 / 2839 / 3289 / 3799 /
+// 4500, Zipf(1.1) 4096 2591 and 2557, int4 4096 2713 and 2698; 64 experts of 2048 / 2048, 4096 / 8000 tokens 674 / 1174 and 656 / 1142, of
+// 4096 / 1024, 8192 tokens 1214 and 1198.  The columns need not divide an XCD's 32 places here (64 of 4096 / 1536, 4096 / 7000 tokens
+// 1014 / 1596 and 1000 / 1579; 2048 / 2816, 4500 1071 and 1052; 7168 / 2560, 4096 2537 and 2532; 7168 / 1408, 8192 2973 and 2959): the
+// rectangles keep them close.  64 are what a wavefront looks at at once.
+int moe355::shared_meeting_columns(int64_t rows, int64_t k, int64_t n)
+{
+    GmmArgs a = {};
+    a.R = rows;
+    a.K = (int)k;
+    a.N = (int)n;
+    a.E = 1;
+    const int64_t columns = (n / 2 + 127) / 128;
+    return columns <= 64 && dense_tiles(a) ? (int)columns : 0;
+}
+
+int moe355::shared_meeting_impl(const int8_t* x, const int8_t* weight_nz, const float* weight_scale, const float* x_scale,
+                                const int64_t* group_list, int64_t rows, int64_t k, int64_t n, float limit, uint32_t* meet,
+                                int looks, int8_t* out, float* out_scale, void* stream)
+{
+    int rc = check_gmm(x, weight_nz, group_list, MOE355_GL_CUMSUM, rows, k, n, 1);
+    if (rc != MOE355_OK) return rc;
+    if (((uintptr_t)weight_scale & 15) || ((uintptr_t)out & 15)) return MOE355_E_SHAPE;
+    GmmArgs a = {};
+    a.x = x;
+    a.w = weight_nz;
+    a.gl = group_list;
+    a.gl_type = MOE355_GL_CUMSUM;
+    a.R = rows;
+    a.K = (int)k;
+    a.N = (int)n;
+    a.E = 1;
+    a.row_scale = x_scale;
+    a.ch_scale = weight_scale;
+    a.limit = limit;
+    a.meet = meet;
+    a.meet_looks = looks;
+    a.q = out;
+    a.q_scale = out_scale;
+    return launched(launch_dense(EPI_MEET_SHARED, a, (hipStream_t)stream, nullptr, nullptr));
+}
+
 int moe355::gmm1_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list,
                       const float* weight_scale, const float* const* scale_list, const float* x_scale,
                       const int64_t* group_list, int group_list_type, int64_t rows, int64_t k, int64_t n,
@@ -1107,8 +1158,7 @@ int moe355::gmm1_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* co
     void* tile_ws = gmm1_tile_ws(workspace, rows, n);
     if (tiles_ready && plan.columns) {
         a.meet = meet;
-        a.meet_looks = t_meet_looks;
-        t_meet_looks = kMeetLooks;
+        a.meet_looks = plan.looks;
         a.q = out;
         a.q_scale = out_scale;
         hipEvent_t ev0, ev1;

@@ -14,10 +14,13 @@
 
 namespace moe355 {
 
-enum { EPI_I32 = 0, EPI_SWIGLU = 1, EPI_DEQUANT = 2, EPI_MEET = 3 };
+enum { EPI_I32 = 0, EPI_SWIGLU = 1, EPI_DEQUANT = 2, EPI_MEET = 3, EPI_MEET_SHARED = 4 };
 
 // EPI_MEET: SwiGLU and the rows' quantisation; the workgroups of a tile exchange the maxima of its rows (gmm_tiled.hip)
-constexpr bool gated(int epi) { return epi == EPI_SWIGLU || epi == EPI_MEET; }
+// EPI_MEET_SHARED: the same with the shared expert's arithmetic (dequant_swiglu_quant_kernel, form_b): the channel's scale before the
+// row's, scale = maximum * (1 / 127), values divided by it
+constexpr bool meets(int epi) { return epi == EPI_MEET || epi == EPI_MEET_SHARED; }
+constexpr bool gated(int epi) { return epi == EPI_SWIGLU || meets(epi); }
 
 struct GmmArgs {
     const int8_t* x;        // [R, K]

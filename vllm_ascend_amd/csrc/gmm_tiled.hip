@@ -204,9 +204,16 @@ __device__ __forceinline__ uint32_t look(const uint32_t* p)
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// a sum with its scales, in the order of the routed experts or of the shared one
+template <bool SHARED>
+__device__ __forceinline__ float scaled(int sum, float rs, float cs)
+{
+    return SHARED ? ((float)sum * cs) * rs : ((float)sum * rs) * cs;
+}
+
 // The maxima of the tile's rows over column block c, by the workgroup itself and one product after the other: only where the
 // workgroup that is meant for that block has not come.  sum: rows words of LDS
-template <bool LIMIT>
+template <bool LIMIT, bool SHARED>
 __device__ __forceinline__ void maxima_of_column(const GmmArgs& a, int e, int64_t row0, int rows, int c, int channels, uint32_t* sum)
 {
     for (int i = threadIdx.x; i < rows; i += (int)blockDim.x) sum[i] = 0u;
@@ -229,7 +236,7 @@ __device__ __forceinline__ void maxima_of_column(const GmmArgs& a, int e, int64_
             g = add(ch, g);
             u = add(ch + I, u);
         }
-        float gg = ((float)g * a.row_scale[src]) * cs[ch], uu = ((float)u * a.row_scale[src]) * cs[ch + I];
+        float gg = scaled<SHARED>(g, a.row_scale[src], cs[ch]), uu = scaled<SHARED>(u, a.row_scale[src], cs[ch + I]);
         if constexpr (LIMIT) {
             gg = gg > a.limit ? a.limit : gg;
             uu = uu > a.limit ? a.limit : uu;
@@ -253,7 +260,7 @@ struct TilePart {
 // acc: the wavefront's 16 NB2 rows.  lds: ROWS * (32 GROUPS + 16) bytes (the maxima of every quarter of a wavefront, then the int8
 // rows), behind them 64 KiB for the values of the widest tiles.  scales: those of the rows (ROWS of them), then 64 of the channels for
 // each group.
-template <int NB2, int GROUPS, int ROWS, bool LIMIT>
+template <int NB2, int GROUPS, int ROWS, bool LIMIT, bool SHARED>
 __device__ __forceinline__ void meet_body(const GmmArgs& a, const TilePart& p, v4i (&acc)[4][NB2], int8_t* lds, float* scales)
 {
     constexpr int PITCH = 32 * GROUPS + 16;
@@ -281,8 +288,8 @@ __device__ __forceinline__ void meet_body(const GmmArgs& a, const TilePart& p, v
             v4f yv;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                float gg = ((float)acc[t][b][j] * rs) * s0[j];
-                float uu = ((float)acc[2 + t][b][j] * rs) * s1[j];
+                float gg = scaled<SHARED>(acc[t][b][j], rs, s0[j]);
+                float uu = scaled<SHARED>(acc[2 + t][b][j], rs, s1[j]);
                 if constexpr (LIMIT) {
                     gg = gg > a.limit ? a.limit : gg;
                     uu = uu > a.limit ? a.limit : uu;
@@ -362,7 +369,7 @@ __device__ __forceinline__ void meet_body(const GmmArgs& a, const TilePart& p, v
         if (!*met) {
             for (int c = 0; c < columns; ++c) {
                 if (c == nt) continue;
-                maxima_of_column<LIMIT>(a, p.e, row0, rows, c, 32 * GROUPS, (uint32_t*)lds);
+                maxima_of_column<LIMIT, SHARED>(a, p.e, row0, rows, c, 32 * GROUPS, (uint32_t*)lds);
                 if (tid < rows) {
                     const float o = __uint_as_float(((const uint32_t*)lds)[tid]);
                     amax = o > amax ? o : amax;
@@ -373,8 +380,8 @@ __device__ __forceinline__ void meet_body(const GmmArgs& a, const TilePart& p, v
     }
     const int I = a.N >> 1;
     if (tid < rows) {
-        const float s = amax / 127.0f;
-        scales[tid] = 1.0f / s;
+        const float s = SHARED ? amax * (float)(1.0 / 127.0) : amax / 127.0f;
+        scales[tid] = SHARED ? s : 1.0f / s;
         if (nt == 0) a.q_scale[row0 + tid] = amax == 0.0f ? 0.0f : s;
     }
     __syncthreads();
@@ -386,7 +393,8 @@ __device__ __forceinline__ void meet_body(const GmmArgs& a, const TilePart& p, v
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
                     const v4f v = b < STASH ? stash[(b * 2 + t) * 64] : y[t][b < STASH ? 0 : b - STASH];
-                    *(uint32_t*)(lds + (lrow + b * 16 + tok) * PITCH + g * 32 + 16 * t + run) = quantise_times(v, by);
+                    *(uint32_t*)(lds + (lrow + b * 16 + tok) * PITCH + g * 32 + 16 * t + run) =
+                        SHARED ? quantise_over(v, by) : quantise_times(v, by);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -419,11 +427,11 @@ __device__ __forceinline__ void meet_body(const GmmArgs& a, const TilePart& p, v
     }
 }
 
-template <int NB2, int GROUPS, int ROWS>
+template <int NB2, int GROUPS, int ROWS, bool SHARED = false>
 __device__ __forceinline__ void meet_epilogue(const GmmArgs& a, const TilePart& p, v4i (&acc)[4][NB2], int8_t* lds, float* scales)
 {
-    if (a.limit > 0.0f) meet_body<NB2, GROUPS, ROWS, true>(a, p, acc, lds, scales);
-    else meet_body<NB2, GROUPS, ROWS, false>(a, p, acc, lds, scales);
+    if (a.limit > 0.0f) meet_body<NB2, GROUPS, ROWS, true, SHARED>(a, p, acc, lds, scales);
+    else meet_body<NB2, GROUPS, ROWS, false, SHARED>(a, p, acc, lds, scales);
 }
 
 template <int EPI, int BMT, bool IN_LDS = false>
@@ -849,7 +857,7 @@ __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_
     // the scales of the epilogue, in front of everything else in the queue of answers
     constexpr int ROWS = WIDE ? 32 * NBLK : 256;
     float rs_own = 0.0f, cs_own = 0.0f;
-    if constexpr (EPI == EPI_MEET) {
+    if constexpr (meets(EPI)) {
         if ((int)threadIdx.x < ROWS) {
             int64_t r = row0 + threadIdx.x < row_end ? row0 + threadIdx.x : row_end - 1;
             if (a.row_src) r = a.row_src[r];
@@ -1012,7 +1020,7 @@ __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_
 
     wait_vmcnt<0>();  // the redirected loads past the end still write LDS
     __builtin_amdgcn_s_barrier();
-    if constexpr (EPI == EPI_MEET) {
+    if constexpr (meets(EPI)) {
         constexpr int SCALES = ROWS * (32 * GROUPS + 16);
         static_assert(16 * GROUPS * ROWS <= SCALES && SCALES + (ROWS + GROUPS * 64) * 4 + 16 + (NBLK > 4 ? 65536 : 0) <= kWideLdsBytes &&
                       ROWS <= 512, "maxima, rows, scales and values fit LDS; a thread for every row");
@@ -1020,8 +1028,8 @@ __device__ __forceinline__ void stream_tile_body(const GmmArgs& a, int e, int64_
         if ((int)threadIdx.x < ROWS) scales[threadIdx.x] = rs_own;
         if (WIDE || h == 0) scales[ROWS + g * 64 + lane] = cs_own;
         __syncthreads();
-        meet_epilogue<2 * NBLK, GROUPS, ROWS>(a, TilePart{e, 128 * h, g, nb0, nt, columns, row0, row_end, active, first, second}, acc,
-                                              lds, scales);
+        const TilePart part = {e, 128 * h, g, nb0, nt, columns, row0, row_end, active, first, second};
+        meet_epilogue<2 * NBLK, GROUPS, ROWS, EPI == EPI_MEET_SHARED>(a, part, acc, lds, scales);
     } else {
         if (active) tiled_epilogue<EPI, NBLK>(a, e, acc, hrow0, row_end, nb0, nb1, lds + wave * (PATCHES * 32 * ROWB), lane);
     }
@@ -1093,7 +1101,7 @@ __global__ __launch_bounds__(512, 1) void gmm_dense_kernel(GmmArgs a, int xn, in
     if (rows > a.R) rows = a.R;
     const int64_t row0 = (int64_t)mt * 256;
     if (row0 >= rows) return;
-    stream_tile_body<EPI, false>(a, 0, row0, rows, nt, false, wide_lds);
+    stream_tile_body<EPI, false>(a, 0, row0, rows, nt, false, wide_lds, n_col_blocks);
 }
 
 // ------------------------------------------------------------------ host side
@@ -1178,8 +1186,8 @@ static bool launch_dense_t(const GmmArgs& a, hipStream_t st, hipEvent_t ev0, hip
     constexpr int lds_bytes = kWideLdsBytes;
     static OncePerDevice once;
     if (!allow_dynamic_lds(once, (const void*)gmm_dense_kernel<EPI>, lds_bytes)) return false;
-    const int channels = (EPI == EPI_SWIGLU) ? a.N / 2 : a.N;
-    const int per_block = (EPI == EPI_SWIGLU) ? kBN / 2 : kBN;
+    const int channels = gated(EPI) ? a.N / 2 : a.N;
+    const int per_block = gated(EPI) ? kBN / 2 : kBN;
     const int n_col_blocks = (channels + per_block - 1) / per_block;
     const int row_tiles = (int)((a.R + 255) / 256);
     // the split of the 8 XCDs over rows x columns with the smallest rectangle perimeter (= bytes fetched per XCD)
@@ -1206,6 +1214,7 @@ bool launch_dense(int epi, const GmmArgs& a, hipStream_t st, hipEvent_t ev0, hip
 {
     if (epi == EPI_I32) return launch_dense_t<EPI_I32>(a, st, ev0, ev1);
     if (epi == EPI_SWIGLU) return launch_dense_t<EPI_SWIGLU>(a, st, ev0, ev1);
+    if (epi == EPI_MEET_SHARED) return launch_dense_t<EPI_MEET_SHARED>(a, st, ev0, ev1);
     return launch_dense_t<EPI_DEQUANT>(a, st, ev0, ev1);
 }
 

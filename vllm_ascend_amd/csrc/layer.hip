@@ -39,7 +39,8 @@ struct Buffers {
     int32_t* dst;
     int32_t* row_token;
     MeetingPlan plan;
-    uint32_t* meet;  // [plan.columns][R]
+    uint32_t* meet;  // [plan.columns][R], behind them [sh_columns][T]
+    int sh_columns, meet_words;  // meet_words: for each of the R pairs
     void* map_ws;
     float* logits;
     void* gate_ws;
@@ -192,7 +193,11 @@ Buffers lay_out(const moe355_layer& l, const Forms& f, int64_t T, void* base)
         b.dst = a.take<int32_t>((size_t)R * 4);
         b.row_token = a.take<int32_t>((size_t)R * 4);
         if (l.weights != W_INT4) b.plan = meeting_plan(R, H, 2 * I, E);
-        b.meet = a.take<uint32_t>((size_t)R * 4 * b.plan.columns);
+        // (on a side stream the column workgroups share the chip with other launches and need not run at the same time)
+        if (l.shared == 1 && l.shared_alpha == 1.0f && l.shared_beta == 0.0f && !f.small && !f.shared_few)
+            b.sh_columns = shared_meeting_columns(T, H, 2 * l.shared_intermediate);
+        b.meet_words = b.plan.columns + (b.sh_columns + l.top_k - 1) / l.top_k;
+        b.meet = a.take<uint32_t>((size_t)R * 4 * b.meet_words);
         b.map_bytes = moe355_init_routing_workspace(T, l.top_k, E);
         b.map_ws = a.take<void>(b.map_bytes);
         // the down GEMM writes its rows where the SwiGLU values were: those are dead once re-quantised
@@ -275,11 +280,20 @@ struct ForkJoinLease {
 };
 
 // dense W8A8 MLP over all tokens, on the rows the routed experts quantised
-int shared_expert(const moe355_layer& l, const Forms& f, const Buffers& b, int64_t T, void* st, bool beside)
+// cleared: the words for its meeting are
+int shared_expert(const moe355_layer& l, const Forms& f, const Buffers& b, int64_t T, void* st, bool beside, bool cleared)
 {
     if (f.shared_few) return few_forward(shared_args(l, b, T), nullptr, (hipStream_t)st);
     const int64_t H = l.hidden, I = l.shared_intermediate;
-    int rc = gmm_i32_impl(b.xq, l.shared_w13, b.one_group, MOE355_GL_CUMSUM, T, H, 2 * I, 1, b.sh_acc, b.sh_ws, b.sh_bytes,
+    int rc;
+    if (cleared && b.sh_columns) {
+        rc = shared_meeting_impl(b.xq, l.shared_w13, l.shared_s13, b.x_scale, b.one_group, T, H, 2 * I, l.shared_limit,
+                                 b.meet + (size_t)b.plan.columns * T * l.top_k, b.plan.looks, b.sh_q, b.sh_q_scale, st);
+        if (rc != MOE355_OK) return rc;
+        return gmm2_impl(b.sh_q, l.shared_w2, nullptr, l.shared_s2, nullptr, b.sh_q_scale, b.one_group, MOE355_GL_CUMSUM, T, I, H,
+                         1, b.sh_out, l.x_dtype, b.sh_ws2, b.sh2_bytes, st, false, beside);
+    }
+    rc = gmm_i32_impl(b.xq, l.shared_w13, b.one_group, MOE355_GL_CUMSUM, T, H, 2 * I, 1, b.sh_acc, b.sh_ws, b.sh_bytes,
                           st, beside);
     if (rc != MOE355_OK) return rc;
     rc = moe355_dequant_swiglu_quant_grouped(b.sh_acc, l.shared_s13, b.x_scale, nullptr, 0, nullptr, 1, T, 2 * I, 1, 1,
@@ -387,7 +401,8 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
     if (!x || !out || (!logits && !l.gate_weight)) return MOE355_E_ARG;
     if (R >= 0x7fffffffLL) return MOE355_E_SHAPE;
     const Forms f = forms_of(l, T);
-    const Buffers b = lay_out(l, f, T, workspace);
+    Buffers b = lay_out(l, f, T, workspace);
+    b.plan.looks = take_meeting_looks();
     if (!workspace || ((uintptr_t)workspace & 255) || workspace_bytes < b.total) return MOE355_E_WORKSPACE;
 
     // measurement hook: the armed events are the routed gate_up product's, whatever is launched in front of it
@@ -434,12 +449,10 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
         // idle.  Experts of 4096 / 2048, two slots, us a call with `beside` / without: 8 experts, 200 / 256 / 320 / 600 tokens
         // 159 / 174 / 130 / 171 against 100 / 107 / 113 / 166; 16 experts, 700 tokens 156 against 173.
         const int64_t routed_bytes = 3 * l.num_experts * l.hidden * l.intermediate / (l.weights == W_INT4 ? 2 : 1);
-        rc = shared_expert(l, f, b, T, side, routed_bytes >= (1ll << 28));
+        rc = shared_expert(l, f, b, T, side, routed_bytes >= (1ll << 28), false);
         // joined below even if a launch was refused: the caller frees the scratch in the order of its own stream
         if (hipEventRecord(lease.fj.join, side) != hipSuccess) return MOE355_E_LAUNCH;
         joined = false;
-    } else if (l.shared == 1) {
-        rc = shared_expert(l, f, b, T, stream, false);
     }
     bool tiles_ready = false;
     if (rc == MOE355_OK && !f.pairs && !f.small) {
@@ -453,8 +466,10 @@ extern "C" int moe355_layer_forward(const moe355_layer* layer, const void* x, co
             n += gemm_tile_specs(R, l.intermediate, l.hidden, l.num_experts, b.gmm2_ws, specs + n);
         }
         rc = route_map_impl(b.topk_ids, T, l.top_k, l.num_experts, 1, b.dst, b.row_token, b.expert_tokens, b.map_ws,
-                            b.map_bytes, specs, n, &tiles_ready, stream, b.meet, b.plan.columns);
+                            b.map_bytes, specs, n, &tiles_ready, stream, b.meet, b.meet_words);
     }
+    // behind the maps, whose launch clears the words that its workgroups meet at
+    if (rc == MOE355_OK && l.shared == 1 && !f.merged) rc = shared_expert(l, f, b, T, stream, false, tiles_ready);
     if (rc == MOE355_OK) {
         (void)moe355_profile_next_gemm(ev0, ev1);
         rc = f.pairs ? routed_pairs(l, f, b, T, stream) : routed_sorted(l, b, T, tiles_ready, stream);

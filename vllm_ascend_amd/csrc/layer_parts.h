@@ -90,9 +90,15 @@ int gmm2_pairs_impl(const int8_t* x, const float* per_token_scale, const float* 
 // the gate_up product whose tiles' workgroups exchange the rows' maxima: rows of its tiles and workgroups of a tile (0: they do not),
 // a word for each of them and every row in `meet`, cleared before the launch
 struct MeetingPlan {
-    int tile_rows = 0, columns = 0;
+    int tile_rows = 0, columns = 0, looks = 0;
 };
+int take_meeting_looks();  // how often the workgroups of this thread's next call look for the others' maxima
 MeetingPlan meeting_plan(int64_t rows, int64_t k, int64_t n, int num_experts);
+// the same for the shared expert's, one expert that owns every row: columns, or 0; meet: [columns][rows], cleared before the launch
+int shared_meeting_columns(int64_t rows, int64_t k, int64_t n);
+int shared_meeting_impl(const int8_t* x, const int8_t* weight_nz, const float* weight_scale, const float* x_scale,
+                        const int64_t* group_list, int64_t rows, int64_t k, int64_t n, float limit, uint32_t* meet, int looks,
+                        int8_t* out, float* out_scale, void* stream);
 // plan, meet: used where the tile map is ready
 int gmm1_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list, const float* weight_scale,
               const float* const* scale_list, const float* x_scale, const int64_t* group_list, int group_list_type,

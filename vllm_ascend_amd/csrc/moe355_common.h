@@ -193,6 +193,12 @@ __device__ __forceinline__ uint32_t quantise_times(v4f v, float inv)
     return pack_low_bytes(sat_rint(v[0] * inv), sat_rint(v[1] * inv), sat_rint(v[2] * inv), sat_rint(v[3] * inv));
 }
 
+// ... divided by their scale
+__device__ __forceinline__ uint32_t quantise_over(v4f v, float s)
+{
+    return pack_low_bytes(sat_rint(v[0] / s), sat_rint(v[1] / s), sat_rint(v[2] / s), sat_rint(v[3] / s));
+}
+
 __device__ __forceinline__ float wave_max(float v)
 {
 #pragma unroll
