@@ -50,12 +50,12 @@ WORKLOADS = ["c4_dsv3_prefill", "c2_qwen3_decode", "c3_qwen3_prefill", "c5_w4a8_
 # kernel of known size), taken from the committed summaries: NOT measured in this run.
 TRAFFIC_FROM_PROFILES = {
     "c2_qwen3_decode": (399_900_000, "profiles/moe_layer_qwen3_decode_kernel_trace.md"),
-    "c3_qwen3_prefill": (960_000_000, "profiles/moe_layer_qwen3_prefill_kernel_trace.md"),
-    "c4_dsv3_prefill": (8_014_000_000, "profiles/moe_layer_dsv3_prefill_kernel_trace.md"),
-    "c5_w4a8_zipf": (1_742_000_000, "profiles/moe_layer_w4a8_zipf_kernel_trace.md"),
-    "c6_dsv3_decode": (6_596_100_000, "profiles/moe_layer_dsv3_decode_kernel_trace.md"),
-    "c7_w8a8_zipf": (3_031_500_000, "profiles/moe_layer_w8a8_zipf_kernel_trace.md"),
-    "c7_w8a8_zipf_4096": (8_188_300_000, "profiles/moe_layer_w8a8_zipf_4096_kernel_trace.md"),
+    "c3_qwen3_prefill": (866_900_000, "profiles/moe_layer_qwen3_prefill_kernel_trace.md"),
+    "c4_dsv3_prefill": (7_863_300_000, "profiles/moe_layer_dsv3_prefill_kernel_trace.md"),
+    "c5_w4a8_zipf": (1_728_200_000, "profiles/moe_layer_w4a8_zipf_kernel_trace.md"),
+    "c6_dsv3_decode": (6_595_500_000, "profiles/moe_layer_dsv3_decode_kernel_trace.md"),
+    "c7_w8a8_zipf": (3_058_600_000, "profiles/moe_layer_w8a8_zipf_kernel_trace.md"),
+    "c7_w8a8_zipf_4096": (7_969_600_000, "profiles/moe_layer_w8a8_zipf_4096_kernel_trace.md"),
 }
 
 
@@ -306,7 +306,9 @@ def run_workload(name, args, lib, torch, np):
                 "traffic": traffic[0] if traffic else None,
                 "traffic_source": (traffic[1] + " (rocprofv3 --pmc of an earlier run of this command, not measured "
                                                 "in this run)") if traffic else None,
-                "kernel": kernel + " (gate_up grouped GEMM + dequant + SwiGLU)",
+                "kernel": kernel + " (gate_up grouped GEMM + dequant + SwiGLU" + (
+                    " + quantisation)" if kernel in ("gmm_tiled_kernel", "gmm_wide_kernel")
+                    and lib.moe355_meeting_tile_rows(R, cfg.H, 2 * cfg.I, cfg.E) else ")"),
                 "kernel_avg_us": round(avg_ms * 1e3, 2),
                 "kernel_p50_us": round(durs[len(durs) // 2] * 1e3, 2),
                 "algorithmic_bytes": abytes,
