@@ -508,6 +508,9 @@ int moe355_profile_next_gemm(void *start_event, void *stop_event);
  * calling thread it gives up after `looks` instead (0: at once).  The results are the same either way.
  */
 int moe355_meeting_tile_rows(int64_t rows, int64_t k, int64_t n, int num_experts);
+/* The same for the shared expert's product in line: the workgroups of a tile, or 0 where its int32 sums go through memory; in
+ * on_an_xcd (or NULL) how many of them run on one XCD, at most. */
+int moe355_shared_meeting_columns(int64_t rows, int64_t k, int64_t n, int *on_an_xcd);
 int moe355_next_meeting_looks(int looks);
 
 /* Which kernel family the int8 grouped GEMMs above launch for a shape, given a workspace of the size their

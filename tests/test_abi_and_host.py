@@ -560,6 +560,26 @@ def test_where_gate_up_tiles_quantise_their_rows(experts, k, n, rows, tile_rows)
     assert _lib.load().moe355_meeting_tile_rows(rows, k, n, experts) == tile_rows
 
 
+# ... and of the shared expert's: all columns of a row of tiles that fall to one XCD have a place there, also beside such a launch on
+# another stream (32 workgroups of 160 KiB of LDS run on one; each launch may hold all but one of a row's columns)
+def test_columns_that_meet_have_places():
+    from vllm_ascend_amd import _lib
+
+    lib, on_one = _lib.load(), ctypes.c_int()
+    admitted = 0
+    for n in (512, 1408, 4096, 4224, 5632, 8192, 8256, 10240, 11264, 16256, 16384):
+        for rows in [*range(1, 65537, 255), 32000, 40192, 44288, 64768, 65536]:
+            columns = lib.moe355_shared_meeting_columns(rows, 64, n, ctypes.byref(on_one))
+            want = -(-n // 256) if -(-rows // 256) * -(-n // 256) >= 192 else 0
+            assert columns == want
+            assert (0 < on_one.value <= min(16, columns)) if columns else on_one.value == 0
+            assert 8 * on_one.value >= columns
+            admitted += columns > 16 and rows > 30000
+    assert admitted > 100
+    assert lib.moe355_shared_meeting_columns(65536, 64, 16384 + 64, ctypes.byref(on_one)) == 0  # 65 columns
+    assert lib.moe355_shared_meeting_columns(0, 64, 4096, None) == 0 == lib.moe355_shared_meeting_columns(4096, 64, 0, None)
+
+
 # one for every 56 pairs, but not where a short launch (fewer than 1536 units of 64 channels) has places in front of its slots
 # (from two pairs per expert on), nor from twelve pairs per expert on
 @pytest.mark.parametrize("experts, n, pairs, blocks", [(128, 1536, 512, 9), (128, 512, 256, 4), (128, 512, 257, 0), (128, 704, 512, 0),

@@ -126,6 +126,7 @@ PROTOTYPES = {
     "moe355_layer_gates_inside": (c_int, [c_void_p, c_int64]),
     "moe355_profile_next_gemm": (c_int, [c_void_p, c_void_p]),
     "moe355_meeting_tile_rows": (c_int, [c_int64, c_int64, c_int64, c_int]),
+    "moe355_shared_meeting_columns": (c_int, [c_int64, c_int64, c_int64, c_void_p]),
     "moe355_next_meeting_looks": (c_int, [c_int]),
     "moe355_gmm_kernel_name": (c_char_p, [c_int, c_int64, c_int64, c_int64, c_int]),
     "moe355_gmm_tile_rows": (c_int, [c_int64, c_int64, c_int64, c_int]),

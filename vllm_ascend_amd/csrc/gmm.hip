@@ -1080,8 +1080,8 @@ extern "C" int moe355_meeting_tile_rows(int64_t rows, int64_t k, int64_t n, int 
 // us: 256 experts of 7168 / 2048, 4096 / 5000 / 6000 / 7000 / 8192 tokens 2641 / 2855 / 3328 / 3828 / 4519 and 2617 / 2839 / 3289 / 3799 /
 // 4500, Zipf(1.1) 4096 2591 and 2557, int4 4096 2713 and 2698; 64 experts of 2048 / 2048, 4096 / 8000 tokens 674 / 1174 and 656 / 1142, of
 // 4096 / 1024, 8192 tokens 1214 and 1198.  The columns need not divide an XCD's 32 places here (64 of 4096 / 1536, 4096 / 7000 tokens
-// 1014 / 1596 and 1000 / 1579; 2048 / 2816, 4500 1071 and 1052; 7168 / 2560, 4096 2537 and 2532; 7168 / 1408, 8192 2973 and 2959): the
-// rectangles keep them close.  64 are what a wavefront looks at at once.
+// 1014 / 1596 and 1000 / 1579; 2048 / 2816, 4500 1071 and 1052; 7168 / 2560, 4096 2537 and 2532; 7168 / 1408, 8192 2973 and 2959), but
+// those of a row of tiles must all have a place there (dense_split).  64 are what a wavefront looks at at once.
 int moe355::shared_meeting_columns(int64_t rows, int64_t k, int64_t n)
 {
     GmmArgs a = {};
@@ -1091,6 +1091,13 @@ int moe355::shared_meeting_columns(int64_t rows, int64_t k, int64_t n)
     a.E = 1;
     const int64_t columns = (n / 2 + 127) / 128;
     return columns <= 64 && dense_tiles(a) ? (int)columns : 0;
+}
+
+extern "C" int moe355_shared_meeting_columns(int64_t rows, int64_t k, int64_t n, int* on_an_xcd)
+{
+    const int columns = rows <= 0 || k <= 0 || n <= 0 ? 0 : moe355::shared_meeting_columns(rows, k, n);
+    if (on_an_xcd) *on_an_xcd = columns ? dense_split(rows, columns, true).pn : 0;
+    return columns;
 }
 
 int moe355::shared_meeting_impl(const int8_t* x, const int8_t* weight_nz, const float* weight_scale, const float* x_scale,

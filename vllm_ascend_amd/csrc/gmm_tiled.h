@@ -25,7 +25,12 @@ bool launch_resident(const GmmArgs& a, void* workspace, hipStream_t st, hipEvent
 // One expert owning every row: 64 x 64 tiles with K cut over the wavefronts (gmm_split.hip), no tile map either.
 void launch_split(int epi, const GmmArgs& a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1);
 
-// One expert owning every row (a.E == 1): 256 x 256 tiles placed by arithmetic, no tile map, no scratch.
+// One expert owning every row (a.E == 1): 256 x 256 tiles placed by arithmetic, no tile map, no scratch.  xn of the 8 XCDs lie side
+// by side, each with a rectangle of pm x pn tiles; meet: the workgroups of a row of tiles exchange its maxima (EPI_MEET_SHARED).
+struct DenseSplit {
+    int xn, pm, pn;
+};
+DenseSplit dense_split(int64_t rows, int columns, bool meet);
 bool launch_dense(int epi, const GmmArgs& a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1);
 
 }  // namespace moe355

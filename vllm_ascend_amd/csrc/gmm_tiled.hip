@@ -1180,6 +1180,21 @@ static bool launch_wide(const GmmArgs& a, void* workspace, hipStream_t st, hipEv
     return true;
 }
 
+// The split of the 8 XCDs over rows x columns with the smallest rectangle perimeter (= bytes fetched per XCD).  Workgroups that
+// exchange maxima hold their places until the last one of their row of tiles has come, so all of a row that fall to an XCD must find
+// a place there: 32 workgroups run on one, 16 columns leave room for such a launch on another stream.  A split like that exists up to
+// 128 columns.
+DenseSplit dense_split(int64_t rows, int columns, bool meet)
+{
+    const int row_tiles = (int)((rows + 255) / 256), most = meet ? 16 : columns;
+    DenseSplit best = {};
+    for (int c = 1; c <= 8; c *= 2) {
+        const DenseSplit s = {c, (row_tiles + 8 / c - 1) / (8 / c), (columns + c - 1) / c};
+        if (s.pn <= most && (best.xn == 0 || s.pm + s.pn < best.pm + best.pn)) best = s;
+    }
+    return best;
+}
+
 template <int EPI>
 static bool launch_dense_t(const GmmArgs& a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1)
 {
@@ -1189,18 +1204,7 @@ static bool launch_dense_t(const GmmArgs& a, hipStream_t st, hipEvent_t ev0, hip
     const int channels = gated(EPI) ? a.N / 2 : a.N;
     const int per_block = gated(EPI) ? kBN / 2 : kBN;
     const int n_col_blocks = (channels + per_block - 1) / per_block;
-    const int row_tiles = (int)((a.R + 255) / 256);
-    // the split of the 8 XCDs over rows x columns with the smallest rectangle perimeter (= bytes fetched per XCD)
-    int xn = 1, best = 0;
-    for (int c = 1; c <= 8; c *= 2) {
-        const int per_m = (row_tiles + 8 / c - 1) / (8 / c), per_n = (n_col_blocks + c - 1) / c;
-        const int cost = per_m + per_n;
-        if (c == 1 || cost < best) {
-            best = cost;
-            xn = c;
-        }
-    }
-    const int pm = (row_tiles + 8 / xn - 1) / (8 / xn), pn = (n_col_blocks + xn - 1) / xn;
+    const auto [xn, pm, pn] = dense_split(a.R, n_col_blocks, meets(EPI));
     const int grid = 8 * pm * pn;
     if (ev0 || ev1)
         hipExtLaunchKernelGGL((gmm_dense_kernel<EPI>), dim3(grid), dim3(512), lds_bytes, st, ev0, ev1, 0, a, xn, pm, pn,
