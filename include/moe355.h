@@ -490,9 +490,9 @@ int moe355_token_unpermute_pairs(const void *rows, int dtype, const void *probs,
                                  void *out, int64_t *expert_tokens, void *stream);
 
 /* ---------------------------------------------------------------------------
- * Measurement hook (no counterpart in the reference; for benchmarks).  The one piece of per-thread host
- * state in the library: the armed pair of events is kept in thread-local storage until the next GEMM launch
- * of the same thread takes it.
+ * Measurement hook (no counterpart in the reference; for benchmarks).  Per-thread host state, as is the number
+ * that moe355_next_meeting_looks sets and nothing else in the library: the armed pair of events is kept in
+ * thread-local storage until the next GEMM launch of the same thread takes it.
  * The next grouped-GEMM kernel launched from the calling thread by
  * moe355_gmm1_swiglu_quant / moe355_gmm2_dequant / moe355_gmm_i32 and their other
  * forms, or the routed gate_up product of moe355_layer_forward, is bracketed
@@ -504,8 +504,8 @@ int moe355_profile_next_gemm(void *start_event, void *stop_event);
 
 /* On the sorted path of moe355_layer_forward the workgroups of a tile of the gate_up product can exchange the maxima of its rows
  * and quantise them in place: the rows of those tiles, or 0 where the fp32 values go through memory and a launch of their own.
- * A workgroup that has looked for the others' maxima some thousand times computes them itself; in the next layer call of the
- * calling thread it gives up after `looks` instead (0: at once).  The results are the same either way.
+ * A workgroup that has looked for the others' maxima 4096 times computes them itself; in the next layer call of the calling
+ * thread it gives up after `looks` instead (0: at once; more than 4096 are 4096).  The results are the same either way.
  */
 int moe355_meeting_tile_rows(int64_t rows, int64_t k, int64_t n, int num_experts);
 /* The same for the shared expert's product in line: the workgroups of a tile, or 0 where its int32 sums go through memory; in

@@ -580,6 +580,20 @@ def test_columns_that_meet_have_places():
     assert lib.moe355_shared_meeting_columns(0, 64, 4096, None) == 0 == lib.moe355_shared_meeting_columns(4096, 64, 0, None)
 
 
+def test_looks_of_the_next_call_are_bounded():
+    """moe355::take_meeting_looks() is what a layer call takes; it has no C name."""
+    from vllm_ascend_amd import _lib
+
+    lib = _lib.load()
+    taken = lib._ZN6moe35518take_meeting_looksEv
+    usual = taken()
+    assert usual == 4096
+    for looks, want in ((0, 0), (1, 1), (4095, 4095), (4096, 4096), (4097, 4096), (2**31 - 1, 4096)):
+        assert lib.moe355_next_meeting_looks(looks) == 0
+        assert taken() == want and taken() == usual
+    assert lib.moe355_next_meeting_looks(-1) == -1 and taken() == usual
+
+
 # one for every 56 pairs, but not where a short launch (fewer than 1536 units of 64 channels) has places in front of its slots
 # (from two pairs per expert on), nor from twelve pairs per expert on
 @pytest.mark.parametrize("experts, n, pairs, blocks", [(128, 1536, 512, 9), (128, 512, 256, 4), (128, 512, 257, 0), (128, 704, 512, 0),

@@ -1005,7 +1005,7 @@ extern "C" size_t moe355_gmm1_swiglu_quant_workspace(int64_t rows, int64_t n, in
     return (((size_t)rows * (size_t)(n / 2) * 4 + 255) & ~(size_t)255) + tiled_ws_max(rows, num_experts);
 }
 
-// a few milliseconds
+// a few milliseconds; nobody may ask for more, so that a launch whose workgroups do not meet ends
 constexpr int kMeetLooks = 4096;
 static thread_local int t_meet_looks = kMeetLooks;
 
@@ -1019,7 +1019,7 @@ int moe355::take_meeting_looks()
 extern "C" int moe355_next_meeting_looks(int looks)
 {
     if (looks < 0) return MOE355_E_ARG;
-    t_meet_looks = looks;
+    t_meet_looks = looks < kMeetLooks ? looks : kMeetLooks;
     return MOE355_OK;
 }
 
