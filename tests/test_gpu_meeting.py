@@ -97,6 +97,34 @@ def test_layers_on_weight_streaming_tiles(E, k, H, I, T, skew):
     _check(layer, x, logits - skew * torch.arange(E, device=DEV).float().log1p(), looks=(None, 0))
 
 
+def _ms(layer, x, logits, looks):
+    """The fastest of five calls."""
+    best = float("inf")
+    for _ in range(5):
+        if looks is not None:
+            assert _lib().moe355_next_meeting_looks(looks) == 0
+        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        start.record()
+        layer(x, logits)
+        end.record()
+        torch.cuda.synchronize()
+        best = min(best, start.elapsed_time(end))
+    return best
+
+
+# A workgroup that gives up computes a column's maxima by one scalar product after the other, some ten times as long as the whole
+# product takes.  After one look in vain it computes the first column that is missing, if that has not come meanwhile; the words of
+# the others come while it does.  Without a look it computes seven of the eight (0.05 and 4.8 ms a call).
+def test_columns_that_have_come_are_not_computed():
+    T, E, H, I = 1024, 8, 2048, 1024
+    cfg, layer, x, logits = _layer(T, E=E, k=1, H=H, I=I)
+    assert _lib().moe355_meeting_tile_rows(T, H, 2 * I, E) and I // 128 == 8
+    layer(x, logits)
+    one, all_of_them = _ms(layer, x, logits, 1), _ms(layer, x, logits, 0)
+    print(f"one look {one:.3f} ms, none {all_of_them:.3f} ms", flush=True)
+    assert one < 0.5 * all_of_them
+
+
 def test_captured_and_from_two_streams():
     cfg, layer, x, logits = _layer(700, E=8, k=2, H=256, I=640)
     want = layer.forward_impl(x, logits).routed_out

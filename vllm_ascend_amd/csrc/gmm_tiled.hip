@@ -191,7 +191,7 @@ __device__ __forceinline__ void tiled_epilogue_body(const GmmArgs& a, int e, v4i
 //   zero is not there yet) and looks at the others' until none is missing: no counter, no order, no fence, since a word is all that
 //   is handed over.  The routing launch clears the words.
 // - They run at the same time, because a launch starts its workgroups in order and those of a tile are neighbours.  Nothing rests on
-//   that: a workgroup that has looked meet_looks times (a few milliseconds) computes the missing maxima itself.
+//   that: a workgroup that has looked meet_looks times (a few milliseconds) computes the maxima that are still missing itself.
 // What it costs is that they wait for the slowest, which is why the number of columns matters (meeting_plan in gmm.hip).  us a layer
 // with / without, 128 experts of 2048 / 768, 777 / 2000 / 4000 / 8192 tokens 138 / 184 / 292 / 496 against 143 / 194 / 313 / 531; 256 of
 // 7168 / 2048, 500 / 1500 / 3000 tokens 1712 / 1831 / 2049 against 1770 / 1956 / 2157; 8 of 1024 / 1408, 6000 tokens 105 against 115.
@@ -369,12 +369,22 @@ __device__ __forceinline__ void meet_body(const GmmArgs& a, const TilePart& p, v
         if (!*met) {
             for (int c = 0; c < columns; ++c) {
                 if (c == nt) continue;
-                maxima_of_column<LIMIT, SHARED>(a, p.e, row0, rows, c, 32 * GROUPS, (uint32_t*)lds);
+                // Column by column, what has come by now is taken (with looks of 0, for tests, nothing is): while one column is
+                // computed the others come, and to compute them too would hold the compute unit that they wait for.
+                uint32_t w = tid < rows && a.meet_looks > 0 ? look(word + c * a.R + tid) : 0u;
+                __syncthreads();  // (everybody has read the note and the maxima)
+                if (tid == 0) *met = 1;
+                __syncthreads();
+                if (tid < rows && w == 0u) *met = 0;
+                __syncthreads();
+                if (!*met) {
+                    maxima_of_column<LIMIT, SHARED>(a, p.e, row0, rows, c, 32 * GROUPS, (uint32_t*)lds);
+                    if (tid < rows) w = ((const uint32_t*)lds)[tid];
+                }
                 if (tid < rows) {
-                    const float o = __uint_as_float(((const uint32_t*)lds)[tid]);
+                    const float o = __uint_as_float(w & ~(1u << 31));
                     amax = o > amax ? o : amax;
                 }
-                __syncthreads();
             }
         }
     }
