@@ -388,6 +388,53 @@ def test_entries_of_tall_tiles(counts, entries):
     _check_tall_tiles(counts, Kd, N)
 
 
+# ... and every tile is listed once, the two halves of a tall one next to each other in the same eight entries (workgroup i runs on
+# XCD i % 8, and the halves of the gate_up product wait for each other): with and without room for all halves, an even and an odd
+# number of whole tall tiles and of others
+@pytest.mark.parametrize("experts,mean,skew", [(64, 80, 0.8), (64, 100, 1.1), (65, 120, 1.1), (63, 200, 0.8), (48, 150, 0.3), (64, 64, 0.0),
+                                               (33, 250, 0.1), (256, 128, 1.1), (255, 96, 0.8), (6, 240, 0.5), (8, 200, 1.1)])
+def test_list_of_tiles_by_length(experts, mean, skew):
+    from vllm_ascend_amd import kernels as K
+    from vllm_ascend_amd._lib import load
+
+    lib, Kd, N = load(), 4096, 64
+    w = torch.zeros(experts, N * Kd, dtype=torch.int8, device="cuda")
+    sw = torch.ones(experts, N, device="cuda")
+    p = lambda t: t.data_ptr()  # noqa: E731
+    seen = set()
+    for seed in range(12):
+        rng = np.random.default_rng(seed)
+        R = experts * mean + seed
+        popular = (1.0 + rng.permutation(experts)) ** -skew
+        counts = rng.multinomial(R, popular / popular.sum())
+        assert lib.moe355_gmm_kernel_name(2, R, Kd, N, experts).decode() == "gmm_wide_kernel"
+        x = torch.zeros(R, Kd, dtype=torch.int8, device="cuda")
+        sx = torch.ones(R, device="cuda")
+        gl = torch.from_numpy(counts.astype(np.int64)).cuda()
+        out = torch.empty(R, N, dtype=torch.bfloat16, device="cuda")
+        ws = torch.zeros(lib.moe355_gmm2_dequant_workspace(R, N, Kd, experts), dtype=torch.uint8, device="cuda")
+        assert lib.moe355_gmm2_dequant(p(x), p(w), p(sw), p(sx), p(gl), 1, R, Kd, N, experts, p(out), K._dt(out, "out"), p(ws), ws.numel(),
+                                       torch.cuda.current_stream().cuda_stream) == 0
+        words = ws.cpu().numpy()[:ws.numel() // 4 * 4].view(np.int32)
+        most = R // 256 + experts
+        n, pitch = int(words[0]), -(-most // 64) * 64
+        assert n <= most
+        listed, begin, end = (words[64 + i * pitch:64 + i * pitch + n].astype(np.int64) for i in range(3))
+        expert, first, second = listed & ((1 << 28) - 1), (listed >> 29) & 1, (listed >> 28) & 1
+        starts = np.cumsum(counts) - counts
+        assert np.array_equal(end, starts[expert] + counts[expert])
+        want = {(e, int(starts[e]) + r) for e in range(experts) for r in range(0, int(counts[e]), 256)}
+        once = [(int(e), int(b)) for e, b, s in zip(expert, begin, second) if not s]
+        assert len(once) == len(want) and set(once) == want
+        at = np.flatnonzero(second)
+        assert np.array_equal(at - 1, np.flatnonzero(first)) and np.all(at % 2 == 1)
+        assert np.array_equal(expert[at], expert[at - 1]) and np.array_equal(begin[at], begin[at - 1])
+        tall = sum(int(counts[e]) - (b - int(starts[e])) > 192 for e, b in want)
+        seen.add((len(at) == tall, (tall - len(at)) % 2, (len(want) - tall) % 2))
+        assert np.all(end[at] - begin[at] > 192)
+    print(f"{experts} experts, all in halves / odd whole ones / odd others: {sorted(seen)}", flush=True)
+
+
 def _check_tall_tiles(counts, Kd, N):
     from oracle import oracle as orc
     from vllm_ascend_amd import kernels as K

@@ -28,6 +28,7 @@ struct TileSpec {
     // the cold experts' tiles for their weights from HBM, and so both are busy all the time.  In eights, because entry t
     // runs on XCD t % 8.  A tall tile has an entry for either half of its columns as long as the list has room for that (a
     // workgroup per entry and column is launched for as many tiles as the rows can make), beyond it one for both.
+    // Both halves are in the same eight entries, since their workgroups wait for each other (EPI_MEET in gmm_tiled.hip).
     // Layers under Zipf(1.1), 256 experts of 7168 / 2048, 2048 / 3000 / 4096 tokens: tall ones whole and last 1662 / 2165 / 2520 us,
     // halves last 1631 / 2108 / 2510, halves first 1617 / 2075 / 2443, spread 1567 / 1998 / 2254; 128 experts of 2048 / 768, 1900
     // tokens 223 whole and last, 214 spread.  4096 tokens of uniform routing, a few of whose experts are tall because of the
@@ -96,12 +97,14 @@ __device__ __forceinline__ void build_tile_map(RowsOf rows_of, int E, const Tile
         // 2560 1453 / 1340 at 250, 96 of 8192 / 2048 1562 / 1505 under Zipf(0.1) at 220, where one tile in eight is tall and shared.
         // Between (one in 33, 24, 22, 21, 17): 1.01, 0.98, 0.95, 1.01, 0.97 of the time.
         const bool few = 16 * total[3] < all_tiles || 24 * all_shared < all_tiles;
-        const int32_t whole = few ? total[3] : total[3] > room ? total[3] - room : 0;  // tall tiles with one entry, the first ones
-        const int32_t tall = 2 * total[3] - whole;
-        if (tid == 0) tm.count[0] = all_tiles < max_tiles ? all_tiles - total[3] + tall : max_tiles;
+        // tall tiles with one entry: an even number in front, so that pairs of halves start at even places, and the last one if there
+        // is one more
+        const int32_t whole = few ? total[3] : total[3] > room ? total[3] - room : 0, in_front = whole & ~1;
+        const int32_t tall = 2 * total[3] - whole, others = all_tiles - total[3];
+        if (tid == 0) tm.count[0] = all_tiles < max_tiles ? others + tall : max_tiles;
         // eight entries, one for every XCD, are a block; the blocks of tall entries lie at ((2 b + 1) n / 2 a) of the a of them among
-        // n blocks, and what fills no block at the end
-        const int32_t a8 = few ? 0 : tall >> 3, n8 = a8 + ((all_tiles - total[3]) >> 3);  // at most 8192 and 12288
+        // n blocks, and what fills no block at the end, the tall ones first
+        const int32_t a8 = few ? 0 : tall >> 3, n8 = a8 + (others >> 3);  // at most 8192 and 12288
         // x / d where the quotient is at most 12288: by the reciprocal it is off by one at most.  One lane walks the tiles
         // of a hot expert, and 64-bit divisions for each of them made the launch of 4096 tokens under Zipf(1.1) 30 us
         // instead of 16.
@@ -111,11 +114,12 @@ __device__ __forceinline__ void build_tile_map(RowsOf rows_of, int E, const Tile
         };
         const float by_a = 1.0f / (float)(2 * a8), by_n = 1.0f / (float)(2 * n8);
         auto tall_at = [&](int32_t i) {
-            return (i >> 3) < a8 ? divide((2 * (i >> 3) + 1) * n8, 2 * a8, by_a) * 8 + (i & 7) : all_tiles - total[3] + i;
+            if ((i >> 3) < a8) return divide((2 * (i >> 3) + 1) * n8, 2 * a8, by_a) * 8 + (i & 7);
+            return few ? others + i : (n8 - a8) * 8 + i;
         };
         auto other_at = [&](int32_t i) {
             int32_t at = i >> 3, before = 0;
-            if (at >= n8 - a8) return a8 * 8 + i;
+            if (at >= n8 - a8) return few ? i : tall + i;
             for (int32_t next = -1; next != before;) {  // the tall blocks in front of it: those at `at` or before
                 next = before;
                 const int32_t reach = 2 * (at + before + 1) * a8 - n8;
@@ -137,11 +141,13 @@ __device__ __forceinline__ void build_tile_map(RowsOf rows_of, int E, const Tile
                 for (int32_t t = 0; t < full + (c == 3 ? 1 : 0); ++t) {
                     const int32_t i = next_tall++;
                     const int64_t begin = row + (int64_t)t * 256;
-                    if (i < whole) {
+                    if (i < in_front) {
                         put(tall_at(i), listed, begin, row + m);
+                    } else if (i == total[3] - 1 && in_front < whole) {
+                        put(tall_at(tall - 1), listed, begin, row + m);
                     } else {
-                        put(tall_at(2 * i - whole), listed | kFirstHalf, begin, row + m);
-                        put(tall_at(2 * i - whole + 1), listed | kSecondHalf, begin, row + m);
+                        put(tall_at(2 * i - in_front), listed | kFirstHalf, begin, row + m);
+                        put(tall_at(2 * i - in_front + 1), listed | kSecondHalf, begin, row + m);
                     }
                 }
                 if (c < 3) put(other_at(next[c]++), listed, row + (int64_t)full * 256, row + m);
