@@ -103,7 +103,8 @@ __device__ __forceinline__ void build_tile_map(RowsOf rows_of, int E, const Tile
         const int32_t in_front = whole - extra, tall = 2 * (total[3] - extra) - in_front, others = all_tiles - total[3] + extra;
         if (tid == 0) tm.count[0] = all_tiles < max_tiles ? others + tall : max_tiles;
         // eight entries, one for every XCD, are a block; the blocks of tall entries lie at ((2 b + 1) n / 2 a) of the a of them among
-        // n blocks, and what fills no block at the end, the tall ones first
+        // n blocks, and what fills no block at the end, the tall ones last (so that their pairs start at even places there too, an odd one
+        // of the others behind them)
         const int32_t a8 = few ? 0 : tall >> 3, n8 = a8 + (others >> 3);  // at most 8192 and 12288
         // x / d where the quotient is at most 12288: by the reciprocal it is off by one at most.  One lane walks the tiles
         // of a hot expert, and 64-bit divisions for each of them made the launch of 4096 tokens under Zipf(1.1) 30 us
@@ -115,11 +116,12 @@ __device__ __forceinline__ void build_tile_map(RowsOf rows_of, int E, const Tile
         const float by_a = 1.0f / (float)(2 * a8), by_n = 1.0f / (float)(2 * n8);
         auto tall_at = [&](int32_t i) {
             if ((i >> 3) < a8) return divide((2 * (i >> 3) + 1) * n8, 2 * a8, by_a) * 8 + (i & 7);
-            return few ? others + i : (n8 - a8) * 8 + i;
+            return (few ? others : others & ~1) + i;
         };
         auto other_at = [&](int32_t i) {
             int32_t at = i >> 3, before = 0;
-            if (at >= n8 - a8) return few ? i : tall + i;
+            if (!few && i == others - 1 && (others & 1)) return tall + i;
+            if (at >= n8 - a8) return a8 * 8 + i;
             for (int32_t next = -1; next != before;) {  // the tall blocks in front of it: those at `at` or before
                 next = before;
                 const int32_t reach = 2 * (at + before + 1) * a8 - n8;
