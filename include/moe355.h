@@ -503,13 +503,14 @@ int moe355_token_unpermute_pairs(const void *rows, int dtype, const void *probs,
 int moe355_profile_next_gemm(void *start_event, void *stop_event);
 
 /* On the sorted path of moe355_layer_forward the workgroups of a tile of the gate_up product can exchange the maxima of its rows
- * and quantise them in place: the rows of those tiles, or 0 where the fp32 values go through memory and a launch of their own.
+ * and quantise them in place: the rows of those tiles, or 0 where the fp32 values go through memory and a launch of their own,
+ * among others with more than 65536 pairs or 512 experts, whose maps are not built by one launch.
  * A workgroup that has looked for the others' maxima 4096 times computes them itself; in the next layer call of the calling
  * thread it gives up after `looks` instead (0: at once; more than 4096 are 4096).  The results are the same either way.
  */
 int moe355_meeting_tile_rows(int64_t rows, int64_t k, int64_t n, int num_experts);
-/* The same for the shared expert's product in line: the workgroups of a tile, or 0 where its int32 sums go through memory; in
- * on_an_xcd (or NULL) how many of them run on one XCD, at most. */
+/* The same for the shared expert's product in line, in a layer of at most so many pairs and experts: the workgroups of a tile, or 0
+ * where its int32 sums go through memory; in on_an_xcd (or NULL) how many of them run on one XCD, at most. */
 int moe355_shared_meeting_columns(int64_t rows, int64_t k, int64_t n, int *on_an_xcd);
 int moe355_next_meeting_looks(int looks);
 

@@ -553,11 +553,34 @@ def test_tokens_of_a_tile_in_lds_lines(rows, experts, k, n, resident):
     (256, 7168, 4096, 4096, 128), (256, 7168, 4096, 256 * 144, 256), (256, 7168, 4096, 256 * 145, 0), (128, 2048, 2048, 1152, 128),
     (128, 2048, 1536, 1024, 64), (128, 2048, 1536, 128 * 64 - 1, 64), (128, 2048, 1536, 128 * 64, 128), (128, 2048, 1536, 65536, 128),
     (256, 2048, 1536, 256 * 48 - 1, 0), (256, 2048, 1536, 256 * 48, 128), (64, 4096, 3072, 1152, 0), (128, 4096, 3072, 10240, 0),
-    (32, 2880, 5760, 9600, 0), (8, 1024, 2816, 1040, 64), (8, 1024, 2816, 16000, 128), (128, 2048, 1536, 512, 0), (1, 2048, 4096, 4096, 0)])
+    (32, 2880, 5760, 9600, 0), (8, 1024, 2816, 1040, 64), (8, 1024, 2816, 16000, 128), (128, 2048, 1536, 512, 0), (1, 2048, 4096, 4096, 0),
+    (128, 2048, 1536, 65544, 0), (128, 2048, 1536, 100000, 0), (512, 1024, 2048, 20000, 128), (513, 1024, 2048, 20000, 0)])
 def test_where_gate_up_tiles_quantise_their_rows(experts, k, n, rows, tile_rows):
     from vllm_ascend_amd import _lib
 
     assert _lib.load().moe355_meeting_tile_rows(rows, k, n, experts) == tile_rows
+
+
+def test_no_words_for_a_meeting_that_does_not_take_place():
+    """The words (a word for every pair and column of a tile) end with the one-launch map, at 65536 pairs."""
+    from vllm_ascend_amd import _lib
+
+    lib = _lib.load()
+
+    def workspace(tokens, weights, shared=0):
+        a = _lib.Layer(hidden=2048, intermediate=768, num_experts=128, top_k=8, k_group=1, group_count=1, weights=weights,
+                       x_dtype=_lib.DT_BF16, w13=256, s13=256, w2=256, s2=256, group13=256, group2=256, shared=shared,
+                       shared_intermediate=1024, shared_alpha=1.0, shared_w13=256, shared_s13=256, shared_w2=256, shared_s2=256)
+        return lib.moe355_layer_workspace(ctypes.byref(a), tokens)
+
+    assert lib.moe355_meeting_tile_rows(65536, 2048, 1536, 128) == 128  # six columns
+    assert lib.moe355_shared_meeting_columns(8192, 2048, 2048, None) == 8  # a word for every pair
+    for weights, shared, words in ((0, 0, 6), (0, 1, 7), (2, 0, 0), (2, 1, 1)):
+        # what one token more adds, above 8192 and there
+        step = [workspace(t + 1, weights, shared) - workspace(t, weights, shared) for t in (8191, 8192, 8193, 8194)]
+        usual = max(abs(s) for s in (step[0], step[2], step[3]))
+        assert usual < 1 << 17
+        assert abs(step[1] + words * 65536 * 4) < 1 << 18, (weights, shared, step)
 
 
 # ... and of the shared expert's: all columns of a row of tiles that fall to one XCD have a place there, also beside such a launch on

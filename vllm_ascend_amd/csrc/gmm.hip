@@ -1054,7 +1054,8 @@ MeetingPlan moe355::meeting_plan(int64_t rows, int64_t k, int64_t n, int num_exp
     a.K = (int)k;
     a.N = (int)n;
     a.E = num_experts;
-    if (dense_tiles(a) || split_tiles(a)) return {};
+    // (the launch that builds the maps clears the words)
+    if (dense_tiles(a) || split_tiles(a) || !one_launch_map(rows, num_experts)) return {};
     const int bm = gemm_family(a, true), columns = (a.N / 2 + 127) / 128;
     const int64_t avg = rows / num_experts, own = n * k;
     const MeetingPlan yes = {bm, columns};

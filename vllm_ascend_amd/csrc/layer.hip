@@ -192,9 +192,9 @@ Buffers lay_out(const moe355_layer& l, const Forms& f, int64_t T, void* base)
     } else {
         b.dst = a.take<int32_t>((size_t)R * 4);
         b.row_token = a.take<int32_t>((size_t)R * 4);
-        if (l.weights != W_INT4) b.plan = meeting_plan(R, H, 2 * I, E);
+        if (l.weights != W_INT4 && !f.small) b.plan = meeting_plan(R, H, 2 * I, E);
         // (on a side stream the column workgroups share the chip with other launches and need not run at the same time)
-        if (l.shared == 1 && l.shared_alpha == 1.0f && l.shared_beta == 0.0f && !f.small && !f.shared_few)
+        if (l.shared == 1 && l.shared_alpha == 1.0f && l.shared_beta == 0.0f && !f.small && !f.shared_few && one_launch_map(R, E))
             b.sh_columns = shared_meeting_columns(T, H, 2 * l.shared_intermediate);
         b.meet_words = b.plan.columns + (b.sh_columns + l.top_k - 1) / l.top_k;
         b.meet = a.take<uint32_t>((size_t)R * 4 * b.meet_words);

@@ -99,7 +99,7 @@ int shared_meeting_columns(int64_t rows, int64_t k, int64_t n);
 int shared_meeting_impl(const int8_t* x, const int8_t* weight_nz, const float* weight_scale, const float* x_scale,
                         const int64_t* group_list, int64_t rows, int64_t k, int64_t n, float limit, uint32_t* meet, int looks,
                         int8_t* out, float* out_scale, void* stream);
-// plan, meet: used where the tile map is ready
+// plan, meet: used where the tile map is ready, which it is where there is a plan and the layer sorts
 int gmm1_impl(const int8_t* x, const int8_t* weight_nz, const int8_t* const* weight_list, const float* weight_scale,
               const float* const* scale_list, const float* x_scale, const int64_t* group_list, int group_list_type,
               int64_t rows, int64_t k, int64_t n, int num_experts, float swiglu_limit, int8_t* out, float* out_scale,
@@ -139,7 +139,8 @@ int gmm2_w4_pairs(const int8_t* x, const float* x_scale, const int32_t* topk_ids
                   int out_dtype, hipStream_t st);
 
 // moe355_route_map with the tile maps of the two products (nspecs of them, at most 2) built by the same launch where it
-// is one launch (returns 1 in *built then), which also clears zeros_per_pair words for every pair
+// is one launch (one_launch_map; returns 1 in *built then), which also clears zeros_per_pair words for every pair
+bool one_launch_map(int64_t pairs, int num_experts);
 int route_map_impl(const int32_t* expert_idx, int64_t num_tokens, int top_k, int num_experts, int tokens_num_type,
                    int32_t* expanded_row_idx, int32_t* row_token, int64_t* expert_tokens, void* workspace,
                    size_t workspace_bytes, const TileSpec* specs, int nspecs, bool* built, void* stream, uint32_t* zeros = nullptr,

@@ -616,6 +616,11 @@ extern "C" int moe355_init_routing(const void* x, int x_dtype, int64_t num_token
                              workspace_bytes, stream);
 }
 
+bool moe355::one_launch_map(int64_t pairs, int num_experts)
+{
+    return pairs > 0 && pairs <= kMapMaxPairs && num_experts <= kMapMaxExperts;
+}
+
 int moe355::route_map_impl(const int32_t* expert_idx, int64_t num_tokens, int top_k, int num_experts,
                            int tokens_num_type, int32_t* expanded_row_idx, int32_t* row_token, int64_t* expert_tokens,
                            void* workspace, size_t workspace_bytes, const TileSpec* specs, int nspecs, bool* built,
@@ -634,7 +639,7 @@ int moe355::route_map_impl(const int32_t* expert_idx, int64_t num_tokens, int to
     if (R > 0 && (!expert_idx || !expanded_row_idx || !row_token)) return MOE355_E_ARG;
     int nch, parts, cpp, nbits;
     const RouteWs ws = route_ws_of(workspace, R, num_experts, nch, parts, cpp, nbits);
-    if (R > 0 && R <= kMapMaxPairs && num_experts <= kMapMaxExperts) {
+    if (one_launch_map(R, num_experts)) {
         RouteMapArgs a = {};
         a.ids = expert_idx;
         a.R = (int)R;
