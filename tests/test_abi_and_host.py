@@ -561,6 +561,23 @@ def test_where_gate_up_tiles_quantise_their_rows(experts, k, n, rows, tile_rows)
     assert _lib.load().moe355_meeting_tile_rows(rows, k, n, experts) == tile_rows
 
 
+def test_columns_of_a_routed_tile_have_places():
+    """96 workgroups of the 64-row tiles run on an XCD, 64 of the 128-row ones and 32 of the wide ones, where a tall tile may wait with
+    both halves; a launch may hold all but one of a tile's columns, and another stream's launch as many."""
+    from vllm_ascend_amd import _lib
+
+    rows_of = _lib.load().moe355_meeting_tile_rows
+    seen = set()
+    for experts in (1, 4, 6, 10, 16, 32, 128, 256, 512):
+        for k in (64, 384, 1024, 2880, 7168):
+            for n in [*range(64, 12289, 192), *range(12288, 50000, 512)]:
+                for rows in (6, 18, 48, 63, 100, 144, 250, 1000):
+                    tile = rows_of(rows * experts, k, n, experts)
+                    seen.add(tile)
+                    assert -(-n // (512 if tile == 256 else 256)) <= {0: n, 64: 48, 128: 16, 256: 8}[tile], (experts, k, n, rows)
+    assert seen == {0, 64, 128, 256}
+
+
 def test_no_words_for_a_meeting_that_does_not_take_place():
     """The words (a word for every pair and column of a tile) end with the one-launch map, at 65536 pairs."""
     from vllm_ascend_amd import _lib

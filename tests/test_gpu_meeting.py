@@ -67,12 +67,12 @@ def _with_shared(layer, S, H, seed, overlap=False, limit=0.0):
     layer.shared_experts = AscendSharedExperts(up, up_scale, down, down_scale, multistream_overlap=overlap, swiglu_limit=limit)
 
 
-# one column block and several, whole and partial ones (128 values each), 64- and 128-row tiles, a list whose tiles two XCDs
-# share, K of one step and of every remainder modulo the ring
+# one column block and several, whole and partial ones (128 values each; 40 and 47 of the 48 that there may be), 64- and 128-row tiles,
+# a list whose tiles two XCDs share, K of one step and of every remainder modulo the ring
 @pytest.mark.parametrize("E, k, T, H, I, tile_rows", [
     (8, 2, 512, 64, 32, 128), (8, 2, 513, 128, 160, 128), (8, 2, 515, 192, 288, 64), (8, 2, 521, 256, 512, 64), (6, 2, 600, 320, 1408, 64),
     (32, 4, 517, 512, 512, 64), (16, 4, 2049, 256, 1024, 128), (64, 8, 384, 448, 640, 128), (128, 8, 257, 256, 640, 64),
-    (96, 8, 257, 256, 1024, 128)])
+    (96, 8, 257, 256, 1024, 128), (16, 2, 500, 384, 5120, 64), (16, 4, 250, 320, 5984, 64)])
 @pytest.mark.parametrize("skew", [0.0, 3.0])
 def test_layers_on_tiles(E, k, T, H, I, tile_rows, skew):
     print(f"E={E} k={k} T={T} H={H} I={I} skew={skew} tiles of {_lib().moe355_meeting_tile_rows(T * k, H, 2 * I, E)}", flush=True)

@@ -1029,7 +1029,9 @@ extern "C" int moe355_next_meeting_looks(int looks)
 // rows per expert in brackets:
 //   - dividing: 8 columns, 64 and 128 experts of 2048 / 1024 (18 to 160) 0.99 .. 0.94 (1.01 .. 0.95); 4 columns, 256 of 2048 / 512 (9 to
 //     160) 1.00 .. 0.92 (0.97 .. 0.93), 64 of 1024 / 512 0.99 .. 0.94 (0.97 .. 0.92); 16 columns, 256 of 7168 / 2048 (6 and 16) 0.98 and
-//     0.96 (0.97 at 16);
+//     0.96 (0.97 at 16), 64 of 4096 / 2048 (12 and 36) 1.00 and 0.95 (1.00 and 0.96), 8 of 2048 / 2048 (40 / 250 / 1000) 1.01 / 0.97 / 0.97
+//     (1.01 / 0.94 / 0.97); 2 columns, 64 of 1024 / 256, 128 of 2048 / 256, 256 and 32 of 4096 / 256 (9 to 48) 0.98 .. 0.95 (0.99 .. 0.95); one,
+//     64 of 2048 / 128 (48) 0.96 (0.93);
 //   - others: 6 columns, 128 of 2048 / 768 (54 / 100 / 200 / 300) 0.98 / 0.99 / 0.96 / 0.94 (0.97 / 0.99 / 0.96 / 0.96), 256 of them (18 / 48 /
 //     100 / 300) 1.03 / 0.97 / 0.98 / 1.00 (1.00 / 0.99 / 0.96 / 0.99); 11 columns, 60 of 2048 / 1408 (30 / 64 / 128 / 300) 0.98 / 0.96 /
 //     0.97 / 0.95 (1.03 / 0.98 / 1.01 / 0.98), 8 of 1024 / 1408 (250 to 2000) 0.96 .. 0.92; 12 columns of 12 and 16 MB an expert, 64 of
@@ -1039,14 +1041,24 @@ extern "C" int moe355_next_meeting_looks(int looks)
 //   - a launch with workgroups for more than two and up to three per compute unit (128 of 2048 / 768: 768) loses on 128-row tiles, which
 //     fill a round and a half (9 / 18 / 27 / 36 rows 1.06 / 1.04 / 1.02 / 1.01, Zipf(1.1) 0.98 / 0.99 / 1.01 / 0.99), and wins on tiles of
 //     64 rows, three of which fit a compute unit: 0.99 / 0.97 / 0.95 / 0.94 (0.96 / 0.94 / 0.95 / 0.98; Zipf(0.8) 0.98 / 1.01 / 0.96 / 0.97),
-//     at 48 and 60 rows 0.99 and 0.94 (0.99 and 0.97; 1.00 and 1.00).  Not with 12 MB an expert, whose hot ones read them again for every
-//     tile (64 of 4096 / 1536, 36 / 48 / 60 rows under Zipf(1.1) 1.06 / 1.08 / 1.09).
+//     at 48 and 60 rows 0.99 and 0.94 (0.99 and 0.97; 1.00 and 1.00).  The same at 18 / 36 / 60 rows of 128 of 2048 / 640 0.96 / 0.93 / 0.90
+//     (1.01 / 0.95 / 0.96; Zipf(0.8) 0.96 at 18), 128 of 3072 / 640 0.98 / 0.96 / 0.96 (0.99 / 0.96 / 0.98), 96 of 2560 / 768 0.97 / 0.95 /
+//     0.90 (0.95 / 0.95 / 0.97), 96 of 2048 / 896 0.96 / 0.94 / 0.93 (1.00 / 0.99 / 0.97), 256 of 4096 / 384 0.96 / 0.95 / 1.00 (0.90 / 0.93 /
+//     0.99), 64 of 1024 / 1536 0.94 / 0.89 / 0.91 (0.94 / 0.97 / 0.97), 64 of 1536 / 1280 0.97 / 0.94 / 0.94 (0.96 / 0.96 / 0.97), at 18 and 36 of
+//     256 of 2048 / 384 0.96 and 0.91 (0.92 and 0.98), 100 of 2048 / 768 0.97 and 0.95 (1.05 and 0.91), at 9 of five of them 0.97 .. 0.98
+//     (0.95 .. 0.97): 1.5 to 3.9 MB an expert.  Not with 12 MB, whose hot experts read them again for every tile (64 of 4096 / 1536, 36 / 48 / 60
+//     rows under Zipf(1.1) 1.06 / 1.08 / 1.09); between 4 and 12 MB nothing was measured.  Up to 48 columns, half of the 96 places of an
+//     XCD, so that two launches can wait there: 30 of 768 / 2304 (18 columns) at 36 and 60 rows 0.93 and 0.88 (0.94 and 0.94), 32 of 768 /
+//     2560 0.92 and 0.98 (1.03 and 0.98), 24 of 512 / 4096 (32) 0.92 and 0.96 (0.97 and 0.97), 16 of 384 / 5120 (40) 0.81 (0.90) at 60.
 //   - wide tiles, 8 columns of 512 channels, 64 experts of 7168 / 2048 (40 / 64 / 96 / 128 / 160 / 200) 0.98 / 0.98 / 0.97 / 0.96 / 0.98 / 1.00
 //     (0.98 / 0.97 / 0.98 / 0.98 / 1.04 / 0.99), 256 of them (47 / 94 / 128) 0.94 / 0.95 / 1.00; 4 columns, 64 of 4096 / 1024 (64 / 128 / 200)
 //     0.97 / 0.95 / 0.99 (0.99 / 0.97 / 0.98); 3 columns, 128 of 2048 / 768 (125) 0.95 (0.98), 160 of 4096 / 768 (40 / 100 / 160) 0.94 / 0.96
 //     / 1.00 (0.99 / 0.97 / 0.98); 6 columns, 128 of 4096 / 1536 (64 / 80 / 112 / 160) 1.03 / 1.04 / 1.03 / 1.08 (1.00 / 0.99 / 1.00 / 1.02);
-//     10 columns, 128 of 5120 / 2560 (40 / 96 / 128 / 160) 1.00 / 1.02 / 1.02 / 1.05 (0.98 / 1.01 / 1.02 / 1.00).  So up to 4 columns and
-//     with 8, to 144 rows.
+//     10 columns, 128 of 5120 / 2560 (40 / 96 / 128 / 160) 1.00 / 1.02 / 1.02 / 1.05 (0.98 / 1.01 / 1.02 / 1.00); 8 columns again, 64 and
+//     16 of 4096 / 2048 (100) 0.94 and 0.95 (1.00 and 1.03; Zipf(0.8) 1.00 with 16).  So up to 4 columns and with 8, to 144 rows.
+//   - beside a shared expert on its side stream, whose workgroups hold places too: 128 of 2048 / 768, 300 / 777 / 2000 / 8192 tokens 1.00 /
+//     0.97 / 0.94 / 0.93; 256 of 7168 / 2048, 512 / 1000 / 2048 / 4096 0.99 / 0.95 / 0.99 / 0.97; 64 of 2048 / 2048, 500 / 1000 / 4000 0.95 / 0.94 /
+//     0.96: as without.
 MeetingPlan moe355::meeting_plan(int64_t rows, int64_t k, int64_t n, int num_experts)
 {
     GmmArgs a = {};
@@ -1066,7 +1078,8 @@ MeetingPlan moe355::meeting_plan(int64_t rows, int64_t k, int64_t n, int num_exp
     if (bm == 0) return {};
     if (columns <= 16 && (columns & (columns - 1)) == 0) return yes;
     const int64_t least = (int64_t)num_experts * columns;
-    if (bm == 128 && least > 2 * kComputeUnits && least <= 3 * kComputeUnits && own <= (4 << 20) && avg < 64) return {64, columns};
+    if (bm == 128 && least > 2 * kComputeUnits && least <= 3 * kComputeUnits && own <= (4 << 20) && avg < 64 && columns <= 48)
+        return {64, columns};
     return columns <= 12 && own <= (8 << 20) && avg >= 48 ? yes : MeetingPlan{};
 }
 
@@ -1082,7 +1095,9 @@ extern "C" int moe355_meeting_tile_rows(int64_t rows, int64_t k, int64_t n, int 
 // 4500, Zipf(1.1) 4096 2591 and 2557, int4 4096 2713 and 2698; 64 experts of 2048 / 2048, 4096 / 8000 tokens 674 / 1174 and 656 / 1142, of
 // 4096 / 1024, 8192 tokens 1214 and 1198.  The columns need not divide an XCD's 32 places here (64 of 4096 / 1536, 4096 / 7000 tokens
 // 1014 / 1596 and 1000 / 1579; 2048 / 2816, 4500 1071 and 1052; 7168 / 2560, 4096 2537 and 2532; 7168 / 1408, 8192 2973 and 2959), but
-// those of a row of tiles must all have a place there (dense_split).  64 are what a wavefront looks at at once.
+// those of a row of tiles must all have a place there: dense_split leaves out the wide rectangles (8 experts of 2048 / 512 with 32000
+// tokens of 4224 channels, 40192 of 5120 and, with 1024, 64768 of 8192: 1826 / 2383 / 4164 and 1494 / 1846 / 2894).  64 are what a
+// wavefront looks at at once.
 int moe355::shared_meeting_columns(int64_t rows, int64_t k, int64_t n)
 {
     GmmArgs a = {};
