@@ -190,8 +190,10 @@ __device__ __forceinline__ void tiled_epilogue_body(const GmmArgs& a, int e, v4i
 // - Every workgroup stores the maxima of its rows over its columns into a word of its own per row (with the sign set: a word of
 //   zero is not there yet) and looks at the others' until none is missing: no counter, no order, no fence, since a word is all that
 //   is handed over.  The routing launch clears the words.
-// - They run at the same time, because a launch starts its workgroups in order and those of a tile are neighbours.  Nothing rests on
-//   that: a workgroup that has looked meet_looks times (a few milliseconds) computes the maxima that are still missing itself.
+// - They run at the same time, because a launch starts its workgroups in order, those of a tile are neighbours, and those of them that
+//   run on one XCD find a place there all at once (at most 48 of 96 for the 64-row tiles, 16 of 64 for the 128-row ones, 8 of 32 for
+//   the wide ones, of a tall tile's two entries 16; dense_split for the dense ones).  No result rests on that: a workgroup
+//   that has looked meet_looks times (a few milliseconds) computes the maxima that are still missing itself.
 // What it costs is that they wait for the slowest, which is why the number of columns matters (meeting_plan in gmm.hip).  us a layer
 // with / without, 128 experts of 2048 / 768, 777 / 2000 / 4000 / 8192 tokens 138 / 184 / 292 / 496 against 143 / 194 / 313 / 531; 256 of
 // 7168 / 2048, 500 / 1500 / 3000 tokens 1712 / 1831 / 2049 against 1770 / 1956 / 2157; 8 of 1024 / 1408, 6000 tokens 105 against 115.
@@ -272,7 +274,9 @@ __device__ __forceinline__ void meet_body(const GmmArgs& a, const TilePart& p, v
     float* const part = (float*)lds + (g * 4 + quarter) * ROWS + lrow + tok;
     int* const met = (int*)(scales + ROWS);  // (in the place of channel scales that have been read by then)
     const float* const cs = scales + ROWS + g * 64;
-    // With ten groups of 16 rows and more there is no room for all values beside the sums: those of the first four go to LDS.
+    // With ten groups of 16 rows and more there is no room for all values beside the sums: those of the first four go to LDS.  That
+    // is enough for ten.  For twelve it is not: gmm_wide_kernel<EPI_MEET> spills 58 registers in the epilogue of the 192-row body
+    // (for up to six groups there is room in LDS, which has not been tried).
     constexpr int STASH = NB2 > 8 ? 4 : 0;
     constexpr int STASH_AT = (ROWS * PITCH + (ROWS + 64 * GROUPS) * 4 + 15) / 16 * 16;  // behind the scales
     v4f* const stash = (v4f*)(lds + STASH_AT) + g * (STASH * 2 * 64) + lane;
