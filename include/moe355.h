@@ -504,7 +504,8 @@ int moe355_profile_next_gemm(void *start_event, void *stop_event);
 
 /* On the sorted path of moe355_layer_forward the workgroups of a tile of the gate_up product can exchange the maxima of its rows
  * and quantise them in place: the rows of those tiles, or 0 where the fp32 values go through memory and a launch of their own,
- * among others with more than 65536 pairs or 512 experts, whose maps are not built by one launch.
+ * among others with more than 65536 pairs or 512 experts, whose maps are not built by one launch.  (Nor do batches of a layer with a
+ * sync_counter that moe355_route_quant_small_supported takes: gating and sorting are one launch there.)
  * A workgroup that has looked for the others' maxima 4096 times computes them itself; in the next layer call of the calling
  * thread it gives up after `looks` instead (0: at once; more than 4096 are 4096).  The results are the same either way.
  */
